@@ -609,16 +609,27 @@ extern "C" int br_add_position_rows(float* x, const void* table, int is_bf16, co
 // ------------------------------------------------------------------ row gather -----
 // out[i, :] = x[rows[i], :] (float)   reference: D2dCopy of the last row,
 // megakernel/megakernel_compile.rs:522-527.
-__global__ void gather_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows,
-                                   float* __restrict__ out, int H) {
+// grid (R, pieces of 256 VEC elements): rows are logits of a single-token step (1 x 32,768 floats: one workgroup a row
+// took 61 us, bound by one compute unit's loads; spread out it is a launch, 2 to 3 us) or hidden rows.  VEC 4: H in steps of 4, aligned rows.
+template <int VEC>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows,
+                                                          float* __restrict__ out, int H) {
     const float* xr = x + (size_t)rows[blockIdx.x] * H;
     float* o = out + (size_t)blockIdx.x * H;
-    for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = xr[i];
+    for (size_t i = ((size_t)blockIdx.y * 256 + threadIdx.x) * VEC; i < (size_t)H; i += (size_t)gridDim.y * 256 * VEC) {
+        float v[VEC];
+        ew_load<float, VEC>(xr + i, v);
+        ew_store<float, VEC>(o + i, v);
+    }
 }
 
 extern "C" int br_gather_rows(const float* x, const int* rows, float* out, int R, int H, hipStream_t s) {
     if (R <= 0 || H <= 0) return BR_OK;
-    gather_rows_kernel<<<R, 128, 0, s>>>(x, rows, out, H);
+    const bool vec = H % 4 == 0 && (((uintptr_t)x | (uintptr_t)out) & 15) == 0;
+    const int pieces = (H + (vec ? 1023 : 255)) / (vec ? 1024 : 256);
+    const dim3 grid(R, pieces < 65535 ? pieces : 65535);
+    if (vec) gather_rows_kernel<4><<<grid, 256, 0, s>>>(x, rows, out, H);
+    else gather_rows_kernel<1><<<grid, 256, 0, s>>>(x, rows, out, H);
     return br_check_launch();
 }
 
