@@ -677,21 +677,269 @@ __global__ __launch_bounds__(256) void experts_down_grouped_kernel(const bf16* _
     }
 }
 
+// ------------------------------------- few tokens, the weights streamed through LDS -----
+// The same two products where K is long enough to share out (K in steps of 128 from 1,024): a step of few tokens is bound
+// by reading the chosen experts' matrices once, and straight loads into operands ask for them in pieces of 32 bytes a row.
+// Here one workgroup a compute unit stays and walks a run of units; a unit is 16 weight rows of one expert against up to
+// XR of its pairs.  The units of the experts that have pairs are counted through, every workgroup takes an equal run of
+// them, so experts without pairs leave no compute unit idle.  As in the library's other streaming products the eight waves
+// take a unit's 128-wide k-chunks in turn, each into an LDS ring of its own by direct loads (256-byte row pieces, the
+// weights non-temporal, the next chunk on its way across unit ends; 16-byte columns XOR-swizzled by the row), and the
+// waves' sums meet in LDS in wave order, one barrier a unit.  Where a unit starts in k depends on its rows only, so a
+// pair's output does not depend on what else is in the step.  An expert with more than XR pairs has its rows' units one
+// after the other; the second read of the rows comes from the caches.
+// 32 experts of 1,792 by 4,096, 8 chosen, `up` / `down` in us (the chosen experts' bytes at TB/s), against straight loads into
+// operands: 1 token 39 / 22 (6.1 / 5.3) against 213 / 99; 6 tokens 127 / 64 (6.5 / 6.4) against 239 / 116; 16 tokens 150 / 81
+// against 253 / 133; 40 tokens 161 / 102 against 277 / 141.  Bound by the memory up to about 16 pairs an expert.
+//   UP: unit t is gate rows 8 t .. + 8 and the up rows of the same channels; y[p, f] = the gated unit, bfloat16.
+//   else: unit t is rows 16 t .. + 16 of W_d; out[p, n] float.
+#ifndef RX_STREAM_TOKENS
+#define RX_STREAM_TOKENS 64
+#endif
+#define RXS_KC 128
+#define RXS_NW 8
+#define RXS_S 2
+#define RXS_MAX_E 512
+#define RXS_MAX_PAIRS 1024
+
+struct RxUnit { int e, t, j, p0, np; };       // expert, unit of its rows, group of its pairs: the group's first pair and size
+
+template <int XR>
+__device__ __forceinline__ RxUnit rx_unit_at(int u, const int* cum, const int* firstL, int E, int tiles) {
+    int lo = 0, hi = E;                                       // the expert with cum[e] <= u < cum[e + 1]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (cum[mid] <= u) lo = mid; else hi = mid;
+    }
+    RxUnit r;
+    r.e = lo;
+    const int n = firstL[lo + 1] - firstL[lo], groups = (n + XR - 1) / XR, at = u - cum[lo];
+    r.t = at / groups;
+    r.j = at - r.t * groups;
+    r.p0 = firstL[lo] + r.j * XR;
+    r.np = min(XR, firstL[lo + 1] - r.p0);
+    r.e = __builtin_amdgcn_readfirstlane(r.e);
+    r.t = __builtin_amdgcn_readfirstlane(r.t);
+    r.j = __builtin_amdgcn_readfirstlane(r.j);
+    r.p0 = __builtin_amdgcn_readfirstlane(r.p0);
+    r.np = __builtin_amdgcn_readfirstlane(r.np);
+    return r;
+}
+
+template <int XR>
+__device__ __forceinline__ void rx_next_unit(RxUnit& r, const int* firstL, int E, int tiles) {
+    int end = __builtin_amdgcn_readfirstlane(firstL[r.e + 1]);
+    if (r.p0 + XR < end) {
+        ++r.j;
+        r.p0 += XR;
+    } else {
+        r.j = 0;
+        if (++r.t == tiles) {
+            r.t = 0;
+            do {
+                ++r.e;
+                r.p0 = end;
+                end = __builtin_amdgcn_readfirstlane(firstL[r.e + 1]);
+            } while (r.e < E && end == r.p0);                 // firstL[E + 1] = firstL[E]: ends behind the last expert
+        } else r.p0 = __builtin_amdgcn_readfirstlane(firstL[r.e]);
+    }
+    r.np = min(XR, end - r.p0);
+}
+
+template <int XR, bool UP>
+__global__ __launch_bounds__(RXS_NW * 64) void experts_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wt,
+                                                                     const int* __restrict__ first, const int* __restrict__ order,
+                                                                     void* __restrict__ C, int E, int N, int K, int top, float limit,
+                                                                     float alpha) {
+    constexpr int ROWB = RXS_KC * 2;                          // bytes of a row's chunk
+    constexpr int STAGE = (16 + XR) * ROWB, WDMA = 4, NDMA = STAGE / 1024, S = RXS_S, NW = RXS_NW, D = S - 1;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    float* red = (float*)(smem + NW * S * STAGE);             // [2][NW][16][17]
+    int* firstL = (int*)(red + 2 * NW * 16 * 17);             // [E + 2]
+    int* cum = firstL + E + 2;                                // [E + 1] units before expert e
+    int* tok = cum + E + 1;                                   // UP: [pairs] the token of a pair
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int tiles = UP ? N / 8 : N / 16;
+    for (int e = tid; e <= E; e += NW * 64) {
+        firstL[e] = first[e];
+        if (e == E) firstL[E + 1] = first[E];
+    }
+    __syncthreads();
+    if (UP)
+        for (int p = tid; p < firstL[E]; p += NW * 64) tok[p] = order[p] / top;
+    if (tid < 64) {
+        int run = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            const int mine = e < E ? (firstL[e + 1] - firstL[e] + XR - 1) / XR * tiles : 0;
+            int sum = mine;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += v;
+            }
+            if (e < E) cum[e] = run + sum - mine;
+            run += __shfl(sum, 63, 64);
+        }
+        if (lane == 0) cum[E] = run;
+    }
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(cum[E]);
+    const int u0 = (int)((long long)total * blockIdx.x / gridDim.x), u1 = (int)((long long)total * (blockIdx.x + 1) / gridDim.x);
+    if (u0 >= u1) return;
+    const int nch = K / RXS_KC, ncw = (nch - wave + NW - 1) / NW;
+    const int nitems = (u1 - u0) * ncw;
+    unsigned char* ring = smem + wave * (S * STAGE);
+    const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)ring);
+    // a wave-load brings 4 rows of 256 bytes; this lane's byte offsets within an expert's matrix at unit 0 and chunk 0
+    const int drow = lane >> 4, dcol = lane & 15;
+    unsigned woff[WDMA], aoff[NDMA - WDMA];
+#pragma unroll
+    for (int q = 0; q < WDMA; ++q) {
+        const int row = q * 4 + drow;
+        const int at = UP ? (row < 8 ? row : N + row - 8) : row;
+        woff[q] = (unsigned)at * (unsigned)K * 2 + (unsigned)((dcol ^ (row & 7)) * 16);
+    }
+    RxUnit is = rx_unit_at<XR>(__builtin_amdgcn_readfirstlane(u0), cum, firstL, E, tiles), cp = is;
+    int is_c = 0, cp_c = 0, buf = 0;
+    int rot = 0;                                              // where unit `is` starts in k
+    const unsigned char* wbase = nullptr;                     // its first weight row
+    auto enter = [&]() {                                      // the issue cursor is at another unit
+        rot = (int)(((unsigned)(is.e * tiles + is.t) * 2654435761u) >> 8) % nch;
+        wbase = (const unsigned char*)Wt + ((size_t)is.e * (UP ? 2 * N : N) + (size_t)is.t * (UP ? 8 : 16)) * K * 2;
+#pragma unroll
+        for (int q = 0; q < NDMA - WDMA; ++q) {
+            const int m = q * 4 + drow, p = is.p0 + min(m, is.np - 1);
+            aoff[q] = (unsigned)(UP ? tok[p] : p) * (unsigned)K * 2 + (unsigned)((dcol ^ (m & 7)) * 16);
+        }
+    };
+    enter();
+    auto issue = [&](int slot) {
+        int chunk = wave + is_c * NW + rot;
+        if (chunk >= nch) chunk -= nch;
+        const unsigned lds = __builtin_amdgcn_readfirstlane(ring_lds + slot * STAGE);
+        const unsigned long long wb = (unsigned long long)(wbase + (size_t)chunk * ROWB), ab = (unsigned long long)A + (size_t)chunk * ROWB;
+#pragma unroll
+        for (int q = 0; q < NDMA; ++q) {
+            if (q < WDMA)                                     // weights pass once: non-temporal
+                asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3 nt" ::"s"(lds), "n"(q * 1024), "v"(woff[q]), "s"(wb) : "m0", "scc", "memory");
+            else
+                asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" ::"s"(lds), "n"(q * 1024), "v"(aoff[q < WDMA ? 0 : q - WDMA]), "s"(ab) : "m0", "scc", "memory");
+        }
+        if (++is_c == ncw) {
+            is_c = 0;
+            rx_next_unit<XR>(is, firstL, E, tiles);
+            if (is.e < E) enter();
+        }
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+        if (j < nitems) issue(j);
+    for (int base = 0; base < nitems; base += S) {
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+            const int it = base + j;
+            if (it >= nitems) break;
+            if (it + D - 1 < nitems) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * NDMA) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (it + D < nitems) issue((j + D) % S);
+            const unsigned char* st = ring + j * STAGE;
+            const int xr = XR == 8 ? (r16 & 7) : r16;
+            bf16x8 wf[4], xv[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                wf[k] = *(const bf16x8*)(st + r16 * ROWB + (((4 * k + g) ^ (r16 & 7)) * 16));
+                xv[k] = *(const bf16x8*)(st + (16 + xr) * ROWB + (((4 * k + g) ^ (xr & 7)) * 16));
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k += 2) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k], xv[k], acc, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k + 1], xv[k + 1], acc1, 0, 0, 0);
+            }
+            if (++cp_c < ncw) continue;
+            cp_c = 0;
+            float* rb = red + buf * (NW * 16 * 17);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rb[(wave * 16 + 4 * g + r) * 17 + r16] = acc[r] + acc1[r];
+            acc = {0.f, 0.f, 0.f, 0.f};
+            acc1 = {0.f, 0.f, 0.f, 0.f};
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (UP) {
+                const int m = tid >> 3, f = tid & 7;
+                if (m < cp.np) {
+                    float gs = 0.f, us = 0.f;
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) { gs += rb[(w * 16 + f) * 17 + m]; us += rb[(w * 16 + f + 8) * 17 + m]; }
+                    ((bf16*)C)[(size_t)(cp.p0 + m) * N + cp.t * 8 + f] = (bf16)rx_glu(gs, us, limit, alpha);
+                }
+            } else {
+                const int m = tid >> 4, n = tid & 15;
+                if (m < cp.np) {
+                    float v = 0.f;
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) v += rb[(w * 16 + n) * 17 + m];
+                    ((float*)C)[(size_t)(cp.p0 + m) * N + cp.t * 16 + n] = v;
+                }
+            }
+            buf ^= 1;
+            rx_next_unit<XR>(cp, firstL, E, tiles);
+        }
+    }
+}
+
+// What experts_stream_kernel asks for: `pairs` pairs, an expert's matrix of `rows` rows of K, every wave a chunk.
+static bool rx_stream_takes(const void* A, const void* Wt, size_t a_rows, int pairs, int E, int rows, int K) {
+    return K % RXS_KC == 0 && K >= RXS_KC * RXS_NW && E <= RXS_MAX_E && pairs <= RXS_MAX_PAIRS && (((uintptr_t)A | (uintptr_t)Wt) & 15) == 0 &&
+           (size_t)rows * K * 2 < (1ull << 32) && a_rows * (size_t)K * 2 < (1ull << 32) &&
+           (long long)E * rows / 8 * ((pairs + 7) / 8) < (1ll << 31);
+}
+
+template <int XR, bool UP>
+static int rx_launch_stream(const void* A, const void* Wt, const int* first, const int* order, void* C, int E, int N, int K, int top,
+                            float limit, float alpha, hipStream_t s) {
+    const int cus = br_device_cus();
+    if (!cus) return BR_LAUNCH_FAILED;
+    constexpr size_t lds = (size_t)RXS_NW * RXS_S * (16 + XR) * RXS_KC * 2 + 2 * RXS_NW * 16 * 17 * 4 + (2 * RXS_MAX_E + 3) * 4 + RXS_MAX_PAIRS * 4;
+    static_assert(lds <= 160 * 1024, "LDS");
+    auto kern = experts_stream_kernel<XR, UP>;
+    static bool set = false;
+    if (!set) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
+        set = true;
+    }
+    kern<<<cus, RXS_NW * 64, lds, s>>>((const bf16*)A, (const bf16*)Wt, first, order, C, E, N, K, top, limit, alpha);
+    return br_check_launch();
+}
+
 // Whether the grouped kernels take these sizes: rows of 16 bytes' multiples.
 extern "C" int br_experts_grouped_takes(int W, int F) { return W > 0 && F > 0 && W % 8 == 0 && F % 8 == 0; }
 
 extern "C" int br_experts_up_grouped(const void* h, const void* w_gu, const int* first, const int* order, void* y, int E,
                                      int W, int F, int top, int n_tokens, float limit, float alpha, hipStream_t s) {
     if (!br_experts_grouped_takes(W, F) || E <= 0 || top <= 0 || (F + 31) / 32 > 65535) return BR_BAD_ARG;
+    const int pairs = n_tokens * top;
+    if (n_tokens <= RX_STREAM_TOKENS && F % 8 == 0 && rx_stream_takes(h, w_gu, n_tokens, pairs, E, 2 * F, W)) {
+        if (n_tokens <= 8) return rx_launch_stream<8, true>(h, w_gu, first, order, y, E, F, W, top, limit, alpha, s);
+        return rx_launch_stream<16, true>(h, w_gu, first, order, y, E, F, W, top, limit, alpha, s);
+    }
     const dim3 grid(E, (F + 31) / 32);
     if (n_tokens <= 32) experts_up_grouped_kernel<1, 1><<<grid, 256, 0, s>>>((const bf16*)h, (const bf16*)w_gu, first, order, (bf16*)y, W, F, top, limit, alpha);
     else experts_up_grouped_kernel<2, 2><<<grid, 256, 0, s>>>((const bf16*)h, (const bf16*)w_gu, first, order, (bf16*)y, W, F, top, limit, alpha);
     return br_check_launch();
 }
 
-extern "C" int br_experts_down_grouped(const void* y, const void* w_down, const int* first, float* out, int E, int W, int F,
+extern "C" int br_experts_down_grouped(const void* y, const void* w_down, const int* first, float* out, int pairs, int E, int W, int F,
                                        int n_tokens, hipStream_t s) {
     if (!br_experts_grouped_takes(W, F) || E <= 0 || (W + 31) / 32 > 65535) return BR_BAD_ARG;
+    if (n_tokens <= RX_STREAM_TOKENS && W % 16 == 0 && rx_stream_takes(y, w_down, pairs, pairs, E, W, F)) {
+        if (n_tokens <= 8) return rx_launch_stream<8, false>(y, w_down, first, nullptr, out, E, W, F, 1, 0.f, 0.f, s);
+        return rx_launch_stream<16, false>(y, w_down, first, nullptr, out, E, W, F, 1, 0.f, 0.f, s);
+    }
     const dim3 grid(E, (W + 31) / 32);
     if (n_tokens <= 32) experts_down_grouped_kernel<1, 1><<<grid, 256, 0, s>>>((const bf16*)y, (const bf16*)w_down, first, out, W, F);
     else experts_down_grouped_kernel<2, 2><<<grid, 256, 0, s>>>((const bf16*)y, (const bf16*)w_down, first, out, W, F);

@@ -1394,8 +1394,8 @@ def experts_down_grouped(y: torch.Tensor, w_down: torch.Tensor, first: torch.Ten
     E, W, _ = w_down.shape
     _req(experts_grouped_takes(y.dtype, W, F) and w_down.dtype == torch.bfloat16 and out.dtype == torch.float32, "experts_down_grouped: types")
     _req(w_down.shape == (E, W, F) and out.shape == (n, W) and first.numel() in (E + 1, E + 2) and first.dtype == torch.int32, "experts_down_grouped: shapes")
-    f = _fn("routed_experts", "br_experts_down_grouped", [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P])
-    _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), E, W, F, int(n_tokens), _stream()), "experts_down_grouped")
+    f = _fn("routed_experts", "br_experts_down_grouped", [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P])
+    _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), n, E, W, F, int(n_tokens), _stream()), "experts_down_grouped")
 
 
 def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: torch.Tensor) -> None:

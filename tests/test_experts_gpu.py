@@ -1,0 +1,103 @@
+"""The routed experts' products at the edges of their kernels' tiles, against float64 products of the same bfloat16 values."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def bf(a):
+    return torch.tensor(a, dtype=torch.float32).to(torch.bfloat16)
+
+
+def sorted_pairs(chosen, bins):
+    from braidinfer_amd import kernels as K
+    n = chosen.numel()
+    first, order, place = (torch.zeros(k, dtype=torch.int32, device="cuda") for k in (bins + 1, n, n))
+    K.experts_sort(chosen, first, order, place, bins)
+    return first, order, place
+
+
+def drawn(T, top, E, how, seed):
+    """[T, top] expert numbers: spread evenly, drawn, or all tokens to the last `top` experts."""
+    rng = np.random.default_rng(seed)
+    if how == "one":
+        rows = [np.arange(E - top, E)] * T
+    else:
+        rows = [rng.permutation(E)[:top] for _ in range(T)]
+    return torch.tensor(np.stack(rows).astype(np.int32)).cuda()
+
+
+def products(h, w_gu, w_down, chosen, limit, alpha):
+    """float64: (y [T, top, F], W_d y with y rounded as the kernels store it [T, top, W])."""
+    h64, gu, dn = h.cuda().double(), w_gu.cuda(), w_down.cuda()
+    T, top = chosen.shape
+    F, W = gu.shape[1] // 2, gu.shape[2]
+    y = torch.zeros(T, top, F, dtype=torch.float64, device="cuda")
+    out = torch.zeros(T, top, W, dtype=torch.float64, device="cuda")
+    for e in range(gu.shape[0]):
+        t, s = (chosen == e).nonzero(as_tuple=True)
+        if len(t):
+            z = h64[t] @ gu[e].double().T
+            g, u = z[:, :F], z[:, F:]
+            if alpha:
+                g, u = g.clamp(max=limit), u.clamp(-limit, limit) + 1.0
+                v = g * torch.sigmoid(alpha * g) * u
+            else:
+                v = g * torch.sigmoid(g) * u
+            y[t, s] = v
+            out[t, s] = v.to(torch.bfloat16).double() @ dn[e].double().T
+    return y, out
+
+
+# widths with 8 to 33 chunks of 128 (every wave one, some two, some four); tokens at 1, around 8 and 16 pairs an expert, and
+# beyond; experts without pairs, all pairs in the last experts, numbers behind the experts (identities)
+@pytest.mark.parametrize("T,top,E,W,F,how,identity,alpha", [
+    (1, 1, 1, 1024, 1024, "drawn", 0, 0.0), (1, 8, 32, 2048, 1408, "drawn", 0, 0.0), (6, 8, 32, 4224, 1792, "drawn", 0, 0.0),
+    (8, 2, 5, 1152, 1032, "one", 0, 1.702), (9, 2, 5, 1152, 1024, "one", 0, 0.0), (16, 3, 7, 1024, 1280, "one", 0, 0.0),
+    (17, 3, 70, 1024, 1152, "drawn", 3, 0.0), (40, 8, 32, 1536, 1792, "drawn", 0, 0.0), (64, 4, 16, 2048, 1408, "one", 2, 1.702),
+    (64, 16, 16, 1024, 1024, "drawn", 0, 0.0)])
+def test_products_of_few_tokens(T, top, E, W, F, how, identity, alpha):
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(T + W + F)
+    h, w_gu, w_down = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5), bf(rng.standard_normal((E, W, F)) / F ** 0.5)
+    chosen = drawn(T, top, E + identity, how, T)
+    want_y, want = products(h, w_gu, w_down, chosen, 0.9, alpha)
+    first, order, place = sorted_pairs(chosen, E + (1 if identity else 0))
+    hd, gu, dn = h.cuda(), w_gu.cuda(), w_down.cuda()
+    n = T * top
+    y = torch.full((n, F), 7.0, dtype=torch.bfloat16, device="cuda")
+    K.experts_up_grouped(hd, gu, first, order, y, top, 0.9 if alpha else 0.0, alpha)
+    out = torch.full((n, W), 7.0, dtype=torch.float32, device="cuda")
+    K.experts_down_grouped(y, dn, first, out, T)
+    real = (chosen < E).cpu()
+    got_y, got = y[place.long()].double().reshape(T, top, F), out[place.long()].double().reshape(T, top, W)
+    # y: one bfloat16 rounding (2^-9) of a value of order one; out: float sums of the same bfloat16 rows, rows that y's
+    # rounding may send to a neighbour (2^-8 of single elements of a sum of F)
+    assert float((got_y - want_y)[real].abs().max()) < 2 ** -8 * float(want_y.abs().max())
+    assert float((got - want)[real].abs().max()) < 2 ** -7 * float(want.abs().max())
+    assert float((got - want)[real].norm() / want[real].norm()) < 1e-3
+    for t, s in [(0, 0), (T - 1, top - 1)]:
+        if chosen[t, s] < E:                       # the product of the stored rows themselves: float sums only
+            exact = dn[int(chosen[t, s])].double() @ y[place[t * top + s].long()].double()
+            assert float((got[t, s] - exact).abs().max()) < 2e-6 * float(exact.abs().max()) * (F / 1024) ** 0.5 + 1e-5 * float(exact.abs().mean())
+
+
+def test_a_tokens_experts_do_not_depend_on_its_batch():
+    """The same rows alone and among others through the streamed products: the same bits."""
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(3)
+    T, top, E, W, F = 12, 4, 9, 1024, 1152
+    h, gu, dn = bf(rng.standard_normal((T, W))).cuda(), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5).cuda(), bf(rng.standard_normal((E, W, F))).cuda()
+    chosen = drawn(T, top, E, "drawn", 4)
+
+    def run(k):
+        first, order, place = sorted_pairs(chosen[:k].contiguous(), E)
+        y = torch.zeros((k * top, F), dtype=torch.bfloat16, device="cuda")
+        K.experts_up_grouped(h[:k].contiguous(), gu, first, order, y, top)
+        out = torch.zeros((k * top, W), dtype=torch.float32, device="cuda")
+        K.experts_down_grouped(y, dn, first, out, k)
+        return out[place.long()].reshape(k, top, W)
+    whole = run(T)
+    for k in (1, 3, 8, 9):
+        assert torch.equal(run(k), whole[:k])
