@@ -494,11 +494,30 @@ __device__ __forceinline__ void quad_wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N_) : "memory");
 }
 
+// Products of several experts in one launch (GROUPED): expert e's activation rows are the pairs first[e] .. first[e + 1] - 1
+// (rows of A themselves, or with `order` the rows order[p] / top), its weights lie N rows behind the expert before.  With
+// the gated epilogue weight row v of a tile is gate row 8 (v / 16) + v % 16 or, from v % 16 = 8 on, the up row N / 2 behind
+// it, so that the matrices stay as they are stacked; `alpha` > 0: the clamped unit.
+struct QuadGroups {
+    const int* first;
+    const int* order;
+    int experts, top;
+    float limit, alpha;
+};
+__device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr) {
+    if (gr.alpha > 0.f) {
+        g = fminf(g, gr.limit);
+        u = fminf(fmaxf(u, -gr.limit), gr.limit);
+        return g / (1.0f + expf(-gr.alpha * g)) * (u + 1.0f);
+    }
+    return silu_mul(g, u);
+}
+
 // acc[i][j][r]: weight row (output column) n1 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, activation
 // row m1 + 32 j + lane % 32.  Needs ldc % 4 == 0 and C aligned to 16 bytes.
-template <int TI, int TJ, int MODE>
+template <int TI, int TJ, int MODE, bool GROUPED>
 __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __restrict__ C, int M, int N, size_t ldc,
-                                              int m1, int n1, int lane) {
+                                              int m1, int n1, int lane, const QuadGroups& gr) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -515,7 +534,9 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
                     if (n >= N) continue;
                     bf16x4 v;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (bf16)silu_mul(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]);
+                    for (int e = 0; e < 4; ++e)
+                        v[e] = (bf16)(GROUPED ? quad_glu(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e], gr)
+                                              : silu_mul(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]));
                     *(bf16x4*)((bf16*)C + (size_t)m * ldc + (n >> 4) * 8 + (n & 7)) = v;
                 }
                 continue;
@@ -547,11 +568,11 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
     }
 }
 
-template <int BM, int BN, int NSA, int NSB, int WVM, int MODE>
+template <int BM, int BN, int NSA, int NSB, int WVM, int MODE, bool GROUPED = false>
 __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C_, int M, int N, int K, size_t lda,
                                                               size_t ldc, int tiles_m, int tiles_n, int kt_per_part,
-                                                              size_t part_stride, int wl) {
+                                                              size_t part_stride, int wl, QuadGroups gr) {
     constexpr int SA = BM * 128, SB = BN * 128;          // bytes of a stage of activation rows, of weight rows
     constexpr int WVN = 4 / WVM;                         // the four waves: WVM along the activation rows x WVN
     constexpr int TI = BN / WVN / 32, TJ = BM / WVM / 32; // blocks of a wave: weight rows, activation rows
@@ -571,17 +592,56 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     // into a float matrix of its own `part_stride` elements on; runs start at an even k-tile)
     void* C = MODE == OUT_F32 ? (void*)((float*)C_ + blockIdx.y * part_stride) : C_;
     const int kt0 = (int)blockIdx.y * kt_per_part;
-    const int total = tiles_m * tiles_n;
+    int total = tiles_m * tiles_n;
     int pid = blockIdx.x;
+    if constexpr (GROUPED) {                             // the tiles that the experts' pairs make; the grid is a bound
+        int sum = 0;
+        for (int e = threadIdx.x & 63; e < gr.experts; e += 64) sum += (gr.first[e + 1] - gr.first[e] + BM - 1) / BM;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+        total = __builtin_amdgcn_readfirstlane(sum) * tiles_n;
+        if (pid >= total) return;
+    }
     {
         const int per = total / 8, xcd = pid % 8, idx = pid / 8;
         if (pid < per * 8) pid = xcd * per + idx;
     }
-    const int grp = pid / (8 * tiles_m), in = pid - grp * 8 * tiles_m;
-    int gn = tiles_n - grp * 8;
-    if (gn > 8) gn = 8;
-    const int tile_n = grp * 8 + in % gn, tile_m = in / gn;
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    int m0, n0;
+    if constexpr (GROUPED) {                             // expert by expert, an expert's row tiles of the same weights in turn
+        int e = 0, p0 = 0, nt = 0, before = 0;
+        for (int e0 = 0, run = 0; e0 < gr.experts; e0 += 64) {
+            const int l = e0 + (threadIdx.x & 63);
+            const int a = l < gr.experts ? gr.first[l] : 0, b = l < gr.experts ? gr.first[l + 1] : 0;
+            const int mine = (b - a + BM - 1) / BM * tiles_n;
+            int sum = mine;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(sum, o, 64);
+                if ((int)(threadIdx.x & 63) >= o) sum += v;
+            }
+            const unsigned long long here = __ballot(run + sum > pid && run + sum - mine <= pid);
+            if (here) {
+                const int at = __ffsll(here) - 1;
+                e = e0 + at;
+                p0 = __builtin_amdgcn_readlane(a, at);
+                M = __builtin_amdgcn_readlane(b, at);
+                nt = __builtin_amdgcn_readlane(mine, at) / tiles_n;
+                before = run + __builtin_amdgcn_readlane(sum - mine, at);
+                break;
+            }
+            run += __builtin_amdgcn_readlane(sum, 63);
+        }
+        const int in = pid - before;
+        m0 = p0 + in % nt * BM;
+        n0 = in / nt * BN;
+        W += (size_t)e * N * K;
+    } else {
+        const int grp = pid / (8 * tiles_m), in = pid - grp * 8 * tiles_m;
+        int gn = tiles_n - grp * 8;
+        if (gn > 8) gn = 8;
+        const int tile_n = grp * 8 + in % gn, tile_m = in / gn;
+        m0 = tile_m * BM, n0 = tile_n * BN;
+    }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = (wave / WVN) * (BM / WVM), wn = (wave % WVN) * (BN / WVN);
     const int lrow = lane & 31, g = lane >> 5;
@@ -604,11 +664,15 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         if (q < LA) {
             int r = m0 + R;
             if (r > M - 1) r = M - 1;
+            if constexpr (GROUPED) {
+                if (gr.order) r = gr.order[r] / gr.top;
+            }
             offA[q] = (unsigned)((size_t)r * lda * 2 + c * 16);
         }
         if (q < LB) {
             int r = n0 + R;
             if (r > N - 1) r = N - 1;
+            if constexpr (GROUPED && MODE == OUT_SWIGLU) r = (r >> 4) * 8 + (r & 7) + ((r & 8) ? N / 2 : 0);
             offB[q] = (unsigned)(w_row_base(r, K, wl) * 2 + c * 16);
         }
     }
@@ -746,7 +810,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     // accumulator stay behind the statement that names it
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     static_for<0, NM>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
-    quad_epilogue<TI, TJ, MODE>(acc, C, M, N, ldc, m0 + wm, n0 + wn, lane);
+    quad_epilogue<TI, TJ, MODE, GROUPED>(acc, C, M, N, ldc, m0 + wm, n0 + wn, lane, gr);
 }
 
 static int launch_split_sum(const float* scratch, int parts, void* C, int M, int N, size_t ldc, int mode, hipStream_t s);
@@ -784,19 +848,19 @@ static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N,
         parts = (nk + kpp - 1) / kpp;                                 // no empty run
         dim3 grid((unsigned)total, (unsigned)parts);
         gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<grid, 256, 0, s>>>(A, W, scratch, M, N, K, lda, (size_t)N, tm, tn, kpp,
-                                                                        (size_t)M * N, wl);
+                                                                        (size_t)M * N, wl, QuadGroups{});
         int rc = br_check_launch();
         if (rc != BR_OK) return rc;
         return launch_split_sum(scratch, parts, C, M, N, ldc, mode, s);
     }
     if (mode == OUT_BF16)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_BF16><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl);
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_BF16><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
     else if (mode == OUT_F32)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl);
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
     else if (mode == OUT_F32_ACC)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32_ACC><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl);
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32_ACC><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
     else
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_SWIGLU><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl);
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_SWIGLU><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
     return br_check_launch();
 }
 
@@ -2115,4 +2179,61 @@ extern "C" int br_gemm_bf16_wide_parts(int M, int N, int K, int mode, size_t scr
 }
 
 // rows of a block of the blocked weight layout (the host lays weights out by it)
+// ------------------------------------------- routed experts by the quad tiles -----
+// Steps whose (token, slot) pairs are grouped by expert: C[p, :] = W[e] A[p, :] for every expert's pairs, all
+// experts in one launch of gemm_tile_quad_kernel (GROUPED).  `gated`: W is [E][2 F][K], C bfloat16 [pairs, F] (N = 2 F), the
+// rows of A taken through `order`; else W is [E][N][K] and C float32 or bfloat16 [pairs, N].
+extern "C" int br_experts_tiles_takes(int N, int K) { return N > 0 && K > 0 && N % 16 == 0 && K % DMA_BK == 0; }
+
+template <int BM, int BN, int NSA, int NSB, int WVM>
+static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode, int pairs, int N, int K, size_t ldc, const QuadGroups& gr,
+                                hipStream_t s) {
+    // no more tiles than the pairs make when every expert's last one is nearly empty
+    const int tn = (N + BN - 1) / BN, nk = K / DMA_BK;
+    const long long tm = (long long)pairs / BM + (gr.experts < pairs ? gr.experts : pairs);
+    if (tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
+    const unsigned grid = (unsigned)(tm * tn);
+#define BR_EXPERTS(MODE_) \
+    gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, MODE_, true><<<grid, 256, 0, s>>>(A, W, C, 0, N, K, (size_t)K, ldc, 0, tn, nk, 0, WL_ROWS, gr)
+    if (mode == OUT_SWIGLU) BR_EXPERTS(OUT_SWIGLU);
+    else if (mode == OUT_F32) BR_EXPERTS(OUT_F32);
+    else BR_EXPERTS(OUT_BF16);
+#undef BR_EXPERTS
+    return br_check_launch();
+}
+
+// 128x256 or 256x256 tiles: the fewer rounds of workgroups by the times a k-tile of `choose_quad`, with every expert's pairs
+// taken as the mean and half a standard deviation of evenly drawn ones, rounded up to tiles (their real numbers stay on the
+// device).  32 experts of 1,792 by 4,096, 8 chosen, gated product / down in us with 128 rows a tile against 256: 200 tokens
+// 179 / 102 against 228 / 112, 800 tokens 295 / 162 against 255 / 135, 1,200 tokens 417 / 213 against 432 / 217, 1,800 tokens
+// 500 / 279 against 445 / 231 (1.19 and 0.91 PFLOP/s), 8,000 tokens 1,892 / 1,208 against 1,626 / 955.  Before, the rows
+// copied into the experts' order, tiles of 128x128 through registers and the unit in a launch of its own: 234 / 122, 522 /
+// 267, 782 / 387, 1,074 / 543 and 4,267 / 1,983.
+static bool experts_tall_tiles(int pairs, int E, int N, int cus) {
+    const double mean = (double)pairs / E, high = mean + 0.5 * sqrt(mean);
+    double t[2];
+    for (int i = 0; i < 2; ++i) {
+        const int bm = i ? 256 : 128, k = i ? 0 : 1;
+        const double units = E * ceil(high / bm) * ((N + 255) / 256), whole = floor(units / cus), share = units / cus - whole;
+        t[i] = whole * QUAD_FULL[k] + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) * QUAD_FULL[k] : 0.0);
+    }
+    return t[1] <= 1.03 * t[0];
+}
+
+extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, const int* order, void* C, int gated, int out_is_bf16,
+                                int a_rows, int pairs, int E, int N, int K, int top, float limit, float alpha, hipStream_t s) {
+    if (pairs <= 0) return BR_OK;
+    const size_t ldc = gated ? (size_t)N / 2 : (size_t)N;
+    if (!br_experts_tiles_takes(N, K) || E <= 0 || top <= 0 || (gated && !out_is_bf16) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 != 0 ||
+        !quad_takes(C, a_rows, N, K, K, ldc))
+        return BR_BAD_ARG;
+    const QuadGroups gr = {first, order, E, top, limit, alpha};
+    const int mode = gated ? OUT_SWIGLU : out_is_bf16 ? OUT_BF16 : OUT_F32;
+    const int cus = br_device_cus();
+    if (!cus) return BR_LAUNCH_FAILED;
+    if (experts_tall_tiles(pairs, E, N, cus))
+        return launch_experts_tiles<256, 256, 2, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
+    return launch_experts_tiles<128, 256, 3, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
+}
+
 extern "C" int br_gemm_bf16_block_rows() { return WL_BLOCK_ROWS; }

@@ -1398,6 +1398,32 @@ def experts_down_grouped(y: torch.Tensor, w_down: torch.Tensor, first: torch.Ten
     _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), n, E, W, F, int(n_tokens), _stream()), "experts_down_grouped")
 
 
+def experts_stream_takes(dtype: torch.dtype, W: int, F: int, pairs: int, experts: int) -> bool:
+    """Whether `experts_up_grouped` and `experts_down_grouped` stream these experts' weights for that many pairs."""
+    return (dtype == torch.bfloat16 and min(W, F) >= 1024 and W % 128 == 0 and F % 128 == 0 and pairs <= min(1024, 8 * experts)
+            and experts <= 512)
+
+
+def experts_tiles_take(dtype: torch.dtype, W: int, F: int) -> bool:
+    """Whether the prompt products' tiles take these experts (bfloat16, both widths in steps of 64)."""
+    return dtype == torch.bfloat16 and W % 64 == 0 and F % 64 == 0
+
+
+def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, order: torch.Tensor, y: torch.Tensor, top: int,
+                     limit: float = 0.0, alpha: float = 0.0) -> None:
+    """`experts_up_grouped` by the tiles of the prompt products, for steps of more tokens."""
+    _dev("experts_up_tiles", h, w_gu, first, order, y)
+    T, W = h.shape
+    E, F2, _ = w_gu.shape
+    n = order.numel()
+    _req(experts_tiles_take(h.dtype, W, F2 // 2) and w_gu.dtype == y.dtype == torch.bfloat16, "experts_up_tiles: bfloat16, widths in steps of 64")
+    _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
+         and first.dtype == order.dtype == torch.int32, "experts_up_tiles: shapes")
+    f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
+    _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), 1, 1, T, n, E, F2, W, top, float(limit), float(alpha), _stream()),
+           "experts_up_tiles")
+
+
 def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: torch.Tensor) -> None:
     """out[p] = w[e] a[p] for the pairs p of every expert e in the experts' order (`experts_sort`): a [pairs, K] bfloat16
     rows in that order, w [E, N, K] bfloat16, out [pairs, N] bfloat16 or float32; one launch for all experts."""
@@ -1406,6 +1432,11 @@ def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: tor
     E, N, _ = w.shape
     _req(a.dtype == w.dtype == torch.bfloat16 and Kd % 8 == 0 and w.shape == (E, N, Kd) and out.shape == (n, N)
          and first.dtype == torch.int32 and first.numel() in (E + 1, E + 2), "experts_gemm: bfloat16 [pairs, K] x [E, N, K], K in steps of 8")
+    if Kd % 64 == 0 and N % 16 == 0:
+        f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
+        _check(f(_ptr(a), _ptr(w), _ptr(first), None, _ptr(out), 0, _is_bf16(out, "experts_gemm"), n, n, E, N, Kd, 1, 0.0, 0.0, _stream()),
+               "experts_gemm")
+        return
     f = _fn("routed_experts", "br_experts_gemm", [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P])
     _check(f(_ptr(a), _ptr(w), _ptr(first), _ptr(out), _is_bf16(out, "experts_gemm"), n, E, N, Kd, _stream()), "experts_gemm")
 

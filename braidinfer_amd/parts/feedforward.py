@@ -280,32 +280,38 @@ class RoutedExperts(FeedForward):
         order = step.ws.get("moe_order", (n,), torch.int32)
         place = step.ws.get("moe_place", (n,), torch.int32)
         K.experts_sort(chosen, first, order, place, bins)
-        if few:
-            # few tokens: an expert's weights are read once for all its pairs, nothing goes back to the host
+        forced = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "") == "1"          # for measurements
+        # Up to eight pairs an expert on average, or sixteen tokens, the weights are streamed once for up to 16 pairs at a time;
+        # beyond, the prompt products' tiles read them once for 128 or 256 (32 experts of 1,792 by 4,096, 8 chosen, both
+        # products: 32 tokens 239 against 257 us, 40 tokens 257 against 256, 64 tokens 350 against 259).
+        streamed = (T <= 16 or n <= 8 * self.E) and (few or K.experts_stream_takes(dt, self.H, self.I, n, self.E))
+        if K.experts_tiles_take(dt, self.H, self.I) and not streamed and not forced:
+            y = step.ws.get("moe_y", (n, self.I), dt)
+            K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
+            out = step.ws.get("moe_out", (n, self.H), torch.float32)
+            K.experts_gemm(y, self.w_down, first, out)
+            K.experts_combine(out, place, share, x, store=store, **ident)
+            return
+        if few or (streamed and not forced):
+            # an expert's weights are read once for its pairs, nothing goes back to the host
             y = step.ws.get("moe_y", (n, self.I), dt)
             K.experts_up_grouped(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             out = step.ws.get("moe_out", (n, self.H), torch.float32)
             K.experts_down_grouped(y, self.w_down, first, out, T)
             K.experts_combine(out, place, share, x, store=store, **ident)
             return
+        # widths that the tiles do not take, and the 32-bit path
         rows = step.ws.get("moe_rows", (n, self.H), dt)
         K.experts_gather(h, order, rows, self.top, n_rows=first[self.E:self.E + 1] if self.identity else None)
         gu = step.ws.get("moe_gu", (n, 2 * self.I), dt)
         act = step.ws.get("moe_act", (n, self.I), dt)
         out = step.ws.get("moe_out", (n, self.H), torch.float32)
-        # Tiles of 128 pairs of one expert, all experts in one launch a product; from about 1,500 pairs an expert the
-        # library's own products, expert by expert, make up for their launches (8 layers of width 4,096, 32 experts,
-        # 8 chosen: 8,192 tokens 56.9 against 78.7 ms, 2,048 tokens 23.1 against 19.4; BRAIDINFER_EXPERTS_ONE_BY_ONE=0
-        # or =1 forces one, for measurements)
-        forced = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "")
-        one_by_one = forced == "1" or (forced != "0" and n // self.E >= self.ONE_BY_ONE_FROM)
-        if K.experts_grouped_takes(dt, self.H, self.I) and not one_by_one:
+        if K.experts_grouped_takes(dt, self.H, self.I) and not forced and n // self.E < self.ONE_BY_ONE_FROM:
             K.experts_gemm(rows, self.w_gu, first, gu)
             self._glu(gu, act)
             K.experts_gemm(act, self.w_down, first, out)
         else:
-            # the 32-bit path and other widths: expert by expert through the library's products, the experts' row
-            # counts read by the host
+            # expert by expert through the library's products, the experts' row counts read by the host
             starts = first.tolist()
             scratch = step.ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32) if dt == torch.bfloat16 else None
             for e in range(self.E):

@@ -70,7 +70,7 @@ def test_products_of_few_tokens(T, top, E, W, F, how, identity, alpha):
     K.experts_up_grouped(hd, gu, first, order, y, top, 0.9 if alpha else 0.0, alpha)
     out = torch.full((n, W), 7.0, dtype=torch.float32, device="cuda")
     K.experts_down_grouped(y, dn, first, out, T)
-    real = (chosen < E).cpu()
+    real = chosen < E
     got_y, got = y[place.long()].double().reshape(T, top, F), out[place.long()].double().reshape(T, top, W)
     # y: one bfloat16 rounding (2^-9) of a value of order one; out: float sums of the same bfloat16 rows, rows that y's
     # rounding may send to a neighbour (2^-8 of single elements of a sum of F)
@@ -101,3 +101,31 @@ def test_a_tokens_experts_do_not_depend_on_its_batch():
     whole = run(T)
     for k in (1, 3, 8, 9):
         assert torch.equal(run(k), whole[:k])
+
+
+# pairs an expert at 0, 1, below, at and beyond a tile's 128 and 256 rows; widths with an odd number of 64-wide steps and of 256
+# output columns cut short; more than 64 experts; identities behind them
+@pytest.mark.parametrize("T,top,E,W,F,how,identity,alpha", [
+    (1, 1, 3, 64, 64, "drawn", 0, 0.0), (65, 2, 2, 192, 320, "one", 0, 0.0), (128, 1, 3, 64, 128, "one", 0, 1.702),
+    (129, 3, 4, 320, 64, "one", 0, 0.0), (257, 2, 5, 256, 192, "one", 1, 0.0), (300, 4, 90, 128, 192, "drawn", 3, 0.0),
+    (520, 2, 3, 448, 320, "drawn", 0, 0.0), (900, 8, 16, 1024, 704, "drawn", 0, 1.702)])
+def test_products_of_many_tokens(T, top, E, W, F, how, identity, alpha):
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(T + W + F)
+    h, w_gu, w_down = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5), bf(rng.standard_normal((E, W, F)) / F ** 0.5)
+    chosen = drawn(T, top, E + identity, how, T)
+    want_y, want = products(h, w_gu, w_down, chosen, 0.9, alpha)
+    first, order, place = sorted_pairs(chosen, E + (1 if identity else 0))
+    n = T * top
+    y = torch.full((n, F), 7.0, dtype=torch.bfloat16, device="cuda")
+    K.experts_up_tiles(h.cuda(), w_gu.cuda(), first, order, y, top, 0.9 if alpha else 0.0, alpha)
+    for dtype, rounding in ((torch.float32, 0.0), (torch.bfloat16, 2 ** -9)):
+        out = torch.full((n, W), 7.0, dtype=dtype, device="cuda")
+        K.experts_gemm(y, w_down.cuda(), first, out)
+        real = chosen < E
+        got_y, got = y[place.long()].double().reshape(T, top, F), out[place.long()].double().reshape(T, top, W)
+        assert float((got_y - want_y)[real].abs().max()) < 2 ** -8 * float(want_y.abs().max())
+        assert float((got - want)[real].abs().max()) < (2 ** -7 + rounding) * float(want.abs().max())
+        assert float((got - want)[real].norm() / want[real].norm()) < 1e-3 + rounding
+        if identity:                               # rows behind the experts' pairs are nobody's
+            assert torch.all(out[int(first[E]):] == 7.0)
