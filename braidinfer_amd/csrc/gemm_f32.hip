@@ -1,27 +1,32 @@
-// True 32-bit matrix product: C[M,N] (+)= A[M,K] * W[N,K]^T with float FMA only (no
-// matrix-core reduced-precision mode).  Every output element is accumulated over k in
-// ascending order by one thread, so its value does not depend on M, on the tile it
-// falls in, or on the other rows of the batch.
+// True 32-bit matrix product: C[M,N] (+)= A[M,K] * W[N,K]^T in float, every product and sum in 32 bits (on the vector units, or
+// on the matrix cores' float instruction, which rounds nothing to fewer bits).
 //
-// reference: op_linear_proj, kernels/megakernel_ops.hip:166-276 (one block per output
-// row, f32 accumulate); the LDS-tiled 64x64x16 form here is the CDNA layout of the
-// same sum.
+// The order of an output element's sum depends on K alone, never on M, on the tile it falls in, on which kernel computed it
+// or on the other rows of the batch, so that whole prompts and token-by-token runs agree bit for bit:
+//  * K in steps of 64 (aligned weights): k is cut into 8 segments of whole 64s (segment s: 64s number s n / 8 .. (s + 1) n / 8
+//    of the n there are).  Within a segment, 16 k at a time, four v_mfma_f32_16x16x4_f32 of which number i takes k + i, k + 4 +
+//    i, k + 8 + i and k + 12 + i (a lane's 16 bytes are four instructions' operands); the segments are added in order.  The
+//    streaming kernel gives each of its 8 waves a segment; the tiles sum segment by segment, or every segment in a workgroup
+//    of its own with the segments added by a second launch.
+//  * any other K: ascending k by one thread, the 64x64x16 LDS-tiled form below.
+//
+// reference: op_linear_proj, kernels/megakernel_ops.hip:166-276 (one block per output row, f32 accumulate).
 #include "common.h"
 
-#define BM 64
-#define BN 64
-#define BK 16
+#define F32_BM 64
+#define F32_BN 64
+#define F32_BK 16
 
 // mode 0: C = AW^T ; mode 1: C += AW^T (C holds the residual stream)
 template <int MODE>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                        float* __restrict__ C, int M, int N, int K,
                                                        size_t lda, size_t ldc) {
-    __shared__ float As[BK][BM + 4];
-    __shared__ float Ws[BK][BN + 4];
+    __shared__ float As[F32_BK][F32_BM + 4];
+    __shared__ float Ws[F32_BK][F32_BN + 4];
     const int tid = threadIdx.x;
     const int tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int m0 = blockIdx.y * F32_BM, n0 = blockIdx.x * F32_BN;
     const int lr = tid >> 2, lk = (tid & 3) * 4;  // loader: row lr, k offset lk..lk+3
     float acc[4][4];
 #pragma unroll
@@ -29,7 +34,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
 
-    for (int k0 = 0; k0 < K; k0 += BK) {
+    for (int k0 = 0; k0 < K; k0 += F32_BK) {
         {
             const int m = m0 + lr, n = n0 + lr;
 #pragma unroll
@@ -41,7 +46,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < BK; ++k) {
+        for (int k = 0; k < F32_BK; ++k) {
             float a[4], w[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
@@ -68,11 +73,298 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
     }
 }
 
-extern "C" int br_gemm_f32(const float* A, const float* W, float* C, int M, int N, int K,
-                           size_t lda, size_t ldc, int accumulate, hipStream_t s) {
+// ------------------------------------------------------------ K in steps of 64 -----
+#define F32_SEGS 8
+#define F32_KC 64            // k that segments are whole multiples of
+
+__device__ __forceinline__ void f32_dma16(unsigned lds, const void* p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
+}
+__device__ __forceinline__ void f32_dma16_nt(unsigned lds, const void* p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(p) : "m0", "memory");
+}
+__device__ __forceinline__ void f32_dma4(unsigned lds, const void* p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
+}
+// 1 KB of LDS from rows of `ROWB` bytes, 16 bytes a lane, the 16-byte columns of a row exchanged by `SW(row)`: `src(row, col)`
+// gives the address of the row's 16-byte column.  Rows that do not lie at multiples of 16 bytes come 4 bytes a lane.
+template <int ROWB, class Src, class Sw>
+__device__ __forceinline__ void f32_bring(unsigned lds, int row0, int lane, bool aligned, bool nt, Src src, Sw sw) {
+    constexpr int CPL = ROWB / 16;
+    if (aligned) {
+        const int row = row0 + lane / CPL, col = (lane % CPL) ^ sw(row);
+        if (nt) f32_dma16_nt(lds, src(row, col));
+        else f32_dma16(lds, src(row, col));
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int at = q * 16 + (lane >> 2), row = row0 + at / CPL, col = (at % CPL) ^ sw(row);
+        f32_dma4(lds + q * 256, (const float*)src(row, col) + (lane & 3));
+    }
+}
+
+// M <= 16, K from 512: bound by reading the weights.  One workgroup a compute unit walks over tiles of 16 weight rows, tile t
+// of workgroup b being b + t * grid; each wave walks its segment of k in chunks of 64 through an LDS ring of its own (direct
+// loads of 256-byte row pieces, the weights non-temporal, the next chunk on its way across tile ends), the waves' sums meet
+// in LDS at a tile's end.  28,672 x 4,096 (470 MB) at 1 / 4 / 16 rows: 69 / 76 / 104 us (6.9 / 6.2 / 4.5 TB/s), 4,096 x 14,336:
+// 37 / 37 / 43, where the 64x64 tiles of one thread a sum took 549 / 552 / 580 and 1,435 / 1,479 / 1,534.
+template <int XR, int MODE>
+__global__ __launch_bounds__(512) void gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                              float* __restrict__ C, int M, int N, int K, size_t lda, size_t ldc,
+                                                              int ntiles, int a_aligned) {
+    constexpr int NW = F32_SEGS, ROWB = F32_KC * 4, STAGE = (16 + XR) * ROWB, S = 2;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    float* red = (float*)(smem + NW * S * STAGE);             // [2][NW][16][17]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    unsigned char* ring = smem + wave * (S * STAGE);
+    const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)ring);
+    const int nch = K / F32_KC, c0 = wave * nch / NW, ncw = (wave + 1) * nch / NW - c0;
+    const int my_tiles = (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, nitems = my_tiles * ncw;
+    int is_t = 0, is_c = 0, cp_t = 0, cp_c = 0, buf = 0;
+    auto issue = [&](int slot) {
+        const int n0 = ((int)blockIdx.x + is_t * (int)gridDim.x) * 16, k0 = (c0 + is_c) * F32_KC;
+        const unsigned lds = __builtin_amdgcn_readfirstlane(ring_lds + slot * STAGE);
+        auto sw = [](int row) { return row & 7; };
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            f32_bring<ROWB>(lds + q * 1024, 4 * q, lane, true, true, [&](int row, int col) { return W + (size_t)min(n0 + row, N - 1) * K + k0 + col * 4; }, sw);
+#pragma unroll
+        for (int q = 0; q < XR / 4; ++q)
+            f32_bring<ROWB>(lds + (4 + q) * 1024, 4 * q, lane, a_aligned, false, [&](int row, int col) { return A + (size_t)min(row, M - 1) * lda + k0 + col * 4; }, sw);
+        if (++is_c == ncw) { is_c = 0; ++is_t; }
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (nitems > 0) issue(0);
+    for (int it = 0; it < nitems; ++it) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (it + 1 < nitems) issue((it + 1) & 1);
+        const unsigned char* st = ring + (it & 1) * STAGE;
+        const int xr = XR == 8 ? (r16 & 7) : r16;
+        f32x4 wf[4], xv[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            wf[b] = *(const f32x4*)(st + r16 * ROWB + (((4 * b + g) ^ (r16 & 7)) * 16));
+            xv[b] = *(const f32x4*)(st + (16 + xr) * ROWB + (((4 * b + g) ^ (xr & 7)) * 16));
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][i], xv[b][i], acc, 0, 0, 0);
+        if (++cp_c < ncw) continue;
+        cp_c = 0;
+        const int n0 = ((int)blockIdx.x + cp_t * (int)gridDim.x) * 16;
+        ++cp_t;
+        float* rb = red + buf * (NW * 16 * 17);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rb[(wave * 16 + 4 * g + r) * 17 + r16] = acc[r];
+        acc = {0.f, 0.f, 0.f, 0.f};
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int m = tid >> 4, nl = tid & 15, n = n0 + nl;
+        if (m < M && n < N) {
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v += rb[(w * 16 + nl) * 17 + m];
+            float* c = C + (size_t)m * ldc + n;
+            *c = MODE == 1 ? *c + v : v;
+        }
+        buf ^= 1;
+    }
+}
+
+// Any M: 16 TJ rows x 128 columns by four waves along the columns (16 TJ x 32 each), two LDS stages of 32 k by direct loads,
+// bound by the matrix cores: 28,672 x 4,096 at 64 / 279 / 2,048 rows 188 / 634 / 3,573 us (80 / 103 / 135 TFLOP/s; the 64x64
+// tiles of one thread a sum 678 / 2,442 / 12,669), 4,096 x 14,336 at 279 rows 281 (2,078; segments apart).  Error against 64
+// bits at 64 rows of 4,096: 4.1e-7 of the norm, 1.1e-6 with one ascending sum.
+// TJ is chosen so that the rows fill their tiles (279 rows: three of 96).  SPLIT: segment
+// blockIdx.y alone, into a matrix of its own.  The accumulators hold the product transposed: four columns of a row a lane.
+template <int TJ, int MODE, bool SPLIT>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                            float* __restrict__ C, int M, int N, int K, size_t lda, size_t ldc,
+                                                            int tiles_m, int a_aligned, int c_aligned) {
+    constexpr int BM = 16 * TJ, BN = 128, ROWB = 128, TI = 2, STAGE = (BM + BN) * ROWB;
+    __shared__ __attribute__((aligned(1024))) unsigned char st[2 * STAGE];
+    int pid = blockIdx.x;
+    {
+        const int total = gridDim.x, per = total / 8, xcd = pid % 8, idx = pid / 8;
+        if (pid < per * 8) pid = xcd * per + idx;
+    }
+    const int m0 = pid % tiles_m * BM, n0 = pid / tiles_m * BN;      // the row tiles of the same weights in turn
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)st);
+    const int nch = K / F32_KC;
+    const int s0 = SPLIT ? (int)blockIdx.y : 0, s1 = SPLIT ? s0 + 1 : F32_SEGS;
+    const int kt0 = s0 * nch / F32_SEGS * 2, kt1 = s1 * nch / F32_SEGS * 2;      // stages of 32 k
+    auto sw = [](int row) { return (row >> 1) & 7; };
+    auto issue = [&](int kt) {
+        const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + (kt & 1) * STAGE);
+        const int k0 = kt * 32;
+#pragma unroll
+        for (int q = 0; q < BM / 8; q += 4)
+            if (q + wave < BM / 8)
+                f32_bring<ROWB>(base + (q + wave) * 1024, (q + wave) * 8, lane, a_aligned, false,
+                                [&](int row, int col) { return A + (size_t)min(m0 + row, M - 1) * lda + k0 + col * 4; }, sw);
+#pragma unroll
+        for (int q = 0; q < BN / 8; q += 4)
+            f32_bring<ROWB>(base + BM * ROWB + (q + wave) * 1024, (q + wave) * 8, lane, true, false,
+                            [&](int row, int col) { return W + (size_t)min(n0 + row, N - 1) * K + k0 + col * 4; }, sw);
+    };
+    f32x4 acc[TI][TJ], sum[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { acc[i][j][r] = 0.f; sum[i][j][r] = 0.f; }
+    if (kt0 < kt1) issue(kt0);
+    int seg = s0, seg_end = (s0 + 1) * nch / F32_SEGS * 2;
+    for (int kt = kt0; kt < kt1; ++kt) {
+        while (kt == seg_end) {                               // a segment is whole: onto the sum, in order
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) { sum[i][j][r] += acc[i][j][r]; acc[i][j][r] = 0.f; }
+            ++seg;
+            seg_end = (seg + 1) * nch / F32_SEGS * 2;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (kt + 1 < kt1) issue(kt + 1);
+        const unsigned char* ap = st + (kt & 1) * STAGE;
+        const unsigned char* wp = ap + (BM + wave * 32) * ROWB;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            f32x4 af[TJ], wf[TI];
+#pragma unroll
+            for (int i = 0; i < TI; ++i) wf[i] = *(const f32x4*)(wp + (16 * i + r16) * ROWB + (((4 * b + g) ^ sw(r16)) * 16));
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) af[j] = *(const f32x4*)(ap + (16 * j + r16) * ROWB + (((4 * b + g) ^ sw(r16)) * 16));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TI; ++i)
+#pragma unroll
+                    for (int j = 0; j < TJ; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
+        }
+        // every wave has read this stage before the loop's next barrier lets the loads of the one after into it
+    }
+    if (SPLIT) C += (size_t)blockIdx.y * M * N;
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+        const int m = m0 + 16 * j + r16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+            const int n = n0 + wave * 32 + 16 * i + 4 * g;
+            float* c = C + (size_t)m * ldc + n;
+            f32x4 v = sum[i][j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += acc[i][j][r];
+            if (c_aligned && n + 3 < N) {
+                if (MODE == 1) {
+                    const f32x4 o = *(const f32x4*)c;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = o[r] + v[r];
+                }
+                *(f32x4*)c = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N) c[r] = MODE == 1 ? c[r] + v[r] : v[r];
+            }
+        }
+    }
+}
+
+// C (+)= the segments' matrices [F32_SEGS][M][N], added in order; a thread an element.
+template <int MODE>
+__global__ __launch_bounds__(256) void gemm_f32_segments_kernel(const float* __restrict__ part, float* __restrict__ C, int M, int N,
+                                                                size_t ldc) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, all = (size_t)M * N;
+    if (i >= all) return;
+    float v = 0.f;
+#pragma unroll
+    for (int s = 0; s < F32_SEGS; ++s) v += part[s * all + i];
+    float* c = C + i / N * ldc + i % N;
+    *c = MODE == 1 ? *c + v : v;
+}
+
+template <int XR>
+static int launch_f32_stream(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int acc, int aligned,
+                             int cus, hipStream_t s) {
+    constexpr size_t lds = (size_t)F32_SEGS * 2 * (16 + XR) * F32_KC * 4 + 2 * F32_SEGS * 16 * 17 * 4;
+    const int ntiles = (N + 15) / 16, grid = ntiles < cus ? ntiles : cus;
+#define BR_F32_STREAM(MODE_)                                                                                                     \
+    do {                                                                                                                         \
+        auto kern = gemm_f32_stream_kernel<XR, MODE_>;                                                                           \
+        static bool set = false;                                                                                                 \
+        if (!set) {                                                                                                              \
+            if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)      \
+                return BR_LAUNCH_FAILED;                                                                                         \
+            set = true;                                                                                                          \
+        }                                                                                                                        \
+        kern<<<grid, 512, lds, s>>>(A, W, C, M, N, K, lda, ldc, ntiles, aligned);                                                \
+    } while (0)
+    if (acc) BR_F32_STREAM(1); else BR_F32_STREAM(0);
+#undef BR_F32_STREAM
+    return br_check_launch();
+}
+
+template <int TJ>
+static int launch_f32_tile(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int acc, int aligned,
+                           int cus, float* scratch, size_t scratch_floats, hipStream_t s) {
+    const int tm = (M + 16 * TJ - 1) / (16 * TJ), tn = (N + 127) / 128;
+    const long long tiles = (long long)tm * tn;
+    if (tiles > 0x7fffffffLL) return BR_BAD_ARG;
+    const int c_aligned = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+    // fewer tiles than two a compute unit: every segment in a workgroup of its own
+    if (tiles < 2 * cus && K >= 512 && (size_t)F32_SEGS * M * N <= scratch_floats) {
+        const dim3 grid((unsigned)tiles, F32_SEGS);
+        gemm_f32_tile_kernel<TJ, 0, true><<<grid, 256, 0, s>>>(A, W, scratch, M, N, K, lda, (size_t)N, tm, aligned, N % 4 == 0 && (uintptr_t)scratch % 16 == 0);
+        const unsigned blocks = (unsigned)(((size_t)M * N + 255) / 256);
+        if (acc) gemm_f32_segments_kernel<1><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+        else gemm_f32_segments_kernel<0><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+        return br_check_launch();
+    }
+    if (acc) gemm_f32_tile_kernel<TJ, 1, false><<<(unsigned)tiles, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
+    else gemm_f32_tile_kernel<TJ, 0, false><<<(unsigned)tiles, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
+    return br_check_launch();
+}
+
+// `scratch`: room for the segments' sums of products with few tiles (null: none).
+extern "C" int br_gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int accumulate,
+                           float* scratch, size_t scratch_floats, hipStream_t s) {
     if (M <= 0 || N <= 0) return BR_OK;
     if (K <= 0 || lda < (size_t)K || ldc < (size_t)N) return BR_BAD_ARG;
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    if (K % F32_KC == 0 && (uintptr_t)W % 16 == 0) {
+        const int cus = br_device_cus();
+        if (!cus) return BR_LAUNCH_FAILED;
+        const int aligned = lda % 4 == 0 && (uintptr_t)A % 16 == 0;
+        if (M <= 8 && K >= F32_KC * F32_SEGS) return launch_f32_stream<8>(A, W, C, M, N, K, lda, ldc, accumulate, aligned, cus, s);
+        if (M <= 16 && K >= F32_KC * F32_SEGS) return launch_f32_stream<16>(A, W, C, M, N, K, lda, ldc, accumulate, aligned, cus, s);
+        const int rows = (M + (M + 127) / 128 - 1) / ((M + 127) / 128);         // of a tile, before rounding up to 16
+#define BR_F32_TILE(TJ_) launch_f32_tile<TJ_>(A, W, C, M, N, K, lda, ldc, accumulate, aligned, cus, scratch, scratch ? scratch_floats : 0, s)
+        switch ((rows + 15) / 16) {
+            case 1: return BR_F32_TILE(1);
+            case 2: return BR_F32_TILE(2);
+            case 3: return BR_F32_TILE(3);
+            case 4: return BR_F32_TILE(4);
+            case 5: return BR_F32_TILE(5);
+            case 6: return BR_F32_TILE(6);
+            case 7: return BR_F32_TILE(7);
+            default: return BR_F32_TILE(8);
+        }
+#undef BR_F32_TILE
+    }
+    dim3 grid((N + F32_BN - 1) / F32_BN, (M + F32_BM - 1) / F32_BM);
     if (grid.y > 65535) return BR_BAD_ARG;
     if (accumulate) gemm_f32_kernel<1><<<grid, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc);
     else gemm_f32_kernel<0><<<grid, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc);

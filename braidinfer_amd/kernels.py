@@ -412,8 +412,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     LDS, M <= 64; 10: a 256x192 tile loaded straight into LDS; 12 to 15: 256x256, 128x256, 256x192 and
     256x224 tiles of four waves, one to a SIMD, K in steps of 64 and output rows in steps of 16 bytes, plus
     16 p for p runs along k); 0 chooses by shape.  A weight from `block_weight` is taken by kernels 4 to 15.
-    `scratch` (float32, on the device): with it, a bf16 product of more than 16 rows with too
-    few tiles to fill the chip is cut along k into runs that a second kernel sums in a fixed order.
+    `scratch` (float32, on the device): with it, a product of more than 16 rows with too
+    few tiles to fill the chip is cut along k into runs that a second kernel sums in a fixed order
+    (float32: the same bits with and without).
     """
     name = "gemm"
     for t in (a, w, out):
@@ -427,8 +428,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     lda, ldc = (a.stride(0) if M > 1 else K), (out.stride(0) if M > 1 else N)
     if a.dtype == torch.float32 and w.dtype == torch.float32:
         _req(out.dtype == torch.float32, "gemm: float32 inputs give a float32 output")
-        f = _fn("gemm_f32", "br_gemm_f32", [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, _P])
-        _check(f(_ptr(a), _ptr(w), _ptr(out), M, N, K, lda, ldc, int(accumulate), _stream()), name)
+        if scratch is not None:
+            _req(scratch.is_cuda and scratch.dtype == torch.float32 and scratch.is_contiguous(), "gemm: scratch must be float32 on the device")
+        f = _fn("gemm_f32", "br_gemm_f32", [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, _P, c_size_t, _P])
+        _check(f(_ptr(a), _ptr(w), _ptr(out), M, N, K, lda, ldc, int(accumulate), _ptr(scratch), 0 if scratch is None else scratch.numel(),
+                 _stream()), name)
     elif a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
         if out.dtype == torch.bfloat16:
             _req(not accumulate, "gemm: accumulation needs a float32 output")
