@@ -888,6 +888,42 @@ def glr_scan_pieces(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: O
              _ptr(piece_state), _ptr(decay), B, pieces, H, d, e, rows.shape[1], state.stride(0), _stream()), "glr_scan_pieces")
 
 
+def chunk_takes(d: int, e: int) -> bool:
+    """Whether `chunk_scan` takes heads of d key and e value channels."""
+    return d in (64, 128) and e > 0 and e % 16 == 0
+
+
+def chunk_scratch_floats(T: int, B: int, H: int, d: int) -> int:
+    return (T // 16 + B + 1) * H * (33 * d + 256)
+
+
+def chunk_scan(form: str, rows: torch.Tensor, b1: Optional[torch.Tensor], b2: Optional[torch.Tensor], out: torch.Tensor,
+               state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, scratch: torch.Tensor, B: int, H: int, d: int,
+               e: int, max_new: int) -> None:
+    """`glr_scan` (form "glr": b1 the gates' bias, b2 their lower bounds) or `wkv_scan` (form "wkv": b1 the decays' bias, b2 the
+    bonus) of a step of prompts, 16 tokens at a time on the matrix cores; `max_new`: the most tokens a sequence brings;
+    `scratch` float32, `chunk_scratch_floats` of them."""
+    _dev("chunk_scan", rows, b1, b2, out, cu_seqlens, slots, scratch)
+    _req(form in ("glr", "wkv"), f"chunk_scan: form {form!r}")
+    wkv = form == "wkv"
+    T = rows.shape[0]
+    n_state = 1
+    for x in glr_state_shape(H, d, e):
+        n_state *= x
+    _req(chunk_takes(d, e), f"chunk_scan: heads of {d} x {e}")
+    _req(state.is_cuda and state[0].numel() >= n_state and state.stride(-1) == 1 and (wkv or state[0].is_contiguous()),
+         "chunk_scan: state, every slot's dense")
+    _req(rows.dtype == out.dtype == state.dtype == scratch.dtype == torch.float32 and rows.dim() == 2, "chunk_scan: float32 only")
+    _req(rows.shape[1] >= (3 if wkv else 2) * H * d + H * e and rows.shape[1] % 4 == 0 and out.shape == (T, H * e), "chunk_scan: rows and out")
+    for v in (b1, b2):
+        _req((v is None and not wkv) or (v is not None and v.dtype == torch.float32 and v.numel() == H * d), "chunk_scan: vectors float32 [H*d]")
+    _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "chunk_scan: arrays shorter than the batch")
+    _req(scratch.numel() >= chunk_scratch_floats(T, B, H, d), "chunk_scan: scratch too small")
+    f = _fn("chunk_walk", "br_chunk_scan", [c_int, _P, c_int, _P, _P, _P, _P, c_size_t, _P, _P, _P, c_size_t] + [c_int] * 6 + [_P])
+    _check(f(int(wkv), _ptr(rows), rows.shape[1], _ptr(b1), _ptr(b2), _ptr(out), _ptr(state), state.stride(0), _ptr(cu_seqlens),
+             _ptr(slots), _ptr(scratch), scratch.numel(), T, B, H, d, e, int(max_new), _stream()), "chunk_scan")
+
+
 def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, H: int, e: int, eps: float) -> None:
     _dev("head_rmsnorm", o, w, out)
     T = o.shape[0]

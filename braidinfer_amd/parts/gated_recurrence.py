@@ -11,8 +11,9 @@ The state S [heads, d, e] starts at zero, lives in float in both precisions and 
 step to step in the sequence's slot of the cache's state area (`StateNeed`, laid out as the scan
 kernel's lanes hold it); the gates' activations, the recurrence and the head norm are float.
 Prompts are walked token by token inside one kernel, a workgroup per 16 columns of a head's state
-with the state in registers and the tokens' rows staged through LDS a chunk ahead; long prompts that
-would leave the chip idle are cut into pieces that are walked side by side (`pieces_for`).  The reference has no recurrent mixer of this form.
+with the state in registers and the tokens' rows staged through LDS a chunk ahead; prompts through heads of 64 or
+128 channels go 16 tokens at a time on the matrix cores (`in_chunks`), other long prompts that would leave the chip idle are
+cut into pieces that are walked side by side (`pieces_for`).  The reference has no recurrent mixer of this form.
 """
 from __future__ import annotations
 
@@ -42,6 +43,20 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
     units = step.n_seqs * units_per_sequence
     want = (int(os.environ.get("BRAIDINFER_GLR_FILL", "4")) * K.device_cus()) // max(1, units)
     return max(1, min(want, step.max_new // min_piece, 16, 65535 // max(1, step.n_seqs)))
+
+
+# From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores (HGRN2, 32 heads of 128 x 128,
+# us against the walk token by token, in pieces where that is faster: 64 tokens 20 / 17, 128 tokens 22 / 30, 512 tokens 44 / 101,
+# 2,048 tokens 125 / 326, 3,517 and 1,501 tokens 279 / 711; WKV, 64 heads of 64 x 64: 17 / 17, 20 / 30, 38 / 75, 111 / 252, 250 / 744).
+CHUNKS_FROM = 96
+
+
+def in_chunks(step, d: int, e: int) -> bool:
+    return not step.is_decode and step.max_new >= CHUNKS_FROM and K.chunk_takes(d, e)
+
+
+def chunk_scratch(step, H: int, d: int) -> torch.Tensor:
+    return step.ws.get("chunk_scratch", (K.chunk_scratch_floats(step.n_tokens, step.n_seqs, H, d),), torch.float32)
 
 
 class HGRN2(Mixer):
@@ -114,8 +129,11 @@ class HGRN2(Mixer):
         rows = step.ws.get("glr_qfv", (T, 2 * nh * d + nh * e), torch.float32)
         linear(h, self.w_qfv, rows, step.ws)
         o = step.ws.get("glr_o", (T, nh * e), torch.float32)
-        pieces = self.pieces_for(step)
-        if pieces > 1:
+        pieces = 1 if in_chunks(step, d, e) else self.pieces_for(step)
+        if in_chunks(step, d, e):
+            K.chunk_scan("glr", rows, self.f_bias, self.lower, o, ctx.state, step.cu_seqlens, step.slots, chunk_scratch(step, nh, d),
+                         step.n_seqs, nh, d, e, step.max_new)
+        elif pieces > 1:
             cu, numbers = self._piece_arrays(step, pieces)
             n = step.n_seqs * pieces
             piece_state = step.ws.get("glr_piece_state", (n,) + tuple(K.glr_state_shape(nh, d, e)), torch.float32)

@@ -27,7 +27,7 @@ from ..cache import StateNeed
 from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, Runtime, register_part
-from .gated_recurrence import HGRN2, pieces_for
+from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
 from .linear import linear, stream_layout
 
 BRANCHES = ("r", "k", "v", "g", "w")
@@ -102,8 +102,11 @@ class WKVTimeMix(Mixer):
         K.tanh(low, low_t)
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
-        pieces = pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
-        if pieces > 1:
+        pieces = 1 if in_chunks(step, self.d, self.d) else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
+        if in_chunks(step, self.d, self.d):
+            K.chunk_scan("wkv", rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, chunk_scratch(step, self.nh, self.d),
+                         step.n_seqs, self.nh, self.d, self.d, step.max_new)
+        elif pieces > 1:
             # long prompts: every sequence cut into pieces that are walked side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)
             n = step.n_seqs * pieces
