@@ -4,20 +4,26 @@
 //
 //     S_t = diag(w_t) S_(t-1) + k_t v_t^T,      o_t = S_t^T q_t                                 (INCLUDING the token's own write)
 //     S_t = diag(w_t) S_(t-1) + k_t v_t^T,      o_t = (S_(t-1) + diag(u) k_t v_t^T)^T q_t       (a bonus u instead of it)
+//     S_t = diag(w_t) S_(t-1) + k_t u_t^T,      u_t = beta_t (v_t - (diag(w_t) S_(t-1))^T k_t)  (the delta rule; o_t as first)
 //
 // Over a chunk of 16 tokens that starts from S, with products of decays over the chunk only (never a quotient of two):
 //     o_t = (q_t . prod_{r <= t} w_r)^T S + sum_{s <= t} A[t, s] v_s,     A[t, s] = sum_c q_t[c] k_s[c] prod_{s < r <= t} w_r[c]
 //     S' = diag(prod_r w_r) S + sum_s (k_s . prod_{r > s} w_r) v_s^T
-// (with the bonus the products stop before t, and A[t, t] = sum_c q_t u k_t).  Everything but the two products with S is the
+// (with the bonus the products stop before t, and A[t, t] = sum_c q_t u k_t).  The delta rule's u take the place of v there:
+// with L[t, s] = beta_t sum_c k_t[c] k_s[c] prod_{s < r <= t} w_r[c] for s < t they are u = U - W S, where the rows of U and W
+// follow by U_t = beta_t v_t - sum_s L[t, s] U_s and W_t = beta_t k_t . prod_{r <= t} w_r - sum_s L[t, s] W_s.  Everything but the products with S is the
 // same for all columns of the state and for all chunks at once, so `chunk_prepare` makes it for every (chunk, head) in
 // parallel, in the order in which a lane of the second kernel wants its operands; `chunk_walk` then walks the chunks of a
 // sequence in order, with S in the matrix cores' accumulators, which are at once the second operand of the read-out.  All
 // products and sums are float; against a walk token by token only their order differs.  Chunks are counted from the
 // sequence's first token of the step; a chunk's tokens beyond the sequence have decay 1, write nothing and read nothing.
 //
-// What bounds it: the walk is a serial chain of (17 + 17) / 2 float matrix instructions a wave and chunk (32 cycles each); a
-// walk token by token is bound by the 49,000 lane operations a head of 128 x 128 takes a token, the matrix cores take a
-// quarter of that time, and only 16 columns' workgroups times 4 waves are needed to have two waves a SIMD.
+// What bounds it: the walk is a serial chain, a chunk of a head of 128 x 128 costing a wave 17 float matrix instructions (32
+// cycles each) and about as much again in operand reads, the exchange of the quarters and the barrier (0.74 us a chunk with a
+// workgroup to a compute unit; a deeper ring changes nothing).  A walk token by token is bound by the 49,000 lane operations a
+// token of such a head takes.  32 heads of 128 x 128: 2,048 tokens 125 us (30 of them `chunk_prepare`, which is bound by its
+// reads and writes), 8,192 tokens 574; token by token, twice in pieces, 326 and 1,236.  64 heads of 64 x 64: 107 and 404,
+// token by token 252 and 1,052.
 #include "common.h"
 
 #define CW_C 16            // tokens of a chunk
@@ -32,48 +38,79 @@ __device__ __forceinline__ float cw_row16_sum(float v) {
 
 // Where a sequence's chunks lie in the scratch: sequence s has room for ceil(tokens / 16) chunks from cu[s] / 16 + s on.
 __device__ __forceinline__ int cw_first(const int* cu, int s) { return cu[s] / CW_C + s; }
-// Floats of a (chunk, head) in the scratch: read factors 16 D | write factors 16 D | A 256 | decay D.
-template <int D> constexpr int cw_block() { return 33 * D + 256; }
+// Floats of a (chunk, head) in the scratch: read factors 16 D | write factors 16 D | A 256 | decay D, and for the delta rule
+// -W 16 D | U 16 e.
+__host__ __device__ constexpr int cw_block(int D, int e, bool delta) { return 33 * D + 256 + (delta ? 16 * (D + e) : 0); }
 
-// rows [T, width] float; FORM 0 (`glr`): q | f at columns 0, H d, `b1` the gate's bias, `b2` its lower bound (null: 0);
-// FORM 1 (`wkv`): r | k at 0, H d and z at 2 H d + H e, `b1` the decay's bias, `b2` the bonus.
+#define CW_GLR 0
+#define CW_WKV 1
+#define CW_FIXED 2
+#define CW_DELTA 3
+// q, k: rows `qk_stride` apart, query/key head h / (H / G) at columns D apart; v: rows `v_stride` apart, head h at columns e apart.
+//  GLR: k holds the gates' sums, `b1` their bias, `b2` their lower bounds (null: 0): w = b2 + (1 - b2) sigmoid(k + b1), the key
+//       1 - w, the query silu(q), as glr_scan_kernel.
+//  WKV: `z` (rows `qk_stride` apart) the decays' sums, `b1` their bias, `b2` the bonus: w = exp(-exp(z + b1)), as wkv_scan_kernel.
+//  FIXED: w = b1[h], one number a head; `silu`: silu of q, k and v, the latter written back over v for the walk.
+//  DELTA: `gb` [T, 2 H] decay and beta a head, or with `gc` [T, H D] a decay a key channel and beta in gb's second half.
+struct CwIn {
+    const float *q, *k, *z, *b1, *b2, *gb, *gc;
+    float* v;
+    size_t qk_stride, v_stride;
+    const int *cu, *slots;
+    int H, G, e, silu;
+};
+
 // grid (chunks of the longest sequence, H, sequences), D threads, a thread a channel.
 template <int FORM, int D>
-__global__ __launch_bounds__(D) void chunk_prepare_kernel(const float* __restrict__ rows, int width, const float* __restrict__ b1,
-                                                          const float* __restrict__ b2, const int* __restrict__ cu_seqlens,
-                                                          const int* __restrict__ slots, float* __restrict__ scratch, int H, int e) {
+__global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* __restrict__ scratch) {
+    constexpr bool DELTA = FORM == CW_DELTA, WKV = FORM == CW_WKV;
     constexpr int KB = D / 16;
     __shared__ __attribute__((aligned(16))) float stage[KB * 272];        // read factors: [channel / 16][channel % 16 / 4][token][4], padded
-    __shared__ float part[136 * (D / 16)];
-    const int s = blockIdx.z, h = blockIdx.y, c = threadIdx.x, lane = c & 63;
-    if (slots[s] < 0) return;
-    const int t0 = cu_seqlens[s] + (int)blockIdx.x * CW_C, n = min(CW_C, cu_seqlens[s + 1] - t0);
+    __shared__ float part[(DELTA ? 256 : 136) * (D / 16)];
+    __shared__ __attribute__((aligned(16))) float Lm[DELTA ? 256 : 4];
+    const int s = blockIdx.z, h = blockIdx.y, c = threadIdx.x, H = in.H, e = in.e;
+    if (in.slots[s] < 0) return;
+    const int t0 = in.cu[s] + (int)blockIdx.x * CW_C, n = min(CW_C, in.cu[s + 1] - t0);
     if (n <= 0) return;
-    const int hd = H * D;
-    float q[CW_C], k[CW_C], w[CW_C];
-    const float bias = b1 ? b1[h * D + c] : 0.f, low = b2 ? b2[h * D + c] : 0.f;
+    const int kh = h / (H / in.G);
+    float q[CW_C], k[CW_C], w[CW_C], beta[DELTA ? CW_C : 1];
+    const float bias = (FORM == CW_GLR || WKV) && in.b1 ? in.b1[h * D + c] : 0.f, low = (FORM == CW_GLR || WKV) && in.b2 ? in.b2[h * D + c] : 0.f;
 #pragma unroll
     for (int t = 0; t < CW_C; ++t) {
-        const float* r = rows + (size_t)(t0 + min(t, n - 1)) * width + h * D + c;
-        q[t] = r[0];
-        k[t] = r[hd];
-        w[t] = FORM == 1 ? r[2 * hd + H * e] : 0.f;
+        const size_t row = (size_t)(t0 + min(t, n - 1));
+        q[t] = in.q[row * in.qk_stride + kh * D + c];
+        k[t] = in.k[row * in.qk_stride + kh * D + c];
+        w[t] = WKV ? in.z[row * in.qk_stride + h * D + c] : FORM == CW_FIXED ? in.b1[h] : 0.f;
+        if (DELTA) {
+            w[t] = in.gc ? in.gc[row * H * D + h * D + c] : in.gb[row * 2 * H + h];
+            beta[DELTA ? t : 0] = t < n ? in.gb[row * 2 * H + H + h] : 0.f;
+        }
     }
 #pragma unroll
     for (int t = 0; t < CW_C; ++t) {
-        if (FORM == 0) {
+        if (FORM == CW_GLR) {
             // as glr_scan_kernel applies them: exp and reciprocal by the hardware's own instructions (about an ulp each)
             const float gt = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (k[t] + bias)));
             q[t] = q[t] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * q[t]));
             w[t] = low + (1.0f - low) * gt;
             k[t] = 1.0f - w[t];
-        } else {
+        } else if (WKV) {
             w[t] = expf(-expf(w[t] + bias));
+        } else if (FORM == CW_FIXED && in.silu) {
+            q[t] = q[t] / (1.0f + expf(-q[t]));
+            k[t] = k[t] / (1.0f + expf(-k[t]));
         }
         if (t >= n) { q[t] = 0.f; k[t] = 0.f; w[t] = 1.f; }
     }
-    float* out = scratch + ((size_t)(cw_first(cu_seqlens, s) + blockIdx.x) * H + h) * cw_block<D>();
-    // A: 136 sums over the channels, 16 lanes at a time here
+    if (FORM == CW_FIXED && in.silu) {
+        for (int i = c; i < n * e; i += D) {
+            float* x = in.v + (size_t)(t0 + i / e) * in.v_stride + h * e + i % e;
+            const float y = *x;
+            *x = y / (1.0f + expf(-y));
+        }
+    }
+    float* out = scratch + ((size_t)(cw_first(in.cu, s) + blockIdx.x) * H + h) * cw_block(D, e, DELTA);
+    // A (and L): 136 (120) sums over the channels, 16 lanes at a time here
     int pair = 0;
 #pragma unroll
     for (int j = 0; j < CW_C; ++j) {
@@ -81,7 +118,7 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const float* __restric
 #pragma unroll
         for (int t = j; t < CW_C; ++t) {
             float term;
-            if (FORM == 0) {
+            if (!WKV) {
                 if (t > j) g *= w[t];
                 term = q[t] * g;
             } else {
@@ -89,17 +126,22 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const float* __restric
                 term = t == j ? q[t] * (low * g) : q[t] * g;
             }
             term = cw_row16_sum(term);
-            if ((lane & 15) == 0) part[pair * (D / 16) + (c >> 4)] = term;
+            if ((c & 15) == 0) part[pair * (D / 16) + (c >> 4)] = term;
+            if (DELTA && t > j) {
+                term = cw_row16_sum(k[t] * g);
+                if ((c & 15) == 0) part[(136 + pair - j - 1) * (D / 16) + (c >> 4)] = term;      // 120 pairs s < t: j + 1 diagonals before
+            }
             ++pair;
         }
     }
     // the factors: prefix products for what reads, suffix products for what writes
-    float p = 1.f;
+    float p = 1.f, W[DELTA ? CW_C : 1];
 #pragma unroll
     for (int t = 0; t < CW_C; ++t) {
-        if (FORM == 0) p *= w[t];
+        if (!WKV) p *= w[t];
         stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + t * 4 + (c & 3)] = q[t] * p;
-        if (FORM == 1) p *= w[t];
+        if (DELTA) W[DELTA ? t : 0] = beta[DELTA ? t : 0] * (k[t] * p);
+        if (WKV) p *= w[t];
     }
     out[32 * D + 256 + c] = p;
     p = 1.f;
@@ -115,11 +157,14 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const float* __restric
         *(f32x4*)(out + 16 * D + (c >> 4) * 256 + (16 * g + (c & 15)) * 4) = v;
     }
     __syncthreads();
+    auto unstage = [&](float* to) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int f = c + i * D, l = f & 63;
-        *(f32x4*)(out + f * 4) = *(const f32x4*)(stage + (f >> 6) * 272 + (l >> 4) * 68 + (l & 15) * 4);
-    }
+        for (int i = 0; i < 4; ++i) {
+            const int f = c + i * D, l = f & 63;
+            *(f32x4*)(to + f * 4) = *(const f32x4*)(stage + (f >> 6) * 272 + (l >> 4) * 68 + (l & 15) * 4);
+        }
+    };
+    unstage(out);
     for (int i = c; i < 256; i += D) {
         const int t = i >> 4, j = i & 15;
         float sum = 0.f;
@@ -129,160 +174,318 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const float* __restric
             for (int x = 0; x < D / 16; ++x) sum += pp[x];
         }
         out[32 * D + i] = sum;
+        if (DELTA) {
+            sum = 0.f;
+            if (j < t) {
+                const float* pp = part + (136 + j * CW_C - j * (j - 1) / 2 + t - j - j - 1) * (D / 16);
+#pragma unroll
+                for (int x = 0; x < D / 16; ++x) sum += pp[x];
+                sum *= t < n ? in.gb[(size_t)(t0 + t) * 2 * H + H + h] : 0.f;
+            }
+            Lm[DELTA ? i : 0] = sum;
+        }
+    }
+    if constexpr (DELTA) {
+        __syncthreads();
+        auto solve = [&](float (&x)[CW_C]) {                  // x_t -= sum_{s < t} L[t, s] x_s
+#pragma unroll
+            for (int t = 1; t < CW_C; ++t)
+#pragma unroll
+                for (int j = 0; j < t; ++j) x[t] = fmaf(-Lm[t * 16 + j], x[j], x[t]);
+        };
+        solve(W);
+#pragma unroll
+        for (int t = 0; t < CW_C; ++t) stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + t * 4 + (c & 3)] = -W[t];
+        float* uo = out + 49 * D + 256;
+        for (int x = c; x < e; x += D) {
+            float u[CW_C];
+#pragma unroll
+            for (int t = 0; t < CW_C; ++t) u[t] = beta[t] * in.v[(size_t)(t0 + min(t, n - 1)) * in.v_stride + h * e + x];
+            solve(u);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 v = {u[4 * g], u[4 * g + 1], u[4 * g + 2], u[4 * g + 3]};
+                *(f32x4*)(uo + (x >> 4) * 256 + (16 * g + (x & 15)) * 4) = v;
+            }
+        }
+        __syncthreads();
+        unstage(out + 33 * D + 256);
     }
 }
 
-// A workgroup walks a sequence's chunks for 16 columns of one head; wave w holds the state's rows w D / 4 .. + D / 4 and adds a
+// A workgroup walks a sequence's chunks for 16 CB columns of one head; wave w holds the state's rows w D / 4 .. + D / 4 and adds a
 // quarter of every output element (its rows' share and, of the sum over A, the tokens 4 g + w), the quarters are added in
 // wave order through LDS a chunk later.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
-// barrier a chunk.  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H, e / 16): the workgroups of a head
+// barrier a chunk.  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H, e / (16 CB)): the workgroups of a head
 // on one XCD where sequences * H is a multiple of 8.
-template <int D, int S>
+template <int D, int CB, int S, bool DELTA>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
                                                          float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
                                                          int zero_padding) {
-    constexpr int NKB = D / 64, RPL = D / 16, STAGE = (32 * D + 768) * 4, L = 2 * NKB + 1, BLOCK = cw_block<D>();
+    constexpr int NKB = D / 64, RPL = D / 16, STAGE = ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4, L = (DELTA ? 3 : 2) * NKB + 1;
+    constexpr int PB = DELTA ? 1 : 2;                         // buffers of output quarters
+    const int BLOCK = cw_block(D, e, DELTA);
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    float* part = (float*)(smem + S * STAGE);                 // [2][4][16][17]
+    float* part = (float*)(smem + S * STAGE);                 // [PB][4][CB][16][17]
+    float* pu = part + PB * 4 * CB * 272;                     // DELTA: [4][CB][64][4] the waves' shares of -W S
     const int s = blockIdx.x / H, h = blockIdx.x - s * H, cb = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int slot = slots[s], t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1], he = H * e;
     if (slot < 0) {
         if (zero_padding)
-            for (int i = tid; i < (t1 - t0) * 16; i += 256) o[(size_t)(t0 + (i >> 4)) * he + h * e + cb * 16 + (i & 15)] = 0.f;
+            for (int i = tid; i < (t1 - t0) * 16; i += 256) for (int x = 0; x < CB; ++x) o[(size_t)(t0 + (i >> 4)) * he + h * e + (cb * CB + x) * 16 + (i & 15)] = 0.f;
         return;
     }
     const int nch = (t1 - t0 + CW_C - 1) / CW_C;
     if (nch <= 0) return;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
     const float* blocks = scratch + ((size_t)cw_first(cu_seqlens, s) * H + h) * BLOCK;
-    auto bring = [&](unsigned lds, const float* p) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "m0", "memory");
+    // a stage: read factors | write factors | A | decay | values (256 floats each of the last three); a lane's byte offsets
+    // within a chunk's block, the block itself is a scalar address that goes on by a chunk's blocks
+    unsigned qoff[NKB], koff[NKB];
+#pragma unroll
+    for (int j = 0; j < NKB; ++j) {
+        qoff[j] = (unsigned)((wave * NKB + j) * 1024 + lane * 16);
+        koff[j] = qoff[j] + D * 64;
+    }
+    // waves 0 and 1 bring A and the decay's D floats, waves 2 and 3 the values (both the same 16 columns, or 16 each): L loads a wave
+    const unsigned moff = wave == 0 ? 128 * D + lane * 16 : 128 * D + 1024 + (lane * 16) % (4 * D);
+    const unsigned values = wave < 2 ? 0u : ~0u;
+    const unsigned long long values64 = wave < 2 ? 0ull : ~0ull;
+    unsigned long long block = (unsigned long long)blocks;
+    const int vx = cb * CB + (CB == 2 ? wave & 1 : 0);        // the 16 columns this wave brings values of
+    const unsigned long long vbase = (unsigned long long)(v + (size_t)t0 * ldv + h * e + vx * 16);
+    const unsigned vcol = ((lane & 3) ^ (lane >> 4)) * 16, uoff = (49 * D + 256) * 4 + vx * 1024 + lane * 16;
+    const int vlast = t1 - 1 - t0;
+    int vrow = lane >> 2, left = nch - 1, slot_i = 0;
+    auto bring = [&](unsigned lds, unsigned off, unsigned long long base) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0", "memory");
     };
-    // a stage: read factors | write factors | A | decay | values (256 floats each of the last three)
-    auto issue = [&](int ch) {
-        const float* b = blocks + (size_t)ch * H * BLOCK;
-        const unsigned st = __builtin_amdgcn_readfirstlane(lds0 + (ch % S) * STAGE);
+    // The next chunk, or behind the last one that again, into a stage nobody reads: no branch stands between a matrix
+    // instruction and the reads of its result, where the compiler has been seen to leave out the idle states they need.
+    auto issue = [&]() {
+        const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + slot_i * STAGE);
 #pragma unroll
         for (int j = 0; j < NKB; ++j) {
-            const int kb = wave * NKB + j;
-            bring(__builtin_amdgcn_readfirstlane(st + kb * 1024), b + kb * 256 + lane * 4);
-            bring(__builtin_amdgcn_readfirstlane(st + D * 64 + kb * 1024), b + 16 * D + kb * 256 + lane * 4);
+            bring(base + (wave * NKB + j) * 1024, qoff[j], block);
+            bring(base + D * 64 + (wave * NKB + j) * 1024, koff[j], block);
+            if (DELTA) bring(base + (32 * D + 512 + 256 * CB) * 4 + (wave * NKB + j) * 1024, qoff[j] + (33 * D + 256) * 4, block);
         }
-        // the decay's D floats: lanes beyond them bring what the first ones bring
-        const float* p = wave == 0   ? b + 32 * D + lane * 4
-                         : wave == 1 ? b + 32 * D + 256 + (lane * 4) % D
-                                     : v + (size_t)min(t0 + ch * CW_C + (lane >> 2), t1 - 1) * ldv + h * e + cb * 16 + ((lane & 3) ^ (lane >> 4)) * 4;
-        const int at = wave < 2 ? wave : 2;                   // waves 2 and 3 both bring the values: every wave L loads
-        bring(__builtin_amdgcn_readfirstlane(st + D * 128 + at * 1024), p);
+        const unsigned voff = DELTA ? uoff : (unsigned)min(vrow, vlast) * (unsigned)ldv * 4 + vcol;
+        bring(base + D * 128 + min(wave, 1 + CB) * 1024, (moff & ~values) | (voff & values),
+              DELTA ? block : (block & ~values64) | (vbase & values64));
+        const int go = left > 0;
+        block += (unsigned long long)(go * H) * (unsigned)(BLOCK * 4);
+        vrow += go * CW_C;
+        left -= go;
+        slot_i = slot_i == S - 1 ? 0 : slot_i + 1;
     };
-    f32x4 st[NKB];
-    const int c = cb * 16 + r16;
-    float* S0 = state + (size_t)slot * slot_stride + ((size_t)h * ((e + 3) >> 2) + (c >> 2)) * RPL * 64 + 16 * (c & 3);
+    f32x4 st[CB][NKB];
+    float* S0[CB];
 #pragma unroll
-    for (int j = 0; j < NKB; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int k = 16 * (wave * NKB + j) + 4 * g + r;
-            st[j][r] = S0[(size_t)(k % RPL) * 64 + k / RPL];
-        }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // from here on only the ring's loads are counted
-#pragma unroll
-    for (int j = 0; j < S - 1; ++j)
-        if (j < nch) issue(j);
-    const int ot = tid >> 4;
-    auto flush = [&](int ch) {                                // the quarters of chunk ch's outputs
-        const float* pp = part + (ch & 1) * 4 * 272 + ot * 17 + (tid & 15);
-        const int t = t0 + ch * CW_C + ot;
-        if (t < t1) o[(size_t)t * he + h * e + cb * 16 + (tid & 15)] = ((pp[0] + pp[272]) + pp[544]) + pp[816];
-    };
-    for (int ch = 0; ch < nch; ++ch) {
-        if (ch + S - 2 < nch) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * L) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (ch > 0) flush(ch - 1);
-        if (ch + S - 1 < nch) issue(ch + S - 1);
-        const float* sf = (const float*)(smem + (ch % S) * STAGE);
-        f32x4 qf[NKB], kf[NKB], dec[NKB];
-        float vv[4];
-#pragma unroll
-        for (int j = 0; j < NKB; ++j) {
-            const int kb = wave * NKB + j;
-            qf[j] = *(const f32x4*)(sf + kb * 256 + lane * 4);
-            kf[j] = *(const f32x4*)(sf + 16 * D + kb * 256 + lane * 4);
-            dec[j] = *(const f32x4*)(sf + 32 * D + 256 + 16 * kb + 4 * g);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vv[i] = sf[32 * D + 512 + (4 * g + i) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
-        const float a = sf[32 * D + r16 * 16 + 4 * g + wave];
-        const float va = sf[32 * D + 512 + (4 * g + wave) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
-        f32x4 oa = {0.f, 0.f, 0.f, 0.f};
-        oa = __builtin_amdgcn_mfma_f32_16x16x4f32(a, va, oa, 0, 0, 0);
+    for (int x = 0; x < CB; ++x) {
+        const int c = (cb * CB + x) * 16 + r16;
+        S0[x] = state + (size_t)slot * slot_stride + ((size_t)h * ((e + 3) >> 2) + (c >> 2)) * RPL * 64 + 16 * (c & 3);
 #pragma unroll
         for (int j = 0; j < NKB; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) oa = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[j][r], st[j][r], oa, 0, 0, 0);
+            for (int r = 0; r < 4; ++r) {
+                const int k = 16 * (wave * NKB + j) + 4 * g + r;
+                st[x][j][r] = S0[x][(size_t)(k % RPL) * 64 + k / RPL];
+            }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // from here on only the ring's loads are counted
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) issue();
+    const int ot = tid >> 4;
+    float* op = o + (size_t)(t0 + ot) * he + h * e + cb * CB * 16 + (tid & 15);       // this thread's element of the chunk before
+    auto flush = [&](int ch) {                                // the quarters of chunk ch's outputs, chunks in order
+#pragma unroll
+        for (int x = 0; x < CB; ++x) {
+            const float* pp = part + ((ch & (PB - 1)) * 4 * CB + x) * 272 + ot * 17 + (tid & 15);
+            const float v = ((pp[0] + pp[CB * 272]) + pp[2 * CB * 272]) + pp[3 * CB * 272];
+            if (t0 + ch * CW_C + ot < t1) op[x * 16] = v;
+        }
+        op += (size_t)CW_C * he;
+    };
+    const float* sf = (const float*)smem;                     // the stage in use
+    int cur = 0;
+    for (int ch = 0; ch < nch; ++ch) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * L) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // the operands first: the matrix instructions start as soon as they are there, the rest runs beside them
+        f32x4 qf[NKB], kf[NKB], dec[NKB], oa[CB];
+        float vv[CB][4], va[CB];
+        const float a = sf[32 * D + r16 * 16 + 4 * g + wave];
+#pragma unroll
+        for (int j = 0; j < NKB; ++j) qf[j] = *(const f32x4*)(sf + (wave * NKB + j) * 256 + lane * 4);
+#pragma unroll
+        for (int j = 0; j < NKB; ++j) {
+            const int kb = wave * NKB + j;
+            dec[j] = *(const f32x4*)(sf + 32 * D + 256 + 16 * kb + 4 * g);
+            kf[j] = *(const f32x4*)(sf + 16 * D + kb * 256 + lane * 4);
+        }
+        auto read_out = [&]() {                               // this wave's rows' share of the outputs
+#pragma unroll
+            for (int j = 0; j < NKB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int x = 0; x < CB; ++x) oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[j][r], st[x][j][r], oa[x], 0, 0, 0);
+        };
+#pragma unroll
+        for (int x = 0; x < CB; ++x) oa[x] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (DELTA) {
+            f32x4 uf[CB], wf[NKB], pa[CB];
+#pragma unroll
+            for (int j = 0; j < NKB; ++j) wf[j] = *(const f32x4*)(sf + 32 * D + 512 + 256 * CB + (wave * NKB + j) * 256 + lane * 4);
+#pragma unroll
+            for (int x = 0; x < CB; ++x) {
+                uf[x] = *(const f32x4*)(sf + 32 * D + 512 + x * 256 + lane * 4);
+                pa[x] = {0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int j = 0; j < NKB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int x = 0; x < CB; ++x) pa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][r], st[x][j][r], pa[x], 0, 0, 0);
+            read_out();
+#pragma unroll
+            for (int x = 0; x < CB; ++x) *(f32x4*)(pu + ((wave * CB + x) * 64 + lane) * 4) = pa[x];
+            if (ch > 0) flush(ch - 1);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int x = 0; x < CB; ++x) {                    // u = U - W S, the waves' shares in their order
+                f32x4 u = uf[x];
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    const f32x4 share = *(const f32x4*)(pu + ((y * CB + x) * 64 + lane) * 4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) u[r] += share[r];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) vv[x][r] = u[r];
+                va[x] = wave < 2 ? (wave == 0 ? u[0] : u[1]) : (wave == 2 ? u[2] : u[3]);
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < CB; ++x) {
+                va[x] = sf[32 * D + 512 + x * 256 + (4 * g + wave) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) vv[x][i] = sf[32 * D + 512 + x * 256 + (4 * g + i) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < CB; ++x) oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, va[x], oa[x], 0, 0, 0);
+        if constexpr (!DELTA) read_out();
+        issue();
 #pragma unroll
         for (int j = 0; j < NKB; ++j) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) st[j][r] *= dec[j][r];
+            for (int x = 0; x < CB; ++x)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[i], st[j], 0, 0, 0);
+                for (int r = 0; r < 4; ++r) st[x][j][r] *= dec[j][r];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int x = 0; x < CB; ++x) st[x][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], st[x][j], 0, 0, 0);
         }
-        float* pw = part + (ch & 1) * 4 * 272 + wave * 272;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = oa[r];
+        for (int x = 0; x < CB; ++x) {
+            float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = oa[x][r];
+        }
+        if (!DELTA && ch > 0) flush(ch - 1);
+        cur = cur == S - 1 ? 0 : cur + 1;
+        sf = (const float*)(smem + cur * STAGE);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");          // no load into LDS outlives the workgroup
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     flush(nch - 1);
 #pragma unroll
-    for (int j = 0; j < NKB; ++j)
+    for (int x = 0; x < CB; ++x)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int k = 16 * (wave * NKB + j) + 4 * g + r;
-            S0[(size_t)(k % RPL) * 64 + k / RPL] = st[j][r];
-        }
+        for (int j = 0; j < NKB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = 16 * (wave * NKB + j) + 4 * g + r;
+                S0[x][(size_t)(k % RPL) * 64 + k / RPL] = st[x][j][r];
+            }
 }
 
 // Whether a head of d x e goes this way.
 extern "C" int br_chunk_takes(int d, int e) { return (d == 64 || d == 128) && e > 0 && e % 16 == 0; }
 // Floats of scratch for T tokens of B sequences.
-extern "C" size_t br_chunk_scratch(int T, int B, int H, int d) { return (size_t)(T / CW_C + B + 1) * H * (33 * (size_t)d + 256); }
+extern "C" size_t br_chunk_scratch(int T, int B, int H, int d, int e, int delta) {
+    return (size_t)(T / CW_C + B + 1) * H * (size_t)cw_block(d, e, delta != 0);
+}
 
-template <int FORM, int D, int S>
-static int chunk_run(const float* rows, int width, const float* b1, const float* b2, float* o, float* state, size_t slot_stride,
-                     const int* cu, const int* slots, float* scratch, int B, int H, int e, int max_new, hipStream_t s) {
-    constexpr size_t lds = (size_t)S * (32 * D + 768) * 4 + 2 * 4 * 272 * 4;
-    static_assert(lds <= 80 * 1024, "two workgroups a compute unit");
-    auto walk = chunk_walk_kernel<D, S>;
+template <int D, int CB, int S, bool DELTA>
+static int chunk_walk(const CwIn& in, const float* scratch, float* o, float* state, size_t slot_stride, int B, int zero_padding,
+                      hipStream_t s) {
+    constexpr size_t lds = (size_t)S * ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4 + (DELTA ? 1 : 2) * 4 * CB * 272 * 4 + (DELTA ? 4096 * CB : 0);
+    static_assert(lds <= 160 * 1024, "LDS");
+    auto walk = chunk_walk_kernel<D, CB, S, DELTA>;
     static bool set = false;
     if (!set) {
         if (hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
         set = true;
     }
-    chunk_prepare_kernel<FORM, D><<<dim3((max_new + CW_C - 1) / CW_C, H, B), D, 0, s>>>(rows, width, b1, b2, cu, slots, scratch, H, e);
-    walk<<<dim3(B * H, e / 16), 256, lds, s>>>(scratch, rows + 2 * H * D, width, o, state, slot_stride, cu, slots, H, e, FORM == 1);
+    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding);
     return br_check_launch();
 }
 
-// One step's tokens of B sequences (`max_new` the most a sequence brings) through the recurrence `form` (0: `glr`, 1: `wkv`,
-// see chunk_prepare_kernel), from and into the slots' states; `scratch`: br_chunk_scratch floats.
-extern "C" int br_chunk_scan(int form, const float* rows, int width, const float* b1, const float* b2, float* o, float* state,
+template <int FORM, int D>
+static int chunk_run(const CwIn& in, float* o, float* state, size_t slot_stride, float* scratch, int B, int max_new, hipStream_t s) {
+    constexpr bool DELTA = FORM == CW_DELTA;
+    chunk_prepare_kernel<FORM, D><<<dim3((max_new + CW_C - 1) / CW_C, in.H, B), D, 0, s>>>(in, scratch);
+    const int rc = br_check_launch();
+    if (rc != BR_OK) return rc;
+    // 16 columns a workgroup where that gives no more workgroups than compute units (two to each for heads of 64); beyond, 32
+    // columns, which share a chunk's loads: with a ring of twice the depth while a compute unit has one such workgroup (32 heads
+    // of 128 x 128, 3,517 and 1,501 tokens: 305 -> 278 us), else two of them to a unit (16 sequences of 300 tokens: 302 -> 225;
+    // 64 heads of 64 x 64: 231 -> 191).
+    const int cus = br_device_cus();
+    if (!cus) return BR_LAUNCH_FAILED;
+    const long long units = (long long)B * in.H * (in.e / 16);
+#define CW_WALK(CB, S) return chunk_walk<D, CB, S, DELTA>(in, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
+    if (in.e % 32 || units <= (D == 64 ? 2 : 1) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
+    if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
+    else {
+        if (D == 128 && units <= 2 * cus) CW_WALK(2, (D == 64 ? 5 : 6));
+        CW_WALK(2, (D == 64 ? 5 : 3));
+    }
+#undef CW_WALK
+}
+
+// One step's tokens of B sequences (`max_new` the most a sequence brings) through a recurrence (see CwIn for the forms' inputs),
+// from and into the slots' states; `scratch`: br_chunk_scratch floats.
+extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v, size_t qk_stride, size_t v_stride, const float* z,
+                             const float* b1, const float* b2, const float* gb, const float* gc, int silu, float* o, float* state,
                              size_t slot_stride, const int* cu_seqlens, const int* slots, float* scratch, size_t scratch_floats, int T,
-                             int B, int H, int d, int e, int max_new, hipStream_t s) {
+                             int B, int H, int G, int d, int e, int max_new, hipStream_t s) {
     if (B <= 0 || T <= 0) return BR_OK;
     if (!br_chunk_takes(d, e) || H <= 0 || H > 65535 || B > 65535 || (long long)B * H > 0x7fffffffLL || e / 16 > 65535 || max_new <= 0 ||
-        max_new > T || (form != 0 && form != 1) || width < (form ? 3 : 2) * H * d + H * e || width % 4 || (uintptr_t)rows % 16 ||
-        (uintptr_t)scratch % 16 || slot_stride < (size_t)H * ((e + 3) / 4) * d * 4 || scratch_floats < br_chunk_scratch(T, B, H, d))
+        max_new > T || G <= 0 || H % G || form < CW_GLR || form > CW_DELTA || v_stride % 4 || ((uintptr_t)v | (uintptr_t)scratch) % 16 ||
+        v_stride > 0x7fffffff || (unsigned long long)max_new * v_stride * 4 >= (1ull << 32) || slot_stride < (size_t)H * ((e + 3) / 4) * d * 4 ||
+        scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA) || (form == CW_WKV && (!z || !b1 || !b2)) ||
+        (form == CW_FIXED && !b1) || (form == CW_DELTA && !gb) || ((form == CW_GLR || form == CW_WKV) && G != H))
         return BR_BAD_ARG;
-#define CW_RUN(F, D_, S_) chunk_run<F, D_, S_>(rows, width, b1, b2, o, state, slot_stride, cu_seqlens, slots, scratch, B, H, e, max_new, s)
-    if (form == 0) return d == 64 ? CW_RUN(0, 64, 4) : CW_RUN(0, 128, 3);
-    return d == 64 ? CW_RUN(1, 64, 4) : CW_RUN(1, 128, 3);
+    const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu};
+#define CW_RUN(F) return d == 64 ? chunk_run<F, 64>(in, o, state, slot_stride, scratch, B, max_new, s) : chunk_run<F, 128>(in, o, state, slot_stride, scratch, B, max_new, s)
+    switch (form) {
+        case CW_GLR: CW_RUN(CW_GLR);
+        case CW_WKV: CW_RUN(CW_WKV);
+        case CW_FIXED: CW_RUN(CW_FIXED);
+        default: CW_RUN(CW_DELTA);
+    }
 #undef CW_RUN
 }

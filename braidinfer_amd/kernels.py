@@ -893,35 +893,48 @@ def chunk_takes(d: int, e: int) -> bool:
     return d in (64, 128) and e > 0 and e % 16 == 0
 
 
-def chunk_scratch_floats(T: int, B: int, H: int, d: int) -> int:
-    return (T // 16 + B + 1) * H * (33 * d + 256)
+def chunk_scratch_floats(T: int, B: int, H: int, d: int, e: int, delta: bool = False) -> int:
+    return (T // 16 + B + 1) * H * (33 * d + 256 + (16 * (d + e) if delta else 0))
 
 
-def chunk_scan(form: str, rows: torch.Tensor, b1: Optional[torch.Tensor], b2: Optional[torch.Tensor], out: torch.Tensor,
-               state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, scratch: torch.Tensor, B: int, H: int, d: int,
-               e: int, max_new: int) -> None:
-    """`glr_scan` (form "glr": b1 the gates' bias, b2 their lower bounds) or `wkv_scan` (form "wkv": b1 the decays' bias, b2 the
-    bonus) of a step of prompts, 16 tokens at a time on the matrix cores; `max_new`: the most tokens a sequence brings;
-    `scratch` float32, `chunk_scratch_floats` of them."""
-    _dev("chunk_scan", rows, b1, b2, out, cu_seqlens, slots, scratch)
-    _req(form in ("glr", "wkv"), f"chunk_scan: form {form!r}")
-    wkv = form == "wkv"
-    T = rows.shape[0]
+def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
+               cu_seqlens: torch.Tensor, slots: torch.Tensor, scratch: torch.Tensor, B: int, H: int, G: int, d: int, e: int,
+               max_new: int, z: Optional[torch.Tensor] = None, b1: Optional[torch.Tensor] = None, b2: Optional[torch.Tensor] = None,
+               gb: Optional[torch.Tensor] = None, gc: Optional[torch.Tensor] = None, silu: bool = False) -> None:
+    """A recurrence over a step of prompts, 16 tokens at a time on the matrix cores: form "glr" as `glr_scan` (k the gates'
+    sums, b1 their bias, b2 their lower bounds), "wkv" as `wkv_scan` (z the decays' sums, b1 their bias, b2 the bonus), "fixed"
+    as `dr_scan` with `g_head` (b1; `silu` is applied to q, k and v, the latter in place) and "delta" as `dr_scan` with `gb`
+    (and `gc`).  q, k, v: float rows, views of wider ones allowed (q, k and z with one stride); `max_new`: the most tokens a
+    sequence brings; `scratch` float32, `chunk_scratch_floats` of them."""
+    _req(form in ("glr", "wkv", "fixed", "delta"), f"chunk_scan: form {form!r}")
+    number = ("glr", "wkv", "fixed", "delta").index(form)
+    T = q.shape[0]
+    rows = [q, k, v] + ([z] if z is not None else [])
+    for t in rows + [state]:
+        _req(t.is_cuda and t.dtype == torch.float32 and t.stride(-1) == 1, "chunk_scan: dense float32 rows on the device")
+    _dev("chunk_scan", out, cu_seqlens, slots, scratch, b1, b2, gb, gc)
     n_state = 1
     for x in glr_state_shape(H, d, e):
         n_state *= x
     _req(chunk_takes(d, e), f"chunk_scan: heads of {d} x {e}")
-    _req(state.is_cuda and state[0].numel() >= n_state and state.stride(-1) == 1 and (wkv or state[0].is_contiguous()),
-         "chunk_scan: state, every slot's dense")
-    _req(rows.dtype == out.dtype == state.dtype == scratch.dtype == torch.float32 and rows.dim() == 2, "chunk_scan: float32 only")
-    _req(rows.shape[1] >= (3 if wkv else 2) * H * d + H * e and rows.shape[1] % 4 == 0 and out.shape == (T, H * e), "chunk_scan: rows and out")
-    for v in (b1, b2):
-        _req((v is None and not wkv) or (v is not None and v.dtype == torch.float32 and v.numel() == H * d), "chunk_scan: vectors float32 [H*d]")
+    _req(state[0].numel() >= n_state and state[0].is_contiguous(), "chunk_scan: state, every slot's dense")
+    _req(q.shape == k.shape == (T, G * d) and v.shape == (T, H * e) and out.shape == (T, H * e) and out.dtype == scratch.dtype == torch.float32
+         and (z is None or z.shape == (T, H * d)), "chunk_scan: q, k [T, G*d], v and out [T, H*e], z [T, H*d]")
+    stride = q.stride(0)
+    _req(all(t.stride(0) == stride for t in ([k] + ([z] if z is not None else []))), "chunk_scan: q, k and z share a row stride")
+    _req((form == "wkv") == (z is not None) and (form == "delta") == (gb is not None) and (gc is None or form == "delta"), "chunk_scan: inputs of another form")
+    width = H if form == "fixed" else H * d
+    for x in (b1, b2):
+        _req(x is None or (x.dtype == torch.float32 and x.numel() == width), "chunk_scan: vectors float32")
+    _req(gb is None or (gb.dtype == torch.float32 and gb.shape == (T, 2 * H)), "chunk_scan: gb float32 [T, 2*H]")
+    _req(gc is None or (gc.dtype == torch.float32 and gc.shape == (T, H * d)), "chunk_scan: gc float32 [T, H*d]")
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "chunk_scan: arrays shorter than the batch")
-    _req(scratch.numel() >= chunk_scratch_floats(T, B, H, d), "chunk_scan: scratch too small")
-    f = _fn("chunk_walk", "br_chunk_scan", [c_int, _P, c_int, _P, _P, _P, _P, c_size_t, _P, _P, _P, c_size_t] + [c_int] * 6 + [_P])
-    _check(f(int(wkv), _ptr(rows), rows.shape[1], _ptr(b1), _ptr(b2), _ptr(out), _ptr(state), state.stride(0), _ptr(cu_seqlens),
-             _ptr(slots), _ptr(scratch), scratch.numel(), T, B, H, d, e, int(max_new), _stream()), "chunk_scan")
+    _req(scratch.numel() >= chunk_scratch_floats(T, B, H, d, e, form == "delta"), "chunk_scan: scratch too small")
+    f = _fn("chunk_walk", "br_chunk_scan", [c_int, _P, _P, _P, c_size_t, c_size_t] + [_P] * 5 + [c_int, _P, _P, c_size_t, _P, _P, _P, c_size_t]
+            + [c_int] * 7 + [_P])
+    _check(f(number, _ptr(q), _ptr(k), _ptr(v), stride, v.stride(0), _ptr(z), _ptr(b1), _ptr(b2), _ptr(gb), _ptr(gc), int(silu), _ptr(out),
+             _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots), _ptr(scratch), scratch.numel(), T, B, H, G, d, e, int(max_new),
+             _stream()), "chunk_scan")
 
 
 def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, H: int, e: int, eps: float) -> None:

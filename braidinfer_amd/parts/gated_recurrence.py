@@ -47,7 +47,9 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
 
 # From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores (HGRN2, 32 heads of 128 x 128,
 # us against the walk token by token, in pieces where that is faster: 64 tokens 20 / 17, 128 tokens 22 / 30, 512 tokens 44 / 101,
-# 2,048 tokens 125 / 326, 3,517 and 1,501 tokens 279 / 711; WKV, 64 heads of 64 x 64: 17 / 17, 20 / 30, 38 / 75, 111 / 252, 250 / 744).
+# 2,048 tokens 125 / 326, 3,517 and 1,501 tokens 278 / 711; WKV, 64 heads of 64 x 64: 17 / 17, 20 / 30, 37 / 75, 107 / 252, 242 / 744;
+# delta rule, 32 heads of 128 x 128: 96 tokens 31 / 30, 128 tokens 34 / 38, 2,048 tokens 185 / 521, 1,307, 804 and 301 tokens 247 / 384;
+# a fixed decay a head: 26 / 34, 29 / 43, 150 / 603, 175 / 446).
 CHUNKS_FROM = 96
 
 
@@ -55,8 +57,8 @@ def in_chunks(step, d: int, e: int) -> bool:
     return not step.is_decode and step.max_new >= CHUNKS_FROM and K.chunk_takes(d, e)
 
 
-def chunk_scratch(step, H: int, d: int) -> torch.Tensor:
-    return step.ws.get("chunk_scratch", (K.chunk_scratch_floats(step.n_tokens, step.n_seqs, H, d),), torch.float32)
+def chunk_scratch(step, H: int, d: int, e: int, delta: bool = False) -> torch.Tensor:
+    return step.ws.get("chunk_scratch", (K.chunk_scratch_floats(step.n_tokens, step.n_seqs, H, d, e, delta),), torch.float32)
 
 
 class HGRN2(Mixer):
@@ -131,8 +133,9 @@ class HGRN2(Mixer):
         o = step.ws.get("glr_o", (T, nh * e), torch.float32)
         pieces = 1 if in_chunks(step, d, e) else self.pieces_for(step)
         if in_chunks(step, d, e):
-            K.chunk_scan("glr", rows, self.f_bias, self.lower, o, ctx.state, step.cu_seqlens, step.slots, chunk_scratch(step, nh, d),
-                         step.n_seqs, nh, d, e, step.max_new)
+            hd = nh * d
+            K.chunk_scan("glr", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:], o, ctx.state, step.cu_seqlens, step.slots,
+                         chunk_scratch(step, nh, d, e), step.n_seqs, nh, nh, d, e, step.max_new, b1=self.f_bias, b2=self.lower)
         elif pieces > 1:
             cu, numbers = self._piece_arrays(step, pieces)
             n = step.n_seqs * pieces

@@ -104,8 +104,9 @@ class WKVTimeMix(Mixer):
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
         pieces = 1 if in_chunks(step, self.d, self.d) else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
         if in_chunks(step, self.d, self.d):
-            K.chunk_scan("wkv", rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, chunk_scratch(step, self.nh, self.d),
-                         step.n_seqs, self.nh, self.d, self.d, step.max_new)
+            r, k, v, z = (rows[:, i * hd:(i + 1) * hd] for i in range(4))
+            K.chunk_scan("wkv", r, k, v, o, state, step.cu_seqlens, step.slots, chunk_scratch(step, self.nh, self.d, self.d), step.n_seqs,
+                         self.nh, self.nh, self.d, self.d, step.max_new, z=z, b1=self.w0, b2=self.u)
         elif pieces > 1:
             # long prompts: every sequence cut into pieces that are walked side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)

@@ -6,28 +6,61 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def walk(form, rows, b1, b2, S, cu, H, d, e):
+def walk(form, i, S, cu, H, G, d, e):
     """float64: o [T, H, e] and the last states [B, H, d, e]."""
-    rows = rows.double().cpu()
-    T, hd = rows.shape[0], H * d
-    b1, b2 = b1.double().cpu().reshape(H, d), b2.double().cpu().reshape(H, d)
-    q = rows[:, :hd].reshape(T, H, d)
-    k = rows[:, hd:2 * hd].reshape(T, H, d)
-    v = rows[:, 2 * hd:2 * hd + H * e].reshape(T, H, e)
+    i = {n: x.double().cpu() if torch.is_tensor(x) else x for n, x in i.items()}
+    T = i["q"].shape[0]
+    q, k = (i[n].reshape(T, G, d).repeat_interleave(H // G, 1) for n in "qk")
+    v = i["v"].reshape(T, H, e)
+    silu = lambda x: x * torch.sigmoid(x)
+    beta = None
     if form == "glr":
-        w = b2 + (1 - b2) * torch.sigmoid(k + b1)
-        q, k = q * torch.sigmoid(q), 1 - w
+        low = i["b2"].reshape(H, d)
+        w = low + (1 - low) * torch.sigmoid(k + i["b1"].reshape(H, d))
+        q, k = silu(q), 1 - w
+    elif form == "wkv":
+        w = torch.exp(-torch.exp(i["z"].reshape(T, H, d) + i["b1"].reshape(H, d)))
+    elif form == "fixed":
+        w = i["b1"].reshape(1, H, 1).expand(T, H, d)
+        if i.get("silu"):
+            q, k, v = silu(q), silu(k), silu(v)
     else:
-        w = torch.exp(-torch.exp(rows[:, 2 * hd + H * e:3 * hd + H * e].reshape(T, H, d) + b1))
+        w = i["gc"].reshape(T, H, d) if "gc" in i else i["gb"][:, :H, None].expand(T, H, d)
+        beta = i["gb"][:, H:]
     o = torch.zeros(T, H, e, dtype=torch.float64)
     S = S.double().cpu().clone()
     for s in range(len(cu) - 1):
         for t in range(cu[s], cu[s + 1]):
-            kv = k[t][:, :, None] * v[t][:, None, :]
-            new = w[t][:, :, None] * S[s] + kv
-            o[t] = torch.einsum("hd,hde->he", q[t], new if form == "glr" else S[s] + b2[:, :, None] * kv)
-            S[s] = new
+            new = w[t][:, :, None] * S[s]
+            u = v[t] if beta is None else beta[t][:, None] * (v[t] - torch.einsum("hde,hd->he", new, k[t]))
+            kv = k[t][:, :, None] * u[:, None, :]
+            o[t] = torch.einsum("hd,hde->he", q[t], S[s] + i["b2"].reshape(H, d)[:, :, None] * kv if form == "wkv" else new + kv)
+            S[s] = new + kv
     return o, S
+
+
+def inputs(form, T, H, G, d, e, strong, g):
+    """Float rows as views of wider ones, and the form's vectors."""
+    r = lambda *s: torch.randn(*s, generator=g) * (4.0 if strong else 1.0)
+    if form in ("glr", "wkv"):
+        rows = r(T, 3 * H * d + H * e + 4)
+        i = {"q": rows[:, :H * d], "k": rows[:, H * d:2 * H * d], "v": rows[:, 2 * H * d:2 * H * d + H * e]}
+        i["b1"] = torch.randn(H * d, generator=g) * (2.0 if strong else 0.3)
+        i["b2"] = torch.rand(H * d, generator=g) * 0.5 if form == "glr" else torch.randn(H * d, generator=g)
+        if form == "wkv":
+            i["z"] = rows[:, 2 * H * d + H * e:3 * H * d + H * e]
+        return i
+    if form == "fixed":
+        rows = r(T, 2 * H * d + H * e)
+        return {"q": rows[:, :H * d], "k": rows[:, H * d:2 * H * d], "v": rows[:, 2 * H * d:], "silu": strong,
+                "b1": torch.rand(H, generator=g) if strong else 1 - torch.rand(H, generator=g) * 0.1}
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)
+    q, k = (unit(torch.randn(T, G, d, generator=g) + (1.0 if strong else 0.0)).reshape(T, G * d) for _ in range(2))
+    gb = torch.rand(T, 2 * H, generator=g) ** (0.2 if strong else 1.0)
+    i = {"q": q, "k": k, "v": r(T, H * e), "gb": gb}
+    if form == "channels":
+        i["gc"] = torch.rand(T, H * d, generator=g) ** (0.1 if strong else 1.0)
+    return i
 
 
 def as_kept(S, d):
@@ -39,31 +72,41 @@ def as_kept(S, d):
 
 # one token, a chunk less one, exactly, and one more, the ring's stages and beyond; widths of both kinds; a sequence whose slot is
 # negative; decays from nearly nothing to nearly one
-@pytest.mark.parametrize("form", ["glr", "wkv"])
+@pytest.mark.parametrize("form", ["glr", "wkv", "fixed", "delta", "channels"])
 @pytest.mark.parametrize("d,e,H,lens,strong", [(64, 64, 3, (1, 15, 16, 17), False), (128, 128, 2, (31, 32, 48, 3), False),
-                                               (64, 16, 2, (49, 64, 65, 80, 97), True), (128, 48, 1, (200,), True), (128, 16, 8, (5, 333), False)])
+                                               (64, 16, 2, (49, 64, 65, 80, 97), True), (128, 48, 1, (200,), True), (128, 16, 8, (5, 333), False),
+                                               (128, 128, 40, (33, 18), True), (64, 64, 130, (35,), False)])
 def test_chunks_against_token_by_token(form, d, e, H, lens, strong):
     from braidinfer_amd import kernels as K
     g = torch.Generator().manual_seed(sum(lens) + d)
-    B, T = len(lens), sum(lens)
+    B, T, G = len(lens), sum(lens), H // 2 if form == "delta" and H % 2 == 0 else H
     cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
-    hd, he = H * d, H * e
-    width = 2 * hd + he if form == "glr" else 3 * hd + he + 4
-    rows = torch.randn(T, width, generator=g) * (4.0 if strong else 1.0)
-    b1 = torch.randn(hd, generator=g) * (2.0 if strong else 0.3)
-    b2 = torch.rand(hd, generator=g) * 0.5 if form == "glr" else torch.randn(hd, generator=g)
+    he = H * e
+    i = inputs(form, T, H, G, d, e, strong, g)
+    form = "delta" if form == "channels" else form
     S = torch.randn(B, H, d, e, generator=g)
-    want_o, want_S = walk(form, rows, b1, b2, S, cu, H, d, e)
+    want_o, want_S = walk(form, i, S, cu, H, G, d, e)
     shape = K.glr_state_shape(H, d, e)
     state = torch.full((B + 2,) + tuple(shape), 7.0, device="cuda")
     slots = torch.arange(B, dtype=torch.int32) + 1
     state[1:B + 1] = as_kept(S, d).reshape((B,) + tuple(shape)).cuda()
     out = torch.full((T, he), 7.0, device="cuda")
-    scratch = torch.full((K.chunk_scratch_floats(T, B, H, d),), float("nan"), device="cuda")
-    args = (rows.cuda(), b1.cuda(), b2.cuda())
+    scratch = torch.full((K.chunk_scratch_floats(T, B, H, d, e, form == "delta"),), float("nan"), device="cuda")
     dcu = torch.tensor(cu, dtype=torch.int32).cuda()
-    flat = state if form == "glr" else state.reshape(B + 2, -1)
-    K.chunk_scan(form, *args, out, flat, dcu, slots.cuda(), scratch, B, H, d, e, max(lens))
+
+    def on_device():                    # with the strides of the views
+        base = {}
+        def put(x):
+            b = x._base if x._base is not None else x
+            if id(b) not in base:
+                base[id(b)] = b.cuda()
+            return base[id(b)].as_strided(x.shape, x.stride(), x.storage_offset())
+        return {n: put(x) if torch.is_tensor(x) else x for n, x in i.items()}
+
+    def chunks(where, st, sl):
+        a = on_device()
+        K.chunk_scan(form, a.pop("q"), a.pop("k"), a.pop("v"), where, st, dcu, sl.cuda(), scratch, B, H, G, d, e, max(lens), **a)
+    chunks(out, state, slots)
     # float sums of at most T + d terms; the gates' own instructions are good to about an ulp of their argument's exponential
     got = out.double().cpu().reshape(T, H, e)
     assert float((got - want_o).abs().max()) < 3e-5 * float(want_o.abs().max())
@@ -73,13 +116,20 @@ def test_chunks_against_token_by_token(form, d, e, H, lens, strong):
     # no further off than the walk token by token
     state2, out2 = torch.zeros_like(state), torch.zeros_like(out)
     state2[1:B + 1] = as_kept(S, d).reshape((B,) + tuple(shape)).cuda()
-    scan = K.glr_scan if form == "glr" else K.wkv_scan
-    scan(*args, out2, state2 if form == "glr" else state2.reshape(B + 2, -1), dcu, slots.cuda(), B, H, d, e)
+    a = on_device()
+    if form == "glr":
+        K.glr_scan(torch.cat([a["q"], a["k"], a["v"]], 1), a["b1"], a["b2"], out2, state2, dcu, slots.cuda(), B, H, d, e)
+    elif form == "wkv":
+        K.wkv_scan(torch.cat([a["q"], a["k"], a["v"], a["z"]], 1), a["b1"], a["b2"], out2, state2.reshape(B + 2, -1), dcu, slots.cuda(), B, H, d, e)
+    elif form == "fixed":
+        K.dr_scan(a["q"], a["k"], a["v"], None, a["b1"], out2, state2, dcu, slots.cuda(), B, H, G, d, e, silu=a["silu"])
+    else:
+        K.dr_scan(a["q"], a["k"], a["v"], a["gb"], None, out2, state2, dcu, slots.cuda(), B, H, G, d, e, gc=a.get("gc"))
     err = lambda x: float((x.double().cpu().reshape(T, H, e) - want_o).norm())
     assert err(out) < 1.5 * err(out2) + 1e-7 * float(want_o.norm())
     # a padding sequence: its state is left alone, its rows are zeros where the walk token by token writes zeros
     slots[0] = -1
     out.fill_(7.0)
     before = state.clone()
-    K.chunk_scan(form, *args, out, flat, dcu, slots.cuda(), scratch, B, H, d, e, max(lens))
+    chunks(out, state, slots)
     assert torch.equal(state[1], before[1]) and torch.all(out[:lens[0]] == (7.0 if form == "glr" else 0.0))
