@@ -213,12 +213,11 @@ class Engine:
                     K.gather_rows(all_logits, which, logits)
             else:
                 try:
-                    step = pack_step(slots, token_lists, starts, self.device, self.ws, position_ids=position_ids)
+                    step = pack_step(slots, token_lists, starts, self.device, self.ws, position_ids=position_ids,
+                                     want=rows)
                 except ValueError as e:
                     raise StepError(str(e)) from None
-                want_rows = (torch.tensor(rows, dtype=torch.int32).to(self.device) if n_want
-                             else torch.empty(0, dtype=torch.int32, device=self.device))
-                logits = self.model.forward(step, self.cache, want_rows, n_want, probe=probe)
+                logits = self.model.forward(step, self.cache, step.want_rows, n_want, probe=probe)
         except BaseException:
             self.cache.release_reserved(slots, held)
             raise

@@ -64,6 +64,7 @@ class StepBatch:
     # what the position encodings read: [T], the same tensor as `positions` unless the caller gave
     # position numbers of its own, which may be k per token: [T, k]
     position_ids: Optional[torch.Tensor] = None
+    want_rows: Any = None            # int32 [wanted]: the packed rows whose logits the caller asked for
     probe: Any = None                # probe(name, tensor) of the running step, or None
     schedule_index: int = 0          # place in the run order of the layer that is running
 
@@ -73,8 +74,11 @@ class StepBatch:
 
 
 def pack_step(slots: Sequence[int], token_lists: Sequence[Sequence[int]], starts: Sequence[int],
-              device, ws: Workspace, pad_seqs: int = 0, position_ids: Optional[Sequence] = None) -> StepBatch:
-    """Build the device arrays of a step in one host-to-device copy.  `pad_seqs` extra
+              device, ws: Workspace, pad_seqs: int = 0, position_ids: Optional[Sequence] = None,
+              want: Sequence[int] = ()) -> StepBatch:
+    """Build the device arrays of a step in one host-to-device copy, from pinned memory and in stream order: the host does
+    not wait for the steps before (with two copies that waited, the GPU stood idle while a step's first kernels
+    were prepared and launched).  `want`: the packed rows whose logits are wanted (`step.want_rows`).  `pad_seqs` extra
     sequences of one dummy token (slot -1, position 0) may follow the real ones.
     `position_ids`: per sequence the position numbers of its tokens for the position
     encodings, one integer or k integers per token (the same k for all); None: each token's
@@ -100,9 +104,16 @@ def pack_step(slots: Sequence[int], token_lists: Sequence[Sequence[int]], starts
         if any(r.shape[1] != k for r in rows) or k == 0:
             raise ValueError("position_ids: every token needs the same number of position numbers")
         pid = np.concatenate(rows + [np.zeros((pad_seqs, k), dtype=np.int64)]).reshape(-1)
-    # layout of the one int32 staging array: tokens | positions | seq_of_token | cu | slots | ctx | position ids
-    flat = np.concatenate([toks, pos, sot, cu, np.asarray(all_slots, dtype=np.int64), ctx, pid]).astype(np.int32)
-    dev = torch.from_numpy(flat).to(device)
+    # layout of the one int32 staging array: tokens | positions | seq_of_token | cu | slots | ctx | position ids | wanted rows
+    parts = [toks, pos, sot, cu, np.asarray(all_slots, dtype=np.int64), ctx, pid, np.asarray(want, dtype=np.int64).reshape(-1)]
+    n_flat = sum(p.size for p in parts)
+    if torch.device(device).type == "cuda":
+        # torch's pinned allocator hands a block out again only behind the copies that read it
+        staged = torch.empty(n_flat, dtype=torch.int32, pin_memory=True)
+        np.concatenate(parts, out=staged.numpy(), casting="unsafe")
+        dev = staged.to(device, non_blocking=True)
+    else:
+        dev = torch.from_numpy(np.concatenate(parts).astype(np.int32)).to(device)
     o = 0
 
     def take(n):
@@ -116,9 +127,10 @@ def pack_step(slots: Sequence[int], token_lists: Sequence[Sequence[int]], starts
     if k:
         pid_d = take(T * k)
         pid_d = pid_d if k == 1 else pid_d.view(T, k)
+    want_d = take(len(want))
     max_ctx = int(ctx.max()) if B else 0
     return StepBatch(
         n_tokens=T, n_seqs=B, tokens=tokens, positions=positions, seq_of_token=seq_of_token,
         cu_seqlens=cu_seqlens, slots=slots_d, ctx_lens=ctx_d, host_slots=all_slots, host_new=new,
         host_start=all_starts, is_decode=all(n == 1 for n in new), max_new=max(new) if new else 0,
-        max_ctx=max_ctx, max_ctx_bound=max_ctx, ws=ws, position_ids=pid_d)
+        max_ctx=max_ctx, max_ctx_bound=max_ctx, ws=ws, position_ids=pid_d, want_rows=want_d)
