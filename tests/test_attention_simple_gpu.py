@@ -1,0 +1,46 @@
+"""attention_simple: a query alone (four waves, a class of key chunks each) and among many (one wave for all classes) gives the
+same bits, at context lengths around the chunks and classes, with and without a window."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hd,window", [(128, None), (128, 100), (48, None), (24, 70), (320, 300), (6, None)])
+def test_alone_and_among_many(dtype, hd, window):
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(hd)
+    page, T, nq, nkv = 64, 600, 2, 1
+    q, k, v = (torch.randn(T, n, hd, generator=g).to(dtype) for n in (nq, nkv, nkv))
+    n_pages = -(-T // page)
+    cache = torch.full((n_pages, 2, nkv, page, hd), float("nan"), dtype=dtype)        # rows not written are never read
+    pages = torch.randperm(n_pages, generator=g).tolist()
+    for t in range(T):
+        cache[pages[t // page], 0, :, t % page] = k[t]
+        cache[pages[t // page], 1].view(nkv, hd, page)[:, :, t % page] = v[t]
+    cache, table = cache.cuda(), torch.tensor([pages], dtype=torch.int32).cuda()
+    qd = q.reshape(T, nq * hd).cuda()
+    pos = torch.arange(T, dtype=torch.int32).cuda()
+    zeros, slots = torch.zeros(20000, dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+
+    def run(rows):
+        out = torch.empty(len(rows), nq * hd, dtype=dtype, device="cuda")
+        K.attention_simple(qd[rows].contiguous(), nq * hd, out, pos[rows].contiguous(), zeros[:len(rows)], slots, table, cache, len(rows),
+                           nq, nkv, hd, page, window, 1 / math.sqrt(hd))
+        return out
+    some = [0, 1, 62, 63, 64, 65, 127, 128, 191, 192, 255, 256, 257, 319, 320, 511, 512, 599]
+    many = torch.arange(T).repeat(20)
+    whole = run(many.cuda())
+    for t in some:
+        assert torch.equal(run(torch.tensor([t]).cuda())[0], whole[t])
+    kd, vd = k[:, 0].double(), v[:, 0].double()
+    for t in some:
+        lo = 0 if window is None else max(0, t - window + 1)
+        for h in range(nq):
+            w = torch.softmax((kd[lo:t + 1] @ q[t, h].double()) / math.sqrt(hd), 0)
+            want = w @ vd[lo:t + 1]
+            tol = 2e-6 if dtype == torch.float32 else 2 ** -8
+            assert float((whole[t, h * hd:(h + 1) * hd].double().cpu() - want).abs().max()) < tol * max(1.0, float(want.abs().max())) * 2
