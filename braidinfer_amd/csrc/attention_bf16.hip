@@ -756,10 +756,14 @@ __device__ __forceinline__ int kswz(int row, int cols) {      // the 16 key rows
 // kernel less per layer).  `q` then points at the step's raw rows [q heads | k heads | v
 // heads]; sequence b's token stands at position ctx - 1 and its angles in row b of cs / sn
 // ([B, HD / 2], pairs (p, p + HD / 2); null = no rotation).  Every workgroup rotates its
-// query heads in registers; the workgroup whose run holds the last page first stores the
-// rotated key and the value of the new token in that page (when `write_cache`), and waits
-// for the stores before the page is fetched.  For groups of up to 16 heads, so that one
-// workgroup alone reads that page.
+// query heads in registers; the workgroup whose run holds the last page puts the rotated key and
+// the value of the new token into that page's stage when the page has come (when `write_cache`),
+// and stores the key's row and the 64-byte piece of each value row that the token lies in from there.
+// (Its value is 2 bytes in each of HD lines of the cache.  Stored by themselves, before the page was
+// fetched, they cost the memory a read and a write each: 71.4 against 64.6 us a launch for 64 sequences
+// of 128 to 2,048 tokens with 8 kv heads of 128, 122 against 113 for 128; 60.5 and 100 without a store;
+// pieces of 32 and 128 bytes 67.  Up to 24 sequences it makes no difference.)  For groups of up to 16
+// heads, so that one workgroup alone reads that page.
 // `qruns` (FUSE only; null = none): the step's raw rows have not been put together yet; they are
 // the sums of `runs` float matrices [B, (nq + 2 nkv) HD], `run_stride` elements apart, as a
 // product cut along k leaves them.  Every value read from `q` is then the runs' sum in run
@@ -842,6 +846,8 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
     }
     const size_t page_elems = (size_t)2 * nkv * PAGE * HD;
     const size_t k_off = (size_t)kvh * PAGE * HD, v_off = ((size_t)nkv + kvh) * PAGE * HD;
+    bool has_new = false;                            // this workgroup's last page gets the new token; threads 0.. hold
+    bf16 new_a = (bf16)0.f, new_b = (bf16)0.f;       // its rotated key in pairs (p, p + HD / 2), those after it its value
     if constexpr (FUSE) {
         constexpr int P = HD / 2;
         if (cs) {
@@ -863,9 +869,8 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
             }
         }
         const int last_pg = ctx > 0 ? (ctx - 1) / PAGE : -1;
-        if (write_cache && hb == 0 && last_pg >= pg_begin && last_pg < pg_end) {
-            const int off = (ctx - 1) % PAGE;
-            bf16* pg = cache + (size_t)bt[last_pg] * page_elems;
+        has_new = write_cache && hb == 0 && last_pg >= pg_begin && last_pg < pg_end;
+        if (has_new) {
             const size_t kcol = (size_t)(nq + kvh) * HD, vcol = kcol + (size_t)nkv * HD;
             // element `col` of sequence b's raw row, from the row or from the runs
             auto raw = [&](size_t col) -> bf16 {
@@ -887,19 +892,16 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
             if (tid < P) {
                 const float a = (float)raw(kcol + tid), bb = (float)raw(kcol + tid + P);
                 const float cc = cs ? cs[(size_t)b * P + tid] : 1.f, ss = cs ? sn[(size_t)b * P + tid] : 0.f;
-                pg[k_off + (size_t)off * HD + tid] = (bf16)(a * cc - bb * ss);
-                pg[k_off + (size_t)off * HD + tid + P] = (bf16)(a * ss + bb * cc);
-            } else if (tid < P + HD) {
-                const int d = tid - P;
-                pg[v_off + (size_t)d * PAGE + off] = raw(vcol + d);
-            }
+                new_a = (bf16)(a * cc - bb * ss);
+                new_b = (bf16)(a * ss + bb * cc);
+            } else if (tid < P + HD)
+                new_a = raw(vcol + tid - P);
         }
-        // __syncthreads below waits for these stores (they have reached the L2) before any page is fetched
     }
     // the query has arrived before the loop: a wait for it inside would also wait for the pages in flight
 #pragma unroll
     for (int s = 0; s < NB; ++s) asm volatile("" ::"v"(qf[s]));
-    if constexpr (FUSE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (FUSE) asm volatile("" ::"v"((int)__builtin_bit_cast(short, new_a)), "v"((int)__builtin_bit_cast(short, new_b)));
     __syncthreads();
 
     const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)dsm);
@@ -931,19 +933,10 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
 
     for (int j = 0; j < D; ++j)
         if (j < n_run) DEC_ISSUE(j);
-    for (int i = 0; i < n_run; ++i) {
-        // page i has landed when at most the loads of the pages after it are in flight
-        int after = n_run - 1 - i;
-        if (after > D - 1) after = D - 1;
-        if (after >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NDMA) : "memory");
-        else if (after == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();                 // every wave's part of page i is there; page i - 1 is done with
-        asm volatile("" ::: "memory");
-        if (i + D < n_run) DEC_ISSUE(i + D);
+    auto multiply = [&](int i) __attribute__((always_inline)) {       // page i of the run, which lies in its stage
         const unsigned char* st = dsm + (i % S) * STAGE;
         const int kb = (pg_begin + i) * PAGE + 32 * kh;        // position of this wave's first key
-        if (kb >= ctx || kb + 32 <= lo) continue;
+        if (kb >= ctx || kb + 32 <= lo) return;
         f32x4 s_acc[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -993,6 +986,48 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc_o[i2][r] *= corr;
             acc_o[i2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, acc_o[i2], 0, 0, 0);
+        }
+    };
+    for (int i = 0; i < n_run - has_new; ++i) {
+        // page i has landed when at most the loads of the pages after it are in flight
+        int after = n_run - 1 - i;
+        if (after > D - 1) after = D - 1;
+        if (after >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NDMA) : "memory");
+        else if (after == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                 // every wave's part of page i is there; page i - 1 is done with
+        asm volatile("" ::: "memory");
+        if (i + D < n_run) DEC_ISSUE(i + D);
+        multiply(i);
+    }
+    if constexpr (FUSE) {
+        if (has_new) {                                // the run's last page takes the new token before its turn
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int i = n_run - 1;
+            unsigned char* st = dsm + (i % S) * STAGE;
+            constexpr int P = HD / 2, VSEG = 4;       // 16-byte columns of a stored piece
+            const int off = (ctx - 1) % PAGE;
+            auto kat = [&](int d) { return (bf16*)(st + off * KROWB + (((d / 8) ^ kswz(off, KCOLS)) * 16)) + d % 8; };
+            if (tid < P) {
+                *kat(tid) = new_a;
+                *kat(tid + P) = new_b;
+            } else if (tid < P + HD) {
+                const int d = tid - P;
+                *((bf16*)(st + KB + d * 128 + (((off / 8) ^ ((d >> 1) & 7)) * 16)) + off % 8) = new_a;
+            }
+            __syncthreads();
+            bf16* pg = cache + (size_t)bts[i] * page_elems;
+            if (tid < KCOLS)
+                *(bf16x8*)(pg + k_off + (size_t)off * HD + tid * 8) = *(const bf16x8*)(st + off * KROWB + ((tid ^ kswz(off, KCOLS)) * 16));
+#pragma unroll
+            for (int j = 0; j < HD * VSEG / 256; ++j) {
+                const int row = (j * 256 + tid) / VSEG, col = off / (8 * VSEG) * VSEG + tid % VSEG;
+                *(bf16x8*)(pg + v_off + (size_t)row * PAGE + col * 8) =
+                    *(const bf16x8*)(st + KB + row * 128 + ((col ^ ((row >> 1) & 7)) * 16));
+            }
+            multiply(i);
         }
     }
 #undef DEC_ISSUE
