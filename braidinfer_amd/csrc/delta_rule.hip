@@ -686,13 +686,111 @@ __global__ __launch_bounds__(256) void dr_scan_kernel(const DrScan p) {
     if (LOCAL && MODE == DR_WEIGHTED && cb16 == 0 && tid == 0) p.piece_decay[(size_t)s * H + h] = decayed;
 }
 
+// The same walk, the same order of sums, for steps of single tokens: a lane asks for the rows it holds of k and q (and of the
+// channels' decays) straight from memory together with its part of the state, with no chunk in LDS and no barrier, so that a
+// compute unit holds twice the waves and each waits once.  Bound by the state, read and written once, and with silu by its
+// arithmetic, which the four columns' lanes repeat.  32 heads of 128 x 128 (us, the chunks' walk before / this):
+//     sequences   delta rule     weighted       channels       fixed with silu
+//     1           3.9 / 3.7      4.0 / 3.4      4.1 / 3.5      5.1 / 4.5
+//     8           9.4 / 8.6      9.7 / 8.2      11.3 / 8.5     13.4 / 12.5
+//     40          43 / 37.5      42 / 36        55 / 38        53 / 45
+//     64          64 / 58        62 / 57        87 / 59        86 / 66          (268 MB: 4.7 TB/s)
+// V4: k, q and the decays 16 bytes at a time.
+template <int RPL, int MODE, bool SILU, bool V4>
+__global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
+    constexpr bool DELTA = MODE == DR_DELTA || MODE == DR_CHANNELS, CHAN = MODE == DR_CHANNELS;
+    constexpr bool TOKEN_G = MODE != DR_FIXED;
+    const int H = p.H, d = p.d, e = p.e;
+    const int s = blockIdx.x, h = blockIdx.y, cb16 = blockIdx.z;
+    const int kh = h / (H / p.G);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cg = lane >> 4, g = lane & 15;
+    const int cb4 = cb16 * 4 + wave, c = cb4 * 4 + cg;
+    const int slot = p.slots[s];
+    const int t0 = p.cu_seqlens[s], t1 = p.cu_seqlens[s + 1];
+    const int ncb4 = (e + p.ones + 3) >> 2, he = H * e;
+    if (cb4 >= ncb4) return;                       // a wave's own matter: there is no barrier
+    const bool live = c < e, is_n = MODE == DR_WEIGHTED && p.ones && c == e;
+    float* orow = is_n ? p.n_out + (size_t)t0 * H + h : p.o + (size_t)t0 * he + h * e + c;
+    const size_t ostep = is_n ? H : he;
+    const bool writes = g == 0 && (live || is_n);
+    if (slot < 0) {
+        if (writes) for (int t = t0; t < t1; ++t, orow += ostep) orow[0] = 0.f;
+        return;
+    }
+    float* S = p.state + (size_t)slot * p.slot_stride + (((size_t)h * ncb4 + cb4) * RPL) * 64 + lane;
+    float st[RPL];
+#pragma unroll
+    for (int r = 0; r < RPL; ++r) st[r] = S[(size_t)r * 64];
+    const float g_fixed = TOKEN_G ? 1.f : p.g_head[h];
+    const float skip = (MODE == DR_WEIGHTED && p.skip && live) ? p.skip[h] : 0.f;
+    auto row = [&](float (&to)[RPL], const float* from, float pad) {
+#pragma unroll
+        for (int r4 = 0; r4 < RPL; r4 += 4) {
+            if (V4) {
+                const bool ok = g * RPL + r4 < d;
+                const f32x4 w = *(const f32x4*)(from + (ok ? g * RPL + r4 : 0));
+#pragma unroll
+                for (int x = 0; x < 4; ++x) to[r4 + x] = ok ? w[x] : pad;
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) to[r4 + x] = g * RPL + r4 + x < d ? from[g * RPL + r4 + x] : pad;
+            }
+        }
+    };
+    for (int t = t0; t < t1; ++t, orow += ostep) {
+        float kr[RPL], qr[RPL], cr[CHAN ? RPL : 4];
+        row(kr, p.k + (size_t)t * p.qk_stride + kh * d, 0.f);
+        row(qr, p.q + (size_t)t * p.qk_stride + kh * d, 0.f);
+        if constexpr (CHAN) row(cr, p.gc + ((size_t)t * H + h) * d, 1.f);
+        float vc = live ? p.v[(size_t)t * p.v_stride + h * e + c] : 0.f;
+        if (is_n) vc = 1.f;
+        float gt = g_fixed, beta = 1.f;
+        if (TOKEN_G) {
+            if (!CHAN) gt = p.gb[(size_t)t * p.gb_stride + h];
+            beta = p.gb[(size_t)t * p.gb_stride + H + h];
+        }
+        if (SILU) {
+#pragma unroll
+            for (int r = 0; r < RPL; ++r) {
+                const bool real = g * RPL + r < d;
+                kr[r] = real ? dr_silu(kr[r]) : 0.f;
+                qr[r] = real ? dr_silu(qr[r]) : 0.f;
+            }
+            vc = dr_silu(vc);
+        }
+        float u = vc;
+        if (DELTA) {
+            float part = 0.f;
+#pragma unroll
+            for (int r = 0; r < RPL; ++r) {
+                st[r] *= CHAN ? cr[CHAN ? r : 0] : gt;
+                part = fmaf(st[r], kr[r], part);
+            }
+            u = beta * (vc - dr_row16_sum(part));
+        } else if (MODE == DR_WEIGHTED)
+            u = beta * vc;
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < RPL; ++r) {
+            st[r] = DELTA ? fmaf(kr[r], u, st[r]) : fmaf(gt, st[r], kr[r] * u);
+            sum = fmaf(st[r], qr[r], sum);
+        }
+        sum = dr_row16_sum(sum);
+        if (MODE == DR_WEIGHTED) sum = fmaf(skip, vc, sum);
+        if (writes) orow[0] = sum;
+    }
+#pragma unroll
+    for (int r = 0; r < RPL; ++r) S[(size_t)r * 64] = st[r];
+}
+
 static inline int dr_rpl(int d) {
     const int r = (d + 15) / 16;
     return r <= 4 ? 4 : (r <= 8 ? 8 : (r <= 16 ? 16 : 32));
 }
 
 template <bool LOCAL>
-static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, hipStream_t s) {
+static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, int singles, hipStream_t s) {
     const int cols = a.e + a.ones, ncb4 = (cols + 3) / 4, rpl = dr_rpl(a.d);
     if (a.H <= 0 || a.H > 65535 || a.G <= 0 || a.H % a.G || a.d <= 0 || a.e <= 0 || a.d > 512 || (cols + 15) / 16 > 65535 || B > 0x7fffffff ||
         (a.ones != 0 && a.ones != 1) || a.qk_stride < (size_t)a.G * a.d || a.v_stride < (size_t)a.H * a.e ||
@@ -702,7 +800,12 @@ static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, hipStream_
         (LOCAL && (mode == DR_DELTA || mode == DR_CHANNELS)) || (LOCAL && mode == DR_WEIGHTED && !a.piece_decay))
         return BR_BAD_ARG;
     dim3 grid(B, a.H, (cols + 15) / 16);
+    const bool v4 = a.d % 4 == 0 && a.qk_stride % 4 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.gc) % 16) == 0;
 #define DR_GO(R, TC, M, A) do { \
+        if constexpr (!LOCAL) if (singles) { \
+            if (v4) dr_token_kernel<R, M, A, true><<<grid, 256, 0, s>>>(a); else dr_token_kernel<R, M, A, false><<<grid, 256, 0, s>>>(a); \
+            break; \
+        } \
         const size_t lds = (size_t)((M == DR_CHANNELS ? 6 : 4) * TC * R * 16 + 2 * TC * 16 + 2 * TC * 2) * sizeof(float); \
         dr_scan_kernel<R, TC, M, A, LOCAL><<<grid, 256, lds, s>>>(a); \
     } while (0)
@@ -721,15 +824,16 @@ static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, hipStream_
 }
 
 // `mode`: DR_FIXED with `g_head`, DR_DELTA and DR_WEIGHTED with `gb`, DR_CHANNELS with `gb` and `gc`.  `silu` 1 (DR_FIXED):
-// q, k, v pass silu.
+// q, k, v pass silu.  `singles` 1: no more tokens than sequences, as in steps of single tokens (a longer sequence among them
+// is walked just as well, only without its next tokens' rows on their way).
 extern "C" int br_dr_scan(const float* q, const float* k, size_t qk_stride, const float* v, size_t v_stride, const float* gb,
                           size_t gb_stride, const float* g_head, const float* gc, const float* skip, float* o, float* n_out,
                           float* state, size_t slot_stride, const int* cu_seqlens, const int* slots, int B, int H, int G, int d,
-                          int e, int mode, int ones, int silu, hipStream_t s) {
+                          int e, int mode, int ones, int silu, int singles, hipStream_t s) {
     if (B <= 0) return BR_OK;
     const DrScan a = {q, k, v, gb, g_head, gc, skip, o, n_out, state, nullptr, cu_seqlens, slots, qk_stride, v_stride, gb_stride, slot_stride,
                       H, G, d, e, ones};
-    return dr_scan_launch<false>(a, B, mode, silu, s);
+    return dr_scan_launch<false>(a, B, mode, silu, singles, s);
 }
 
 // Between the two passes over a prompt cut into `pieces` pieces per sequence, for the outer sums: from the
@@ -779,11 +883,11 @@ extern "C" int br_dr_scan_pieces(const float* q, const float* k, size_t qk_strid
     if ((long long)H * ncb4 > 65535 || slot_stride < piece_stride) return BR_BAD_ARG;
     const DrScan a = {q, k, v, gb, g_head, nullptr, skip, o, n_out, piece_state, piece_decay, piece_cu, piece_slots, qk_stride, v_stride,
                       gb_stride, piece_stride, H, G, d, e, ones};
-    int rc = dr_scan_launch<true>(a, B * pieces, mode, silu, s);
+    int rc = dr_scan_launch<true>(a, B * pieces, mode, silu, 0, s);
     if (rc != BR_OK) return rc;
     dr_carry_kernel<<<dim3(B, H * ncb4), 64, 0, s>>>(state, slot_stride, slots, piece_state, piece_stride, piece_cu, g_head,
                                                      mode == DR_WEIGHTED ? piece_decay : nullptr, pieces, H, ncb4, rpl);
     rc = br_check_launch();
     if (rc != BR_OK) return rc;
-    return dr_scan_launch<false>(a, B * pieces, mode, silu, s);
+    return dr_scan_launch<false>(a, B * pieces, mode, silu, 0, s);
 }

@@ -859,9 +859,9 @@ def glr_scan(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional
         _req(v is None or (v.dtype == torch.float32 and v.numel() == H * d), "glr_scan: bias and lower bound float32 [H*d]")
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "glr_scan: arrays shorter than the batch")
     _req(d <= 512, f"glr_scan: {d} query channels a head are beyond the kernel's 512")
-    f = _fn("gated_recurrence", "br_glr_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, _P])
+    f = _fn("gated_recurrence", "br_glr_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, _P])
     _check(f(_ptr(rows), _ptr(f_bias), _ptr(lower), _ptr(out), _ptr(state), _ptr(cu_seqlens), _ptr(slots), B, H, d, e,
-             rows.shape[1], state.stride(0), _stream()), "glr_scan")
+             rows.shape[1], state.stride(0), int(T <= B), _stream()), "glr_scan")
 
 
 def glr_scan_pieces(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], out: torch.Tensor,
@@ -1173,9 +1173,10 @@ def dr_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gb: Optional[torc
     T = out.shape[0]
     qs = q.stride(0) if T > 1 else G * d
     vs = v.stride(0) if T > 1 else H * e
-    f = _fn("delta_rule", "br_dr_scan", [_P, _P, c_size_t, _P, c_size_t, _P, c_size_t] + [_P] * 6 + [c_size_t, _P, _P] + [c_int] * 8 + [_P])
+    f = _fn("delta_rule", "br_dr_scan", [_P, _P, c_size_t, _P, c_size_t, _P, c_size_t] + [_P] * 6 + [c_size_t, _P, _P] + [c_int] * 9 + [_P])
     _check(f(_ptr(q), _ptr(k), qs, _ptr(v), vs, _ptr(gb), 2 * H, _ptr(decay), _ptr(gc), _ptr(skip), _ptr(out), _ptr(n_out), _ptr(state),
-             state.stride(0), _ptr(cu_seqlens), _ptr(slots), B, H, G, d, e, mode, int(n_out is not None), int(bool(silu)), _stream()), "dr_scan")
+             state.stride(0), _ptr(cu_seqlens), _ptr(slots), B, H, G, d, e, mode, int(n_out is not None), int(bool(silu)), int(T <= B),
+             _stream()), "dr_scan")
 
 
 def dr_rotate_rows(q: torch.Tensor, k: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], rotary_dim: int,
