@@ -635,19 +635,33 @@ __device__ __forceinline__ int pwa_key_of_row(int c) { return 16 * (c >> 4) + 8 
 // One block of 32 keys (rows kb .. kb + 31 of a unit): `kblock` is the block's first key row (rows `ks` elements
 // apart), `vblock` the first value channel at the block's first row (channels `vs` elements apart), in the cache
 // or in LDS; rows of the block from `limit` on are not written and their values read as zero.  A key is seen by
-// this lane's query if first_ok <= key <= last_ok.
-template <int NBK, int NBV>
+// this lane's query if first_ok <= key <= last_ok.  EARLY: all of the block's keys and values are asked for before the
+// first product, without a branch between them (channels from dv on read the last row, and nobody writes what becomes of it;
+// a key row's elements from dk on, at most 127, are the next row's or the values' that follow the keys in a page, not used).
+template <int NBK, int NBV, bool EARLY = false>
 __device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int ks, const bf16* __restrict__ vblock, int vs,
                                           int kb, int limit, int first_ok, int last_ok, int dk, int dv, int c, int g,
                                           const bf16x8* qf, f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
     const bf16* krow = kblock + (size_t)pwa_key_of_row(c) * ks;
+    bf16x8 ke[EARLY ? 2 * NBK : 1], ve[EARLY ? 2 * NBV : 1];
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int s = 0; s < 2 * NBK; ++s)
+            ke[s] = *(const bf16x8*)(kblock + (unsigned)(pwa_key_of_row(c) * ks + 8 * g) + s * 16);
+#pragma unroll
+        for (int i = 0; i < 2 * NBV; ++i)
+            ve[i] = *(const bf16x8*)(vblock + (unsigned)(min(i / 2 * 32 + c, dv - 1) * vs + 8 * g) + (i & 1) * 16);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     f32x16 s_acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
 #pragma unroll
     for (int s = 0; s < 2 * NBK; ++s) {
         const int d = s * 16 + 8 * g;
-        const bf16x8 kf = (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
+        bf16x8 kf;
+        if constexpr (EARLY) kf = d < dk ? ke[s] : pwa_zero8();
+        else kf = (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
         s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], s_acc, 0, 0, 0);
     }
     if (cap_out != 0.f) {
@@ -696,7 +710,17 @@ __device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int k
         }
         const int ch = i * 32 + c;
         bf16x8 v1 = pwa_zero8(), v2 = pwa_zero8();
-        if (ch < dv) {
+        if constexpr (EARLY) {
+            v1 = ve[2 * i];
+            v2 = ve[2 * i + 1];
+            if (limit < 32) {                             // uniform
+#pragma unroll
+                for (int x = 0; x < 8; ++x) {
+                    if (8 * g + x >= limit) v1[x] = (bf16)0.f;
+                    if (16 + 8 * g + x >= limit) v2[x] = (bf16)0.f;
+                }
+            }
+        } else if (ch < dv) {
             const bf16* vrow = vblock + (size_t)ch * vs;
             v1 = pwa_load_vt8(vrow, 8 * g, limit);
             v2 = pwa_load_vt8(vrow, 16 + 8 * g, limit);
@@ -825,11 +849,13 @@ __global__ __launch_bounds__(256, ((NBK <= 4 && NBV <= 4) ? 2 : 1)) void pwa_pre
 // head are the columns of the score blocks (G <= 32; the other columns idle), so the keys and values of a kv
 // head are read once for all of its query heads.  The blocks of 32 keys the token sees (pooled rows first,
 // then its window) are dealt to the waves in turn; each wave runs the online softmax over its blocks
-// (wave 0 starts with the sink), and the waves' (m, l, O) are merged through LDS in wave order.  Eight waves:
-// a wave's blocks follow one another with their loads' latencies in between (8 sequences that hold 1,024
-// tokens: 31 us against 37 with four waves; 64 sequences: 102 against 92).
+// (wave 0 starts with the sink), and the waves' (m, l, O) are merged through LDS in wave order.  Where that leaves
+// compute units idle the value channels are dealt to several workgroups (blockIdx.z), each of which forms all the scores, with
+// the same bits.  Bound by the latency of a block's reads, which is why they are asked for together (EARLY).  Eight waves:
+// a wave's blocks follow one another with their loads' latencies in between (with one read after the other, 8 sequences that
+// hold 1,024 tokens: 31 us against 37 with four waves; 64 sequences: 102 against 92).
 #define PWA_DW 8
-template <int NBK, int NBV>
+template <int NBK, int NBV, bool EARLY>
 __global__ __launch_bounds__(64 * PWA_DW) void pwa_decode_kernel(
     const bf16* __restrict__ q, bf16* __restrict__ out, const int* __restrict__ slots,
     const int* __restrict__ ctx_lens, const int* __restrict__ block_table, int table_stride,
@@ -838,13 +864,15 @@ __global__ __launch_bounds__(64 * PWA_DW) void pwa_decode_kernel(
     int chunk, int keep, float softcap) {
     extern __shared__ float lds[];
     const int b = blockIdx.y, kvh = blockIdx.x;
+    const int ch0 = blockIdx.z * NBV * 32;     // this workgroup's share of the value channels
     const int slot = slots[b];
     const int G = nq / nkv;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 31, g = lane >> 5;
     const bool row_ok = c < G;
     const int head = kvh * G + (row_ok ? c : G - 1);
     if (slot < 0) {       // padding: no cache behind it
+        if (blockIdx.z) return;
         for (int i = threadIdx.x; i < G * dv; i += 64 * PWA_DW) out[((size_t)b * nq + kvh * G) * dv + i] = (bf16)0.f;
         return;
     }
@@ -887,7 +915,8 @@ __global__ __launch_bounds__(64 * PWA_DW) void pwa_decode_kernel(
         const bf16* pg = far ? pooled + (size_t)pt[kb / PWA_PAGE] * page_elems : storage + (size_t)bt[kb / PWA_PAGE] * page_elems;
         const int limit = (far ? ctx / pool : ctx) - (kb - kl);
         const int first_ok = row_ok ? ((far || early) ? 0 : lo) : 1, last_ok = row_ok ? (far ? seen - 1 : (early ? kept - 1 : pq)) : 0;
-        pwa_block<NBK, NBV>(pg + k_off + (size_t)kl * dk, dk, pg + v_off + kl, PWA_PAGE, kb, limit - kl, first_ok, last_ok, dk, dv, c, g,
+        pwa_block<NBK, NBV, EARLY>(pg + k_off + (size_t)kl * dk, dk, pg + v_off + (size_t)ch0 * PWA_PAGE + kl, PWA_PAGE, kb, limit - kl, first_ok, last_ok,
+                                   dk, dv - ch0, c, g,
                             qf, acc_o, m, lsum, scale2, cap_in, cap_out);
     }
     lsum += __shfl_xor(lsum, 32, 64);
@@ -922,7 +951,7 @@ __global__ __launch_bounds__(64 * PWA_DW) void pwa_decode_kernel(
     for (int i = 0; i < NBV; ++i)
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
-            const int d = i * 32 + 8 * r4 + 4 * g;
+            const int d = ch0 + i * 32 + 8 * r4 + 4 * g;
             if (d < dv) {
                 bf16x4 o;
 #pragma unroll
@@ -943,8 +972,8 @@ static int pwa_decode_launch_v(int nbv, dim3 grid, size_t lds_of_nbv16, hipStrea
                                int nq, int nkv, int dk, int dv, int size, int pool, float scale, int sink, const float* __restrict__ sinks, size_t head_lds, int cache_heads,
                                int chunk, int keep, float softcap) {
     // merges beyond 64 KB of LDS (many query heads to a kv head with wide values) are asked for once per kernel
-#define PWA_GO(V) do { \
-        auto kern = pwa_decode_kernel<NBK, V>; \
+#define PWA_GO(V, E) do { \
+        auto kern = pwa_decode_kernel<NBK, V, E>; \
         const size_t lds = head_lds + lds_of_nbv16 * V; \
         static size_t have = 65536; \
         if (lds > have) { \
@@ -953,11 +982,31 @@ static int pwa_decode_launch_v(int nbv, dim3 grid, size_t lds_of_nbv16, hipStrea
         } \
         kern<<<grid, 64 * PWA_DW, lds, s>>>(q, out, slots, ctx, bt, ts, st, pt, ps, pl, nq, nkv, dk, dv, size, pool, scale, sink, sinks, cache_heads, chunk, keep, softcap); \
     } while (0)
-    if (nbv <= 1) PWA_GO(1);
-    else if (nbv <= 2) PWA_GO(2);
-    else if (nbv <= 3) PWA_GO(3);
-    else if (nbv <= 4) PWA_GO(4);
-    else PWA_GO(8);
+    // Value channels of a workgroup, in blocks of 32: as few as keep the workgroups within a quarter more than the compute
+    // units; beyond, all of them, or two blocks of five and more while that makes at most two workgroups a compute unit.
+    // us (128 x 128: contexts of 65 to 1,203, 8 kv heads, window 512; 256 x 224: one row a token for 32 heads, two workgroups of
+    // 16 heads a sequence, as a captured step runs them; "was": all channels in one workgroup, asked for one after the other):
+    //     sequences         1     6     16    40    64    128   256
+    //     128 x 128  was    20.1  24.0  24.5  45.1  58.9  105   203
+    //                1      10.2  11.1  18.4  40.3  62.4  118   245
+    //                2      12.9  13.8  14.2  35.8  50.8  100   203
+    //                4      18.1  18.8  19.1  32.8  42.3  78    150
+    //     256 x 224  was    63.9  64.6  64.7  65.6  67.6  88    126
+    //                1      25.3  25.8  26.2  50.3  72.2  125   240
+    //                2      29.1  29.4  29.5  34.9  50.7  80    159
+    //                all    61.0  61.4  62.1  63.2  64.5  84    120
+    const long long cus = br_device_cus(), wgs = (long long)grid.x * grid.y;
+    auto parts = [&](int part) { return (nbv + part - 1) / part; };
+    int part = nbv;
+    if (4 * wgs * parts(1) <= 5 * cus) part = 1;
+    else if (4 * wgs * parts(2) <= 5 * cus || (nbv > 4 && wgs * parts(2) <= 2 * cus)) part = 2;
+    grid.z = parts(part);
+    // wide keys leave no registers to ask for more than two blocks of values early
+    if (part <= 1) PWA_GO(1, true);
+    else if (part <= 2) PWA_GO(2, true);
+    else if (part <= 3) PWA_GO(3, (NBK <= 4));
+    else if (part <= 4) PWA_GO(4, (NBK <= 4));
+    else PWA_GO(8, false);
 #undef PWA_GO
     return br_check_launch();
 }
