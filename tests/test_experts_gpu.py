@@ -129,3 +129,20 @@ def test_products_of_many_tokens(T, top, E, W, F, how, identity, alpha):
         assert float((got - want)[real].norm() / want[real].norm()) < 1e-3 + rounding
         if identity:                               # rows behind the experts' pairs are nobody's
             assert torch.all(out[int(first[E]):] == 7.0)
+
+
+@pytest.mark.parametrize("top", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("W", [4, 1028, 30])
+def test_combine_adds_every_slot(top, W):
+    """Outputs asked for eight slots at a time: numbers of slots around that, widths with and without 16-byte reads."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(top)
+    T = 5
+    out, share, x = torch.randn(T * top, W, generator=g), torch.rand(T, top, generator=g), torch.randn(T, W, generator=g)
+    place = torch.randperm(T * top, generator=g)
+    terms = share[:, :, None].double() * out[place].reshape(T, top, W).double()
+    for store in (False, True):
+        got = x.cuda()
+        K.experts_combine(out.cuda(), place.int().cuda(), share.cuda(), got, store=store)
+        want = terms.sum(1) + (0 if store else x.double())
+        assert ((got.cpu().double() - want).abs() <= (top + 1) * 2 ** -23 * (terms.abs().sum(1) + x.abs().double())).all()
