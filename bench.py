@@ -76,7 +76,8 @@ LAUNCHERS = ["embedding", "rmsnorm", "layernorm", "scale_", "rope_table", "rope_
              "latent_prepare", "head_linear", "route_topk", "experts_up", "experts_down", "experts_sort", "experts_gather",
              "experts_combine", "experts_up_grouped", "experts_down_grouped", "experts_gemm", "clamped_glu", "add_bias_rows",
              "add_position_rows", "pwa_gate", "dr_conv_prepare", "dr_scan", "dr_scan_pieces", "silu_rows", "pwa_pair_combine",
-             "route_sigmoid", "dr_rotate_rows", "route_softmax", "rows_into", "streams_spread", "streams_open", "streams_join", "ssm_prepare", "exp_gates"]
+             "route_sigmoid", "dr_rotate_rows", "route_softmax", "rows_into", "streams_spread", "streams_open", "streams_join", "ssm_prepare", "exp_gates",
+             "experts_up_tiles", "chunk_scan"]
 
 
 def kernel_share(torch, eng, entries_of, classes):
