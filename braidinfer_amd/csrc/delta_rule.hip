@@ -688,13 +688,14 @@ __global__ __launch_bounds__(256) void dr_scan_kernel(const DrScan p) {
 
 // The same walk, the same order of sums, for steps of single tokens: a lane asks for the rows it holds of k and q (and of the
 // channels' decays) straight from memory together with its part of the state, with no chunk in LDS and no barrier, so that a
-// compute unit holds twice the waves and each waits once.  Bound by the state, read and written once, and with silu by its
-// arithmetic, which the four columns' lanes repeat.  32 heads of 128 x 128 (us, the chunks' walk before / this):
+// compute unit holds twice the waves and each waits once.  Bound by the state, read and written once; silu of k and q is
+// formed once for the four columns of a wave (each forming its own: 45 and 66 us where 37 and 58 stand below).  32 heads of
+// 128 x 128 (us, the chunks' walk before / this):
 //     sequences   delta rule     weighted       channels       fixed with silu
-//     1           3.9 / 3.7      4.0 / 3.4      4.1 / 3.5      5.1 / 4.5
-//     8           9.4 / 8.6      9.7 / 8.2      11.3 / 8.5     13.4 / 12.5
-//     40          43 / 37.5      42 / 36        55 / 38        53 / 45
-//     64          64 / 58        62 / 57        87 / 59        86 / 66          (268 MB: 4.7 TB/s)
+//     1           3.9 / 3.7      4.0 / 3.4      4.1 / 3.5
+//     8           9.4 / 8.6      9.7 / 8.2      11.3 / 8.5
+//     40          43 / 37.5      42 / 36        55 / 38        53 / 37
+//     64          64 / 58        62 / 57        87 / 59        86 / 58          (268 MB: 4.7 TB/s)
 // V4: k, q and the decays 16 bytes at a time.
 template <int RPL, int MODE, bool SILU, bool V4>
 __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
@@ -740,8 +741,38 @@ __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
     };
     for (int t = t0; t < t1; ++t, orow += ostep) {
         float kr[RPL], qr[RPL], cr[CHAN ? RPL : 4];
-        row(kr, p.k + (size_t)t * p.qk_stride + kh * d, 0.f);
-        row(qr, p.q + (size_t)t * p.qk_stride + kh * d, 0.f);
+        if constexpr (SILU) {
+            // the four columns' lanes of a row group read a quarter each of its k and q, and share what silu made of it
+            __shared__ __attribute__((aligned(16))) float kq[4][2][16 * RPL];
+            constexpr int N = RPL / 2;
+            const int r0 = g * RPL + (cg & 1) * N;
+            const float* from = (cg < 2 ? p.k : p.q) + (size_t)t * p.qk_stride + kh * d;
+            float part[N];
+            if constexpr (V4 && N % 4 == 0) {
+#pragma unroll
+                for (int r4 = 0; r4 < N; r4 += 4) {
+                    const f32x4 w = *(const f32x4*)(from + (r0 + r4 < d ? r0 + r4 : 0));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) part[r4 + x] = w[x];
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < N; ++r) part[r] = r0 + r < d ? from[r0 + r] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < N; ++r) kq[wave][cg >> 1][r0 + r] = r0 + r < d ? dr_silu(part[r]) : 0.f;
+            __builtin_amdgcn_wave_barrier();               // the wave's own piece of LDS: its writes, then its reads, in order
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int r = 0; r < RPL; ++r) {
+                kr[r] = kq[wave][0][g * RPL + r];
+                qr[r] = kq[wave][1][g * RPL + r];
+            }
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            row(kr, p.k + (size_t)t * p.qk_stride + kh * d, 0.f);
+            row(qr, p.q + (size_t)t * p.qk_stride + kh * d, 0.f);
+        }
         if constexpr (CHAN) row(cr, p.gc + ((size_t)t * H + h) * d, 1.f);
         float vc = live ? p.v[(size_t)t * p.v_stride + h * e + c] : 0.f;
         if (is_n) vc = 1.f;
@@ -750,15 +781,7 @@ __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
             if (!CHAN) gt = p.gb[(size_t)t * p.gb_stride + h];
             beta = p.gb[(size_t)t * p.gb_stride + H + h];
         }
-        if (SILU) {
-#pragma unroll
-            for (int r = 0; r < RPL; ++r) {
-                const bool real = g * RPL + r < d;
-                kr[r] = real ? dr_silu(kr[r]) : 0.f;
-                qr[r] = real ? dr_silu(qr[r]) : 0.f;
-            }
-            vc = dr_silu(vc);
-        }
+        if (SILU) vc = dr_silu(vc);
         float u = vc;
         if (DELTA) {
             float part = 0.f;
