@@ -655,7 +655,15 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     // wave-load q of this wave: rows (4 q + wave) 8 .. + 8 of the operand's tile, reached by a 32-bit byte
-    // offset from the matrix's first element (the launcher checks that this suffices)
+    // offset from the matrix's first element (the launcher checks that this suffices); the pairs of an expert
+    // without `order`, of which a step may bring more than 4 GB, from the tile's first row
+    int row0 = 0;
+    if constexpr (GROUPED) {
+        if (!gr.order) {
+            A += (size_t)m0 * lda;
+            row0 = m0;
+        }
+    }
     unsigned offA[LA], offB[LB];
 #pragma unroll
     for (int q = 0; q < (LA > LB ? LA : LB); ++q) {
@@ -665,7 +673,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
             int r = m0 + R;
             if (r > M - 1) r = M - 1;
             if constexpr (GROUPED) {
-                if (gr.order) r = gr.order[r] / gr.top;
+                r = gr.order ? gr.order[r] / gr.top : r - row0;
             }
             offA[q] = (unsigned)((size_t)r * lda * 2 + c * 16);
         }
@@ -2182,7 +2190,7 @@ extern "C" int br_gemm_bf16_wide_parts(int M, int N, int K, int mode, size_t scr
 // ------------------------------------------- routed experts by the quad tiles -----
 // Steps whose (token, slot) pairs are grouped by expert: C[p, :] = W[e] A[p, :] for every expert's pairs, all
 // experts in one launch of gemm_tile_quad_kernel (GROUPED).  `gated`: W is [E][2 F][K], C bfloat16 [pairs, F] (N = 2 F), the
-// rows of A taken through `order`; else W is [E][N][K] and C float32 or bfloat16 [pairs, N].
+// rows of A taken through `order` (A below 4 GB); else W is [E][N][K] and C float32 or bfloat16 [pairs, N].
 extern "C" int br_experts_tiles_takes(int N, int K) { return N > 0 && K > 0 && N % 16 == 0 && K % DMA_BK == 0; }
 
 template <int BM, int BN, int NSA, int NSB, int WVM>
@@ -2225,7 +2233,7 @@ extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, 
     if (pairs <= 0) return BR_OK;
     const size_t ldc = gated ? (size_t)N / 2 : (size_t)N;
     if (!br_experts_tiles_takes(N, K) || E <= 0 || top <= 0 || (gated && !out_is_bf16) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 != 0 ||
-        !quad_takes(C, a_rows, N, K, K, ldc))
+        !quad_takes(C, order ? a_rows : min(a_rows, 256), N, K, K, ldc))
         return BR_BAD_ARG;
     const QuadGroups gr = {first, order, E, top, limit, alpha};
     const int mode = gated ? OUT_SWIGLU : out_is_bf16 ? OUT_BF16 : OUT_F32;

@@ -1458,9 +1458,16 @@ def experts_stream_takes(dtype: torch.dtype, W: int, F: int, pairs: int, experts
             and experts <= 512)
 
 
-def experts_tiles_take(dtype: torch.dtype, W: int, F: int) -> bool:
-    """Whether the prompt products' tiles take these experts (bfloat16, both widths in steps of 64)."""
-    return dtype == torch.bfloat16 and W % 64 == 0 and F % 64 == 0
+def _experts_gemm_tiles_take(N: int, Kd: int) -> bool:
+    """Steps of the widths, and an expert's matrix and a tile of 256 rows within the kernel's 32-bit byte offsets."""
+    return Kd % 64 == 0 and N % 16 == 0 and (max(N, 240) + 16) * Kd * 2 < 2 ** 32
+
+
+def experts_tiles_take(dtype: torch.dtype, W: int, F: int, tokens: int) -> bool:
+    """Whether the prompt products' tiles take both products of a step of `tokens` tokens (bfloat16, both widths in steps of
+    64, the rows h below 4 GB, which they are gathered from by 32-bit byte offsets)."""
+    return (dtype == torch.bfloat16 and W % 64 == 0 and F % 64 == 0 and tokens * W * 2 < 2 ** 32
+            and _experts_gemm_tiles_take(2 * F, W) and _experts_gemm_tiles_take(W, F))
 
 
 def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, order: torch.Tensor, y: torch.Tensor, top: int,
@@ -1470,7 +1477,8 @@ def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, o
     T, W = h.shape
     E, F2, _ = w_gu.shape
     n = order.numel()
-    _req(experts_tiles_take(h.dtype, W, F2 // 2) and w_gu.dtype == y.dtype == torch.bfloat16, "experts_up_tiles: bfloat16, widths in steps of 64")
+    _req(experts_tiles_take(h.dtype, W, F2 // 2, T) and w_gu.dtype == y.dtype == torch.bfloat16,
+         "experts_up_tiles: bfloat16, widths in steps of 64, rows below 4 GB")
     _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
          and first.dtype == order.dtype == torch.int32, "experts_up_tiles: shapes")
     f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
@@ -1486,7 +1494,7 @@ def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: tor
     E, N, _ = w.shape
     _req(a.dtype == w.dtype == torch.bfloat16 and Kd % 8 == 0 and w.shape == (E, N, Kd) and out.shape == (n, N)
          and first.dtype == torch.int32 and first.numel() in (E + 1, E + 2), "experts_gemm: bfloat16 [pairs, K] x [E, N, K], K in steps of 8")
-    if Kd % 64 == 0 and N % 16 == 0:
+    if _experts_gemm_tiles_take(N, Kd) and out.data_ptr() % 16 == 0:
         f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
         _check(f(_ptr(a), _ptr(w), _ptr(first), None, _ptr(out), 0, _is_bf16(out, "experts_gemm"), n, n, E, N, Kd, 1, 0.0, 0.0, _stream()),
                "experts_gemm")

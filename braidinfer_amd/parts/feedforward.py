@@ -285,7 +285,7 @@ class RoutedExperts(FeedForward):
         # beyond, the prompt products' tiles read them once for 128 or 256 (32 experts of 1,792 by 4,096, 8 chosen, both
         # products: 32 tokens 239 against 257 us, 40 tokens 257 against 256, 64 tokens 350 against 259).
         streamed = (T <= 16 or n <= 8 * self.E) and (few or K.experts_stream_takes(dt, self.H, self.I, n, self.E))
-        if K.experts_tiles_take(dt, self.H, self.I) and not streamed and not forced:
+        if K.experts_tiles_take(dt, self.H, self.I, T) and not streamed and not forced:
             y = step.ws.get("moe_y", (n, self.I), dt)
             K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             out = step.ws.get("moe_out", (n, self.H), torch.float32)
@@ -300,7 +300,7 @@ class RoutedExperts(FeedForward):
             K.experts_down_grouped(y, self.w_down, first, out, T)
             K.experts_combine(out, place, share, x, store=store, **ident)
             return
-        # widths that the tiles do not take, and the 32-bit path
+        # widths and steps that the tiles do not take, and the 32-bit path
         rows = step.ws.get("moe_rows", (n, self.H), dt)
         K.experts_gather(h, order, rows, self.top, n_rows=first[self.E:self.E + 1] if self.identity else None)
         gu = step.ws.get("moe_gu", (n, 2 * self.I), dt)

@@ -146,3 +146,25 @@ def test_combine_adds_every_slot(top, W):
         K.experts_combine(out.cuda(), place.int().cuda(), share.cuda(), got, store=store)
         want = terms.sum(1) + (0 if store else x.double())
         assert ((got.cpu().double() - want).abs() <= (top + 1) * 2 ** -23 * (terms.abs().sum(1) + x.abs().double())).all()
+
+
+def test_rows_beyond_4_gb():
+    """The second product of a step whose pairs' rows take more than 4 GB: the first and the last rows of every expert."""
+    from braidinfer_amd import kernels as K
+    Kd, N, n = 64, 16, 2 ** 25 + 700
+    g = torch.Generator(device="cuda").manual_seed(1)
+    starts = [0, 0, 300, 2 ** 25 - 131, 2 ** 25 + 200, n, n]
+    E = len(starts) - 1
+    first = torch.tensor(starts, dtype=torch.int32).cuda()
+    w = torch.randn(E, N, Kd, device="cuda", generator=g).to(torch.bfloat16)
+    a = torch.empty(n, Kd, dtype=torch.bfloat16, device="cuda")
+    for i in range(0, n, 2 ** 22):
+        a[i:i + 2 ** 22] = torch.randn(min(2 ** 22, n - i), Kd, device="cuda", generator=g)
+    out = torch.full((n, N), 7.0, device="cuda")
+    K.experts_gemm(a, w, first, out)
+    for e in range(E):
+        for lo, hi in {(starts[e], min(starts[e] + 400, starts[e + 1])), (max(starts[e], starts[e + 1] - 400), starts[e + 1])}:
+            if hi > lo:
+                want = a[lo:hi].double() @ w[e].double().T
+                # float sums of 64 products: 64 2^-24 of the terms' sum, which is about 50
+                assert float((out[lo:hi].double() - want).abs().max()) < 64 * 2 ** -24 * 50
