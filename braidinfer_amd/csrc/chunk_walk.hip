@@ -256,10 +256,10 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     const unsigned long long values64 = wave < 2 ? 0ull : ~0ull;
     unsigned long long block = (unsigned long long)blocks;
     const int vx = cb * CB + (CB == 2 ? wave & 1 : 0);        // the 16 columns this wave brings values of
-    const unsigned long long vbase = (unsigned long long)(v + (size_t)t0 * ldv + h * e + vx * 16);
+    unsigned long long vbase = (unsigned long long)(v + (size_t)t0 * ldv + h * e + vx * 16);      // the chunk's first row: rows of a prompt reach beyond 4 GB
     const unsigned vcol = ((lane & 3) ^ (lane >> 4)) * 16, uoff = (49 * D + 256) * 4 + vx * 1024 + lane * 16;
-    const int vlast = t1 - 1 - t0;
-    int vrow = lane >> 2, left = nch - 1, slot_i = 0;
+    const int vrow = lane >> 2;
+    int vlast = t1 - 1 - t0, left = nch - 1, slot_i = 0;      // the sequence's last row, counted from the chunk's first
     auto bring = [&](unsigned lds, unsigned off, unsigned long long base) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0", "memory");
     };
@@ -278,7 +278,8 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
               DELTA ? block : (block & ~values64) | (vbase & values64));
         const int go = left > 0;
         block += (unsigned long long)(go * H) * (unsigned)(BLOCK * 4);
-        vrow += go * CW_C;
+        vbase += (unsigned long long)(go * CW_C * 4) * (unsigned)ldv;
+        vlast -= go * CW_C;
         left -= go;
         slot_i = slot_i == S - 1 ? 0 : slot_i + 1;
     };
@@ -475,7 +476,7 @@ extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v,
     if (B <= 0 || T <= 0) return BR_OK;
     if (!br_chunk_takes(d, e) || H <= 0 || H > 65535 || B > 65535 || (long long)B * H > 0x7fffffffLL || e / 16 > 65535 || max_new <= 0 ||
         max_new > T || G <= 0 || H % G || form < CW_GLR || form > CW_DELTA || v_stride % 4 || ((uintptr_t)v | (uintptr_t)scratch) % 16 ||
-        v_stride > 0x7fffffff || (unsigned long long)max_new * v_stride * 4 >= (1ull << 32) || slot_stride < (size_t)H * ((e + 3) / 4) * d * 4 ||
+        v_stride >= (1ull << 26) || slot_stride < (size_t)H * ((e + 3) / 4) * d * 4 ||
         scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA) || (form == CW_WKV && (!z || !b1 || !b2)) ||
         (form == CW_FIXED && !b1) || (form == CW_DELTA && !gb) || ((form == CW_GLR || form == CW_WKV) && G != H))
         return BR_BAD_ARG;

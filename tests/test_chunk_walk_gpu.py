@@ -133,3 +133,21 @@ def test_chunks_against_token_by_token(form, d, e, H, lens, strong):
     before = state.clone()
     chunks(out, state, slots)
     assert torch.equal(state[1], before[1]) and torch.all(out[:lens[0]] == (7.0 if form == "glr" else 0.0))
+
+
+def test_values_beyond_4_gb():
+    """Values as columns of rows so wide that a prompt's reach over more than 4 GB: the same bits as of dense rows."""
+    from braidinfer_amd import kernels as K
+    T, H, d, e, wide = 300, 1, 64, 32, 2 ** 22
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(T, H * n, device="cuda", generator=g) for n in (d, d, e))
+    rows = torch.empty(T, wide, device="cuda")
+    rows[:, 8:8 + H * e] = v
+    decay, cu, slots = torch.full((H,), 0.95, device="cuda"), torch.tensor([0, T], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    got = []
+    for x in (v, rows[:, 8:8 + H * e]):
+        out, state = torch.zeros(T, H * e, device="cuda"), torch.zeros((1,) + tuple(K.glr_state_shape(H, d, e)), device="cuda")
+        scratch = torch.empty(K.chunk_scratch_floats(T, 1, H, d, e), device="cuda")
+        K.chunk_scan("fixed", q, k, x, out, state, cu, slots, scratch, 1, H, H, d, e, T, b1=decay)
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][0].abs().max() > 0
