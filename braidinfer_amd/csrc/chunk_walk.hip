@@ -15,7 +15,8 @@
 // same for all columns of the state and for all chunks at once, so `chunk_prepare` makes it for every (chunk, head) in
 // parallel, in the order in which a lane of the second kernel wants its operands; `chunk_walk` then walks the chunks of a
 // sequence in order, with S in the matrix cores' accumulators, which are at once the second operand of the read-out.  All
-// products and sums are float; against a walk token by token only their order differs.  Chunks are counted from the
+// products and sums are float; against a walk token by token only their order differs, and an infinite value or one that is
+// not a number shows from its token on, not before.  Chunks are counted from the
 // sequence's first token of the step; a chunk's tokens beyond the sequence have decay 1, write nothing and read nothing.
 //
 // What bounds it: the walk is a serial chain, a chunk of a head of 128 x 128 costing a wave 17 float matrix instructions (32
@@ -27,6 +28,7 @@
 #include "common.h"
 
 #define CW_C 16            // tokens of a chunk
+#define CW_FINITE 3.402823466e38f
 
 __device__ __forceinline__ float cw_row16_sum(float v) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
@@ -382,8 +384,15 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
                 for (int i = 0; i < 4; ++i) vv[x][i] = sf[32 * D + 512 + x * 256 + (4 * g + i) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
             }
         }
+        // A's zeros above the diagonal keep a token's value from the tokens before it only while it is finite: others pass here as
+        // zero and are added to their own and later tokens' sums below
+        unsigned long long odd = 0;
 #pragma unroll
-        for (int x = 0; x < CB; ++x) oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, va[x], oa[x], 0, 0, 0);
+        for (int x = 0; x < CB; ++x) {
+            const bool fine = fabsf(va[x]) <= CW_FINITE;
+            odd |= __ballot(!fine);
+            oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, fine ? va[x] : 0.f, oa[x], 0, 0, 0);
+        }
         if constexpr (!DELTA) read_out();
         issue();
 #pragma unroll
@@ -402,6 +411,16 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
 #pragma unroll
             for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = oa[x][r];
+        }
+        if (odd) {                                            // infinite or not a number: this wave's tokens 4 i + wave of A
+            for (int x = 0; x < CB; ++x) {
+                float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
+                for (int i = 0; i < 4; ++i) {
+                    const float u = __shfl(va[x], 16 * i + r16, 64);
+                    for (int r = 0; r < 4; ++r)
+                        if (!(fabsf(u) <= CW_FINITE) && 4 * i + wave <= 4 * g + r) pw[(4 * g + r) * 17 + r16] += sf[32 * D + (4 * g + r) * 16 + 4 * i + wave] * u;
+                }
+            }
         }
         if (!DELTA && ch > 0) flush(ch - 1);
         cur = cur == S - 1 ? 0 : cur + 1;

@@ -151,3 +151,46 @@ def test_values_beyond_4_gb():
         K.chunk_scan("fixed", q, k, x, out, state, cu, slots, scratch, 1, H, H, d, e, T, b1=decay)
         got.append((out, state))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][0].abs().max() > 0
+
+
+@pytest.mark.parametrize("form", ["glr", "wkv", "fixed", "delta"])
+@pytest.mark.parametrize("d,e", [(64, 16), (64, 64), (128, 128)])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_values_that_are_not_finite_show_from_their_token_on(form, d, e, bad):
+    """An infinite value, one that is not a number, at a token of a chunk: the tokens before it and the other columns keep their
+    bits, its own column shows it from its token on, as the walk token by token has it.  The same for a key, whose head shows it."""
+    from braidinfer_amd import kernels as K
+    T, H = 40, 2
+    g = torch.Generator().manual_seed(d + e)
+    i = {n: x.clone().cuda() if torch.is_tensor(x) else x for n, x in inputs(form, T, H, H, d, e, False, g).items()}
+    cu, slots = torch.tensor([0, T], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+
+    def run(**other):
+        a = dict(i, **other)
+        q, k, v = a.pop("q"), a.pop("k"), a.pop("v")
+        out, state = torch.zeros(T, H * e, device="cuda"), torch.zeros((1,) + tuple(K.glr_state_shape(H, d, e)), device="cuda")
+        scratch = torch.empty(K.chunk_scratch_floats(T, 1, H, d, e, form == "delta"), device="cuda")
+        if form == "wkv":                                    # q, k and z share a row stride
+            wide = torch.cat([q, k, a["z"]], 1)
+            q, k, a["z"] = (wide[:, n * H * d:(n + 1) * H * d] for n in range(3))
+        K.chunk_scan(form, q, k, v, out, state, cu, slots, scratch, 1, H, H, d, e, T, **a)
+        return out
+    clean = run()
+    assert clean.isfinite().all()
+    for t in (0, 5, 15, 16, 22, 35, 39):
+        c = (7 * t + 3) % e + e * (t % 2)
+        v = i["v"].clone()
+        v[t, c] = bad
+        got = run(v=v)
+        assert not got[t:, c].isfinite().any() and torch.equal(got[:t, c], clean[:t, c])
+        rest = torch.arange(H * e, device="cuda") != c
+        assert torch.equal(got[:, rest], clean[:, rest])
+        if form == "glr" and bad == float("inf"):            # a gate's sum of plus infinity is a decay of one
+            continue
+        k = i["k"].clone()
+        k[t, d * (t % 2) + 9] = bad
+        got = run(k=k)
+        head = slice(e * (t % 2), e * (t % 2) + e)
+        assert torch.equal(got[:t], clean[:t])
+        if bad != bad:
+            assert not got[t + 1:, head].isfinite().any()
