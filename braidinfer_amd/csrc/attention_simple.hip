@@ -30,10 +30,14 @@ template <> struct as_vec<bf16> { static constexpr int N = 8; typedef bf16x8 typ
 
 struct AsPart { float m, l, acc[MAX_DPL]; };            // a lane's channels lane, lane + 64, ..
 
+// What weights are taken relative to: the largest score so far, and while all of them are minus infinity (weight 0) or not a number
+// (which is to show in the sums) a finite one.
+__device__ __forceinline__ float as_base(float m) { return m == -INFINITY ? 0.f : m; }
+
 // onto `a` the keys that `b` summed: the recurrence's own step for more than one key
 __device__ __forceinline__ void as_join(AsPart& a, const AsPart& b) {
-    if (b.m == -INFINITY) return;
-    const float m = fmaxf(a.m, b.m), ca = expf(a.m - m), cb = expf(b.m - m);          // exp(-inf) = 0 on the first
+    if (b.m == -INFINITY && b.l == 0.f) return;
+    const float m = fmaxf(a.m, b.m), ca = expf(a.m - as_base(m)), cb = expf(b.m - as_base(m));          // exp(-inf) = 0 on the first
     a.l = fmaf(b.l, cb, a.l * ca);
 #pragma unroll
     for (int i = 0; i < MAX_DPL; ++i) a.acc[i] = fmaf(b.acc[i], cb, a.acc[i] * ca);
@@ -94,9 +98,9 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
                     for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], to_f32<T>(kr[d]), dot);
                 s = dot * scale;
             }
-            const float m_new = fmaxf(a.m, wave_max(s));
-            const float corr = expf(a.m - m_new);        // exp(-inf) = 0 on the first chunk
-            const float w = (j <= p) ? expf(s - m_new) : 0.f;
+            const float m_new = fmaxf(a.m, wave_max(s)), base = as_base(m_new);
+            const float corr = expf(a.m - base);         // exp(-inf) = 0 on the first chunk
+            const float w = (j <= p) ? expf(s - base) : 0.f;
             a.l = fmaf(a.l, corr, wave_sum(w));
             // `ps` is this wave's own: its reads of the chunk before are done, its writes wait here
             __builtin_amdgcn_wave_barrier();

@@ -44,3 +44,35 @@ def test_alone_and_among_many(dtype, hd, window):
             want = w @ vd[lo:t + 1]
             tol = 2e-6 if dtype == torch.float32 else 2 ** -8
             assert float((whole[t, h * hd:(h + 1) * hd].double().cpu() - want).abs().max()) < tol * max(1.0, float(want.abs().max())) * 2
+
+
+@pytest.mark.parametrize("keys", [(0, 64), (64, 128), (70, 90), (128, 192), (64, 320), (0, 320)])
+@pytest.mark.parametrize("what", ["not a number", "minus infinity"])
+def test_scores_that_are_not_finite(keys, what):
+    """Keys whose scores are not numbers show in every query that sees them, whichever chunks and classes they fill; scores of
+    minus infinity weigh nothing, unless there are no others.  A query alone and among many."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(2)
+    page, T, hd = 64, 320, 32
+    q, k, v = (torch.randn(T, hd, generator=g) for _ in range(3))
+    q[:, 0] = q[:, 0].abs() + 0.1
+    k[keys[0]:keys[1], 0] = float("nan") if what == "not a number" else float("-inf")
+    cache = torch.zeros(T // page, 2, 1, page, hd)
+    cache[:, 0, 0] = k.reshape(-1, page, hd)
+    cache[:, 1, 0].view(-1, hd, page)[:] = v.reshape(-1, page, hd).transpose(1, 2)
+    cache, table = cache.cuda(), torch.arange(T // page, dtype=torch.int32).reshape(1, -1).cuda()
+    zeros, slots = torch.zeros(20000, dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    qd, pos = q.cuda(), torch.arange(T, dtype=torch.int32).cuda()
+
+    def run(rows):
+        out = torch.empty(len(rows), hd, device="cuda")
+        K.attention_simple(qd[rows].contiguous(), hd, out, pos[rows].contiguous(), zeros[:len(rows)], slots, table, cache, len(rows),
+                           1, 1, hd, page, None, 1 / math.sqrt(hd))
+        return out.cpu()
+    whole = run(torch.arange(T).repeat(40).cuda())[:T]
+    for t in (0, 63, 64, 75, 127, 128, 200, 255, 256, 319):
+        want = torch.softmax((k[:t + 1].double() @ q[t].double()) / math.sqrt(hd), 0) @ v[:t + 1].double()
+        for got in (whole[t], run(torch.tensor([t]).cuda())[0]):
+            assert torch.equal(got.isnan(), want.isnan())
+            if not want.isnan().any():
+                assert float((got.double() - want).abs().max()) < 4e-6 * max(1.0, float(want.abs().max()))
