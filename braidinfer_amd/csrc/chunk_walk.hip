@@ -38,11 +38,17 @@ __device__ __forceinline__ float cw_row16_sum(float v) {
     return v;
 }
 
+template <int N>
+__device__ __forceinline__ double cw_sum(const float* x) {
+    if constexpr (N == 1) return x[0];
+    else return cw_sum<N / 2>(x) + cw_sum<N / 2>(x + N / 2);
+}
+
 // Where a sequence's chunks lie in the scratch: sequence s has room for ceil(tokens / 16) chunks from cu[s] / 16 + s on.
 __device__ __forceinline__ int cw_first(const int* cu, int s) { return cu[s] / CW_C + s; }
-// Floats of a (chunk, head) in the scratch: read factors 16 D | write factors 16 D | A 256 | decay D, and for the delta rule
-// -W 16 D | U 16 e.
-__host__ __device__ constexpr int cw_block(int D, int e, bool delta) { return 33 * D + 256 + (delta ? 16 * (D + e) : 0); }
+// Floats of a (chunk, head) in the scratch: read factors 16 D | write factors 16 D | A 256 | the chunk's decay D | what its
+// rounding left D, and for the delta rule -W 16 D | U 16 e.
+__host__ __device__ constexpr int cw_block(int D, int e, bool delta) { return 34 * D + 256 + (delta ? 16 * (D + e) : 0); }
 
 #define CW_GLR 0
 #define CW_WKV 1
@@ -136,26 +142,29 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
             ++pair;
         }
     }
-    // the factors: prefix products for what reads, suffix products for what writes
-    float p = 1.f, W[DELTA ? CW_C : 1];
+    // the factors: prefix products for what reads, suffix products for what writes, rounded to float once at their end
+    double p = 1.0;
+    float W[DELTA ? CW_C : 1];
 #pragma unroll
     for (int t = 0; t < CW_C; ++t) {
         if (!WKV) p *= w[t];
-        stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + t * 4 + (c & 3)] = q[t] * p;
-        if (DELTA) W[DELTA ? t : 0] = beta[DELTA ? t : 0] * (k[t] * p);
+        stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + t * 4 + (c & 3)] = (float)(q[t] * p);
+        if (DELTA) W[DELTA ? t : 0] = (float)(beta[DELTA ? t : 0] * (k[t] * p));
         if (WKV) p *= w[t];
     }
-    out[32 * D + 256 + c] = p;
-    p = 1.f;
+    // a decay that is the same in every chunk must not carry the same rounding error through all of them
+    out[32 * D + 256 + c] = (float)p;
+    out[33 * D + 256 + c] = (float)(p - (float)p);
+    p = 1.0;
 #pragma unroll
     for (int t = CW_C - 1; t >= 0; --t) {
         const float x = w[t];
-        w[t] = k[t] * p;
+        w[t] = (float)(k[t] * p);
         p *= x;
     }
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        const f32x4 v = {w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
+        const f32x4 v = {w[g], w[4 + g], w[8 + g], w[12 + g]};
         *(f32x4*)(out + 16 * D + (c >> 4) * 256 + (16 * g + (c & 15)) * 4) = v;
     }
     __syncthreads();
@@ -172,17 +181,14 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
         float sum = 0.f;
         if (j <= t) {
             const float* pp = part + (j * CW_C - j * (j - 1) / 2 + t - j) * (D / 16);
-#pragma unroll
-            for (int x = 0; x < D / 16; ++x) sum += pp[x];
+            sum = (float)cw_sum<D / 16>(pp);
         }
         out[32 * D + i] = sum;
         if (DELTA) {
             sum = 0.f;
             if (j < t) {
                 const float* pp = part + (136 + j * CW_C - j * (j - 1) / 2 + t - j - j - 1) * (D / 16);
-#pragma unroll
-                for (int x = 0; x < D / 16; ++x) sum += pp[x];
-                sum *= t < n ? in.gb[(size_t)(t0 + t) * 2 * H + H + h] : 0.f;
+                sum = t < n ? (float)(cw_sum<D / 16>(pp) * in.gb[(size_t)(t0 + t) * 2 * H + H + h]) : 0.f;
             }
             Lm[DELTA ? i : 0] = sum;
         }
@@ -191,14 +197,18 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
         __syncthreads();
         auto solve = [&](float (&x)[CW_C]) {                  // x_t -= sum_{s < t} L[t, s] x_s
 #pragma unroll
-            for (int t = 1; t < CW_C; ++t)
+            for (int t = 1; t < CW_C; ++t) {
+                float sum = 0.f;
 #pragma unroll
-                for (int j = 0; j < t; ++j) x[t] = fmaf(-Lm[t * 16 + j], x[j], x[t]);
+                for (int j = 0; j < t; ++j) sum = fmaf(Lm[t * 16 + j], x[j], sum);
+                x[t] -= sum;
+            }
         };
         solve(W);
+        // token t in row 4 (t % 4) + t / 4 of the product with S, so that its results lie as the state's update wants them
 #pragma unroll
-        for (int t = 0; t < CW_C; ++t) stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + t * 4 + (c & 3)] = -W[t];
-        float* uo = out + 49 * D + 256;
+        for (int t = 0; t < CW_C; ++t) stage[(c >> 4) * 272 + ((c >> 2) & 3) * 68 + (4 * (t & 3) + (t >> 2)) * 4 + (c & 3)] = -W[t];
+        float* uo = out + 50 * D + 256;
         for (int x = c; x < e; x += D) {
             float u[CW_C];
 #pragma unroll
@@ -206,18 +216,23 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
             solve(u);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const f32x4 v = {u[4 * g], u[4 * g + 1], u[4 * g + 2], u[4 * g + 3]};
+                const f32x4 v = {u[g], u[4 + g], u[8 + g], u[12 + g]};
                 *(f32x4*)(uo + (x >> 4) * 256 + (16 * g + (x & 15)) * 4) = v;
             }
         }
         __syncthreads();
-        unstage(out + 33 * D + 256);
+        unstage(out + 34 * D + 256);
     }
 }
 
 // A workgroup walks a sequence's chunks for 16 CB columns of one head; wave w holds the state's rows w D / 4 .. + D / 4 and adds a
-// quarter of every output element (its rows' share and, of the sum over A, the tokens 4 g + w), the quarters are added in
-// wave order through LDS a chunk later.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
+// quarter of every output element (its rows' share and, of the sum over A, the tokens 4 w .. + 4), the quarters are added
+// in a fixed order through LDS a chunk later.  Sums are kept short and their largest terms late, so that they round about as
+// often as a walk token by token: the products with S in chains of 8 terms that are added in pairs, A's on top of them, the
+// state's update by itself in the order of the tokens and then onto the decayed state.  Error against 64 bits over 96 to 1,801 tokens with
+// gates from nearly 0 to nearly 1, as a share of the walk's: outputs 0.47 to 0.97, gated 0.86 to 1.08 (5.6e-8 of the norm against
+// 5.3e-8); states 0.39 to 1.18, gated to 1.45 where both are one rounding (4.4e-8 against 3.1e-8).  With one chain a sum, float
+// products of decays and the rounded decay alone the outputs were at 1.0 to 3.0, the states at up to 2.6, for 3 to 15 % less time.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
 // barrier a chunk.  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H, e / (16 CB)): the workgroups of a head
 // on one XCD where sequences * H is a multiple of 8.
 template <int D, int CB, int S, bool DELTA>
@@ -244,7 +259,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     if (nch <= 0) return;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
     const float* blocks = scratch + ((size_t)cw_first(cu_seqlens, s) * H + h) * BLOCK;
-    // a stage: read factors | write factors | A | decay | values (256 floats each of the last three); a lane's byte offsets
+    // a stage: read factors | write factors | A | both parts of the decay | values (256 floats each of the last three); a lane's byte offsets
     // within a chunk's block, the block itself is a scalar address that goes on by a chunk's blocks
     unsigned qoff[NKB], koff[NKB];
 #pragma unroll
@@ -252,14 +267,14 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         qoff[j] = (unsigned)((wave * NKB + j) * 1024 + lane * 16);
         koff[j] = qoff[j] + D * 64;
     }
-    // waves 0 and 1 bring A and the decay's D floats, waves 2 and 3 the values (both the same 16 columns, or 16 each): L loads a wave
-    const unsigned moff = wave == 0 ? 128 * D + lane * 16 : 128 * D + 1024 + (lane * 16) % (4 * D);
+    // waves 0 and 1 bring A and the decay's 2 D floats, waves 2 and 3 the values (both the same 16 columns, or 16 each): L loads a wave
+    const unsigned moff = wave == 0 ? 128 * D + lane * 16 : 128 * D + 1024 + (lane * 16) % (8 * D);
     const unsigned values = wave < 2 ? 0u : ~0u;
     const unsigned long long values64 = wave < 2 ? 0ull : ~0ull;
     unsigned long long block = (unsigned long long)blocks;
     const int vx = cb * CB + (CB == 2 ? wave & 1 : 0);        // the 16 columns this wave brings values of
     unsigned long long vbase = (unsigned long long)(v + (size_t)t0 * ldv + h * e + vx * 16);      // the chunk's first row: rows of a prompt reach beyond 4 GB
-    const unsigned vcol = ((lane & 3) ^ (lane >> 4)) * 16, uoff = (49 * D + 256) * 4 + vx * 1024 + lane * 16;
+    const unsigned vcol = ((lane & 3) ^ (lane >> 4)) * 16, uoff = (50 * D + 256) * 4 + vx * 1024 + lane * 16;
     const int vrow = lane >> 2;
     int vlast = t1 - 1 - t0, left = nch - 1, slot_i = 0;      // the sequence's last row, counted from the chunk's first
     auto bring = [&](unsigned lds, unsigned off, unsigned long long base) {
@@ -273,7 +288,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         for (int j = 0; j < NKB; ++j) {
             bring(base + (wave * NKB + j) * 1024, qoff[j], block);
             bring(base + D * 64 + (wave * NKB + j) * 1024, koff[j], block);
-            if (DELTA) bring(base + (32 * D + 512 + 256 * CB) * 4 + (wave * NKB + j) * 1024, qoff[j] + (33 * D + 256) * 4, block);
+            if (DELTA) bring(base + (32 * D + 512 + 256 * CB) * 4 + (wave * NKB + j) * 1024, qoff[j] + (34 * D + 256) * 4, block);
         }
         const unsigned voff = DELTA ? uoff : (unsigned)min(vrow, vlast) * (unsigned)ldv * 4 + vcol;
         bring(base + D * 128 + min(wave, 1 + CB) * 1024, (moff & ~values) | (voff & values),
@@ -308,8 +323,8 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
 #pragma unroll
         for (int x = 0; x < CB; ++x) {
             const float* pp = part + ((ch & (PB - 1)) * 4 * CB + x) * 272 + ot * 17 + (tid & 15);
-            const float v = ((pp[0] + pp[CB * 272]) + pp[2 * CB * 272]) + pp[3 * CB * 272];
-            if (t0 + ch * CW_C + ot < t1) op[x * 16] = v;
+            const double v = ((double)pp[0] + pp[CB * 272]) + ((double)pp[2 * CB * 272] + pp[3 * CB * 272]);
+            if (t0 + ch * CW_C + ot < t1) op[x * 16] = (float)v;
         }
         op += (size_t)CW_C * he;
     };
@@ -320,58 +335,56 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         // the operands first: the matrix instructions start as soon as they are there, the rest runs beside them
-        f32x4 qf[NKB], kf[NKB], dec[NKB], oa[CB];
-        float vv[CB][4], va[CB];
-        const float a = sf[32 * D + r16 * 16 + 4 * g + wave];
+        f32x4 qf[NKB], kf[NKB], dec[NKB], rest[NKB];
+        float vv[CB][4], va[CB], vz[CB];
+        const float a = sf[32 * D + r16 * 16 + 4 * wave + g];
 #pragma unroll
         for (int j = 0; j < NKB; ++j) qf[j] = *(const f32x4*)(sf + (wave * NKB + j) * 256 + lane * 4);
 #pragma unroll
         for (int j = 0; j < NKB; ++j) {
             const int kb = wave * NKB + j;
             dec[j] = *(const f32x4*)(sf + 32 * D + 256 + 16 * kb + 4 * g);
+            rest[j] = *(const f32x4*)(sf + 33 * D + 256 + 16 * kb + 4 * g);
             kf[j] = *(const f32x4*)(sf + 16 * D + kb * 256 + lane * 4);
         }
-        auto read_out = [&]() {                               // this wave's rows' share of the outputs
+        // factors of this wave's rows times the state, in chains of 8 rows
+        auto times_state = [&](const f32x4 (&f)[NKB], f32x4 (&to)[CB][2 * NKB]) {
 #pragma unroll
             for (int j = 0; j < NKB; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int x = 0; x < CB; ++x) oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[j][r], st[x][j][r], oa[x], 0, 0, 0);
+                    for (int x = 0; x < CB; ++x) {
+                        f32x4 from = {0.f, 0.f, 0.f, 0.f};
+                        if (r & 1) from = to[x][2 * j + r / 2];
+                        to[x][2 * j + r / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[j][r], st[x][j][r], from, 0, 0, 0);
+                    }
         };
-#pragma unroll
-        for (int x = 0; x < CB; ++x) oa[x] = {0.f, 0.f, 0.f, 0.f};
+        auto pairs = [&](const f32x4 (&p)[2 * NKB]) {
+            if constexpr (NKB == 1) return p[0] + p[1];
+            else return (p[0] + p[1]) + (p[2] + p[3]);
+        };
+        f32x4 ro[CB][2 * NKB];
         if constexpr (DELTA) {
-            f32x4 uf[CB], wf[NKB], pa[CB];
+            f32x4 uf[CB], wf[NKB], pa[CB][2 * NKB];
 #pragma unroll
             for (int j = 0; j < NKB; ++j) wf[j] = *(const f32x4*)(sf + 32 * D + 512 + 256 * CB + (wave * NKB + j) * 256 + lane * 4);
 #pragma unroll
-            for (int x = 0; x < CB; ++x) {
-                uf[x] = *(const f32x4*)(sf + 32 * D + 512 + x * 256 + lane * 4);
-                pa[x] = {0.f, 0.f, 0.f, 0.f};
-            }
+            for (int x = 0; x < CB; ++x) uf[x] = *(const f32x4*)(sf + 32 * D + 512 + x * 256 + lane * 4);
+            times_state(wf, pa);
+            times_state(qf, ro);
 #pragma unroll
-            for (int j = 0; j < NKB; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int x = 0; x < CB; ++x) pa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][r], st[x][j][r], pa[x], 0, 0, 0);
-            read_out();
-#pragma unroll
-            for (int x = 0; x < CB; ++x) *(f32x4*)(pu + ((wave * CB + x) * 64 + lane) * 4) = pa[x];
+            for (int x = 0; x < CB; ++x) *(f32x4*)(pu + ((wave * CB + x) * 64 + lane) * 4) = pairs(pa[x]);
             if (ch > 0) flush(ch - 1);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
 #pragma unroll
-            for (int x = 0; x < CB; ++x) {                    // u = U - W S, the waves' shares in their order
-                f32x4 u = uf[x];
+            for (int x = 0; x < CB; ++x) {                    // u = U - W S
+                f32x4 share[4];
 #pragma unroll
-                for (int y = 0; y < 4; ++y) {
-                    const f32x4 share = *(const f32x4*)(pu + ((y * CB + x) * 64 + lane) * 4);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) u[r] += share[r];
-                }
+                for (int y = 0; y < 4; ++y) share[y] = *(const f32x4*)(pu + ((y * CB + x) * 64 + lane) * 4);
+                const f32x4 u = uf[x] + ((share[0] + share[1]) + (share[2] + share[3]));
 #pragma unroll
                 for (int r = 0; r < 4; ++r) vv[x][r] = u[r];
                 va[x] = wave < 2 ? (wave == 0 ? u[0] : u[1]) : (wave == 2 ? u[2] : u[3]);
@@ -379,9 +392,9 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         } else {
 #pragma unroll
             for (int x = 0; x < CB; ++x) {
-                va[x] = sf[32 * D + 512 + x * 256 + (4 * g + wave) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
+                va[x] = sf[32 * D + 512 + x * 256 + (4 * wave + g) * 16 + (((r16 >> 2) ^ wave) << 2) + (r16 & 3)];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) vv[x][i] = sf[32 * D + 512 + x * 256 + (4 * g + i) * 16 + (((r16 >> 2) ^ g) << 2) + (r16 & 3)];
+                for (int i = 0; i < 4; ++i) vv[x][i] = sf[32 * D + 512 + x * 256 + (4 * i + g) * 16 + (((r16 >> 2) ^ i) << 2) + (r16 & 3)];
             }
         }
         // A's zeros above the diagonal keep a token's value from the tokens before it only while it is finite: others pass here as
@@ -391,34 +404,43 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         for (int x = 0; x < CB; ++x) {
             const bool fine = fabsf(va[x]) <= CW_FINITE;
             odd |= __ballot(!fine);
-            oa[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, fine ? va[x] : 0.f, oa[x], 0, 0, 0);
+            vz[x] = fine ? va[x] : 0.f;
         }
-        if constexpr (!DELTA) read_out();
+        if constexpr (!DELTA) times_state(qf, ro);
         issue();
 #pragma unroll
         for (int j = 0; j < NKB; ++j) {
+            // the decayed state, rounded once, and what the chunk adds to it, summed on top of that rounding's error
+            f32x4 add[CB];
 #pragma unroll
             for (int x = 0; x < CB; ++x)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) st[x][j][r] *= dec[j][r];
+                for (int r = 0; r < 4; ++r) {
+                    const float old = st[x][j][r], kept = old * dec[j][r];
+                    add[x][r] = fmaf(old, rest[j][r], fmaf(old, dec[j][r], -kept));
+                    st[x][j][r] = kept;
+                }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int x = 0; x < CB; ++x) st[x][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], st[x][j], 0, 0, 0);
+                for (int x = 0; x < CB; ++x) add[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], add[x], 0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < CB; ++x) st[x][j] += add[x];
         }
 #pragma unroll
         for (int x = 0; x < CB; ++x) {
             float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
+            const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vz[x], pairs(ro[x]), 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = oa[x][r];
+            for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = sum[r];
         }
-        if (odd) {                                            // infinite or not a number: this wave's tokens 4 i + wave of A
+        if (odd) {                                            // infinite or not a number: this wave's tokens 4 wave + i of A
             for (int x = 0; x < CB; ++x) {
                 float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
                 for (int i = 0; i < 4; ++i) {
                     const float u = __shfl(va[x], 16 * i + r16, 64);
                     for (int r = 0; r < 4; ++r)
-                        if (!(fabsf(u) <= CW_FINITE) && 4 * i + wave <= 4 * g + r) pw[(4 * g + r) * 17 + r16] += sf[32 * D + (4 * g + r) * 16 + 4 * i + wave] * u;
+                        if (!(fabsf(u) <= CW_FINITE) && 4 * wave + i <= 4 * g + r) pw[(4 * g + r) * 17 + r16] += sf[32 * D + (4 * g + r) * 16 + 4 * wave + i] * u;
                 }
             }
         }

@@ -894,7 +894,7 @@ def chunk_takes(d: int, e: int) -> bool:
 
 
 def chunk_scratch_floats(T: int, B: int, H: int, d: int, e: int, delta: bool = False) -> int:
-    return (T // 16 + B + 1) * H * (33 * d + 256 + (16 * (d + e) if delta else 0))
+    return (T // 16 + B + 1) * H * (34 * d + 256 + (16 * (d + e) if delta else 0))
 
 
 def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,

@@ -194,3 +194,71 @@ def test_values_that_are_not_finite_show_from_their_token_on(form, d, e, bad):
         assert torch.equal(got[:t], clean[:t])
         if bad != bad:
             assert not got[t + 1:, head].isfinite().any()
+
+
+@pytest.mark.parametrize("form", ["glr", "wkv", "fixed", "delta", "channels"])
+@pytest.mark.parametrize("decay", ["slow", "middle", "fast"])
+@pytest.mark.parametrize("T", [96, 1001])
+def test_error_beside_the_walk_token_by_token(form, decay, T):
+    """Rounding errors of chunks and of the walk token by token against float64, for decays near one, between and near zero."""
+    from braidinfer_amd import kernels as K
+    H, d = 4, 64 if form == "wkv" else 128
+    e, x = d, {"slow": 1, "middle": 0, "fast": -1}[decay]
+    g = torch.Generator(device="cuda").manual_seed(T + x)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    u = lambda *s: torch.rand(*s, device="cuda", generator=g)
+    q, k, v, a = r(T, H * d), r(T, H * d), r(T, H * e), {}
+    if form == "glr":
+        a = {"b1": r(H * d) * 0.3 + 3 * x, "b2": u(H * d) * 0.3}
+    elif form == "wkv":
+        a = {"z": r(T, H * d), "b1": r(H * d) * 0.3 - 3 * x, "b2": r(H * d)}
+    elif form == "fixed":
+        a = {"b1": 1 - u(H) * {1: 0.01, 0: 0.2, -1: 0.9}[x]}
+    else:
+        q, k = (torch.nn.functional.normalize(y.view(T, H, d), dim=-1).reshape(T, H * d) for y in (q, k))
+        power = {1: 0.02, 0: 0.3, -1: 2.0}[x]
+        a = {"gb": torch.cat([u(T, H) ** power, u(T, H)], 1)}
+        if form == "channels":
+            a["gc"] = u(T, H * d) ** power
+    form = "delta" if form == "channels" else form
+    # float64, on the device
+    D = {n: y.double() for n, y in a.items()}
+    q64, k64, v64, beta = q.double().view(T, H, d), k.double().view(T, H, d), v.double().view(T, H, e), None
+    if form == "glr":
+        low = D["b2"].view(H, d)
+        w = low + (1 - low) * torch.sigmoid(k64 + D["b1"].view(H, d))
+        q64, k64 = q64 * torch.sigmoid(q64), 1 - w
+    elif form == "wkv":
+        w = torch.exp(-torch.exp(D["z"].view(T, H, d) + D["b1"].view(H, d)))
+    elif form == "fixed":
+        w = D["b1"].view(1, H, 1).expand(T, H, d)
+    else:
+        w, beta = D["gc"].view(T, H, d) if "gc" in D else D["gb"][:, :H, None].expand(T, H, d), D["gb"][:, H:]
+    S, want = torch.zeros(H, d, e, dtype=torch.float64, device="cuda"), torch.empty(T, H, e, dtype=torch.float64, device="cuda")
+    for t in range(T):
+        old, S = S, w[t][:, :, None] * S
+        write = v64[t] if beta is None else beta[t][:, None] * (v64[t] - (S * k64[t][:, :, None]).sum(1))
+        kv = k64[t][:, :, None] * write[:, None, :]
+        S = S + kv
+        want[t] = (q64[t][:, :, None] * (old + D["b2"].view(H, d)[:, :, None] * kv if form == "wkv" else S)).sum(1)
+    want_S = as_kept(S[None], d)[0]
+    cu, slots = torch.tensor([0, T], dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+
+    def error(chunks):
+        out, state = torch.empty(T, H * e, device="cuda"), torch.zeros((1,) + tuple(K.glr_state_shape(H, d, e)), device="cuda")
+        if chunks:
+            scratch = torch.empty(K.chunk_scratch_floats(T, 1, H, d, e, form == "delta"), device="cuda")
+            K.chunk_scan(form, q, k, v.clone(), out, state, cu, slots, scratch, 1, H, H, d, e, T, **a)
+        elif form == "glr":
+            K.glr_scan(torch.cat([q, k, v], 1), a["b1"], a["b2"], out, state, cu, slots, 1, H, d, e)
+        elif form == "wkv":
+            K.wkv_scan(torch.cat([q, k, v, a["z"]], 1), a["b1"], a["b2"], out, state.view(1, -1), cu, slots, 1, H, d, e)
+        else:
+            K.dr_scan(q, k, v, a.get("gb"), a.get("b1"), out, state, cu, slots, 1, H, H, d, e, gc=a.get("gc"))
+        return (float((out.double().view(T, H, e) - want).norm() / want.norm()),
+                float((state.double().view(want_S.shape) - want_S).norm() / want_S.norm()))
+    (out, state), (out_walk, state_walk) = error(True), error(False)
+    # no further off but for what the draw does to sums of roundings (0.425 2^-24 of the norm each); a state of which little is older
+    # than its last token is at most five of them: the value or its correction, the write factor, their product and two sums
+    assert out < 1.12 * out_walk, (out, out_walk)
+    assert state < max(1.12 * state_walk, 2 ** -24), (state, state_walk)
