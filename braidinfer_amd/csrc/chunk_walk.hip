@@ -66,6 +66,7 @@ struct CwIn {
     size_t qk_stride, v_stride;
     const int *cu, *slots;
     int H, G, e, silu;
+    int least;            // sequences that bring fewer tokens are left alone
 };
 
 // grid (chunks of the longest sequence, H, sequences), D threads, a thread a channel.
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
     const int s = blockIdx.z, h = blockIdx.y, c = threadIdx.x, H = in.H, e = in.e;
     if (in.slots[s] < 0) return;
     const int t0 = in.cu[s] + (int)blockIdx.x * CW_C, n = min(CW_C, in.cu[s + 1] - t0);
-    if (n <= 0) return;
+    if (n <= 0 || in.cu[s + 1] - in.cu[s] < in.least) return;
     const int kh = h / (H / in.G);
     float q[CW_C], k[CW_C], w[CW_C], beta[DELTA ? CW_C : 1];
     const float bias = (FORM == CW_GLR || WKV) && in.b1 ? in.b1[h * D + c] : 0.f, low = (FORM == CW_GLR || WKV) && in.b2 ? in.b2[h * D + c] : 0.f;
@@ -239,7 +240,7 @@ template <int D, int CB, int S, bool DELTA>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
                                                          float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
-                                                         int zero_padding) {
+                                                         int zero_padding, int least) {
     constexpr int NKB = D / 64, RPL = D / 16, STAGE = ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4, L = (DELTA ? 3 : 2) * NKB + 1;
     constexpr int PB = DELTA ? 1 : 2;                         // buffers of output quarters
     const int BLOCK = cw_block(D, e, DELTA);
@@ -250,6 +251,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int slot = slots[s], t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1], he = H * e;
+    if (t1 - t0 < least) return;
     if (slot < 0) {
         if (zero_padding)
             for (int i = tid; i < (t1 - t0) * 16; i += 256) for (int x = 0; x < CB; ++x) o[(size_t)(t0 + (i >> 4)) * he + h * e + (cb * CB + x) * 16 + (i & 15)] = 0.f;
@@ -481,7 +483,7 @@ static int chunk_walk(const CwIn& in, const float* scratch, float* o, float* sta
         if (hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
         set = true;
     }
-    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding);
+    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding, in.least);
     return br_check_launch();
 }
 
@@ -509,11 +511,12 @@ static int chunk_run(const CwIn& in, float* o, float* state, size_t slot_stride,
 }
 
 // One step's tokens of B sequences (`max_new` the most a sequence brings) through a recurrence (see CwIn for the forms' inputs),
-// from and into the slots' states; `scratch`: br_chunk_scratch floats.
+// from and into the slots' states; `scratch`: br_chunk_scratch floats.  Sequences of fewer than `least` tokens are left alone: their
+// outputs and states are another kernel's.
 extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v, size_t qk_stride, size_t v_stride, const float* z,
                              const float* b1, const float* b2, const float* gb, const float* gc, int silu, float* o, float* state,
                              size_t slot_stride, const int* cu_seqlens, const int* slots, float* scratch, size_t scratch_floats, int T,
-                             int B, int H, int G, int d, int e, int max_new, hipStream_t s) {
+                             int B, int H, int G, int d, int e, int max_new, int least, hipStream_t s) {
     if (B <= 0 || T <= 0) return BR_OK;
     if (!br_chunk_takes(d, e) || H <= 0 || H > 65535 || B > 65535 || (long long)B * H > 0x7fffffffLL || e / 16 > 65535 || max_new <= 0 ||
         max_new > T || G <= 0 || H % G || form < CW_GLR || form > CW_DELTA || v_stride % 4 || ((uintptr_t)v | (uintptr_t)scratch) % 16 ||
@@ -521,7 +524,7 @@ extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v,
         scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA) || (form == CW_WKV && (!z || !b1 || !b2)) ||
         (form == CW_FIXED && !b1) || (form == CW_DELTA && !gb) || ((form == CW_GLR || form == CW_WKV) && G != H))
         return BR_BAD_ARG;
-    const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu};
+    const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu, least};
 #define CW_RUN(F) return d == 64 ? chunk_run<F, 64>(in, o, state, slot_stride, scratch, B, max_new, s) : chunk_run<F, 128>(in, o, state, slot_stride, scratch, B, max_new, s)
     switch (form) {
         case CW_GLR: CW_RUN(CW_GLR);

@@ -516,6 +516,7 @@ struct DrScan {
     const int *cu_seqlens, *slots;
     size_t qk_stride, v_stride, gb_stride, slot_stride;
     int H, G, d, e, ones;
+    int below;            // > 0: sequences that bring as many tokens or more are left alone
 };
 
 template <int RPL, int TC, int MODE, bool SILU, bool LOCAL>
@@ -542,6 +543,7 @@ __global__ __launch_bounds__(256) void dr_scan_kernel(const DrScan p) {
     const int cb4 = cb16 * 4 + wave, c = cb4 * 4 + cg;
     const int slot = p.slots[s];
     const int t0 = p.cu_seqlens[s], t1 = p.cu_seqlens[s + 1];
+    if (p.below && t1 - t0 >= p.below) return;
     const bool live = c < e, is_n = MODE == DR_WEIGHTED && p.ones && c == e;
     const int he = H * e;
     // where this lane's column is read out to: o's column, or the extra column's own array
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
     const int slot = p.slots[s];
     const int t0 = p.cu_seqlens[s], t1 = p.cu_seqlens[s + 1];
     const int ncb4 = (e + p.ones + 3) >> 2, he = H * e;
-    if (cb4 >= ncb4) return;                       // a wave's own matter: there is no barrier
+    if (cb4 >= ncb4 || (p.below && t1 - t0 >= p.below)) return;          // a wave's own matter: there is no barrier
     const bool live = c < e, is_n = MODE == DR_WEIGHTED && p.ones && c == e;
     float* orow = is_n ? p.n_out + (size_t)t0 * H + h : p.o + (size_t)t0 * he + h * e + c;
     const size_t ostep = is_n ? H : he;
@@ -848,14 +850,15 @@ static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, int single
 
 // `mode`: DR_FIXED with `g_head`, DR_DELTA and DR_WEIGHTED with `gb`, DR_CHANNELS with `gb` and `gc`.  `silu` 1 (DR_FIXED):
 // q, k, v pass silu.  `singles` 1: no more tokens than sequences, as in steps of single tokens (a longer sequence among them
-// is walked just as well, only without its next tokens' rows on their way).
+// is walked just as well, only without its next tokens' rows on their way).  `below` > 0: sequences of as many tokens or more are
+// left alone, outputs and states (`chunk_walk.hip` has them).
 extern "C" int br_dr_scan(const float* q, const float* k, size_t qk_stride, const float* v, size_t v_stride, const float* gb,
                           size_t gb_stride, const float* g_head, const float* gc, const float* skip, float* o, float* n_out,
                           float* state, size_t slot_stride, const int* cu_seqlens, const int* slots, int B, int H, int G, int d,
-                          int e, int mode, int ones, int silu, int singles, hipStream_t s) {
+                          int e, int mode, int ones, int silu, int singles, int below, hipStream_t s) {
     if (B <= 0) return BR_OK;
     const DrScan a = {q, k, v, gb, g_head, gc, skip, o, n_out, state, nullptr, cu_seqlens, slots, qk_stride, v_stride, gb_stride, slot_stride,
-                      H, G, d, e, ones};
+                      H, G, d, e, ones, below};
     return dr_scan_launch<false>(a, B, mode, silu, singles, s);
 }
 
@@ -905,7 +908,7 @@ extern "C" int br_dr_scan_pieces(const float* q, const float* k, size_t qk_strid
     const size_t piece_stride = (size_t)H * ncb4 * rpl * 64;
     if ((long long)H * ncb4 > 65535 || slot_stride < piece_stride) return BR_BAD_ARG;
     const DrScan a = {q, k, v, gb, g_head, nullptr, skip, o, n_out, piece_state, piece_decay, piece_cu, piece_slots, qk_stride, v_stride,
-                      gb_stride, piece_stride, H, G, d, e, ones};
+                      gb_stride, piece_stride, H, G, d, e, ones, 0};
     int rc = dr_scan_launch<true>(a, B * pieces, mode, silu, 0, s);
     if (rc != BR_OK) return rc;
     dr_carry_kernel<<<dim3(B, H * ncb4), 64, 0, s>>>(state, slot_stride, slots, piece_state, piece_stride, piece_cu, g_head,

@@ -44,7 +44,7 @@ template <int RPL, int TC, bool V4, bool LOCAL>
 __global__ __launch_bounds__(256) void glr_scan_kernel(
     const float* __restrict__ rows, const float* __restrict__ f_bias, const float* __restrict__ lower,
     float* __restrict__ o, float* __restrict__ state, const int* __restrict__ cu_seqlens,
-    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride, float* __restrict__ decay) {
+    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride, float* __restrict__ decay, int below) {
     constexpr int DP = RPL * 16;                   // rows of a column with padding
     constexpr int NL = TC * DP / 1024;             // groups of 4 rows a thread brings per chunk and array
     extern __shared__ float lds[];
@@ -56,8 +56,8 @@ __global__ __launch_bounds__(256) void glr_scan_kernel(
     const int cg = lane >> 4, g = lane & 15;
     const int cb4 = cb16 * 4 + wave, c = cb4 * 4 + cg;
     const int slot = slots[s];
-    if (slot < 0) return;
     const int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
+    if (slot < 0 || (below && t1 - t0 >= below)) return;
     const bool live = c < e;
     const int ncb4 = (e + 3) >> 2;
     float* S = state + (size_t)slot * slot_stride + (((size_t)h * ncb4 + cb4) * RPL) * 64 + lane;
@@ -211,7 +211,7 @@ template <int RPL, bool V4>
 __global__ __launch_bounds__(256) void glr_token_kernel(
     const float* __restrict__ rows, const float* __restrict__ f_bias, const float* __restrict__ lower,
     float* __restrict__ o, float* __restrict__ state, const int* __restrict__ cu_seqlens,
-    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride) {
+    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride, int below) {
     const int s = blockIdx.x, h = blockIdx.y, cb16 = blockIdx.z;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int cg = lane >> 4, g = lane & 15;
@@ -219,6 +219,7 @@ __global__ __launch_bounds__(256) void glr_token_kernel(
     const int slot = slots[s], ncb4 = (e + 3) >> 2, hd = H * d;
     if (slot < 0 || cb4 >= ncb4) return;           // a wave's own matter: there is no barrier
     const int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
+    if (below && t1 - t0 >= below) return;
     const bool live = c < e;
     float* S = state + (size_t)slot * slot_stride + (((size_t)h * ncb4 + cb4) * RPL) * 64 + lane;
     float st[RPL], lo[RPL], bias[RPL];
@@ -274,7 +275,7 @@ extern "C" int br_glr_rows_per_lane(int d) { return glr_rpl(d); }
 template <bool LOCAL>
 static int glr_scan_launch(const float* rows, const float* f_bias, const float* lower, float* o, float* state,
                            const int* cu_seqlens, const int* slots, int B, int H, int d, int e, int width,
-                           size_t slot_stride, float* decay, int singles, hipStream_t s) {
+                           size_t slot_stride, float* decay, int singles, int below, hipStream_t s) {
     const int ncb4 = (e + 3) / 4, rpl = glr_rpl(d);
     if (H <= 0 || H > 65535 || d <= 0 || e <= 0 || d > 512 || (e + 15) / 16 > 65535 || width < 2 * H * d + H * e ||
         slot_stride < (size_t)H * ncb4 * rpl * 64 || (LOCAL && !decay))
@@ -284,13 +285,13 @@ static int glr_scan_launch(const float* rows, const float* f_bias, const float* 
     const bool v4 = d % 4 == 0 && width % 4 == 0 && ((uintptr_t)rows % 16) == 0;
 #define GLR_SCAN(R, TC) do { \
         if (!LOCAL && singles) { \
-            if (v4) glr_token_kernel<R, true><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride); \
-            else glr_token_kernel<R, false><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride); \
+            if (v4) glr_token_kernel<R, true><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
+            else glr_token_kernel<R, false><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
             break; \
         } \
         const size_t lds = (size_t)(4 * TC * R * 16 + 2 * TC * 16) * sizeof(float); \
-        if (v4) glr_scan_kernel<R, TC, true, LOCAL><<<grid, 256, lds, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay); \
-        else glr_scan_kernel<R, TC, false, LOCAL><<<grid, 256, lds, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay); \
+        if (v4) glr_scan_kernel<R, TC, true, LOCAL><<<grid, 256, lds, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay, below); \
+        else glr_scan_kernel<R, TC, false, LOCAL><<<grid, 256, lds, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay, below); \
     } while (0)
     if (rpl == 4) GLR_SCAN(4, 16);
     else if (rpl == 8) GLR_SCAN(8, 16);
@@ -302,12 +303,13 @@ static int glr_scan_launch(const float* rows, const float* f_bias, const float* 
 
 // `slot_stride`: floats from one slot's state to the next (at least H * ceil(e / 4) * rows per lane * 64).  `singles` 1: no
 // more tokens than sequences, as in steps of single tokens (a longer sequence among them is walked just as well, only
-// without its next tokens' rows on their way).
+// without its next tokens' rows on their way).  `below` > 0: sequences of as many tokens or more are left alone, outputs
+// and states (`chunk_walk.hip` has them).
 extern "C" int br_glr_scan(const float* rows, const float* f_bias, const float* lower, float* o, float* state,
                            const int* cu_seqlens, const int* slots, int B, int H, int d, int e, int width,
-                           size_t slot_stride, int singles, hipStream_t s) {
+                           size_t slot_stride, int singles, int below, hipStream_t s) {
     if (B <= 0) return BR_OK;
-    return glr_scan_launch<false>(rows, f_bias, lower, o, state, cu_seqlens, slots, B, H, d, e, width, slot_stride, nullptr, singles, s);
+    return glr_scan_launch<false>(rows, f_bias, lower, o, state, cu_seqlens, slots, B, H, d, e, width, slot_stride, nullptr, singles, below, s);
 }
 
 // A step of long prompts with every sequence cut into `pieces` pieces that run side by side: the recurrence is
@@ -327,7 +329,7 @@ extern "C" int br_glr_scan_pieces(const float* rows, const float* f_bias, const 
     const int ncb4 = (e + 3) / 4, rpl = glr_rpl(d);
     const size_t piece_stride = (size_t)H * ncb4 * rpl * 64;
     int rc = glr_scan_launch<true>(rows, f_bias, lower, o, piece_state, piece_cu, piece_slots, B * pieces, H, d, e, width,
-                                   piece_stride, decay, 0, s);
+                                   piece_stride, decay, 0, 0, s);
     if (rc != BR_OK) return rc;
     if ((long long)H * ncb4 > 65535) return BR_BAD_ARG;
     glr_carry_kernel<<<dim3(B, H * ncb4), 64, 0, s>>>(state, slot_stride, slots, piece_state, piece_stride, decay, pieces, H,
@@ -335,7 +337,7 @@ extern "C" int br_glr_scan_pieces(const float* rows, const float* f_bias, const 
     rc = br_check_launch();
     if (rc != BR_OK) return rc;
     return glr_scan_launch<false>(rows, f_bias, lower, o, piece_state, piece_cu, piece_slots, B * pieces, H, d, e, width,
-                                  piece_stride, nullptr, 0, s);
+                                  piece_stride, nullptr, 0, 0, s);
 }
 
 // ------------------------------------------------------------------ head norm ------
@@ -407,7 +409,7 @@ template <int RPL, int TC, bool V4, bool LOCAL>
 __global__ __launch_bounds__(256) void wkv_scan_kernel(
     const float* __restrict__ rows, const float* __restrict__ w0, const float* __restrict__ bonus,
     float* __restrict__ o, float* __restrict__ state, const int* __restrict__ cu_seqlens,
-    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride, float* __restrict__ decay) {
+    const int* __restrict__ slots, int H, int d, int e, int width, size_t slot_stride, float* __restrict__ decay, int below) {
     constexpr int DP = RPL * 16;
     constexpr int NL = TC * DP / 1024;
     extern __shared__ float lds[];
@@ -422,6 +424,7 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(
     const int slot = slots[s];
     const int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
     const bool live = c < e;
+    if (below && t1 - t0 >= below) return;
     if (slot < 0) {                                // padding: no state behind it; its rows of o are zero
         if (!LOCAL && g == 0 && live) for (int t = t0; t < t1; ++t) o[(size_t)t * H * e + h * e + c] = 0.f;
         return;
@@ -555,7 +558,7 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(
 template <bool LOCAL>
 static int wkv_scan_launch(const float* rows, const float* w0, const float* bonus, float* o, float* state,
                            const int* cu_seqlens, const int* slots, int B, int H, int d, int e, int width,
-                           size_t slot_stride, float* decay, hipStream_t s) {
+                           size_t slot_stride, float* decay, int below, hipStream_t s) {
     const int ncb4 = (e + 3) / 4, rpl = glr_rpl(d);
     if (H <= 0 || H > 65535 || d <= 0 || e <= 0 || d > 512 || (e + 15) / 16 > 65535 || width < 3 * H * d + H * e ||
         slot_stride < (size_t)H * ncb4 * rpl * 64 || !w0 || !bonus || (LOCAL && !decay))
@@ -564,8 +567,8 @@ static int wkv_scan_launch(const float* rows, const float* w0, const float* bonu
     const bool v4 = d % 4 == 0 && e % 4 == 0 && width % 4 == 0 && ((uintptr_t)rows % 16) == 0;
 #define WKV_SCAN(R, TC) do { \
         const size_t lds = (size_t)(6 * TC * R * 16 + 2 * TC * 16) * sizeof(float); \
-        if (v4) wkv_scan_kernel<R, TC, true, LOCAL><<<grid, 256, lds, s>>>(rows, w0, bonus, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay); \
-        else wkv_scan_kernel<R, TC, false, LOCAL><<<grid, 256, lds, s>>>(rows, w0, bonus, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay); \
+        if (v4) wkv_scan_kernel<R, TC, true, LOCAL><<<grid, 256, lds, s>>>(rows, w0, bonus, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay, below); \
+        else wkv_scan_kernel<R, TC, false, LOCAL><<<grid, 256, lds, s>>>(rows, w0, bonus, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, decay, below); \
     } while (0)
     if (rpl == 4) WKV_SCAN(4, 16);
     else if (rpl == 8) WKV_SCAN(8, 16);
@@ -575,11 +578,12 @@ static int wkv_scan_launch(const float* rows, const float* w0, const float* bonu
     return br_check_launch();
 }
 
+// `below` > 0: sequences of as many tokens or more are left alone, outputs and states (`chunk_walk.hip` has them).
 extern "C" int br_wkv_scan(const float* rows, const float* w0, const float* bonus, float* o, float* state,
                            const int* cu_seqlens, const int* slots, int B, int H, int d, int e, int width,
-                           size_t slot_stride, hipStream_t s) {
+                           size_t slot_stride, int below, hipStream_t s) {
     if (B <= 0) return BR_OK;
-    return wkv_scan_launch<false>(rows, w0, bonus, o, state, cu_seqlens, slots, B, H, d, e, width, slot_stride, nullptr, s);
+    return wkv_scan_launch<false>(rows, w0, bonus, o, state, cu_seqlens, slots, B, H, d, e, width, slot_stride, nullptr, below, s);
 }
 
 // A step of long prompts with every sequence cut into `pieces` pieces that run side by side, as `br_glr_scan_pieces`
@@ -594,7 +598,7 @@ extern "C" int br_wkv_scan_pieces(const float* rows, const float* w0, const floa
     const int ncb4 = (e + 3) / 4, rpl = glr_rpl(d);
     const size_t piece_stride = (size_t)H * ncb4 * rpl * 64;
     int rc = wkv_scan_launch<true>(rows, w0, bonus, o, piece_state, piece_cu, piece_slots, B * pieces, H, d, e, width,
-                                   piece_stride, decay, s);
+                                   piece_stride, decay, 0, s);
     if (rc != BR_OK) return rc;
     if ((long long)H * ncb4 > 65535 || slot_stride < piece_stride) return BR_BAD_ARG;
     glr_carry_kernel<<<dim3(B, H * ncb4), 64, 0, s>>>(state, slot_stride, slots, piece_state, piece_stride, decay, pieces, H,
@@ -602,7 +606,7 @@ extern "C" int br_wkv_scan_pieces(const float* rows, const float* w0, const floa
     rc = br_check_launch();
     if (rc != BR_OK) return rc;
     return wkv_scan_launch<false>(rows, w0, bonus, o, piece_state, piece_cu, piece_slots, B * pieces, H, d, e, width,
-                                  piece_stride, nullptr, s);
+                                  piece_stride, nullptr, 0, s);
 }
 
 // ------------------------------------------------------------- shifted mixes --------

@@ -845,10 +845,12 @@ def glr_state_dense(state: torch.Tensor, H: int, d: int, e: int) -> torch.Tensor
 
 
 def glr_scan(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], out: torch.Tensor,
-             state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int) -> None:
+             state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int,
+             below: int = 0, singles: Optional[bool] = None) -> None:
     """rows [T, 2*H*d + H*e] float, the projections' sums q | f | v; q = silu(.), f = lower + (1 - lower) *
     sigmoid(. + f_bias) are applied on the way.  state [slots, *glr_state_shape]: walks every sequence's new
-    tokens in order, writes o [T, H*e] float and leaves the state."""
+    tokens in order, writes o [T, H*e] float and leaves the state.  `below` > 0: sequences of as many tokens or more are left
+    alone; `singles`: the others bring a token each (None: told by T and B)."""
     _dev("glr_scan", rows, f_bias, lower, out, cu_seqlens, slots)
     T = rows.shape[0]
     _req(state.is_cuda and state.shape[1:] == glr_state_shape(H, d, e) and state[0].is_contiguous(),
@@ -859,9 +861,9 @@ def glr_scan(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional
         _req(v is None or (v.dtype == torch.float32 and v.numel() == H * d), "glr_scan: bias and lower bound float32 [H*d]")
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "glr_scan: arrays shorter than the batch")
     _req(d <= 512, f"glr_scan: {d} query channels a head are beyond the kernel's 512")
-    f = _fn("gated_recurrence", "br_glr_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, _P])
+    f = _fn("gated_recurrence", "br_glr_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, c_int, _P])
     _check(f(_ptr(rows), _ptr(f_bias), _ptr(lower), _ptr(out), _ptr(state), _ptr(cu_seqlens), _ptr(slots), B, H, d, e,
-             rows.shape[1], state.stride(0), int(T <= B), _stream()), "glr_scan")
+             rows.shape[1], state.stride(0), int(T <= B if singles is None else singles), int(below), _stream()), "glr_scan")
 
 
 def glr_scan_pieces(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], out: torch.Tensor,
@@ -900,12 +902,12 @@ def chunk_scratch_floats(T: int, B: int, H: int, d: int, e: int, delta: bool = F
 def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
                cu_seqlens: torch.Tensor, slots: torch.Tensor, scratch: torch.Tensor, B: int, H: int, G: int, d: int, e: int,
                max_new: int, z: Optional[torch.Tensor] = None, b1: Optional[torch.Tensor] = None, b2: Optional[torch.Tensor] = None,
-               gb: Optional[torch.Tensor] = None, gc: Optional[torch.Tensor] = None, silu: bool = False) -> None:
+               gb: Optional[torch.Tensor] = None, gc: Optional[torch.Tensor] = None, silu: bool = False, least: int = 0) -> None:
     """A recurrence over a step of prompts, 16 tokens at a time on the matrix cores: form "glr" as `glr_scan` (k the gates'
     sums, b1 their bias, b2 their lower bounds), "wkv" as `wkv_scan` (z the decays' sums, b1 their bias, b2 the bonus), "fixed"
     as `dr_scan` with `g_head` (b1; `silu` is applied to q, k and v, the latter in place) and "delta" as `dr_scan` with `gb`
     (and `gc`).  q, k, v: float rows, views of wider ones allowed (q, k and z with one stride); `max_new`: the most tokens a
-    sequence brings; `scratch` float32, `chunk_scratch_floats` of them."""
+    sequence brings; `scratch` float32, `chunk_scratch_floats` of them.  Sequences of fewer than `least` tokens are left alone."""
     _req(form in ("glr", "wkv", "fixed", "delta"), f"chunk_scan: form {form!r}")
     number = ("glr", "wkv", "fixed", "delta").index(form)
     T = q.shape[0]
@@ -931,10 +933,10 @@ def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "chunk_scan: arrays shorter than the batch")
     _req(scratch.numel() >= chunk_scratch_floats(T, B, H, d, e, form == "delta"), "chunk_scan: scratch too small")
     f = _fn("chunk_walk", "br_chunk_scan", [c_int, _P, _P, _P, c_size_t, c_size_t] + [_P] * 5 + [c_int, _P, _P, c_size_t, _P, _P, _P, c_size_t]
-            + [c_int] * 7 + [_P])
+            + [c_int] * 8 + [_P])
     _check(f(number, _ptr(q), _ptr(k), _ptr(v), stride, v.stride(0), _ptr(z), _ptr(b1), _ptr(b2), _ptr(gb), _ptr(gc), int(silu), _ptr(out),
              _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots), _ptr(scratch), scratch.numel(), T, B, H, G, d, e, int(max_new),
-             _stream()), "chunk_scan")
+             int(least), _stream()), "chunk_scan")
 
 
 def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, H: int, e: int, eps: float) -> None:
@@ -948,11 +950,12 @@ def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, 
 
 # ------------------------------------------------- decayed recurrence with a bonus -----
 def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
-             cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int) -> None:
+             cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int, below: int = 0) -> None:
     """rows [T, >= 3*H*d + H*e] float, the projections' sums r | k | v | z (the decay is exp(-exp(z + w0)), made on the
     way); bonus float [H*d].  state [slots, n] float with a slot's first prod(glr_state_shape(H, d, e)) floats its S as
     `glr_scan` keeps it: walks every sequence's new tokens in order, o_t = (S + diag(bonus) k v^T)^T r before
-    S <- diag(decay) S + k v^T, writes o [T, H*e] float and leaves the state."""
+    S <- diag(decay) S + k v^T, writes o [T, H*e] float and leaves the state.  `below` > 0: sequences of as many tokens or more
+    are left alone."""
     _dev("wkv_scan", rows, w0, bonus, out, cu_seqlens, slots)
     T = rows.shape[0]
     need = 1
@@ -966,9 +969,9 @@ def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: tor
         _req(v.dtype == torch.float32 and v.numel() == H * d, "wkv_scan: w0 and bonus float32 [H*d]")
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "wkv_scan: arrays shorter than the batch")
     _req(d <= 512, f"wkv_scan: {d} key channels a head are beyond the kernel's 512")
-    f = _fn("gated_recurrence", "br_wkv_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, _P])
+    f = _fn("gated_recurrence", "br_wkv_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, _P])
     _check(f(_ptr(rows), _ptr(w0), _ptr(bonus), _ptr(out), _ptr(state), _ptr(cu_seqlens), _ptr(slots), B, H, d, e,
-             rows.shape[1], state.stride(0), _stream()), "wkv_scan")
+             rows.shape[1], state.stride(0), int(below), _stream()), "wkv_scan")
 
 
 def wkv_scan_pieces(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
@@ -1160,23 +1163,26 @@ def _dr_scan_check(name, q, k, v, gb, decay, gc, weighted, skip, n_out, out, sta
 def dr_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gb: Optional[torch.Tensor], decay: Optional[torch.Tensor],
             out: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, G: int,
             d: int, e: int, silu: bool = False, gc: Optional[torch.Tensor] = None, weighted: bool = False,
-            skip: Optional[torch.Tensor] = None, n_out: Optional[torch.Tensor] = None) -> None:
+            skip: Optional[torch.Tensor] = None, n_out: Optional[torch.Tensor] = None, below: int = 0,
+            singles: Optional[bool] = None) -> None:
     """A walk over every sequence's new tokens with a state S [d, e] a head, float, in `state` [slots, *glr_state_shape]
     (a view whose slots may be strided).  q, k float views [T, G d], v [T, H e] (rows may be strided; head h reads
     q/k head h // (H / G)).  With `gb` [T, 2 H] (g | beta) the gated delta rule
     S <- g S; u = beta (v - S^T k); S <- S + k u^T (`gc` [T, H d]: one decay a key channel instead of g, diag(gc) S); with
     `weighted` S <- g S + beta k v^T; else with `decay` [H] S <- decay_h S + k v^T.  o = S^T q after the write, into out
     float [T, H e].  `silu` (with `decay`): q, k, v pass silu on their way in.  With `weighted`: `skip` [H] adds skip_h v to
-    o, and `n_out` [T, H] takes the read-out of one column more, whose value is 1 (the state is then [d, e + 1] a head)."""
+    o, and `n_out` [T, H] takes the read-out of one column more, whose value is 1 (the state is then [d, e + 1] a head).
+    `below` > 0: sequences of as many tokens or more are left alone; `singles`: the others bring a token each (None: told by T
+    and B)."""
     mode = _dr_scan_check("dr_scan", q, k, v, gb, decay, gc, weighted, skip, n_out, out, state, cu_seqlens, slots, B, H, G, d, e, silu)
     _req(cu_seqlens.numel() >= B + 1, "dr_scan: arrays shorter than the batch")
     T = out.shape[0]
     qs = q.stride(0) if T > 1 else G * d
     vs = v.stride(0) if T > 1 else H * e
-    f = _fn("delta_rule", "br_dr_scan", [_P, _P, c_size_t, _P, c_size_t, _P, c_size_t] + [_P] * 6 + [c_size_t, _P, _P] + [c_int] * 9 + [_P])
+    f = _fn("delta_rule", "br_dr_scan", [_P, _P, c_size_t, _P, c_size_t, _P, c_size_t] + [_P] * 6 + [c_size_t, _P, _P] + [c_int] * 10 + [_P])
     _check(f(_ptr(q), _ptr(k), qs, _ptr(v), vs, _ptr(gb), 2 * H, _ptr(decay), _ptr(gc), _ptr(skip), _ptr(out), _ptr(n_out), _ptr(state),
-             state.stride(0), _ptr(cu_seqlens), _ptr(slots), B, H, G, d, e, mode, int(n_out is not None), int(bool(silu)), int(T <= B),
-             _stream()), "dr_scan")
+             state.stride(0), _ptr(cu_seqlens), _ptr(slots), B, H, G, d, e, mode, int(n_out is not None), int(bool(silu)),
+             int(T <= B if singles is None else singles), int(below), _stream()), "dr_scan")
 
 
 def dr_rotate_rows(q: torch.Tensor, k: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], rotary_dim: int,

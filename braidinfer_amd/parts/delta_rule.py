@@ -39,7 +39,7 @@ from ..cache import StateNeed
 from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, RotaryTables, Runtime, register_part
-from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
+from .gated_recurrence import CHUNKS_FROM, HGRN2, chunk_scratch, in_chunks, pieces_for
 from .linear import fused_layout, linear, padded_rows, stream_layout
 
 
@@ -166,11 +166,12 @@ class GatedDeltaRule(Mixer):
                           q, k, v, gb, step.n_seqs, ng, nh, d, e, taps_t=self.conv_t, decay=decay, gc=gc, single_tokens=step.is_decode)
         o = step.ws.get("dr_o", (T, nh * e), torch.float32)
         S = ctx.state[:, :self.state_floats].view((-1,) + tuple(K.glr_state_shape(nh, d, e)))
-        if in_chunks(step, d, e):
+        chunks, walk, rest = in_chunks(step, d, e)
+        if chunks:
             K.chunk_scan("delta", q, k, v, o, S, step.cu_seqlens, step.slots, chunk_scratch(step, nh, d, e, True), step.n_seqs, nh, ng, d, e,
-                         step.max_new, gb=gb, gc=gc)
-        else:
-            K.dr_scan(q, k, v, gb, None, o, S, step.cu_seqlens, step.slots, step.n_seqs, nh, ng, d, e, gc=gc)
+                         step.max_new, gb=gb, gc=gc, least=CHUNKS_FROM)
+        if walk:
+            K.dr_scan(q, k, v, gb, None, o, S, step.cu_seqlens, step.slots, step.n_seqs, nh, ng, d, e, gc=gc, **rest)
         y = step.ws.get("dr_y", (T, nh * e), self.rt.dtype)
         K.head_norm_gate(o, self.norm_w, gate, y, nh, e, self.eps, gate_sigmoid=self.gate_sigmoid)
         linear(y, self.w_o, x, step.ws, accumulate=True)
@@ -260,11 +261,13 @@ class LightningAttention(Mixer):
                 silu = False
             K.dr_rotate_rows(rows[:, :hd], rows[:, hd:2 * hd], tables.cos if tables else None, tables.sin if tables else None,
                              tables.rotary_dim if tables else 0, nh, d, 1.0, self.key_scale)
-        pieces = 1 if in_chunks(step, d, e) else pieces_for(step, nh * -(-e // 16), self.MIN_PIECE)
-        if in_chunks(step, d, e):
+        chunks, walk, rest = in_chunks(step, d, e)
+        pieces = 1 if chunks else pieces_for(step, nh * -(-e // 16), self.MIN_PIECE)
+        if chunks:
             K.chunk_scan("fixed", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], o, ctx.state, step.cu_seqlens, step.slots,
-                         chunk_scratch(step, nh, d, e), step.n_seqs, nh, nh, d, e, step.max_new, b1=self.decay, silu=silu)
-        elif pieces > 1:
+                         chunk_scratch(step, nh, d, e), step.n_seqs, nh, nh, d, e, step.max_new, b1=self.decay, silu=silu,
+                         least=CHUNKS_FROM)
+        if pieces > 1:
             # long prompts: the recurrence is linear in the state, so every sequence is cut into pieces that are walked
             # side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)
@@ -274,9 +277,9 @@ class LightningAttention(Mixer):
                 K.silu_rows(rows[:, :2 * hd + he])
             K.dr_scan_pieces(rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], self.decay, o, ctx.state, step.slots,
                              cu, numbers, piece_state, step.n_seqs, pieces, nh, d, e, silu=False)
-        else:
+        elif walk:
             K.dr_scan(rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], None, self.decay, o, ctx.state,
-                      step.cu_seqlens, step.slots, step.n_seqs, nh, nh, d, e, silu=silu)
+                      step.cu_seqlens, step.slots, step.n_seqs, nh, nh, d, e, silu=silu, **rest)
         y = step.ws.get("la_y", (T, he), self.rt.dtype)
         if self.norm_per_head:
             K.head_norm_gate(o, self.norm_w, rows[:, 2 * hd + he:], y, nh, e, self.eps, gate_sigmoid=self.gate_sigmoid)

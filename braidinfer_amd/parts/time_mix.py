@@ -27,7 +27,7 @@ from ..cache import StateNeed
 from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, Runtime, register_part
-from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
+from .gated_recurrence import CHUNKS_FROM, HGRN2, chunk_scratch, in_chunks, pieces_for
 from .linear import linear, stream_layout
 
 BRANCHES = ("r", "k", "v", "g", "w")
@@ -102,12 +102,13 @@ class WKVTimeMix(Mixer):
         K.tanh(low, low_t)
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
-        pieces = 1 if in_chunks(step, self.d, self.d) else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
-        if in_chunks(step, self.d, self.d):
+        chunks, walk, rest = in_chunks(step, self.d, self.d)
+        pieces = 1 if chunks else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
+        if chunks:
             r, k, v, z = (rows[:, i * hd:(i + 1) * hd] for i in range(4))
             K.chunk_scan("wkv", r, k, v, o, state, step.cu_seqlens, step.slots, chunk_scratch(step, self.nh, self.d, self.d), step.n_seqs,
-                         self.nh, self.nh, self.d, self.d, step.max_new, z=z, b1=self.w0, b2=self.u)
-        elif pieces > 1:
+                         self.nh, self.nh, self.d, self.d, step.max_new, z=z, b1=self.w0, b2=self.u, least=CHUNKS_FROM)
+        if pieces > 1:
             # long prompts: every sequence cut into pieces that are walked side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)
             n = step.n_seqs * pieces
@@ -115,8 +116,9 @@ class WKVTimeMix(Mixer):
             decay = step.ws.get("wkv_decay", (n, self.nh, 16 * K.glr_rows_per_lane(self.d)), torch.float32)
             K.wkv_scan_pieces(rows, self.w0, self.u, o, state, step.slots, cu, numbers, piece_state, decay, step.n_seqs, pieces,
                               self.nh, self.d, self.d)
-        else:
-            K.wkv_scan(rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, step.n_seqs, self.nh, self.d, self.d)
+        elif walk:
+            K.wkv_scan(rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, step.n_seqs, self.nh, self.d, self.d,
+                       below=rest.get("below", 0))
         y = step.ws.get("wkv_y", (T, hd), dt)
         K.head_norm_gate(o, self.norm_w, rows[:, 4 * hd:5 * hd], y, self.nh, self.d, self.eps)
         linear(y, self.w_o, x, step.ws, accumulate=True)

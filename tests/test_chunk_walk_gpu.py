@@ -262,3 +262,48 @@ def test_error_beside_the_walk_token_by_token(form, decay, T):
     # than its last token is at most five of them: the value or its correction, the write factor, their product and two sums
     assert out < 1.12 * out_walk, (out, out_walk)
     assert state < max(1.12 * state_walk, 2 ** -24), (state, state_walk)
+
+
+@pytest.mark.parametrize("form", ["glr", "wkv", "fixed", "delta", "channels"])
+@pytest.mark.parametrize("lens", [(96, 1, 1, 200, 1), (95, 130, 96, 2, 1), (1, 1, 97)])
+def test_long_sequences_in_chunks_beside_others_token_by_token(form, lens):
+    """The two launches of a mixed step, each over its own sequences: the bits of each kernel over all of them."""
+    from braidinfer_amd import kernels as K
+    H, d, e, T, B = 3, 64, 32, sum(lens), len(lens)
+    g = torch.Generator().manual_seed(T)
+    i = {n: x.cuda() if torch.is_tensor(x) else x for n, x in inputs(form, T, H, H, d, e, False, g).items()}
+    form = "delta" if form == "channels" else form
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32).cuda()
+    slots = torch.arange(B, dtype=torch.int32).cuda()
+    slots[-2] = -1                                           # a padding sequence
+    first = torch.randn((B,) + tuple(K.glr_state_shape(H, d, e)), generator=g).cuda()
+    scratch = torch.empty(K.chunk_scratch_floats(T, B, H, d, e, form == "delta"), device="cuda")
+    wide = torch.cat([i["q"], i["k"], i["v"]] + ([i["z"]] if form == "wkv" else []), 1).contiguous()
+    hd, he = H * d, H * e
+    q, k, v = wide[:, :hd], wide[:, hd:2 * hd], wide[:, 2 * hd:2 * hd + he]
+    rest = {n: x for n, x in i.items() if n not in ("q", "k", "v", "z")}
+
+    def chunks(out, state, least):
+        z = {"z": wide[:, 2 * hd + he:]} if form == "wkv" else {}
+        K.chunk_scan(form, q, k, v, out, state, cu, slots, scratch, B, H, H, d, e, max(lens), least=least, **z, **rest)
+
+    def walk(out, state, **kw):
+        if form == "glr":
+            K.glr_scan(wide, i["b1"], i["b2"], out, state, cu, slots, B, H, d, e, **kw)
+        elif form == "wkv":
+            kw.pop("singles", None)
+            K.wkv_scan(wide, i["b1"], i["b2"], out, state.view(B, -1), cu, slots, B, H, d, e, **kw)
+        else:
+            K.dr_scan(q, k, v, i.get("gb"), i.get("b1"), out, state, cu, slots, B, H, H, d, e, gc=i.get("gc"), **kw)
+
+    def run(*calls):
+        out, state = torch.full((T, he), 7.0, device="cuda"), first.clone()
+        for call in calls:
+            call(out, state)
+        return out, state
+    whole, token = run(lambda o, s: chunks(o, s, 0)), run(lambda o, s: walk(o, s))
+    few = max(n for n in lens if n < 96) <= 1
+    both = run(lambda o, s: chunks(o, s, 96), lambda o, s: walk(o, s, below=96, singles=few))
+    for b, n in enumerate(lens):
+        want, at = (whole if n >= 96 else token), slice(int(cu[b]), int(cu[b + 1]))
+        assert torch.equal(both[0][at], want[0][at]) and torch.equal(both[1][b], want[1][b]), (b, n)
