@@ -203,11 +203,14 @@ __global__ __launch_bounds__(64) void glr_carry_kernel(float* __restrict__ state
     }
 }
 
-// The same walk, the same order of sums, for steps of single tokens: a lane asks for the rows it holds straight from memory
-// together with its part of the state, with no chunk in LDS (whose other 15 tokens' gates are work for nothing) and no
-// barrier, so that a compute unit holds twice the waves and each waits once.  Bound by the state, read and written once.
-// 32 heads of 128 x 128, the chunks' walk before / this: 1 sequence 4.2 / 3.4 us, 8 10.2 / 8.8, 40 43 / 36, 64 (268 MB) 69 / 57.
-template <int RPL, bool V4>
+// The same walk, the same order of sums, for steps of single tokens: a lane asks for the rows it holds, and for their biases and
+// bounds, straight from memory 16 bytes at a time together with its part of the state, with no chunk in LDS (whose other 15
+// tokens' gates are work for nothing) and no barrier, so that a compute unit holds twice the waves and each waits once.  Bound by
+// the state, read and written once.  32 heads of 128 x 128 with bias and bounds, the chunks' walk before / this: 40 sequences
+// 47 / 30 us, 64 (268 MB) 72 / 46 (5.8 TB/s); up to 8 both take the launch.  Element by element, as rows that do not lie at
+// multiples of 16 bytes would have it, the many small reads cost more than the chunks do (heads of 126, 64 sequences: 231
+// against 75), so those keep the chunks' walk.
+template <int RPL>
 __global__ __launch_bounds__(256) void glr_token_kernel(
     const float* __restrict__ rows, const float* __restrict__ f_bias, const float* __restrict__ lower,
     float* __restrict__ o, float* __restrict__ state, const int* __restrict__ cu_seqlens,
@@ -225,28 +228,23 @@ __global__ __launch_bounds__(256) void glr_token_kernel(
     float st[RPL], lo[RPL], bias[RPL];
 #pragma unroll
     for (int r = 0; r < RPL; ++r) st[r] = S[(size_t)r * 64];
-    auto row = [&](float (&to)[RPL], const float* from, bool vec) {
+    auto row = [&](float (&to)[RPL], const float* from) {
 #pragma unroll
         for (int r4 = 0; r4 < RPL; r4 += 4) {
-            if (vec) {
-                const f32x4 w = *(const f32x4*)(from + (g * RPL + r4 < d ? g * RPL + r4 : 0));
+            const f32x4 w = *(const f32x4*)(from + (g * RPL + r4 < d ? g * RPL + r4 : 0));
 #pragma unroll
-                for (int x = 0; x < 4; ++x) to[r4 + x] = w[x];
-            } else {
-#pragma unroll
-                for (int x = 0; x < 4; ++x) to[r4 + x] = g * RPL + r4 + x < d ? from[g * RPL + r4 + x] : 0.f;
-            }
+            for (int x = 0; x < 4; ++x) to[r4 + x] = w[x];
         }
     };
 #pragma unroll
     for (int r = 0; r < RPL; ++r) lo[r] = bias[r] = 0.f;
-    if (lower) row(lo, lower + h * d, false);
-    if (f_bias) row(bias, f_bias + h * d, false);
+    if (lower) row(lo, lower + h * d);
+    if (f_bias) row(bias, f_bias + h * d);
     for (int t = t0; t < t1; ++t) {
         const float* at = rows + (size_t)t * width + h * d;
         float q[RPL], f[RPL];
-        row(q, at, V4);
-        row(f, at + hd, V4);
+        row(q, at);
+        row(f, at + hd);
         const float vc = live ? rows[(size_t)t * width + 2 * hd + h * e + c] : 0.f;
         float sum = 0.f;
 #pragma unroll
@@ -284,9 +282,8 @@ static int glr_scan_launch(const float* rows, const float* f_bias, const float* 
     // 16-byte loads where every row piece starts at a multiple of 16 bytes
     const bool v4 = d % 4 == 0 && width % 4 == 0 && ((uintptr_t)rows % 16) == 0;
 #define GLR_SCAN(R, TC) do { \
-        if (!LOCAL && singles) { \
-            if (v4) glr_token_kernel<R, true><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
-            else glr_token_kernel<R, false><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
+        if (!LOCAL && singles && v4 && (((uintptr_t)f_bias | (uintptr_t)lower) % 16) == 0) { \
+            glr_token_kernel<R><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
             break; \
         } \
         const size_t lds = (size_t)(4 * TC * R * 16 + 2 * TC * 16) * sizeof(float); \

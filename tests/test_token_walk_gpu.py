@@ -65,3 +65,23 @@ def test_gated(gates, H, d, e):
         K.glr_scan(rows_all[rows].contiguous(), bias, lower, out, state, cu, slots, B + 1, H, d, e)
         return [out]
     _one_by_one(walk, K.glr_state_shape(H, d, e), T, B)
+
+
+def test_gates_at_any_address():
+    """Biases and bounds at odd multiples of 4 bytes (the chunks' walk takes those): the same bits as at multiples of 16."""
+    from braidinfer_amd import kernels as K
+    H, d, e, B = 3, 64, 32, 5
+    g = torch.Generator().manual_seed(1)
+    rows, first = _rand(g, B, 2 * H * d + H * e), _rand(g, B, *K.glr_state_shape(H, d, e))
+    vectors = [_rand(g, H * d + 4), torch.rand(H * d + 4, generator=g).cuda()]
+    cu, slots = torch.arange(B + 1, dtype=torch.int32).cuda(), torch.arange(B, dtype=torch.int32).cuda()
+
+    def run(bias, lower):
+        out, state = torch.zeros(B, H * e, device="cuda"), first.clone()
+        K.glr_scan(rows, bias, lower, out, state, cu, slots, B, H, d, e)
+        return out, state
+    moved = [v[1:1 + H * d] for v in vectors]
+    dense = [v.clone() for v in moved]
+    want = run(*dense)
+    for got in (run(*moved), run(moved[0], dense[1]), run(dense[0], moved[1])):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
