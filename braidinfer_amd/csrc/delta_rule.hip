@@ -698,11 +698,14 @@ __global__ __launch_bounds__(256) void dr_scan_kernel(const DrScan p) {
 //     8           9.4 / 8.6      9.7 / 8.2      11.3 / 8.5
 //     40          43 / 37.5      42 / 36        55 / 38        53 / 37
 //     64          64 / 58        62 / 57        87 / 59        86 / 58          (268 MB: 4.7 TB/s)
-// V4: k, q and the decays 16 bytes at a time.
+// V4: k, q and the decays 16 bytes at a time.  Rows that do not lie so keep the chunks' walk, since element by element every column's
+// lanes pay for as many reads as rows (heads of 126, 64 sequences: 126 against 45 us, with channels' decays 179 against 60), unless
+// silu has the four columns share them (50 against 67).
 template <int RPL, int MODE, bool SILU, bool V4>
 __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
     constexpr bool DELTA = MODE == DR_DELTA || MODE == DR_CHANNELS, CHAN = MODE == DR_CHANNELS;
     constexpr bool TOKEN_G = MODE != DR_FIXED;
+    static_assert(V4 || SILU, "rows element by element: only where the columns share them");
     const int H = p.H, d = p.d, e = p.e;
     const int s = blockIdx.x, h = blockIdx.y, cb16 = blockIdx.z;
     const int kh = h / (H / p.G);
@@ -730,15 +733,10 @@ __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
     auto row = [&](float (&to)[RPL], const float* from, float pad) {
 #pragma unroll
         for (int r4 = 0; r4 < RPL; r4 += 4) {
-            if (V4) {
-                const bool ok = g * RPL + r4 < d;
-                const f32x4 w = *(const f32x4*)(from + (ok ? g * RPL + r4 : 0));
+            const bool ok = g * RPL + r4 < d;
+            const f32x4 w = *(const f32x4*)(from + (ok ? g * RPL + r4 : 0));
 #pragma unroll
-                for (int x = 0; x < 4; ++x) to[r4 + x] = ok ? w[x] : pad;
-            } else {
-#pragma unroll
-                for (int x = 0; x < 4; ++x) to[r4 + x] = g * RPL + r4 + x < d ? from[g * RPL + r4 + x] : pad;
-            }
+            for (int x = 0; x < 4; ++x) to[r4 + x] = ok ? w[x] : pad;
         }
     };
     for (int t = t0; t < t1; ++t, orow += ostep) {
@@ -827,8 +825,8 @@ static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, int single
     dim3 grid(B, a.H, (cols + 15) / 16);
     const bool v4 = a.d % 4 == 0 && a.qk_stride % 4 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.gc) % 16) == 0;
 #define DR_GO(R, TC, M, A) do { \
-        if constexpr (!LOCAL) if (singles) { \
-            if (v4) dr_token_kernel<R, M, A, true><<<grid, 256, 0, s>>>(a); else dr_token_kernel<R, M, A, false><<<grid, 256, 0, s>>>(a); \
+        if constexpr (!LOCAL) if (singles && (v4 || A)) { \
+            if (v4) dr_token_kernel<R, M, A, true><<<grid, 256, 0, s>>>(a); else dr_token_kernel<R, M, A, !A><<<grid, 256, 0, s>>>(a); \
             break; \
         } \
         const size_t lds = (size_t)((M == DR_CHANNELS ? 6 : 4) * TC * R * 16 + 2 * TC * 16 + 2 * TC * 2) * sizeof(float); \
