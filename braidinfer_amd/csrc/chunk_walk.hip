@@ -44,8 +44,19 @@ __device__ __forceinline__ double cw_sum(const float* x) {
     else return cw_sum<N / 2>(x) + cw_sum<N / 2>(x + N / 2);
 }
 
-// Where a sequence's chunks lie in the scratch: sequence s has room for ceil(tokens / 16) chunks from cu[s] / 16 + s on.
-__device__ __forceinline__ int cw_first(const int* cu, int s) { return cu[s] / CW_C + s; }
+// Which chunks a launch is over, and where a sequence's lie in the scratch.  All at once (`run` 0): sequence s has room for
+// ceil(tokens / 16) chunks from cu[s] / 16 + s on.  Where the scratch is smaller: chunks `from` .. from + run of every sequence,
+// those of the i-th of the `longs` sequences of at least `least` tokens from i run on; the states wait in their slots
+// between the launches, so the bits are the same.
+struct CwPart {
+    int least, longs, from, run;
+};
+__device__ __forceinline__ int cw_first(const int* cu, int s, const CwPart& part) {
+    if (!part.run) return cu[s] / CW_C + s;
+    int rank = 0;
+    for (int i = 0; i < s; ++i) rank += cu[i + 1] - cu[i] >= part.least;
+    return rank < part.longs ? rank * part.run : -1;
+}
 // Floats of a (chunk, head) in the scratch: read factors 16 D | write factors 16 D | A 256 | the chunk's decay D | what its
 // rounding left D, and for the delta rule -W 16 D | U 16 e.
 __host__ __device__ constexpr int cw_block(int D, int e, bool delta) { return 34 * D + 256 + (delta ? 16 * (D + e) : 0); }
@@ -66,12 +77,11 @@ struct CwIn {
     size_t qk_stride, v_stride;
     const int *cu, *slots;
     int H, G, e, silu;
-    int least;            // sequences that bring fewer tokens are left alone
 };
 
-// grid (chunks of the longest sequence, H, sequences), D threads, a thread a channel.
+// grid (chunks of the longest sequence in the launch, H, sequences), D threads, a thread a channel.
 template <int FORM, int D>
-__global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* __restrict__ scratch) {
+__global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const CwPart run, float* __restrict__ scratch) {
     constexpr bool DELTA = FORM == CW_DELTA, WKV = FORM == CW_WKV;
     constexpr int KB = D / 16;
     __shared__ __attribute__((aligned(16))) float stage[KB * 272];        // read factors: [channel / 16][channel % 16 / 4][token][4], padded
@@ -79,8 +89,10 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
     __shared__ __attribute__((aligned(16))) float Lm[DELTA ? 256 : 4];
     const int s = blockIdx.z, h = blockIdx.y, c = threadIdx.x, H = in.H, e = in.e;
     if (in.slots[s] < 0) return;
-    const int t0 = in.cu[s] + (int)blockIdx.x * CW_C, n = min(CW_C, in.cu[s + 1] - t0);
-    if (n <= 0 || in.cu[s + 1] - in.cu[s] < in.least) return;
+    const int t0 = in.cu[s] + (run.from + (int)blockIdx.x) * CW_C, n = min(CW_C, in.cu[s + 1] - t0);
+    if (n <= 0 || in.cu[s + 1] - in.cu[s] < run.least) return;
+    const int first = cw_first(in.cu, s, run);
+    if (first < 0) return;
     const int kh = h / (H / in.G);
     float q[CW_C], k[CW_C], w[CW_C], beta[DELTA ? CW_C : 1];
     const float bias = (FORM == CW_GLR || WKV) && in.b1 ? in.b1[h * D + c] : 0.f, low = (FORM == CW_GLR || WKV) && in.b2 ? in.b2[h * D + c] : 0.f;
@@ -118,7 +130,7 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, float* 
             *x = y / (1.0f + expf(-y));
         }
     }
-    float* out = scratch + ((size_t)(cw_first(in.cu, s) + blockIdx.x) * H + h) * cw_block(D, e, DELTA);
+    float* out = scratch + ((size_t)(first + (int)blockIdx.x) * H + h) * cw_block(D, e, DELTA);
     // A (and L): 136 (120) sums over the channels, 16 lanes at a time here
     int pair = 0;
 #pragma unroll
@@ -240,7 +252,7 @@ template <int D, int CB, int S, bool DELTA>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
                                                          float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
-                                                         int zero_padding, int least) {
+                                                         int zero_padding, const CwPart run) {
     constexpr int NKB = D / 64, RPL = D / 16, STAGE = ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4, L = (DELTA ? 3 : 2) * NKB + 1;
     constexpr int PB = DELTA ? 1 : 2;                         // buffers of output quarters
     const int BLOCK = cw_block(D, e, DELTA);
@@ -250,8 +262,14 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     const int s = blockIdx.x / H, h = blockIdx.x - s * H, cb = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int slot = slots[s], t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1], he = H * e;
-    if (t1 - t0 < least) return;
+    const int slot = slots[s], he = H * e;
+    int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
+    const int first = cw_first(cu_seqlens, s, run);
+    if (t1 - t0 < run.least || first < 0) return;
+    if (run.run) {
+        t0 += run.from * CW_C;
+        t1 = min(t1, t0 + run.run * CW_C);
+    }
     if (slot < 0) {
         if (zero_padding)
             for (int i = tid; i < (t1 - t0) * 16; i += 256) for (int x = 0; x < CB; ++x) o[(size_t)(t0 + (i >> 4)) * he + h * e + (cb * CB + x) * 16 + (i & 15)] = 0.f;
@@ -260,7 +278,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     const int nch = (t1 - t0 + CW_C - 1) / CW_C;
     if (nch <= 0) return;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
-    const float* blocks = scratch + ((size_t)cw_first(cu_seqlens, s) * H + h) * BLOCK;
+    const float* blocks = scratch + ((size_t)first * H + h) * BLOCK;
     // a stage: read factors | write factors | A | both parts of the decay | values (256 floats each of the last three); a lane's byte offsets
     // within a chunk's block, the block itself is a scalar address that goes on by a chunk's blocks
     unsigned qoff[NKB], koff[NKB];
@@ -467,14 +485,15 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
 
 // Whether a head of d x e goes this way.
 extern "C" int br_chunk_takes(int d, int e) { return (d == 64 || d == 128) && e > 0 && e % 16 == 0; }
-// Floats of scratch for T tokens of B sequences.
+// Floats of scratch for a chunk of all heads, and for all of T tokens of B sequences at once.
+extern "C" size_t br_chunk_block(int H, int d, int e, int delta) { return (size_t)H * (size_t)cw_block(d, e, delta != 0); }
 extern "C" size_t br_chunk_scratch(int T, int B, int H, int d, int e, int delta) {
-    return (size_t)(T / CW_C + B + 1) * H * (size_t)cw_block(d, e, delta != 0);
+    return (size_t)(T / CW_C + B + 1) * br_chunk_block(H, d, e, delta);
 }
 
 template <int D, int CB, int S, bool DELTA>
-static int chunk_walk(const CwIn& in, const float* scratch, float* o, float* state, size_t slot_stride, int B, int zero_padding,
-                      hipStream_t s) {
+static int chunk_walk(const CwIn& in, const CwPart& part, const float* scratch, float* o, float* state, size_t slot_stride, int B,
+                      int zero_padding, hipStream_t s) {
     constexpr size_t lds = (size_t)S * ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4 + (DELTA ? 1 : 2) * 4 * CB * 272 * 4 + (DELTA ? 4096 * CB : 0);
     static_assert(lds <= 160 * 1024, "LDS");
     auto walk = chunk_walk_kernel<D, CB, S, DELTA>;
@@ -483,14 +502,15 @@ static int chunk_walk(const CwIn& in, const float* scratch, float* o, float* sta
         if (hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
         set = true;
     }
-    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding, in.least);
+    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding, part);
     return br_check_launch();
 }
 
 template <int FORM, int D>
-static int chunk_run(const CwIn& in, float* o, float* state, size_t slot_stride, float* scratch, int B, int max_new, hipStream_t s) {
+static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state, size_t slot_stride, float* scratch, int B, int chunks,
+                     hipStream_t s) {
     constexpr bool DELTA = FORM == CW_DELTA;
-    chunk_prepare_kernel<FORM, D><<<dim3((max_new + CW_C - 1) / CW_C, in.H, B), D, 0, s>>>(in, scratch);
+    chunk_prepare_kernel<FORM, D><<<dim3(chunks, in.H, B), D, 0, s>>>(in, part, scratch);
     const int rc = br_check_launch();
     if (rc != BR_OK) return rc;
     // 16 columns a workgroup where that gives no more workgroups than compute units (two to each for heads of 64); beyond, 32
@@ -500,7 +520,7 @@ static int chunk_run(const CwIn& in, float* o, float* state, size_t slot_stride,
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
     const long long units = (long long)B * in.H * (in.e / 16);
-#define CW_WALK(CB, S) return chunk_walk<D, CB, S, DELTA>(in, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
+#define CW_WALK(CB, S) return chunk_walk<D, CB, S, DELTA>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
     if (in.e % 32 || units <= (D == 64 ? 2 : 1) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
     if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
     else {
@@ -511,26 +531,34 @@ static int chunk_run(const CwIn& in, float* o, float* state, size_t slot_stride,
 }
 
 // One step's tokens of B sequences (`max_new` the most a sequence brings) through a recurrence (see CwIn for the forms' inputs),
-// from and into the slots' states; `scratch`: br_chunk_scratch floats.  Sequences of fewer than `least` tokens are left alone: their
-// outputs and states are another kernel's.
+// from and into the slots' states.  Sequences of fewer than `least` tokens are left alone: their outputs and states are another
+// kernel's.  `scratch`: br_chunk_scratch floats, or fewer, then the chunks are taken in several launches; at least a chunk of each of
+// the `longs` sequences that are not left alone.
 extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v, size_t qk_stride, size_t v_stride, const float* z,
                              const float* b1, const float* b2, const float* gb, const float* gc, int silu, float* o, float* state,
                              size_t slot_stride, const int* cu_seqlens, const int* slots, float* scratch, size_t scratch_floats, int T,
-                             int B, int H, int G, int d, int e, int max_new, int least, hipStream_t s) {
+                             int B, int H, int G, int d, int e, int max_new, int least, int longs, hipStream_t s) {
     if (B <= 0 || T <= 0) return BR_OK;
     if (!br_chunk_takes(d, e) || H <= 0 || H > 65535 || B > 65535 || (long long)B * H > 0x7fffffffLL || e / 16 > 65535 || max_new <= 0 ||
         max_new > T || G <= 0 || H % G || form < CW_GLR || form > CW_DELTA || v_stride % 4 || ((uintptr_t)v | (uintptr_t)scratch) % 16 ||
         v_stride >= (1ull << 26) || slot_stride < (size_t)H * ((e + 3) / 4) * d * 4 ||
-        scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA) || (form == CW_WKV && (!z || !b1 || !b2)) ||
+        longs <= 0 || longs > B || scratch_floats < longs * br_chunk_block(H, d, e, form == CW_DELTA) || (form == CW_WKV && (!z || !b1 || !b2)) ||
         (form == CW_FIXED && !b1) || (form == CW_DELTA && !gb) || ((form == CW_GLR || form == CW_WKV) && G != H))
         return BR_BAD_ARG;
-    const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu, least};
-#define CW_RUN(F) return d == 64 ? chunk_run<F, 64>(in, o, state, slot_stride, scratch, B, max_new, s) : chunk_run<F, 128>(in, o, state, slot_stride, scratch, B, max_new, s)
-    switch (form) {
-        case CW_GLR: CW_RUN(CW_GLR);
-        case CW_WKV: CW_RUN(CW_WKV);
-        case CW_FIXED: CW_RUN(CW_FIXED);
-        default: CW_RUN(CW_DELTA);
-    }
+    const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu};
+    const int all = (max_new + CW_C - 1) / CW_C;
+    int run = all;
+    if (scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA)) {
+        const size_t room = scratch_floats / br_chunk_block(H, d, e, form == CW_DELTA) / longs;
+        run = room < (size_t)all ? (int)room : all;
+    } else longs = 0;
+    for (int from = 0; from < all; from += run) {
+        const CwPart part = {least, longs, from, longs ? run : 0};
+        const int chunks = all - from < run ? all - from : run;
+#define CW_RUN(F) d == 64 ? chunk_run<F, 64>(in, part, o, state, slot_stride, scratch, B, chunks, s) : chunk_run<F, 128>(in, part, o, state, slot_stride, scratch, B, chunks, s)
+        const int rc = form == CW_GLR ? CW_RUN(CW_GLR) : form == CW_WKV ? CW_RUN(CW_WKV) : form == CW_FIXED ? CW_RUN(CW_FIXED) : CW_RUN(CW_DELTA);
 #undef CW_RUN
+        if (rc != BR_OK) return rc;
+    }
+    return BR_OK;
 }

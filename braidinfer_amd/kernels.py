@@ -895,19 +895,28 @@ def chunk_takes(d: int, e: int) -> bool:
     return d in (64, 128) and e > 0 and e % 16 == 0
 
 
+def chunk_block_floats(H: int, d: int, e: int, delta: bool = False) -> int:
+    """Floats of scratch that `chunk_scan` takes for 16 tokens of a sequence."""
+    return H * (34 * d + 256 + (16 * (d + e) if delta else 0))
+
+
 def chunk_scratch_floats(T: int, B: int, H: int, d: int, e: int, delta: bool = False) -> int:
-    return (T // 16 + B + 1) * H * (34 * d + 256 + (16 * (d + e) if delta else 0))
+    """Floats of scratch with which `chunk_scan` takes all tokens of a step at once."""
+    return (T // 16 + B + 1) * chunk_block_floats(H, d, e, delta)
 
 
 def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
                cu_seqlens: torch.Tensor, slots: torch.Tensor, scratch: torch.Tensor, B: int, H: int, G: int, d: int, e: int,
                max_new: int, z: Optional[torch.Tensor] = None, b1: Optional[torch.Tensor] = None, b2: Optional[torch.Tensor] = None,
-               gb: Optional[torch.Tensor] = None, gc: Optional[torch.Tensor] = None, silu: bool = False, least: int = 0) -> None:
+               gb: Optional[torch.Tensor] = None, gc: Optional[torch.Tensor] = None, silu: bool = False, least: int = 0,
+               longs: Optional[int] = None) -> None:
     """A recurrence over a step of prompts, 16 tokens at a time on the matrix cores: form "glr" as `glr_scan` (k the gates'
     sums, b1 their bias, b2 their lower bounds), "wkv" as `wkv_scan` (z the decays' sums, b1 their bias, b2 the bonus), "fixed"
     as `dr_scan` with `g_head` (b1; `silu` is applied to q, k and v, the latter in place) and "delta" as `dr_scan` with `gb`
     (and `gc`).  q, k, v: float rows, views of wider ones allowed (q, k and z with one stride); `max_new`: the most tokens a
-    sequence brings; `scratch` float32, `chunk_scratch_floats` of them.  Sequences of fewer than `least` tokens are left alone."""
+    sequence brings.  Sequences of fewer than `least` tokens are left alone, `longs` (None: B) are not.  `scratch` float32,
+    `chunk_scratch_floats` of them; with fewer (at least `longs` times `chunk_block_floats`) the chunks are taken in several runs,
+    to the same bits."""
     _req(form in ("glr", "wkv", "fixed", "delta"), f"chunk_scan: form {form!r}")
     number = ("glr", "wkv", "fixed", "delta").index(form)
     T = q.shape[0]
@@ -931,12 +940,13 @@ def chunk_scan(form: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out
     _req(gb is None or (gb.dtype == torch.float32 and gb.shape == (T, 2 * H)), "chunk_scan: gb float32 [T, 2*H]")
     _req(gc is None or (gc.dtype == torch.float32 and gc.shape == (T, H * d)), "chunk_scan: gc float32 [T, H*d]")
     _req(cu_seqlens.numel() >= B + 1 and slots.numel() >= B, "chunk_scan: arrays shorter than the batch")
-    _req(scratch.numel() >= chunk_scratch_floats(T, B, H, d, e, form == "delta"), "chunk_scan: scratch too small")
+    longs = B if longs is None else int(longs)
+    _req(0 < longs <= B and scratch.numel() >= longs * chunk_block_floats(H, d, e, form == "delta"), "chunk_scan: scratch too small")
     f = _fn("chunk_walk", "br_chunk_scan", [c_int, _P, _P, _P, c_size_t, c_size_t] + [_P] * 5 + [c_int, _P, _P, c_size_t, _P, _P, _P, c_size_t]
-            + [c_int] * 8 + [_P])
+            + [c_int] * 9 + [_P])
     _check(f(number, _ptr(q), _ptr(k), _ptr(v), stride, v.stride(0), _ptr(z), _ptr(b1), _ptr(b2), _ptr(gb), _ptr(gc), int(silu), _ptr(out),
              _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots), _ptr(scratch), scratch.numel(), T, B, H, G, d, e, int(max_new),
-             int(least), _stream()), "chunk_scan")
+             int(least), longs, _stream()), "chunk_scan")
 
 
 def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, H: int, e: int, eps: float) -> None:

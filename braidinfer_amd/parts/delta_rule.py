@@ -39,7 +39,7 @@ from ..cache import StateNeed
 from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, RotaryTables, Runtime, register_part
-from .gated_recurrence import CHUNKS_FROM, HGRN2, chunk_scratch, in_chunks, pieces_for
+from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
 from .linear import fused_layout, linear, padded_rows, stream_layout
 
 
@@ -168,8 +168,8 @@ class GatedDeltaRule(Mixer):
         S = ctx.state[:, :self.state_floats].view((-1,) + tuple(K.glr_state_shape(nh, d, e)))
         chunks, walk, rest = in_chunks(step, d, e)
         if chunks:
-            K.chunk_scan("delta", q, k, v, o, S, step.cu_seqlens, step.slots, chunk_scratch(step, nh, d, e, True), step.n_seqs, nh, ng, d, e,
-                         step.max_new, gb=gb, gc=gc, least=CHUNKS_FROM)
+            K.chunk_scan("delta", q, k, v, o, S, step.cu_seqlens, step.slots, B=step.n_seqs, H=nh, G=ng, d=d, e=e,
+                         max_new=step.max_new, gb=gb, gc=gc, **chunk_scratch(step, nh, d, e, True))
         if walk:
             K.dr_scan(q, k, v, gb, None, o, S, step.cu_seqlens, step.slots, step.n_seqs, nh, ng, d, e, gc=gc, **rest)
         y = step.ws.get("dr_y", (T, nh * e), self.rt.dtype)
@@ -265,8 +265,8 @@ class LightningAttention(Mixer):
         pieces = 1 if chunks else pieces_for(step, nh * -(-e // 16), self.MIN_PIECE)
         if chunks:
             K.chunk_scan("fixed", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], o, ctx.state, step.cu_seqlens, step.slots,
-                         chunk_scratch(step, nh, d, e), step.n_seqs, nh, nh, d, e, step.max_new, b1=self.decay, silu=silu,
-                         least=CHUNKS_FROM)
+                         B=step.n_seqs, H=nh, G=nh, d=d, e=e, max_new=step.max_new, b1=self.decay, silu=silu,
+                         **chunk_scratch(step, nh, d, e))
         if pieces > 1:
             # long prompts: the recurrence is linear in the state, so every sequence is cut into pieces that are walked
             # side by side, twice

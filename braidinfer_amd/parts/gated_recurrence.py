@@ -64,8 +64,18 @@ def in_chunks(step, d: int, e: int) -> Tuple[bool, bool, dict]:
     return True, bool(rest), {"below": CHUNKS_FROM, "singles": max(rest, default=0) <= 1}
 
 
-def chunk_scratch(step, H: int, d: int, e: int, delta: bool = False) -> torch.Tensor:
-    return step.ws.get("chunk_scratch", (K.chunk_scratch_floats(step.n_tokens, step.n_seqs, H, d, e, delta),), torch.float32)
+# Bytes of scratch for the chunks' factors, which are 36 KB a token for 32 heads of 128 x 128 (delta rule 68 KB) and stay with the
+# engine: longer steps are taken in runs of chunks, each of which reads and writes the states once (one of 16,384 tokens:
+# HGRN2 1,143 us, all at once 1,128; delta rule 1,612 and 1,561).
+CHUNK_SCRATCH = 512 << 20
+
+
+def chunk_scratch(step, H: int, d: int, e: int, delta: bool = False) -> dict:
+    """`scratch`, and the arguments of `chunk_scan` that say which sequences it is for."""
+    longs = sum(n >= CHUNKS_FROM for n in step.host_new)
+    floats = min(K.chunk_scratch_floats(step.n_tokens, step.n_seqs, H, d, e, delta),
+                 max(CHUNK_SCRATCH // 4, longs * K.chunk_block_floats(H, d, e, delta)))
+    return {"scratch": step.ws.get("chunk_scratch", (floats,), torch.float32), "least": CHUNKS_FROM, "longs": longs}
 
 
 class HGRN2(Mixer):
@@ -143,8 +153,8 @@ class HGRN2(Mixer):
         if chunks:
             hd = nh * d
             K.chunk_scan("glr", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:], o, ctx.state, step.cu_seqlens, step.slots,
-                         chunk_scratch(step, nh, d, e), step.n_seqs, nh, nh, d, e, step.max_new, b1=self.f_bias, b2=self.lower,
-                         least=CHUNKS_FROM)
+                         B=step.n_seqs, H=nh, G=nh, d=d, e=e, max_new=step.max_new, b1=self.f_bias, b2=self.lower,
+                         **chunk_scratch(step, nh, d, e))
         if pieces > 1:
             cu, numbers = self._piece_arrays(step, pieces)
             n = step.n_seqs * pieces

@@ -27,7 +27,7 @@ from ..cache import StateNeed
 from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, Runtime, register_part
-from .gated_recurrence import CHUNKS_FROM, HGRN2, chunk_scratch, in_chunks, pieces_for
+from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
 from .linear import linear, stream_layout
 
 BRANCHES = ("r", "k", "v", "g", "w")
@@ -106,8 +106,9 @@ class WKVTimeMix(Mixer):
         pieces = 1 if chunks else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
         if chunks:
             r, k, v, z = (rows[:, i * hd:(i + 1) * hd] for i in range(4))
-            K.chunk_scan("wkv", r, k, v, o, state, step.cu_seqlens, step.slots, chunk_scratch(step, self.nh, self.d, self.d), step.n_seqs,
-                         self.nh, self.nh, self.d, self.d, step.max_new, z=z, b1=self.w0, b2=self.u, least=CHUNKS_FROM)
+            K.chunk_scan("wkv", r, k, v, o, state, step.cu_seqlens, step.slots, B=step.n_seqs, H=self.nh, G=self.nh,
+                         d=self.d, e=self.d, max_new=step.max_new, z=z, b1=self.w0, b2=self.u,
+                         **chunk_scratch(step, self.nh, self.d, self.d))
         if pieces > 1:
             # long prompts: every sequence cut into pieces that are walked side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)

@@ -307,3 +307,38 @@ def test_long_sequences_in_chunks_beside_others_token_by_token(form, lens):
     for b, n in enumerate(lens):
         want, at = (whole if n >= 96 else token), slice(int(cu[b]), int(cu[b + 1]))
         assert torch.equal(both[0][at], want[0][at]) and torch.equal(both[1][b], want[1][b]), (b, n)
+
+
+@pytest.mark.parametrize("form", ["glr", "wkv", "fixed", "delta"])
+def test_chunks_in_runs_where_the_scratch_is_small(form):
+    """Fewer chunks at once: the same bits, nothing written behind the scratch, too little of it refused."""
+    from braidinfer_amd import kernels as K
+    from braidinfer_amd.errors import KernelError
+    H, d, e, lens = 3, 64, 32, (400, 1, 130, 96, 20, 97)
+    T, B, longs = sum(lens), len(lens), 4
+    g = torch.Generator().manual_seed(5)
+    i = {n: x.cuda() if torch.is_tensor(x) else x for n, x in inputs(form, T, H, H, d, e, form == "fixed", g).items()}
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32).cuda()
+    slots = torch.arange(B, dtype=torch.int32).cuda()
+    slots[2] = -1
+    first = torch.randn((B,) + tuple(K.glr_state_shape(H, d, e)), generator=g).cuda()
+    wide = torch.cat([i["q"], i["k"], i["v"]] + ([i["z"]] if form == "wkv" else []), 1).contiguous()
+    hd, he, block = H * d, H * e, K.chunk_block_floats(H, d, e, form == "delta")
+    rest = {n: x for n, x in i.items() if n not in ("q", "k", "v", "z")}
+
+    def run(floats, **kw):
+        rows = wide.clone()                                  # silu goes back into the values
+        if form == "wkv":
+            kw["z"] = rows[:, 2 * hd + he:]
+        out, state, scratch = torch.full((T, he), 7.0, device="cuda"), first.clone(), torch.full((floats + 64,), 5.0, device="cuda")
+        K.chunk_scan(form, rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], out, state, cu, slots, scratch[:floats], B, H, H, d, e,
+                     max(lens), least=96, **kw, **rest)
+        assert torch.all(scratch[floats:] == 5.0)
+        return out, state
+    want = run(K.chunk_scratch_floats(T, B, H, d, e, form == "delta"))
+    assert torch.all(want[0][400] == 7.0) and torch.equal(want[1][1], first[1]) and not torch.equal(want[1][5], first[5])
+    for chunks in (1, 2, 5, 6, 7, 24):
+        for got in (run(longs * chunks * block + 40, longs=longs), run(B * chunks * block)):
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    with pytest.raises(KernelError):
+        run(longs * block - 4, longs=longs)

@@ -79,3 +79,14 @@ def test_every_sequence_by_its_own_tokens(monkeypatch, kind):
 def test_heads_that_chunks_do_not_take(monkeypatch, kind):
     assert set(itertools.chain(*(walks(monkeypatch, kind, lens, d=48) for lens in ((1, 1), (200, 1), (400,))))) == {"walk"}
     assert walks(monkeypatch, kind, (2000, 1), d=48) == ["walk" if kind == "delta" else "pieces"] * 2
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_scratch_of_long_steps_is_bounded(monkeypatch, delta):
+    H, d, e = 32, 128, 128
+    block = K.chunk_block_floats(H, d, e, delta)
+    for lens, floats in (((2048, 1), K.chunk_scratch_floats(2049, 2, H, d, e, delta)), ((200000, 1, 1), gated_recurrence.CHUNK_SCRATCH // 4),
+                         ((FROM,) * 2000, 2000 * block)):
+        a = gated_recurrence.chunk_scratch(Step(lens), H, d, e, delta)
+        assert a["scratch"].numel() == floats and a["least"] == FROM and a["longs"] == sum(n >= FROM for n in lens)
+        assert floats >= a["longs"] * block
