@@ -138,7 +138,7 @@ __global__ __launch_bounds__(512) void gemm_f32_stream_kernel(const float* __res
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     if (nitems > 0) issue(0);
     for (int it = 0; it < nitems; ++it) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         if (it + 1 < nitems) issue((it + 1) & 1);
         const unsigned char* st = ring + (it & 1) * STAGE;
         const int xr = XR == 8 ? (r16 & 7) : r16;
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
             ++seg;
             seg_end = (seg + 1) * nch / F32_SEGS * 2;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (kt + 1 < kt1) issue(kt + 1);
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
                     for (int j = 0; j < TJ; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
         }
-        // every wave has read this stage before the loop's next barrier lets the loads of the one after into it
+        // every wave's reads of this stage are waited for ahead of the loop's next barrier, behind which the loads of the one after go into it
     }
     if (SPLIT) C += (size_t)blockIdx.y * M * N;
 #pragma unroll

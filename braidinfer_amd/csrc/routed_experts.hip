@@ -862,8 +862,8 @@ __global__ __launch_bounds__(RXS_NW * 64) void experts_stream_kernel(const bf16*
         for (int j = 0; j < S; ++j) {
             const int it = base + j;
             if (it >= nitems) break;
-            if (it + D - 1 < nitems) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * NDMA) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (it + D - 1 < nitems) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((D - 1) * NDMA) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             if (it + D < nitems) issue((j + D) % S);
             const unsigned char* st = ring + j * STAGE;
             const int xr = XR == 8 ? (r16 & 7) : r16;
