@@ -714,7 +714,6 @@ __global__ __launch_bounds__(256) void experts_down_grouped_kernel(const bf16* _
 // against 253 / 133; 40 tokens 161 / 102 against 277 / 141.  Bound by the memory up to about 16 pairs an expert.
 //   UP: unit t is gate rows 8 t .. + 8 and the up rows of the same channels; y[p, f] = the gated unit, bfloat16.
 //   else: unit t is rows 16 t .. + 16 of W_d; out[p, n] float.
-#define RXS_TOKENS 64               // up to here, or up to eight pairs an expert on average: beyond, rows are read again too often
 #define RXS_KC 128
 #define RXS_NW 8
 #define RXS_S 2
@@ -935,14 +934,15 @@ static int rx_launch_stream(const void* A, const void* Wt, const int* first, con
     return br_check_launch();
 }
 
-// Whether the grouped kernels take these sizes: rows of 16 bytes' multiples.
+// Whether the grouped kernels take these sizes: rows of 16 bytes' multiples.  `stream`: the caller finds the pairs few enough for
+// the stream to pay; it is used where it can be.
 extern "C" int br_experts_grouped_takes(int W, int F) { return W > 0 && F > 0 && W % 8 == 0 && F % 8 == 0; }
 
 extern "C" int br_experts_up_grouped(const void* h, const void* w_gu, const int* first, const int* order, void* y, int E,
-                                     int W, int F, int top, int n_tokens, float limit, float alpha, hipStream_t s) {
+                                     int W, int F, int top, int n_tokens, float limit, float alpha, int stream, hipStream_t s) {
     if (!br_experts_grouped_takes(W, F) || E <= 0 || top <= 0 || (F + 31) / 32 > 65535) return BR_BAD_ARG;
     const int pairs = n_tokens * top;
-    if ((n_tokens <= RXS_TOKENS || pairs <= 8 * E) && rx_stream_takes(h, w_gu, n_tokens, pairs, E, 2 * F, W)) {
+    if (stream && rx_stream_takes(h, w_gu, n_tokens, pairs, E, 2 * F, W)) {
         if (n_tokens <= 8) return rx_launch_stream<8, true>(h, w_gu, first, order, y, E, F, W, top, limit, alpha, s);
         return rx_launch_stream<16, true>(h, w_gu, first, order, y, E, F, W, top, limit, alpha, s);
     }
@@ -953,9 +953,9 @@ extern "C" int br_experts_up_grouped(const void* h, const void* w_gu, const int*
 }
 
 extern "C" int br_experts_down_grouped(const void* y, const void* w_down, const int* first, float* out, int pairs, int E, int W, int F,
-                                       int n_tokens, hipStream_t s) {
+                                       int n_tokens, int stream, hipStream_t s) {
     if (!br_experts_grouped_takes(W, F) || E <= 0 || (W + 31) / 32 > 65535) return BR_BAD_ARG;
-    if ((n_tokens <= RXS_TOKENS || pairs <= 8 * E) && W % 16 == 0 && rx_stream_takes(y, w_down, pairs, pairs, E, W, F)) {
+    if (stream && W % 16 == 0 && rx_stream_takes(y, w_down, pairs, pairs, E, W, F)) {
         if (n_tokens <= 8) return rx_launch_stream<8, false>(y, w_down, first, nullptr, out, E, W, F, 1, 0.f, 0.f, s);
         return rx_launch_stream<16, false>(y, w_down, first, nullptr, out, E, W, F, 1, 0.f, 0.f, s);
     }

@@ -1452,9 +1452,9 @@ def experts_up_grouped(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor,
     _req(experts_grouped_takes(h.dtype, W, F2 // 2) and w_gu.dtype == y.dtype == torch.bfloat16, "experts_up_grouped: bfloat16, widths in steps of 8")
     _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
          and first.dtype == order.dtype == torch.int32, "experts_up_grouped: shapes")
-    f = _fn("routed_experts", "br_experts_up_grouped", [_P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P])
-    _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), E, W, F2 // 2, top, T, float(limit), float(alpha), _stream()),
-           "experts_up_grouped")
+    f = _fn("routed_experts", "br_experts_up_grouped", [_P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P])
+    _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), E, W, F2 // 2, top, T, float(limit), float(alpha),
+             int(_experts_stream_pays(T, n, E)), _stream()), "experts_up_grouped")
 
 
 def experts_down_grouped(y: torch.Tensor, w_down: torch.Tensor, first: torch.Tensor, out: torch.Tensor, n_tokens: int) -> None:
@@ -1464,14 +1464,20 @@ def experts_down_grouped(y: torch.Tensor, w_down: torch.Tensor, first: torch.Ten
     E, W, _ = w_down.shape
     _req(experts_grouped_takes(y.dtype, W, F) and w_down.dtype == torch.bfloat16 and out.dtype == torch.float32, "experts_down_grouped: types")
     _req(w_down.shape == (E, W, F) and out.shape == (n, W) and first.numel() in (E + 1, E + 2) and first.dtype == torch.int32, "experts_down_grouped: shapes")
-    f = _fn("routed_experts", "br_experts_down_grouped", [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P])
-    _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), n, E, W, F, int(n_tokens), _stream()), "experts_down_grouped")
+    f = _fn("routed_experts", "br_experts_down_grouped", [_P, _P, _P, _P] + [c_int] * 6 + [_P])
+    _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), n, E, W, F, int(n_tokens), int(_experts_stream_pays(n_tokens, n, E)), _stream()),
+           "experts_down_grouped")
+
+
+def _experts_stream_pays(tokens: int, pairs: int, experts: int) -> bool:
+    """Whether streaming the experts' weights through LDS pays against loading them straight into operands: up to 64 tokens or 8
+    pairs an expert on average; beyond, the stream reads an expert's rows again for every 16 of its pairs."""
+    return tokens <= 64 or pairs <= 8 * experts
 
 
 def experts_stream_takes(dtype: torch.dtype, W: int, F: int, pairs: int, experts: int) -> bool:
-    """Whether `experts_up_grouped` and `experts_down_grouped` stream these experts' weights for that many pairs."""
-    return (dtype == torch.bfloat16 and min(W, F) >= 1024 and W % 128 == 0 and F % 128 == 0 and pairs <= min(1024, 8 * experts)
-            and experts <= 512)
+    """Whether `experts_up_grouped` and `experts_down_grouped` can stream these experts' weights for that many pairs, both products."""
+    return (dtype == torch.bfloat16 and min(W, F) >= 1024 and W % 128 == 0 and F % 128 == 0 and pairs <= 1024 and experts <= 512)
 
 
 def _experts_gemm_tiles_take(N: int, Kd: int) -> bool:

@@ -229,10 +229,13 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             self.shared.load(tensors, prefix, rt)
 
-    # from this many tokens a step goes expert by expert through the matrix products (below it, every (token, slot)
-    # pair reads its expert's rows itself, which is what a step of few tokens costs anyway)
+    # For widths that the prompt products' tiles do not take (no steps of 64; float): from this many tokens of a prompt the rows are
+    # gathered and multiplied expert by expert, in one launch up to ONE_BY_ONE_FROM pairs an expert and by the library's products one
+    # expert after the other from there on; below, and in steps of single tokens, the kernels for few pairs read them.
+    # BRAIDINFER_EXPERTS_ONE_BY_ONE, for measurements and tests: 1 takes every prompt of as many tokens one expert after the other,
+    # whatever the widths, 0 none.
     BY_EXPERT_FROM = 48
-    ONE_BY_ONE_FROM = 1536          # pairs an expert from which the experts go one by one through the library's products
+    ONE_BY_ONE_FROM = 1536
 
     def _glu(self, gu, act) -> None:
         """The experts' activation of a gate/up product whose rows are dense."""
@@ -280,19 +283,22 @@ class RoutedExperts(FeedForward):
         order = step.ws.get("moe_order", (n,), torch.int32)
         place = step.ws.get("moe_place", (n,), torch.int32)
         K.experts_sort(chosen, first, order, place, bins)
-        forced = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "") == "1"          # for measurements
+        one_by_one = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "")
         # Up to eight pairs an expert on average, or sixteen tokens, the weights are streamed once for up to 16 pairs at a time;
-        # beyond, the prompt products' tiles read them once for 128 or 256 (32 experts of 1,792 by 4,096, 8 chosen, both
-        # products: 32 tokens 239 against 257 us, 40 tokens 257 against 256, 64 tokens 350 against 259).
+        # beyond, the prompt products' tiles read them once for 128 or 256.  Both products in us, streams against tiles: 32 experts of
+        # 1,792 by 4,096, 8 chosen: 32 tokens 239 / 257, 40 tokens 257 / 256, 64 tokens 350 / 259; 7 chosen: 32 tokens 251 / 254, 48
+        # tokens 262 / 255, 64 tokens 323 / 257.  16 experts of 1,408 by 2,048, 4 chosen: 16 tokens 54 / 74, 32 tokens 58 / 74, 48
+        # tokens 61 / 73, 64 tokens 81 / 74; 3 chosen: 48 tokens 56 / 71, 64 tokens 63 / 71, 96 tokens 91 / 72 (there the streams
+        # stay ahead up to twelve pairs an expert).
         streamed = (T <= 16 or n <= 8 * self.E) and (few or K.experts_stream_takes(dt, self.H, self.I, n, self.E))
-        if K.experts_tiles_take(dt, self.H, self.I, T) and not streamed and not forced:
+        if K.experts_tiles_take(dt, self.H, self.I, T) and not streamed and one_by_one != "1":
             y = step.ws.get("moe_y", (n, self.I), dt)
             K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             out = step.ws.get("moe_out", (n, self.H), torch.float32)
             K.experts_gemm(y, self.w_down, first, out)
             K.experts_combine(out, place, share, x, store=store, **ident)
             return
-        if few or (streamed and not forced):
+        if few or (streamed and one_by_one != "1"):
             # an expert's weights are read once for its pairs, nothing goes back to the host
             y = step.ws.get("moe_y", (n, self.I), dt)
             K.experts_up_grouped(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
@@ -306,7 +312,7 @@ class RoutedExperts(FeedForward):
         gu = step.ws.get("moe_gu", (n, 2 * self.I), dt)
         act = step.ws.get("moe_act", (n, self.I), dt)
         out = step.ws.get("moe_out", (n, self.H), torch.float32)
-        if K.experts_grouped_takes(dt, self.H, self.I) and not forced and n // self.E < self.ONE_BY_ONE_FROM:
+        if K.experts_grouped_takes(dt, self.H, self.I) and one_by_one != "1" and (one_by_one == "0" or n // self.E < self.ONE_BY_ONE_FROM):
             K.experts_gemm(rows, self.w_gu, first, gu)
             self._glu(gu, act)
             K.experts_gemm(act, self.w_down, first, out)

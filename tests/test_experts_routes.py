@@ -50,3 +50,32 @@ def test_tiles_say_what_they_take(W, F):
     assert not K.experts_tiles_take(torch.float32, W, F, 100)
     for w, f in ((W + 8, F), (W, F + 8), (2 ** 17, 2 ** 14), (2 ** 14, 2 ** 17)):          # matrices of 4 GB an expert
         assert not K.experts_tiles_take(torch.bfloat16, w, f, 100)
+
+
+FEW, GATHERED = ["experts_up_grouped", "experts_down_grouped"], ["experts_gather", "experts_gemm", "silu_mul", "experts_gemm"]
+
+
+@pytest.mark.parametrize("W,F,E,top", [(4096, 1792, 32, 8), (2048, 1408, 16, 4)])
+def test_few_pairs_and_many(monkeypatch, W, F, E, top):
+    for tokens, decode, want in ((1, True, FEW), (16, True, FEW), (32, True, FEW), (33, True, TILES), (200, True, TILES), (17, False, FEW),
+                                 (32, False, FEW), (33, False, TILES), (47, False, TILES), (48, False, TILES), (4000, False, TILES)):
+        assert route(monkeypatch, tokens, decode, W, F, E, top) == want, tokens
+
+
+def test_widths_that_the_tiles_do_not_take(monkeypatch):
+    for tokens, decode, want in ((1, True, FEW), (100, True, FEW), (47, False, FEW), (48, False, GATHERED), (6143, False, GATHERED),
+                                 (6144, False, GATHERED[:1])):
+        assert route(monkeypatch, tokens, decode, 96, 40, 8, 2) == want, tokens
+    assert route(monkeypatch, 5, False, 50, 9, 3, 2) == ["experts_up", "experts_down"]
+    assert route(monkeypatch, 5, True, dtype=torch.float32) == ["experts_up", "experts_down"]
+    assert route(monkeypatch, 50, False, dtype=torch.float32) == ["experts_gather"]
+
+
+def test_the_forced_routes(monkeypatch):
+    monkeypatch.setenv("BRAIDINFER_EXPERTS_ONE_BY_ONE", "1")
+    for W, F in ((4096, 1792), (96, 40)):
+        assert route(monkeypatch, 300, False, W, F) == ["experts_gather"]
+        assert route(monkeypatch, 300, True, W, F) == FEW
+    monkeypatch.setenv("BRAIDINFER_EXPERTS_ONE_BY_ONE", "0")
+    assert route(monkeypatch, 300, False) == TILES
+    assert route(monkeypatch, 100000, False, 96, 40, 8, 2) == GATHERED          # 25,000 pairs an expert, in one launch all the same
