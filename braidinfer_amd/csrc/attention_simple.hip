@@ -20,8 +20,8 @@
 #define MAX_DPL 8   // head_dim <= 64 * MAX_DPL
 
 // VEC: the rows of keys and the rows of a value channel are read 16 bytes at a time, in the same order of sums (head sizes in
-// steps of a 16-byte load, pages of whole 64s, aligned cache; a chunk that does not start with its page, as windows make
-// them, reads its values one by one).  Bound by the latency of those reads.  Short requests (3 sequences of
+// steps of a 16-byte load, pages of whole 64s, aligned cache; where a chunk does not start with its page, as windows make
+// them, the values up to the first such piece one by one).  Bound by the latency of those reads.  Short requests (3 sequences of
 // 29 to 163 tokens, 32 heads of 128 in float): a step of single tokens takes 12.8 us with a wave a class, the prompt 94 with one
 // wave for all; both forms with one wave and no classes averaged 35 over a prompt and six steps, one element a read 106.
 template <typename T> struct as_vec;
@@ -75,12 +75,16 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
     const size_t page_elems = (size_t)2 * nkv * page * hd;
     const size_t k_off = (size_t)kvh * page * hd, v_off = ((size_t)nkv + kvh) * page * hd;
 
-    auto walk = [&](int cls) {
+    auto nothing = []() {
         AsPart a;
         a.m = -INFINITY;
         a.l = 0.f;
 #pragma unroll
         for (int i = 0; i < MAX_DPL; ++i) a.acc[i] = 0.f;
+        return a;
+    };
+    auto walk = [&](int cls) {
+        AsPart a = nothing();
         for (int j0 = lo + 64 * cls; j0 <= p; j0 += 256) {
             const int j = j0 + lane;
             float s = -INFINITY;
@@ -110,11 +114,24 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
             const int nk = (p - j0 + 1) < 64 ? (p - j0 + 1) : 64;
 #pragma unroll
             for (int i = 0; i < MAX_DPL; ++i) a.acc[i] *= corr;
-            int jj = 0;
-            if (VEC && j0 % 64 == 0) {                   // the chunk lies in one page
-                const T* vc = cache + (size_t)bt[j0 / page] * page_elems + v_off + (j0 % page);
+            auto one = [&](int jj, const T* vc) {        // key jj of the chunk, its value's channels a page's row apart
+                const float pw = ps[jj];
+#pragma unroll
+                for (int i = 0; i < MAX_DPL; ++i) {
+                    const int d = lane + 64 * i;
+                    if (d < hd) a.acc[i] = fmaf(pw, to_f32<T>(vc[(size_t)d * page]), a.acc[i]);
+                }
+            };
+            for (int jj = 0; jj < nk;) {                 // page by page: a chunk lies in one, or in two behind a window's edge
+                const int off = (j0 + jj) % page, end = min(nk, jj + page - off);
+                const T* vc = cache + (size_t)bt[(j0 + jj) / page] * page_elems + v_off + off - jj;
+                if (!VEC) {
+                    for (; jj < end; ++jj) one(jj, vc + jj);
+                    continue;
+                }
+                for (; jj < end && (j0 + jj) % VN; ++jj) one(jj, vc + jj);
 #pragma unroll 4
-                for (; jj + VN <= nk; jj += VN) {
+                for (; jj + VN <= end; jj += VN) {
                     vec_t vv[MAX_DPL];
 #pragma unroll
                     for (int i = 0; i < MAX_DPL; ++i)
@@ -125,25 +142,18 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
 #pragma unroll
                             for (int e = 0; e < VN; ++e) a.acc[i] = fmaf(ps[jj + e], to_f32<T>(vv[i][e]), a.acc[i]);
                 }
-            }
-            for (; jj < nk; ++jj) {
-                const int jk = j0 + jj;
-                const T* vc = cache + (size_t)bt[jk / page] * page_elems + v_off + (jk % page);
-                const float pw = ps[jj];
-#pragma unroll
-                for (int i = 0; i < MAX_DPL; ++i) {
-                    const int d = lane + 64 * i;
-                    if (d < hd) a.acc[i] = fmaf(pw, to_f32<T>(vc[(size_t)d * page]), a.acc[i]);
-                }
+                for (; jj < end; ++jj) one(jj, vc + jj);
             }
             a.m = m_new;
         }
         return a;
     };
-    AsPart a = walk(WAVES == 1 ? 0 : wave);
+    AsPart a;
     if (WAVES == 1) {
-        for (int cls = 1; cls < 4 && lo + 64 * cls <= p; ++cls) as_join(a, walk(cls));
+        a = nothing();
+        for (int cls = 0; cls < 4 && lo + 64 * cls <= p; ++cls) as_join(a, walk(cls));
     } else {
+        a = walk(wave);
         float* mine = joinL + wave * (2 + hd);
         if (wave > 0) {
             if (lane == 0) { mine[0] = a.m; mine[1] = a.l; }

@@ -76,3 +76,33 @@ def test_scores_that_are_not_finite(keys, what):
             assert torch.equal(got.isnan(), want.isnan())
             if not want.isnan().any():
                 assert float((got.double() - want).abs().max()) < 4e-6 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hd,window", [(128, 100), (64, 65), (40, 3), (72, 129), (128, None)])
+def test_values_read_one_by_one_and_16_bytes_at_a_time(dtype, hd, window):
+    """Pages of 32 tokens read values one by one, pages of 64 and 128 16 bytes at a time from wherever a window's chunks start: the
+    same bits, for a query alone and among many."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(hd)
+    T, nq, nkv = 384, 2, 1
+    q, k, v = (torch.randn(T, n, hd, generator=g).to(dtype) for n in (nq, nkv, nkv))
+    qd, pos = q.reshape(T, nq * hd).cuda(), torch.arange(T, dtype=torch.int32).cuda()
+    zeros, slots = torch.zeros(20000, dtype=torch.int32).cuda(), torch.zeros(1, dtype=torch.int32).cuda()
+    some = torch.tensor([0, 1, 30, 63, 64, 99, 100, 101, 163, 200, 229, 383])
+    got = []
+    for page in (32, 64, 128):
+        n = T // page
+        pages = torch.randperm(n, generator=g)
+        cache = torch.empty(n, 2, nkv, page, hd, dtype=dtype)
+        cache[pages, 0, 0] = k[:, 0].reshape(n, page, hd)
+        cache[pages, 1, 0] = v[:, 0].reshape(n, page, hd).transpose(1, 2).reshape(n, page, hd)        # channels of a page's keys
+        cache, table = cache.cuda(), pages.int().reshape(1, -1).cuda()
+
+        def run(rows):
+            out = torch.empty(len(rows), nq * hd, dtype=dtype, device="cuda")
+            K.attention_simple(qd[rows].contiguous(), nq * hd, out, pos[rows].contiguous(), zeros[:len(rows)], slots, table, cache, len(rows),
+                               nq, nkv, hd, page, window, 1 / math.sqrt(hd))
+            return out
+        got += [run(torch.arange(T).repeat(20).cuda())[some], torch.cat([run(t[None].cuda()) for t in some])]
+    assert all(torch.equal(x, got[0]) for x in got[1:])
