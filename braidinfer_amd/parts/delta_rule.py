@@ -261,13 +261,13 @@ class LightningAttention(Mixer):
                 silu = False
             K.dr_rotate_rows(rows[:, :hd], rows[:, hd:2 * hd], tables.cos if tables else None, tables.sin if tables else None,
                              tables.rotary_dim if tables else 0, nh, d, 1.0, self.key_scale)
-        chunks, walk, rest = in_chunks(step, d, e)
-        pieces = 1 if chunks else pieces_for(step, nh * -(-e // 16), self.MIN_PIECE)
+        pieces = pieces_for(step, nh * -(-e // 16), self.MIN_PIECE)
+        chunks, walk, rest = in_chunks(step, d, e, pieces)
         if chunks:
             K.chunk_scan("fixed", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], o, ctx.state, step.cu_seqlens, step.slots,
                          B=step.n_seqs, H=nh, G=nh, d=d, e=e, max_new=step.max_new, b1=self.decay, silu=silu,
                          **chunk_scratch(step, nh, d, e))
-        if pieces > 1:
+        elif pieces > 1:
             # long prompts: the recurrence is linear in the state, so every sequence is cut into pieces that are walked
             # side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)
@@ -277,7 +277,7 @@ class LightningAttention(Mixer):
                 K.silu_rows(rows[:, :2 * hd + he])
             K.dr_scan_pieces(rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], self.decay, o, ctx.state, step.slots,
                              cu, numbers, piece_state, step.n_seqs, pieces, nh, d, e, silu=False)
-        elif walk:
+        if walk and (chunks or pieces == 1):
             K.dr_scan(rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:2 * hd + he], None, self.decay, o, ctx.state,
                       step.cu_seqlens, step.slots, step.n_seqs, nh, nh, d, e, silu=silu, **rest)
         y = step.ws.get("la_y", (T, he), self.rt.dtype)

@@ -53,12 +53,20 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
 CHUNKS_FROM = 96
 
 
-def in_chunks(step, d: int, e: int) -> Tuple[bool, bool, dict]:
+# A recurrence that can be walked in pieces goes so, and not in chunks, where its prompt can be cut into this many: a lone prompt
+# through few heads leaves most compute units idle behind a chain of chunks, which the pieces fill.  Chunks against pieces, us: 1 to 4 heads
+# of 128 x 128, 16 pieces: 2,048 tokens 135 / 80 to 110, 8,192 tokens 490 / 200 to 240, 30,000 tokens 1,750 / 570 to 670; 8 heads, 16
+# pieces: 140 / 130, 500 / 340, 1,720 / 1,090; 16 heads, 8 pieces: 145 / 180, 515 / 595, 1,820 / 2,100; heads of 64 x 64: 16 of them, 16
+# pieces: 100 / 75 to 88, 340 / 200 to 260; 32, 8 pieces: 104 / 110 to 136, 366 / 346 to 490; 600 tokens, 4 pieces: 38 to 58 / 50 to 82.
+PIECES_FROM = 12
+
+
+def in_chunks(step, d: int, e: int, pieces: int = 1) -> Tuple[bool, bool, dict]:
     """(whether sequences of the step go in chunks, whether others are walked token by token, how the walk is told apart):
     every sequence by its own number of tokens, so that what is beside it in the step does not change its bits, and the
     single tokens of running requests do not pay for whole chunks (a prompt of 96 tokens among 63 of them, 32 heads of 128 x 128: delta
     rule 90 us so, 230 all in chunks, 325 all token by token; beside 16 prompts of 60 tokens one of 1,500 takes 413, 397 and 614)."""
-    if step.is_decode or step.max_new < CHUNKS_FROM or not K.chunk_takes(d, e):
+    if step.is_decode or step.max_new < CHUNKS_FROM or not K.chunk_takes(d, e) or pieces >= PIECES_FROM:
         return False, True, {}
     rest = [n for n in step.host_new if n < CHUNKS_FROM]
     return True, bool(rest), {"below": CHUNKS_FROM, "singles": max(rest, default=0) <= 1}
@@ -148,21 +156,21 @@ class HGRN2(Mixer):
         rows = step.ws.get("glr_qfv", (T, 2 * nh * d + nh * e), torch.float32)
         linear(h, self.w_qfv, rows, step.ws)
         o = step.ws.get("glr_o", (T, nh * e), torch.float32)
-        chunks, walk, rest = in_chunks(step, d, e)
-        pieces = 1 if chunks else self.pieces_for(step)
+        pieces = self.pieces_for(step)
+        chunks, walk, rest = in_chunks(step, d, e, pieces)
         if chunks:
             hd = nh * d
             K.chunk_scan("glr", rows[:, :hd], rows[:, hd:2 * hd], rows[:, 2 * hd:], o, ctx.state, step.cu_seqlens, step.slots,
                          B=step.n_seqs, H=nh, G=nh, d=d, e=e, max_new=step.max_new, b1=self.f_bias, b2=self.lower,
                          **chunk_scratch(step, nh, d, e))
-        if pieces > 1:
+        elif pieces > 1:
             cu, numbers = self._piece_arrays(step, pieces)
             n = step.n_seqs * pieces
             piece_state = step.ws.get("glr_piece_state", (n,) + tuple(K.glr_state_shape(nh, d, e)), torch.float32)
             decay = step.ws.get("glr_decay", (n, nh, 16 * K.glr_rows_per_lane(d)), torch.float32)
             K.glr_scan_pieces(rows, self.f_bias, self.lower, o, ctx.state, step.slots, cu, numbers, piece_state, decay,
                               step.n_seqs, pieces, nh, d, e)
-        elif walk:
+        if walk and (chunks or pieces == 1):
             K.glr_scan(rows, self.f_bias, self.lower, o, ctx.state, step.cu_seqlens, step.slots, step.n_seqs, nh, d, e, **rest)
         on = step.ws.get("glr_on", (T, nh * e), self.rt.dtype)
         K.head_rmsnorm(o, self.norm_w, on, nh, e, self.eps)

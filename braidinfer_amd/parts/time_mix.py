@@ -102,14 +102,14 @@ class WKVTimeMix(Mixer):
         K.tanh(low, low_t)
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
-        chunks, walk, rest = in_chunks(step, self.d, self.d)
-        pieces = 1 if chunks else pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
+        pieces = pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
+        chunks, walk, rest = in_chunks(step, self.d, self.d, pieces)
         if chunks:
             r, k, v, z = (rows[:, i * hd:(i + 1) * hd] for i in range(4))
             K.chunk_scan("wkv", r, k, v, o, state, step.cu_seqlens, step.slots, B=step.n_seqs, H=self.nh, G=self.nh,
                          d=self.d, e=self.d, max_new=step.max_new, z=z, b1=self.w0, b2=self.u,
                          **chunk_scratch(step, self.nh, self.d, self.d))
-        if pieces > 1:
+        elif pieces > 1:
             # long prompts: every sequence cut into pieces that are walked side by side, twice
             cu, numbers = HGRN2._piece_arrays(step, pieces)
             n = step.n_seqs * pieces
@@ -117,7 +117,7 @@ class WKVTimeMix(Mixer):
             decay = step.ws.get("wkv_decay", (n, self.nh, 16 * K.glr_rows_per_lane(self.d)), torch.float32)
             K.wkv_scan_pieces(rows, self.w0, self.u, o, state, step.slots, cu, numbers, piece_state, decay, step.n_seqs, pieces,
                               self.nh, self.d, self.d)
-        elif walk:
+        if walk and (chunks or pieces == 1):
             K.wkv_scan(rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, step.n_seqs, self.nh, self.d, self.d,
                        below=rest.get("below", 0))
         y = step.ws.get("wkv_y", (T, hd), dt)

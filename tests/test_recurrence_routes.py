@@ -24,22 +24,22 @@ class Step:
         self.position_data = {}
 
 
-def mixer(kind, d):
+def mixer(kind, d, heads):
     if kind == "hgrn2":
-        part = gated_recurrence.HGRN2(64, 2, d, 32, 1e-5)
+        part = gated_recurrence.HGRN2(64, heads, d, 32, 1e-5)
     elif kind == "wkv":
-        part = time_mix.WKVTimeMix(64, 2, d, 8, 1e-5)
+        part = time_mix.WKVTimeMix(64, heads, d, 8, 1e-5)
         part.w = {s: None for s in ("r", "k", "v", "g", "w1", "w2")}
     elif kind == "delta":
-        part = delta_rule.GatedDeltaRule(64, 2, 2, d, 32, 4, 1e-5)
+        part = delta_rule.GatedDeltaRule(64, heads, heads, d, 32, 4, 1e-5)
         part.conv = part.conv_t = None
     else:
-        part = delta_rule.LightningAttention(64, 2, d, 32, [0.9, 0.8], 1e-5)
+        part = delta_rule.LightningAttention(64, heads, d, 32, [0.9] * heads, 1e-5)
     part.rt = type("Runtime", (), {"dtype": torch.float32})
     return part
 
 
-def walks(monkeypatch, kind, lens, d=64):
+def walks(monkeypatch, kind, lens, d=64, heads=64):
     """For every sequence the kernels that walk it, from the arguments of the launches."""
     by = [[] for _ in lens]
 
@@ -60,7 +60,7 @@ def walks(monkeypatch, kind, lens, d=64):
     monkeypatch.setattr(K, "glr_rows_per_lane", lambda d: 4 if d <= 64 else 8)
     for module in (delta_rule, gated_recurrence, time_mix):
         monkeypatch.setattr(module, "linear", lambda *a, **k: None)
-    part = mixer(kind, d)
+    part = mixer(kind, d, heads)
     need = part.state_need()
     state = torch.empty((len(lens),) + tuple(need.shape), device="meta")
     part.forward(torch.empty(sum(lens), 64, device="meta"), torch.empty(sum(lens), 64, device="meta"), Step(lens), MixerContext(state=state))
@@ -78,7 +78,17 @@ def test_every_sequence_by_its_own_tokens(monkeypatch, kind):
 @pytest.mark.parametrize("kind", ["hgrn2", "wkv", "delta", "lightning"])
 def test_heads_that_chunks_do_not_take(monkeypatch, kind):
     assert set(itertools.chain(*(walks(monkeypatch, kind, lens, d=48) for lens in ((1, 1), (200, 1), (400,))))) == {"walk"}
-    assert walks(monkeypatch, kind, (2000, 1), d=48) == ["walk" if kind == "delta" else "pieces"] * 2
+    assert walks(monkeypatch, kind, (2000, 1), d=48, heads=16) == ["walk" if kind == "delta" else "pieces"] * 2
+
+
+@pytest.mark.parametrize("kind", ["hgrn2", "wkv", "delta", "lightning"])
+def test_lone_prompts_through_few_heads(monkeypatch, kind):
+    # columns of 16 to a head: 2, WKV 4; 1,024 workgroups fill the chip, a piece has 128 tokens at least
+    per_head = 4 if kind == "wkv" else 2
+    for heads, tokens, pieces in ((2, 8192, 16), (1024 // per_head // 12, 8192, 12), (1024 // per_head // 11, 8192, 11), (2, 12 * 128, 12),
+                                  (2, 12 * 128 - 1, 11), (2, 600, 4), (1024 // per_head // 8, 8192, 8)):
+        got = walks(monkeypatch, kind, (tokens,), heads=heads)
+        assert got == ["pieces" if pieces >= 12 and kind != "delta" else "chunks"], (heads, tokens)
 
 
 @pytest.mark.parametrize("delta", [False, True])
