@@ -20,8 +20,10 @@
 #define MAX_DPL 8   // head_dim <= 64 * MAX_DPL
 
 // VEC: the rows of keys and the rows of a value channel are read 16 bytes at a time, in the same order of sums (head sizes in
-// steps of a 16-byte load, pages of whole 64s, aligned cache; where a chunk does not start with its page, as windows make
-// them, the values up to the first such piece one by one).  Bound by the latency of those reads.  Short requests (3 sequences of
+// steps of a 16-byte load, pages of whole 64s, aligned cache).  WIN: behind a window's edge chunks seldom start with a page; their
+// values are read one by one up to the first such piece and then so, page by page, in the same order (32 tokens through windows
+// of 100, 32 heads of 128 in bfloat16: 30 us; all of them one by one 88, by one wave 64).  A kernel of its own: in the other it takes
+// registers (contexts of 2,000 keys without a window, 8 heads of 64, 500 tokens: 520 us, 690 with it).  Bound by the latency of those reads.  Short requests (3 sequences of
 // 29 to 163 tokens, 32 heads of 128 in float): a step of single tokens takes 12.8 us with a wave a class, the prompt 94 with one
 // wave for all; both forms with one wave and no classes averaged 35 over a prompt and six steps, one element a read 106.
 template <typename T> struct as_vec;
@@ -44,7 +46,7 @@ __device__ __forceinline__ void as_join(AsPart& a, const AsPart& b) {
     a.m = m;
 }
 
-template <typename T, bool VEC, int WAVES>
+template <typename T, bool VEC, int WAVES, bool WIN>
 __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
     const T* __restrict__ q, size_t q_stride, T* __restrict__ out, const int* __restrict__ pos,
     const int* __restrict__ seq_of_token, const int* __restrict__ slots,
@@ -122,16 +124,33 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
                     if (d < hd) a.acc[i] = fmaf(pw, to_f32<T>(vc[(size_t)d * page]), a.acc[i]);
                 }
             };
-            for (int jj = 0; jj < nk;) {                 // page by page: a chunk lies in one, or in two behind a window's edge
-                const int off = (j0 + jj) % page, end = min(nk, jj + page - off);
-                const T* vc = cache + (size_t)bt[(j0 + jj) / page] * page_elems + v_off + off - jj;
-                if (!VEC) {
-                    for (; jj < end; ++jj) one(jj, vc + jj);
-                    continue;
-                }
-                for (; jj < end && (j0 + jj) % VN; ++jj) one(jj, vc + jj);
+            if constexpr (WIN && VEC) {
+                for (int jj = 0; jj < nk;) {
+                    const int off = (j0 + jj) % page, end = min(nk, jj + page - off);
+                    const T* vc = cache + (size_t)bt[(j0 + jj) / page] * page_elems + v_off + off - jj;
+                    for (; jj < end && (j0 + jj) % VN; ++jj) one(jj, vc + jj);
 #pragma unroll 4
-                for (; jj + VN <= end; jj += VN) {
+                    for (; jj + VN <= end; jj += VN) {
+                        vec_t vv[MAX_DPL];
+#pragma unroll
+                        for (int i = 0; i < MAX_DPL; ++i)
+                            if (64 * i < hd) vv[i] = *(const vec_t*)(vc + (size_t)min(lane + 64 * i, hd - 1) * page + jj);
+#pragma unroll
+                        for (int i = 0; i < MAX_DPL; ++i)
+                            if (64 * i < hd)
+#pragma unroll
+                                for (int e = 0; e < VN; ++e) a.acc[i] = fmaf(ps[jj + e], to_f32<T>(vv[i][e]), a.acc[i]);
+                    }
+                    for (; jj < end; ++jj) one(jj, vc + jj);
+                }
+                a.m = m_new;
+                continue;
+            }
+            int jj = 0;
+            if (VEC) {                                   // the chunk lies in one page
+                const T* vc = cache + (size_t)bt[j0 / page] * page_elems + v_off + (j0 % page);
+#pragma unroll 4
+                for (; jj + VN <= nk; jj += VN) {
                     vec_t vv[MAX_DPL];
 #pragma unroll
                     for (int i = 0; i < MAX_DPL; ++i)
@@ -142,7 +161,10 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
 #pragma unroll
                             for (int e = 0; e < VN; ++e) a.acc[i] = fmaf(ps[jj + e], to_f32<T>(vv[i][e]), a.acc[i]);
                 }
-                for (; jj < end; ++jj) one(jj, vc + jj);
+            }
+            for (; jj < nk; ++jj) {
+                const int jk = j0 + jj;
+                one(jj, cache + (size_t)bt[jk / page] * page_elems + v_off + (jk % page));
             }
             a.m = m_new;
         }
@@ -150,16 +172,18 @@ __global__ __launch_bounds__(64 * WAVES) void attn_simple_kernel(
     };
     AsPart a;
     if (WAVES == 1) {
-        a = nothing();
-        for (int cls = 0; cls < 4 && lo + 64 * cls <= p; ++cls) as_join(a, walk(cls));
+        // with windows the walk stands here once, in the loop: twice it takes registers that a third of the waves are missing
+        constexpr bool ONCE = WIN && VEC;
+        a = ONCE ? nothing() : walk(0);
+        for (int cls = ONCE ? 0 : 1; cls < 4 && lo + 64 * cls <= p; ++cls) as_join(a, walk(cls));
     } else {
         a = walk(wave);
-        float* mine = joinL + wave * (2 + hd);
+        float* part = joinL + wave * (2 + hd);
         if (wave > 0) {
-            if (lane == 0) { mine[0] = a.m; mine[1] = a.l; }
+            if (lane == 0) { part[0] = a.m; part[1] = a.l; }
 #pragma unroll
             for (int i = 0; i < MAX_DPL; ++i)
-                if (lane + 64 * i < hd) mine[2 + lane + 64 * i] = a.acc[i];
+                if (lane + 64 * i < hd) part[2 + lane + 64 * i] = a.acc[i];
         }
         __syncthreads();
         if (wave > 0) return;
@@ -193,10 +217,13 @@ extern "C" int br_attn_simple(const void* q, size_t q_stride, void* out, int is_
     const bool four = (long long)T * nq * 4 <= 16ll * br_device_cus();
     const size_t lds = (size_t)(((hd + 3) & ~3) + (four ? 4 * 64 + 4 * (2 + hd) : 64)) * sizeof(float);
     const bool vec = hd % (is_bf16 ? 8 : 4) == 0 && page % 64 == 0 && (uintptr_t)cache % 16 == 0;
-#define AS_LAUNCH(TT, V, W) \
-    attn_simple_kernel<TT, V, W><<<grid, 64 * W, lds, s>>>((const TT*)q, q_stride, (TT*)out, pos, seq_of_token, slots, block_table, \
+#define AS_LAUNCH(TT, V, W, N) \
+    attn_simple_kernel<TT, V, W, N><<<grid, 64 * W, lds, s>>>((const TT*)q, q_stride, (TT*)out, pos, seq_of_token, slots, block_table, \
                                                            table_stride, (const TT*)cache, nq, nkv, hd, page, window, scale)
-#define AS_FORM(TT, V) do { if (four) AS_LAUNCH(TT, V, 4); else AS_LAUNCH(TT, V, 1); } while (0)
+#define AS_FORM(TT, V) do { \
+        if (V && window > 0) { if (four) AS_LAUNCH(TT, V, 4, V); else AS_LAUNCH(TT, V, 1, V); } \
+        else { if (four) AS_LAUNCH(TT, V, 4, false); else AS_LAUNCH(TT, V, 1, false); } \
+    } while (0)
     if (is_bf16) { if (vec) AS_FORM(bf16, true); else AS_FORM(bf16, false); }
     else { if (vec) AS_FORM(float, true); else AS_FORM(float, false); }
 #undef AS_FORM
