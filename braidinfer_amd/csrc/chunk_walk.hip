@@ -242,17 +242,18 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const C
 // quarter of every output element (its rows' share and, of the sum over A, the tokens 4 w .. + 4), the quarters are added
 // in a fixed order through LDS a chunk later.  Sums are kept short and their largest terms late, so that they round about as
 // often as a walk token by token: the products with S in chains of 8 terms that are added in pairs, A's on top of them, the
-// state's update by itself in the order of the tokens and then onto the decayed state.  Error against 64 bits over 96 to 1,801 tokens with
-// gates from nearly 0 to nearly 1, as a share of the walk's: outputs 0.47 to 0.97, gated 0.86 to 1.08 (5.6e-8 of the norm against
-// 5.3e-8); states 0.39 to 1.18, gated to 1.45 where both are one rounding (4.4e-8 against 3.1e-8).  With one chain a sum, float
-// products of decays and the rounded decay alone the outputs were at 1.0 to 3.0, the states at up to 2.6, for 3 to 15 % less time.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
+// state's update in the order of the tokens.  Error against 64 bits over 96 to 1,801 tokens with gates from nearly 0 to nearly 1, as a
+// share of the walk's: outputs 0.47 to 0.97, gated 0.86 to 1.09 (5.6e-8 of the norm against 5.3e-8); states 0.39 to 1.06, gated to 1.27
+// where both are about one rounding (3.9e-8 against 3.1e-8).  With one chain a sum, float products of decays and the rounded decay
+// alone the outputs were at 1.0 to 3.0 and the states at up to 2.6, for a tenth to a fifth less of the walk's time.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
 // barrier a chunk.  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H, e / (16 CB)): the workgroups of a head
 // on one XCD where sequences * H is a multiple of 8.
-template <int D, int CB, int S, bool DELTA>
+template <int D, int CB, int S, int FORM>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
                                                          float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
                                                          int zero_padding, const CwPart run) {
+    constexpr bool DELTA = FORM == CW_DELTA, FIXED = FORM == CW_FIXED;
     constexpr int NKB = D / 64, RPL = D / 16, STAGE = ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4, L = (DELTA ? 3 : 2) * NKB + 1;
     constexpr int PB = DELTA ? 1 : 2;                         // buffers of output quarters
     const int BLOCK = cw_block(D, e, DELTA);
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         // the operands first: the matrix instructions start as soon as they are there, the rest runs beside them
-        f32x4 qf[NKB], kf[NKB], dec[NKB], rest[NKB];
+        f32x4 qf[NKB], kf[NKB], dec[NKB], rest[FIXED ? NKB : 1];
         float vv[CB][4], va[CB], vz[CB];
         const float a = sf[32 * D + r16 * 16 + 4 * wave + g];
 #pragma unroll
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
         for (int j = 0; j < NKB; ++j) {
             const int kb = wave * NKB + j;
             dec[j] = *(const f32x4*)(sf + 32 * D + 256 + 16 * kb + 4 * g);
-            rest[j] = *(const f32x4*)(sf + 33 * D + 256 + 16 * kb + 4 * g);
+            if constexpr (FIXED) rest[j] = *(const f32x4*)(sf + 33 * D + 256 + 16 * kb + 4 * g);
             kf[j] = *(const f32x4*)(sf + 16 * D + kb * 256 + lane * 4);
         }
         // factors of this wave's rows times the state, in chains of 8 rows
@@ -384,6 +385,21 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             if constexpr (NKB == 1) return p[0] + p[1];
             else return (p[0] + p[1]) + (p[2] + p[3]);
         };
+        // The decayed state, on which the chunk's writes are summed.  A decay that never changes (FIXED) rounds it once: what it and the
+        // decay's own rounding leave goes ahead of the chunk's writes, and their sum onto the state.
+        f32x4 kept[CB][NKB], add[CB][NKB];
+        auto decay = [&]() {
+#pragma unroll
+            for (int j = 0; j < NKB; ++j)
+#pragma unroll
+                for (int x = 0; x < CB; ++x)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float old = st[x][j][r], k = old * dec[j][r];
+                        kept[x][j][r] = k;
+                        add[x][j][r] = FIXED ? fmaf(old, rest[FIXED ? j : 0][r], fmaf(old, dec[j][r], -k)) : k;
+                    }
+        };
         f32x4 ro[CB][2 * NKB];
         if constexpr (DELTA) {
             f32x4 uf[CB], wf[NKB], pa[CB][2 * NKB];
@@ -393,6 +409,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             for (int x = 0; x < CB; ++x) uf[x] = *(const f32x4*)(sf + 32 * D + 512 + x * 256 + lane * 4);
             times_state(wf, pa);
             times_state(qf, ro);
+            decay();
 #pragma unroll
             for (int x = 0; x < CB; ++x) *(f32x4*)(pu + ((wave * CB + x) * 64 + lane) * 4) = pairs(pa[x]);
             if (ch > 0) flush(ch - 1);
@@ -426,33 +443,29 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             odd |= __ballot(!fine);
             vz[x] = fine ? va[x] : 0.f;
         }
-        if constexpr (!DELTA) times_state(qf, ro);
+        if constexpr (!DELTA) {
+            times_state(qf, ro);
+            decay();
+        }
         issue();
 #pragma unroll
-        for (int j = 0; j < NKB; ++j) {
-            // the decayed state, rounded once, and what the chunk adds to it, summed on top of that rounding's error
-            f32x4 add[CB];
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int x = 0; x < CB; ++x)
+            for (int j = 0; j < NKB; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float old = st[x][j][r], kept = old * dec[j][r];
-                    add[x][r] = fmaf(old, rest[j][r], fmaf(old, dec[j][r], -kept));
-                    st[x][j][r] = kept;
-                }
+                for (int x = 0; x < CB; ++x) add[x][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], add[x][j], 0, 0, 0);
+        f32x4 outs[CB];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int x = 0; x < CB; ++x) outs[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vz[x], pairs(ro[x]), 0, 0, 0);
 #pragma unroll
-                for (int x = 0; x < CB; ++x) add[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], add[x], 0, 0, 0);
+        for (int j = 0; j < NKB; ++j)
 #pragma unroll
-            for (int x = 0; x < CB; ++x) st[x][j] += add[x];
-        }
+            for (int x = 0; x < CB; ++x) st[x][j] = FIXED ? kept[x][j] + add[x][j] : add[x][j];
 #pragma unroll
         for (int x = 0; x < CB; ++x) {
             float* pw = part + (((ch & (PB - 1)) * 4 + wave) * CB + x) * 272;
-            const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vz[x], pairs(ro[x]), 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = sum[r];
+            for (int r = 0; r < 4; ++r) pw[(4 * g + r) * 17 + r16] = outs[x][r];
         }
         if (odd) {                                            // infinite or not a number: this wave's tokens 4 wave + i of A
             for (int x = 0; x < CB; ++x) {
@@ -491,12 +504,13 @@ extern "C" size_t br_chunk_scratch(int T, int B, int H, int d, int e, int delta)
     return (size_t)(T / CW_C + B + 1) * br_chunk_block(H, d, e, delta);
 }
 
-template <int D, int CB, int S, bool DELTA>
+template <int D, int CB, int S, int FORM>
 static int chunk_walk(const CwIn& in, const CwPart& part, const float* scratch, float* o, float* state, size_t slot_stride, int B,
                       int zero_padding, hipStream_t s) {
+    constexpr bool DELTA = FORM == CW_DELTA;
     constexpr size_t lds = (size_t)S * ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4 + (DELTA ? 1 : 2) * 4 * CB * 272 * 4 + (DELTA ? 4096 * CB : 0);
     static_assert(lds <= 160 * 1024, "LDS");
-    auto walk = chunk_walk_kernel<D, CB, S, DELTA>;
+    auto walk = chunk_walk_kernel<D, CB, S, FORM>;
     static bool set = false;
     if (!set) {
         if (hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
@@ -520,7 +534,7 @@ static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state,
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
     const long long units = (long long)B * in.H * (in.e / 16);
-#define CW_WALK(CB, S) return chunk_walk<D, CB, S, DELTA>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
+#define CW_WALK(CB, S) return chunk_walk<D, CB, S, FORM == CW_WKV ? CW_GLR : FORM>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
     if (in.e % 32 || units <= (D == 64 ? 2 : 1) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
     if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
     else {
