@@ -20,11 +20,11 @@
 // sequence's first token of the step; a chunk's tokens beyond the sequence have decay 1, write nothing and read nothing.
 //
 // What bounds it: the walk is a serial chain, a chunk of a head of 128 x 128 costing a wave 17 float matrix instructions (32
-// cycles each) and about as much again in operand reads, the exchange of the quarters and the barrier (0.74 us a chunk with a
+// cycles each) and about as much again in operand reads, the exchange of the quarters and the barrier (0.9 us a chunk with a
 // workgroup to a compute unit; a deeper ring changes nothing).  A walk token by token is bound by the 49,000 lane operations a
-// token of such a head takes.  32 heads of 128 x 128: 2,048 tokens 125 us (30 of them `chunk_prepare`, which is bound by its
-// reads and writes), 8,192 tokens 574; token by token, twice in pieces, 326 and 1,236.  64 heads of 64 x 64: 107 and 404,
-// token by token 252 and 1,052.
+// token of such a head takes.  32 heads of 128 x 128: 2,048 tokens 141 us (30 of them `chunk_prepare`, which is bound by its
+// reads and writes), 8,192 tokens 546; token by token, twice in pieces, 307 and 1,153.  64 heads of 64 x 64: 113 and 426,
+// token by token 235 and 938.
 #include "common.h"
 
 #define CW_C 16            // tokens of a chunk
@@ -527,20 +527,18 @@ static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state,
     chunk_prepare_kernel<FORM, D><<<dim3(chunks, in.H, B), D, 0, s>>>(in, part, scratch);
     const int rc = br_check_launch();
     if (rc != BR_OK) return rc;
-    // 16 columns a workgroup where that gives no more workgroups than compute units (two to each for heads of 64); beyond, 32
-    // columns, which share a chunk's loads: with a ring of twice the depth while a compute unit has one such workgroup (32 heads
-    // of 128 x 128, 3,517 and 1,501 tokens: 305 -> 278 us), else two of them to a unit (16 sequences of 300 tokens: 302 -> 225;
-    // 64 heads of 64 x 64: 231 -> 191).
+    // 16 columns a workgroup up to three workgroups to a compute unit (delta rule with heads of 128: one, it holds the most in
+    // LDS); beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of 128 x 128, gated, 2,048 tokens 142 / 193, 3,517 and
+    // 1,501 tokens 315 / 340, three times 1,000 167 / 165, 16 times 300 307 / 236; fixed, 1,307, 804 and 301 tokens 162 / 181; delta rule,
+    // 2,048 tokens 213 / 320, twice 1,000 211 / 197, 16 times 300 556 / 410; 64 heads of 64 x 64, WKV, 1,801 tokens 100 / 138, three times 900
+    // 123 / 122, 16 times 300 233 / 198; delta rule, 900, 900 and 300 tokens 156 / 166.
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    const long long units = (long long)B * in.H * (in.e / 16);
+    const long long units = (long long)part.longs * in.H * (in.e / 16);
 #define CW_WALK(CB, S) return chunk_walk<D, CB, S, FORM == CW_WKV ? CW_GLR : FORM>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
-    if (in.e % 32 || units <= (D == 64 ? 2 : 1) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
+    if (in.e % 32 || units <= (D == 128 && DELTA ? 1 : 3) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
     if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
-    else {
-        if (D == 128 && units <= 2 * cus) CW_WALK(2, (D == 64 ? 5 : 6));
-        CW_WALK(2, (D == 64 ? 5 : 3));
-    }
+    else CW_WALK(2, (D == 64 ? 5 : 3));
 #undef CW_WALK
 }
 
@@ -561,13 +559,14 @@ extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v,
         return BR_BAD_ARG;
     const CwIn in = {q, k, z, b1, b2, gb, gc, v, qk_stride, v_stride, cu_seqlens, slots, H, G, e, silu};
     const int all = (max_new + CW_C - 1) / CW_C;
+    const bool once = scratch_floats >= br_chunk_scratch(T, B, H, d, e, form == CW_DELTA);
     int run = all;
-    if (scratch_floats < br_chunk_scratch(T, B, H, d, e, form == CW_DELTA)) {
+    if (!once) {
         const size_t room = scratch_floats / br_chunk_block(H, d, e, form == CW_DELTA) / longs;
         run = room < (size_t)all ? (int)room : all;
-    } else longs = 0;
+    }
     for (int from = 0; from < all; from += run) {
-        const CwPart part = {least, longs, from, longs ? run : 0};
+        const CwPart part = {least, longs, from, once ? 0 : run};
         const int chunks = all - from < run ? all - from : run;
 #define CW_RUN(F) d == 64 ? chunk_run<F, 64>(in, part, o, state, slot_stride, scratch, B, chunks, s) : chunk_run<F, 128>(in, part, o, state, slot_stride, scratch, B, chunks, s)
         const int rc = form == CW_GLR ? CW_RUN(CW_GLR) : form == CW_WKV ? CW_RUN(CW_WKV) : form == CW_FIXED ? CW_RUN(CW_FIXED) : CW_RUN(CW_DELTA);

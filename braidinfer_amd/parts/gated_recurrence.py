@@ -46,10 +46,11 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
 
 
 # From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores (HGRN2, 32 heads of 128 x 128,
-# us against the walk token by token, in pieces where that is faster: 64 tokens 20 / 17, 128 tokens 22 / 30, 512 tokens 44 / 101,
-# 2,048 tokens 125 / 326, 3,517 and 1,501 tokens 278 / 711; WKV, 64 heads of 64 x 64: 17 / 17, 20 / 30, 37 / 75, 107 / 252, 242 / 744;
-# delta rule, 32 heads of 128 x 128: 96 tokens 31 / 30, 128 tokens 34 / 38, 2,048 tokens 185 / 521, 1,307, 804 and 301 tokens 247 / 384;
-# a fixed decay a head: 26 / 34, 29 / 43, 150 / 603, 175 / 446).
+# us against the walk token by token, in pieces where it can be: 64 tokens 18 / 17, 96 tokens 21 / 24, 128 tokens 22 / 30, 512 tokens 48 / 102,
+# 2,048 tokens 141 / 307, 3,517 and 1,501 tokens 313 / 948; WKV, 64 heads of 64 x 64: 64 tokens 16 / 17, 96 tokens 18 / 23, 512 tokens 40 /
+# 76, 2,048 tokens 113 / 235; delta rule, 32 heads of 128 x 128: 64 tokens 27 / 21, 96 tokens 30 / 29, 128 tokens 33 / 38, 2,048 tokens 214 /
+# 517, 1,307, 804 and 301 tokens 286 / 382; a fixed decay a head: 64 tokens 18 / 15, 96 tokens 20 / 21, 2,048 tokens 148 / 299, 1,307, 804 and
+# 301 tokens 161 / 295).
 CHUNKS_FROM = 96
 
 
@@ -74,7 +75,7 @@ def in_chunks(step, d: int, e: int, pieces: int = 1) -> Tuple[bool, bool, dict]:
 
 # Bytes of scratch for the chunks' factors, which are 36 KB a token for 32 heads of 128 x 128 (delta rule 68 KB) and stay with the
 # engine: longer steps are taken in runs of chunks, each of which reads and writes the states once (one of 16,384 tokens:
-# HGRN2 1,143 us, all at once 1,128; delta rule 1,612 and 1,561).
+# HGRN2 1,074 us, all at once 1,076; delta rule 1,607 and 1,557).
 CHUNK_SCRATCH = 512 << 20
 
 
