@@ -610,7 +610,7 @@ extern "C" int br_add_position_rows(float* x, const void* table, int is_bf16, co
 // out[i, :] = x[rows[i], :] (float)   reference: D2dCopy of the last row,
 // megakernel/megakernel_compile.rs:522-527.
 // grid (R, pieces of 256 VEC elements): rows are logits of a single-token step (1 x 32,768 floats: one workgroup a row
-// took 61 us, bound by one compute unit's loads; spread out about 6) or hidden rows.  VEC 4: H in steps of 4, aligned rows.
+// took 61 us, bound by one compute unit's loads; spread out 4.1, as 64 rows do) or hidden rows.  VEC 4: H in steps of 4, aligned rows.
 template <int VEC>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                                           float* __restrict__ out, int H) {

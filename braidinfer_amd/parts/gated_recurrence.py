@@ -64,8 +64,8 @@ PIECES_FROM = 12
 
 def in_chunks(step, d: int, e: int, pieces: int = 1) -> Tuple[bool, bool, dict]:
     """(whether sequences of the step go in chunks, whether others are walked token by token, how the walk is told apart):
-    every sequence by its own number of tokens, so that what is beside it in the step does not change its bits, and the
-    single tokens of running requests do not pay for whole chunks (a prompt of 96 tokens among 63 of them, 32 heads of 128 x 128: delta
+    every sequence by its own number of tokens, so that what is beside it in the step does not change its bits (but for steps in
+    pieces, of which the whole step decides), and the single tokens of running requests do not pay for whole chunks (a prompt of 96 tokens among 63 of them, 32 heads of 128 x 128: delta
     rule 90 us so, 230 all in chunks, 325 all token by token; beside 16 prompts of 60 tokens one of 1,500 takes 413, 397 and 614)."""
     if step.is_decode or step.max_new < CHUNKS_FROM or not K.chunk_takes(d, e) or pieces >= PIECES_FROM:
         return False, True, {}
