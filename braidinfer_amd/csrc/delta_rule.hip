@@ -700,7 +700,8 @@ __global__ __launch_bounds__(256) void dr_scan_kernel(const DrScan p) {
 //     64          64 / 58        62 / 57        87 / 59        86 / 58          (268 MB: 4.7 TB/s)
 // V4: k, q and the decays 16 bytes at a time.  Rows that do not lie so keep the chunks' walk, since element by element every column's
 // lanes pay for as many reads as rows (heads of 126, 64 sequences: 126 against 45 us, with channels' decays 179 against 60), unless
-// silu has the four columns share them (50 against 67).
+// silu has the four columns share them (50 against 67).  The same for heads of more than 256 channels, 32 rows of everything a lane
+// (8 heads of 512 x 64, 64 sequences: 28 against 25 us, channels' decays 37 against 32, with silu 26 either way).
 template <int RPL, int MODE, bool SILU, bool V4>
 __global__ __launch_bounds__(256) void dr_token_kernel(const DrScan p) {
     constexpr bool DELTA = MODE == DR_DELTA || MODE == DR_CHANNELS, CHAN = MODE == DR_CHANNELS;
@@ -825,7 +826,7 @@ static int dr_scan_launch(const DrScan& a, int B, int mode, int silu, int single
     dim3 grid(B, a.H, (cols + 15) / 16);
     const bool v4 = a.d % 4 == 0 && a.qk_stride % 4 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.gc) % 16) == 0;
 #define DR_GO(R, TC, M, A) do { \
-        if constexpr (!LOCAL) if (singles && (v4 || A)) { \
+        if constexpr (!LOCAL && (A || R <= 16)) if (singles && (v4 || A)) { \
             if (v4) dr_token_kernel<R, M, A, true><<<grid, 256, 0, s>>>(a); else dr_token_kernel<R, M, A, !A><<<grid, 256, 0, s>>>(a); \
             break; \
         } \

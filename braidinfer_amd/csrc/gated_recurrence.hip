@@ -209,7 +209,8 @@ __global__ __launch_bounds__(64) void glr_carry_kernel(float* __restrict__ state
 // the state, read and written once.  32 heads of 128 x 128 with bias and bounds, the chunks' walk before / this: 40 sequences
 // 47 / 30 us, 64 (268 MB) 72 / 46 (5.8 TB/s); up to 8 both take the launch.  Element by element, as rows that do not lie at
 // multiples of 16 bytes would have it, the many small reads cost more than the chunks do (heads of 126, 64 sequences: 231
-// against 75), so those keep the chunks' walk.
+// against 75), so those keep the chunks' walk; so do heads of more than 256 channels, of which a lane would hold 32 rows of everything
+// (8 heads of 512, 64 sequences: 79 against 64).
 template <int RPL>
 __global__ __launch_bounds__(256) void glr_token_kernel(
     const float* __restrict__ rows, const float* __restrict__ f_bias, const float* __restrict__ lower,
@@ -282,7 +283,7 @@ static int glr_scan_launch(const float* rows, const float* f_bias, const float* 
     // 16-byte loads where every row piece starts at a multiple of 16 bytes
     const bool v4 = d % 4 == 0 && width % 4 == 0 && ((uintptr_t)rows % 16) == 0;
 #define GLR_SCAN(R, TC) do { \
-        if (!LOCAL && singles && v4 && (((uintptr_t)f_bias | (uintptr_t)lower) % 16) == 0) { \
+        if constexpr (!LOCAL && R <= 16) if (singles && v4 && (((uintptr_t)f_bias | (uintptr_t)lower) % 16) == 0) { \
             glr_token_kernel<R><<<grid, 256, 0, s>>>(rows, f_bias, lower, o, state, cu_seqlens, slots, H, d, e, width, slot_stride, below); \
             break; \
         } \
