@@ -20,10 +20,10 @@
 // sequence's first token of the step; a chunk's tokens beyond the sequence have decay 1, write nothing and read nothing.
 //
 // What bounds it: the walk is a serial chain, a chunk of a head of 128 x 128 costing a wave 17 float matrix instructions (32
-// cycles each) and about as much again in operand reads, the exchange of the quarters and the barrier (0.9 us a chunk with a
+// cycles each) and twice as much again in operand reads, the exchange of the quarters and the barrier (0.7 us a chunk with a
 // workgroup to a compute unit; a deeper ring changes nothing).  A walk token by token is bound by the 49,000 lane operations a
-// token of such a head takes.  32 heads of 128 x 128: 2,048 tokens 141 us (30 of them `chunk_prepare`, which is bound by its
-// reads and writes), 8,192 tokens 546; token by token, twice in pieces, 307 and 1,153.  64 heads of 64 x 64: 113 and 426,
+// token of such a head takes.  32 heads of 128 x 128: 2,048 tokens 123 us (30 of them `chunk_prepare`, which is bound by its
+// reads and writes), 8,192 tokens 465; token by token, twice in pieces, 307 and 1,153.  64 heads of 64 x 64: 106 and 411,
 // token by token 235 and 938.
 #include "common.h"
 
@@ -245,14 +245,17 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const C
 // state's update in the order of the tokens.  Error against 64 bits over 96 to 1,801 tokens with gates from nearly 0 to nearly 1, as a
 // share of the walk's: outputs 0.47 to 0.97, gated 0.86 to 1.09 (5.6e-8 of the norm against 5.3e-8); states 0.39 to 1.06, gated to 1.27
 // where both are about one rounding (3.9e-8 against 3.1e-8).  With one chain a sum, float products of decays and the rounded decay
-// alone the outputs were at 1.0 to 3.0 and the states at up to 2.6, for a tenth to a fifth less of the walk's time.  S chunks of everything a chunk needs lie in an LDS ring filled by direct loads; one
-// barrier a chunk.  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H, e / (16 CB)): the workgroups of a head
-// on one XCD where sequences * H is a multiple of 8.
+// alone the outputs were at 1.0 to 3.0 and the states at up to 2.6.  S chunks of everything a chunk needs lie in an LDS ring filled
+// by direct loads; one barrier a chunk.  Registers for two workgroups to a compute unit, all of them ordinary ones: with room for twice
+// as many the compiler keeps the sums in accumulation registers and moves the state back and forth.  That, with the chunk before left
+// and A's product formed behind the update, took 142 us for 2,048 tokens of 32 heads where this takes 123 (a fixed decay 148 and 125,
+// delta rule 213 and 190; 64 heads of 64 x 64 113 and 106).  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H,
+// e / (16 CB)): the workgroups of a head on one XCD where sequences * H is a multiple of 8.
 template <int D, int CB, int S, int FORM>
-__global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
-                                                         float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
-                                                         const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
-                                                         int zero_padding, const CwPart run) {
+__global__ __launch_bounds__(256, 2) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
+                                                            float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
+                                                            const int* __restrict__ cu_seqlens, const int* __restrict__ slots, int H, int e,
+                                                            int zero_padding, const CwPart run) {
     constexpr bool DELTA = FORM == CW_DELTA, FIXED = FORM == CW_FIXED;
     constexpr int NKB = D / 64, RPL = D / 16, STAGE = ((DELTA ? 48 : 32) * D + 512 + 256 * CB) * 4, L = (DELTA ? 3 : 2) * NKB + 1;
     constexpr int PB = DELTA ? 1 : 2;                         // buffers of output quarters
@@ -340,11 +343,17 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
     for (int j = 0; j < S - 1; ++j) issue();
     const int ot = tid >> 4;
     float* op = o + (size_t)(t0 + ot) * he + h * e + cb * CB * 16 + (tid & 15);       // this thread's element of the chunk before
-    auto flush = [&](int ch) {                                // the quarters of chunk ch's outputs, chunks in order
+    float quarter[CB][4];                                     // of chunk ch's output elements, chunks in order
+    auto collect = [&](int ch) {
+#pragma unroll
+        for (int x = 0; x < CB; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) quarter[x][y] = part[((ch & (PB - 1)) * 4 * CB + y * CB + x) * 272 + ot * 17 + (tid & 15)];
+    };
+    auto leave = [&](int ch) {
 #pragma unroll
         for (int x = 0; x < CB; ++x) {
-            const float* pp = part + ((ch & (PB - 1)) * 4 * CB + x) * 272 + ot * 17 + (tid & 15);
-            const double v = ((double)pp[0] + pp[CB * 272]) + ((double)pp[2 * CB * 272] + pp[3 * CB * 272]);
+            const double v = ((double)quarter[x][0] + quarter[x][1]) + ((double)quarter[x][2] + quarter[x][3]);
             if (t0 + ch * CW_C + ot < t1) op[x * 16] = (float)v;
         }
         op += (size_t)CW_C * he;
@@ -412,7 +421,10 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             decay();
 #pragma unroll
             for (int x = 0; x < CB; ++x) *(f32x4*)(pu + ((wave * CB + x) * 64 + lane) * 4) = pairs(pa[x]);
-            if (ch > 0) flush(ch - 1);
+            if (ch > 0) {
+                collect(ch - 1);
+                leave(ch - 1);
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -443,20 +455,30 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
             odd |= __ballot(!fine);
             vz[x] = fine ? va[x] : 0.f;
         }
+        // Everything that is not on the chain from one chunk's state to the next stands between matrix instructions: the chunk before
+        // leaves while the products with S run, A's product half way through the update, so that its results are there at the end
         if constexpr (!DELTA) {
+            if (ch > 0) collect(ch - 1);
             times_state(qf, ro);
             decay();
+            if (ch > 0) leave(ch - 1);
         }
         issue();
+        auto update = [&](int i0, int i1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = i0; i < i1; ++i)
 #pragma unroll
-            for (int j = 0; j < NKB; ++j)
+                for (int j = 0; j < NKB; ++j)
 #pragma unroll
-                for (int x = 0; x < CB; ++x) add[x][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], add[x][j], 0, 0, 0);
+                    for (int x = 0; x < CB; ++x) add[x][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], vv[x][i], add[x][j], 0, 0, 0);
+        };
         f32x4 outs[CB];
+        update(0, 2);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int x = 0; x < CB; ++x) outs[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vz[x], pairs(ro[x]), 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        update(2, 4);
 #pragma unroll
         for (int j = 0; j < NKB; ++j)
 #pragma unroll
@@ -477,14 +499,14 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
                 }
             }
         }
-        if (!DELTA && ch > 0) flush(ch - 1);
         cur = cur == S - 1 ? 0 : cur + 1;
         sf = (const float*)(smem + cur * STAGE);
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");          // no load into LDS outlives the workgroup
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    flush(nch - 1);
+    collect(nch - 1);
+    leave(nch - 1);
 #pragma unroll
     for (int x = 0; x < CB; ++x)
 #pragma unroll
@@ -528,10 +550,10 @@ static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state,
     const int rc = br_check_launch();
     if (rc != BR_OK) return rc;
     // 16 columns a workgroup up to three workgroups to a compute unit (delta rule with heads of 128: one, it holds the most in
-    // LDS); beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of 128 x 128, gated, 2,048 tokens 142 / 193, 3,517 and
-    // 1,501 tokens 315 / 340, three times 1,000 167 / 165, 16 times 300 307 / 236; fixed, 1,307, 804 and 301 tokens 162 / 181; delta rule,
-    // 2,048 tokens 213 / 320, twice 1,000 211 / 197, 16 times 300 556 / 410; 64 heads of 64 x 64, WKV, 1,801 tokens 100 / 138, three times 900
-    // 123 / 122, 16 times 300 233 / 198; delta rule, 900, 900 and 300 tokens 156 / 166.
+    // LDS); beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of 128 x 128, gated, 2,048 tokens 122 / 166, 3,517 and
+    // 1,501 tokens 302 / 292, three times 1,000 156 / 154, four times 900 187 / 154, 16 times 300 303 / 227; fixed, 1,307, 804 and 301 tokens
+    // 162 / 164; delta rule, 2,048 tokens 190 / 282, twice 1,000 189 / 179, 16 times 300 518 / 392; 64 heads of 64 x 64, WKV, 1,801 tokens
+    // 94 / 119, three times 900 121 / 117, four times 171 / 136; delta rule, 900, 900 and 300 tokens 154 / 158.
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
     const long long units = (long long)part.longs * in.H * (in.e / 16);

@@ -46,27 +46,28 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
 
 
 # From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores (HGRN2, 32 heads of 128 x 128,
-# us against the walk token by token, in pieces where it can be: 64 tokens 18 / 17, 96 tokens 21 / 24, 128 tokens 22 / 30, 512 tokens 48 / 102,
-# 2,048 tokens 141 / 307, 3,517 and 1,501 tokens 313 / 948; WKV, 64 heads of 64 x 64: 64 tokens 16 / 17, 96 tokens 18 / 23, 512 tokens 40 /
-# 76, 2,048 tokens 113 / 235; delta rule, 32 heads of 128 x 128: 64 tokens 27 / 21, 96 tokens 30 / 29, 128 tokens 33 / 38, 2,048 tokens 214 /
-# 517, 1,307, 804 and 301 tokens 286 / 382; a fixed decay a head: 64 tokens 18 / 15, 96 tokens 20 / 21, 2,048 tokens 148 / 299, 1,307, 804 and
-# 301 tokens 161 / 295).
+# us against the walk token by token, in pieces where it can be: 64 tokens 18 / 17, 96 tokens 21 / 24, 128 tokens 22 / 30, 512 tokens 44 / 102,
+# 2,048 tokens 123 / 307, 3,517 and 1,501 tokens 302 / 948; WKV, 64 heads of 64 x 64: 64 tokens 16 / 17, 96 tokens 18 / 23, 512 tokens 38 /
+# 76, 2,048 tokens 106 / 235; delta rule, 32 heads of 128 x 128: 64 tokens 27 / 21, 96 tokens 30 / 29, 128 tokens 33 / 38, 2,048 tokens 190 /
+# 517, 1,307, 804 and 301 tokens 260 / 382; a fixed decay a head: 64 tokens 18 / 15, 96 tokens 20 / 21, 2,048 tokens 125 / 299, 1,307, 804 and
+# 301 tokens 162 / 295).
 CHUNKS_FROM = 96
 
 
 # A recurrence that can be walked in pieces goes so, and not in chunks, where its prompt can be cut into this many: a lone prompt
 # through few heads leaves most compute units idle behind a chain of chunks, which the pieces fill.  Chunks against pieces, us: 1 to 4 heads
-# of 128 x 128, 16 pieces: 2,048 tokens 135 / 80 to 110, 8,192 tokens 490 / 200 to 240, 30,000 tokens 1,750 / 570 to 670; 8 heads, 16
-# pieces: 140 / 130, 500 / 340, 1,720 / 1,090; 16 heads, 8 pieces: 145 / 180, 515 / 595, 1,820 / 2,100; heads of 64 x 64: 16 of them, 16
-# pieces: 100 / 75 to 88, 340 / 200 to 260; 32, 8 pieces: 104 / 110 to 136, 366 / 346 to 490; 600 tokens, 4 pieces: 38 to 58 / 50 to 82.
+# of 128 x 128, 16 pieces: 2,048 tokens 100 / 80 to 110, 8,192 tokens 358 / 200 to 240, 30,000 tokens 1,254 / 570 to 670; 8 heads, 16
+# pieces: 106 / 130, 368 / 340, 1,333 / 1,090; 16 heads, 8 pieces: 108 / 180, 404 / 595, 1,442 / 2,100; heads of 64 x 64: 16 of them, 16
+# pieces: 86 / 75 to 88, 296 / 200 to 260; 32, 8 pieces: 89 / 110 to 136, 331 / 346 to 490; 600 tokens, 4 pieces: 39 to 44 / 50 to 82.
 PIECES_FROM = 12
 
 
 def in_chunks(step, d: int, e: int, pieces: int = 1) -> Tuple[bool, bool, dict]:
     """(whether sequences of the step go in chunks, whether others are walked token by token, how the walk is told apart):
     every sequence by its own number of tokens, so that what is beside it in the step does not change its bits (but for steps in
-    pieces, of which the whole step decides), and the single tokens of running requests do not pay for whole chunks (a prompt of 96 tokens among 63 of them, 32 heads of 128 x 128: delta
-    rule 90 us so, 230 all in chunks, 325 all token by token; beside 16 prompts of 60 tokens one of 1,500 takes 413, 397 and 614)."""
+    pieces, of which the whole step decides), and the single tokens of running requests do not pay for whole chunks (a prompt of 96
+    tokens among 63 of them, 32 heads of 128 x 128: delta rule 87 us so, 227 all in chunks, 323 all token by token; 16 prompts of 60
+    tokens beside one of 1,500: 269, 358 and 608, a fixed decay 223, 212 and 502)."""
     if step.is_decode or step.max_new < CHUNKS_FROM or not K.chunk_takes(d, e) or pieces >= PIECES_FROM:
         return False, True, {}
     rest = [n for n in step.host_new if n < CHUNKS_FROM]
@@ -75,7 +76,7 @@ def in_chunks(step, d: int, e: int, pieces: int = 1) -> Tuple[bool, bool, dict]:
 
 # Bytes of scratch for the chunks' factors, which are 36 KB a token for 32 heads of 128 x 128 (delta rule 68 KB) and stay with the
 # engine: longer steps are taken in runs of chunks, each of which reads and writes the states once (one of 16,384 tokens:
-# HGRN2 1,074 us, all at once 1,076; delta rule 1,607 and 1,557).
+# HGRN2 921 us, all at once 907; delta rule 1,420 and 1,380).
 CHUNK_SCRATCH = 512 << 20
 
 
