@@ -45,12 +45,14 @@ def pieces_for(step, units_per_sequence: int, min_piece: int) -> int:
     return max(1, min(want, step.max_new // min_piece, 16, 65535 // max(1, step.n_seqs)))
 
 
-# From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores (HGRN2, 32 heads of 128 x 128,
-# us against the walk token by token, in pieces where it can be: 64 tokens 18 / 17, 96 tokens 21 / 24, 128 tokens 22 / 30, 512 tokens 44 / 102,
-# 2,048 tokens 123 / 307, 3,517 and 1,501 tokens 302 / 948; WKV, 64 heads of 64 x 64: 64 tokens 16 / 17, 96 tokens 18 / 23, 512 tokens 38 /
-# 76, 2,048 tokens 106 / 235; delta rule, 32 heads of 128 x 128: 64 tokens 27 / 21, 96 tokens 30 / 29, 128 tokens 33 / 38, 2,048 tokens 190 /
-# 517, 1,307, 804 and 301 tokens 260 / 382; a fixed decay a head: 64 tokens 18 / 15, 96 tokens 20 / 21, 2,048 tokens 125 / 299, 1,307, 804 and
-# 301 tokens 162 / 295).
+# From this many tokens of a sequence a prompt is walked 16 tokens at a time on the matrix cores.  us against the walk token by token, in
+# pieces where it can be: HGRN2, 32 heads of 128 x 128: 48 tokens 16 / 13, 64 tokens 17 / 16, 96 tokens 19 / 23, 128 tokens 21 / 28, 512
+# tokens 44 / 102, 2,048 tokens 123 / 307, 3,517 and 1,501 tokens 302 / 948; WKV, 64 heads of 64 x 64: 64 tokens 16 / 17, 96 tokens 18 / 23,
+# 512 tokens 38 / 76, 2,048 tokens 106 / 235; a fixed decay a head: 64 tokens 17 / 15, 96 tokens 19 / 21, 2,048 tokens 125 / 299, 1,307, 804
+# and 301 tokens 162 / 295; delta rule: 64 tokens 26 / 20, 96 tokens 29 / 28, 128 tokens 32 / 36, 2,048 tokens 190 / 517, 1,307, 804 and 301
+# tokens 260 / 382.  One line for all, where the delta rule's lies.  A short prompt beside longer ones would be nearly free in their chunks
+# and is walked behind them (200, 153, 107 and 60 tokens: HGRN2 73 us, 50 all in chunks), the price of bits that do not depend on what is
+# beside it; the line is not lowered for that, as gated outputs of 48 tokens round up to 1.16 times as far off in chunks as in the walk.
 CHUNKS_FROM = 96
 
 
