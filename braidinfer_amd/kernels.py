@@ -1398,15 +1398,18 @@ def experts_up(h: torch.Tensor, w_gu: torch.Tensor, chosen: torch.Tensor, y: tor
              float(alpha), _stream()), "experts_up")
 
 
-def experts_sort(chosen: torch.Tensor, first: torch.Tensor, order: torch.Tensor, place: torch.Tensor, E: int) -> None:
+def experts_sort(chosen: torch.Tensor, first: torch.Tensor, order: torch.Tensor, place: torch.Tensor, E: int,
+                 slots: Optional[torch.Tensor] = None) -> None:
     """The (token, slot) pairs of chosen [T, top] grouped by expert: first int32 [E + 1], order and place int32 [T * top].
-    Numbers from E - 1 on share the last bin (with identity experts, E is the experts with matrices and one more)."""
-    _dev("experts_sort", chosen, first, order, place)
+    Numbers from E - 1 on share the last bin (with identity experts, E is the experts with matrices and one more).
+    `slots` int32 [T]: tokens whose number is negative are left out (place -1), and first[E] counts the others' pairs."""
+    _dev("experts_sort", chosen, first, order, place, slots)
     n = chosen.numel()
+    _req(chosen.dim() == 2 and (slots is None or (slots.dtype == torch.int32 and slots.numel() == chosen.shape[0])), "experts_sort: slots int32 [T]")
     _req(chosen.dtype == first.dtype == order.dtype == place.dtype == torch.int32 and first.numel() == E + 1 and order.numel() == n
          and place.numel() == n, "experts_sort: int32 arrays [E + 1], [pairs], [pairs]")
-    f = _fn("routed_experts", "br_experts_sort", [_P, _P, _P, _P, c_int, c_int, _P])
-    _check(f(_ptr(chosen), _ptr(first), _ptr(order), _ptr(place), n, E, _stream()), "experts_sort")
+    f = _fn("routed_experts", "br_experts_sort", [_P, _P, _P, _P, _P, c_int, c_int, c_int, _P])
+    _check(f(_ptr(chosen), _ptr(slots), _ptr(first), _ptr(order), _ptr(place), n, E, chosen.shape[1], _stream()), "experts_sort")
 
 
 def experts_gather(h: torch.Tensor, order: torch.Tensor, rows: torch.Tensor, top: int, n_rows: Optional[torch.Tensor] = None) -> None:
@@ -1423,7 +1426,8 @@ def experts_combine(out: torch.Tensor, place: torch.Tensor, share: torch.Tensor,
                     chosen: Optional[torch.Tensor] = None, h: Optional[torch.Tensor] = None, experts: int = 0,
                     store: bool = False) -> None:
     """x[t] += sum_s share[t, s] * out[place[t * top + s]] (`store`: = instead of +=); out float [T * top, W].  With `chosen`
-    [T, top] and `h` [T, W], a slot whose number is `experts` or more (an identity expert) takes h[t] instead of an output."""
+    [T, top] and `h` [T, W], a slot whose number is `experts` or more (an identity expert) takes h[t] instead of an output.
+    Tokens that `experts_sort` left out (place -1) add nothing (`store`: zeros)."""
     _dev("experts_combine", out, place, share, x, chosen, h)
     _req((chosen is None) == (h is None) and (chosen is None or (chosen.dtype == torch.int32 and chosen.shape == share.shape and h.shape == x.shape)),
          "experts_combine: chosen int32 [T, top] and h [T, W] come together")

@@ -282,7 +282,8 @@ class RoutedExperts(FeedForward):
         first = step.ws.get("moe_first", (bins + 1,), torch.int32)
         order = step.ws.get("moe_order", (n,), torch.int32)
         place = step.ws.get("moe_place", (n,), torch.int32)
-        K.experts_sort(chosen, first, order, place, bins)
+        # (a recorded step of single tokens is padded with sequences of no slot: their rows go to no expert)
+        K.experts_sort(chosen, first, order, place, bins, slots=getattr(step, "slots", None) if step.is_decode else None)
         one_by_one = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "")
         # Up to eight pairs an expert on average, or sixteen tokens, the weights are streamed once for up to 16 pairs at a time;
         # beyond, the prompt products' tiles read them once for 128 or 256.  Both products in us, streams against tiles: 32 experts of

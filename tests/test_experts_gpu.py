@@ -131,6 +131,37 @@ def test_products_of_many_tokens(T, top, E, W, F, how, identity, alpha):
             assert torch.all(out[int(first[E]):] == 7.0)
 
 
+@pytest.mark.parametrize("T,live", [(1, 1), (8, 6), (8, 0), (64, 40), (1024, 1000)])
+def test_tokens_without_a_slot_go_to_no_expert(T, live):
+    """Pairs of padding tokens are in nobody's run, and the outputs' sum leaves their rows as they are (or zero)."""
+    from braidinfer_amd import kernels as K
+    top, E, W = 3, 7, 20
+    chosen = drawn(T, top, E, "drawn", T)
+    g = torch.Generator().manual_seed(T + live)
+    slots = torch.full((T,), -1, dtype=torch.int32)
+    alive = torch.randperm(T, generator=g)[:live]
+    slots[alive] = torch.arange(live, dtype=torch.int32)
+    n = T * top
+    first, order, place = (torch.full((k,), 9999, dtype=torch.int32, device="cuda") for k in (E + 1, n, n))
+    K.experts_sort(chosen, first, order, place, E, slots=slots.cuda())
+    c, first, order, place = chosen.cpu(), first.cpu(), order.cpu(), place.cpu().reshape(T, top)
+    keep = slots >= 0
+    assert first.tolist() == [int((c[keep] < e).sum()) for e in range(E + 1)]
+    assert torch.all(place[~keep] == -1) and sorted(place[keep].reshape(-1).tolist()) == list(range(live * top))
+    for t in alive.tolist():
+        for s in range(top):
+            assert int(order[place[t, s]]) == t * top + s and first[c[t, s]] <= place[t, s] < first[c[t, s] + 1]
+    out = torch.full((n, W), float("nan"))
+    out[:live * top] = torch.randn(live * top, W, generator=g)
+    share, x = torch.rand(T, top, generator=g), torch.randn(T, W, generator=g)
+    for store in (False, True):
+        got = x.cuda()
+        K.experts_combine(out.cuda(), place.reshape(-1).cuda(), share.cuda(), got, store=store)
+        want = torch.zeros(T, W, dtype=torch.float64) if store else x.double()
+        want[keep] += (share[keep][:, :, None].double() * out[place[keep].long()].double()).sum(1)
+        assert (got.cpu().double() - want).abs().max() < 1e-5
+
+
 @pytest.mark.parametrize("top", [1, 7, 8, 9, 17])
 @pytest.mark.parametrize("W", [4, 1028, 30])
 def test_combine_adds_every_slot(top, W):
