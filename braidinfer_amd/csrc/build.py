@@ -42,9 +42,10 @@ MODULES: Dict[str, List[str]] = {
     "delta_rule": ["delta_rule.hip"],
     "latent_attention": ["latent_attention.hip"],
     "routed_experts": ["routed_experts.hip"],
+    "experts_wide": ["experts_wide.hip"],
     "streams": ["streams.hip"],
 }
-HEADERS = ["common.h", "no_alloc.h"]
+HEADERS = ["common.h", "no_alloc.h", "expert_units.h"]
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

@@ -16,18 +16,9 @@
 // row.  Such pairs are sorted into one bin behind the experts', no product sees them, and `down` / `combine` take the
 // row of h itself.  The gated unit may be the clamped one (`alpha` > 0): g sigmoid(alpha g) (u + 1) with
 // g = min(W_g h, limit), u = clamp(W_u h, -limit, limit).
-#include "common.h"
+#include "expert_units.h"
 
 #define RX_MAX_PER_LANE 8          // experts a lane keeps: up to 512 experts
-
-__device__ __forceinline__ float rx_glu(float g, float u, float limit, float alpha) {
-    if (alpha > 0.f) {
-        g = fminf(g, limit);
-        u = fminf(fmaxf(u, -limit), limit);
-        return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
-    }
-    return g / (1.0f + expf(-g)) * u;
-}
 
 // grid (T), one wave a token.
 __global__ __launch_bounds__(64) void route_topk_kernel(const float* __restrict__ scores, const float* __restrict__ bias,
@@ -729,50 +720,6 @@ __global__ __launch_bounds__(256) void experts_down_grouped_kernel(const bf16* _
 #define RXS_S 2
 #define RXS_MAX_E 512
 #define RXS_MAX_PAIRS 1024
-
-struct RxUnit { int e, t, j, p0, np; };       // expert, unit of its rows, group of its pairs: the group's first pair and size
-
-template <int XR>
-__device__ __forceinline__ RxUnit rx_unit_at(int u, const int* cum, const int* firstL, int E, int tiles) {
-    int lo = 0, hi = E;                                       // the expert with cum[e] <= u < cum[e + 1]
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (cum[mid] <= u) lo = mid; else hi = mid;
-    }
-    RxUnit r;
-    r.e = lo;
-    const int n = firstL[lo + 1] - firstL[lo], groups = (n + XR - 1) / XR, at = u - cum[lo];
-    r.t = at / groups;
-    r.j = at - r.t * groups;
-    r.p0 = firstL[lo] + r.j * XR;
-    r.np = min(XR, firstL[lo + 1] - r.p0);
-    r.e = __builtin_amdgcn_readfirstlane(r.e);
-    r.t = __builtin_amdgcn_readfirstlane(r.t);
-    r.j = __builtin_amdgcn_readfirstlane(r.j);
-    r.p0 = __builtin_amdgcn_readfirstlane(r.p0);
-    r.np = __builtin_amdgcn_readfirstlane(r.np);
-    return r;
-}
-
-template <int XR>
-__device__ __forceinline__ void rx_next_unit(RxUnit& r, const int* firstL, int E, int tiles) {
-    int end = __builtin_amdgcn_readfirstlane(firstL[r.e + 1]);
-    if (r.p0 + XR < end) {
-        ++r.j;
-        r.p0 += XR;
-    } else {
-        r.j = 0;
-        if (++r.t == tiles) {
-            r.t = 0;
-            do {
-                ++r.e;
-                r.p0 = end;
-                end = __builtin_amdgcn_readfirstlane(firstL[r.e + 1]);
-            } while (r.e < E && end == r.p0);                 // firstL[E + 1] = firstL[E]: ends behind the last expert
-        } else r.p0 = __builtin_amdgcn_readfirstlane(firstL[r.e]);
-    }
-    r.np = min(XR, end - r.p0);
-}
 
 template <int XR, bool UP>
 __global__ __launch_bounds__(RXS_NW * 64) void experts_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wt,

@@ -131,6 +131,44 @@ def test_products_of_many_tokens(T, top, E, W, F, how, identity, alpha):
             assert torch.all(out[int(first[E]):] == 7.0)
 
 
+# experts' pairs at 1, 31 to 33 (a group of 32 rows), 63 to 65 (of 64) and none; widths of 2 and 3 chunks of 128 and of no whole
+# number of any unit's rows; identities behind the experts
+@pytest.mark.parametrize("T,top,E,W,F,how,identity,alpha", [
+    (31, 1, 1, 256, 256, "one", 0, 0.0), (32, 2, 3, 384, 256, "one", 0, 0.0), (33, 1, 2, 256, 400, "drawn", 1, 1.702), (63, 1, 2, 400, 256, "one", 0, 0.0),
+    (65, 2, 4, 512, 384, "one", 0, 0.0), (40, 8, 32, 640, 1152, "drawn", 0, 0.0), (100, 3, 9, 1024, 256, "drawn", 2, 1.702), (24, 8, 32, 1024, 888, "drawn", 0, 0.0)])
+def test_products_by_all_waves_together(T, top, E, W, F, how, identity, alpha):
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(T + W + F)
+    h, w_gu = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5)
+    w_down = bf(rng.standard_normal((E, W, F)) / F ** 0.5)
+    chosen = drawn(T, top, E + identity, how, T)
+    want_y, want = products(h, w_gu, w_down, chosen, 0.9, alpha)
+    first, order, place = sorted_pairs(chosen, E + (1 if identity else 0))
+    n, real = T * top, chosen < E
+    if W % 128 == 0:
+        y = torch.full((n, F), 7.0, dtype=torch.bfloat16, device="cuda")
+        K.experts_wide(h.cuda(), w_gu.cuda(), first, order, y, top, 0.9 if alpha else 0.0, alpha)
+        got_y = y[place.long()].double().reshape(T, top, F)
+        assert float((got_y - want_y)[real].abs().max()) < 2 ** -8 * float(want_y.abs().max())      # one bfloat16 rounding, 2^-9
+        assert torch.all(y[int(first[E]):] == 7.0)                                                  # identities' rows are nobody's
+    if F % 128 == 0:
+        y = want_y.to(torch.bfloat16).reshape(n, F)[order.long()].contiguous()
+        out = torch.full((n, W), 7.0, dtype=torch.float32, device="cuda")
+        K.experts_wide(y, w_down.cuda(), first, None, out)
+        got = out[place.long()].double().reshape(T, top, W)
+        # float sums of the same rows: F products in any order, each of at most the largest |row| x |weight|
+        assert float((got - want)[real].abs().max()) < F * 2 ** -24 * float(want_y.abs().max()) * float(w_down.abs().max())
+        assert float((got - want)[real].norm() / want[real].norm()) < 1e-5
+        assert torch.all(out[int(first[E]):] == 7.0)
+
+
+@pytest.mark.parametrize("E,N,K_,pairs,takes", [(1, 1, 256, 1, True), (512, 64, 256, 2048, True), (513, 64, 256, 8, False), (4, 64, 128, 8, False),
+                                                (4, 64, 320, 8, False), (4, 64, 256, 2049, False)])
+def test_what_all_waves_together_take(E, N, K_, pairs, takes):
+    from braidinfer_amd import kernels as K
+    assert bool(K._fn("experts_wide", "br_experts_wide_takes", [K.c_int] * 4)(E, N, K_, pairs)) == takes
+
+
 @pytest.mark.parametrize("T,live", [(1, 1), (8, 6), (8, 0), (64, 40), (1024, 1000)])
 def test_tokens_without_a_slot_go_to_no_expert(T, live):
     """Pairs of padding tokens are in nobody's run, and the outputs' sum leaves their rows as they are (or zero)."""
