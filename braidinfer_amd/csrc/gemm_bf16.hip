@@ -9,6 +9,8 @@
 //  * gemm_tile: LDS-staged tiles for many rows (prompts): 4 waves, each a TM x TN grid of
 //    v_mfma_f32_32x32x16_bf16 blocks; global loads of the next k-tile are issued before the
 //    current one is multiplied and written to the other LDS buffer after it.
+//  * gemm_narrow: more than 16 rows against at most 64 weight rows (a router): operands straight from memory, K
+//    shared out over the waves of a workgroup.
 //  * gemm_skinny: M <= 64 rows (decode): pure weight streaming.  A workgroup owns 16*RB
 //    weight rows; its 4 waves take interleaved 128-element k-chunks, every lane reading
 //    64 contiguous bytes of one weight row per chunk straight into v_mfma_f32_16x16x32_bf16
@@ -1130,6 +1132,122 @@ static int launch_skinny(const bf16* A, const bf16* W, void* C, int M, int N, in
     return br_check_launch();
 }
 
+// ------------------------------------------------------------- gemm_narrow ----------
+// More than 16 rows against at most 64 weight rows (a router's scores, the narrow half of a low-rank pair).  The tiles above
+// give such a product one workgroup to 128 rows, 15 compute units for 1,801 rows that each walk all of K.  Here a workgroup takes 16 rows
+// of A and 16 NB weight rows, its eight waves U chunks of 128 k each at a time straight into operands (with K = 4,096 all of a
+// wave's loads are under way at once), and the waves' sums meet in LDS in wave order.  The weights come from the L2, once per
+// workgroup.  grid (ceil(M / 16), ceil(N / (16 NB))).  Needs K % 8 == 0 and 16-byte aligned rows; rows beyond M or N are
+// read from the last one and dropped at the store.
+// 32 weight rows of 4,096 (us, launch to launch): 64 rows 10.2 -> 8.7, 300 rows 14.3 -> 8.7, 1,801 rows 39.0 -> 9.2, 7,000 rows
+// 39.6 -> 23.2; the error against 64 bits 1.0e-7 of the result (before 1.0e-7 to 4.0e-7).  Bound by the latency of one
+// round of loads and the sum of the waves; each further round of workgroups costs the same again.
+template <int NB, int U, int MODE>
+__global__ __launch_bounds__(512) void gemm_narrow_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, void* __restrict__ C,
+                                                          int M, int N, int K, size_t lda, size_t ldc) {
+    constexpr int NW = 8, COLS = 16 * NB;
+    __shared__ float red[NW][16][COLS + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int m0 = blockIdx.x * 16, n0 = blockIdx.y * COLS;
+    f32x4 acc[2][NB];                                         // two chains each: shorter sums round less
+    const bf16* wp[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        acc[0][j] = acc[1][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        wp[j] = W + (size_t)min(n0 + 16 * j + r16, N - 1) * K + g * 8;
+    }
+    const bf16* ap = A + (size_t)min(m0 + r16, M - 1) * lda + g * 8;
+    // lane (row r16, group g) holds k = chunk * 128 + s * 32 + g * 8 + [0, 8) for s = 0..3
+    const int nfull = K / 128, nch = (K + 127) / 128;
+    int c = wave * U;
+    for (; c + U <= nfull; c += NW * U) {
+        bf16x8 fa[U][4], fw[U][NB][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int kb = (c + u) * 128 + s * 32;
+                fa[u][s] = *(const bf16x8*)(ap + kb);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) fw[u][j][s] = *(const bf16x8*)(wp[j] + kb);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) acc[s & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[u][s], fw[u][j][s], acc[s & 1][j], 0, 0, 0);
+    }
+    // this wave's leftover chunks (fewer than U, or the partial last chunk), guarded along k
+    for (int u = 0; u < U && c + u < nch; ++u) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int kb = (c + u) * 128 + s * 32;
+            const bool in = kb + g * 8 + 8 <= K;
+            const bf16x8 a = in ? *(const bf16x8*)(ap + kb) : zero8();
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                const bf16x8 b = in ? *(const bf16x8*)(wp[j] + kb) : zero8();
+                acc[s & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[s & 1][j], 0, 0, 0);
+            }
+        }
+    }
+    // acc[..][j][r]: row 4 g + r, weight row 16 j + r16
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][4 * g + r][16 * j + r16] = acc[0][j][r] + acc[1][j][r];
+    __syncthreads();
+    for (int e = tid; e < 16 * COLS; e += NW * 64) {
+        const int m = e / COLS, n = e % COLS;
+        if (m0 + m < M && n0 + n < N) {
+            float v[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v[w] = red[w][m][n];
+#pragma unroll
+            for (int h = 1; h < NW; h *= 2)
+#pragma unroll
+                for (int w = 0; w < NW; w += 2 * h) v[w] += v[w + h];
+            store_out<MODE>(C, (size_t)(m0 + m) * ldc + n0 + n, v[0]);
+        }
+    }
+}
+
+template <int NB, int U>
+static int launch_narrow(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode, hipStream_t s) {
+    const dim3 grid((unsigned)((M + 15) / 16), (unsigned)((N + 16 * NB - 1) / (16 * NB)));
+    if (mode == OUT_BF16) gemm_narrow_kernel<NB, U, OUT_BF16><<<grid, 512, 0, s>>>(A, W, C, M, N, K, lda, ldc);
+    else if (mode == OUT_F32) gemm_narrow_kernel<NB, U, OUT_F32><<<grid, 512, 0, s>>>(A, W, C, M, N, K, lda, ldc);
+    else gemm_narrow_kernel<NB, U, OUT_F32_ACC><<<grid, 512, 0, s>>>(A, W, C, M, N, K, lda, ldc);
+    return br_check_launch();
+}
+
+// How many blocks of 16 weight rows a workgroup takes (1, 2 or 4), or 0 where the tiles are as fast: rounds of workgroups
+// over the compute units times what a round takes, 7, 10.5 and 17.5 us with K = 4,096 and in proportion otherwise, against the 37
+// of the tiles' single round (measured, us; K = 4,096, 64 weight rows: 1,801 rows 17 / 13 / 20 by 1 / 2 / 4 blocks and 39 by the
+// tiles, 3,000 rows 23 / 23 / 20 and 39, 5,000 rows 37 / 34 / 37 and 39, 7,000 rows 51 / 44 / 37 and 40).
+static int narrow_blocks(int M, int N, int K, int mode, int cus) {
+    if (M <= 16 || N > 64 || K < 256 || mode == OUT_SWIGLU || cus <= 0) return 0;
+    static const double round_us[3] = {7.0, 10.5, 17.5};
+    int best = 0;
+    double least = 32.0;
+    for (int i = 0; i < 3 && (i == 0 || 16 << (i - 1) < N); ++i) {
+        const long long units = (long long)((M + 15) / 16) * ((N + (16 << i) - 1) / (16 << i));
+        const double t = (double)((units + cus - 1) / cus) * round_us[i];
+        if (t < least) { least = t; best = 1 << i; }
+    }
+    return best;
+}
+
+static int launch_narrow_blocks(int blocks, const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode,
+                                hipStream_t s) {
+    // a wave's share of K in one go where it has four chunks, two where it has fewer
+    if (blocks == 1) return K >= 4096 ? launch_narrow<1, 4>(A, W, C, M, N, K, lda, ldc, mode, s) : launch_narrow<1, 2>(A, W, C, M, N, K, lda, ldc, mode, s);
+    if (blocks == 2) return K >= 4096 ? launch_narrow<2, 4>(A, W, C, M, N, K, lda, ldc, mode, s) : launch_narrow<2, 2>(A, W, C, M, N, K, lda, ldc, mode, s);
+    return launch_narrow<4, 2>(A, W, C, M, N, K, lda, ldc, mode, s);
+}
+
 // ------------------------------------------------------------- gemm_skinny_lds ------
 // 16 < M <= 64: the activations of a 512-wide k-slab are staged in LDS once per workgroup
 // with direct global-to-LDS loads (one 1 KB row per wave-load, no registers), because at
@@ -1956,6 +2074,10 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
         if (kernel == 0 && M <= 16 && !stream_ok) return BR_BAD_ARG;      // blocked weights have K from 1024
     }
     const bool chosen = kernel == 0;
+    if (chosen && wl == WL_ROWS && aligned) {
+        const int blocks = narrow_blocks(M, N, K, mode, br_device_cus());
+        if (blocks) return launch_narrow_blocks(blocks, A, W, C, M, N, K, lda, ldc, mode, s);
+    }
     if (kernel == 0)
         kernel = stream_ok ? 7
                  : wide_ok ? 8
