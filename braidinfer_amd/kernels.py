@@ -1398,16 +1398,33 @@ def experts_up(h: torch.Tensor, w_gu: torch.Tensor, chosen: torch.Tensor, y: tor
              float(alpha), _stream()), "experts_up")
 
 
+def route_sorts_too(T: int, E: int, top: int) -> bool:
+    """Whether `experts_sort` with `route` takes a step of T tokens."""
+    return bool(_fn("routed_experts", "br_experts_route_sort_takes", [c_int] * 3)(T, E, top))
+
+
 def experts_sort(chosen: torch.Tensor, first: torch.Tensor, order: torch.Tensor, place: torch.Tensor, E: int,
-                 slots: Optional[torch.Tensor] = None) -> None:
+                 slots: Optional[torch.Tensor] = None, route=None) -> None:
     """The (token, slot) pairs of chosen [T, top] grouped by expert: first int32 [E + 1], order and place int32 [T * top].
     Numbers from E - 1 on share the last bin (with identity experts, E is the experts with matrices and one more).
-    `slots` int32 [T]: tokens whose number is negative are left out (place -1), and first[E] counts the others' pairs."""
+    `slots` int32 [T]: tokens whose number is negative are left out (place -1), and first[E] counts the others' pairs.
+    `route` = (scores [T, E], bias [E] or None, share [T, top], out_scale): the choice is made here first, as `route_topk` makes it,
+    and `chosen` and `share` are written (`route_sorts_too` says whether one launch can)."""
     _dev("experts_sort", chosen, first, order, place, slots)
     n = chosen.numel()
     _req(chosen.dim() == 2 and (slots is None or (slots.dtype == torch.int32 and slots.numel() == chosen.shape[0])), "experts_sort: slots int32 [T]")
     _req(chosen.dtype == first.dtype == order.dtype == place.dtype == torch.int32 and first.numel() == E + 1 and order.numel() == n
          and place.numel() == n, "experts_sort: int32 arrays [E + 1], [pairs], [pairs]")
+    if route is not None:
+        scores, bias, share, out_scale = route
+        T, top = chosen.shape
+        _dev("experts_sort", scores, bias, share)
+        _req(scores.dtype == share.dtype == torch.float32 and scores.shape == (T, E) and share.shape == (T, top)
+             and (bias is None or (bias.dtype == torch.float32 and bias.numel() == E)), "experts_sort: scores float32 [T, E], bias float32 [E], share float32 [T, top]")
+        f = _fn("routed_experts", "br_experts_route_sort", [_P] * 8 + [c_int] * 3 + [c_float, _P])
+        _check(f(_ptr(scores), _ptr(bias), _ptr(chosen), _ptr(share), _ptr(slots), _ptr(first), _ptr(order), _ptr(place), T, E, top,
+                 float(out_scale), _stream()), "experts_sort")
+        return
     f = _fn("routed_experts", "br_experts_sort", [_P, _P, _P, _P, _P, c_int, c_int, c_int, _P])
     _check(f(_ptr(chosen), _ptr(slots), _ptr(first), _ptr(order), _ptr(place), n, E, chosen.shape[1], _stream()), "experts_sort")
 

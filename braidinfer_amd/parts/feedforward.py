@@ -255,7 +255,13 @@ class RoutedExperts(FeedForward):
         linear(h, self.w_router, scores, step.ws)
         chosen = step.ws.get("moe_chosen", (T, self.top), torch.int32)
         share = step.ws.get("moe_share", (T, self.top), torch.float32)
-        if self.softmax_all:
+        few = step.is_decode or T < int(os.environ.get("BRAIDINFER_BY_EXPERT_FROM", str(self.BY_EXPERT_FROM)))
+        sorts = not few or K.experts_grouped_takes(dt, self.H, self.I)
+        # the plain choice of a few tokens is made where their pairs are sorted
+        route = None
+        if sorts and not self.softmax_all and not self.sigmoid and self.n_scores == self.E and K.route_sorts_too(T, self.E, self.top):
+            route = (scores, self.b_router, share, self.out_scale)
+        elif self.softmax_all:
             K.route_softmax(scores[:, :self.n_out], self.correction, chosen, share, self.top, self.out_scale, self.groups, self.groups_keep)
         elif self.sigmoid:
             K.route_sigmoid(scores, self.correction, chosen, share, self.top, self.groups, self.groups_keep, self.out_scale)
@@ -270,8 +276,7 @@ class RoutedExperts(FeedForward):
         # identity experts return the token's own row
         ident = dict(chosen=chosen, h=h, experts=self.E) if self.identity else {}
         bins = self.E + (1 if self.identity else 0)
-        few = step.is_decode or T < int(os.environ.get("BRAIDINFER_BY_EXPERT_FROM", str(self.BY_EXPERT_FROM)))
-        if few and not K.experts_grouped_takes(dt, self.H, self.I):
+        if not sorts:
             # every pair reads its expert's rows itself: the 32-bit path, and widths the grouped kernels do not take
             y = step.ws.get("moe_y", (T, self.top, self.I), dt)
             K.experts_up(h, self.w_gu, chosen, y, self.limit, self.alpha)
@@ -283,7 +288,7 @@ class RoutedExperts(FeedForward):
         order = step.ws.get("moe_order", (n,), torch.int32)
         place = step.ws.get("moe_place", (n,), torch.int32)
         # (a recorded step of single tokens is padded with sequences of no slot: their rows go to no expert)
-        K.experts_sort(chosen, first, order, place, bins, slots=getattr(step, "slots", None) if step.is_decode else None)
+        K.experts_sort(chosen, first, order, place, bins, slots=getattr(step, "slots", None) if step.is_decode else None, route=route)
         one_by_one = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "")
         # Up to eight pairs an expert on average, or sixteen tokens, the weights are streamed once for up to 16 pairs at a time;
         # beyond, the prompt products' tiles read them once for 128 or 256.  Both products in us, streams against tiles: 32 experts of

@@ -237,3 +237,34 @@ def test_rows_beyond_4_gb():
                 want = a[lo:hi].double() @ w[e].double().T
                 # float sums of 64 products: 64 2^-24 of the terms' sum, which is about 50
                 assert float((out[lo:hi].double() - want).abs().max()) < 64 * 2 ** -24 * 50
+
+
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (8, 32, 8), (16, 64, 64), (13, 63, 5), (5, 65, 3), (16, 512, 8)])
+def test_choice_and_sort_in_one_launch(T, E, top):
+    """The same choice, shares and runs as by two launches, with equal scores, scores that are not numbers and infinite ones among
+    them; the choice of finite scores is that of a stable sort, the shares its softmax."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(T + E)
+    scores, bias = torch.randn(T, E, generator=g).mul(2).round(decimals=1), torch.randn(E, generator=g).round(decimals=1)
+    wild = torch.zeros(T, dtype=torch.bool)
+    if T > 4:
+        scores[1, ::2], scores[2], scores[3, 0], scores[4, E // 2] = float("nan"), float("-inf"), float("inf"), float("-inf")
+        wild[1:5] = True
+    for b in (bias, None):
+        bd, sd = (None if b is None else b.cuda()), scores.cuda()
+        chosen, share = torch.full((T, top), -5, dtype=torch.int32, device="cuda"), torch.zeros(T, top, device="cuda")
+        K.route_topk(sd, bd, chosen, share, top, 1.5)
+        assert int(chosen.min()) >= 0 and int(chosen.max()) < E
+        chosen2, share2 = torch.full_like(chosen, -5), torch.zeros_like(share)
+        first, order, place = (torch.full((k,), 9999, dtype=torch.int32, device="cuda") for k in (E + 1, T * top, T * top))
+        K.experts_sort(chosen2, first, order, place, E, route=(sd, bd, share2, 1.5))
+        assert torch.equal(chosen, chosen2) and torch.equal(share.view(torch.int32), share2.view(torch.int32))
+        c = chosen.cpu().reshape(-1)
+        assert first.tolist() == [int((c < e).sum()) for e in range(E + 1)]
+        assert torch.equal(order.cpu()[place.cpu().long()], torch.arange(T * top, dtype=torch.int32))
+        assert all(int(first[e]) <= int(p) < int(first[e + 1]) for e, p in zip(c.tolist(), place.tolist()))
+        z = (scores if b is None else scores + b)[~wild]
+        v, at = torch.sort(z, dim=1, descending=True, stable=True)
+        assert torch.equal(chosen.cpu()[~wild].long(), at[:, :top])
+        want = 1.5 * torch.softmax(v[:, :top].double(), 1)
+        assert float((share.cpu()[~wild].double() - want).abs().max()) < 1.5 * (top + 8) * 2 ** -24
