@@ -1477,6 +1477,7 @@ static int split_parts(int M, int N, int K, int mode, size_t scratch_bytes) {
 //    tile it adds the `ssq_tiles` sums of every row in a fixed order, and 1 / rms, the same
 //    for a whole row, multiplies the sums at a tile's end:
 //    y = rsqrt(mean(h^2) + eps) * sum_k W[n,k] (h[k] g[k]).
+// NORM = 3: products of several inputs by stacked weights in one launch (br_gemm_bf16_branches).
 struct StreamNorm {
     const float* gain;     // producer: the next norm's weights [N]
     bf16* xg;              // producer: [M, ldx]
@@ -1484,13 +1485,18 @@ struct StreamNorm {
     float* ssq;            // producer writes, consumer reads: [tiles, SSQ_LD]
     int ssq_tiles;         // consumer: tiles of the producer
     float inv_k, eps;      // consumer: 1 / width of the normed rows, the norm's eps
+    // branches: weight rows b per .. + per multiply the activations b a_step elements on; output columns from gap_at on lie
+    // `gap` further on
+    int per;
+    size_t a_step;
+    int gap_at, gap;
 };
 
 template <int RT, int XR, int KC, int S, int NW, int MODE, int NORM>
 __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C, int M, int N, int K, size_t lda,
                                                               size_t ldc, int ntiles, StreamNorm nrm, int wl) {
-    static_assert(NORM == 0 || (NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC), "norm forms");
+    static_assert(NORM == 0 || (NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC) || (NORM == 3 && MODE == OUT_F32), "norm forms");
     constexpr int STEPS = KC / 32;
     constexpr int ROWB = KC * 2;
     constexpr int STAGE = (RT + XR) * ROWB;
@@ -1528,6 +1534,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
     int cp_t = 0, cp_c = 0;      // compute cursor
     int buf = 0;
 
+    // NORM 3: where the activations of the tile to ask for lie behind the first branch's
+#define BRANCH_OFF(T) ((size_t)((((int)blockIdx.x + (T) * (int)gridDim.x) * RT) / nrm.per) * nrm.a_step)
+    size_t a_off = NORM == 3 ? BRANCH_OFF(0) : 0;
 #define ISSUE(J)                                                                                         \
     do {                                                                                                 \
         int chunk_ = wave + is_c * NW + rot;                                                             \
@@ -1544,6 +1553,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                 int m_ = row_ - RT;                                                                      \
                 if (m_ > M - 1) m_ = M - 1;                                                              \
                 gp_ = A + (size_t)m_ * lda + (size_t)chunk_ * KC + ((dcol ^ (row_ & 7)) * 8);            \
+                if (NORM == 3) gp_ += a_off;                                                             \
             }                                                                                            \
             const unsigned lds_ = __builtin_amdgcn_readfirstlane(ring_lds + (J) * STAGE + q_ * 1024);    \
             if (q_ < WDMA)                              /* weights pass once: non-temporal */            \
@@ -1551,7 +1561,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
             else                                        /* activations are every workgroup's: they stay cached */ \
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_), "v"(gp_) : "m0"); \
         }                                                                                                \
-        if (++is_c == ncw) { is_c = 0; ++is_t; }                                                         \
+        if (++is_c == ncw) {                                                                             \
+            is_c = 0;                                                                                    \
+            ++is_t;                                                                                      \
+            if (NORM == 3) a_off = BRANCH_OFF(is_t);                                                     \
+        }                                                                                                \
     } while (0)
 
     // prologue
@@ -1654,7 +1668,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
 #pragma unroll
                                 for (int w = 0; w < NW; ++w) v += rb[(w * 16 + nl) * 17 + m];
                                 if (NORM == 2) v *= rstd[m];
-                                const size_t idx = (size_t)m * ldc + n;
+                                const size_t idx = (size_t)m * ldc + n + (NORM == 3 && n0 >= nrm.gap_at ? nrm.gap : 0);
                                 if (MODE == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
                                 else if (MODE == OUT_F32) ((float*)C)[idx] = v;
                                 // one add per element and product, without a read that this wave would
@@ -1669,6 +1683,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
         }
     }
 #undef ISSUE
+#undef BRANCH_OFF
 }
 
 
@@ -1699,6 +1714,9 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
     } while (0)
     if constexpr (NORM == 1) {
         BR_STREAM(OUT_F32_ACC);
+    } else if constexpr (NORM == 3) {
+        if (mode != OUT_F32) return BR_BAD_ARG;
+        BR_STREAM(OUT_F32);
     } else {
         if (mode == OUT_BF16) BR_STREAM(OUT_BF16);
         else if (mode == OUT_F32) BR_STREAM(OUT_F32);
@@ -1727,7 +1745,8 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
 // scale: the activations are the bf16(h * g) rows that the product before left for an RMS norm
 // (see gemm_stream's NORM forms); the sums are multiplied by 1 / rms of their row, run by run.
 #define WIDE_S 3
-template <int MB, int HB>
+// BRANCHES: products of several inputs by stacked weights in one launch (br_gemm_bf16_branches); a unit lies in one branch.
+template <int MB, int HB, bool BRANCHES = false>
 __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                void* __restrict__ C, int M, int N, int K, size_t lda,
                                                                size_t ldc, int mode, int partial, int scale,
@@ -1796,6 +1815,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                 int m_ = row_ - H;                                                                            \
                 if (m_ > M - 1) m_ = M - 1;                                                                   \
                 gp_ = A + (size_t)m_ * lda + (size_t)(c0_ + rot_) * 128;                                      \
+                if (BRANCHES) gp_ += (size_t)(tile_ * H / nrm.per) * nrm.a_step;                              \
             }                                                                                                 \
             src[q_] = gp_ + (((lane & 15) ^ (row_ & 7)) * 8);                                                 \
         }                                                                                                     \
@@ -1918,7 +1938,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                 if (m < M && n < N) {
                     float v = red[nl * RLD + m];
                     if (scale) v *= rstd[m];
-                    const size_t idx = (size_t)m * ldc + n;
+                    const size_t idx = (size_t)m * ldc + n + (BRANCHES && n0 >= nrm.gap_at ? nrm.gap : 0);
                     if (partial) ((float*)C)[part * part_stride + (size_t)m * N + n] = v;
                     else if (mode == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
                     else if (mode == OUT_F32) ((float*)C)[idx] = v;
@@ -2278,6 +2298,54 @@ extern "C" int br_gemm_bf16_norm_scaled(const void* XG, const void* W, void* C, 
                                                scratch_bytes, s, 2, nrm, 0, 0, wl);
     }
     return BR_BAD_ARG;
+}
+
+// Several products in one launch: C[m, col(n)] = sum_k A[b][m, k] W[n, k] with b = n / per the branch of weight row n, A[b] the
+// branch's rows b a_step elements behind the first's, and col(n) = n, or n + gap from n = gap_at on; float results, up to 64
+// rows.  A mixer's projections of inputs that differ are four launches otherwise, each with its own ramp and, from 17 rows on, a
+// second launch for the sums of its runs along k: four of 4,096 by 4,096, weights in no cache,
+// 6 rows 34.4 -> 25.6 us, 24 rows 58.6 -> 25.9, 64 rows 60.0 -> 30.7; four of 2,048 by 2,048 20.4 -> 10.6, 39.0 -> 14.1, 46.0 -> 17.4.
+template <int MB, int HB>
+static int launch_branches_wide(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const StreamNorm& br, int cus,
+                                hipStream_t s) {
+    auto kern = gemm_stream_wide_kernel<MB, HB, true>;
+    constexpr size_t lds = (size_t)WIDE_S * (16 * HB + 16 * MB) * 256 + 64 * 4;
+    static bool set = false;
+    if (!set) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
+        set = true;
+    }
+    const int ntiles = N / (16 * HB);
+    kern<<<ntiles < cus ? ntiles : cus, 512, lds, s>>>(A, W, C, M, N, K, lda, ldc, OUT_F32, 0, 0, ntiles, 1, K / 128, 0, br, WL_ROWS);
+    return br_check_launch();
+}
+
+extern "C" int br_gemm_bf16_branches_takes(int M, int per, int K) {
+    return M > 0 && M <= 64 && per > 0 && per % 128 == 0 && K % STREAM_KC == 0 && K / STREAM_KC >= STREAM_NW;
+}
+
+extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, int M, int branches, int per, int K, size_t a_step, size_t lda,
+                                     size_t ldc, int gap_at, int gap, hipStream_t s) {
+    const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
+    if (branches < 1 || branches > 64 || !br_gemm_bf16_branches_takes(M, per, K) || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 ||
+        gap_at % per || ((uintptr_t)A | (uintptr_t)W) % 16 || ldc < (size_t)branches * per || (long long)branches * per > 0x3fffffff)
+        return BR_BAD_ARG;
+    const int N = branches * per, cus = br_device_cus();
+    if (!cus) return BR_LAUNCH_FAILED;
+    StreamNorm br{};
+    br.per = per;
+    br.a_step = a_step;
+    br.gap_at = gap_at;
+    br.gap = gap;
+    if (M <= 8) return launch_stream<8, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
+    if (M <= 16) return launch_stream<16, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
+    // units of 64 rows, or of 128 where these fill the chip's rounds better (a unit's chunk costs its rows and 16 more, as in wide_shape)
+    const long long r64 = (N / 64 + cus - 1) / cus, r128 = (N / 128 + cus - 1) / cus;
+    if (r128 * 144 < r64 * 80)
+        return M <= 32 ? launch_branches_wide<2, 8>(A, W, C, M, N, K, lda, ldc, br, cus, s)
+                       : launch_branches_wide<4, 8>(A, W, C, M, N, K, lda, ldc, br, cus, s);
+    return M <= 32 ? launch_branches_wide<2, 4>(A, W, C, M, N, K, lda, ldc, br, cus, s)
+                   : launch_branches_wide<4, 4>(A, W, C, M, N, K, lda, ldc, br, cus, s);
 }
 
 // The float sums of the runs of A W^T (17 to 64 rows, bf16 result meant), left in `scratch` as

@@ -28,7 +28,7 @@ from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, Runtime, register_part
 from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
-from .linear import linear, stream_layout
+from .linear import blocks_at_load, linear, stream_layout
 
 BRANCHES = ("r", "k", "v", "g", "w")
 
@@ -47,7 +47,7 @@ class WKVTimeMix(Mixer):
         self.H, self.nh, self.d, self.rank = int(hidden_size), int(num_heads), int(head_dim), int(decay_rank)
         self.eps = float(norm_eps)
         self.names = dict(self.NAMES, **(names or {}))
-        self.mu = self.w = self.w0 = self.u = self.norm_w = self.w_o = None
+        self.mu = self.w = self.w0 = self.u = self.norm_w = self.w_o = self.w_four = None
         self.state_floats = 1
         for n in K.glr_state_shape(self.nh, self.d, self.d):
             self.state_floats *= n
@@ -71,7 +71,19 @@ class WKVTimeMix(Mixer):
         for i, s in enumerate(BRANCHES):
             mu[i].copy_(tensors[prefix + n["mu_" + s]].to(torch.float32).reshape(-1))
         self.mu = mu
-        self.w = {s: stream_layout(tensors[prefix + n[s]], rt) for s in ("r", "k", "v", "g", "w1", "w2")}
+        # r, k, v and g stacked, where a step of few tokens can take them in one launch; their rows otherwise
+        hd, four = self.nh * self.d, ("r", "k", "v", "g")
+        mats = {s: tensors[prefix + n[s]] for s in four}
+        self.w_four = None
+        if all(m.dtype == torch.bfloat16 for m in mats.values()) and not blocks_at_load(hd, self.H, torch.bfloat16, rt) \
+                and K.gemm_branches_takes(1, hd, self.H):
+            self.w_four = rt.empty((4 * hd, self.H), torch.bfloat16)
+            for i, s in enumerate(four):
+                self.w_four[i * hd:(i + 1) * hd].copy_(mats[s])
+            self.w = {s: self.w_four[i * hd:(i + 1) * hd] for i, s in enumerate(four)}
+        else:
+            self.w = {s: stream_layout(m, rt) for s, m in mats.items()}
+        self.w.update({s: stream_layout(tensors[prefix + n[s]], rt) for s in ("w1", "w2")})
         self.w_o = stream_layout(tensors[prefix + n["o"]], rt)
         self.w0 = rt.own(tensors[prefix + n["w0"]].to(torch.float32).reshape(-1))
         self.u = rt.own(tensors[prefix + n["u"]].to(torch.float32).reshape(-1))
@@ -93,9 +105,12 @@ class WKVTimeMix(Mixer):
         K.shift_mix(h, self.mu, mixes, kept, step.seq_of_token, step.cu_seqlens, step.slots, step.n_seqs, step.is_decode)
         # float sums r | k | v | z | g side by side
         rows = step.ws.get("wkv_rows", (T, 5 * hd), torch.float32)
-        for i, s in enumerate(("r", "k", "v")):
-            linear(mixes[i], self.w[s], rows[:, i * hd:(i + 1) * hd], step.ws)
-        linear(mixes[3], self.w["g"], rows[:, 4 * hd:5 * hd], step.ws)
+        if self.w_four is not None and dt == torch.bfloat16 and K.gemm_branches_takes(T, hd, self.H):
+            K.gemm_branches(mixes[:4], self.w_four, rows, gap_at=3, gap=hd)
+        else:
+            for i, s in enumerate(("r", "k", "v")):
+                linear(mixes[i], self.w[s], rows[:, i * hd:(i + 1) * hd], step.ws)
+            linear(mixes[3], self.w["g"], rows[:, 4 * hd:5 * hd], step.ws)
         low = step.ws.get("wkv_low", (T, self.rank), torch.float32)
         linear(mixes[4], self.w["w1"], low, step.ws)
         low_t = step.ws.get("wkv_low_t", (T, self.rank), dt)

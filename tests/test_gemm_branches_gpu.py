@@ -1,0 +1,36 @@
+"""Several products of few rows in one launch, against float64 products branch by branch."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# rows at the edges of the kernels' 8, 16, 32 and 64; one branch and several; with 128 weight rows a branch (more compute units than
+# tiles) and 16,384 (more tiles than compute units); an odd number of 128-wide chunks; a gap in front, between, behind and none
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("B,per,K_,gap_at,gap", [(4, 128, 1024, 3, 128), (1, 256, 1152, 0, 5), (3, 384, 1024, 3, 7), (2, 16384, 1152, 1, 16), (4, 2048, 2048, 0, 0)])
+def test_branches(M, B, per, K_, gap_at, gap):
+    from braidinfer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(M + per)
+    a = torch.randn(B, M, K_, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(B * per, K_, generator=g, device="cuda").to(torch.bfloat16)
+    wide = torch.full((M, B * per + gap + 4), 7.0, device="cuda")
+    out = wide[:, :B * per + gap]
+    K.gemm_branches(a, w, out, gap_at=gap_at, gap=gap)
+    cols = torch.arange(B * per, device="cuda")
+    cols = cols + gap * (cols >= gap_at * per)
+    want = torch.cat([a[b].double() @ w[b * per:(b + 1) * per].double().T for b in range(B)], 1)
+    assert float((out[:, cols].double() - want).norm() / want.norm()) < 4e-7        # float sums of K products
+    left = torch.ones(wide.shape[1], dtype=torch.bool, device="cuda")
+    left[cols] = False
+    assert torch.all(wide[:, left] == 7.0)
+
+
+def test_branches_refuse():
+    from braidinfer_amd import kernels as K
+    from braidinfer_amd.errors import KernelError
+    for M, per, K_ in ((65, 128, 1024), (4, 64, 1024), (4, 128, 896), (4, 128, 1088)):
+        assert not K.gemm_branches_takes(M, per, K_)
+        a, w = torch.zeros(2, M, K_, dtype=torch.bfloat16, device="cuda"), torch.zeros(2 * per, K_, dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(KernelError):
+            K.gemm_branches(a, w, torch.zeros(M, 2 * per, device="cuda"))
