@@ -846,7 +846,7 @@ static bool quad_takes(const void* C, int M, int N, int K, size_t lda, size_t ld
 #endif
 template <int BM, int BN, int NSA, int NSB, int WVM = 2>
 static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc,
-                            int mode, hipStream_t s, int wl, int parts = 1, float* scratch = nullptr) {
+                            int mode, hipStream_t s, int wl, int parts = 1, float* scratch = nullptr, int* leave = nullptr) {
     const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
     const long long total = (long long)tm * tn;
     if (total > 0x7fffffffLL || !quad_takes(C, M, N, K, lda, ldc)) return BR_BAD_ARG;
@@ -861,8 +861,13 @@ static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N,
                                                                         (size_t)M * N, wl, QuadGroups{});
         int rc = br_check_launch();
         if (rc != BR_OK) return rc;
+        if (leave) {                                                  // the runs' sums are the caller's
+            *leave = parts;
+            return rc;
+        }
         return launch_split_sum(scratch, parts, C, M, N, ldc, mode, s);
     }
+    if (leave) return BR_BAD_ARG;
     if (mode == OUT_BF16)
         gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_BF16><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
     else if (mode == OUT_F32)
@@ -935,7 +940,7 @@ static int quad_whole_rounds(int M, int N, int K, int mode, int cus, size_t scra
 // run order and applies the epilogue (for products with too few tiles to fill the chip).
 template <int BM, int BN, int WAVES_M, int WAVES_N, int S>
 static int launch_tile_dma(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc,
-                           int mode, hipStream_t s, int parts = 1, float* scratch = nullptr, int wl = 0) {
+                           int mode, hipStream_t s, int parts = 1, float* scratch = nullptr, int wl = 0, int* leave = nullptr) {
     const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
     const long long total = (long long)tm * tn;
     if (total > 0x7fffffffLL) return BR_BAD_ARG;
@@ -949,8 +954,13 @@ static int launch_tile_dma(const bf16* A, const bf16* W, void* C, int M, int N, 
             A, W, scratch, M, N, K, lda, (size_t)N, tm, tn, kpp, (size_t)M * N, wl);
         int rc = br_check_launch();
         if (rc != BR_OK) return rc;
+        if (leave) {                                                  // the runs' sums are the caller's
+            *leave = parts;
+            return rc;
+        }
         return launch_split_sum(scratch, parts, C, M, N, ldc, mode, s);
     }
+    if (leave) return BR_BAD_ARG;
     if (mode == OUT_BF16)
         gemm_tile_dma_kernel<BM, BN, WAVES_M, WAVES_N, S, OUT_BF16><<<(unsigned)total, NT, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl);
     else if (mode == OUT_F32)
@@ -1415,6 +1425,64 @@ __global__ __launch_bounds__(256) void gemm_split_sum_prep_kernel(const float* _
     xg[m * ldx + n] = (bf16)(h * gain[n]);
     const float tot = block_sum(h * h, red);
     if (threadIdx.x == 0) ssq[(n / 256) * SSQ_LD + m] = tot;
+}
+
+// The sum of the runs added into the residual rows C, and the RMS norm that reads them next in the same pass: h = bf16(C gain /
+// rms(C)).  A workgroup takes a row and keeps it in registers, 4 NV columns a thread; the runs are asked for eight at a time and added in
+// run order.  The sum and the norm are two launches otherwise, each reading and writing the rows (us, 4,096 columns): 100 rows in 8 runs
+// 5.9 + 4.1 -> 5.8, 400 rows in 4 runs 10.6 + 5.0 -> 8.6, 700 rows 14.4 + 5.3 -> 11.5.
+template <int NV>
+__global__ __launch_bounds__(1024) void gemm_split_sum_norm_kernel(const float* __restrict__ part, int parts, size_t part_stride,
+                                                                   float* __restrict__ C, int N, size_t ldc, const float* __restrict__ gain,
+                                                                   float eps, bf16* __restrict__ h, size_t ldh) {
+    __shared__ float scratch[16];
+    const size_t m = blockIdx.x;
+    const int nv = N >> 2;
+    const float* pr = part + m * N;
+    f32x4* cr = (f32x4*)(C + m * ldc);
+    f32x4 v[NV], c[NV], g[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = threadIdx.x + blockDim.x * j;
+        v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (i < nv) { c[j] = cr[i]; g[j] = ((const f32x4*)gain)[i]; }
+    }
+    for (int p0 = 0; p0 < parts; p0 += 8) {
+        f32x4 t[8][NV];
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int i = threadIdx.x + blockDim.x * j;
+                if (p0 + p < parts && i < nv) t[p][j] = *(const f32x4*)(pr + (size_t)(p0 + p) * part_stride + 4 * i);
+            }
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (p0 + p < parts && (int)(threadIdx.x + blockDim.x * j) < nv) v[j] += t[p][j];
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = threadIdx.x + blockDim.x * j;
+        if (i < nv) {
+            v[j] = c[j] + v[j];
+            cr[i] = v[j];
+            ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
+        }
+    }
+    const float inv = rsqrtf(block_sum(ss, scratch) / (float)N + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = threadIdx.x + blockDim.x * j;
+        if (i < nv) {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (bf16)(v[j][e] * inv * g[j][e]);
+            *(bf16x4*)(h + m * ldh + 4 * i) = o;
+        }
+    }
 }
 
 static int launch_split_sum(const float* scratch, int parts, void* C, int M, int N, size_t ldc, int mode, hipStream_t s) {
@@ -2375,6 +2443,47 @@ extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, i
                        : launch_branches_wide<4, 8>(A, W, C, M, N, K, lda, ldc, br, cus, s);
     return M <= 32 ? launch_branches_wide<2, 4>(A, W, C, M, N, K, lda, ldc, br, cus, s)
                    : launch_branches_wide<4, 4>(A, W, C, M, N, K, lda, ldc, br, cus, s);
+}
+
+// The runs along k of A W^T (65 to 1,024 rows, a product meant to be added into float rows), left in `scratch` as [*runs][M][N] floats for
+// br_gemm_bf16_add_runs_norm, where br_gemm_bf16_ex would cut the product.  Refuses (BR_BAD_ARG, nothing launched) where it would not,
+// and more than 8,192 columns.
+extern "C" int br_gemm_bf16_leave_runs(const void* A_, const void* W_, int M, int N, int K, size_t lda, void* scratch_, size_t scratch_bytes, int wl,
+                                       int* runs, hipStream_t s) {
+    const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
+    float* scratch = (float*)scratch_;
+    if (M <= 64 || M > 1024 || N <= 64 || N > 8192 || N % 4 || K <= 0 || K % DMA_BK || lda < (size_t)K || lda % 8 || !scratch || !runs ||
+        ((uintptr_t)A | (uintptr_t)W | (uintptr_t)scratch) % 16 || (wl != WL_ROWS && (wl != WL_BLOCKED || K % 128)))
+        return BR_BAD_ARG;
+    const int cus = br_device_cus(), mode = OUT_F32_ACC;
+    if (!cus) return BR_LAUNCH_FAILED;
+    int kernel = 0, parts = 1, k2, p2;
+    if (M > 128 && quad_takes(scratch, M, N, K, lda, N)) {
+        const double single = choose_quad(M, N, K, mode, cus, scratch_bytes, &kernel, &parts);
+        if (quad_whole_rounds(M, N, K, mode, cus, scratch_bytes, single, &k2, &p2) > 0) return BR_BAD_ARG;
+    } else choose_tile(M, N, K, mode, cus, scratch_bytes, &kernel, &parts);
+    if (parts < 2) return BR_BAD_ARG;
+    if (kernel == 12) return launch_tile_quad<256, 256, QUAD12>(A, W, scratch, M, N, K, lda, N, mode, s, wl, parts, scratch, runs);
+    if (kernel == 13) return launch_tile_quad<128, 256, QUAD13>(A, W, scratch, M, N, K, lda, N, mode, s, wl, parts, scratch, runs);
+    if (kernel == 14) return launch_tile_quad<256, 192, QUAD14>(A, W, scratch, M, N, K, lda, N, mode, s, wl, parts, scratch, runs);
+    if (kernel == 15) return launch_tile_quad<256, 224, 2, 3, 4>(A, W, scratch, M, N, K, lda, N, mode, s, wl, parts, scratch, runs);
+    if (kernel == 5) return launch_tile_dma<128, 256, 2, 4, 3>(A, W, scratch, M, N, K, lda, N, mode, s, parts, scratch, wl, runs);
+    if (kernel == 6) return launch_tile_dma<128, 128, 2, 2, 2>(A, W, scratch, M, N, K, lda, N, mode, s, parts, scratch, wl, runs);
+    return BR_BAD_ARG;
+}
+
+// C += the runs [runs][M][N] in run order, and h[M, ldh] = bf16(C gain / rms(C)).
+extern "C" int br_gemm_bf16_add_runs_norm(const float* sums, int runs, float* C, int M, int N, size_t ldc, const float* gain, float eps, void* h,
+                                          size_t ldh, hipStream_t s) {
+    if (M <= 0) return BR_OK;
+    if (N <= 0 || N > 8192 || N % 4 || runs < 1 || ldc < (size_t)N || ldc % 4 || ldh < (size_t)N || ldh % 4 ||
+        ((uintptr_t)sums | (uintptr_t)C | (uintptr_t)gain | (uintptr_t)h) % 16)
+        return BR_BAD_ARG;
+    const size_t stride = (size_t)M * N;
+    const int threads = N >= 4096 ? 1024 : (N / 4 + 63) / 64 * 64;
+    if (N <= 4096) gemm_split_sum_norm_kernel<1><<<M, threads, 0, s>>>(sums, runs, stride, C, N, ldc, gain, eps, (bf16*)h, ldh);
+    else gemm_split_sum_norm_kernel<2><<<M, threads, 0, s>>>(sums, runs, stride, C, N, ldc, gain, eps, (bf16*)h, ldh);
+    return br_check_launch();
 }
 
 // The float sums of the runs of A W^T (17 to 64 rows, bf16 result meant), left in `scratch` as

@@ -105,10 +105,20 @@ def embedding(table: torch.Tensor, tokens: torch.Tensor, out: torch.Tensor, scal
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, eps: float,
-            rows: Optional[torch.Tensor] = None) -> None:
+            rows: Optional[torch.Tensor] = None, add=None) -> None:
+    """out = x / sqrt(mean(x^2) + eps) * w, of the rows `rows` of x where given.  `add` = (sums, runs): a product's runs
+    (`gemm_leave_runs`) are first added into x, in the same kernel (bfloat16 `out`, up to 8,192 columns in steps of 4, no `rows`)."""
     _dev("rmsnorm", x, w, out, rows)
     H = x.shape[-1]
     R = out.shape[0]
+    if add is not None:
+        sums, runs = add
+        _dev("rmsnorm", sums)
+        _req(x.dtype == w.dtype == sums.dtype == torch.float32 and out.dtype == torch.bfloat16 and rows is None and x.shape == out.shape == (R, H)
+             and w.numel() == H and runs >= 1 and sums.numel() >= runs * R * H, "rmsnorm: runs to add are float32 [runs, R, H], out bfloat16 [R, H]")
+        f = _fn("gemm_bf16", "br_gemm_bf16_add_runs_norm", [_P, c_int, _P, c_int, c_int, c_size_t, _P, c_float, _P, c_size_t, _P])
+        _check(f(_ptr(sums), int(runs), _ptr(x), R, H, H, _ptr(w), float(eps), _ptr(out), H, _stream()), "rmsnorm")
+        return
     _req(x.dtype == torch.float32 and w.dtype == torch.float32, "rmsnorm: x and w must be float32")
     _req(w.numel() == H and out.shape[-1] == H, "rmsnorm: widths of x, w and out differ")
     if rows is None:
@@ -587,6 +597,23 @@ def gemm_norm_prepare(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, gain: t
              _ptr(xg), xg.stride(0) if M > 1 else N, _ptr(ssq), ctypes.byref(tiles), _ptr(scratch),
              0 if scratch is None else scratch.numel() * 4, wl, _stream()), "gemm_norm_prepare")
     return tiles.value
+
+
+def gemm_leave_runs(a: torch.Tensor, w: torch.Tensor, n_out: int, scratch: torch.Tensor) -> int:
+    """The runs along k of a @ w^T (65 to 1,024 bfloat16 rows, `n_out` columns) as float sums in `scratch`, [runs][M][n_out], for `rmsnorm`
+    to add; returns their number, or 0 (nothing launched) where such a product is not cut or the sizes are not taken."""
+    _dev("gemm_leave_runs", scratch)
+    M, K = a.shape
+    N, wk, wl = _weight_dims("gemm_leave_runs", w, n_out)
+    _req(a.is_cuda and a.dtype == w.dtype == torch.bfloat16 and scratch.dtype == torch.float32 and wk == K and N == n_out and a.stride(1) == 1,
+         "gemm_leave_runs: bfloat16 rows and matrix")
+    runs = c_int(0)
+    f = _fn("gemm_bf16", "br_gemm_bf16_leave_runs", [_P, _P, c_int, c_int, c_int, c_size_t, _P, c_size_t, c_int, _P, _P])
+    rc = f(_ptr(a), _ptr(w), M, N, K, a.stride(0) if M > 1 else K, _ptr(scratch), scratch.numel() * 4, wl, ctypes.byref(runs), _stream())
+    if rc == 1:
+        return 0
+    _check(rc, "gemm_leave_runs")
+    return runs.value
 
 
 def gemm_norm_scaled(xg: torch.Tensor, ssq: torch.Tensor, tiles: int, eps: float, w: torch.Tensor, out: torch.Tensor,

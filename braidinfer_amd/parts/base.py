@@ -123,6 +123,10 @@ class Norm(Part):
         return False
 
 
+    def rows_of_prepared(self, prepared: Any) -> Optional[torch.Tensor]:
+        """The normed rows themselves where `prepare_in_product` left them, else None."""
+        return None
+
     def runs_of_prepared(self, prepared: Any, w: torch.Tensor, n_out: int, ws) -> Optional["ProductRuns"]:
         """norm(x) @ w^T from what `prepare_in_product` left, as the float sums of its runs
         along k (see `ProductRuns`); None with nothing done if the product is not cut so."""
@@ -167,6 +171,8 @@ class NormedInput:
         self._tensor: Optional[torch.Tensor] = None
 
     def tensor(self) -> torch.Tensor:
+        if self._tensor is None and self.prepared is not None:
+            self._tensor = self.norm.rows_of_prepared(self.prepared)
         if self._tensor is None:
             self._tensor = self.ws.get("block_h", tuple(self.x.shape), self.dtype)
             self.norm.forward(self.x, self._tensor)

@@ -65,6 +65,17 @@ class RMSNorm(Norm):
 
     def prepare_in_product(self, a, w, x, ws):
         M, N = x.shape
+        if 64 < M <= 1024:
+            # more rows: the kernel that adds the product's runs along k norms the rows too, where there is one
+            if not (a.dtype == w.dtype == torch.bfloat16 and x.dtype == torch.float32 and N == self.size and x.is_contiguous()):
+                return None
+            h = ws.get("norm_rows", (M, N), torch.bfloat16)
+            scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32)
+            runs = K.gemm_leave_runs(a, w, N, scratch)
+            if not runs:
+                return None
+            K.rmsnorm(x, self.weight, h, self.eps, add=(scratch, runs))
+            return "rows", h
         if not (a.dtype == w.dtype == torch.bfloat16 and x.dtype == torch.float32 and N == self.size
                 and N % (16 if M <= 16 else 256) == 0 and K.gemm_stream_takes(M, a.shape[1])
                 and K.gemm_stream_takes(M, N) and a.is_contiguous() and x.is_contiguous()):
@@ -78,7 +89,12 @@ class RMSNorm(Norm):
         tiles = K.gemm_norm_prepare(a, w, x, self.weight, xg, ssq, scratch)
         return xg, ssq, tiles, scratch
 
+    def rows_of_prepared(self, prepared):
+        return prepared[1] if isinstance(prepared[0], str) and prepared[0] == "rows" else None
+
     def product_of_prepared(self, prepared, w, out, swiglu=False):
+        if self.rows_of_prepared(prepared) is not None:      # an ordinary product of `NormedInput.tensor`
+            return False
         xg, ssq, tiles, scratch = prepared
         if w.dtype != torch.bfloat16 or (not swiglu and out.dtype not in (torch.bfloat16, torch.float32)):
             return False
@@ -86,6 +102,8 @@ class RMSNorm(Norm):
         return True
 
     def runs_of_prepared(self, prepared, w, n_out, ws):
+        if self.rows_of_prepared(prepared) is not None:
+            return None
         xg, ssq, tiles, scratch = prepared
         if w.dtype != torch.bfloat16 or scratch is None:
             return None
