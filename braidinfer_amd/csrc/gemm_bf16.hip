@@ -2544,15 +2544,21 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
 // 500 / 279 against 445 / 231 (1.19 and 0.91 PFLOP/s), 8,000 tokens 1,892 / 1,208 against 1,626 / 955.  Before, the rows
 // copied into the experts' order, tiles of 128x128 through registers and the unit in a launch of its own: 234 / 122, 522 /
 // 267, 782 / 387, 1,074 / 543; 8,000 tokens expert by expert 2,365 / 1,115.
-static bool experts_tall_tiles(int pairs, int E, int N, int cus) {
+// The down product (`gated` false) has a short k and writes float rows: from four rounds of 128-row tiles on the taller tile gains more there than
+// the k-tiles say.  The same experts, down in us with 128 rows a tile against 256, scores drawn evenly and unevenly: 1,000 tokens 188 / 191
+// against 173 / 173, 1,400 tokens 220 / 246 against 211 / 204, 2,400 tokens 362 / 388 against 317 / 312; 16 experts of 1,408 by 2,048, 4 chosen,
+// 5,000 tokens 148 / 148 against 133 / 131; with fewer rounds: 600 tokens 33 / 31 against 43 / 42, 2,400 tokens 74 / 73 against 83 / 82.
+static bool experts_tall_tiles(int pairs, int E, int N, bool gated, int cus) {
     const double mean = (double)pairs / E, high = mean + 0.5 * sqrt(mean);
     double t[2];
+    bool many = false;
     for (int i = 0; i < 2; ++i) {
         const int bm = i ? 256 : 128, k = i ? 0 : 1;
         const double units = E * ceil(high / bm) * ((N + 255) / 256), whole = floor(units / cus), share = units / cus - whole;
+        if (i == 0) many = units >= 4.0 * cus;
         t[i] = whole * QUAD_FULL[k] + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) * QUAD_FULL[k] : 0.0);
     }
-    return t[1] <= 1.03 * t[0];
+    return t[1] <= (!gated && many ? 1.2 : 1.03) * t[0];
 }
 
 extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, const int* order, void* C, int gated, int out_is_bf16,
@@ -2566,7 +2572,7 @@ extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, 
     const int mode = gated ? OUT_SWIGLU : out_is_bf16 ? OUT_BF16 : OUT_F32;
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    if (experts_tall_tiles(pairs, E, N, cus))
+    if (experts_tall_tiles(pairs, E, N, gated != 0, cus))
         return launch_experts_tiles<256, 256, 2, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
     return launch_experts_tiles<128, 256, 3, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
 }
