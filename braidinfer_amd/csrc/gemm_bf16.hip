@@ -1553,17 +1553,25 @@ struct StreamNorm {
     float* ssq;            // producer writes, consumer reads: [tiles, SSQ_LD]
     int ssq_tiles;         // consumer: tiles of the producer
     float inv_k, eps;      // consumer: 1 / width of the normed rows, the norm's eps
-    // branches: weight rows b per .. + per multiply the activations b a_step elements on; output columns from gap_at on lie
-    // `gap` further on
+};
+// Branches: weight rows b per .. + per multiply the activations b a_step elements on; output columns from gap_at on lie `gap`
+// further on.  (A type of its own, so that the arguments of the other forms stay as short as they are.)
+struct StreamBranches {
     int per;
     size_t a_step;
     int gap_at, gap;
 };
+template <int NORM> struct StreamArg { typedef StreamNorm type; };
+template <> struct StreamArg<3> { typedef StreamBranches type; };
+__device__ __forceinline__ size_t branch_rows(const StreamNorm&, int) { return 0; }
+__device__ __forceinline__ size_t branch_rows(const StreamBranches& b, int n) { return (size_t)(n / b.per) * b.a_step; }
+__device__ __forceinline__ int branch_gap(const StreamNorm&, int) { return 0; }
+__device__ __forceinline__ int branch_gap(const StreamBranches& b, int n) { return n >= b.gap_at ? b.gap : 0; }
 
 template <int RT, int XR, int KC, int S, int NW, int MODE, int NORM>
 __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C, int M, int N, int K, size_t lda,
-                                                              size_t ldc, int ntiles, StreamNorm nrm, int wl) {
+                                                              size_t ldc, int ntiles, typename StreamArg<NORM>::type nrm, int wl) {
     static_assert(NORM == 0 || (NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC) || (NORM == 3 && MODE == OUT_F32), "norm forms");
     constexpr int STEPS = KC / 32;
     constexpr int ROWB = KC * 2;
@@ -1603,8 +1611,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
     int buf = 0;
 
     // NORM 3: where the activations of the tile to ask for lie behind the first branch's
-#define BRANCH_OFF(T) ((size_t)((((int)blockIdx.x + (T) * (int)gridDim.x) * RT) / nrm.per) * nrm.a_step)
-    size_t a_off = NORM == 3 ? BRANCH_OFF(0) : 0;
+    size_t a_off = branch_rows(nrm, (int)blockIdx.x * RT);
 #define ISSUE(J)                                                                                         \
     do {                                                                                                 \
         int chunk_ = wave + is_c * NW + rot;                                                             \
@@ -1632,7 +1639,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
         if (++is_c == ncw) {                                                                             \
             is_c = 0;                                                                                    \
             ++is_t;                                                                                      \
-            if (NORM == 3) a_off = BRANCH_OFF(is_t);                                                     \
+            if (NORM == 3) a_off = branch_rows(nrm, ((int)blockIdx.x + is_t * (int)gridDim.x) * RT);     \
         }                                                                                                \
     } while (0)
 
@@ -1679,7 +1686,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                     const int n0 = ((int)blockIdx.x + cp_t * (int)gridDim.x) * RT;
                     ++cp_t;
                     float* rb = red + buf * (NW * 16 * 17);
-                    if (NORM == 2 && cp_t == 1) {
+                    if constexpr (NORM == 2) if (cp_t == 1) {
                         const int m = tid >> 5, l = tid & 31;
                         float t = 0.f;
 #pragma unroll
@@ -1697,7 +1704,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
-                    if (MODE == OUT_SWIGLU) {
+                    if constexpr (MODE == OUT_SWIGLU) {
                         for (int e = tid; e < 8 * 16; e += NW * 64) {
                             const int m = e >> 3, jl = e & 7;
                             if (m < M && n0 + jl + 8 < N) {
@@ -1708,7 +1715,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                                 ((bf16*)C)[(size_t)m * ldc + n0 / 2 + jl] = (bf16)silu_mul(gv, uv);
                             }
                         }
-                    } else if (NORM == 1) {
+                    } else if constexpr (NORM == 1) {
                         // whole waves (16 lanes a row): the row's 16 squares of this tile are added by shuffles
                         if (tid < 16 * XR) {
                             const int m = tid >> 4, nl = tid & 15, n = n0 + nl;
@@ -1736,7 +1743,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
 #pragma unroll
                                 for (int w = 0; w < NW; ++w) v += rb[(w * 16 + nl) * 17 + m];
                                 if (NORM == 2) v *= rstd[m];
-                                const size_t idx = (size_t)m * ldc + n + (NORM == 3 && n0 >= nrm.gap_at ? nrm.gap : 0);
+                                const size_t idx = (size_t)m * ldc + n + branch_gap(nrm, n0);
                                 if (MODE == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
                                 else if (MODE == OUT_F32) ((float*)C)[idx] = v;
                                 // one add per element and product, without a read that this wave would
@@ -1751,7 +1758,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
         }
     }
 #undef ISSUE
-#undef BRANCH_OFF
 }
 
 
@@ -1760,7 +1766,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
 #define STREAM_NW 8
 template <int XR, int NORM>
 static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc,
-                         int mode, hipStream_t s, StreamNorm nrm = StreamNorm{}, int wl = 0) {
+                         int mode, hipStream_t s, typename StreamArg<NORM>::type nrm = typename StreamArg<NORM>::type{}, int wl = 0) {
     constexpr int RT = 16, KC = STREAM_KC, S = 2, NW = STREAM_NW;
     static_assert(KC == 128, "the blocked weight layout has 128 k a block");
     const int cus = br_device_cus();
@@ -1819,7 +1825,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                                                                void* __restrict__ C, int M, int N, int K, size_t lda,
                                                                size_t ldc, int mode, int partial, int scale,
                                                                int ntiles, int parts, int cpp, size_t part_stride,
-                                                               StreamNorm nrm, int wl) {
+                                                               typename StreamArg<BRANCHES ? 3 : 0>::type nrm, int wl) {
     constexpr int S = WIDE_S, D = S - 1, NW = 8, H = 16 * HB;
     constexpr int ROWS = H + 16 * MB;                // stacked rows of a stage: weights, then activations
     constexpr int STAGE = ROWS * 256;
@@ -1891,7 +1897,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                 int m_ = row_ - H;                                                                            \
                 if (m_ > M - 1) m_ = M - 1;                                                                   \
                 gp_ = A + (size_t)m_ * lda + (size_t)(c0_ + rot_) * 128;                                      \
-                if (BRANCHES) gp_ += (size_t)(tile_ * H / nrm.per) * nrm.a_step;                              \
+                gp_ += branch_rows(nrm, tile_ * H);                                                           \
             }                                                                                                 \
             src[q_] = gp_ + (((lane & 15) ^ (row_ & 7)) * 8);                                                 \
         }                                                                                                     \
@@ -1918,7 +1924,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
     if (my_units > 0) WIDE_SETUP();
     for (int j = 0; j < D; ++j)
         if (is_u < my_units) WIDE_ISSUE();
-    if (scale) {
+    if constexpr (!BRANCHES) if (scale) {
         // row m = tid / 8: its 8 lanes take the tiles' sums in turn, then a butterfly; read at the first unit's end
         const int m = tid >> 3, l = tid & 7;
         float t = 0.f;
@@ -2035,7 +2041,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                 if (m < M && n < N) {
                     float v = red[nl * RLD + m];
                     if (scale) v *= rstd[m];
-                    const size_t idx = (size_t)m * ldc + n + (BRANCHES && n0 >= nrm.gap_at ? nrm.gap : 0);
+                    const size_t idx = (size_t)m * ldc + n + branch_gap(nrm, n0);
                     if (partial) ((float*)C)[part * part_stride + (size_t)m * N + n] = v;
                     else if (mode == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
                     else if (mode == OUT_F32) ((float*)C)[idx] = v;
@@ -2403,7 +2409,7 @@ extern "C" int br_gemm_bf16_norm_scaled(const void* XG, const void* W, void* C, 
 // second launch for the sums of its runs along k: four of 4,096 by 4,096, weights in no cache,
 // 6 rows 34.4 -> 25.6 us, 24 rows 58.6 -> 25.9, 64 rows 60.0 -> 30.7; four of 2,048 by 2,048 20.4 -> 10.6, 39.0 -> 14.1, 46.0 -> 17.4.
 template <int MB, int HB>
-static int launch_branches_wide(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const StreamNorm& br, int cus,
+static int launch_branches_wide(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const StreamBranches& br, int cus,
                                 hipStream_t s) {
     auto kern = gemm_stream_wide_kernel<MB, HB, true>;
     constexpr size_t lds = (size_t)WIDE_S * (16 * HB + 16 * MB) * 256 + 64 * 4;
@@ -2429,11 +2435,7 @@ extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, i
         return BR_BAD_ARG;
     const int N = branches * per, cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    StreamNorm br{};
-    br.per = per;
-    br.a_step = a_step;
-    br.gap_at = gap_at;
-    br.gap = gap;
+    const StreamBranches br = {per, a_step, gap_at, gap};
     if (M <= 8) return launch_stream<8, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
     if (M <= 16) return launch_stream<16, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
     // units of 64 rows, or of 128 where these fill the chip's rounds better (a unit's chunk costs its rows and 16 more, as in wide_shape)
