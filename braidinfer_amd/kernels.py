@@ -1538,9 +1538,6 @@ def experts_up_grouped(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor,
     _req(experts_grouped_takes(h.dtype, W, F2 // 2) and w_gu.dtype == y.dtype == torch.bfloat16, "experts_up_grouped: bfloat16, widths in steps of 8")
     _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
          and first.dtype == order.dtype == torch.int32, "experts_up_grouped: shapes")
-    if _experts_wide_pays(F2 // 2, W, n, E):
-        experts_wide(h, w_gu, first, order, y, top, limit, alpha)
-        return
     f = _fn("routed_experts", "br_experts_up_grouped", [_P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P])
     _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), E, W, F2 // 2, top, T, float(limit), float(alpha),
              int(_experts_stream_pays(T, n, E)), _stream()), "experts_up_grouped")
@@ -1553,9 +1550,6 @@ def experts_down_grouped(y: torch.Tensor, w_down: torch.Tensor, first: torch.Ten
     E, W, _ = w_down.shape
     _req(experts_grouped_takes(y.dtype, W, F) and w_down.dtype == torch.bfloat16 and out.dtype == torch.float32, "experts_down_grouped: types")
     _req(w_down.shape == (E, W, F) and out.shape == (n, W) and first.numel() in (E + 1, E + 2) and first.dtype == torch.int32, "experts_down_grouped: shapes")
-    if _experts_wide_pays(W, F, n, E):
-        experts_wide(y, w_down, first, None, out)
-        return
     f = _fn("routed_experts", "br_experts_down_grouped", [_P, _P, _P, _P] + [c_int] * 6 + [_P])
     _check(f(_ptr(y), _ptr(w_down), _ptr(first), _ptr(out), n, E, W, F, int(n_tokens), int(_experts_stream_pays(n_tokens, n, E)), _stream()),
            "experts_down_grouped")
@@ -1577,14 +1571,16 @@ def _experts_gemm_tiles_take(N: int, Kd: int) -> bool:
     return Kd % 64 == 0 and N % 16 == 0 and (max(N, 240) + 16) * Kd * 2 < 2 ** 32
 
 
-def _experts_wide_pays(N: int, Kd: int, pairs: int, experts: int) -> bool:
-    """Whether the experts' weights are streamed by all waves of a workgroup together (`experts_wide`): from five and a half pairs an
-    expert on average, where a wave's own ring of 16 pairs begins to read rows twice, to 24, beyond which experts that are chosen
-    more often than others have more than a group of 64 pairs and the prompt products' tiles are faster (160 tokens, 8 of 32
-    experts: 271 us against 268 with evenly drawn scores, 338 against 284 with uneven ones); and sizes that the kernel takes.
-    csrc/experts_wide.hip has the times around the first line."""
-    return 11 * experts < 2 * pairs <= 48 * experts and bool(
-        _fn("experts_wide", "br_experts_wide_takes", [c_int] * 4)(experts, N, Kd, pairs))
+def experts_wide_pays(a: torch.Tensor, w: torch.Tensor, pairs: int) -> bool:
+    """Whether a product of `pairs` pairs with the experts' matrices w [E, N, K] goes to `experts_wide`, which streams the weights
+    by all waves of a workgroup together: from five and a half pairs an expert on average, where a wave's own ring of 16 pairs begins to
+    read rows twice, to 24, beyond which experts that are chosen more often than others have more than a group of 64 pairs and
+    the prompt products' tiles are faster (160 tokens, 8 of 32 experts: 271 us against 268 with evenly drawn scores, 338 against 284
+    with uneven ones); and types, sizes and addresses (multiples of 16 bytes) that the kernel takes.  csrc/experts_wide.hip has the
+    times around the first line."""
+    E, N, Kd = w.shape
+    return (11 * E < 2 * pairs <= 48 * E and a.dtype == w.dtype == torch.bfloat16 and a.data_ptr() % 16 == w.data_ptr() % 16 == 0
+            and bool(_fn("experts_wide", "br_experts_wide_takes", [c_int] * 4)(E, N, Kd, pairs)))
 
 
 def experts_wide(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, order: Optional[torch.Tensor], out: torch.Tensor, top: int = 1,
@@ -1622,9 +1618,6 @@ def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, o
          "experts_up_tiles: bfloat16, widths in steps of 64, rows below 4 GB")
     _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
          and first.dtype == order.dtype == torch.int32, "experts_up_tiles: shapes")
-    if _experts_wide_pays(F2 // 2, W, n, E):
-        experts_wide(h, w_gu, first, order, y, top, limit, alpha)
-        return
     f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
     _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), 1, 1, T, n, E, F2, W, top, float(limit), float(alpha), _stream()),
            "experts_up_tiles")
@@ -1638,9 +1631,6 @@ def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: tor
     E, N, _ = w.shape
     _req(a.dtype == w.dtype == torch.bfloat16 and Kd % 8 == 0 and w.shape == (E, N, Kd) and out.shape == (n, N)
          and first.dtype == torch.int32 and first.numel() in (E + 1, E + 2), "experts_gemm: bfloat16 [pairs, K] x [E, N, K], K in steps of 8")
-    if out.dtype == torch.float32 and a.data_ptr() % 16 == w.data_ptr() % 16 == 0 and _experts_wide_pays(N, Kd, n, E):
-        experts_wide(a, w, first, None, out)
-        return
     if _experts_gemm_tiles_take(N, Kd) and out.data_ptr() % 16 == 0:
         f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
         _check(f(_ptr(a), _ptr(w), _ptr(first), None, _ptr(out), 0, _is_bf16(out, "experts_gemm"), n, n, E, N, Kd, 1, 0.0, 0.0, _stream()),

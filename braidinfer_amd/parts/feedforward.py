@@ -290,26 +290,31 @@ class RoutedExperts(FeedForward):
         # (a recorded step of single tokens is padded with sequences of no slot: their rows go to no expert)
         K.experts_sort(chosen, first, order, place, bins, slots=getattr(step, "slots", None) if step.is_decode else None, route=route)
         one_by_one = os.environ.get("BRAIDINFER_EXPERTS_ONE_BY_ONE", "")
-        # Up to eight pairs an expert on average, or sixteen tokens, the weights are streamed once for up to 16 pairs at a time;
-        # beyond, the prompt products' tiles read them once for 128 or 256.  Both products in us, streams against tiles: 32 experts of
+        # Three kernels read the experts' weights; `experts_wide_pays` says where all waves of a workgroup stream them together, product
+        # by product.  Outside its range, up to eight pairs an expert on average, or sixteen tokens, each wave streams them for up to 16 pairs
+        # at a time; beyond, the prompt products' tiles read them once for 128 or 256.  Both products in us, streams against tiles: 32 experts of
         # 1,792 by 4,096, 8 chosen: 32 tokens 239 / 257, 40 tokens 257 / 256, 64 tokens 350 / 259; 7 chosen: 32 tokens 251 / 254, 48
         # tokens 262 / 255, 64 tokens 323 / 257.  16 experts of 1,408 by 2,048, 4 chosen: 16 tokens 54 / 74, 32 tokens 58 / 74, 48
         # tokens 61 / 73, 64 tokens 81 / 74; 3 chosen: 48 tokens 56 / 71, 64 tokens 63 / 71, 96 tokens 91 / 72 (there the streams
         # stay ahead up to twelve pairs an expert).
         streamed = (T <= 16 or n <= 8 * self.E) and (few or K.experts_stream_takes(dt, self.H, self.I, n, self.E))
-        if K.experts_tiles_take(dt, self.H, self.I, T) and not streamed and one_by_one != "1":
+        tiles = K.experts_tiles_take(dt, self.H, self.I, T) and not streamed and one_by_one != "1"
+        if tiles or few or (streamed and one_by_one != "1"):
+            # an expert's weights are read once or twice for its pairs, nothing goes back to the host
             y = step.ws.get("moe_y", (n, self.I), dt)
-            K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
+            if K.experts_wide_pays(h, self.w_gu, n):
+                K.experts_wide(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
+            elif tiles:
+                K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
+            else:
+                K.experts_up_grouped(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             out = step.ws.get("moe_out", (n, self.H), torch.float32)
-            K.experts_gemm(y, self.w_down, first, out)
-            K.experts_combine(out, place, share, x, store=store, **ident)
-            return
-        if few or (streamed and one_by_one != "1"):
-            # an expert's weights are read once for its pairs, nothing goes back to the host
-            y = step.ws.get("moe_y", (n, self.I), dt)
-            K.experts_up_grouped(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
-            out = step.ws.get("moe_out", (n, self.H), torch.float32)
-            K.experts_down_grouped(y, self.w_down, first, out, T)
+            if K.experts_wide_pays(y, self.w_down, n):
+                K.experts_wide(y, self.w_down, first, None, out)
+            elif tiles:
+                K.experts_gemm(y, self.w_down, first, out)
+            else:
+                K.experts_down_grouped(y, self.w_down, first, out, T)
             K.experts_combine(out, place, share, x, store=store, **ident)
             return
         # widths and steps that the tiles do not take, and the 32-bit path
@@ -321,7 +326,10 @@ class RoutedExperts(FeedForward):
         if K.experts_grouped_takes(dt, self.H, self.I) and one_by_one != "1" and (one_by_one == "0" or n // self.E < self.ONE_BY_ONE_FROM):
             K.experts_gemm(rows, self.w_gu, first, gu)
             self._glu(gu, act)
-            K.experts_gemm(act, self.w_down, first, out)
+            if K.experts_wide_pays(act, self.w_down, n):
+                K.experts_wide(act, self.w_down, first, None, out)
+            else:
+                K.experts_gemm(act, self.w_down, first, out)
         else:
             # expert by expert through the library's products, the experts' row counts read by the host
             starts = first.tolist()

@@ -83,6 +83,29 @@ def test_products_of_few_tokens(T, top, E, W, F, how, identity, alpha):
             assert float((got[t, s] - exact).abs().max()) < 2e-6 * float(exact.abs().max()) * (F / 1024) ** 0.5 + 1e-5 * float(exact.abs().mean())
 
 
+def test_rows_and_weights_off_16_bytes():
+    """Rows and matrices that start 8 bytes behind a multiple of 16, at ten pairs an expert: taken, with the products of aligned ones."""
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(5)
+    T, top, E, W, F = 20, 4, 8, 1024, 1152
+
+    def shifted(t):
+        room = torch.zeros(t.numel() + 4, dtype=t.dtype, device="cuda")
+        room[4:] = t.reshape(-1).cuda()
+        return room[4:].view(t.shape)
+    h, gu, dn = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5), bf(rng.standard_normal((E, W, F)) / F ** 0.5)
+    chosen = drawn(T, top, E, "drawn", 6)
+    first, order, place = sorted_pairs(chosen, E)
+    want_y, want = products(h, gu, dn, chosen, 0.0, 0.0)
+    for shift in ((shifted, torch.Tensor.cuda), (torch.Tensor.cuda, shifted)):
+        y, out = torch.zeros((T * top, F), dtype=torch.bfloat16, device="cuda"), torch.zeros((T * top, W), device="cuda")
+        K.experts_up_grouped(shift[0](h), shift[1](gu), first, order, y, top)
+        K.experts_down_grouped(shift[0](y), shift[1](dn), first, out, T)
+        got_y, got = y[place.long()].double().reshape(T, top, F), out[place.long()].double().reshape(T, top, W)
+        assert float((got_y - want_y).abs().max()) < 2 ** -8 * float(want_y.abs().max())           # one bfloat16 rounding, 2^-9
+        assert float((got - want).norm() / want.norm()) < 1e-3                                     # rows that y's rounding may send to a neighbour
+
+
 def test_a_tokens_experts_do_not_depend_on_its_batch():
     """The same rows alone and among others through the streamed products: the same bits."""
     from braidinfer_amd import kernels as K

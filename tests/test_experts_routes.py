@@ -22,12 +22,12 @@ def route(monkeypatch, tokens, decode=False, W=4096, F=1792, E=32, top=8, dtype=
     """The experts' launches of a step, in order."""
     called = []
     for name in ("route_topk", "experts_sort", "experts_up", "experts_down", "experts_up_grouped", "experts_down_grouped",
-                 "experts_up_tiles", "experts_gather", "experts_gemm", "experts_combine", "silu_mul", "gemm"):
+                 "experts_up_tiles", "experts_wide", "experts_gather", "experts_gemm", "experts_combine", "silu_mul", "gemm"):
         monkeypatch.setattr(K, name, lambda *a, _name=name, **k: called.append(_name))
     monkeypatch.setattr(feedforward, "linear", lambda *a, **k: None)
     part = feedforward.RoutedExperts(W, F, E, top)
     part.rt, part.n_scores = type("Runtime", (), {"dtype": dtype}), E
-    part.w_gu = part.w_down = [torch.empty(0)] * E
+    part.w_gu, part.w_down = (torch.empty(shape, dtype=dtype, device="meta") for shape in ((E, 2 * F, W), (E, W, F)))
     part.forward(torch.empty((tokens, W), dtype=dtype, device="meta"), torch.empty((tokens, W), device="meta"), Step(tokens, decode))
     return [n for n in called if n not in ("route_topk", "experts_sort", "experts_combine")]
 
@@ -53,13 +53,45 @@ def test_tiles_say_what_they_take(W, F):
 
 
 FEW, GATHERED = ["experts_up_grouped", "experts_down_grouped"], ["experts_gather", "experts_gemm", "silu_mul", "experts_gemm"]
+WIDE = ["experts_wide", "experts_wide"]
 
 
+# 22 tokens: five and a half pairs an expert, the last that the streams take; 96: 24, the last before the tiles
 @pytest.mark.parametrize("W,F,E,top", [(4096, 1792, 32, 8), (2048, 1408, 16, 4)])
 def test_few_pairs_and_many(monkeypatch, W, F, E, top):
-    for tokens, decode, want in ((1, True, FEW), (16, True, FEW), (32, True, FEW), (33, True, TILES), (200, True, TILES), (17, False, FEW),
-                                 (32, False, FEW), (33, False, TILES), (47, False, TILES), (48, False, TILES), (4000, False, TILES)):
+    for tokens, decode, want in ((1, True, FEW), (16, True, FEW), (22, True, FEW), (23, True, WIDE), (96, True, WIDE), (97, True, TILES), (200, True, TILES),
+                                 (17, False, FEW), (22, False, FEW), (23, False, WIDE), (47, False, WIDE), (48, False, WIDE), (96, False, WIDE),
+                                 (97, False, TILES), (4000, False, TILES)):
         assert route(monkeypatch, tokens, decode, W, F, E, top) == want, tokens
+
+
+def test_each_product_by_its_own_widths(monkeypatch):
+    """Widths of which one is no whole number of chunks of 128: that product stays with the streams, or with the tiles."""
+    assert route(monkeypatch, 23, True, 4096, 1800) == ["experts_wide", "experts_down_grouped"]
+    assert route(monkeypatch, 64, False, 4096, 1856) == ["experts_wide", "experts_gemm"]
+    assert route(monkeypatch, 64, False, 4160, 1792) == ["experts_up_tiles", "experts_wide"]
+    assert route(monkeypatch, 64, False, 4104, 1792) == ["experts_gather", "experts_gemm", "silu_mul", "experts_wide"]
+
+
+def test_rows_off_16_bytes(monkeypatch):
+    """Rows or weights that start between multiples of 16 bytes are not for `experts_wide`, and the wrappers of the kernels that take
+    them call these, whatever the number of pairs."""
+    E, F, W, T, top = 4, 256, 256, 8, 4
+    wide, called = torch.zeros(2 * E * F * W + 8, dtype=torch.bfloat16), []
+    monkeypatch.setattr(K, "_dev", lambda *a: None)
+    monkeypatch.setattr(K, "_stream", lambda: 0)
+    takes = K._fn("experts_wide", "br_experts_wide_takes", [K.c_int] * 4)
+    monkeypatch.setattr(K, "_fn", lambda module, name, types: takes if name == "br_experts_wide_takes" else lambda *a: called.append(name) or 0)
+    first, order = torch.zeros(E + 1, dtype=torch.int32), torch.zeros(T * top, dtype=torch.int32)
+    y, out = torch.zeros(T * top, F, dtype=torch.bfloat16), torch.zeros(T * top, W)
+    for off in (0, 4, 8):
+        gu, dn = wide[off:off + 2 * E * F * W].view(E, 2 * F, W), wide[off:off + E * F * W].view(E, W, F)
+        h = wide[off:off + T * W].view(T, W)
+        for a, w in ((h, gu), (h.clone(), gu), (h, gu.clone()), (y, dn)):
+            assert K.experts_wide_pays(a, w, T * top) == (a.data_ptr() % 16 == w.data_ptr() % 16 == 0)
+        K.experts_up_grouped(h, gu, first, order, y, top)
+        K.experts_down_grouped(y, dn, first, out, T)
+    assert called == 3 * ["br_experts_up_grouped", "br_experts_down_grouped"]
 
 
 def test_widths_that_the_tiles_do_not_take(monkeypatch):
