@@ -1592,8 +1592,9 @@ def experts_wide(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, order: O
     E, N, K = w.shape
     up = order is not None
     n = out.shape[0]
-    _req(a.dtype == w.dtype == torch.bfloat16 and out.dtype == (torch.bfloat16 if up else torch.float32), "experts_wide: dtypes")
-    _req(a.dim() == 2 and a.shape[1] == K and out.dim() == 2 and out.shape[1] * (2 if up else 1) == N and first.numel() >= E + 1, "experts_wide: shapes")
+    _req(a.dtype == w.dtype == torch.bfloat16 and out.dtype == (torch.bfloat16 if up else torch.float32)
+         and first.dtype == torch.int32 and (not up or order.dtype == torch.int32), "experts_wide: bfloat16 rows and matrices, int32 first and order")
+    _req(a.dim() == 2 and a.shape[1] == K and out.dim() == 2 and out.shape[1] * (2 if up else 1) == N and first.numel() in (E + 1, E + 2), "experts_wide: shapes")
     _req((order.numel() == n and a.shape[0] * top >= n) if up else a.shape[0] >= n, "experts_wide: rows")
     f = _fn("experts_wide", "br_experts_wide", [_P] * 5 + [c_int] * 6 + [c_float, c_float, _P])
     _check(f(_ptr(a), _ptr(w), _ptr(first), _ptr(order), _ptr(out), int(up), n, E, out.shape[1], K, int(top), float(limit), float(alpha),

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from braidinfer_amd import kernels as K
+from braidinfer_amd.errors import KernelError
 from braidinfer_amd.parts import feedforward
 
 
@@ -111,3 +112,25 @@ def test_the_forced_routes(monkeypatch):
     monkeypatch.setenv("BRAIDINFER_EXPERTS_ONE_BY_ONE", "0")
     assert route(monkeypatch, 300, False) == TILES
     assert route(monkeypatch, 100000, False, 96, 40, 8, 2) == GATHERED          # 25,000 pairs an expert, in one launch all the same
+
+
+def test_all_waves_together_refuse(monkeypatch):
+    """Arrays of other types or sizes than the kernel reads are an error before anything is launched."""
+    E, F, W, T, top = 3, 256, 384, 9, 2
+    called = []
+    monkeypatch.setattr(K, "_dev", lambda *a: None)
+    monkeypatch.setattr(K, "_stream", lambda: 0)
+    monkeypatch.setattr(K, "_fn", lambda module, name, types: lambda *a: called.append(name) or 0)
+    n = T * top
+    h, gu, dn = (torch.zeros(shape, dtype=torch.bfloat16) for shape in ((T, W), (E, 2 * F, W), (E, W, F)))
+    first, order = torch.zeros(E + 1, dtype=torch.int32), torch.zeros(n, dtype=torch.int32)
+    y, out = torch.zeros(n, F, dtype=torch.bfloat16), torch.zeros(n, W)
+    K.experts_wide(h, gu, first, order, y, top)
+    K.experts_wide(y, dn, first, None, out)
+    assert called == 2 * ["br_experts_wide"]
+    for args in ((h, gu, first.long(), order, y, top), (h, gu, first, order.long(), y, top), (y, dn, first.long(), None, out), (h, gu, first[:E], order, y, top),
+                 (h.float(), gu, first, order, y, top), (h, gu, first, order, y.float(), top), (y, dn, first, None, out.bfloat16()),
+                 (h[:4], gu, first, order, y, top), (y[:4], dn, first, None, out), (h, gu, first, order[:4], y, top), (h[:, :256], gu, first, order, y, top)):
+        with pytest.raises(KernelError):
+            K.experts_wide(*args)
+    assert len(called) == 2
