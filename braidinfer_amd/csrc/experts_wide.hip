@@ -12,66 +12,39 @@
 // matrices only, so a pair's output does not depend on what else is in the step.
 //   UP: a unit's rows are blocks of 8 gate rows and the up rows of the same channels, y[p, f] the gated unit, bfloat16;
 //   else rows of W_d, out[p, n] float.
-// 32 experts of 1,792 by 4,096, 8 of them chosen evenly, weights in no cache, both products in us, streams / these / the prompt products'
-// tiles: 16 tokens 225 / 230 / 260, 24 tokens 246 / 231 / 263, 40 tokens 266 / 242 / 259 (6.1 and 5.5 TB/s), 64 tokens 362 / 237 / 259,
-// 96 tokens 500 / 257 / 262.  16 experts of 1,408 by 2,048, 4 chosen: 16 tokens 59 / 59 / 70, 32 tokens 56 / 56 / 77, 64 tokens
-// 84 / 57 / 76, 100 tokens 115 / 62 / 82.  In a step of 40 sequences among other work: 193 + 87 by the tiles, 152 + 83 by these.  Bound
-// by the memory; the rest is each launch's start (routing tables, first chunks) and the barriers at a unit's end.
+// Groups of 32 pairs or of 64, by what the experts' real pairs cost: an expert with more than a group has its rows read again, and a chunk of
+// the larger group brings 32 activation rows more.  32 experts of 1,792 by 4,096, 8 chosen, weights in no cache, both products in us, by
+// groups of 32 / of 64 / as chosen (the prompt products' tiles), scores drawn evenly; with as much spread between the experts as between the
+// tokens: 23 tokens 228 / 239 / 229 (251); 219 / 233 / 218 (231).  40 tokens 232 / 239 / 232 (251); 226 / 242 / 228 (230).  64 tokens 238 / 248 / 239
+// (251); 285 / 261 / 264 (250).  16 experts of 1,408 by 2,048, 4 chosen, 64 tokens 58 / 64 / 59 (77); 80 / 66 / 67 (80).  Among a
+// step's other work the tiles take longer, 193 + 87 at 40 sequences, and these 152 + 83.  Bound by the memory (6.1 and 5.5 TB/s at 40 tokens); the
+// rest is each launch's start (routing tables, first chunks) and the barriers at a unit's end.
+// (Both groups in one launch, every expert by its own, was tried: the workgroup whose run of units crosses from one to the other
+// fills its ring twice, and all wait for it: 278 us at 64 uneven tokens, where one group for all takes 264.)
 #include "expert_units.h"
 
 #define RXW_S 3
 #define RXW_NW 8
 #define RXW_MAX_E 512
 #define RXW_MAX_PAIRS 2048
+#define RXW_MAX_XR 64              // pairs of the larger group
 
+// Units u0 .. u1, groups of 16 MB pairs.
 template <int MB, int HB, bool UP>
-__global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wt,
-                                                                   const int* __restrict__ first, const int* __restrict__ order,
-                                                                   void* __restrict__ C, int pairs, int E, int N, int K, int top,
-                                                                   float limit, float alpha) {
+__device__ __forceinline__ void experts_wide_walk(const bf16* __restrict__ A, const bf16* __restrict__ Wt, void* __restrict__ C, unsigned char* smem,
+                                                  const int* cum, const int* firstL, const int* tok, int u0, int u1, int E, int N, int K,
+                                                  int tiles, float limit, float alpha) {
     constexpr int S = RXW_S, D = S - 1, NW = RXW_NW, H = 16 * HB, XR = 16 * MB;
     constexpr int ROWS = H + XR, STAGE = ROWS * 256;          // stacked rows of a stage: weights, then activations
     constexpr int NLD = ROWS / 4, NDMA = (NLD + NW - 1) / NW; // wave-loads of 4 rows; of each wave (surplus ones repeat the last)
     constexpr int RLD = XR + 1, UROWS = UP ? H / 2 : H;       // output columns of a unit
     constexpr bool TWO = HB > 4;
-    static_assert(HB >= 4 && HB <= 8 && NDMA <= 63 && H * RLD * 4 <= STAGE, "stage");
-    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    int* firstL = (int*)(smem + S * STAGE);                   // [E + 2]
-    int* cum = firstL + E + 2;                                // [E + 1] units before expert e
-    int* tok = cum + E + 1;                                   // UP: [pairs] the token of a pair
+    static_assert(HB >= 4 && HB <= 8 && XR <= RXW_MAX_XR && NDMA <= 63 && H * RLD * 4 <= STAGE, "stage");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int rb = wave & 3, khalf = wave >> 2;
     const bool has1 = TWO && rb + 4 < HB;
-    const int tiles = (N + UROWS - 1) / UROWS;
-    for (int e = tid; e <= E; e += NW * 64) {
-        firstL[e] = first[e];
-        if (e == E) firstL[E + 1] = first[E];
-    }
-    if (UP)
-        for (int p = tid; p < pairs; p += NW * 64) tok[p] = order[p] / top;
-    __syncthreads();
-    if (tid < 64) {
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int mine = e < E ? (firstL[e + 1] - firstL[e] + XR - 1) / XR * tiles : 0;
-            int sum = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if (lane >= o) sum += v;
-            }
-            if (e < E) cum[e] = run + sum - mine;
-            run += __shfl(sum, 63, 64);
-        }
-        if (lane == 0) cum[E] = run;
-    }
-    __syncthreads();
-    const int total = __builtin_amdgcn_readfirstlane(cum[E]);
-    const int u0 = (int)((long long)total * blockIdx.x / gridDim.x), u1 = (int)((long long)total * (blockIdx.x + 1) / gridDim.x);
-    if (u0 >= u1) return;
     const int nch = K / 128, nitems = (u1 - u0) * nch;
     const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
 
@@ -225,6 +198,73 @@ __global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* _
     }
 }
 
+template <int HB, bool UP>
+__global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* __restrict__ A, const bf16* __restrict__ Wt,
+                                                                   const int* __restrict__ first, const int* __restrict__ order,
+                                                                   void* __restrict__ C, int pairs, int E, int N, int K, int top,
+                                                                   float limit, float alpha, int group) {
+    constexpr int NW = RXW_NW, H = 16 * HB, UROWS = UP ? H / 2 : H;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    int* firstL = (int*)(smem + RXW_S * (H + RXW_MAX_XR) * 256);      // [E + 2]
+    int* cum = firstL + E + 2;                                // [E + 1] units before expert e, then the group's pairs
+    int* tok = cum + E + 2;                                   // UP: [pairs] the token of a pair
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int tiles = (N + UROWS - 1) / UROWS;
+    for (int e = tid; e <= E; e += NW * 64) {
+        firstL[e] = first[e];
+        if (e == E) firstL[E + 1] = first[E];
+    }
+    if (UP)
+        for (int p = tid; p < pairs; p += NW * 64) tok[p] = order[p] / top;
+    __syncthreads();
+    if (tid < 64) {
+        int xr = group;
+        if (!xr) {
+            int groups = 0;                                   // of 32 pairs, and of 64 in the upper half
+            bool more = false;
+            for (int e = lane; e < E; e += 64) {
+                const int n = firstL[e + 1] - firstL[e];
+                groups += ((n + 31) >> 5) + (((n + 63) >> 6) << 16);
+                more |= n > 32;
+            }
+            xr = 32;
+            if (__ballot(more)) {
+                // rounds of units over the workgroups times what a unit's chunk costs, its rows and 24 more for the activations and the barrier,
+                // 48 with groups of 64 (seven sets of 8 to 128 experts, 6 to 16 pairs each, even and uneven: 0.1 % behind the better of the two
+                // on average, 9 % at most; by the number of units without rounds 2.5 and 33 %)
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) groups += __shfl_xor(groups, o, 64);
+                const int G = (int)gridDim.x;
+                if (((groups >> 16) * tiles + G - 1) / G * (H + 48) < ((groups & 0xffff) * tiles + G - 1) / G * (H + 24)) xr = 64;
+            }
+        }
+        int run = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            const int mine = e < E ? (firstL[e + 1] - firstL[e] + xr - 1) / xr * tiles : 0;
+            int sum = mine;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += v;
+            }
+            if (e < E) cum[e] = run + sum - mine;
+            run += __shfl(sum, 63, 64);
+        }
+        if (lane == 0) {
+            cum[E] = run;
+            cum[E + 1] = xr;
+        }
+    }
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(cum[E]);
+    const bool tall = __builtin_amdgcn_readfirstlane(cum[E + 1]) == 64;
+    const int u0 = (int)((long long)total * blockIdx.x / gridDim.x), u1 = (int)((long long)total * (blockIdx.x + 1) / gridDim.x);
+    if (u0 >= u1) return;
+    if (tall) experts_wide_walk<4, HB, UP>(A, Wt, C, smem, cum, firstL, tok, u0, u1, E, N, K, tiles, limit, alpha);
+    else experts_wide_walk<2, HB, UP>(A, Wt, C, smem, cum, firstL, tok, u0, u1, E, N, K, tiles, limit, alpha);
+}
+
 // Blocks of 16 weight rows of a unit (4 to 8): the least of rounds of units over the compute units (every expert one group of
 // pairs) times what a unit's chunk costs, its rows and a constant for the activations and the barrier.  By the matrices only.
 // Measured (32 pairs a group, us): gate/up of 32 experts of 1,792 by 4,096 (112 rows make four whole rounds) 148 at 112 rows,
@@ -242,19 +282,19 @@ static int rx_wide_height(int E, int N, bool up, int cus) {
     return best;
 }
 
-template <int MB, int HB, bool UP>
+template <int HB, bool UP>
 static int rx_launch_wide(const void* A, const void* Wt, const int* first, const int* order, void* C, int pairs, int E, int N, int K, int top,
-                          float limit, float alpha, int cus, hipStream_t s) {
-    constexpr size_t ring = (size_t)RXW_S * (16 * HB + 16 * MB) * 256, most = ring + (2 * RXW_MAX_E + 3) * 4 + RXW_MAX_PAIRS * 4;
+                          float limit, float alpha, int group, int cus, hipStream_t s) {
+    constexpr size_t ring = (size_t)RXW_S * (16 * HB + RXW_MAX_XR) * 256, most = ring + (2 * RXW_MAX_E + 4) * 4 + RXW_MAX_PAIRS * 4;
     static_assert(most <= 160 * 1024, "LDS");
-    auto kern = experts_wide_kernel<MB, HB, UP>;
+    auto kern = experts_wide_kernel<HB, UP>;
     static bool set = false;
     if (!set) {
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most) != hipSuccess) return BR_LAUNCH_FAILED;
         set = true;
     }
-    const size_t lds = ring + (size_t)(2 * E + 3) * 4 + (size_t)pairs * 4;
-    kern<<<cus, RXW_NW * 64, lds, s>>>((const bf16*)A, (const bf16*)Wt, first, order, C, pairs, E, N, K, top, limit, alpha);
+    const size_t lds = ring + (size_t)(2 * E + 4) * 4 + (size_t)pairs * 4;
+    kern<<<cus, RXW_NW * 64, lds, s>>>((const bf16*)A, (const bf16*)Wt, first, order, C, pairs, E, N, K, top, limit, alpha, group);
     return br_check_launch();
 }
 
@@ -264,25 +304,23 @@ extern "C" int br_experts_wide_takes(int E, int N, int K, int pairs) {
            ((long long)E + pairs / 32) * ((N + 31) / 32) * (K / 128) < (1ll << 31);
 }
 
+// The weight rows of a unit for these matrices on this device, 0 without one (tests ask).
+extern "C" int br_experts_wide_rows(int E, int N, int up) {
+    const int cus = br_device_cus();
+    return cus ? 16 * rx_wide_height(E, N, up != 0, cus) : 0;
+}
+
 // `up`: Wt [E][2 N][K], A the tokens' rows (through `order`), C bfloat16 [pairs, N]; else Wt [E][N][K], A the pairs' rows, C float
-// [pairs, N].  Groups of 32 pairs up to 16 an expert on average, of 64 beyond: few experts then have more than a group, whose rows
-// would be read again.  32 experts of 1,792 by 4,096, both products in us at groups of 32 / 64 (tiles), scores drawn evenly; with as
-// much spread between the experts as between the tokens: 32 tokens 236 / 244 (257); 180 / 188 (225).  64 tokens 237 / 250 (259);
-// 291 / 265 (259).  80 tokens 247 / 253 (259); 343 / 263 (251).  128 tokens 363 / 267 (268); 409 / 328 (257).  (A recorded
-// step's tokens count with its padding, 64 for 33 to 64 that go to experts: 16 an expert are about 12 there.)
+// [pairs, N].  `group`: 0 (the kernel finds by the experts' pairs what is faster), or groups of 32 or 64 pairs.
 extern "C" int br_experts_wide(const void* A, const void* Wt, const int* first, const int* order, void* C, int up, int pairs, int E,
-                               int N, int K, int top, float limit, float alpha, hipStream_t s) {
+                               int N, int K, int top, float limit, float alpha, int group, hipStream_t s) {
     if (pairs <= 0) return BR_OK;
-    if (!br_experts_wide_takes(E, N, K, pairs) || top <= 0 || (up && !order) || (((uintptr_t)A | (uintptr_t)Wt) & 15) != 0) return BR_BAD_ARG;
+    if (!br_experts_wide_takes(E, N, K, pairs) || top <= 0 || (up && !order) || (((uintptr_t)A | (uintptr_t)Wt) & 15) != 0 ||
+        (group != 0 && group != 32 && group != 64))
+        return BR_BAD_ARG;
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    const bool tall = pairs > 16 * E;
-#define RX_WIDE(HB_)                                                                                                           \
-    case HB_:                                                                                                                  \
-        if (up) return tall ? rx_launch_wide<4, HB_, true>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, cus, s)  \
-                            : rx_launch_wide<2, HB_, true>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, cus, s); \
-        return tall ? rx_launch_wide<4, HB_, false>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, cus, s)         \
-                    : rx_launch_wide<2, HB_, false>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, cus, s);
+#define RX_WIDE(HB_)                                                                                                                        case HB_:                                                                                                                                   return up ? rx_launch_wide<HB_, true>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, group, cus, s)                                   : rx_launch_wide<HB_, false>(A, Wt, first, order, C, pairs, E, N, K, top, limit, alpha, group, cus, s);
     switch (rx_wide_height(E, N, up != 0, cus)) {
         RX_WIDE(4)
         RX_WIDE(5)

@@ -1571,23 +1571,37 @@ def _experts_gemm_tiles_take(N: int, Kd: int) -> bool:
     return Kd % 64 == 0 and N % 16 == 0 and (max(N, 240) + 16) * Kd * 2 < 2 ** 32
 
 
-def experts_wide_pays(a: torch.Tensor, w: torch.Tensor, pairs: int) -> bool:
-    """Whether a product of `pairs` pairs with the experts' matrices w [E, N, K] goes to `experts_wide`, which streams the weights
-    by all waves of a workgroup together: from five and a half pairs an expert on average, where a wave's own ring of 16 pairs begins to
-    read rows twice, to 24, beyond which experts that are chosen more often than others have more than a group of 64 pairs and
-    the prompt products' tiles are faster (160 tokens, 8 of 32 experts: 271 us against 268 with evenly drawn scores, 338 against 284
-    with uneven ones); and types, sizes and addresses (multiples of 16 bytes) that the kernel takes.  csrc/experts_wide.hip has the
-    times around the first line."""
+def experts_wide_pays(a: torch.Tensor, w: torch.Tensor, tokens: int, pairs: int) -> bool:
+    """Whether a product of `tokens` tokens' `pairs` pairs with the experts' matrices w [E, N, K] goes to `experts_wide`, which streams the
+    weights by all waves of a workgroup together.  From five and a half pairs an expert on average and more than 16 tokens, where an expert
+    can have more than the 16 pairs of a wave's own ring, whose rows that ring reads again.  Up to 16 pairs an expert, beyond which
+    the prompt products' tiles are as fast: 22 where their tiles of 256 rows are not one to each of the 256 compute units, and 10
+    where these make three rounds or more.
+    Whole steps in us, without / with this kernel, scores drawn evenly, with half as much spread between the experts as between the tokens, and
+    with as much; two layers with 8 of 32 experts of 1,792 by 4,096 (448 and 512 tiles): a prompt of 23 tokens 832 / 784, 846 / 791, 791 / 768, of 64
+    tokens 936 / 853, 907 / 882, 888 / 884, of 80 tokens 959 / 942, 966 / 985, 964 / 990, of 112 996 / 1,014, 1,013 / 1,075, 996 / 1,082; 40
+    sequences 998 / 901, 990 / 934, 962 / 895, 64 sequences 1,071 / 1,027, 1,087 / 1,050, 1,075 / 1,041.  Both products alone, evenly and with as much
+    spread: 4 of 16 experts of 1,408 by 2,048 (176 and 128 tiles), 64 tokens 77 / 59, 80 / 67, 88 tokens 80 / 61, 80 / 73; 8 of 128 experts of
+    768 by 2,048 (768 and 1,024), gate/up and down apart, eight pairs an expert 156 / 136 and 83 / 77, 124 / 108 and 62 / 64, sixteen
+    158 / 148 and 87 / 88, 143 / 152 and 82 / 89.
+    And types, sizes and addresses (multiples of 16 bytes) that the kernel takes."""
     E, N, Kd = w.shape
-    return (11 * E < 2 * pairs <= 48 * E and a.dtype == w.dtype == torch.bfloat16 and a.data_ptr() % 16 == w.data_ptr() % 16 == 0
+    tiles = E * -(-N // 256)
+    most = 22 if tiles <= 256 else 16 if tiles < 768 else 10
+    return (tokens > 16 and 11 * E < 2 * pairs <= 2 * most * E and a.dtype == w.dtype == torch.bfloat16 and a.data_ptr() % 16 == w.data_ptr() % 16 == 0
             and bool(_fn("experts_wide", "br_experts_wide_takes", [c_int] * 4)(E, N, Kd, pairs)))
 
 
+def experts_wide_rows(E: int, N: int, up: bool) -> int:
+    """The weight rows of a unit of `experts_wide` for E experts' matrices of N output channels, on this device."""
+    return int(_fn("experts_wide", "br_experts_wide_rows", [c_int] * 3)(E, N, int(up)))
+
+
 def experts_wide(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, order: Optional[torch.Tensor], out: torch.Tensor, top: int = 1,
-                 limit: float = 0.0, alpha: float = 0.0) -> None:
+                 limit: float = 0.0, alpha: float = 0.0, group: int = 0) -> None:
     """Both products of routed experts for steps of some ten pairs an expert, every weight read once.  With `order`: y = the gated
     unit of h's rows (through order[p] / top) and w [E, 2 F, W], bfloat16 [pairs, F]; without: out = a @ w[e]^T for the pairs' rows
-    and w [E, W, F], float32 [pairs, W]."""
+    and w [E, W, F], float32 [pairs, W].  `group`: 32 or 64 pairs of an expert at a time (tests and measurements), 0 by the pairs."""
     _dev("experts_wide", a, w, first, order, out)
     E, N, K = w.shape
     up = order is not None
@@ -1596,9 +1610,9 @@ def experts_wide(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, order: O
          and first.dtype == torch.int32 and (not up or order.dtype == torch.int32), "experts_wide: bfloat16 rows and matrices, int32 first and order")
     _req(a.dim() == 2 and a.shape[1] == K and out.dim() == 2 and out.shape[1] * (2 if up else 1) == N and first.numel() in (E + 1, E + 2), "experts_wide: shapes")
     _req((order.numel() == n and a.shape[0] * top >= n) if up else a.shape[0] >= n, "experts_wide: rows")
-    f = _fn("experts_wide", "br_experts_wide", [_P] * 5 + [c_int] * 6 + [c_float, c_float, _P])
+    f = _fn("experts_wide", "br_experts_wide", [_P] * 5 + [c_int] * 6 + [c_float, c_float, c_int, _P])
     _check(f(_ptr(a), _ptr(w), _ptr(first), _ptr(order), _ptr(out), int(up), n, E, out.shape[1], K, int(top), float(limit), float(alpha),
-             _stream()), "experts_wide")
+             int(group), _stream()), "experts_wide")
 
 
 def experts_tiles_take(dtype: torch.dtype, W: int, F: int, tokens: int) -> bool:

@@ -302,14 +302,14 @@ class RoutedExperts(FeedForward):
         if tiles or few or (streamed and one_by_one != "1"):
             # an expert's weights are read once or twice for its pairs, nothing goes back to the host
             y = step.ws.get("moe_y", (n, self.I), dt)
-            if K.experts_wide_pays(h, self.w_gu, n):
+            if K.experts_wide_pays(h, self.w_gu, T, n):
                 K.experts_wide(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             elif tiles:
                 K.experts_up_tiles(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             else:
                 K.experts_up_grouped(h, self.w_gu, first, order, y, self.top, self.limit, self.alpha)
             out = step.ws.get("moe_out", (n, self.H), torch.float32)
-            if K.experts_wide_pays(y, self.w_down, n):
+            if K.experts_wide_pays(y, self.w_down, T, n):
                 K.experts_wide(y, self.w_down, first, None, out)
             elif tiles:
                 K.experts_gemm(y, self.w_down, first, out)
@@ -326,7 +326,7 @@ class RoutedExperts(FeedForward):
         if K.experts_grouped_takes(dt, self.H, self.I) and one_by_one != "1" and (one_by_one == "0" or n // self.E < self.ONE_BY_ONE_FROM):
             K.experts_gemm(rows, self.w_gu, first, gu)
             self._glu(gu, act)
-            if K.experts_wide_pays(act, self.w_down, n):
+            if K.experts_wide_pays(act, self.w_down, T, n):
                 K.experts_wide(act, self.w_down, first, None, out)
             else:
                 K.experts_gemm(act, self.w_down, first, out)

@@ -154,8 +154,8 @@ def test_products_of_many_tokens(T, top, E, W, F, how, identity, alpha):
             assert torch.all(out[int(first[E]):] == 7.0)
 
 
-# experts' pairs at 1, 31 to 33 (a group of 32 rows), 63 to 65 (of 64) and none; widths of 2 and 3 chunks of 128 and of no whole
-# number of any unit's rows; identities behind the experts
+# few experts with up to a group of 64 pairs and one more; widths of 2 and 3 chunks of 128 and of no whole number of any unit's rows;
+# identities behind the experts
 @pytest.mark.parametrize("T,top,E,W,F,how,identity,alpha", [
     (31, 1, 1, 256, 256, "one", 0, 0.0), (32, 2, 3, 384, 256, "one", 0, 0.0), (33, 1, 2, 256, 400, "drawn", 1, 1.702), (63, 1, 2, 400, 256, "one", 0, 0.0),
     (65, 2, 4, 512, 384, "one", 0, 0.0), (40, 8, 32, 640, 1152, "drawn", 0, 0.0), (100, 3, 9, 1024, 256, "drawn", 2, 1.702), (24, 8, 32, 1024, 888, "drawn", 0, 0.0)])
@@ -183,6 +183,58 @@ def test_products_by_all_waves_together(T, top, E, W, F, how, identity, alpha):
         assert float((got - want)[real].abs().max()) < F * 2 ** -24 * float(want_y.abs().max()) * float(w_down.abs().max())
         assert float((got - want)[real].norm() / want[real].norm()) < 1e-5
         assert torch.all(out[int(first[E]):] == 7.0)
+
+
+# every height of a unit, 64 to 128 weight rows, in both products (the rule on the matrices picks it, for 256 compute units); experts of
+# no pair, one, and around one and two groups of 32 and of 64; every height by groups of 32, of 64 and as the kernel chooses
+@pytest.mark.parametrize("W,F,up,down", [(640, 512, 64, 64), (1664, 896, 80, 80), (2048, 1024, 96, 96), (2432, 1280, 112, 112), (2816, 1408, 128, 128)])
+@pytest.mark.parametrize("few", [True, False])
+def test_heights_and_groups(W, F, up, down, few):
+    from braidinfer_amd import kernels as K
+    counts = [31, 32, 0, 33, 1, 31, 32, 33, 7, 0] if few else [63, 64, 65, 31, 32, 33, 0, 1, 128, 129]
+    E, T = len(counts), sum(counts)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (K.experts_wide_rows(E, F, True), K.experts_wide_rows(E, W, False)) == (up, down)
+    rng = np.random.default_rng(W + few)
+    h, w_gu = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5)
+    w_down = bf(rng.standard_normal((E, W, F)) / F ** 0.5)
+    chosen = torch.tensor(rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)).cuda().reshape(T, 1)
+    want_y, want = products(h, w_gu, w_down, chosen, 0.0, 0.0)
+    first, order, place = sorted_pairs(chosen, E)
+    rows = want_y.to(torch.bfloat16).reshape(T, F)[order.long()].contiguous()
+    hd, gu, dn = h.cuda(), w_gu.cuda(), w_down.cuda()
+    got = []
+    for group in (32, 64, 0):
+        y, out = torch.full((T, F), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((T, W), 7.0, device="cuda")
+        K.experts_wide(hd, gu, first, order, y, 1, group=group)
+        K.experts_wide(rows, dn, first, None, out, group=group)
+        got.append((y, out))
+        assert torch.equal(y, got[0][0]) and torch.equal(out, got[0][1])           # a pair's sums do not depend on its group
+    y, out = got[0][0][place.long()].double(), got[0][1][place.long()].double()
+    assert float((y - want_y[:, 0]).abs().max()) < 2 ** -8 * float(want_y.abs().max())                           # one bfloat16 rounding, 2^-9
+    # float sums of the same rows: F products in any order, each of at most the largest |row| x |weight|
+    assert float((out - want[:, 0]).abs().max()) < F * 2 ** -24 * float(want_y.abs().max()) * float(w_down.abs().max())
+    assert float((out - want[:, 0]).norm() / want.norm()) < 1e-6
+
+
+def test_a_tokens_experts_do_not_depend_on_its_batch_among_all_waves():
+    """The same rows in steps of other sizes, by groups of 32 and of 64: the same bits.  (By the streams and by these kernels a token's
+    outputs differ in the order of their sums: up to 16 tokens, or five and a half pairs an expert, they are the streams'.)"""
+    from braidinfer_amd import kernels as K
+    rng = np.random.default_rng(8)
+    T, top, E, W, F = 90, 4, 8, 512, 640
+    h, gu, dn = bf(rng.standard_normal((T, W))).cuda(), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5).cuda(), bf(rng.standard_normal((E, W, F))).cuda()
+    chosen = drawn(T, top, E, "drawn", 4)
+
+    def run(k):
+        first, order, place = sorted_pairs(chosen[:k].contiguous(), E)
+        y, out = torch.zeros((k * top, F), dtype=torch.bfloat16, device="cuda"), torch.zeros((k * top, W), device="cuda")
+        K.experts_wide(h[:k].contiguous(), gu, first, order, y, top)
+        K.experts_wide(y, dn, first, None, out)
+        return out[place.long()].reshape(k, top, W)
+    whole = run(T)
+    for k in (1, 17, 32, 33, 64):
+        assert torch.equal(run(k), whole[:k])
 
 
 @pytest.mark.parametrize("E,N,K_,pairs,takes", [(1, 1, 256, 1, True), (512, 64, 256, 2048, True), (513, 64, 256, 8, False), (4, 64, 128, 8, False),

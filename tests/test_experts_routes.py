@@ -57,13 +57,20 @@ FEW, GATHERED = ["experts_up_grouped", "experts_down_grouped"], ["experts_gather
 WIDE = ["experts_wide", "experts_wide"]
 
 
-# 22 tokens: five and a half pairs an expert, the last that the streams take; 96: 24, the last before the tiles
-@pytest.mark.parametrize("W,F,E,top", [(4096, 1792, 32, 8), (2048, 1408, 16, 4)])
-def test_few_pairs_and_many(monkeypatch, W, F, E, top):
-    for tokens, decode, want in ((1, True, FEW), (16, True, FEW), (22, True, FEW), (23, True, WIDE), (96, True, WIDE), (97, True, TILES), (200, True, TILES),
-                                 (17, False, FEW), (22, False, FEW), (23, False, WIDE), (47, False, WIDE), (48, False, WIDE), (96, False, WIDE),
-                                 (97, False, TILES), (4000, False, TILES)):
+# 22 tokens: five and a half pairs an expert, the last that the streams take; 64 and 88: 16 and 22, the last before the tiles
+@pytest.mark.parametrize("W,F,E,top,last", [(4096, 1792, 32, 8, 64), (2048, 1408, 16, 4, 88)])
+def test_few_pairs_and_many(monkeypatch, W, F, E, top, last):
+    for tokens, decode, want in ((1, True, FEW), (16, True, FEW), (22, True, FEW), (23, True, WIDE), (last, True, WIDE), (last + 1, True, TILES), (200, True, TILES),
+                                 (17, False, FEW), (22, False, FEW), (23, False, WIDE), (47, False, WIDE), (48, False, WIDE), (last, False, WIDE),
+                                 (last + 1, False, TILES), (4000, False, TILES)):
         assert route(monkeypatch, tokens, decode, W, F, E, top) == want, tokens
+
+
+def test_sixteen_tokens_stay_with_the_streams(monkeypatch):
+    """No expert has more than 16 of them, whatever their average."""
+    for decode in (True, False):
+        assert route(monkeypatch, 16, decode, E=8, top=4) == FEW and route(monkeypatch, 17, decode, E=8, top=4) == WIDE
+        assert route(monkeypatch, 16, decode, E=4, top=4) == FEW and route(monkeypatch, 23, decode, E=4, top=4) == TILES
 
 
 def test_each_product_by_its_own_widths(monkeypatch):
@@ -77,7 +84,7 @@ def test_each_product_by_its_own_widths(monkeypatch):
 def test_rows_off_16_bytes(monkeypatch):
     """Rows or weights that start between multiples of 16 bytes are not for `experts_wide`, and the wrappers of the kernels that take
     them call these, whatever the number of pairs."""
-    E, F, W, T, top = 4, 256, 256, 8, 4
+    E, F, W, T, top = 4, 256, 256, 20, 2
     wide, called = torch.zeros(2 * E * F * W + 8, dtype=torch.bfloat16), []
     monkeypatch.setattr(K, "_dev", lambda *a: None)
     monkeypatch.setattr(K, "_stream", lambda: 0)
@@ -89,7 +96,7 @@ def test_rows_off_16_bytes(monkeypatch):
         gu, dn = wide[off:off + 2 * E * F * W].view(E, 2 * F, W), wide[off:off + E * F * W].view(E, W, F)
         h = wide[off:off + T * W].view(T, W)
         for a, w in ((h, gu), (h.clone(), gu), (h, gu.clone()), (y, dn)):
-            assert K.experts_wide_pays(a, w, T * top) == (a.data_ptr() % 16 == w.data_ptr() % 16 == 0)
+            assert K.experts_wide_pays(a, w, T, T * top) == (a.data_ptr() % 16 == w.data_ptr() % 16 == 0)
         K.experts_up_grouped(h, gu, first, order, y, top)
         K.experts_down_grouped(y, dn, first, out, T)
     assert called == 3 * ["br_experts_up_grouped", "br_experts_down_grouped"]
@@ -134,3 +141,12 @@ def test_all_waves_together_refuse(monkeypatch):
         with pytest.raises(KernelError):
             K.experts_wide(*args)
     assert len(called) == 2
+
+
+def test_where_all_waves_together_end():
+    """By the tiles of 256 rows that the prompt products would have: up to one to a compute unit, up to three rounds of them, beyond."""
+    a = torch.empty(1, 256, dtype=torch.bfloat16, device="meta")
+    for E, N, most in ((16, 4096, 22), (16, 4097, 16), (32, 4096, 16), (64, 2816, 16), (64, 3072, 10), (128, 1536, 10)):
+        w = torch.empty(E, N, 256, dtype=torch.bfloat16, device="meta")
+        assert K.experts_wide_pays(a, w, 17, most * E) and not K.experts_wide_pays(a, w, 17, most * E + 1), (E, N)
+        assert K.experts_wide_pays(a, w, 17, 6 * E) and not K.experts_wide_pays(a, w, 16, 6 * E) and not K.experts_wide_pays(a, w, 17, 11 * E // 2)
