@@ -1233,12 +1233,25 @@ static int launch_narrow(const bf16* A, const bf16* W, void* C, int M, int N, in
     return br_check_launch();
 }
 
+// The longest K that the narrow kernel takes where scratch lets the kernels it stands for cut the product into runs along k (without, they
+// are at least 1.1 times as long at every K).  It brings all of K to each of its few workgroups, 2 us and 1.65 for every 1,000 of K (one block
+// of 16 weight rows), and the runs spread K over the chip.  Runs against it, us, 32 weight rows: 32 rows, K = 3,072 / 3,584 / 4,096 /
+// 8,192 / 14,336: 8.1 / 8.0 / 8.2 / 10.0 / 12.3 against 7.0 / 7.8 / 8.6 / 15.6 / 25.7; 64 rows, 4,096 / 5,120 / 8,192: 9.8 / 10.3 /
+// 11.9 against 8.8 / 10.5 / 15.7; 128 rows 12.8 / 13.8 / 15.9 and, at 7,168, 15.5 against 8.9 / 10.6 / 15.9 and 14.1, 1,000 rows 14.9 / 15.6 / 17.2 and 16.5 against
+// 9.0 / 10.7 / 16.0 and 14.2.
+// Above 1,024 rows (no caller here brings scratch then) it is ahead up to 3,072 rows of K = 3,072 (64 weight rows, 3,000 rows: 1.1 times, 5,000: 0.8).
+static int narrow_longest(int M, int N, int K, size_t room) {
+    if (room < (size_t)8 * M * N * sizeof(float) || (M > 64 && K % DMA_BK)) return 0x7fffffff;
+    return M <= 32 ? 3584 : M <= 64 ? 4608 : M <= 1024 ? 7168 : M <= 3072 ? 3072 : 0;
+}
+
 // How many blocks of 16 weight rows a workgroup takes (1, 2 or 4), or 0 where the tiles are as fast: rounds of workgroups
-// over the compute units times what a round takes, 7, 10.5 and 17.5 us with K = 4,096 and in proportion otherwise, against the 37
-// of the tiles' single round (measured, us; K = 4,096, 64 weight rows: 1,801 rows 17 / 13 / 20 by 1 / 2 / 4 blocks and 39 by the
+// over the compute units times what a round takes, 7, 10.5 and 17.5 us with K = 4,096 and nearly in proportion otherwise (one block: 2.4,
+// 5.4, 15.6 and 25.8 us at K = 256, 2,048, 8,192 and 14,336), against the 37 of the tiles' single round, which go with K in the same way
+// (9, 23, 71 and 121; measured, us; K = 4,096, 64 weight rows: 1,801 rows 17 / 13 / 20 by 1 / 2 / 4 blocks and 39 by the
 // tiles, 3,000 rows 23 / 23 / 20 and 39, 5,000 rows 37 / 34 / 37 and 39, 7,000 rows 51 / 44 / 37 and 40).
-static int narrow_blocks(int M, int N, int K, int mode, int cus) {
-    if (M <= 16 || N > 64 || K < 256 || mode == OUT_SWIGLU || cus <= 0) return 0;
+static int narrow_blocks(int M, int N, int K, int mode, int cus, size_t room) {
+    if (M <= 16 || N > 64 || K < 256 || mode == OUT_SWIGLU || cus <= 0 || K > narrow_longest(M, N, K, room)) return 0;
     static const double round_us[3] = {7.0, 10.5, 17.5};
     int best = 0;
     double least = 32.0;
@@ -2158,7 +2171,8 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
     return launch_split_sum(scratch, parts, C, M, N, ldc, mode, s);
 }
 
-// kernel: 0 = choose, 1 = tile 128x128 through registers (any shape), 2 = the same 256x128,
+// kernel: 0 = choose, 1 = tile 128x128 through registers (any shape; plus 16 b: the narrow kernel with b blocks of 16 weight rows a
+// workgroup, 1, 2 or 4, aligned rows), 2 = the same 256x128,
 // 3 = skinny (M <= 64), 4..6 = direct-to-LDS tiles 256x128, 128x256, 128x128 (K a multiple
 // of 64, aligned rows), 7 = stream (M <= 16, K a multiple of 128 and at least 1024, aligned
 // rows), 8 = stream wide (16 < M <= 64, K a multiple of 128), 9 = direct-to-LDS tile 64x128
@@ -2198,8 +2212,12 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     }
     const bool chosen = kernel == 0;
     if (chosen && wl == WL_ROWS && aligned) {
-        const int blocks = narrow_blocks(M, N, K, mode, br_device_cus());
+        const int blocks = narrow_blocks(M, N, K, mode, br_device_cus(), (scratch && (uintptr_t)scratch % 16 == 0) ? scratch_bytes : 0);
         if (blocks) return launch_narrow_blocks(blocks, A, W, C, M, N, K, lda, ldc, mode, s);
+    }
+    if (kernel == 1 && forced_parts) {
+        if (!aligned || wl != WL_ROWS || mode == OUT_SWIGLU || (forced_parts != 1 && forced_parts != 2 && forced_parts != 4)) return BR_BAD_ARG;
+        return launch_narrow_blocks(forced_parts, A, W, C, M, N, K, lda, ldc, mode, s);
     }
     if (kernel == 0)
         kernel = stream_ok ? 7
@@ -2321,14 +2339,20 @@ extern "C" int br_gemm_bf16(const void* A, const void* W, void* C, int M, int N,
     return br_gemm_bf16_ex(A, W, C, M, N, K, lda, ldc, mode, 0, nullptr, 0, WL_ROWS, s);
 }
 
-// What br_gemm_bf16_ex picks for a product of more than 64 rows with K in steps of 64, aligned rows and a
+// What br_gemm_bf16_ex picks for a product of more than 64 rows with K in steps of 64, aligned rows of the plain layout and a
 // contiguous, aligned output (tests and benchmarks ask): the kernel and its runs along k; and, where the product is
-// cut along its weight rows, `n1` > 0 rows by the 256x256 tile first and `kernel`, `parts` for the rest.
+// cut along its weight rows, `n1` > 0 rows by the 256x256 tile first and `kernel`, `parts` for the rest.  The narrow kernel is
+// kernel 1 with its blocks of 16 weight rows as `parts`.
 extern "C" int br_gemm_bf16_tile_choice(int M, int N, int K, int mode, size_t scratch_bytes, int* kernel, int* parts,
                                         int* n1) {
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
     *n1 = 0;
+    *parts = narrow_blocks(M, N, K, mode, cus, scratch_bytes);
+    if (*parts) {
+        *kernel = 1;
+        return BR_OK;
+    }
     if (M > 128 && quad_takes(nullptr, M, N, K, (size_t)K, (size_t)(mode == OUT_SWIGLU ? N / 2 : N))) {
         const double single = choose_quad(M, N, K, mode, cus, scratch_bytes, kernel, parts);
         int k2, p2;
@@ -2498,6 +2522,7 @@ extern "C" int br_gemm_bf16_wide_partial(const void* A, const void* W, int M, in
     if (M <= 16 || M > 64 || N <= 0 || !parts || (wl != WL_ROWS && wl != WL_BLOCKED)) return BR_BAD_ARG;
     if (!scratch || (uintptr_t)scratch % 16 || !wide_takes(A, W, M, K, lda)) return BR_BAD_ARG;
     if (ssq && (ssq_tiles <= 0 || norm_width <= 0)) return BR_BAD_ARG;
+    if (!ssq && wl == WL_ROWS && narrow_blocks(M, N, K, OUT_BF16, br_device_cus(), scratch_bytes)) return BR_BAD_ARG;
     StreamNorm nrm{};
     if (ssq) nrm = StreamNorm{nullptr, nullptr, 0, (float*)ssq, ssq_tiles, 1.f / (float)norm_width, eps};
     const int norm = ssq ? 2 : 0;
@@ -2511,6 +2536,7 @@ extern "C" int br_gemm_bf16_wide_partial(const void* A, const void* W, int M, in
 extern "C" int br_gemm_bf16_wide_parts(int M, int N, int K, int mode, size_t scratch_bytes) {
     const int cus = br_device_cus();
     if (!cus || M <= 16 || M > 64 || K % 128 || K < 256) return 0;
+    if (narrow_blocks(M, N, K, mode, cus, scratch_bytes)) return 1;
     int hb, parts;
     wide_shape(M, N, K, mode, cus, scratch_bytes, &hb, &parts);
     return parts;

@@ -432,7 +432,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     then accumulate, which is how a projection adds into the residual stream).
     Rows of `a` and `out` may be strided (a view of a wider buffer); w is contiguous.
     `kernel` forces one bf16 kernel (1, 2: 128x128 and 256x128 tiles staged through
-    registers, any shape; 3: skinny, M <= 64; 4, 5, 6: 256x128, 128x256 and 128x128 tiles
+    registers, any shape; 1 plus 16 b: the kernel for few weight rows, b = 1, 2 or 4 blocks of 16 to a workgroup; 3: skinny, M <= 64; 4, 5, 6: 256x128, 128x256 and 128x128 tiles
     loaded straight into LDS, K in steps of 64; 7: streaming by workgroups that stay, M <= 16
     and K in steps of 128 from 1024; 8: the same for 17 to 64 rows, K in steps of 128; 5 or 6 plus
     16 p: that tile with p runs along k, for measurements; 9: a 64x128 tile loaded straight into
@@ -532,7 +532,7 @@ def gemm_tile_choice(M: int, N: int, K: int, mode: int = 0, scratch_floats: int 
     """What a bf16 product of more than 64 rows runs on when its K is a multiple of 64 and its rows and output
     are aligned: (kernel, runs along k, n1).  n1 > 0: the first n1 weight rows go to the 256x256 tile of one
     wave per SIMD in whole rounds over the chip, the rest to `kernel`.  mode: 0 bf16 out, 1 float out,
-    2 float out added to, 3 SwiGLU."""
+    2 float out added to, 3 SwiGLU.  Kernel 1: the one for few weight rows, with its blocks of 16 in place of the runs."""
     f = _fn("gemm_bf16", "br_gemm_bf16_tile_choice", [c_int, c_int, c_int, c_int, c_size_t, _P, _P, _P])
     k, p, n1 = c_int(0), c_int(0), c_int(0)
     _check(f(M, N, K, mode, scratch_floats * 4, ctypes.byref(k), ctypes.byref(p), ctypes.byref(n1)), "gemm_tile_choice")
