@@ -66,8 +66,10 @@ class RMSNorm(Norm):
     def prepare_in_product(self, a, w, x, ws):
         M, N = x.shape
         if 64 < M <= 1024:
-            # more rows: the kernel that adds the product's runs along k norms the rows too, where there is one
-            if not (a.dtype == w.dtype == torch.bfloat16 and x.dtype == torch.float32 and N == self.size and x.is_contiguous()):
+            # more rows: the kernel that adds the product's runs along k norms the rows too, where there is one; it reads rows and
+            # weight 16 bytes at a time
+            if not (a.dtype == w.dtype == torch.bfloat16 and x.dtype == torch.float32 and N == self.size and x.is_contiguous()
+                    and x.data_ptr() % 16 == self.weight.data_ptr() % 16 == 0):
                 return None
             h = ws.get("norm_rows", (M, N), torch.bfloat16)
             scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32)
