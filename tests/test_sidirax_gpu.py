@@ -585,6 +585,35 @@ def test_whole_prompt_against_plain(folders, engines, name, dtype):
     close(run(engines(name, dtype), toks[:3], [1, 1, 1]), want[:3], dtype, "the first tokens one by one")
 
 
+def test_recurrent_layers_of_the_products_widths(tmp_path, monkeypatch):
+    """Widths that the launch for several inputs takes (1,024 channels, heads of 128 and 256 rows together): its four stacked matrices, the
+    gap it leaves for the decay's rows and, beyond 64 tokens, the products by each matrix's own rows, all against the plain
+    implementation; and the same steps by those products alone, which add in another order only."""
+    import braidinfer_amd as B
+    from braidinfer_amd import kernels as K
+    cfg = plain_cfg(model(1024, 128, [wkv(2, 64, 8, mlp=dense(64)), wkv(4, 64, 24)]))
+    w = P.random_weights(cfg, seed=31, gain=1.5)
+    P.write_folder(str(tmp_path), cfg, w)
+    eng = B.Engine.from_folder(str(tmp_path), dtype="bfloat16", max_tokens=1024, use_graphs=False)
+    mixers = [layer.mixer for layer in eng.model.layers]
+    assert all(m.w_four.shape == (4 * m.nh * m.d, 1024) for m in mixers)
+    stacked, called, real = [m.w_four for m in mixers], [], K.gemm_branches
+    monkeypatch.setattr(K, "gemm_branches", lambda *a, **k: (called.append(1), real(*a, **k))[1])
+    toks = tokens_of(cfg, 80, 12)
+    want = P.forward(cfg, w, toks)
+    for portions in ([1], [8], [17], [64], [65], [70, 1, 9]):
+        n, got = sum(portions), []
+        for four in (stacked, [None] * len(mixers)):
+            for m, f in zip(mixers, four):
+                m.w_four = f
+            called.clear()
+            got.append(run(eng, toks[:n], portions))
+            assert len(called) == (2 * sum(p <= 64 for p in portions) if four is stacked else 0), portions
+            close(got[-1], want[:n], "bfloat16", f"{portions}")
+        # what is left of float sums in another order once activations are rounded to bfloat16 (2^-9 of a value, over two layers)
+        assert np.abs(got[0] - got[1]).max() < 2e-2 * np.abs(got[1]).max(), portions
+
+
 def test_residual_rows_after_every_layer(folders, engines):
     import braidinfer_amd as B
     _, cfg, w = folders[("a", "float32")]
