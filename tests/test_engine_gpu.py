@@ -457,25 +457,50 @@ def test_serving_sizes_whole_then_one_by_one_then_batched(serving, dtype):
 
 
 def test_single_token_steps_launch_few_norm_kernels(serving, monkeypatch):
-    """bfloat16, steps of up to 64 rows, sizes the streaming products take: only the first
-    layer's first norm and the final norm run as kernels of their own; the others are prepared
-    by the product before them.  A longer prompt runs all five."""
+    """bfloat16, sizes the streaming products take: only the first layer's first norm and the final norm run as
+    kernels of their own.  In steps of up to 64 rows the others are prepared by the product before them; in longer ones (to
+    1,024 rows) the kernel that adds that product's runs along k norms the rows too."""
     from braidinfer_amd import kernels as K
     folder, cfg, w = serving
     eng = B.Engine.from_folder(folder, dtype="bfloat16", max_tokens=1024, use_graphs=False)
-    calls = []
+    alone, fused = [], []
     real = K.rmsnorm
-    monkeypatch.setattr(K, "rmsnorm", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    monkeypatch.setattr(K, "rmsnorm", lambda *a, **k: ((alone if k.get("add") is None else fused).append(1), real(*a, **k))[1])
     s = eng.alloc_slot()
     eng.step([StepEntry(s, tokens(cfg, 100, 1), [99])])
-    assert len(calls) == 2 * cfg["num_hidden_layers"] + 1
-    calls.clear()
-    eng.step([StepEntry(s, [5], [0])])
-    assert len(calls) == 2
-    calls.clear()
-    eng.step([StepEntry(s, tokens(cfg, 40, 2), [39])])
-    assert len(calls) == 2
+    assert (len(alone), len(fused)) == (2, 2 * cfg["num_hidden_layers"] - 1)
+    for toks, rows in (([5], [0]), (tokens(cfg, 40, 2), [39])):
+        alone.clear(), fused.clear()
+        eng.step([StepEntry(s, toks, rows)])
+        assert (len(alone), len(fused)) == (2, 0)
     eng.free_slot(s)
+
+
+@pytest.mark.parametrize("n", [65, 100, 128, 300, 800])
+def test_rows_normed_with_the_sum_of_runs_are_what_the_next_half_reads(serving, n, monkeypatch):
+    """The logits of every place and of the single tokens behind, with norms in the sum of a product's runs and with the sum and
+    the norm as two kernels: the same but for the order in which a row's squares are added."""
+    from braidinfer_amd.parts.norm import RMSNorm
+    folder, cfg, w = serving
+    toks, out = tokens(cfg, n + 2, 60 + n), []
+    real = RMSNorm.prepare_in_product
+    for two in (False, True):
+        kinds = []
+
+        def prepare(self, a, w_, x, ws):
+            got = None if two and x.shape[0] > 64 else real(self, a, w_, x, ws)
+            if x.shape[0] > 64:
+                kinds.append(got is not None and self.rows_of_prepared(got) is not None)
+            return got
+        monkeypatch.setattr(RMSNorm, "prepare_in_product", prepare)
+        eng = B.Engine.from_folder(folder, dtype="bfloat16", max_tokens=1024, use_graphs=False)
+        s = eng.alloc_slot()
+        parts = [eng.step([StepEntry(s, toks[:n], list(range(n)))])] + [eng.step([StepEntry(s, [t], [0])]) for t in toks[n:]]
+        out.append(torch.cat(parts).float().cpu().numpy())
+        assert kinds and (not any(kinds) if two else any(kinds))
+    ref = P.forward(cfg, w, toks)
+    close(out[0], ref, "bfloat16", f"{n} rows")
+    assert np.abs(out[0] - out[1]).max() <= CUT_TOL["bfloat16"] * np.abs(ref).max()
 
 
 @pytest.mark.parametrize("live", [17, 24, 48, 64])
