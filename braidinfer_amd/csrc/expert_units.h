@@ -11,6 +11,24 @@ __device__ __forceinline__ float rx_glu(float g, float u, float limit, float alp
     return g / (1.0f + expf(-g)) * u;
 }
 
+// By one wave: put(e, the sum of of(..) over the experts before e) for e < E; returns the sum over all.
+template <typename Of, typename Put>
+__device__ __forceinline__ int rx_sums_before(int E, int lane, Of of, Put put) {
+    int run = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane, mine = e < E ? of(e) : 0;
+        int sum = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(sum, o, 64);
+            if (lane >= o) sum += v;
+        }
+        if (e < E) put(e, run + sum - mine);
+        run += __shfl(sum, 63, 64);
+    }
+    return run;
+}
+
 // A unit is a run of output rows of one expert against up to XR of its pairs; the units are numbered expert by expert (experts
 // without pairs have none), rows by rows, and for the same rows group by group of pairs.  In LDS: firstL[e] the first pair of expert
 // e in the experts' order (firstL[E + 1] = firstL[E]), cum[e] the units before expert e; `tiles` runs of rows an expert.

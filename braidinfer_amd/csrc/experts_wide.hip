@@ -206,7 +206,7 @@ __global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* _
     constexpr int NW = RXW_NW, H = 16 * HB, UROWS = UP ? H / 2 : H;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     int* firstL = (int*)(smem + RXW_S * (H + RXW_MAX_XR) * 256);      // [E + 2]
-    int* cum = firstL + E + 2;                                // [E + 1] units before expert e, then the group's pairs
+    int* cum = firstL + E + 2;                                // [E + 1] units before expert e, then whether groups are of 64 pairs
     int* tok = cum + E + 2;                                   // UP: [pairs] the token of a pair
     const int tid = threadIdx.x, lane = tid & 63;
     const int tiles = (N + UROWS - 1) / UROWS;
@@ -218,47 +218,25 @@ __global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* _
         for (int p = tid; p < pairs; p += NW * 64) tok[p] = order[p] / top;
     __syncthreads();
     if (tid < 64) {
-        int xr = group;
-        if (!xr) {
-            int groups = 0;                                   // of 32 pairs, and of 64 in the upper half
-            bool more = false;
-            for (int e = lane; e < E; e += 64) {
-                const int n = firstL[e + 1] - firstL[e];
-                groups += ((n + 31) >> 5) + (((n + 63) >> 6) << 16);
-                more |= n > 32;
-            }
-            xr = 32;
-            if (__ballot(more)) {
-                // rounds of units over the workgroups times what a unit's chunk costs, its rows and 24 more for the activations and the barrier,
-                // 48 with groups of 64 (seven sets of 8 to 128 experts, 6 to 16 pairs each, even and uneven: 0.1 % behind the better of the two
-                // on average, 9 % at most; by the number of units without rounds 2.5 and 33 %)
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) groups += __shfl_xor(groups, o, 64);
-                const int G = (int)gridDim.x;
-                if (((groups >> 16) * tiles + G - 1) / G * (H + 48) < ((groups & 0xffff) * tiles + G - 1) / G * (H + 24)) xr = 64;
-            }
-        }
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int mine = e < E ? (firstL[e + 1] - firstL[e] + xr - 1) / xr * tiles : 0;
-            int sum = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if (lane >= o) sum += v;
-            }
-            if (e < E) cum[e] = run + sum - mine;
-            run += __shfl(sum, 63, 64);
-        }
+        // groups of 32 pairs before each expert, and groups of 64 in the upper half
+        const int groups = rx_sums_before(E, lane, [&](int e) {
+            const int n = firstL[e + 1] - firstL[e];
+            return ((n + 31) >> 5) + (((n + 63) >> 6) << 16);
+        }, [&](int e, int before) { cum[e] = before; });
+        // rounds of units over the workgroups times what a unit's chunk costs, its rows and 24 more for the activations and the barrier, 48
+        // with groups of 64 (seven sets of 8 to 128 experts, 6 to 16 pairs each, even and uneven: 0.1 % behind the better of the two on
+        // average, 9 % at most; by the number of units without rounds 2.5 and 33 %)
+        const int G = (int)gridDim.x, u32 = (groups & 0xffff) * tiles, u64 = (groups >> 16) * tiles;
+        const bool larger = group ? group == 64 : (u64 + G - 1) / G * (H + 48) < (u32 + G - 1) / G * (H + 24);
+        for (int e = lane; e < E; e += 64) cum[e] = (larger ? cum[e] >> 16 : cum[e] & 0xffff) * tiles;
         if (lane == 0) {
-            cum[E] = run;
-            cum[E + 1] = xr;
+            cum[E] = larger ? u64 : u32;
+            cum[E + 1] = larger;
         }
     }
     __syncthreads();
     const int total = __builtin_amdgcn_readfirstlane(cum[E]);
-    const bool tall = __builtin_amdgcn_readfirstlane(cum[E + 1]) == 64;
+    const bool tall = __builtin_amdgcn_readfirstlane(cum[E + 1]) != 0;
     const int u0 = (int)((long long)total * blockIdx.x / gridDim.x), u1 = (int)((long long)total * (blockIdx.x + 1) / gridDim.x);
     if (u0 >= u1) return;
     if (tall) experts_wide_walk<4, HB, UP>(A, Wt, C, smem, cum, firstL, tok, u0, u1, E, N, K, tiles, limit, alpha);

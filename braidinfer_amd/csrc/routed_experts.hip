@@ -442,7 +442,7 @@ extern "C" int br_experts_down(const void* y, const void* w_down, const int* cho
 // ------------------------------------------------------------ expert by expert -----
 // The (token, slot) pairs grouped by expert: first[e] .. first[e + 1] - 1 are the places of expert e's pairs in
 // `order` (pair numbers t * top + s), and place[pair] is where a pair went.  One workgroup: counts in LDS, a scan by
-// one thread, places handed out by counters.  Which of an expert's pairs comes first is left to the counters; a
+// one wave, places handed out by counters.  Which of an expert's pairs comes first is left to the counters; a
 // pair's output does not depend on its place.  Numbers from E - 1 on count as E - 1: with identity experts E is one more
 // than the experts with matrices, and the last bin holds the identities' pairs.  `slots` (null: all tokens count): the pairs of
 // tokens whose slot is negative, the padding of recorded steps, are left out (place -1, first[E] the pairs that count), so
@@ -457,18 +457,7 @@ __device__ __forceinline__ void sort_pairs(const int* chosen, const int* __restr
         if (!slots || slots[i / top] >= 0) atomicAdd(&cnt[min(chosen[i], E - 1)], 1);
     __syncthreads();
     if (threadIdx.x < 64) {
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + threadIdx.x, mine = e < E ? cnt[e] : 0;
-            int sum = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if ((int)threadIdx.x >= o) sum += v;
-            }
-            if (e < E) first[e] = cur[e] = run + sum - mine;
-            run += __shfl(sum, 63, 64);
-        }
+        const int run = rx_sums_before(E, threadIdx.x, [&](int e) { return cnt[e]; }, [&](int e, int before) { first[e] = cur[e] = before; });
         if (threadIdx.x == 0) first[E] = run;
     }
     __syncthreads();
@@ -819,19 +808,8 @@ __global__ __launch_bounds__(RXS_NW * 64) void experts_stream_kernel(const bf16*
     if (UP)
         for (int p = tid; p < firstL[E]; p += NW * 64) tok[p] = order[p] / top;
     if (tid < 64) {
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int mine = e < E ? (firstL[e + 1] - firstL[e] + XR - 1) / XR * tiles : 0;
-            int sum = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if (lane >= o) sum += v;
-            }
-            if (e < E) cum[e] = run + sum - mine;
-            run += __shfl(sum, 63, 64);
-        }
+        const int run = rx_sums_before(E, lane, [&](int e) { return (firstL[e + 1] - firstL[e] + XR - 1) / XR * tiles; },
+                                       [&](int e, int before) { cum[e] = before; });
         if (lane == 0) cum[E] = run;
     }
     __syncthreads();
