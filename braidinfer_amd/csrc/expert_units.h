@@ -19,12 +19,13 @@ __device__ __forceinline__ int rx_sums_before(int E, int lane, Of of, Put put) {
         const int e = e0 + lane, mine = e < E ? of(e) : 0;
         int sum = mine;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(sum, o, 64);
-            if (lane >= o) sum += v;
-        }
+        for (int o = 1; o < 64; o <<= 1)
+            if (o < E) {                                      // uniform
+                const int v = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += v;
+            }
         if (e < E) put(e, run + sum - mine);
-        run += __shfl(sum, 63, 64);
+        run += __shfl(sum, min(63, E - 1 - e0), 64);
     }
     return run;
 }

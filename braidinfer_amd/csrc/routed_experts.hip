@@ -23,10 +23,12 @@
 // One token's choice and shares by one wave, E scores at `scores`, results at `chosen` and `share` (`top` each).
 __device__ __forceinline__ void route_token(const float* __restrict__ scores, const float* __restrict__ bias, int* chosen, float* share,
                                             int E, int top, float out_scale, int lane) {
-    if (E <= 64) {
+    if (E <= 16 || (E <= 64 && top > 1 && E <= 12 * top)) {
         // Finite scores, a lane each: every expert counts those that go before it (a larger score, or the same and a lower number),
         // which is its slot if it is below `top`: E steps without a shuffle where rounds of wave-wide maxima take 12 shuffles a
-        // slot.  (8 of 32 experts, 8 tokens: 7.7 -> 4.7 us with the launch; the same bits.)
+        // slot.  (8 of 32 experts, 8 tokens: 7.7 -> 4.7 us with the launch; the same bits.  For one or two slots of more than 16 experts the
+        // rounds are the shorter way, sort included: 7,000 tokens, 1 of 32 experts 11.5 us against 12.7 by counting, 1 of 64 13.1 and 16.2, 2 of 64
+        // 19.2 and 21.5; 1 of 8 11.3 and 10.5.)
         const float z = lane < E ? scores[lane] + (bias ? bias[lane] : 0.f) : -INFINITY;
         if (!__ballot(lane < E && !(fabsf(z) < INFINITY))) {
             int before = 0;

@@ -314,7 +314,9 @@ def test_rows_beyond_4_gb():
                 assert float((out[lo:hi].double() - want).abs().max()) < 64 * 2 ** -24 * 50
 
 
-@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (8, 32, 8), (16, 64, 64), (13, 63, 5), (5, 65, 3), (16, 512, 8)])
+# slots by counting (up to 16 experts, or 12 a slot for two slots and more) and by rounds of maxima
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (8, 32, 8), (16, 64, 64), (13, 63, 5), (5, 65, 3), (16, 512, 8), (9, 16, 1), (9, 17, 1), (7, 64, 1), (8, 24, 2),
+                                     (8, 25, 2), (6, 48, 4), (6, 49, 4)])
 def test_choice_and_sort_in_one_launch(T, E, top):
     """The same choice, shares and runs as by two launches, with equal scores, scores that are not numbers and infinite ones among
     them; the choice of finite scores is that of a stable sort, the shares its softmax."""
