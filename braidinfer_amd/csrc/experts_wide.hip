@@ -226,8 +226,10 @@ __global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* _
         // rounds of units over the workgroups times what a unit's chunk costs, its rows and 24 more for the activations and the barrier, 48
         // with groups of 64 (seven sets of 8 to 128 experts, 6 to 16 pairs each, even and uneven: 0.1 % behind the better of the two on
         // average, 9 % at most; by the number of units without rounds 2.5 and 33 %)
-        const int G = (int)gridDim.x, u32 = (groups & 0xffff) * tiles, u64 = (groups >> 16) * tiles;
-        const bool larger = group ? group == 64 : (u64 + G - 1) / G * (H + 48) < (u32 + G - 1) / G * (H + 24);
+        const int u32 = (groups & 0xffff) * tiles, u64 = (groups >> 16) * tiles;
+        const float per = __builtin_amdgcn_rcpf((float)gridDim.x);
+        const bool larger = group ? group == 64
+                                  : ceilf((float)u64 * per - 1e-3f) * (float)(H + 48) < ceilf((float)u32 * per - 1e-3f) * (float)(H + 24);
         for (int e = lane; e < E; e += 64) cum[e] = (larger ? cum[e] >> 16 : cum[e] & 0xffff) * tiles;
         if (lane == 0) {
             cum[E] = larger ? u64 : u32;
@@ -237,7 +239,9 @@ __global__ __launch_bounds__(RXW_NW * 64) void experts_wide_kernel(const bf16* _
     __syncthreads();
     const int total = __builtin_amdgcn_readfirstlane(cum[E]);
     const bool tall = __builtin_amdgcn_readfirstlane(cum[E + 1]) != 0;
-    const int u0 = (int)((long long)total * blockIdx.x / gridDim.x), u1 = (int)((long long)total * (blockIdx.x + 1) / gridDim.x);
+    // total b / grid, in 32 bits (at most a few hundred workgroups)
+    const unsigned G = gridDim.x, each = (unsigned)total / G, over = (unsigned)total - each * G;
+    const int u0 = (int)(blockIdx.x * each + blockIdx.x * over / G), u1 = (int)((blockIdx.x + 1) * each + (blockIdx.x + 1) * over / G);
     if (u0 >= u1) return;
     if (tall) experts_wide_walk<4, HB, UP>(A, Wt, C, smem, cum, firstL, tok, u0, u1, E, N, K, tiles, limit, alpha);
     else experts_wide_walk<2, HB, UP>(A, Wt, C, smem, cum, firstL, tok, u0, u1, E, N, K, tiles, limit, alpha);
