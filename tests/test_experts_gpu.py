@@ -195,19 +195,18 @@ def test_heights_and_groups(W, F, up, down, few):
     E, T = len(counts), sum(counts)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert (K.experts_wide_rows(E, F, True), K.experts_wide_rows(E, W, False)) == (up, down)
-    rng = np.random.default_rng(W + few)
-    h, w_gu = bf(rng.standard_normal((T, W))), bf(rng.standard_normal((E, 2 * F, W)) / W ** 0.5)
-    w_down = bf(rng.standard_normal((E, W, F)) / F ** 0.5)
-    chosen = torch.tensor(rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)).cuda().reshape(T, 1)
+    g = torch.Generator(device="cuda").manual_seed(W + few)
+    h, w_gu, w_down = (torch.randn(shape, generator=g, device="cuda").div(shape[-1] ** 0.5 if len(shape) > 2 else 1.0).to(torch.bfloat16)
+                       for shape in ((T, W), (E, 2 * F, W), (E, W, F)))
+    chosen = torch.tensor(np.random.default_rng(W + few).permutation(np.repeat(np.arange(E), counts)).astype(np.int32)).cuda().reshape(T, 1)
     want_y, want = products(h, w_gu, w_down, chosen, 0.0, 0.0)
     first, order, place = sorted_pairs(chosen, E)
     rows = want_y.to(torch.bfloat16).reshape(T, F)[order.long()].contiguous()
-    hd, gu, dn = h.cuda(), w_gu.cuda(), w_down.cuda()
     got = []
     for group in (32, 64, 0):
         y, out = torch.full((T, F), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((T, W), 7.0, device="cuda")
-        K.experts_wide(hd, gu, first, order, y, 1, group=group)
-        K.experts_wide(rows, dn, first, None, out, group=group)
+        K.experts_wide(h, w_gu, first, order, y, 1, group=group)
+        K.experts_wide(rows, w_down, first, None, out, group=group)
         got.append((y, out))
         assert torch.equal(y, got[0][0]) and torch.equal(out, got[0][1])           # a pair's sums do not depend on its group
     y, out = got[0][0][place.long()].double(), got[0][1][place.long()].double()
