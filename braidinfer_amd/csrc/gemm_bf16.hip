@@ -6,6 +6,7 @@
 //  * gemm_stream: M <= 16 rows (decode): weight streaming by one resident workgroup per
 //    compute unit, weights and activations brought into per-wave LDS rings by direct
 //    global-to-LDS loads (described at the kernel).
+//  * gemm_stream_tile: up to 128 rows against few enough weight rows: a workgroup a tile of 16 to 32 of them over all of K.
 //  * gemm_tile: LDS-staged tiles for many rows (prompts): 4 waves, each a TM x TN grid of
 //    v_mfma_f32_32x32x16_bf16 blocks; global loads of the next k-tile are issued before the
 //    current one is multiplied and written to the other LDS buffer after it.
@@ -1815,6 +1816,336 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
     return br_check_launch();
 }
 
+// ------------------------------------------------------------- gemm_stream_tile ------
+// Few rows (up to 128) against few enough weight rows that a tile of 16, 24 or 32 of them for every workgroup covers the matrix in
+// one round: K in steps of 128, the whole of it in one workgroup, shared over its waves (wave w takes the 64-wide chunks w, w + NW,
+// ..), so that no sums of runs are written, read and added by another launch.  A wave brings its chunk of the tile's weights and the
+// same chunk of all activations (16 MB rows) into two LDS stages of its own by direct loads; what has landed goes to registers at
+// once and the stage is asked for again before the matrix instructions, so that two stages are in flight all but a few
+// cycles.  At the end the waves' sums meet in LDS and are added in wave order.
+//
+// Up to 16 rows the memory bounds it: what counts is that all compute units stream the same share (6,144 weight rows are 256 tiles of
+// 24, where gemm_stream's 384 tiles of 16 leave half of the workgroups with twice the work of the others).  With more rows it is the
+// compute unit's path from the L2, 62 to 70 GB/s here, which carries 16 MB activation rows for the tile's 16 to 32: gemm_stream_wide
+// shares them over more weight rows and pays with runs along k and their sum, and wins where K is long (see tile_pays).
+// us, weights in no cache, before -> now (before: gemm_stream up to 16 rows, gemm_stream_wide with the sum of its runs up to 64,
+// the eight-wave tiles with theirs beyond): 6,144 x 4,096 by 8 rows 12.7 -> 10.9; 4,096 x 4,096, 2,048 x 2,048, 8,192 x 4,096 by 24 rows
+// 14.3 -> 9.2, 9.5 -> 5.6, 18.7 -> 13.6, by 64 rows 14.9 -> 13.3, 11.6 -> 7.8, 19.9 -> 18.3, by 80 rows 22.4 -> 15.3, 11.5 -> 8.8, 28.1 -> 20.9.
+// Chunks of 128 in one stage took 0 to 10 % longer; rows of activations further apart than a power of two changed nothing.
+//
+// NORM 1, 2: as gemm_stream's forms (the tile's columns as sums of squares by 16); C, or the sums of squares, are asked for
+// before the first weights and used at the end.
+constexpr int tile_waves(int RT, int MB) { return 640 / (RT + 16 * MB) < 8 ? 640 / (RT + 16 * MB) : 8; }     // 160 KB of LDS
+#define TILE_KC 64
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ const bf16* uniform(const bf16* p) {
+    const unsigned long long a = (unsigned long long)p;
+    return (const bf16*)((unsigned long long)(unsigned)uniform((int)(unsigned)a) |
+                         (unsigned long long)(unsigned)uniform((int)(a >> 32)) << 32);
+}
+template <int RT, int MB, int NORM>
+__global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                                                   void* __restrict__ C, int M, int N, int K, size_t lda,
+                                                                                   size_t ldc, int mode, int vec, StreamNorm nrm, int wl) {
+    static_assert(NORM != 1 || RT % 16 == 0, "sums of squares by 16 columns");
+    constexpr int NW = tile_waves(RT, MB), RB = (RT + 15) / 16, ROWS = RT + 16 * MB, STAGE = ROWS * TILE_KC * 2, NL = STAGE / 1024;
+    constexpr int WL_LOADS = RT / 8;   // loads of 8 rows by 128 bytes: the weights', then the activations'
+    constexpr int GROUPS = RB * MB, PER = (GROUPS + NW - 1) / NW;        // blocks of 16 x 16 results; those of a wave
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = uniform((int)threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+    unsigned char* ring = smem + wave * (2 * STAGE);
+    const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)ring);
+    const int nch = K / TILE_KC, ncw = (nch - wave + NW - 1) / NW;
+    const int n0 = (int)blockIdx.x * RT;
+    // where in k the workgroup starts: see gemm_stream
+    const int rot = uniform((int)((((unsigned)blockIdx.x * 2654435761u) >> 8) % (unsigned)nch));
+
+    // blocks of results: block t = wave + i NW of this wave; lane (r16, g) holds row 16 j + r16, columns col .. col + 3
+    auto block_of = [&](int i) { return wave + i * NW; };
+    auto row_of = [&](int t) { return 16 * (t % MB) + r16; };
+    auto col_of = [&](int t) {          // -1: columns of another block (the last block of 24 weight rows begins at the eighth)
+        const int b = t / MB;
+        if (RT % 16 && b == RB - 1) return g < 2 ? -1 : n0 + RT - 16 + 4 * g;
+        return n0 + 16 * b + 4 * g;
+    };
+    // sums of squares: a lane a row, and where rows are few its wave's other lanes the next tiles; 32 loads or less for 256 tiles
+    constexpr int QR = MB == 1 ? 16 : MB == 2 ? 32 : 64, QT = 64 / QR, QN = 32 / QT;
+    const int q_row = lane % QR, q_tile = wave * QT + lane / QR;
+    f32x4 c_pre[PER], g_pre[PER];
+    float q_pre[QN];
+    if constexpr (NORM == 1) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int t = block_of(i), m = row_of(t), n = col_of(t);
+            c_pre[i] = g_pre[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (t >= GROUPS || m >= M || n >= N) continue;
+            if (vec) {
+                c_pre[i] = *(const f32x4*)((const float*)C + (size_t)m * ldc + n);
+                g_pre[i] = *(const f32x4*)(nrm.gain + n);
+            } else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    c_pre[i][e] = ((const float*)C)[(size_t)m * ldc + n + e];
+                    g_pre[i][e] = nrm.gain[n + e];
+                }
+        }
+    }
+    if constexpr (NORM == 2) {
+#pragma unroll
+        for (int i = 0; i < QN; ++i) {
+            const int t = q_tile + i * NW * QT;
+            q_pre[i] = t < nrm.ssq_tiles && q_row < M ? nrm.ssq[(size_t)t * SSQ_LD + q_row] : 0.f;
+        }
+    }
+
+    // A lane's 16 bytes of each load.  Rows beyond M or N are fetched from the last valid row and dropped at the store.
+    const bf16* src[NL];
+    const size_t w_k128 = wl ? WL_BLOCK_ELEMS : 128;                     // elements from 128 k of a weight row to the next
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int row = 8 * i + (lane >> 3), col = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+        if (i < WL_LOADS) {
+            const int n = n0 + row < N ? n0 + row : N - 1;
+            src[i] = W + w_row_base(n, K, wl) + col;
+        } else {
+            const int m = row - RT < M ? row - RT : M - 1;
+            src[i] = A + (size_t)m * lda + col;
+        }
+    }
+    int asked = 0;
+    auto ask = [&](int st) {
+        int c = wave + asked * NW + rot;
+        if (c >= nch) c -= nch;
+        const size_t w_at = (size_t)(c >> 1) * w_k128 + (c & 1) * TILE_KC, a_at = (size_t)c * TILE_KC;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const unsigned to = uniform((int)(ring_lds + st * STAGE + i * 1024));
+            if (i < WL_LOADS)          // weights pass once: non-temporal
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(to), "v"(src[i] + w_at) : "m0", "memory");
+            else
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(src[i] + a_at) : "m0", "memory");
+        }
+        ++asked;
+    };
+    f32x4 acc[2][RB][MB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int j = 0; j < MB; ++j) acc[0][b][j] = acc[1][b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (0 < ncw) ask(0);
+    if (1 < ncw) ask(1);
+    for (int base = 0; base < ncw; base += 2) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            if (base + st >= ncw) continue;
+            if (base + st + 1 < ncw) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const unsigned char* at = ring + st * STAGE;
+            bf16x8 wf[RB][2], xv[MB][2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int b = 0; b < RB; ++b) {
+                    const int row = (b == RB - 1 ? RT - 16 : 16 * b) + r16;
+                    wf[b][s] = *(const bf16x8*)(at + row * 128 + (((4 * s + g) ^ ((row >> 1) & 7)) * 16));
+                }
+#pragma unroll
+                for (int j = 0; j < MB; ++j) {
+                    const int row = RT + 16 * j + r16;
+                    xv[j][s] = *(const bf16x8*)(at + row * 128 + (((4 * s + g) ^ ((row >> 1) & 7)) * 16));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (base + st + 2 < ncw) ask(st);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int b = 0; b < RB; ++b)
+#pragma unroll
+                    for (int j = 0; j < MB; ++j) acc[s][b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][s], xv[j][s], acc[s][b][j], 0, 0, 0);
+        }
+    }
+    // the waves' sums meet where the stages were
+    f32x4* red = (f32x4*)smem;                         // [NW][GROUPS][64]
+    float* sq = (float*)(smem + NW * GROUPS * 1024);   // NORM 2: [NW][64]
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int j = 0; j < MB; ++j) red[(wave * GROUPS + b * MB + j) * 64 + lane] = acc[0][b][j] + acc[1][b][j];
+    if constexpr (NORM == 2) {
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < QN; ++i) t += q_pre[i];
+        if (q_row < M)
+            for (int c = q_tile + QN * NW * QT; c < nrm.ssq_tiles; c += NW * QT) t += nrm.ssq[(size_t)c * SSQ_LD + q_row];
+#pragma unroll
+        for (int o = QR; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+        sq[wave * 64 + lane] = t;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int t = block_of(i), m = row_of(t), n = col_of(t);
+        if (t >= GROUPS) break;
+        f32x4 v = red[t * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += red[(w * GROUPS + t) * 64 + lane];
+        if constexpr (NORM == 2) {
+            float q = sq[m];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) q += sq[w * 64 + m];
+            v *= rsqrtf(q * nrm.inv_k + nrm.eps);
+        }
+        if (mode == OUT_SWIGLU) {
+            // 16 weight rows are 8 gates, then the 8 up values of the same outputs
+            f32x4 up;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(v[e], 32, 64);
+            if (m < M && g < 2 && n < N) {
+                bf16x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (bf16)silu_mul(v[e], up[e]);
+                bf16* to = (bf16*)C + (size_t)m * ldc + (n0 + 16 * (t / MB)) / 2 + 4 * g;
+                if (vec) *(bf16x4*)to = o;
+                else
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) to[e] = o[e];
+            }
+            continue;
+        }
+        if constexpr (NORM == 1) {
+            // whole waves: a row's 16 squares of this block are added by shuffles
+            const f32x4 h = c_pre[i] + v;
+            float q = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q += h[e] * h[e];
+            q += __shfl_xor(q, 16, 64);
+            q += __shfl_xor(q, 32, 64);
+            if (m >= M) continue;
+            if (g == 0) nrm.ssq[(size_t)(n / 16) * SSQ_LD + m] = q;
+            float* to = (float*)C + (size_t)m * ldc + n;
+            bf16* xg = nrm.xg + (size_t)m * nrm.ldx + n;
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (bf16)(h[e] * g_pre[i][e]);
+            if (vec) {
+                *(f32x4*)to = h;
+                *(bf16x4*)xg = o;
+            } else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { to[e] = h[e]; xg[e] = o[e]; }
+            continue;
+        }
+        if (m >= M || n < 0 || n >= N) continue;
+        float* to = (float*)C + (size_t)m * ldc + n;
+        bf16* to16 = (bf16*)C + (size_t)m * ldc + n;
+        if (vec && mode != OUT_F32_ACC) {              // N in steps of 4: all four columns
+            if (mode == OUT_BF16) {
+                bf16x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
+                *(bf16x4*)to16 = o;
+            } else *(f32x4*)to = v;
+            continue;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (n + e >= N) break;
+            if (mode == OUT_BF16) to16[e] = (bf16)v[e];
+            else if (mode == OUT_F32) to[e] = v[e];
+            else unsafeAtomicAdd(to + e, v[e]);        // one add per element, no read to wait for
+        }
+    }
+}
+
+// rt: weight rows of a workgroup (16, 24, 32).  norm as NORM above; 1 and 2 up to 64 rows, 1 with N and rt in steps of 16.
+template <int RT, int MB, int NORM>
+static int launch_tile_form(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode, hipStream_t s,
+                            const StreamNorm& nrm, int wl) {
+    constexpr int lds = tile_waves(RT, MB) * 2 * (RT + 16 * MB) * TILE_KC * 2;
+    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+    auto kern = gemm_stream_tile_kernel<RT, MB, NORM>;
+    static bool set = false;
+    if (!set) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return BR_LAUNCH_FAILED;
+        set = true;
+    }
+    // rows that 16-byte stores (8 of bf16) can take
+    const bool half = mode == OUT_BF16 || mode == OUT_SWIGLU;
+    const int vec = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0 &&
+                    (NORM != 1 || (nrm.ldx % 4 == 0 && (uintptr_t)nrm.xg % 8 == 0 && (uintptr_t)nrm.gain % 16 == 0));
+    kern<<<(N + RT - 1) / RT, 64 * tile_waves(RT, MB), lds, s>>>(A, W, C, M, N, K, lda, ldc, mode, vec, nrm, wl);
+    return br_check_launch();
+}
+template <int MB>
+static int launch_tile_rows(int rt, int norm, const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode, hipStream_t s,
+                            const StreamNorm& nrm, int wl) {
+#define BR_TILE(RT_, NORM_) return launch_tile_form<RT_, MB, NORM_>(A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl)
+    if (norm == 0) {
+        if (rt == 16) BR_TILE(16, 0);
+        if (rt == 24) BR_TILE(24, 0);
+        if (rt == 32) BR_TILE(32, 0);
+    }
+    if constexpr (MB <= 4) {
+        if (norm == 1 && rt == 16) BR_TILE(16, 1);
+        if (norm == 1 && rt == 32) BR_TILE(32, 1);
+        if (norm == 2 && rt == 16) BR_TILE(16, 2);
+        if (norm == 2 && rt == 24) BR_TILE(24, 2);
+        if (norm == 2 && rt == 32) BR_TILE(32, 2);
+    }
+#undef BR_TILE
+    return BR_BAD_ARG;
+}
+#define TILE_MAX_ROWS 128
+static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode, hipStream_t s,
+                              const StreamNorm& nrm, int wl) {
+    if (rt == 24 && (mode == OUT_SWIGLU || norm == 1)) return BR_BAD_ARG;
+    switch ((M + 15) / 16) {
+        case 1: return launch_tile_rows<1>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 2: return launch_tile_rows<2>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 3: return launch_tile_rows<3>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 4: return launch_tile_rows<4>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 5: return launch_tile_rows<5>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 6: return launch_tile_rows<6>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 7: return launch_tile_rows<7>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+        case 8: return launch_tile_rows<8>(rt, norm, A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+    }
+    return BR_BAD_ARG;
+}
+// The weight rows of a workgroup (16, 24 or 32) where gemm_stream_tile is the faster kernel, else 0.
+// Up to 16 rows, K from 1,024 up to 8,191: where one workgroup a compute unit has the matrix (N up to 32 a unit), with
+// the fewest rows for the busiest unit, the same for every number of rows, so that a row's bits do not depend on the others'.  With longer K a
+// tile of 16 rows gains nothing over gemm_stream (14,336: 21.7 against 21.5 us), and beyond 32 rows a unit gemm_stream's loads go on across tiles.
+// More rows: by counts in microseconds, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at nine numbers of rows from 17
+// to 96, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's; gemm_stream_wide
+// with the sum of its runs (up to 64 rows); the eight-wave tiles with theirs (beyond; single rounds only, where the count is sound).
+// The line it draws gains 1.3 in the mean over these, and loses 5 % at most.  by16: whole blocks of 16 columns only (NORM 1).
+static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) {
+    if (M <= 0 || M > TILE_MAX_ROWS || K % 128 || K < (M <= 16 ? 1024 : 256) || cus <= 0) return 0;
+    if (M <= 16 && (K >= 8192 || N > 32 * cus)) return 0;
+    int best_rt = 0;
+    double best = 1e30;
+    for (int rt = 32; rt >= 16; rt -= 8) {
+        if (rt == 24 && (mode == OUT_SWIGLU || by16)) continue;
+        const int rounds = (N + rt * cus - 1) / (rt * cus);
+        const double t = M <= 16 ? (double)rounds * rt : 3.1 + rounds * (double)(rt + M) * K * 2.9e-5 + (double)N * K * 1.27e-7;
+        if (t < best * (1.0 - 1e-9)) { best = t; best_rt = rt; }
+    }
+    if (M <= 16) return best_rt;
+    const double mb = (double)N * K * 2e-7;                              // weights in 10 MB
+    const double other = M <= 64 ? 0.96 * (6.2 + 0.043 * M + 1.61 * mb + 1.6e-6 * M * N + 4.7e-6 * M * K - (mode == OUT_SWIGLU ? 2.4 : 0.0))
+                                 : 9.1 + 1.9 * mb + 0.125e-3 * K + 0.41e-3 * N + 0.027 * M;
+    if (M > 64 && N > best_rt * cus) return 0;
+    return best < other ? best_rt : 0;
+}
+
+// What launch_stream_tile needs of its operands beside aligned rows.
+static bool tile_takes(int M, int K, size_t lda) { return M > 0 && M <= TILE_MAX_ROWS && K % 128 == 0 && K >= 256 && lda >= (size_t)K; }
+
 // ------------------------------------------------------------- gemm_stream_wide ------
 // 16 < M <= 64, K in steps of 128: the same streaming by workgroups that stay, with the
 // activations shared.  A unit of work is a tile of 16 HB weight rows (64 to 128) over one run of
@@ -1849,6 +2180,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
     static_assert(HB >= 4 && HB <= 8 && (D - 1) * NDMA <= 63 && H * RLD * 4 <= STAGE, "stage");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     float* rstd = (float*)(smem + S * STAGE);        // scale: [64]
+    float* sq = rstd + 64;                           // scale: [NW][64], see below
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -1938,14 +2270,13 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
     for (int j = 0; j < D; ++j)
         if (is_u < my_units) WIDE_ISSUE();
     if constexpr (!BRANCHES) if (scale) {
-        // row m = tid / 8: its 8 lanes take the tiles' sums in turn, then a butterfly; read at the first unit's end
-        const int m = tid >> 3, l = tid & 7;
+        // wave w takes the tiles w, w + 8, .. of all rows, a lane a row; the eight sums are added at the first unit's end
         float t = 0.f;
-        if (m < M)
-            for (int c = l; c < nrm.ssq_tiles; c += 8) t += nrm.ssq[(size_t)c * SSQ_LD + m];
-#pragma unroll
-        for (int o = 4; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-        if (l == 0) rstd[m] = m < M ? rsqrtf(t * nrm.inv_k + nrm.eps) : 0.f;
+        if (lane < M) {
+#pragma unroll 8
+            for (int c = wave; c < nrm.ssq_tiles; c += NW) t += nrm.ssq[(size_t)c * SSQ_LD + lane];
+        }
+        sq[tid] = t;
     }
     if (my_units > 0) WIDE_RUN_LENGTH(0, cp_left);
     while (cp_u < my_units) {
@@ -2003,6 +2334,12 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
         const int n0 = (unit / parts) * H;
         if (++cp_u < my_units) WIDE_RUN_LENGTH(cp_u, cp_left);
         float* red = (float*)st;                 // [H][RLD]
+        if constexpr (!BRANCHES) if (scale && cp_u == 1 && tid < 64) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) t += sq[w * 64 + tid];
+            rstd[tid] = rsqrtf(t * nrm.inv_k + nrm.eps);
+        }
         __builtin_amdgcn_s_barrier();            // every wave has read its operands of the stage
         asm volatile("" ::: "memory");
         if (khalf == 1) {
@@ -2137,7 +2474,7 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
 #define BR_WIDE(HB_)                                                                                            \
     do {                                                                                                        \
         auto kern = gemm_stream_wide_kernel<MB, HB_>;                                                           \
-        constexpr size_t lds = (size_t)WIDE_S * (16 * HB_ + 16 * MB) * 256 + 64 * 4;                            \
+        constexpr size_t lds = (size_t)WIDE_S * (16 * HB_ + 16 * MB) * 256 + 9 * 64 * 4;                            \
         static_assert(lds <= 160 * 1024, "LDS of a compute unit");                                              \
         static bool set = false;                                                                                \
         if (!set) {                                                                                             \
@@ -2175,7 +2512,7 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
 // workgroup, 1, 2 or 4, aligned rows), 2 = the same 256x128,
 // 3 = skinny (M <= 64), 4..6 = direct-to-LDS tiles 256x128, 128x256, 128x128 (K a multiple
 // of 64, aligned rows), 7 = stream (M <= 16, K a multiple of 128 and at least 1024, aligned
-// rows), 8 = stream wide (16 < M <= 64, K a multiple of 128), 9 = direct-to-LDS tile 64x128
+// rows; plus 16 b: gemm_stream_tile, 8 (b + 1) weight rows a workgroup, M <= 128, K from 256), 8 = stream wide (16 < M <= 64, K a multiple of 128), 9 = direct-to-LDS tile 64x128
 // (M <= 64), 10 = direct-to-LDS tile 256x192, 11 = the same 256x256 (SwiGLU epilogue only), 12..15 = the tiles of
 // four waves, one to a SIMD: 256x256, 128x256, 256x192, 256x224 (K a multiple of 64, aligned rows, output rows in steps
 // of 16 bytes; plus 16 p: with p runs along k); tests force one.  (A 256x256 tile of 8 waves for every epilogue
@@ -2202,7 +2539,7 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     if (kernel >= 4 && kernel <= 6 && !dma_ok) return BR_BAD_ARG;
     const bool wide_ok = aligned && M > 16 && M <= 64 && K % 128 == 0 && K >= 256 &&
                          (!scratch || (uintptr_t)scratch % 16 == 0);
-    if ((kernel == 7 && !stream_ok) || (kernel == 8 && !wide_ok) || kernel > 15 || kernel < 0 || (kernel >= 10 && !dma_ok) ||
+    if ((kernel == 7 && (forced_parts ? !(aligned && tile_takes(M, K, lda)) : !stream_ok)) || (kernel == 8 && !wide_ok) || kernel > 15 || kernel < 0 || (kernel >= 10 && !dma_ok) ||
         (kernel == 11 && mode != OUT_SWIGLU) ||
         (kernel == 9 && (!dma_ok || M > 64)))
         return BR_BAD_ARG;
@@ -2214,6 +2551,12 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     if (chosen && wl == WL_ROWS && aligned) {
         const int blocks = narrow_blocks(M, N, K, mode, br_device_cus(), (scratch && (uintptr_t)scratch % 16 == 0) ? scratch_bytes : 0);
         if (blocks) return launch_narrow_blocks(blocks, A, W, C, M, N, K, lda, ldc, mode, s);
+    }
+    // Up to 16 and beyond 64 rows the tile kernel where it is the faster; in between only when asked for a product without runs
+    // (kernel 16): the sums of runs that br_gemm_bf16_wide_partial leaves are those of the product that is chosen without being asked.
+    if (chosen && aligned && tile_takes(M, K, lda) && (M <= 16 || M > 64 || forced_parts == 1)) {
+        const int rt = tile_rows(M, N, K, mode, br_device_cus());
+        if (rt) return launch_stream_tile(rt, 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     }
     if (kernel == 1 && forced_parts) {
         if (!aligned || wl != WL_ROWS || mode == OUT_SWIGLU || (forced_parts != 1 && forced_parts != 2 && forced_parts != 4)) return BR_BAD_ARG;
@@ -2230,6 +2573,9 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
                                                StreamNorm{}, fh, fp, wl)
                        : launch_stream_wide<4>(A, W, C, M, N, K, lda, ldc, mode, (float*)scratch, scratch_bytes, s, 0,
                                                StreamNorm{}, fh, fp, wl);
+    }
+    if (kernel == 7 && forced_parts) {                 // 7 + 16 b: a workgroup a tile of 8 (b + 1) weight rows, b = 1, 2, 3
+        return launch_stream_tile(8 * (forced_parts + 1), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     }
     if (kernel == 7) return M <= 8 ? launch_stream<8, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl)
                                    : launch_stream<16, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
@@ -2353,6 +2699,11 @@ extern "C" int br_gemm_bf16_tile_choice(int M, int N, int K, int mode, size_t sc
         *kernel = 1;
         return BR_OK;
     }
+    if (M > 64 && tile_takes(M, K, (size_t)K) && tile_rows(M, N, K, mode, cus)) {
+        *kernel = 7;
+        *parts = 1;
+        return BR_OK;
+    }
     if (M > 128 && quad_takes(nullptr, M, N, K, (size_t)K, (size_t)(mode == OUT_SWIGLU ? N / 2 : N))) {
         const double single = choose_quad(M, N, K, mode, cus, scratch_bytes, kernel, parts);
         int k2, p2;
@@ -2366,6 +2717,11 @@ extern "C" int br_gemm_bf16_tile_choice(int M, int N, int K, int mode, size_t sc
     }
     choose_tile(M, N, K, mode, cus, scratch_bytes, kernel, parts);
     return BR_OK;
+}
+
+// Whether a product of up to 128 aligned rows goes to gemm_stream_tile (17 to 64 rows: when asked for one without runs).
+extern "C" int br_gemm_bf16_whole_pays(int M, int N, int K, int by16) {
+    return tile_rows(M, N, K, OUT_BF16, br_device_cus(), by16 != 0) != 0;
 }
 
 static bool stream_takes(const void* A, const void* W, int M, int K, size_t lda) {
@@ -2384,10 +2740,17 @@ static bool wide_takes(const void* A, const void* W, int M, int K, size_t lda) {
 // needed).  Refuses (BR_BAD_ARG) anything else: the caller then runs the norm itself.
 extern "C" int br_gemm_bf16_norm_prepare(const void* A, const void* W, float* C, int M, int N, int K, size_t lda,
                                          size_t ldc, const float* gain, void* xg, size_t ldx, float* ssq,
-                                         int* ssq_tiles, void* scratch, size_t scratch_bytes, int wl, hipStream_t s) {
+                                         int* ssq_tiles, void* scratch, size_t scratch_bytes, int wl, int whole, hipStream_t s) {
     if (M <= 0 || N <= 0 || (wl != WL_ROWS && wl != WL_BLOCKED)) return BR_BAD_ARG;
     if (ldc < (size_t)N || ldx < (size_t)N || !gain || !xg || !ssq || !ssq_tiles) return BR_BAD_ARG;
     StreamNorm nrm{gain, (bf16*)xg, ldx, ssq, 0, 0.f, 0.f};
+    if (N % 16 == 0 && M <= 64 && (stream_takes(A, W, M, K, lda) || (whole && wide_takes(A, W, M, K, lda)))) {
+        const int rt = tile_rows(M, N, K, OUT_F32_ACC, br_device_cus(), true);
+        if (rt) {
+            *ssq_tiles = N / 16;
+            return launch_stream_tile(rt, 1, (const bf16*)A, (const bf16*)W, C, M, N, K, lda, ldc, OUT_F32_ACC, s, nrm, wl);
+        }
+    }
     if (stream_takes(A, W, M, K, lda) && N % 16 == 0) {
         *ssq_tiles = N / 16;
         return M <= 8 ? launch_stream<8, 1>((const bf16*)A, (const bf16*)W, C, M, N, K, lda, ldc, OUT_F32_ACC, s, nrm, wl)
@@ -2407,13 +2770,17 @@ extern "C" int br_gemm_bf16_norm_prepare(const void* A, const void* W, float* C,
 // the product of the normed rows.  mode: 0 bf16, 1 float, 3 SwiGLU.
 extern "C" int br_gemm_bf16_norm_scaled(const void* XG, const void* W, void* C, int M, int N, int K, size_t lda,
                                         size_t ldc, int mode, const float* ssq, int ssq_tiles, int norm_width,
-                                        float eps, void* scratch, size_t scratch_bytes, int wl, hipStream_t s) {
+                                        float eps, void* scratch, size_t scratch_bytes, int wl, int whole, hipStream_t s) {
     if (M <= 0 || N <= 0) return BR_OK;
     if (wl != WL_ROWS && wl != WL_BLOCKED) return BR_BAD_ARG;
     if (!ssq || ssq_tiles <= 0 || norm_width <= 0 || (mode != OUT_BF16 && mode != OUT_F32 && mode != OUT_SWIGLU))
         return BR_BAD_ARG;
     if (mode == OUT_SWIGLU ? (N % 16 != 0 || ldc < (size_t)N / 2) : ldc < (size_t)N) return BR_BAD_ARG;
     StreamNorm nrm{nullptr, nullptr, 0, (float*)ssq, ssq_tiles, 1.f / (float)norm_width, eps};
+    if (M <= 64 && (stream_takes(XG, W, M, K, lda) || (whole && wide_takes(XG, W, M, K, lda)))) {
+        const int rt = tile_rows(M, N, K, mode, br_device_cus());
+        if (rt) return launch_stream_tile(rt, 2, (const bf16*)XG, (const bf16*)W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
+    }
     if (stream_takes(XG, W, M, K, lda))
         return M <= 8 ? launch_stream<8, 2>((const bf16*)XG, (const bf16*)W, C, M, N, K, lda, ldc, mode, s, nrm, wl)
                       : launch_stream<16, 2>((const bf16*)XG, (const bf16*)W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
@@ -2473,9 +2840,9 @@ extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, i
 
 // The runs along k of A W^T (65 to 1,024 rows, a product meant to be added into float rows), left in `scratch` as [*runs][M][N] floats for
 // br_gemm_bf16_add_runs_norm, where br_gemm_bf16_ex would cut the product.  Refuses (BR_BAD_ARG, nothing launched) where it would not,
-// and more than 8,192 columns.
+// and more than 8,192 columns.  whole: a product that gemm_stream_tile takes is left, too, as one run.
 extern "C" int br_gemm_bf16_leave_runs(const void* A_, const void* W_, int M, int N, int K, size_t lda, void* scratch_, size_t scratch_bytes, int wl,
-                                       int* runs, hipStream_t s) {
+                                       int whole, int* runs, hipStream_t s) {
     const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
     float* scratch = (float*)scratch_;
     if (M <= 64 || M > 1024 || N <= 64 || N > 8192 || N % 4 || K <= 0 || K % DMA_BK || lda < (size_t)K || lda % 8 || !scratch || !runs ||
@@ -2483,6 +2850,12 @@ extern "C" int br_gemm_bf16_leave_runs(const void* A_, const void* W_, int M, in
         return BR_BAD_ARG;
     const int cus = br_device_cus(), mode = OUT_F32_ACC;
     if (!cus) return BR_LAUNCH_FAILED;
+    const int rt = tile_takes(M, K, lda) ? tile_rows(M, N, K, mode, cus) : 0;
+    if (rt) {
+        if (!whole || (size_t)M * N * sizeof(float) > scratch_bytes) return BR_BAD_ARG;
+        *runs = 1;
+        return launch_stream_tile(rt, 0, A, W, scratch, M, N, K, lda, N, OUT_F32, s, StreamNorm{}, wl);
+    }
     int kernel = 0, parts = 1, k2, p2;
     if (M > 128 && quad_takes(scratch, M, N, K, lda, N)) {
         const double single = choose_quad(M, N, K, mode, cus, scratch_bytes, &kernel, &parts);

@@ -424,7 +424,7 @@ def _weight_dims(name: str, w: torch.Tensor, n_out: int):
 
 
 def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool = False, kernel: int = 0,
-         scratch: Optional[torch.Tensor] = None) -> None:
+         scratch: Optional[torch.Tensor] = None, whole: bool = False) -> None:
     """out[M, N] (+)= a[M, K] @ w[N, K]^T.
 
     float32 a and w: the true 32-bit kernel (out float32).  bfloat16 a and w: the
@@ -441,7 +441,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     16 p for p runs along k); 0 chooses by shape.  A weight from `block_weight` is taken by kernels 4 to 15.
     `scratch` (float32, on the device): with it, a product of more than 16 rows with too
     few tiles to fill the chip is cut along k into runs that a second kernel sums in a fixed order
-    (float32: the same bits with and without).
+    (float32: the same bits with and without).  `whole`: 17 to 64 rows may also take the kernel that leaves no runs
+    (kernel 7 + 16 b, tiles of 8 (b + 1) weight rows) where it is the faster; without, their bits are those that
+    `gemm_wide_partial` leaves in runs.
     """
     name = "gemm"
     for t in (a, w, out):
@@ -472,7 +474,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             _req(scratch.is_cuda and scratch.dtype == torch.float32 and scratch.is_contiguous(), "gemm: scratch must be float32 on the device")
         f = _fn("gemm_bf16", "br_gemm_bf16_ex",
                 [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, c_int, _P, c_size_t, c_int, _P])
-        _check(f(_ptr(a), _ptr(w), _ptr(out), M, N, K, lda, ldc, mode, kernel, _ptr(scratch),
+        _check(f(_ptr(a), _ptr(w), _ptr(out), M, N, K, lda, ldc, mode, kernel or (16 if whole else 0), _ptr(scratch),
                  0 if scratch is None else scratch.numel() * 4, wl, _stream()), name)
     else:
         raise KernelError(f"gemm: a is {a.dtype} and w is {w.dtype}; both float32 or both bfloat16")
@@ -500,10 +502,10 @@ def gemm_branches(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gap_at: i
 
 
 def gemm_swiglu(a: torch.Tensor, w_gu: torch.Tensor, out: torch.Tensor, kernel: int = 0,
-                scratch: Optional[torch.Tensor] = None) -> None:
+                scratch: Optional[torch.Tensor] = None, whole: bool = False) -> None:
     """out[M, I] = silu(a @ Wg^T) * (a @ Wu^T) in one bf16 product: `w_gu` [2 I, K] holds
-    gate and up rows interleaved in blocks of 16 (see `interleave_gate_up`).  `scratch` as
-    for `gemm`."""
+    gate and up rows interleaved in blocks of 16 (see `interleave_gate_up`).  `scratch`
+    and `whole` as for `gemm`."""
     for t in (a, w_gu, out):
         if not t.is_cuda:
             raise KernelError(f"gemm_swiglu: tensor on {t.device}; kernels run on the GPU only")
@@ -517,7 +519,7 @@ def gemm_swiglu(a: torch.Tensor, w_gu: torch.Tensor, out: torch.Tensor, kernel: 
             [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, c_int, _P, c_size_t, c_int, _P])
     if scratch is not None:
         _req(scratch.is_cuda and scratch.dtype == torch.float32 and scratch.is_contiguous(), "gemm_swiglu: scratch must be float32 on the device")
-    _check(f(_ptr(a), _ptr(w_gu), _ptr(out), M, N, K, lda, ldc, 3, kernel, _ptr(scratch),
+    _check(f(_ptr(a), _ptr(w_gu), _ptr(out), M, N, K, lda, ldc, 3, kernel or (16 if whole else 0), _ptr(scratch),
              0 if scratch is None else scratch.numel() * 4, wl, _stream()), "gemm_swiglu")
 
 
@@ -537,6 +539,12 @@ def gemm_tile_choice(M: int, N: int, K: int, mode: int = 0, scratch_floats: int 
     k, p, n1 = c_int(0), c_int(0), c_int(0)
     _check(f(M, N, K, mode, scratch_floats * 4, ctypes.byref(k), ctypes.byref(p), ctypes.byref(n1)), "gemm_tile_choice")
     return k.value, p.value, n1.value
+
+
+def gemm_whole_pays(M: int, N: int, K: int, by16: bool = False) -> bool:
+    """Whether a bf16 product of up to 128 aligned rows goes to the kernel that leaves no runs along k (for 17 to 64 rows:
+    when asked for it, `whole` of `gemm`).  `by16`: as `gemm_norm_prepare` asks for it."""
+    return bool(_fn("gemm_bf16", "br_gemm_bf16_whole_pays", [c_int] * 4)(M, N, K, int(by16)))
 
 
 def gemm_wide_parts(M: int, N: int, K: int, scratch_floats: int, accumulate: bool = True) -> int:
@@ -575,13 +583,13 @@ SSQ_LD = 64        # row stride of the sums of squares that a product leaves for
 
 
 def gemm_norm_prepare(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, xg: torch.Tensor,
-                      ssq: torch.Tensor, scratch: Optional[torch.Tensor] = None) -> int:
+                      ssq: torch.Tensor, scratch: Optional[torch.Tensor] = None, whole: bool = False) -> int:
     """x += a @ w^T (x float32: rows of the residual stream) and, in the same kernels, what
     the RMS norm that reads x next needs: xg = bfloat16(x * gain) and, in ssq[tiles, 64],
     sums of x^2 per row over runs of columns.  Returns the number of tiles; `gemm_norm_scaled`
     takes all three.  Up to 16 rows: N in steps of 16.  17 to 64 rows: N in steps of 256 and
-    `scratch` (float32, as for `gemm`) for the product's runs along k.  Raises KernelError for
-    anything else."""
+    `scratch` (float32, as for `gemm`) for the product's runs along k; `whole` as for `gemm` (N in steps
+    of 16 columns then have a tile each).  Raises KernelError for anything else."""
     _dev("gemm_norm_prepare", a, w, x, gain, xg, ssq, scratch)
     M, K = a.shape
     N, wk, wl = _weight_dims("gemm_norm_prepare", w, x.shape[1])
@@ -592,24 +600,25 @@ def gemm_norm_prepare(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, gain: t
          and ssq.numel() >= (N // 16) * SSQ_LD, "gemm_norm_prepare: shapes")
     tiles = c_int(0)
     f = _fn("gemm_bf16", "br_gemm_bf16_norm_prepare",
-            [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, _P, _P, c_size_t, _P, ctypes.POINTER(c_int), _P, c_size_t, c_int, _P])
+            [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, _P, _P, c_size_t, _P, ctypes.POINTER(c_int), _P, c_size_t, c_int, c_int, _P])
     _check(f(_ptr(a), _ptr(w), _ptr(x), M, N, K, a.stride(0) if M > 1 else K, x.stride(0) if M > 1 else N, _ptr(gain),
              _ptr(xg), xg.stride(0) if M > 1 else N, _ptr(ssq), ctypes.byref(tiles), _ptr(scratch),
-             0 if scratch is None else scratch.numel() * 4, wl, _stream()), "gemm_norm_prepare")
+             0 if scratch is None else scratch.numel() * 4, wl, int(whole), _stream()), "gemm_norm_prepare")
     return tiles.value
 
 
-def gemm_leave_runs(a: torch.Tensor, w: torch.Tensor, n_out: int, scratch: torch.Tensor) -> int:
+def gemm_leave_runs(a: torch.Tensor, w: torch.Tensor, n_out: int, scratch: torch.Tensor, whole: bool = False) -> int:
     """The runs along k of a @ w^T (65 to 1,024 bfloat16 rows, `n_out` columns) as float sums in `scratch`, [runs][M][n_out], for `rmsnorm`
-    to add; returns their number, or 0 (nothing launched) where such a product is not cut or the sizes are not taken."""
+    to add; returns their number, or 0 (nothing launched) where such a product is not cut or the sizes are not taken.  `whole`: one run
+    of a product that is not cut, where the kernel that leaves none is the one chosen."""
     _dev("gemm_leave_runs", scratch)
     M, K = a.shape
     N, wk, wl = _weight_dims("gemm_leave_runs", w, n_out)
     _req(a.is_cuda and a.dtype == w.dtype == torch.bfloat16 and scratch.dtype == torch.float32 and wk == K and N == n_out and a.stride(1) == 1,
          "gemm_leave_runs: bfloat16 rows and matrix")
     runs = c_int(0)
-    f = _fn("gemm_bf16", "br_gemm_bf16_leave_runs", [_P, _P, c_int, c_int, c_int, c_size_t, _P, c_size_t, c_int, _P, _P])
-    rc = f(_ptr(a), _ptr(w), M, N, K, a.stride(0) if M > 1 else K, _ptr(scratch), scratch.numel() * 4, wl, ctypes.byref(runs), _stream())
+    f = _fn("gemm_bf16", "br_gemm_bf16_leave_runs", [_P, _P, c_int, c_int, c_int, c_size_t, _P, c_size_t, c_int, c_int, _P, _P])
+    rc = f(_ptr(a), _ptr(w), M, N, K, a.stride(0) if M > 1 else K, _ptr(scratch), scratch.numel() * 4, wl, int(whole), ctypes.byref(runs), _stream())
     if rc == 1:
         return 0
     _check(rc, "gemm_leave_runs")
@@ -617,11 +626,11 @@ def gemm_leave_runs(a: torch.Tensor, w: torch.Tensor, n_out: int, scratch: torch
 
 
 def gemm_norm_scaled(xg: torch.Tensor, ssq: torch.Tensor, tiles: int, eps: float, w: torch.Tensor, out: torch.Tensor,
-                     swiglu: bool = False, scratch: Optional[torch.Tensor] = None) -> None:
+                     swiglu: bool = False, scratch: Optional[torch.Tensor] = None, whole: bool = False) -> None:
     """out = rmsnorm(x) @ w^T from what `gemm_norm_prepare` left: xg = bfloat16(x * gain)
     [M, K], the sums of squares ssq and their number of tiles; 1 / rms multiplies the
     product's sums.  `out` bfloat16 or float32 [M, N]; with `swiglu`, bfloat16 [M, N / 2] as
-    `gemm_swiglu`."""
+    `gemm_swiglu`.  `whole` as for `gemm`."""
     _dev("gemm_norm_scaled", xg, ssq, w, out, scratch)
     M, K = xg.shape
     N, wk, wl = _weight_dims("gemm_norm_scaled", w, 2 * out.shape[1] if swiglu else out.shape[1])
@@ -634,10 +643,10 @@ def gemm_norm_scaled(xg: torch.Tensor, ssq: torch.Tensor, tiles: int, eps: float
         _req(out.shape == (M, N) and out.dtype in (torch.bfloat16, torch.float32), "gemm_norm_scaled: out must be [M, N]")
         mode = 0 if out.dtype == torch.bfloat16 else 1
     f = _fn("gemm_bf16", "br_gemm_bf16_norm_scaled",
-            [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, _P, c_int, c_int, c_float, _P, c_size_t, c_int, _P])
+            [_P, _P, _P, c_int, c_int, c_int, c_size_t, c_size_t, c_int, _P, c_int, c_int, c_float, _P, c_size_t, c_int, c_int, _P])
     _check(f(_ptr(xg), _ptr(w), _ptr(out), M, N, K, xg.stride(0) if M > 1 else K, out.stride(0) if M > 1 else out.shape[1],
              mode, _ptr(ssq), int(tiles), K, float(eps), _ptr(scratch), 0 if scratch is None else scratch.numel() * 4,
-             wl, _stream()), "gemm_norm_scaled")
+             wl, int(whole), _stream()), "gemm_norm_scaled")
 
 
 def interleave_gate_up(w_gate: torch.Tensor, w_up: torch.Tensor, alloc=None) -> torch.Tensor:

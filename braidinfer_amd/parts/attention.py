@@ -109,7 +109,7 @@ class GQAAttention(Mixer):
             # step's rows: where their product is cut into runs it adds the runs too
             runs = linear_runs(h, self.w_qkv, qkv.shape[1], step.ws)
             if runs is None:
-                linear(h, self.w_qkv, qkv, step.ws)
+                linear(h, self.w_qkv, qkv, step.ws, whole=False)
             return self._finish(qkv, x, step, ctx, tables, True, runs)
         linear(h, self.w_qkv, qkv, step.ws)
         K.rope_kv_write(qkv, tables.cos if tables else None, tables.sin if tables else None,

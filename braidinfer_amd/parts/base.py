@@ -117,9 +117,9 @@ class Norm(Part):
         takes, or None with nothing done."""
         return None
 
-    def product_of_prepared(self, prepared: Any, w: torch.Tensor, out: torch.Tensor, swiglu: bool = False) -> bool:
+    def product_of_prepared(self, prepared: Any, w: torch.Tensor, out: torch.Tensor, swiglu: bool = False, whole: bool = True) -> bool:
         """out = norm(x) @ w^T from what `prepare_in_product` left; False with nothing done
-        if there is no kernel for these sizes."""
+        if there is no kernel for these sizes.  `whole` as for `linear`."""
         return False
 
 

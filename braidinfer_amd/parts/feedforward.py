@@ -74,7 +74,7 @@ class SwiGLU(FeedForward):
                     h = h.tensor()
             if h is not None:
                 scratch = step.ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32) if 64 < T <= 1024 else None
-                K.gemm_swiglu(h, self.w_gu, a, scratch=scratch)
+                K.gemm_swiglu(h, self.w_gu, a, scratch=scratch, whole=True)
         else:
             gu = step.ws.get("ffn_gu", (T, 2 * self.I), dt)
             linear(h, self.w_gu, gu, step.ws)

@@ -13,16 +13,17 @@ from .. import kernels as K
 from .base import NormedInput, ProductRuns, ResidualSink
 
 
-def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False) -> None:
+def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False, whole: bool = True) -> None:
     """out (+)= a @ w^T.  `accumulate` needs a float32 `out`.  `w` is [N, K] or what
     `stream_layout` made of it.
 
     `a` may be a `NormedInput` (the product is then taken of the normed rows, from what the
     product before prepared where it did) and `out` a `ResidualSink` (the product is added
-    to its rows and, where the next norm can, prepares that norm in the same kernel)."""
+    to its rows and, where the next norm can, prepares that norm in the same kernel).  `whole`
+    False: the bits that `linear_runs` leaves in runs (see `kernels.gemm`)."""
     if isinstance(a, NormedInput):
         if a.prepared is not None and not accumulate and not isinstance(out, ResidualSink) \
-                and a.norm.product_of_prepared(a.prepared, w, out):
+                and a.norm.product_of_prepared(a.prepared, w, out, whole=whole):
             return
         a = a.tensor()
     if isinstance(out, ResidualSink):
@@ -43,7 +44,7 @@ def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False) -> None:
             scratch = None
             if 16 < a.shape[0] <= 1024:     # products that may be split along k
                 scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32)
-            K.gemm(a, w, out, accumulate, scratch=scratch)
+            K.gemm(a, w, out, accumulate, scratch=scratch, whole=whole)
             return
     if w.dtype == torch.float32 and a.dtype == torch.bfloat16:
         a32 = ws.get("linear_in32", a.shape, torch.float32)
@@ -51,7 +52,7 @@ def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False) -> None:
             K.convert(a, a32)
         else:
             a32.copy_(a)
-        linear(a32, w, out, ws, accumulate)
+        linear(a32, w, out, ws, accumulate, whole)
         return
     if w.dtype == torch.bfloat16 and a.dtype == torch.float32:
         a16 = ws.get("linear_in16", a.shape, torch.bfloat16)
@@ -59,7 +60,7 @@ def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False) -> None:
             K.convert(a, a16)
         else:                              # a column range of wider rows
             K.rows_into(a, a16)
-        linear(a16, w, out, ws, accumulate)
+        linear(a16, w, out, ws, accumulate, whole)
         return
     raise TypeError(f"linear: activations {a.dtype}, weight {w.dtype}")
 

@@ -73,7 +73,7 @@ class RMSNorm(Norm):
                 return None
             h = ws.get("norm_rows", (M, N), torch.bfloat16)
             scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32)
-            runs = K.gemm_leave_runs(a, w, N, scratch)
+            runs = K.gemm_leave_runs(a, w, N, scratch, True)
             if not runs:
                 return None
             K.rmsnorm(x, self.weight, h, self.eps, add=(scratch, runs))
@@ -82,25 +82,25 @@ class RMSNorm(Norm):
                 and N % (16 if M <= 16 else 256) == 0 and K.gemm_stream_takes(M, a.shape[1])
                 and K.gemm_stream_takes(M, N) and a.is_contiguous() and x.is_contiguous()):
             return None
-        # 17 to 64 rows: the preparation rides on the sum of a product cut along k
-        if M > 16 and K.gemm_wide_parts(M, N, a.shape[1], K.GEMM_SCRATCH_FLOATS) < 2:
+        # 17 to 64 rows: the preparation rides on a product that is not cut, or on the sum of one that is
+        if M > 16 and not K.gemm_whole_pays(M, N, a.shape[1], by16=True) and K.gemm_wide_parts(M, N, a.shape[1], K.GEMM_SCRATCH_FLOATS) < 2:
             return None
         xg = ws.get("norm_xg", (M, N), torch.bfloat16)
         ssq = ws.get("norm_ssq", ((N // 16) * K.SSQ_LD,), torch.float32)
         scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32) if M > 16 else None
-        tiles = K.gemm_norm_prepare(a, w, x, self.weight, xg, ssq, scratch)
+        tiles = K.gemm_norm_prepare(a, w, x, self.weight, xg, ssq, scratch, whole=True)
         return xg, ssq, tiles, scratch
 
     def rows_of_prepared(self, prepared):
         return prepared[1] if isinstance(prepared[0], str) and prepared[0] == "rows" else None
 
-    def product_of_prepared(self, prepared, w, out, swiglu=False):
+    def product_of_prepared(self, prepared, w, out, swiglu=False, whole=True):
         if self.rows_of_prepared(prepared) is not None:      # an ordinary product of `NormedInput.tensor`
             return False
         xg, ssq, tiles, scratch = prepared
         if w.dtype != torch.bfloat16 or (not swiglu and out.dtype not in (torch.bfloat16, torch.float32)):
             return False
-        K.gemm_norm_scaled(xg, ssq, tiles, self.eps, w, out, swiglu=swiglu, scratch=scratch)
+        K.gemm_norm_scaled(xg, ssq, tiles, self.eps, w, out, swiglu=swiglu, scratch=scratch, whole=whole)
         return True
 
     def runs_of_prepared(self, prepared, w, n_out, ws):
