@@ -3,10 +3,10 @@
 // checkpoints store it ([out, in], row-major), so both operands are read along k.
 //
 // Kernels:
-//  * gemm_stream: M <= 16 rows (decode): weight streaming by one resident workgroup per
-//    compute unit, weights and activations brought into per-wave LDS rings by direct
-//    global-to-LDS loads (described at the kernel).
-//  * gemm_stream_tile: up to 128 rows against few enough weight rows: a workgroup a tile of 16 to 32 of them over all of K.
+//  * gemm_stream_tile: up to 16 rows (decode), and up to 128 against few weight rows: a workgroup a tile of 16 to 32 weight rows
+//    over all of K, weights and activations brought into per-wave LDS rings by direct global-to-LDS loads.
+//  * gemm_stream: up to 16 rows with an RMS norm before or behind, where tiles are many or K long: the same streaming by one
+//    resident workgroup per compute unit.
 //  * gemm_tile: LDS-staged tiles for many rows (prompts): 4 waves, each a TM x TN grid of
 //    v_mfma_f32_32x32x16_bf16 blocks; global loads of the next k-tile are issued before the
 //    current one is multiplied and written to the other LDS buffer after it.
@@ -1538,7 +1538,7 @@ static int split_parts(int M, int N, int K, int mode, size_t scratch_bytes) {
 }
 
 // ------------------------------------------------------------------ gemm_stream ------
-// M <= 16, K in steps of 128: weight streaming by workgroups that stay.  One workgroup per
+// M <= 16, K in steps of 128, a norm before or behind: weight streaming by workgroups that stay.  One workgroup per
 // compute unit walks over tiles of 16 weight rows (tile t of workgroup b is b + t * grid);
 // its 8 waves take the tile's 128-wide k-chunks in turn.  A wave brings a chunk of the
 // tile (16 rows x 256 bytes) and the same chunk of the activations (8 or 16 rows) into a
@@ -1559,7 +1559,6 @@ static int split_parts(int M, int N, int K, int mode, size_t scratch_bytes) {
 //    tile it adds the `ssq_tiles` sums of every row in a fixed order, and 1 / rms, the same
 //    for a whole row, multiplies the sums at a tile's end:
 //    y = rsqrt(mean(h^2) + eps) * sum_k W[n,k] (h[k] g[k]).
-// NORM = 3: products of several inputs by stacked weights in one launch (br_gemm_bf16_branches).
 struct StreamNorm {
     const float* gain;     // producer: the next norm's weights [N]
     bf16* xg;              // producer: [M, ldx]
@@ -1585,8 +1584,8 @@ __device__ __forceinline__ int branch_gap(const StreamBranches& b, int n) { retu
 template <int RT, int XR, int KC, int S, int NW, int MODE, int NORM>
 __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C, int M, int N, int K, size_t lda,
-                                                              size_t ldc, int ntiles, typename StreamArg<NORM>::type nrm, int wl) {
-    static_assert(NORM == 0 || (NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC) || (NORM == 3 && MODE == OUT_F32), "norm forms");
+                                                              size_t ldc, int ntiles, StreamNorm nrm, int wl) {
+    static_assert((NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC), "norm forms");
     constexpr int STEPS = KC / 32;
     constexpr int ROWB = KC * 2;
     constexpr int STAGE = (RT + XR) * ROWB;
@@ -1624,8 +1623,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
     int cp_t = 0, cp_c = 0;      // compute cursor
     int buf = 0;
 
-    // NORM 3: where the activations of the tile to ask for lie behind the first branch's
-    size_t a_off = branch_rows(nrm, (int)blockIdx.x * RT);
 #define ISSUE(J)                                                                                         \
     do {                                                                                                 \
         int chunk_ = wave + is_c * NW + rot;                                                             \
@@ -1642,7 +1639,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                 int m_ = row_ - RT;                                                                      \
                 if (m_ > M - 1) m_ = M - 1;                                                              \
                 gp_ = A + (size_t)m_ * lda + (size_t)chunk_ * KC + ((dcol ^ (row_ & 7)) * 8);            \
-                if (NORM == 3) gp_ += a_off;                                                             \
             }                                                                                            \
             const unsigned lds_ = __builtin_amdgcn_readfirstlane(ring_lds + (J) * STAGE + q_ * 1024);    \
             if (q_ < WDMA)                              /* weights pass once: non-temporal */            \
@@ -1653,7 +1649,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
         if (++is_c == ncw) {                                                                             \
             is_c = 0;                                                                                    \
             ++is_t;                                                                                      \
-            if (NORM == 3) a_off = branch_rows(nrm, ((int)blockIdx.x + is_t * (int)gridDim.x) * RT);     \
         }                                                                                                \
     } while (0)
 
@@ -1757,12 +1752,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
 #pragma unroll
                                 for (int w = 0; w < NW; ++w) v += rb[(w * 16 + nl) * 17 + m];
                                 if (NORM == 2) v *= rstd[m];
-                                const size_t idx = (size_t)m * ldc + n + branch_gap(nrm, n0);
+                                const size_t idx = (size_t)m * ldc + n;
                                 if (MODE == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
-                                else if (MODE == OUT_F32) ((float*)C)[idx] = v;
-                                // one add per element and product, without a read that this wave would
-                                // have to wait for behind its loads in flight
-                                else unsafeAtomicAdd((float*)C + idx, v);
+                                else ((float*)C)[idx] = v;
                             }
                         }
                     }
@@ -1780,7 +1772,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
 #define STREAM_NW 8
 template <int XR, int NORM>
 static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc,
-                         int mode, hipStream_t s, typename StreamArg<NORM>::type nrm = typename StreamArg<NORM>::type{}, int wl = 0) {
+                         int mode, hipStream_t s, const StreamNorm& nrm, int wl) {
     constexpr int RT = 16, KC = STREAM_KC, S = 2, NW = STREAM_NW;
     static_assert(KC == 128, "the blocked weight layout has 128 k a block");
     const int cus = br_device_cus();
@@ -1802,14 +1794,10 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
     } while (0)
     if constexpr (NORM == 1) {
         BR_STREAM(OUT_F32_ACC);
-    } else if constexpr (NORM == 3) {
-        if (mode != OUT_F32) return BR_BAD_ARG;
-        BR_STREAM(OUT_F32);
     } else {
         if (mode == OUT_BF16) BR_STREAM(OUT_BF16);
         else if (mode == OUT_F32) BR_STREAM(OUT_F32);
         else if (mode == OUT_SWIGLU) BR_STREAM(OUT_SWIGLU);
-        else if constexpr (NORM == 0) BR_STREAM(OUT_F32_ACC);
         else return BR_BAD_ARG;
     }
 #undef BR_STREAM
@@ -1825,16 +1813,19 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
 // cycles.  At the end the waves' sums meet in LDS and are added in wave order.
 //
 // Up to 16 rows the memory bounds it: what counts is that all compute units stream the same share (6,144 weight rows are 256 tiles of
-// 24, where gemm_stream's 384 tiles of 16 leave half of the workgroups with twice the work of the others).  With more rows it is the
-// compute unit's path from the L2, 62 to 70 GB/s here, which carries 16 MB activation rows for the tile's 16 to 32: gemm_stream_wide
-// shares them over more weight rows and pays with runs along k and their sum, and wins where K is long (see tile_pays).
-// us, weights in no cache, before -> now (before: gemm_stream up to 16 rows, gemm_stream_wide with the sum of its runs up to 64,
-// the eight-wave tiles with theirs beyond): 6,144 x 4,096 by 8 rows 12.7 -> 10.9; 4,096 x 4,096, 2,048 x 2,048, 8,192 x 4,096 by 24 rows
-// 14.3 -> 9.2, 9.5 -> 5.6, 18.7 -> 13.6, by 64 rows 14.9 -> 13.3, 11.6 -> 7.8, 19.9 -> 18.3, by 80 rows 22.4 -> 15.3, 11.5 -> 8.8, 28.1 -> 20.9.
+// 24; 384 tiles of 16 leave half of the units with twice the work of the others), and that two workgroups share a unit where there are
+// more tiles than units.  With more rows it is the compute unit's path from the L2, 62 to 70 GB/s here, which carries 16 MB activation
+// rows for the tile's 16 to 32: gemm_stream_wide shares them over more weight rows and pays with runs along k and their sum, and wins
+// where K is long (see tile_rows).
+// us, weights in no cache, before -> now (before: resident workgroups that walk tiles of 16 rows up to 16 rows, gemm_stream_wide with the
+// sum of its runs up to 64, the eight-wave tiles with theirs beyond): 6,144 x 4,096 by 8 rows 12.7 -> 10.9; 4,096 x 4,096, 2,048 x 2,048,
+// 8,192 x 4,096 by 24 rows 14.3 -> 9.2, 9.5 -> 5.6, 18.7 -> 13.6, by 64 rows 14.9 -> 13.3, 11.6 -> 7.8, 19.9 -> 18.3, by 80 rows
+// 22.4 -> 15.3, 11.5 -> 8.8, 28.1 -> 20.9.
 // Chunks of 128 in one stage took 0 to 10 % longer; rows of activations further apart than a power of two changed nothing.
 //
 // NORM 1, 2: as gemm_stream's forms (the tile's columns as sums of squares by 16); C, or the sums of squares, are asked for
-// before the first weights and used at the end.
+// before the first weights and used at the end.  NORM 3: products of several inputs by stacked weights in one launch
+// (br_gemm_bf16_branches); a tile lies in one branch.
 constexpr int tile_waves(int RT, int MB) { return 640 / (RT + 16 * MB) < 8 ? 640 / (RT + 16 * MB) : 8; }     // 160 KB of LDS
 #define TILE_KC 64
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -1846,7 +1837,7 @@ __device__ __forceinline__ const bf16* uniform(const bf16* p) {
 template <int RT, int MB, int NORM>
 __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                                    void* __restrict__ C, int M, int N, int K, size_t lda,
-                                                                                   size_t ldc, int mode, int vec, StreamNorm nrm, int wl) {
+                                                                                   size_t ldc, int mode, int vec, typename StreamArg<NORM>::type nrm, int wl) {
     static_assert(NORM != 1 || RT % 16 == 0, "sums of squares by 16 columns");
     constexpr int NW = tile_waves(RT, MB), RB = (RT + 15) / 16, ROWS = RT + 16 * MB, STAGE = ROWS * TILE_KC * 2, NL = STAGE / 1024;
     constexpr int WL_LOADS = RT / 8;   // loads of 8 rows by 128 bytes: the weights', then the activations'
@@ -1909,7 +1900,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
             src[i] = W + w_row_base(n, K, wl) + col;
         } else {
             const int m = row - RT < M ? row - RT : M - 1;
-            src[i] = A + (size_t)m * lda + col;
+            src[i] = A + branch_rows(nrm, n0) + (size_t)m * lda + col;
         }
     }
     int asked = 0;
@@ -2041,7 +2032,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
             continue;
         }
         if (m >= M || n < 0 || n >= N) continue;
-        float* to = (float*)C + (size_t)m * ldc + n;
+        float* to = (float*)C + (size_t)m * ldc + n + branch_gap(nrm, n0);
         bf16* to16 = (bf16*)C + (size_t)m * ldc + n;
         if (vec && mode != OUT_F32_ACC) {              // N in steps of 4: all four columns
             if (mode == OUT_BF16) {
@@ -2065,7 +2056,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
 // rt: weight rows of a workgroup (16, 24, 32).  norm as NORM above; 1 and 2 up to 64 rows, 1 with N and rt in steps of 16.
 template <int RT, int MB, int NORM>
 static int launch_tile_form(const bf16* A, const bf16* W, void* C, int M, int N, int K, size_t lda, size_t ldc, int mode, hipStream_t s,
-                            const StreamNorm& nrm, int wl) {
+                            const typename StreamArg<NORM>::type& nrm, int wl) {
     constexpr int lds = tile_waves(RT, MB) * 2 * (RT + 16 * MB) * TILE_KC * 2;
     static_assert(lds <= 160 * 1024, "LDS of a compute unit");
     auto kern = gemm_stream_tile_kernel<RT, MB, NORM>;
@@ -2076,8 +2067,9 @@ static int launch_tile_form(const bf16* A, const bf16* W, void* C, int M, int N,
     }
     // rows that 16-byte stores (8 of bf16) can take
     const bool half = mode == OUT_BF16 || mode == OUT_SWIGLU;
-    const int vec = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0 &&
-                    (NORM != 1 || (nrm.ldx % 4 == 0 && (uintptr_t)nrm.xg % 8 == 0 && (uintptr_t)nrm.gain % 16 == 0));
+    int vec = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0;
+    if constexpr (NORM == 1) vec = vec && (nrm.ldx % 4 == 0 && (uintptr_t)nrm.xg % 8 == 0 && (uintptr_t)nrm.gain % 16 == 0);
+    if constexpr (NORM == 3) vec = vec && nrm.gap % 4 == 0;
     kern<<<(N + RT - 1) / RT, 64 * tile_waves(RT, MB), lds, s>>>(A, W, C, M, N, K, lda, ldc, mode, vec, nrm, wl);
     return br_check_launch();
 }
@@ -2117,19 +2109,24 @@ static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, vo
     return BR_BAD_ARG;
 }
 // The weight rows of a workgroup (16, 24 or 32) where gemm_stream_tile is the faster kernel, else 0.
-// Up to 16 rows, K from 1,024 up to 8,191: where one workgroup a compute unit has the matrix (N up to 32 a unit), with
-// the fewest rows for the busiest unit, the same for every number of rows, so that a row's bits do not depend on the others'.  With longer K a
-// tile of 16 rows gains nothing over gemm_stream (14,336: 21.7 against 21.5 us), and beyond 32 rows a unit gemm_stream's loads go on across tiles.
+// Up to 16 rows always (K in steps of 128 from 1,024): the fewest weight rows for the busiest compute unit, the same for every number
+// of rows, so that a row's bits do not depend on the others'; of two that are alike the taller where one round covers the matrix
+// (8,192 x 4,096: 12.6 us by 32, 13.7 by 16), else the lower, of which two workgroups share a unit (32,768 x 4,096 by 8 rows:
+// 43.9 by 16, 46.0 by 24, 46.5 by 32).  One resident workgroup a unit that walked tiles of 16 rows, as gemm_stream does, took, at 1, 8
+// and 16 rows: 6,144 x 4,096 12.2 / 12.7 / 13.8 (now 10.6 / 10.9 / 11.0), 32,768 x 4,096 45.3 / 47.0 / 54.3 (43.3 / 43.9 / 49.2),
+// 5,120 x 13,824 32.0 / 32.9 / 36.8 (25.5 / 27.2 / 28.0), 4,096 x 14,336 21.2 / 21.4 / 24.3 (20.7 / 21.5 / 23.5), 2,048 x 8,192
+// 10.7 / 9.9 / 11.2 (9.9 / 9.8 / 11.6).
 // More rows: by counts in microseconds, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at nine numbers of rows from 17
 // to 96, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's; gemm_stream_wide
 // with the sum of its runs (up to 64 rows); the eight-wave tiles with theirs (beyond; single rounds only, where the count is sound).
 // The line it draws gains 1.3 in the mean over these, and loses 5 % at most.  by16: whole blocks of 16 columns only (NORM 1).
 static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) {
     if (M <= 0 || M > TILE_MAX_ROWS || K % 128 || K < (M <= 16 ? 1024 : 256) || cus <= 0) return 0;
-    if (M <= 16 && (K >= 8192 || N > 32 * cus)) return 0;
     int best_rt = 0;
     double best = 1e30;
-    for (int rt = 32; rt >= 16; rt -= 8) {
+    const bool low = M <= 16 && N > 32 * cus;
+    for (int i = 0; i < 3; ++i) {
+        const int rt = low ? 16 + 8 * i : 32 - 8 * i;
         if (rt == 24 && (mode == OUT_SWIGLU || by16)) continue;
         const int rounds = (N + rt * cus - 1) / (rt * cus);
         const double t = M <= 16 ? (double)rounds * rt : 3.1 + rounds * (double)(rt + M) * K * 2.9e-5 + (double)N * K * 1.27e-7;
@@ -2142,6 +2139,11 @@ static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) 
     if (M > 64 && N > best_rt * cus) return 0;
     return best < other ? best_rt : 0;
 }
+
+// Whether the norm forms of up to 16 rows, too, leave gemm_stream: one round of tiles (every workgroup reads all sums of squares:
+// 28,672 x 4,096 by 8 rows 38.7 us by tiles, 37.2 by resident workgroups; 6,144 x 4,096 11.5 and 12.9), and K below 8,192 (4,096 x 14,336
+// by 8 and 16 rows 21.4 and 24.0 against 20.9 and 23.2; 4,096 x 4,096 8.1 and 9.0 against 8.6 and 9.0).
+static bool tile_norms(int M, int N, int K, int cus) { return M > 16 || (N <= 32 * cus && K < 8192); }
 
 // What launch_stream_tile needs of its operands beside aligned rows.
 static bool tile_takes(int M, int K, size_t lda) { return M > 0 && M <= TILE_MAX_ROWS && K % 128 == 0 && K >= 256 && lda >= (size_t)K; }
@@ -2511,8 +2513,8 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
 // kernel: 0 = choose, 1 = tile 128x128 through registers (any shape; plus 16 b: the narrow kernel with b blocks of 16 weight rows a
 // workgroup, 1, 2 or 4, aligned rows), 2 = the same 256x128,
 // 3 = skinny (M <= 64), 4..6 = direct-to-LDS tiles 256x128, 128x256, 128x128 (K a multiple
-// of 64, aligned rows), 7 = stream (M <= 16, K a multiple of 128 and at least 1024, aligned
-// rows; plus 16 b: gemm_stream_tile, 8 (b + 1) weight rows a workgroup, M <= 128, K from 256), 8 = stream wide (16 < M <= 64, K a multiple of 128), 9 = direct-to-LDS tile 64x128
+// of 64, aligned rows), 7 = gemm_stream_tile (M <= 16, K a multiple of 128 and at least 1024, aligned
+// rows; plus 16 b: 8 (b + 1) weight rows a workgroup, M <= 128, K from 256), 8 = stream wide (16 < M <= 64, K a multiple of 128), 9 = direct-to-LDS tile 64x128
 // (M <= 64), 10 = direct-to-LDS tile 256x192, 11 = the same 256x256 (SwiGLU epilogue only), 12..15 = the tiles of
 // four waves, one to a SIMD: 256x256, 128x256, 256x192, 256x224 (K a multiple of 64, aligned rows, output rows in steps
 // of 16 bytes; plus 16 p: with p runs along k); tests force one.  (A 256x256 tile of 8 waves for every epilogue
@@ -2552,9 +2554,9 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
         const int blocks = narrow_blocks(M, N, K, mode, br_device_cus(), (scratch && (uintptr_t)scratch % 16 == 0) ? scratch_bytes : 0);
         if (blocks) return launch_narrow_blocks(blocks, A, W, C, M, N, K, lda, ldc, mode, s);
     }
-    // Up to 16 and beyond 64 rows the tile kernel where it is the faster; in between only when asked for a product without runs
+    // Beyond 64 rows the tile kernel where it is the faster; 17 to 64 rows only when asked for a product without runs
     // (kernel 16): the sums of runs that br_gemm_bf16_wide_partial leaves are those of the product that is chosen without being asked.
-    if (chosen && aligned && tile_takes(M, K, lda) && (M <= 16 || M > 64 || forced_parts == 1)) {
+    if (chosen && aligned && M > 16 && tile_takes(M, K, lda) && (M > 64 || forced_parts == 1)) {
         const int rt = tile_rows(M, N, K, mode, br_device_cus());
         if (rt) return launch_stream_tile(rt, 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     }
@@ -2574,11 +2576,10 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
                        : launch_stream_wide<4>(A, W, C, M, N, K, lda, ldc, mode, (float*)scratch, scratch_bytes, s, 0,
                                                StreamNorm{}, fh, fp, wl);
     }
-    if (kernel == 7 && forced_parts) {                 // 7 + 16 b: a workgroup a tile of 8 (b + 1) weight rows, b = 1, 2, 3
+    if (kernel == 7 && !chosen && forced_parts) {      // 7 + 16 b: a workgroup a tile of 8 (b + 1) weight rows, b = 1, 2, 3
         return launch_stream_tile(8 * (forced_parts + 1), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     }
-    if (kernel == 7) return M <= 8 ? launch_stream<8, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl)
-                                   : launch_stream<16, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
+    if (kernel == 7) return launch_stream_tile(tile_rows(M, N, K, mode, br_device_cus()), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     int parts = 1;
     if (chosen && M > 128 && (kernel == 5 || kernel == 6) && quad_takes(C, M, N, K, lda, ldc)) {
         // More than 128 rows, K in steps of 64: the tiles of one wave per SIMD, where the product's addresses
@@ -2745,7 +2746,7 @@ extern "C" int br_gemm_bf16_norm_prepare(const void* A, const void* W, float* C,
     if (ldc < (size_t)N || ldx < (size_t)N || !gain || !xg || !ssq || !ssq_tiles) return BR_BAD_ARG;
     StreamNorm nrm{gain, (bf16*)xg, ldx, ssq, 0, 0.f, 0.f};
     if (N % 16 == 0 && M <= 64 && (stream_takes(A, W, M, K, lda) || (whole && wide_takes(A, W, M, K, lda)))) {
-        const int rt = tile_rows(M, N, K, OUT_F32_ACC, br_device_cus(), true);
+        const int rt = tile_norms(M, N, K, br_device_cus()) ? tile_rows(M, N, K, OUT_F32_ACC, br_device_cus(), true) : 0;
         if (rt) {
             *ssq_tiles = N / 16;
             return launch_stream_tile(rt, 1, (const bf16*)A, (const bf16*)W, C, M, N, K, lda, ldc, OUT_F32_ACC, s, nrm, wl);
@@ -2778,7 +2779,7 @@ extern "C" int br_gemm_bf16_norm_scaled(const void* XG, const void* W, void* C, 
     if (mode == OUT_SWIGLU ? (N % 16 != 0 || ldc < (size_t)N / 2) : ldc < (size_t)N) return BR_BAD_ARG;
     StreamNorm nrm{nullptr, nullptr, 0, (float*)ssq, ssq_tiles, 1.f / (float)norm_width, eps};
     if (M <= 64 && (stream_takes(XG, W, M, K, lda) || (whole && wide_takes(XG, W, M, K, lda)))) {
-        const int rt = tile_rows(M, N, K, mode, br_device_cus());
+        const int rt = tile_norms(M, N, K, br_device_cus()) ? tile_rows(M, N, K, mode, br_device_cus()) : 0;
         if (rt) return launch_stream_tile(rt, 2, (const bf16*)XG, (const bf16*)W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
     }
     if (stream_takes(XG, W, M, K, lda))
@@ -2798,7 +2799,7 @@ extern "C" int br_gemm_bf16_norm_scaled(const void* XG, const void* W, void* C, 
 // branch's rows b a_step elements behind the first's, and col(n) = n, or n + gap from n = gap_at on; float results, up to 64
 // rows.  A mixer's projections of inputs that differ are four launches otherwise, each with its own ramp and, from 17 rows on, a
 // second launch for the sums of its runs along k: four of 4,096 by 4,096, weights in no cache,
-// 6 rows 34.4 -> 25.6 us, 24 rows 58.6 -> 25.9, 64 rows 60.0 -> 30.7; four of 2,048 by 2,048 20.4 -> 10.6, 39.0 -> 14.1, 46.0 -> 17.4.
+// 6 rows 34.4 -> 21.4 us, 24 rows 58.6 -> 23.5, 64 rows 60.0 -> 27.9; four of 2,048 by 2,048 20.4 -> 7.7, 39.0 -> 8.3, 46.0 -> 10.9.
 template <int MB, int HB>
 static int launch_branches_wide(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const StreamBranches& br, int cus,
                                 hipStream_t s) {
@@ -2827,8 +2828,19 @@ extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, i
     const int N = branches * per, cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
     const StreamBranches br = {per, a_step, gap_at, gap};
-    if (M <= 8) return launch_stream<8, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
-    if (M <= 16) return launch_stream<16, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br);
+    // Tiles of one round also beyond 16 rows (four of 2,048 by 2,048: 24 rows 11.6 -> 8.3 us, 64 rows 15.0 -> 10.9); four of 4,096 by 4,096 by 24 and 64
+    // rows stay with the shared activations (23.6 and 27.8, by tiles 25 and 34).
+    if (M <= 16 || N <= 32 * cus) {
+        const int rt = tile_rows(M <= 16 ? M : 1, N, K, OUT_F32, cus, true);
+#define BR_BRANCH_TILE(MB_)                                                                                                              \
+    return rt == 16 ? launch_tile_form<16, MB_, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br, WL_ROWS)                                   \
+                    : launch_tile_form<32, MB_, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br, WL_ROWS)
+        if (M <= 16) BR_BRANCH_TILE(1);
+        if (M <= 32) BR_BRANCH_TILE(2);
+        if (M <= 48) BR_BRANCH_TILE(3);
+        BR_BRANCH_TILE(4);
+#undef BR_BRANCH_TILE
+    }
     // units of 64 rows, or of 128 where these fill the chip's rounds better (a unit's chunk costs its rows and 16 more, as in wide_shape)
     const long long r64 = (N / 64 + cus - 1) / cus, r128 = (N / 128 + cus - 1) / cus;
     if (r128 * 144 < r64 * 80)

@@ -433,7 +433,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     Rows of `a` and `out` may be strided (a view of a wider buffer); w is contiguous.
     `kernel` forces one bf16 kernel (1, 2: 128x128 and 256x128 tiles staged through
     registers, any shape; 1 plus 16 b: the kernel for few weight rows, b = 1, 2 or 4 blocks of 16 to a workgroup; 3: skinny, M <= 64; 4, 5, 6: 256x128, 128x256 and 128x128 tiles
-    loaded straight into LDS, K in steps of 64; 7: streaming by workgroups that stay, M <= 16
+    loaded straight into LDS, K in steps of 64; 7: streaming by a workgroup a tile of 16 to 32 weight rows, M <= 16
     and K in steps of 128 from 1024; 8: the same for 17 to 64 rows, K in steps of 128; 5 or 6 plus
     16 p: that tile with p runs along k, for measurements; 9: a 64x128 tile loaded straight into
     LDS, M <= 64; 10: a 256x192 tile loaded straight into LDS; 12 to 15: 256x256, 128x256, 256x192 and

@@ -108,7 +108,7 @@ def test_a_norm_prepared_and_used(M, H, Kd, N2, swiglu):
         assert off(out, want) < bound(H)
 
 
-@pytest.mark.parametrize("M,N,K_,pays", [(8, 6144, 4096, True), (8, 8192, 4096, True), (8, 8208, 4096, False), (16, 4096, 8192, False), (24, 4096, 4096, True),
+@pytest.mark.parametrize("M,N,K_,pays", [(8, 6144, 4096, True), (8, 8192, 4096, True), (8, 8208, 4096, True), (16, 5120, 13824, True), (1, 28672, 4096, True), (24, 4096, 4096, True),
                                          (64, 4096, 4096, True), (64, 4096, 14336, False), (64, 28672, 4096, False), (67, 4096, 4096, True),
                                          (67, 4096, 14336, False), (67, 12288, 4096, False), (128, 2048, 2048, True), (129, 2048, 2048, False), (24, 4096, 4160, False)])
 def test_where_the_rule_takes_it(M, N, K_, pays):
