@@ -2118,10 +2118,11 @@ static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, vo
 // 10.7 / 9.9 / 11.2 (9.9 / 9.8 / 11.6).
 // More rows: by counts in microseconds, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at nine numbers of rows from 17
 // to 96, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's; gemm_stream_wide
-// with the sum of its runs (up to 64 rows); the eight-wave tiles with theirs (beyond; single rounds only, where the count is sound).
+// with the sum of its runs (up to 64 rows); the eight-wave tiles with theirs (beyond).  Single rounds only: matrices of more (32,768 x 4,096
+// by 32 rows: 47 us shared, 50 by tiles) have no sums to save.
 // The line it draws gains 1.3 in the mean over these, and loses 5 % at most.  by16: whole blocks of 16 columns only (NORM 1).
 static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) {
-    if (M <= 0 || M > TILE_MAX_ROWS || K % 128 || K < (M <= 16 ? 1024 : 256) || cus <= 0) return 0;
+    if (M <= 0 || M > TILE_MAX_ROWS || K % 128 || K < (M <= 16 ? 1024 : 256) || cus <= 0 || (M > 16 && N > 32 * cus)) return 0;
     int best_rt = 0;
     double best = 1e30;
     const bool low = M <= 16 && N > 32 * cus;
@@ -2136,7 +2137,6 @@ static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) 
     const double mb = (double)N * K * 2e-7;                              // weights in 10 MB
     const double other = M <= 64 ? 0.96 * (6.2 + 0.043 * M + 1.61 * mb + 1.6e-6 * M * N + 4.7e-6 * M * K - (mode == OUT_SWIGLU ? 2.4 : 0.0))
                                  : 9.1 + 1.9 * mb + 0.125e-3 * K + 0.41e-3 * N + 0.027 * M;
-    if (M > 64 && N > best_rt * cus) return 0;
     return best < other ? best_rt : 0;
 }
 
