@@ -1569,10 +1569,14 @@ struct StreamNorm {
 };
 // Branches: weight rows b per .. + per multiply the activations b a_step elements on; output columns from gap_at on lie `gap`
 // further on.  (A type of its own, so that the arguments of the other forms stay as short as they are.)
+// Weight rows from tail_at on are one more branch, whose sums' tanh goes to bf16 rows of their own (the first half of a low-rank pair).
 struct StreamBranches {
     int per;
     size_t a_step;
     int gap_at, gap;
+    int tail_at;
+    bf16* tail;
+    size_t tail_ld;
 };
 template <int NORM> struct StreamArg { typedef StreamNorm type; };
 template <> struct StreamArg<3> { typedef StreamBranches type; };
@@ -2032,6 +2036,12 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
             continue;
         }
         if (m >= M || n < 0 || n >= N) continue;
+        if constexpr (NORM == 3) if (n0 >= nrm.tail_at) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) nrm.tail[(size_t)m * nrm.tail_ld + n - nrm.tail_at + e] = (bf16)tanhf(v[e]);
+            continue;
+        }
         float* to = (float*)C + (size_t)m * ldc + n + branch_gap(nrm, n0);
         bf16* to16 = (bf16*)C + (size_t)m * ldc + n;
         if (vec && mode != OUT_F32_ACC) {              // N in steps of 4: all four columns
@@ -2819,22 +2829,25 @@ extern "C" int br_gemm_bf16_branches_takes(int M, int per, int K) {
     return M > 0 && M <= 64 && per > 0 && per % 128 == 0 && K % STREAM_KC == 0 && K / STREAM_KC >= STREAM_NW;
 }
 
+// tail_rows > 0 (up to 16 rows, in steps of 16, at most per): further weight rows, multiplying one more branch's activations, the
+// tanh of whose sums goes to tail [M, tail_ld]: instead of two launches of their own, 8.4 us of a single-token step a layer.
 extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, int M, int branches, int per, int K, size_t a_step, size_t lda,
-                                     size_t ldc, int gap_at, int gap, hipStream_t s) {
+                                     size_t ldc, int gap_at, int gap, int tail_rows, void* tail, size_t tail_ld, hipStream_t s) {
     const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
     if (branches < 1 || branches > 64 || !br_gemm_bf16_branches_takes(M, per, K) || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 ||
         gap_at % per || ((uintptr_t)A | (uintptr_t)W) % 16 || ldc < (size_t)branches * per || (long long)branches * per > 0x3fffffff)
         return BR_BAD_ARG;
+    if (tail_rows && (M > 16 || tail_rows < 0 || tail_rows > per || tail_rows % 16 || !tail || tail_ld < (size_t)tail_rows)) return BR_BAD_ARG;
     const int N = branches * per, cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    const StreamBranches br = {per, a_step, gap_at, gap};
+    const StreamBranches br = {per, a_step, gap_at, gap, tail_rows ? N : 0x7fffffff, (bf16*)tail, tail_ld};
     // Tiles of one round also beyond 16 rows (four of 2,048 by 2,048: 24 rows 11.6 -> 8.3 us, 64 rows 15.0 -> 10.9); four of 4,096 by 4,096 by 24 and 64
     // rows stay with the shared activations (23.6 and 27.8, by tiles 25 and 34).
     if (M <= 16 || N <= 32 * cus) {
         const int rt = tile_rows(M <= 16 ? M : 1, N, K, OUT_F32, cus, true);
 #define BR_BRANCH_TILE(MB_)                                                                                                              \
-    return rt == 16 ? launch_tile_form<16, MB_, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br, WL_ROWS)                                   \
-                    : launch_tile_form<32, MB_, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br, WL_ROWS)
+    return rt == 16 || tail_rows ? launch_tile_form<16, MB_, 3>(A, W, C, M, N + tail_rows, K, lda, ldc, OUT_F32, s, br, WL_ROWS)          \
+                                 : launch_tile_form<32, MB_, 3>(A, W, C, M, N, K, lda, ldc, OUT_F32, s, br, WL_ROWS)
         if (M <= 16) BR_BRANCH_TILE(1);
         if (M <= 32) BR_BRANCH_TILE(2);
         if (M <= 48) BR_BRANCH_TILE(3);

@@ -74,16 +74,26 @@ class WKVTimeMix(Mixer):
         # r, k, v and g stacked, where a step of few tokens can take them in one launch; their rows otherwise
         hd, four = self.nh * self.d, ("r", "k", "v", "g")
         mats = {s: tensors[prefix + n[s]] for s in four}
-        self.w_four = None
+        self.w_four = self.w_five = None
         if all(m.dtype == torch.bfloat16 for m in mats.values()) and not blocks_at_load(hd, self.H, torch.bfloat16, rt) \
                 and K.gemm_branches_takes(1, hd, self.H):
-            self.w_four = rt.empty((4 * hd, self.H), torch.bfloat16)
+            # behind them the first half of the low-rank pair, where its rows make whole blocks
+            w1 = tensors[prefix + n["w1"]]
+            low = self.rank if w1.dtype == torch.bfloat16 and self.rank % 16 == 0 and self.rank <= hd else 0
+            stack = rt.empty((4 * hd + low, self.H), torch.bfloat16)
             for i, s in enumerate(four):
-                self.w_four[i * hd:(i + 1) * hd].copy_(mats[s])
-            self.w = {s: self.w_four[i * hd:(i + 1) * hd] for i, s in enumerate(four)}
+                stack[i * hd:(i + 1) * hd].copy_(mats[s])
+            self.w_four = stack[:4 * hd]
+            self.w = {s: stack[i * hd:(i + 1) * hd] for i, s in enumerate(four)}
+            if low:
+                self.w_five = stack
+                stack[4 * hd:].copy_(w1)
+                self.w["w1"] = stack[4 * hd:]
         else:
             self.w = {s: stream_layout(m, rt) for s, m in mats.items()}
-        self.w.update({s: stream_layout(tensors[prefix + n[s]], rt) for s in ("w1", "w2")})
+        for s in ("w1", "w2"):
+            if s not in self.w:
+                self.w[s] = stream_layout(tensors[prefix + n[s]], rt)
         self.w_o = stream_layout(tensors[prefix + n["o"]], rt)
         self.w0 = rt.own(tensors[prefix + n["w0"]].to(torch.float32).reshape(-1))
         self.u = rt.own(tensors[prefix + n["u"]].to(torch.float32).reshape(-1))
@@ -105,16 +115,22 @@ class WKVTimeMix(Mixer):
         K.shift_mix(h, self.mu, mixes, kept, step.seq_of_token, step.cu_seqlens, step.slots, step.n_seqs, step.is_decode)
         # float sums r | k | v | z | g side by side
         rows = step.ws.get("wkv_rows", (T, 5 * hd), torch.float32)
+        low_t = step.ws.get("wkv_low_t", (T, self.rank), dt)
+        tail = None
         if self.w_four is not None and dt == torch.bfloat16 and K.gemm_branches_takes(T, hd, self.H):
-            K.gemm_branches(mixes[:4], self.w_four, rows, gap_at=3, gap=hd)
+            tail = low_t if self.w_five is not None and T <= 16 else None
+            if tail is not None:
+                K.gemm_branches(mixes, self.w_five, rows, gap_at=3, gap=hd, tail=tail)
+            else:
+                K.gemm_branches(mixes[:4], self.w_four, rows, gap_at=3, gap=hd)
         else:
             for i, s in enumerate(("r", "k", "v")):
                 linear(mixes[i], self.w[s], rows[:, i * hd:(i + 1) * hd], step.ws)
             linear(mixes[3], self.w["g"], rows[:, 4 * hd:5 * hd], step.ws)
-        low = step.ws.get("wkv_low", (T, self.rank), torch.float32)
-        linear(mixes[4], self.w["w1"], low, step.ws)
-        low_t = step.ws.get("wkv_low_t", (T, self.rank), dt)
-        K.tanh(low, low_t)
+        if tail is None:
+            low = step.ws.get("wkv_low", (T, self.rank), torch.float32)
+            linear(mixes[4], self.w["w1"], low, step.ws)
+            K.tanh(low, low_t)
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
         pieces = pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)

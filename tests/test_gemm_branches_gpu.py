@@ -34,3 +34,27 @@ def test_branches_refuse():
         a, w = torch.zeros(2, M, K_, dtype=torch.bfloat16, device="cuda"), torch.zeros(2 * per, K_, dtype=torch.bfloat16, device="cuda")
         with pytest.raises(KernelError):
             K.gemm_branches(a, w, torch.zeros(M, 2 * per, device="cuda"))
+
+
+# one more branch whose sums' tanh goes to rows of its own: rows of one block, whole; few and many tiles; a tail of one tile, of several, as long as a branch
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("B,per,K_,R,gap", [(4, 128, 1024, 16, 128), (1, 256, 1152, 256, 0), (4, 2048, 2048, 64, 2048), (2, 8192, 1024, 48, 3)])
+def test_a_tail(M, B, per, K_, R, gap):
+    from braidinfer_amd import kernels as K
+    from braidinfer_amd.errors import KernelError
+    g = torch.Generator(device="cuda").manual_seed(M + per)
+    a = torch.randn(B + 1, M, K_, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(B * per + R, K_, generator=g, device="cuda").mul(K_ ** -0.5).to(torch.bfloat16)
+    wide = torch.full((M, B * per + gap), 7.0, device="cuda")
+    room = torch.full((M + 1, R), 7.0, device="cuda", dtype=torch.bfloat16)
+    K.gemm_branches(a, w, wide, gap_at=B - 1, gap=gap, tail=room[:M])
+    plain = torch.full_like(wide, 7.0)
+    for b in range(B):                                   # (each branch as a product of its own)
+        at = b * per + (gap if b == B - 1 else 0)
+        K.gemm(a[b], w[b * per:(b + 1) * per], plain[:, at:at + per])
+    assert float((wide - plain).norm() / plain.norm()) < 4e-7
+    want = torch.tanh(a[B].double() @ w[B * per:].double().T)
+    assert float((room[:M].double() - want).norm() / want.norm()) < 2 ** -8
+    assert bool((room[M:] == 7.0).all())
+    with pytest.raises(KernelError):
+        K.gemm_branches(torch.cat([a] * 17, 1)[:, :17], w, torch.zeros(17, B * per, device="cuda"), tail=torch.zeros(17, R, device="cuda", dtype=torch.bfloat16))
