@@ -29,14 +29,26 @@ MAX_HEAD_DIM = 512      # attention_simple's limit; the matrix-core kernels take
 
 
 def decode_splits(batch: int, nkv: int, max_ctx: int, page: int, cus: int = 256) -> int:
-    """Into how many runs a sequence's pages are cut for single-token steps: about one
-    workgroup per compute unit (measured: more runs cost more in the combine than they gain)
-    and at least two pages per run; beyond that, runs of at most 64 pages.  It depends on the
-    step's shape only (batch and an upper bound of the context) and on the device's number
-    of compute units, never on the tokens."""
+    """Into how many runs a sequence's pages are cut for single-token steps.  It depends on the
+    step's shape only (batch and an upper bound of the context) and on the device's number of
+    compute units, never on the tokens.
+
+    A power of two, since a run's workgroup then keeps to the XCDs its neighbours' are on (24 runs of one
+    sequence: 10.4 us a launch with its sum, 16 or 32: 9.9 and 9.7).  About one workgroup per compute unit
+    where that takes 8 runs or more: twice as many cost more in the sum than they gain (4 sequences of 8 kv
+    heads, 8 and 16 runs: 8.8 and 10.1 us up to 512 tokens, 12.3 and 11.4 up to 2,048).  Fewer runs are long:
+    two workgroups per unit, which its LDS holds, from a bound on that lets them be so (8 sequences of 128 to
+    2,048 tokens, 4 and 8 runs: 16.6 and 14.4 us; 16, 2 and 4: 25.3 and 20.9; 32, 1 and 2: 39.3 and 35.5; but
+    up to 512 tokens 9.9 and 10.5, 13.0 and 12.2, 15.1 and 16.5).  About two pages per run at
+    least, and at most 64."""
     pages = max(1, -(-max_ctx // page))
-    want = -(-max(1, cus) // max(1, batch * nkv))
-    n = max(1, min(want, pages // 2 if pages >= 2 else 1, 64))
+    heads = max(1, batch * nkv)
+    want = max(1, max(1, cus) // heads)
+    n = 1 << (want.bit_length() - 1)
+    if n <= 4 and 2 * n * heads <= 2 * cus and pages >= (24 if n >= 2 else 32):
+        n *= 2
+    most = max(1, min(pages // 2, 64))
+    n = min(n, 1 << (most - 1).bit_length())
     while n < 64 and pages > 64 * n:
         n *= 2
     return n

@@ -927,6 +927,27 @@ def test_attention_decode_over_long_contexts(window, nsplit, variant):
             assert (got - want[b]).abs().max() < 2e-2 * want[b].abs().max(), f"sequence of {lens[b]}, {ns} splits"
 
 
+@pytest.mark.parametrize("nsplit", [2, 15, 16, 17, 33, 63, 64, 65, 130])
+@pytest.mark.parametrize("nq,nkv,hd", [(4, 2, 16), (4, 1, 80), (8, 2, 128), (2, 2, 256)])
+def test_sums_of_decode_runs(nq, nkv, hd, nsplit):
+    """Runs around the counts that are added at once and that a wave has lanes for, of contexts that
+    leave many runs (whose sums are never written) without a page."""
+    lens = [64 * 70 - 3, 1, 64 * 17, 640]
+    ks, vs, cache, table = _long_cache(lens, nkv, hd, seed=5)
+    B = len(lens)
+    q = rnd(B, nq, hd, seed=98, dtype=torch.bfloat16)
+    out = torch.full((B, nq * hd), 5.0, device=DEV, dtype=torch.bfloat16)
+    part_o = torch.full((B * nq * nsplit * hd,), float("nan"), device=DEV)
+    part_ml = torch.full((B * nq * nsplit * 2,), float("nan"), device=DEV)
+    K.attention_decode_bf16(q.reshape(B, nq * hd), nq * hd, out, i32([1, 2, -1, 4]), i32(lens), table, cache, B, nq, nkv,
+                            hd, 64, None, 1 / math.sqrt(hd), nsplit, part_o, part_ml, 0)
+    assert (out[2] == 0).all()                                     # a row of a graph that no sequence fills
+    for b in (0, 1, 3):
+        want = _rows_ref(q[b:b + 1].cpu(), [lens[b] - 1], ks[b], vs[b], nq, nkv, None)[0]
+        got = out[b].reshape(nq, hd).cpu().double()
+        assert torch.isfinite(got).all() and (got - want).abs().max() < 2e-2 * want.abs().max(), (b, lens[b])
+
+
 def test_decode_splits_double_beyond_64_pages_a_run():
     from braidinfer_amd.parts.attention import decode_splits
     assert decode_splits(64, 8, 4096, 64) == 1 and decode_splits(1, 8, 2048, 64) == 16
