@@ -139,28 +139,53 @@ __global__ void layernorm_kernel(const float* __restrict__ x, const float* __res
     }
 }
 
+// The sum over a block of at most four waves, with one barrier: `scratch` (four floats) is used once.
+__device__ __forceinline__ float block_sum_once(float v, float* scratch) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    const int nw = (blockDim.x + 63) >> 6;
+    float t = scratch[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) t += i < nw ? scratch[i] : 0.f;
+    return t;
+}
+
 // The same for widths in steps of 4 up to 4 * VPT * blockDim: a row is read once, 16 bytes a load, and kept
 // in registers between the sums and the scaling.  With `w2` the kernel goes on: the row it has just added
 // to (the residual row) is normed once more with the weight `w2` into `y2` (compute dtype): the norm
 // behind one half of a layer and the norm in front of the next in one pass over the row.
+// Few rows are bound by a chain of latencies (loads, four sums over the block), so that everything the row
+// needs is asked for before the first sum and a sum takes one barrier; many rows by memory.  (8 rows of
+// 4,096 with `w2`: 6.3 us a launch among others; 7.9 with the weights and the residual row asked for
+// where they are used and two barriers a sum; 5,018 rows 52 either way.)
 template <typename T, typename T2, bool ADD, int VPT>
-__global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* __restrict__ w, T* __restrict__ y,
+__global__ __launch_bounds__(256) void layernorm_vec_kernel(const float* __restrict__ x, const float* __restrict__ w, T* __restrict__ y,
                                      const int* __restrict__ rows, int H, float eps, int center, int plain,
                                      const float* __restrict__ w2, T2* __restrict__ y2, float eps2, int center2) {
     __shared__ float scratch[16];
     const int r = blockIdx.x;
     const f32x4* xr = (const f32x4*)(x + (size_t)(rows ? rows[r] : r) * H);
-    const f32x4* wr = (const f32x4*)w;
     T* yr = y + (size_t)r * H;
     const int nv = H >> 2;
-    f32x4 v[VPT];
+    f32x4 v[VPT], wv[VPT], acc[VPT], w2v[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int i = threadIdx.x + j * blockDim.x;
+        if (i < nv) {
+            v[j] = xr[i];
+            wv[j] = ((const f32x4*)w)[i];
+            if (ADD) acc[j] = ((const f32x4*)yr)[i];
+            if (ADD && w2) w2v[j] = ((const f32x4*)w2)[i];
+        }
+    }
     float sm = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = threadIdx.x + j * blockDim.x;
-        if (i < nv) { v[j] = xr[i]; sm += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]); }
+        if (i < nv) sm += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
     }
-    const float mean = center ? block_sum(sm, scratch) / (float)H : 0.f;
+    const float mean = center ? block_sum_once(sm, scratch) / (float)H : 0.f;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
@@ -170,39 +195,41 @@ __global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* _
             for (int e = 0; e < 4; ++e) { v[j][e] -= mean; ss += v[j][e] * v[j][e]; }
         }
     }
-    const float inv = plain ? 1.0f : 1.0f / sqrtf(block_sum(ss, scratch) / (float)H + eps);
+    const float inv = plain ? 1.0f : 1.0f / sqrtf(block_sum_once(ss, scratch + 4) / (float)H + eps);
     float sm2 = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = threadIdx.x + j * blockDim.x;
         if (i < nv) {
-            const f32x4 wv = wr[i];
             if (ADD) {
-                f32x4 acc = ((const f32x4*)yr)[i];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { acc[e] += v[j][e] * inv * wv[e]; v[j][e] = acc[e]; sm2 += acc[e]; }
-                ((f32x4*)yr)[i] = acc;
+                for (int e = 0; e < 4; ++e) { acc[j][e] += v[j][e] * inv * wv[j][e]; v[j][e] = acc[j][e]; sm2 += acc[j][e]; }
+                ((f32x4*)yr)[i] = acc[j];
             } else {
+                float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) yr[4 * i + e] = from_f32<T>(v[j][e] * inv * wv[e]);
+                for (int e = 0; e < 4; ++e) o[e] = v[j][e] * inv * wv[j][e];
+                ew_store<T, 4>(yr + 4 * i, o);
             }
         }
     }
     if (!ADD || !y2) return;
+    T2* y2r = y2 + (size_t)r * H;
     if (!w2) {      // no second norm: the new residual row as it is, in y2's type
-        T2* y2c = y2 + (size_t)r * H;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
             const int i = threadIdx.x + j * blockDim.x;
             if (i < nv) {
+                float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) y2c[4 * i + e] = from_f32<T2>(v[j][e]);
+                for (int e = 0; e < 4; ++e) o[e] = v[j][e];
+                ew_store<T2, 4>(y2r + 4 * i, o);
             }
         }
         return;
     }
     // v holds the new residual row: its norm with w2
-    const float mean2 = center2 ? block_sum(sm2, scratch) / (float)H : 0.f;
+    const float mean2 = center2 ? block_sum_once(sm2, scratch + 8) / (float)H : 0.f;
     float ss2 = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
@@ -212,15 +239,15 @@ __global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* _
             for (int e = 0; e < 4; ++e) { v[j][e] -= mean2; ss2 += v[j][e] * v[j][e]; }
         }
     }
-    const float inv2 = 1.0f / sqrtf(block_sum(ss2, scratch) / (float)H + eps2);
-    T2* y2r = y2 + (size_t)r * H;
+    const float inv2 = 1.0f / sqrtf(block_sum_once(ss2, scratch + 12) / (float)H + eps2);
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = threadIdx.x + j * blockDim.x;
         if (i < nv) {
-            const f32x4 wv = ((const f32x4*)w2)[i];
+            float o[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y2r[4 * i + e] = from_f32<T2>(v[j][e] * inv2 * wv[e]);
+            for (int e = 0; e < 4; ++e) o[e] = v[j][e] * inv2 * w2v[j][e];
+            ew_store<T2, 4>(y2r + 4 * i, o);
         }
     }
 }
