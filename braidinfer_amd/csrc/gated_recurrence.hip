@@ -884,6 +884,150 @@ extern "C" int br_head_norm_gate(const float* o, const float* w, const float* ga
     return br_check_launch();
 }
 
+// ------------------------------------- single tokens of the recurrence with a bonus, normed and gated ------
+// The recurrence with a bonus, the head norm, its weight and the gate for steps of one token a sequence: token s is sequence s's.  A
+// workgroup takes a whole head, so that its output can be normed before it leaves; wave w walks the blocks of four columns w, w + 4, ...,
+// up to CB of them, all of whose state is asked for together with the rows, from memory straight into registers.  The arithmetic
+// and the order of every sum are those of `wkv_scan_kernel` and `head_norm_gate_kernel` (silu, 16-byte loads).  Bound by the
+// launch and one latency for few sequences, by the state, read and written once, for many (64 heads of 64 x 64, less than
+// the two launches in a recorded step: 2 us a layer for 1 sequence, 4 for 8, 11 for 24; those took 9.0 and 4.6 at 8).
+// Padding sequences' rows of y are zero.
+template <int RPL, int CB, typename T>
+__global__ __launch_bounds__(256) void wkv_token_kernel(
+    const float* __restrict__ rows, const float* __restrict__ w0, const float* __restrict__ bonus, float* __restrict__ state,
+    const int* __restrict__ slots, const float* __restrict__ norm_w, const float* __restrict__ gate, T* __restrict__ y,
+    int H, int d, int e, int width, size_t gate_stride, size_t slot_stride, float eps) {
+    typedef T out_t __attribute__((ext_vector_type(4)));
+    constexpr int NV = (CB + 3) / 4;
+    __shared__ __attribute__((aligned(16))) float oL[16 * CB];
+    const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int cg = lane >> 4, g = lane & 15;
+    const int slot = slots[s], ncb4 = e >> 2, hd = H * d;
+    out_t* yrow = (out_t*)(y + ((size_t)s * H + h) * e);
+    if (slot < 0) {
+        if (tid < ncb4) {
+            out_t zero;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) zero[x] = from_f32<T>(0.f);
+            yrow[tid] = zero;
+        }
+        return;
+    }
+    const float* at = rows + (size_t)s * width;
+    float* S = state + (size_t)slot * slot_stride + (size_t)h * ncb4 * RPL * 64 + lane;
+    float st[CB][RPL], vc[CB];
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+        const int cb4 = 4 * i + wave;
+        vc[i] = 0.f;
+#pragma unroll
+        for (int k = 0; k < RPL; ++k) st[i][k] = 0.f;
+        if (cb4 < ncb4) {
+            vc[i] = at[2 * hd + h * e + cb4 * 4 + cg];
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) st[i][k] = S[((size_t)cb4 * RPL + k) * 64];
+        }
+    }
+    auto row = [&](float (&to)[RPL], const float* from) {
+#pragma unroll
+        for (int r4 = 0; r4 < RPL; r4 += 4) {
+            const f32x4 w = *(const f32x4*)(from + h * d + (g * RPL + r4 < d ? g * RPL + r4 : 0));
+#pragma unroll
+            for (int x = 0; x < 4; ++x) to[r4 + x] = w[x];
+        }
+    };
+    float rr[RPL], kk[RPL], ww[RPL], bb[RPL], uu[RPL];
+    row(rr, at);
+    row(kk, at + hd);
+    row(ww, at + 2 * hd + H * e);
+    row(bb, w0);
+    row(uu, bonus);
+    f32x4 z[NV], nw[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = g + 16 * j;
+        if (i < ncb4) {
+            z[j] = ((const f32x4*)(gate + (size_t)s * gate_stride + (size_t)h * e))[i];
+            nw[j] = ((const f32x4*)(norm_w + (size_t)h * e))[i];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) {
+        const bool real = g * RPL + k < d;
+        ww[k] = real ? expf(-expf(ww[k] + bb[k])) : 1.f;
+        if (!real) rr[k] = kk[k] = uu[k] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+        float sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < RPL; ++k) {
+            const float kv = kk[k] * vc[i];
+            sum = fmaf(rr[k], fmaf(uu[k], kv, st[i][k]), sum);
+            st[i][k] = fmaf(ww[k], st[i][k], kv);
+        }
+        sum = glr_row16_sum(sum);
+        if (g == 0) oL[(4 * i + wave) * 4 + cg] = sum;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+        const int cb4 = 4 * i + wave;
+        if (cb4 < ncb4) {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) S[((size_t)cb4 * RPL + k) * 64] = st[i][k];
+        }
+    }
+    if (wave) return;
+    f32x4 v[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = g + 16 * j;
+        if (i < ncb4) {
+            v[j] = *(const f32x4*)(oL + 4 * i);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) ss = fmaf(v[j][x], v[j][x], ss);
+        }
+    }
+    const float inv = 1.0f / sqrtf(glr_row16_sum(ss) / (float)e + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int i = g + 16 * j;
+        if (i < ncb4 && cg == 0) {
+            out_t out;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) out[x] = from_f32<T>(v[j][x] * inv * nw[j][x] * hng_gate(z[j][x], 0));
+            yrow[i] = out;
+        }
+    }
+}
+
+static bool wkv_token_takes(int d, int e) { return d > 0 && d <= 128 && d % 4 == 0 && e > 0 && e <= 128 && e % 4 == 0; }
+
+// rows, w0, bonus, state and `slot_stride` as for `br_wkv_scan`, norm_w [H e], gate rows `gate_stride` floats apart, y [B, H e];
+// all of them but the state at multiples of 16 bytes (y of four elements).
+extern "C" int br_wkv_token(const float* rows, const float* w0, const float* bonus, float* state, const int* slots, const float* norm_w,
+                            const float* gate, size_t gate_stride, void* y, int y_is_bf16, int B, int H, int d, int e, int width,
+                            size_t slot_stride, float eps, hipStream_t s) {
+    if (B <= 0) return BR_OK;
+    const int rpl = glr_rpl(d);
+    if (!wkv_token_takes(d, e) || H <= 0 || H > 65535 || width < 3 * H * d + H * e || width % 4 || gate_stride % 4 ||
+        slot_stride < (size_t)H * (e / 4) * rpl * 64 || !norm_w || !gate || !w0 || !bonus ||
+        (((uintptr_t)rows | (uintptr_t)w0 | (uintptr_t)bonus | (uintptr_t)norm_w | (uintptr_t)gate) % 16) ||
+        (uintptr_t)y % (y_is_bf16 ? 8 : 16))
+        return BR_BAD_ARG;
+    const dim3 grid(B, H);
+#define WKV_TOKEN(R, C) do { \
+        if (y_is_bf16) wkv_token_kernel<R, C, bf16><<<grid, 256, 0, s>>>(rows, w0, bonus, state, slots, norm_w, gate, (bf16*)y, H, d, e, width, gate_stride, slot_stride, eps); \
+        else wkv_token_kernel<R, C, float><<<grid, 256, 0, s>>>(rows, w0, bonus, state, slots, norm_w, gate, (float*)y, H, d, e, width, gate_stride, slot_stride, eps); \
+    } while (0)
+    if (rpl == 4) { if (e <= 64) WKV_TOKEN(4, 4); else WKV_TOKEN(4, 8); }
+    else { if (e <= 64) WKV_TOKEN(8, 4); else WKV_TOKEN(8, 8); }
+#undef WKV_TOKEN
+    return br_check_launch();
+}
+
 // y = tanh(x) elementwise, float sums in, the products' type out (the middle of a low-rank projection).
 template <typename T>
 __global__ __launch_bounds__(256) void tanh_kernel(const float* __restrict__ x, T* __restrict__ y, size_t n) {

@@ -1041,12 +1041,15 @@ def head_rmsnorm(o: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, 
 
 # ------------------------------------------------- decayed recurrence with a bonus -----
 def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
-             cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int, below: int = 0) -> None:
+             cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int, below: int = 0, normed=None) -> None:
     """rows [T, >= 3*H*d + H*e] float, the projections' sums r | k | v | z (the decay is exp(-exp(z + w0)), made on the
     way); bonus float [H*d].  state [slots, n] float with a slot's first prod(glr_state_shape(H, d, e)) floats its S as
     `glr_scan` keeps it: walks every sequence's new tokens in order, o_t = (S + diag(bonus) k v^T)^T r before
     S <- diag(decay) S + k v^T, writes o [T, H*e] float and leaves the state.  `below` > 0: sequences of as many tokens or more
-    are left alone."""
+    are left alone.  `normed` = (norm_w, gate, y, eps), for steps of single tokens that `wkv_token_takes`: y is written by
+    `wkv_token` in place of `out`."""
+    if normed is not None:
+        return wkv_token(rows, w0, bonus, state, slots, normed[0], normed[1], normed[2], B, H, d, e, normed[3])
     _dev("wkv_scan", rows, w0, bonus, out, cu_seqlens, slots)
     T = rows.shape[0]
     need = 1
@@ -1063,6 +1066,33 @@ def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: tor
     f = _fn("gated_recurrence", "br_wkv_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, _P])
     _check(f(_ptr(rows), _ptr(w0), _ptr(bonus), _ptr(out), _ptr(state), _ptr(cu_seqlens), _ptr(slots), B, H, d, e,
              rows.shape[1], state.stride(0), int(below), _stream()), "wkv_scan")
+
+
+def wkv_token_takes(d: int, e: int) -> bool:
+    """Whether `wkv_token` takes heads of `d` key and `e` value channels."""
+    return 0 < d <= 128 and d % 4 == 0 and 0 < e <= 128 and e % 4 == 0
+
+
+def wkv_token(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, state: torch.Tensor, slots: torch.Tensor,
+              norm_w: torch.Tensor, gate: torch.Tensor, out: torch.Tensor, B: int, H: int, d: int, e: int, eps: float) -> None:
+    """`wkv_scan` of one token a sequence (row b of `rows` and `out` is sequence b's), then `head_norm_gate` with the weight
+    norm_w [H*e] and the gate [B, H*e] (silu), in one launch: out [B, H*e] in the compute dtype, the same bits as the two.
+    Rows and gate rows start at multiples of 16 bytes; padding sequences' rows of `out` are zero."""
+    _dev("wkv_token", rows, w0, bonus, slots, norm_w, out)
+    need = 1
+    for n in glr_state_shape(H, d, e):
+        need *= n
+    _req(state.is_cuda and state.dim() == 2 and state.shape[1] >= need and state.stride(1) == 1,
+         "wkv_token: state [slots, at least the head states' floats], every slot's dense")
+    _req(rows.dtype == state.dtype == torch.float32, "wkv_token: float32 only")
+    _req(rows.shape[0] == B and rows.shape[1] >= 3 * H * d + H * e and out.shape == (B, H * e), "wkv_token: rows [B, >= 3*H*d + H*e], out [B, H*e]")
+    for v, n in ((w0, H * d), (bonus, H * d), (norm_w, H * e)):
+        _req(v.dtype == torch.float32 and v.numel() == n, "wkv_token: w0 and bonus float32 [H*d], norm_w float32 [H*e]")
+    _req(gate.is_cuda and gate.dtype == torch.float32 and gate.shape == (B, H * e) and gate.stride(1) == 1, "wkv_token: gate float32 [B, H*e]")
+    _req(slots.numel() >= B, "wkv_token: arrays shorter than the batch")
+    f = _fn("gated_recurrence", "br_wkv_token", [_P] * 7 + [c_size_t, _P] + [c_int] * 6 + [c_size_t, c_float, _P])
+    _check(f(_ptr(rows), _ptr(w0), _ptr(bonus), _ptr(state), _ptr(slots), _ptr(norm_w), _ptr(gate), gate.stride(0), _ptr(out),
+             _is_bf16(out, "wkv_token"), B, H, d, e, rows.shape[1], state.stride(0), float(eps), _stream()), "wkv_token")
 
 
 def wkv_scan_pieces(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: torch.Tensor, state: torch.Tensor,

@@ -132,6 +132,9 @@ class WKVTimeMix(Mixer):
             linear(mixes[4], self.w["w1"], low, step.ws)
             K.tanh(low, low_t)
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
+        y = step.ws.get("wkv_y", (T, hd), dt)
+        gate = rows[:, 4 * hd:5 * hd]
+        one_launch = step.is_decode and T == step.n_seqs and K.wkv_token_takes(self.d, self.d)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
         pieces = pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
         chunks, walk, rest = in_chunks(step, self.d, self.d, pieces)
@@ -150,9 +153,9 @@ class WKVTimeMix(Mixer):
                               self.nh, self.d, self.d)
         if walk and (chunks or pieces == 1):
             K.wkv_scan(rows, self.w0, self.u, o, state, step.cu_seqlens, step.slots, step.n_seqs, self.nh, self.d, self.d,
-                       below=rest.get("below", 0))
-        y = step.ws.get("wkv_y", (T, hd), dt)
-        K.head_norm_gate(o, self.norm_w, rows[:, 4 * hd:5 * hd], y, self.nh, self.d, self.eps)
+                       below=rest.get("below", 0), normed=(self.norm_w, gate, y, self.eps) if one_launch else None)
+        if not one_launch:
+            K.head_norm_gate(o, self.norm_w, gate, y, self.nh, self.d, self.eps)
         linear(y, self.w_o, x, step.ws, accumulate=True)
 
 
