@@ -884,25 +884,33 @@ extern "C" int br_head_norm_gate(const float* o, const float* w, const float* ga
     return br_check_launch();
 }
 
-// ------------------------------------- single tokens of the recurrence with a bonus, normed and gated ------
-// The recurrence with a bonus, the head norm, its weight and the gate for steps of one token a sequence: token s is sequence s's.  A
+// ------------------------------------------------ single tokens of a recurrence, normed by heads ------
+// A recurrence of the two above, the head norm and its weight for steps of one token a sequence: token s is sequence s's.  A
 // workgroup takes a whole head, so that its output can be normed before it leaves; wave w walks the blocks of four columns w, w + 4, ...,
 // up to CB of them, all of whose state is asked for together with the rows, from memory straight into registers.  The arithmetic
-// and the order of every sum are those of `wkv_scan_kernel` and `head_norm_gate_kernel` (silu, 16-byte loads).  Bound by the
-// launch and one latency for few sequences, by the state, read and written once, for many (64 heads of 64 x 64, less than
-// the two launches in a recorded step: 2 us a layer for 1 sequence, 4 for 8, 11 for 24; those took 9.0 and 4.6 at 8).
-// Padding sequences' rows of y are zero.
-template <int RPL, int CB, typename T>
-__global__ __launch_bounds__(256) void wkv_token_kernel(
-    const float* __restrict__ rows, const float* __restrict__ w0, const float* __restrict__ bonus, float* __restrict__ state,
-    const int* __restrict__ slots, const float* __restrict__ norm_w, const float* __restrict__ gate, T* __restrict__ y,
-    int H, int d, int e, int width, size_t gate_stride, size_t slot_stride, float eps) {
+// and the order of every sum are those of the launches that it stands for: WKV: `wkv_scan_kernel` and `head_norm_gate_kernel`
+// (a weight per head, silu of the gate, 16-byte loads); else `glr_token_kernel` and `glr_head_norm_kernel`.  Bound by the
+// launch and one latency for few sequences, by the state, read and written once, for many (64 heads of 64 x 64 with a bonus, less than
+// the two launches in a recorded step: 2 us a layer for 1 sequence, 4 for 8, 11 for 24; those took 9.0 and 4.6 at 8.  32 heads of
+// 128 x 128 without: 4 us a layer for 8 sequences).  Padding sequences' rows of y are zero.
+struct HeadToken {
+    const float *rows, *b1, *b2;        // WKV: the decays' bias, the bonus; else the gates' bias and bounds (either null)
+    float* state;
+    const int* slots;
+    const float *norm_w, *gate;         // the gate: WKV only
+    int H, d, e, width;
+    size_t gate_stride, slot_stride;
+    float eps;
+};
+
+template <bool WKV, int RPL, int CB, typename T>
+__global__ __launch_bounds__(256) void head_token_kernel(const HeadToken p, T* __restrict__ y) {
     typedef T out_t __attribute__((ext_vector_type(4)));
     constexpr int NV = (CB + 3) / 4;
     __shared__ __attribute__((aligned(16))) float oL[16 * CB];
     const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int cg = lane >> 4, g = lane & 15;
-    const int slot = slots[s], ncb4 = e >> 2, hd = H * d;
+    const int cg = lane >> 4, g = lane & 15, H = p.H, d = p.d, e = p.e;
+    const int slot = p.slots[s], ncb4 = e >> 2, hd = H * d;
     out_t* yrow = (out_t*)(y + ((size_t)s * H + h) * e);
     if (slot < 0) {
         if (tid < ncb4) {
@@ -913,8 +921,8 @@ __global__ __launch_bounds__(256) void wkv_token_kernel(
         }
         return;
     }
-    const float* at = rows + (size_t)s * width;
-    float* S = state + (size_t)slot * slot_stride + (size_t)h * ncb4 * RPL * 64 + lane;
+    const float* at = p.rows + (size_t)s * p.width;
+    float* S = p.state + (size_t)slot * p.slot_stride + (size_t)h * ncb4 * RPL * 64 + lane;
     float st[CB][RPL], vc[CB];
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
@@ -936,35 +944,50 @@ __global__ __launch_bounds__(256) void wkv_token_kernel(
             for (int x = 0; x < 4; ++x) to[r4 + x] = w[x];
         }
     };
-    float rr[RPL], kk[RPL], ww[RPL], bb[RPL], uu[RPL];
+    // WKV: the receptance, the key, the decay and the bonus; else the query, the gate and its bound
+    float rr[RPL], kk[RPL], ww[RPL], uu[RPL], bb[RPL];
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) kk[k] = bb[k] = uu[k] = 0.f;
     row(rr, at);
-    row(kk, at + hd);
-    row(ww, at + 2 * hd + H * e);
-    row(bb, w0);
-    row(uu, bonus);
+    if (WKV) row(kk, at + hd);
+    row(ww, at + (WKV ? 2 * hd + H * e : hd));
+    if (WKV || p.b1) row(bb, p.b1);
+    if (WKV || p.b2) row(uu, p.b2);
     f32x4 z[NV], nw[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int i = g + 16 * j;
+        nw[j] = f32x4{1.f, 1.f, 1.f, 1.f};
         if (i < ncb4) {
-            z[j] = ((const f32x4*)(gate + (size_t)s * gate_stride + (size_t)h * e))[i];
-            nw[j] = ((const f32x4*)(norm_w + (size_t)h * e))[i];
+            if (WKV) z[j] = ((const f32x4*)(p.gate + (size_t)s * p.gate_stride + (size_t)h * e))[i];
+            if (WKV || p.norm_w) nw[j] = ((const f32x4*)(p.norm_w + (WKV ? (size_t)h * e : 0)))[i];
         }
     }
 #pragma unroll
     for (int k = 0; k < RPL; ++k) {
         const bool real = g * RPL + k < d;
-        ww[k] = real ? expf(-expf(ww[k] + bb[k])) : 1.f;
-        if (!real) rr[k] = kk[k] = uu[k] = 0.f;
+        if (WKV) {
+            ww[k] = real ? expf(-expf(ww[k] + bb[k])) : 1.f;
+            if (!real) rr[k] = kk[k] = uu[k] = 0.f;
+        } else {
+            rr[k] = real ? rr[k] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * rr[k])) : 0.f;
+            const float gt = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (ww[k] + bb[k])));
+            ww[k] = real ? uu[k] + (1.0f - uu[k]) * gt : 1.f;
+        }
     }
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
         float sum = 0.f;
 #pragma unroll
         for (int k = 0; k < RPL; ++k) {
-            const float kv = kk[k] * vc[i];
-            sum = fmaf(rr[k], fmaf(uu[k], kv, st[i][k]), sum);
-            st[i][k] = fmaf(ww[k], st[i][k], kv);
+            if (WKV) {
+                const float kv = kk[k] * vc[i];
+                sum = fmaf(rr[k], fmaf(uu[k], kv, st[i][k]), sum);
+                st[i][k] = fmaf(ww[k], st[i][k], kv);
+            } else {
+                st[i][k] = fmaf(ww[k], st[i][k] - vc[i], vc[i]);
+                sum = fmaf(st[i][k], rr[k], sum);
+            }
         }
         sum = glr_row16_sum(sum);
         if (g == 0) oL[(4 * i + wave) * 4 + cg] = sum;
@@ -986,46 +1009,68 @@ __global__ __launch_bounds__(256) void wkv_token_kernel(
         const int i = g + 16 * j;
         if (i < ncb4) {
             v[j] = *(const f32x4*)(oL + 4 * i);
+            if (WKV) {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) ss = fmaf(v[j][x], v[j][x], ss);
+                for (int x = 0; x < 4; ++x) ss = fmaf(v[j][x], v[j][x], ss);
+            } else
+                ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
         }
     }
-    const float inv = 1.0f / sqrtf(glr_row16_sum(ss) / (float)e + eps);
+    const float inv = 1.0f / sqrtf(glr_row16_sum(ss) / (float)e + p.eps);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int i = g + 16 * j;
         if (i < ncb4 && cg == 0) {
             out_t out;
 #pragma unroll
-            for (int x = 0; x < 4; ++x) out[x] = from_f32<T>(v[j][x] * inv * nw[j][x] * hng_gate(z[j][x], 0));
+            for (int x = 0; x < 4; ++x) {
+                float f = v[j][x] * inv * nw[j][x];
+                if (WKV) f *= hng_gate(z[j][x], 0);
+                out[x] = from_f32<T>(f);
+            }
             yrow[i] = out;
         }
     }
 }
 
-static bool wkv_token_takes(int d, int e) { return d > 0 && d <= 128 && d % 4 == 0 && e > 0 && e <= 128 && e % 4 == 0; }
+template <bool WKV>
+static int head_token_launch(const HeadToken& p, void* y, int y_is_bf16, int B, hipStream_t s) {
+    const int rpl = glr_rpl(p.d);
+    if (p.d <= 0 || p.d > 128 || p.d % 4 || p.e <= 0 || p.e > 128 || p.e % 4 || p.H <= 0 || p.H > 65535 || p.width % 4 ||
+        p.gate_stride % 4 || p.slot_stride < (size_t)p.H * (p.e / 4) * rpl * 64 ||
+        (((uintptr_t)p.rows | (uintptr_t)p.b1 | (uintptr_t)p.b2 | (uintptr_t)p.norm_w | (uintptr_t)p.gate) % 16) ||
+        (uintptr_t)y % (y_is_bf16 ? 8 : 16))
+        return BR_BAD_ARG;
+    const dim3 grid(B, p.H);
+#define HEAD_TOKEN(R, C) do { \
+        if (y_is_bf16) head_token_kernel<WKV, R, C, bf16><<<grid, 256, 0, s>>>(p, (bf16*)y); \
+        else head_token_kernel<WKV, R, C, float><<<grid, 256, 0, s>>>(p, (float*)y); \
+    } while (0)
+    if (rpl == 4) { if (p.e <= 64) HEAD_TOKEN(4, 4); else HEAD_TOKEN(4, 8); }
+    else { if (p.e <= 64) HEAD_TOKEN(8, 4); else HEAD_TOKEN(8, 8); }
+#undef HEAD_TOKEN
+    return br_check_launch();
+}
 
-// rows, w0, bonus, state and `slot_stride` as for `br_wkv_scan`, norm_w [H e], gate rows `gate_stride` floats apart, y [B, H e];
-// all of them but the state at multiples of 16 bytes (y of four elements).
+// d and e of at most 128 in steps of 4; rows, w0, bonus, state and `slot_stride` as for `br_wkv_scan`, norm_w [H e], gate rows
+// `gate_stride` floats apart, y [B, H e]; all of them but the state at multiples of 16 bytes (y of four elements).
 extern "C" int br_wkv_token(const float* rows, const float* w0, const float* bonus, float* state, const int* slots, const float* norm_w,
                             const float* gate, size_t gate_stride, void* y, int y_is_bf16, int B, int H, int d, int e, int width,
                             size_t slot_stride, float eps, hipStream_t s) {
     if (B <= 0) return BR_OK;
-    const int rpl = glr_rpl(d);
-    if (!wkv_token_takes(d, e) || H <= 0 || H > 65535 || width < 3 * H * d + H * e || width % 4 || gate_stride % 4 ||
-        slot_stride < (size_t)H * (e / 4) * rpl * 64 || !norm_w || !gate || !w0 || !bonus ||
-        (((uintptr_t)rows | (uintptr_t)w0 | (uintptr_t)bonus | (uintptr_t)norm_w | (uintptr_t)gate) % 16) ||
-        (uintptr_t)y % (y_is_bf16 ? 8 : 16))
-        return BR_BAD_ARG;
-    const dim3 grid(B, H);
-#define WKV_TOKEN(R, C) do { \
-        if (y_is_bf16) wkv_token_kernel<R, C, bf16><<<grid, 256, 0, s>>>(rows, w0, bonus, state, slots, norm_w, gate, (bf16*)y, H, d, e, width, gate_stride, slot_stride, eps); \
-        else wkv_token_kernel<R, C, float><<<grid, 256, 0, s>>>(rows, w0, bonus, state, slots, norm_w, gate, (float*)y, H, d, e, width, gate_stride, slot_stride, eps); \
-    } while (0)
-    if (rpl == 4) { if (e <= 64) WKV_TOKEN(4, 4); else WKV_TOKEN(4, 8); }
-    else { if (e <= 64) WKV_TOKEN(8, 4); else WKV_TOKEN(8, 8); }
-#undef WKV_TOKEN
-    return br_check_launch();
+    if (!norm_w || !gate || !w0 || !bonus || width < 3 * H * d + H * e) return BR_BAD_ARG;
+    const HeadToken p = {rows, w0, bonus, state, slots, norm_w, gate, H, d, e, width, gate_stride, slot_stride, eps};
+    return head_token_launch<true>(p, y, y_is_bf16, B, s);
+}
+
+// The same for `br_glr_scan` with `br_glr_head_norm`: f_bias and lower [H d] or null, norm_w [e] or null.
+extern "C" int br_glr_token(const float* rows, const float* f_bias, const float* lower, float* state, const int* slots,
+                            const float* norm_w, void* y, int y_is_bf16, int B, int H, int d, int e, int width,
+                            size_t slot_stride, float eps, hipStream_t s) {
+    if (B <= 0) return BR_OK;
+    if (width < 2 * H * d + H * e) return BR_BAD_ARG;
+    const HeadToken p = {rows, f_bias, lower, state, slots, norm_w, nullptr, H, d, e, width, 0, slot_stride, eps};
+    return head_token_launch<false>(p, y, y_is_bf16, B, s);
 }
 
 // y = tanh(x) elementwise, float sums in, the products' type out (the middle of a low-rank projection).

@@ -927,11 +927,14 @@ def glr_state_dense(state: torch.Tensor, H: int, d: int, e: int) -> torch.Tensor
 
 def glr_scan(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], out: torch.Tensor,
              state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, B: int, H: int, d: int, e: int,
-             below: int = 0, singles: Optional[bool] = None) -> None:
+             below: int = 0, singles: Optional[bool] = None, normed=None) -> None:
     """rows [T, 2*H*d + H*e] float, the projections' sums q | f | v; q = silu(.), f = lower + (1 - lower) *
     sigmoid(. + f_bias) are applied on the way.  state [slots, *glr_state_shape]: walks every sequence's new
     tokens in order, writes o [T, H*e] float and leaves the state.  `below` > 0: sequences of as many tokens or more are left
-    alone; `singles`: the others bring a token each (None: told by T and B)."""
+    alone; `singles`: the others bring a token each (None: told by T and B).  `normed` = (norm_w, y, eps), for steps of single
+    tokens that `head_token_takes`: y is written by `glr_token` in place of `out`."""
+    if normed is not None:
+        return glr_token(rows, f_bias, lower, state, slots, normed[0], normed[1], B, H, d, e, normed[2])
     _dev("glr_scan", rows, f_bias, lower, out, cu_seqlens, slots)
     T = rows.shape[0]
     _req(state.is_cuda and state.shape[1:] == glr_state_shape(H, d, e) and state[0].is_contiguous(),
@@ -945,6 +948,24 @@ def glr_scan(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional
     f = _fn("gated_recurrence", "br_glr_scan", [_P, _P, _P, _P, _P, _P, _P] + [c_int] * 5 + [c_size_t, c_int, c_int, _P])
     _check(f(_ptr(rows), _ptr(f_bias), _ptr(lower), _ptr(out), _ptr(state), _ptr(cu_seqlens), _ptr(slots), B, H, d, e,
              rows.shape[1], state.stride(0), int(T <= B if singles is None else singles), int(below), _stream()), "glr_scan")
+
+
+def glr_token(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], state: torch.Tensor,
+              slots: torch.Tensor, norm_w: Optional[torch.Tensor], out: torch.Tensor, B: int, H: int, d: int, e: int, eps: float) -> None:
+    """`glr_scan` of one token a sequence (row b of `rows` and `out` is sequence b's), then `head_rmsnorm` with the weight
+    norm_w [e], in one launch: out [B, H*e] in the compute dtype, the same bits as the two; padding sequences' rows of `out`
+    are zero."""
+    _dev("glr_token", rows, f_bias, lower, slots, norm_w, out)
+    _req(state.is_cuda and state.shape[1:] == glr_state_shape(H, d, e) and state[0].is_contiguous(),
+         "glr_token: state [slots, H, ceil(e/4), rows per lane, 64], every slot's dense")
+    _req(rows.dtype == state.dtype == torch.float32, "glr_token: float32 only")
+    _req(rows.shape == (B, 2 * H * d + H * e) and out.shape == (B, H * e), "glr_token: rows [B, 2*H*d + H*e], out [B, H*e]")
+    for v, n in ((f_bias, H * d), (lower, H * d), (norm_w, e)):
+        _req(v is None or (v.dtype == torch.float32 and v.numel() == n), "glr_token: bias and lower bound float32 [H*d], norm_w float32 [e]")
+    _req(slots.numel() >= B, "glr_token: arrays shorter than the batch")
+    f = _fn("gated_recurrence", "br_glr_token", [_P] * 7 + [c_int] * 6 + [c_size_t, c_float, _P])
+    _check(f(_ptr(rows), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots), _ptr(norm_w), _ptr(out), _is_bf16(out, "glr_token"),
+             B, H, d, e, rows.shape[1], state.stride(0), float(eps), _stream()), "glr_token")
 
 
 def glr_scan_pieces(rows: torch.Tensor, f_bias: Optional[torch.Tensor], lower: Optional[torch.Tensor], out: torch.Tensor,
@@ -1046,7 +1067,7 @@ def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: tor
     way); bonus float [H*d].  state [slots, n] float with a slot's first prod(glr_state_shape(H, d, e)) floats its S as
     `glr_scan` keeps it: walks every sequence's new tokens in order, o_t = (S + diag(bonus) k v^T)^T r before
     S <- diag(decay) S + k v^T, writes o [T, H*e] float and leaves the state.  `below` > 0: sequences of as many tokens or more
-    are left alone.  `normed` = (norm_w, gate, y, eps), for steps of single tokens that `wkv_token_takes`: y is written by
+    are left alone.  `normed` = (norm_w, gate, y, eps), for steps of single tokens that `head_token_takes`: y is written by
     `wkv_token` in place of `out`."""
     if normed is not None:
         return wkv_token(rows, w0, bonus, state, slots, normed[0], normed[1], normed[2], B, H, d, e, normed[3])
@@ -1068,8 +1089,8 @@ def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: tor
              rows.shape[1], state.stride(0), int(below), _stream()), "wkv_scan")
 
 
-def wkv_token_takes(d: int, e: int) -> bool:
-    """Whether `wkv_token` takes heads of `d` key and `e` value channels."""
+def head_token_takes(d: int, e: int) -> bool:
+    """Whether `wkv_token` and `glr_token` take heads of `d` key and `e` value channels."""
     return 0 < d <= 128 and d % 4 == 0 and 0 < e <= 128 and e % 4 == 0
 
 

@@ -160,6 +160,8 @@ class HGRN2(Mixer):
         rows = step.ws.get("glr_qfv", (T, 2 * nh * d + nh * e), torch.float32)
         linear(h, self.w_qfv, rows, step.ws)
         o = step.ws.get("glr_o", (T, nh * e), torch.float32)
+        on = step.ws.get("glr_on", (T, nh * e), self.rt.dtype)
+        one_launch = step.is_decode and T == step.n_seqs and K.head_token_takes(d, e)
         pieces = self.pieces_for(step)
         chunks, walk, rest = in_chunks(step, d, e, pieces)
         if chunks:
@@ -175,9 +177,10 @@ class HGRN2(Mixer):
             K.glr_scan_pieces(rows, self.f_bias, self.lower, o, ctx.state, step.slots, cu, numbers, piece_state, decay,
                               step.n_seqs, pieces, nh, d, e)
         if walk and (chunks or pieces == 1):
-            K.glr_scan(rows, self.f_bias, self.lower, o, ctx.state, step.cu_seqlens, step.slots, step.n_seqs, nh, d, e, **rest)
-        on = step.ws.get("glr_on", (T, nh * e), self.rt.dtype)
-        K.head_rmsnorm(o, self.norm_w, on, nh, e, self.eps)
+            K.glr_scan(rows, self.f_bias, self.lower, o, ctx.state, step.cu_seqlens, step.slots, step.n_seqs, nh, d, e,
+                       normed=(self.norm_w, on, self.eps) if one_launch else None, **rest)
+        if not one_launch:
+            K.head_rmsnorm(o, self.norm_w, on, nh, e, self.eps)
         linear(on, self.w_o, x, step.ws, accumulate=True)
 
 
