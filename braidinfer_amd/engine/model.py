@@ -37,6 +37,7 @@ class Layer:
         # an arrangement is an object with `run` (and optionally `first_norm`), or a plain function
         self.run = getattr(arrangement, "run", arrangement)
         self._first_norm = getattr(arrangement, "first_norm", None)
+        self._rows_norm = getattr(arrangement, "rows_norm", None)
         self._opening = getattr(arrangement, "opening", None)
         self.takes_streams = bool(getattr(arrangement, "takes_streams", False))
         self.rt: Optional[Runtime] = None
@@ -54,6 +55,11 @@ class Layer:
         """The norm that reads the residual rows first when this layer runs, if its
         arrangement says."""
         return self._first_norm(self) if self._first_norm is not None else None
+
+    def rows_norm(self):
+        """The norm that reads the residual rows first when this layer runs, if its arrangement takes the normed rows
+        themselves from the layer before."""
+        return self._rows_norm(self) if self._rows_norm is not None else None
 
     def opening(self):
         """(connection, norm) through which the layer's first half reads a residual of several streams, or None."""

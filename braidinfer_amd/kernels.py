@@ -1554,12 +1554,20 @@ def experts_gather(h: torch.Tensor, order: torch.Tensor, rows: torch.Tensor, top
     _check(f(_ptr(h), _ptr(order), _ptr(n_rows), _ptr(rows), _is_bf16(h, "experts_gather"), n, W, top, _stream()), "experts_gather")
 
 
+def experts_combine_norms(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `experts_combine` takes `then` for these rows and this norm weight."""
+    W = x.shape[1]
+    return (W % 4 == 0 and W <= 16 * (256 if W >= 2048 else 128 if W >= 512 else 64) and w.dtype == torch.float32 and w.numel() == W
+            and (out.data_ptr() | x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
 def experts_combine(out: torch.Tensor, place: torch.Tensor, share: torch.Tensor, x: torch.Tensor,
                     chosen: Optional[torch.Tensor] = None, h: Optional[torch.Tensor] = None, experts: int = 0,
-                    store: bool = False) -> None:
+                    store: bool = False, then=None) -> None:
     """x[t] += sum_s share[t, s] * out[place[t * top + s]] (`store`: = instead of +=); out float [T * top, W].  With `chosen`
     [T, top] and `h` [T, W], a slot whose number is `experts` or more (an identity expert) takes h[t] instead of an output.
-    Tokens that `experts_sort` left out (place -1) add nothing (`store`: zeros)."""
+    Tokens that `experts_sort` left out (place -1) add nothing (`store`: zeros).  `then` = (w, eps, y), without those two and where
+    `experts_combine_norms` says so: also y = x / rms(x) * w of the new rows, as `rmsnorm` would store it."""
     _dev("experts_combine", out, place, share, x, chosen, h)
     _req((chosen is None) == (h is None) and (chosen is None or (chosen.dtype == torch.int32 and chosen.shape == share.shape and h.shape == x.shape)),
          "experts_combine: chosen int32 [T, top] and h [T, W] come together")
@@ -1567,6 +1575,14 @@ def experts_combine(out: torch.Tensor, place: torch.Tensor, share: torch.Tensor,
     W = x.shape[1]
     _req(out.dtype == x.dtype == share.dtype == torch.float32 and place.dtype == torch.int32 and out.shape == (T * top, W)
          and x.shape == (T, W) and place.numel() == T * top, "experts_combine: shapes")
+    if then is not None:
+        w, eps, y = then
+        _dev("experts_combine", w, y)
+        _req(chosen is None and not store and y.shape == x.shape and experts_combine_norms(out, x, w), "experts_combine: then")
+        f = _fn("routed_experts", "br_experts_combine_norm", [_P] * 6 + [c_int] * 4 + [c_float, _P])
+        _check(f(_ptr(out), _ptr(place), _ptr(share), _ptr(x), _ptr(w), _ptr(y), _is_bf16(y, "experts_combine"), T, W, top, float(eps),
+                 _stream()), "experts_combine")
+        return
     f = _fn("routed_experts", "br_experts_combine", [_P, _P, _P, _P, _P, c_int, _P] + [c_int] * 5 + [_P])
     _check(f(_ptr(out), _ptr(place), _ptr(share), _ptr(chosen), _ptr(h), 0 if h is None else _is_bf16(h, "experts_combine"), _ptr(x),
              T, W, top, int(experts), int(store), _stream()), "experts_combine")

@@ -82,6 +82,9 @@ class Part:
     # arrangement wants a branch's own output, it is handed a `ResidualSink` with `overwrite` over rows that hold nothing
     # yet (without it, rows of zeros).
     stores_output = False
+    # a part that, given a `ResidualSink` with the norm that reads the rows next, may leave the normed rows themselves in
+    # `prepared`, as ("normed", rows)
+    norms_rows = False
 
     def weight_specs(self, prefix: str) -> List[TensorSpec]:
         return []

@@ -31,7 +31,10 @@ def run_residual_branch(part, norm, next_norm, x, step, dtype, *extra) -> None:
         if norm is not None:
             h = step.ws.get("block_h", tuple(x.shape), dtype)
             norm.forward(x, h)
-        part.forward(h, x, step, *extra)
+        if extra:
+            part.forward(h, x, step, *extra)
+        else:
+            into_rows(part, h, x, step)
         return
     h = x
     if norm is not None:
@@ -43,6 +46,27 @@ def run_residual_branch(part, norm, next_norm, x, step, dtype, *extra) -> None:
     part.forward(h, sink, step, *extra)
     if sink.prepared is not None:
         step.prepared_norm = (next_norm, x, sink.prepared)
+
+
+def ready_rows(prepared, norm, x):
+    """norm(x) where the layer before left the normed rows themselves, else None."""
+    if norm is not None and prepared is not None and prepared[0] is norm and prepared[1] is x \
+            and isinstance(prepared[2], tuple) and isinstance(prepared[2][0], str) and prepared[2][0] == "normed":
+        return prepared[2][1]
+    return None
+
+
+def into_rows(part, h, x, step) -> None:
+    """x += part(h) of a layer's last half; a part that can leaves the rows normed as the next layer's arrangement reads them."""
+    layer = getattr(step, "next_layer", None)
+    norm = layer.rows_norm() if layer is not None and getattr(part, "norms_rows", False) else None
+    if norm is None:
+        part.forward(h, x, step)
+        return
+    sink = ResidualSink(x, norm)
+    part.forward(h, sink, step)
+    if sink.prepared is not None:
+        step.prepared_norm = (norm, x, sink.prepared)
 
 
 class PrenormResidual:
@@ -124,20 +148,25 @@ class ParallelResidual:
     def first_norm(self, layer):
         return None          # the norm's output is kept for both halves: nothing a product before could prepare in passing
 
+    def rows_norm(self, layer):
+        return layer.norms.get("mixer")
+
     def run(self, layer, x, step, mixer_ctx) -> None:
-        step.prepared_norm = None
+        prepared, step.prepared_norm = step.prepared_norm, None
         dtype = layer.rt.dtype
         norm = layer.norms.get("mixer")
-        h = x
-        if norm is not None:
-            h = step.ws.get("block_h", tuple(x.shape), dtype)
-            norm.forward(x, h)
+        h = ready_rows(prepared, norm, x)
+        if h is None:
+            h = x
+            if norm is not None:
+                h = step.ws.get("block_h", tuple(x.shape), dtype)
+                norm.forward(x, h)
         if layer.mixer is not None:
             layer.mixer.forward(h, x, step, mixer_ctx)
         if step.probe is not None:
             step.probe(f"L{step.schedule_index}.post_mixer", x)
         if layer.feed_forward is not None:
-            layer.feed_forward.forward(h, x, step)
+            into_rows(layer.feed_forward, h, x, step)
         if step.probe is not None:
             step.probe(f"L{step.schedule_index}.post_ffn", x)
 
@@ -153,14 +182,19 @@ class PrenormSideBySide:
     def first_norm(self, layer):
         return None          # the norm's output is kept for all mixers: nothing a product before could prepare in passing
 
+    def rows_norm(self, layer):
+        return layer.norms.get("mixer")
+
     def run(self, layer, x, step, mixer_ctx) -> None:
-        step.prepared_norm = None
+        prepared, step.prepared_norm = step.prepared_norm, None
         dtype = layer.rt.dtype
         norm = layer.norms.get("mixer")
-        h = x
-        if norm is not None:
-            h = step.ws.get("block_h", tuple(x.shape), dtype)
-            norm.forward(x, h)
+        h = ready_rows(prepared, norm, x)
+        if h is None:
+            h = x
+            if norm is not None:
+                h = step.ws.get("block_h", tuple(x.shape), dtype)
+                norm.forward(x, h)
         mixers = ([(None, layer.mixer, mixer_ctx)] if layer.mixer is not None else []) + \
                  [(role, m, mixer_ctx.others[role]) for role, m in layer.more_mixers.items()]
         for role, mixer, ctx in mixers:

@@ -133,6 +133,7 @@ class ClampedGLU(FeedForward):
 class RoutedExperts(FeedForward):
     graph_safe = True
     stores_output = True
+    norms_rows = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, num_experts: int, top: int, router_bias: bool = True,
                  names: Optional[Dict[str, str]] = None, out_scale: float = 1.0, scoring: str = "softmax",
@@ -244,6 +245,19 @@ class RoutedExperts(FeedForward):
         else:
             K.silu_mul(gu, act)
 
+    def _join(self, out, place, share, x, rows_in, step, sink, **how) -> None:
+        """The experts' outputs into the rows, and the rows normed as they are read next where the sink asks for that."""
+        norm = sink.next_norm if sink is not None and not sink.overwrite else None
+        then = norm.then_args() if norm is not None else None
+        if then is None or then[2] or how["store"] or "chosen" in how or not K.experts_combine_norms(out, x, then[0]):
+            K.experts_combine(out, place, share, x, **how)
+            return
+        # two buffers in turn: whoever called may still read the rows that came in
+        name = "block_h2" if rows_in.data_ptr() == step.ws.get("block_h", tuple(x.shape), self.rt.dtype).data_ptr() else "block_h"
+        rows = step.ws.get(name, tuple(x.shape), self.rt.dtype)
+        K.experts_combine(out, place, share, x, then=(then[0], then[1], rows))
+        sink.prepared = ("normed", rows)
+
     def forward(self, h, x, step) -> None:
         T, dt = step.n_tokens, self.rt.dtype
         # rows that are to be stored rather than added to: the first of the two parts stores, the other adds
@@ -268,7 +282,7 @@ class RoutedExperts(FeedForward):
         else:
             K.route_topk(scores, self.b_router, chosen, share, self.top, self.out_scale)
         if self.shared is not None:                  # every token's: joins like the experts' outputs
-            to = x if sink is None else sink
+            to = sink if sink is not None and sink.overwrite else x
             if self.shared_gate:
                 self.shared.forward(h, to, step, row_gate=scores[:, self.n_out])
             else:
@@ -315,7 +329,7 @@ class RoutedExperts(FeedForward):
                 K.experts_gemm(y, self.w_down, first, out)
             else:
                 K.experts_down_grouped(y, self.w_down, first, out, T)
-            K.experts_combine(out, place, share, x, store=store, **ident)
+            self._join(out, place, share, x, h, step, sink, store=store, **ident)
             return
         # widths and steps that the tiles do not take, and the 32-bit path
         rows = step.ws.get("moe_rows", (n, self.H), dt)
@@ -341,7 +355,7 @@ class RoutedExperts(FeedForward):
                     K.gemm(rows[a:b], self.w_gu[e], gu[a:b], scratch=sc)
                     self._glu(gu[a:b], act[a:b])
                     K.gemm(act[a:b], self.w_down[e], out[a:b], scratch=sc)
-        K.experts_combine(out, place, share, x, store=store, **ident)
+        self._join(out, place, share, x, h, step, sink, store=store, **ident)
 
 
 register_part("feed_forward", "swiglu", SwiGLU, replace=True)

@@ -291,6 +291,32 @@ def test_combine_adds_every_slot(top, W):
         assert ((got.cpu().double() - want).abs() <= (top + 1) * 2 ** -23 * (terms.abs().sum(1) + x.abs().double())).all()
 
 
+@pytest.mark.parametrize("top", [1, 4, 5, 8])
+@pytest.mark.parametrize("W,dtype", [(4, torch.bfloat16), (512, torch.float32), (1024, torch.bfloat16), (2044, torch.bfloat16),
+                                     (2048, torch.bfloat16), (4096, torch.bfloat16), (4096, torch.float32)])
+def test_combine_with_the_norm_behind_it(W, dtype, top):
+    """The sum and the norm in one launch: the bits of the two, at widths around the workgroups' sizes; a token without outputs."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(top + W)
+    T = 6
+    out, share, x = (torch.randn(s, generator=g).cuda() for s in ((T * top, W), (T, top), (T, W)))
+    place = torch.randperm(T * top, generator=g).int().reshape(T, top)
+    place[2] = -1
+    place, w = place.reshape(-1).cuda(), (1 + torch.randn(W, generator=g) / 4).cuda()
+    assert K.experts_combine_norms(out, x, w)
+    x2, y, y2 = x.clone(), torch.empty(T, W, dtype=dtype, device="cuda"), torch.empty(T, W, dtype=dtype, device="cuda")
+    K.experts_combine(out, place, share, x)
+    K.rmsnorm(x, w, y, 1e-5)
+    K.experts_combine(out, place, share, x2, then=(w, 1e-5, y2))
+    assert torch.equal(x, x2) and torch.equal(y, y2)
+
+
+def test_combine_without_room_for_the_norm():
+    from braidinfer_amd import kernels as K
+    for W in (6, 2046, 4100, 8192):          # not in steps of 4, or beyond 16 floats a thread of 256
+        assert not K.experts_combine_norms(torch.empty(2, W), torch.empty(2, W), torch.empty(W))
+
+
 def test_rows_beyond_4_gb():
     """The second product of a step whose pairs' rows take more than 4 GB: the first and the last rows of every expert."""
     from braidinfer_amd import kernels as K
