@@ -908,16 +908,11 @@ __global__ __launch_bounds__(64 * PWA_DW) void pwa_decode_kernel(
     const int n_blocks = far_blocks + kept_blocks + (pq - kb0) / 32 + 1;
     const int* bt = block_table + (size_t)slot * table_stride;
     const int* pt = pooled_table ? pooled_table + (size_t)slot * pooled_stride : nullptr;
-    // a block's first row in its unit, and its page's number: asked for a block ahead, as the page's reads wait for it
-    auto row_of = [&](int n) { return n < far_blocks ? n * 32 : n < far_blocks + kept_blocks ? (n - far_blocks) * 32 : kb0 + (n - far_blocks - kept_blocks) * 32; };
-    auto page_of = [&](int n) { return (n < far_blocks ? pt : bt)[row_of(n) / PWA_PAGE]; };
-    int page = wave < n_blocks ? page_of(wave) : 0;
     for (int n = wave; n < n_blocks; n += PWA_DW) {
         const bool far = n < far_blocks, early = !far && n < far_blocks + kept_blocks;
-        const int kb = row_of(n), kl = kb % PWA_PAGE;
-        const bf16* pg = (far ? pooled : storage) + (size_t)page * page_elems;
-        __builtin_amdgcn_sched_barrier(0);
-        if (n + PWA_DW < n_blocks) page = page_of(n + PWA_DW);
+        const int kb = far ? n * 32 : (early ? (n - far_blocks) * 32 : kb0 + (n - far_blocks - kept_blocks) * 32);
+        const int kl = kb % PWA_PAGE;
+        const bf16* pg = far ? pooled + (size_t)pt[kb / PWA_PAGE] * page_elems : storage + (size_t)bt[kb / PWA_PAGE] * page_elems;
         const int limit = (far ? ctx / pool : ctx) - (kb - kl);
         const int first_ok = row_ok ? ((far || early) ? 0 : lo) : 1, last_ok = row_ok ? (far ? seen - 1 : (early ? kept - 1 : pq)) : 0;
         pwa_block<NBK, NBV, EARLY>(pg + k_off + (size_t)kl * dk, dk, pg + v_off + (size_t)ch0 * PWA_PAGE + kl, PWA_PAGE, kb, limit - kl, first_ok, last_ok,
