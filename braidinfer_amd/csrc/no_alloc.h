@@ -10,7 +10,7 @@
 //
 // Limits: nsplit == 1, or  roundup64(B * nq * nsplit * hd) + B * nq * nsplit * 2
 // <= BR_NO_ALLOC_SCRATCH_FLOATS; beyond that it returns BR_TOO_LARGE and prints why.
-// Nothing in the scratch has to start at zero: every run writes its partial sums before
+// Nothing in the scratch has to start at zero: every run writes its maximum and sum (with a page, its outputs too) before
 // the combining kernel reads them, so the contents a call leaves behind do no harm.
 // Every call on one GPU uses that GPU's one array: calls that overlap on a GPU (two
 // streams, two threads) race on it and must be ordered by the caller.

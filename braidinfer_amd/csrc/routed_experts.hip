@@ -616,8 +616,8 @@ extern "C" int br_experts_combine(const float* out, const int* place, const floa
 
 // The same without identity experts, x += ..., and the RMS norm of the new row behind it: y[t, :] = x[t, :] / rms(x[t, :]) * w.  One
 // workgroup a token, in the row norm's own partition and order of sums, the slots added in slot order: the bits of the two launches.
-// Bound by memory, or by its latency for few tokens; what is saved is the second
-// launch and its read of the rows (1,801 tokens of 4,096: 9 of 66 us; seven layers of such experts 10,682 -> 10,594 us in all).
+// Bound by memory, or by its latency for few tokens; what is saved is the second launch and its read of the rows (1,801
+// tokens of 4,096: 9 of 66 us; eight layers, seven of such experts, 10,682 -> 10,594 us in all).
 template <typename T>
 __global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* __restrict__ out, const int* __restrict__ place,
                                                                    const float* __restrict__ share, float* __restrict__ x,
