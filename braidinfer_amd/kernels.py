@@ -1089,9 +1089,11 @@ def wkv_scan(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, out: tor
              rows.shape[1], state.stride(0), int(below), _stream()), "wkv_scan")
 
 
-def head_token_takes(d: int, e: int) -> bool:
-    """Whether `wkv_token` and `glr_token` take heads of `d` key and `e` value channels."""
-    return 0 < d <= 128 and d % 4 == 0 and 0 < e <= 128 and e % 4 == 0
+def head_token_takes(d: int, e: int, *tensors) -> bool:
+    """Whether `wkv_token` and `glr_token` take heads of `d` key and `e` value channels, with `tensors` (all they are given
+    but the state and the slots; None: absent), which they read and write 16 bytes at a time."""
+    return (0 < d <= 128 and d % 4 == 0 and 0 < e <= 128 and e % 4 == 0
+            and all(t is None or t.data_ptr() % 16 == 0 for t in tensors))
 
 
 def wkv_token(rows: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, state: torch.Tensor, slots: torch.Tensor,

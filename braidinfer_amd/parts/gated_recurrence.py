@@ -161,7 +161,7 @@ class HGRN2(Mixer):
         linear(h, self.w_qfv, rows, step.ws)
         o = step.ws.get("glr_o", (T, nh * e), torch.float32)
         on = step.ws.get("glr_on", (T, nh * e), self.rt.dtype)
-        one_launch = step.is_decode and T == step.n_seqs and K.head_token_takes(d, e)
+        one_launch = step.is_decode and T == step.n_seqs and K.head_token_takes(d, e, rows, self.f_bias, self.lower, self.norm_w, on)
         pieces = self.pieces_for(step)
         chunks, walk, rest = in_chunks(step, d, e, pieces)
         if chunks:

@@ -134,7 +134,7 @@ class WKVTimeMix(Mixer):
         linear(low_t, self.w["w2"], rows[:, 3 * hd:4 * hd], step.ws)
         y = step.ws.get("wkv_y", (T, hd), dt)
         gate = rows[:, 4 * hd:5 * hd]
-        one_launch = step.is_decode and T == step.n_seqs and K.head_token_takes(self.d, self.d)
+        one_launch = step.is_decode and T == step.n_seqs and K.head_token_takes(self.d, self.d, rows, self.w0, self.u, self.norm_w, y)
         o = step.ws.get("wkv_o", (T, hd), torch.float32)
         pieces = pieces_for(step, self.nh * -(-self.d // 16), self.MIN_PIECE)
         chunks, walk, rest = in_chunks(step, self.d, self.d, pieces)

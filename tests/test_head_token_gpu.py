@@ -65,3 +65,9 @@ def test_single_tokens_without_a_bonus(H, d, e, dtype, biased):
 @pytest.mark.parametrize("d,e", [(130, 64), (64, 132), (6, 8), (8, 6), (0, 8)])
 def test_other_widths_are_refused(d, e):
     assert not K.head_token_takes(d, e)
+
+
+def test_vectors_at_odd_places_are_refused():
+    """A checkpoint's vectors may be views that start anywhere."""
+    v = torch.zeros(132, device="cuda")
+    assert K.head_token_takes(64, 64, v, None, v[4:68]) and not K.head_token_takes(64, 64, v, v[1:65])
