@@ -1,5 +1,7 @@
 """Products by workgroups that hold a tile of 16, 24 or 32 weight rows over the whole of K: against double sums, at the edges
 of tiles, rows and chunks, and where the rule takes them."""
+import ctypes
+
 import pytest
 import torch
 
@@ -106,6 +108,33 @@ def test_a_norm_prepared_and_used(M, H, Kd, N2, swiglu):
         out = torch.empty(M, N2, device="cuda")
         K.gemm_norm_scaled(xg, ssq, tiles, 1e-5, w2, out, scratch=scratch, whole=True)
         assert off(out, want) < bound(H)
+
+
+# widths that end in the middle of a tile of 32: nothing is written behind the last column, row or tile of squares
+@pytest.mark.parametrize("M", [1, 8, 16, 24, 64])
+@pytest.mark.parametrize("H", [4112, 5200, 8176])
+def test_a_norm_prepared_up_to_the_last_column(M, H):
+    from braidinfer_amd import kernels as K
+    a, _, w, y = operands(M, H, 1024, M)
+    x0, gain = torch.randn(M, H, device="cuda"), 1.0 + 0.2 * torch.randn(H, device="cuda")
+    P, I, Z = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
+    prepare = K._fn("gemm_bf16", "br_gemm_bf16_norm_prepare", [P, P, P, I, I, I, Z, Z, P, P, Z, P, ctypes.POINTER(I), P, Z, I, I, P])
+    for dense in (True, False):                          # the next row's first columns behind a row's last, or a margin
+        width = H if dense else H + 64
+        x = torch.full((M + 1, width), 7.0, device="cuda")
+        xg = torch.full((M + 1, width), 7.0, dtype=torch.bfloat16, device="cuda")
+        ssq = torch.full(((H // 16 + 2) * K.SSQ_LD,), 7.0, device="cuda")
+        x[:M, :H] = x0
+        tiles = ctypes.c_int(0)                          # (rows in a wider room are for the C entry: the Python one takes dense rows)
+        assert prepare(a.data_ptr(), w.data_ptr(), x.data_ptr(), M, H, 1024, 1024, width, gain.data_ptr(), xg.data_ptr(), width, ssq.data_ptr(),
+                       ctypes.byref(tiles), None, 0, 0, 1, torch.cuda.current_stream().cuda_stream) == 0
+        assert tiles.value == H // 16 and K.gemm_whole_pays(M, H, 1024, by16=True)
+        assert off(x[:M, :H], x0.double() + y) < bound(1024)
+        assert torch.equal(xg[:M, :H], (x[:M, :H] * gain).to(torch.bfloat16))
+        squares = ssq.view(-1, K.SSQ_LD)[:H // 16, :M].double().sum(0)
+        assert float((squares / (x[:M, :H].double() ** 2).sum(1) - 1).abs().max()) < bound(H)
+        for t in (x[:, H:], x[M], xg[:, H:], xg[M], ssq[H // 16 * K.SSQ_LD:]):
+            assert bool((t == 7.0).all())
 
 
 @pytest.mark.parametrize("M,N,K_,pays", [(8, 6144, 4096, True), (8, 8192, 4096, True), (8, 8208, 4096, True), (16, 5120, 13824, True), (1, 28672, 4096, True), (24, 4096, 4096, True),
