@@ -2341,6 +2341,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
             for (int c = wave; c < nrm.ssq_tiles; c += NW) t += nrm.ssq[(size_t)c * SSQ_LD + lane];
         }
         sq[tid] = t;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the barrier in front of the first chunk publishes it: units may have one chunk
     }
     if (my_units > 0) WIDE_RUN_LENGTH(0, cp_left);
     while (cp_u < my_units) {

@@ -137,6 +137,22 @@ def test_a_norm_prepared_up_to_the_last_column(M, H):
             assert bool((t == 7.0).all())
 
 
+# K of 7 and 13 chunks in runs of 3 and 4: the last run of a tile has a single chunk, and 1 / rms of a row is added up beside it
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K_,runs", [(2048, 896, 3), (4096, 896, 3), (4096, 1664, 4)])
+def test_a_prepared_norm_over_runs_of_one_chunk(M, N, K_, runs):
+    from braidinfer_amd import kernels as K
+    xg, _, w, y = operands(M, N, K_, M + N)
+    tiles = K_ // 16
+    ssq = torch.rand(tiles * K.SSQ_LD, device="cuda")
+    scratch = torch.full((K.GEMM_SCRATCH_FLOATS,), float("nan"), device="cuda")
+    assert K.gemm_wide_parts(M, N, K_, scratch.numel()) == runs
+    want = y * torch.rsqrt(ssq.view(tiles, K.SSQ_LD)[:, :M].double().sum(0) / K_ + 1e-5)[:, None]
+    out = torch.empty(M, N, device="cuda")
+    K.gemm_norm_scaled(xg, ssq, tiles, 1e-5, w, out, scratch=scratch)
+    assert off(out, want) < bound(K_) + 2 ** -24 * runs
+
+
 @pytest.mark.parametrize("M,N,K_,pays", [(8, 6144, 4096, True), (8, 8192, 4096, True), (8, 8208, 4096, True), (16, 5120, 13824, True), (1, 28672, 4096, True), (24, 4096, 4096, True),
                                          (64, 4096, 4096, True), (64, 4096, 14336, False), (64, 28672, 4096, False), (67, 4096, 4096, True),
                                          (67, 4096, 14336, False), (67, 12288, 4096, False), (128, 2048, 2048, True), (129, 2048, 2048, False), (24, 4096, 4160, False)])

@@ -13,3 +13,11 @@ def test_waits_for_loads_are_waits_for_reads(source, waits):
     with open(os.path.join(CSRC, source)) as f:
         found = re.findall(r'asm volatile\("s_waitcnt (vmcnt\([^"]*)"', f.read())
     assert len(found) == waits and all("lgkmcnt(0)" in w for w in found), found
+
+
+def test_sums_of_squares_are_in_lds_before_a_barrier():
+    """All waves write sums that one wave adds: nothing else orders the two where a workgroup's first unit has a single chunk."""
+    with open(os.path.join(CSRC, "gemm_bf16.hip")) as f:
+        source = f.read()
+    after = re.findall(r"sq\[tid\] = t;\s*([^;]*);", source)
+    assert len(after) == 1 and "s_waitcnt lgkmcnt(0)" in after[0], after
