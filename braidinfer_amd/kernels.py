@@ -1556,10 +1556,10 @@ def experts_gather(h: torch.Tensor, order: torch.Tensor, rows: torch.Tensor, top
     _check(f(_ptr(h), _ptr(order), _ptr(n_rows), _ptr(rows), _is_bf16(h, "experts_gather"), n, W, top, _stream()), "experts_gather")
 
 
-def experts_combine_norms(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether `experts_combine` takes `then` for these rows and this norm weight."""
+def experts_combine_norms(out: torch.Tensor, x: torch.Tensor, w: Optional[torch.Tensor]) -> bool:
+    """Whether `experts_combine` takes `then` for these rows and this norm weight (None: rows that are read without a norm)."""
     W = x.shape[1]
-    return (W % 4 == 0 and W <= 16 * (256 if W >= 2048 else 128 if W >= 512 else 64) and w.dtype == torch.float32 and w.numel() == W
+    return (w is not None and W % 4 == 0 and W <= 16 * (256 if W >= 2048 else 128 if W >= 512 else 64) and w.dtype == torch.float32 and w.numel() == W
             and (out.data_ptr() | x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
