@@ -120,11 +120,15 @@ class Norm(Part):
         takes, or None with nothing done."""
         return None
 
-    def product_of_prepared(self, prepared: Any, w: torch.Tensor, out: torch.Tensor, swiglu: bool = False, whole: bool = True) -> bool:
+    def product_of_prepared(self, prepared: Any, w: torch.Tensor, out: torch.Tensor, swiglu: bool = False) -> bool:
         """out = norm(x) @ w^T from what `prepare_in_product` left; False with nothing done
-        if there is no kernel for these sizes.  `whole` as for `linear`."""
+        if there is no kernel for these sizes."""
         return False
 
+    def product_beside_runs(self, prepared: Any, w: torch.Tensor, out: torch.Tensor) -> bool:
+        """The same for a product that `runs_of_prepared` may leave in runs at other sizes: with the bits of their sum where
+        the norm has kernels of both kinds."""
+        return self.product_of_prepared(prepared, w, out)
 
     def rows_of_prepared(self, prepared: Any) -> Optional[torch.Tensor]:
         """The normed rows themselves where `prepare_in_product` left them, else None."""

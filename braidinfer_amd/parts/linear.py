@@ -22,9 +22,10 @@ def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False, whole: bool = 
     to its rows and, where the next norm can, prepares that norm in the same kernel).  `whole`
     False: the bits that `linear_runs` leaves in runs (see `kernels.gemm`)."""
     if isinstance(a, NormedInput):
-        if a.prepared is not None and not accumulate and not isinstance(out, ResidualSink) \
-                and a.norm.product_of_prepared(a.prepared, w, out, whole=whole):
-            return
+        if a.prepared is not None and not accumulate and not isinstance(out, ResidualSink):
+            product = a.norm.product_of_prepared if whole else a.norm.product_beside_runs
+            if product(a.prepared, w, out):
+                return
         a = a.tensor()
     if isinstance(out, ResidualSink):
         sink, out = out, out.x

@@ -94,7 +94,13 @@ class RMSNorm(Norm):
     def rows_of_prepared(self, prepared):
         return prepared[1] if isinstance(prepared[0], str) and prepared[0] == "rows" else None
 
-    def product_of_prepared(self, prepared, w, out, swiglu=False, whole=True):
+    def product_of_prepared(self, prepared, w, out, swiglu=False):
+        return self._product(prepared, w, out, swiglu, True)
+
+    def product_beside_runs(self, prepared, w, out):
+        return self._product(prepared, w, out, False, False)
+
+    def _product(self, prepared, w, out, swiglu, whole):
         if self.rows_of_prepared(prepared) is not None:      # an ordinary product of `NormedInput.tensor`
             return False
         xg, ssq, tiles, scratch = prepared

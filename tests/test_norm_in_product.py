@@ -4,6 +4,8 @@ import torch
 
 from braidinfer_amd import kernels as K
 from braidinfer_amd.engine.step import Workspace
+from braidinfer_amd.parts.base import Norm, NormedInput, ResidualSink
+from braidinfer_amd.parts.linear import linear
 from braidinfer_amd.parts.norm import RMSNorm
 
 
@@ -25,3 +27,21 @@ def test_rows_and_weights_off_16_bytes_keep_their_two_kernels(monkeypatch, rows,
         assert called == ["runs", "sum and norm"] and norm.rows_of_prepared(prepared).shape == (rows, n)
     else:
         assert called == [] and prepared is None
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_a_norm_with_a_product_of_its_own(whole):
+    """A norm from outside gives what it prepared and takes (prepared, w, out) back, whichever bits the product is asked for."""
+    class Own(Norm):
+        def prepare_in_product(self, a, w, x, ws):
+            return "mine"
+
+        def product_of_prepared(self, prepared, w, out, swiglu=False):
+            assert prepared == "mine" and not swiglu
+            out.fill_(3.0)
+            return True
+    norm, x, w, out = Own(), torch.zeros(4, 8), torch.zeros(6, 8), torch.zeros(4, 6)
+    sink = ResidualSink(x, norm)
+    linear(torch.zeros(4, 8), torch.zeros(8, 8), sink, Workspace("cpu"), accumulate=True)
+    linear(NormedInput(x, norm, Workspace("cpu"), torch.float32, sink.prepared), w, out, Workspace("cpu"), whole=whole)
+    assert (out == 3.0).all()
