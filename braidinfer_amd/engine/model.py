@@ -294,10 +294,12 @@ class DecoderModel:
                 step.prepared_norm = None
             # the norm that reads the residual rows after this layer: the next scheduled layer's first
             # (the final norm reads chosen rows only and is left alone)
-            step.norm_after_layer = None
+            step.norm_after_layer = step.rows_norm_after_layer = None
             step.next_layer = self.layers[self.schedule[i + 1].layer] if i + 1 < len(self.schedule) else None
             if i + 1 < len(self.schedule) and self.schedule[i + 1].input_join is None:
-                step.norm_after_layer = self.layers[self.schedule[i + 1].layer].first_norm()
+                step.norm_after_layer = step.next_layer.first_norm()
+                if not self.schedule[i + 1].adds_embedding:            # it would read other rows
+                    step.rows_norm_after_layer = step.next_layer.rows_norm()
             ctx = (self._mixer_context(cache, e, i, None) if layer.mixer is not None
                    else MixerContext(unit=e.cache, writes_cache=e.writes_cache))
             for role in layer.more_mixers:

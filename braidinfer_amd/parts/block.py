@@ -58,8 +58,7 @@ def ready_rows(prepared, norm, x):
 
 def into_rows(part, h, x, step) -> None:
     """x += part(h) of a layer's last half; a part that can leaves the rows normed as the next layer's arrangement reads them."""
-    layer = getattr(step, "next_layer", None)
-    norm = layer.rows_norm() if layer is not None and getattr(part, "norms_rows", False) else None
+    norm = step.rows_norm_after_layer if getattr(part, "norms_rows", False) else None
     if norm is None:
         part.forward(h, x, step)
         return

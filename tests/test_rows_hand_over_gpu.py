@@ -57,9 +57,10 @@ def logits(cfg, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("norm,rides", [("rmsnorm", 2), ("rows", 1)])
-def test_rows_handed_over(monkeypatch, norm, rides, dtype):
-    """The bits of both ways, prompts and single tokens; what is read without a norm keeps its own launch."""
+@pytest.mark.parametrize("norm,adds,rides", [("rmsnorm", False, 2), ("rows", False, 1), ("rmsnorm", True, 1)])
+def test_rows_handed_over(monkeypatch, norm, adds, rides, dtype):
+    """The bits of both ways, prompts and single tokens; rows that are read without a norm, or that the embedding is added to
+    first, are left to their own launch."""
     seen, combine = [], K.experts_combine
 
     def counted(*a, then=None, **how):
@@ -68,12 +69,12 @@ def test_rows_handed_over(monkeypatch, norm, rides, dtype):
     register_architecture("ToyExpertsForCausalLM", ToyConfig, toy_spec)
     try:
         monkeypatch.setattr(K, "experts_combine", counted)
-        got = logits(ToyConfig(norm=norm), dtype)
+        got = logits(ToyConfig(norm=norm, adds=adds), dtype)
         if dtype == "bfloat16":
             assert seen[:3].count(True) == rides, seen[:3]
         monkeypatch.setattr(RoutedExperts, "norms_rows", False)
         del seen[:]
-        want = logits(ToyConfig(norm=norm), dtype)
+        want = logits(ToyConfig(norm=norm, adds=adds), dtype)
         assert not any(seen) and torch.equal(got, want) and torch.isfinite(want).all()
     finally:
         unregister_architecture("ToyExpertsForCausalLM")
