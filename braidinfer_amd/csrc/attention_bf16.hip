@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* _
     for (int s0 = 0; s0 < nsplit; s0 += AHEAD) {
         if (s0 % 64 == 0) {
             const int s = s0 + lane;
-            w = 0.f;
+            w = -1.f;                                 // no run, or a run without a page
             if (s < nsplit && ml[2 * s] > -INFINITY) {
                 w = fast_exp2(ml[2 * s] - M);
                 l += ml[2 * s + 1] * w;
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* _
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
             const float wj = __shfl(w, s0 % 64 + j);
-            O += (wj > 0.f ? v[j] : 0.f) * wj;
+            O += wj < 0.f ? 0.f : v[j] * wj;          // a weight that underflows is 0: a sum that is not finite shows, as in one run
         }
         if (s0 + AHEAD < nsplit) ask(s0 + AHEAD);
     }

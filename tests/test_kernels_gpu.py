@@ -948,6 +948,27 @@ def test_sums_of_decode_runs(nq, nkv, hd, nsplit):
         assert torch.isfinite(got).all() and (got - want).abs().max() < 2e-2 * want.abs().max(), (b, lens[b])
 
 
+@pytest.mark.parametrize("nsplit", [1, 2, 4, 5])
+@pytest.mark.parametrize("hd", [80, 128])
+def test_values_that_are_not_finite_show_in_any_number_of_runs(nsplit, hd):
+    """An infinite value under a key whose weight is 0 beside the largest: the dims it stands in are NaN, however the pages are cut."""
+    n = 64 * 5 - 3
+    ks, vs, cache, table = _long_cache([n], 1, hd, seed=6)
+    q = torch.zeros(1, hd, dtype=torch.bfloat16, device=DEV)
+    q[0, 0] = 64.0
+    cache[:, 0, :, :, 0] = 0.0                                     # one key stands out by far more than float weights reach
+    cache[int(table[1, 4]), 0, 0, 0, 0] = 64.0
+    cache[int(table[1, 0]), 1] = cache[int(table[1, 0]), 1].reshape(-1).index_fill(0, torch.tensor([3 * 64 + 7, (hd - 1) * 64], device=DEV), float("inf")).view(1, 64, hd)
+    out = torch.full((1, hd), 5.0, device=DEV, dtype=torch.bfloat16)
+    part_o = torch.full((nsplit * hd,), float("nan"), device=DEV)
+    part_ml = torch.full((nsplit * 2,), float("nan"), device=DEV)
+    K.attention_decode_bf16(q, hd, out, i32([1]), i32([n]), table, cache, 1, 1, 1, hd, 64, None, 1.0, nsplit, part_o, part_ml, 0)
+    bad = torch.isnan(out[0]).nonzero().flatten().tolist()
+    assert bad == [3, hd - 1]
+    rest = [d for d in range(hd) if d not in bad]
+    assert torch.equal(out[0].cpu()[rest], vs[0][256, 0].to(torch.bfloat16)[rest])
+
+
 def test_decode_splits_double_beyond_64_pages_a_run():
     from braidinfer_amd.parts.attention import decode_splits
     assert decode_splits(64, 8, 4096, 64) == 1 and decode_splits(1, 8, 2048, 64) == 16
