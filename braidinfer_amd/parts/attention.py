@@ -38,14 +38,19 @@ def decode_splits(batch: int, nkv: int, max_ctx: int, page: int, cus: int = 256)
     where that takes 8 runs or more: twice as many cost more in the sum than they gain (4 sequences of 8 kv
     heads, 8 and 16 runs: 8.8 and 10.1 us up to 512 tokens, 12.3 and 11.4 up to 2,048).  Fewer runs are long:
     two workgroups per unit, which its LDS holds, from a bound on that lets them be so (8 sequences of 128 to
-    2,048 tokens, 4 and 8 runs: 16.6 and 14.4 us; 16, 2 and 4: 25.3 and 20.9; 32, 1 and 2: 39.3 and 35.5; but
-    up to 512 tokens 9.9 and 10.5, 13.0 and 12.2, 15.1 and 16.5).  About two pages per run at
-    least, and at most 64."""
+    2,048 tokens, 4 and 8 runs: 16.6 and 14.4 us; 16, 2 and 4: 25.3 and 20.9; but up to 512 tokens 9.9 and 10.5,
+    13.0 and 12.2).  Two runs instead of one from a bound on that grows with the square of the units taken: the
+    second workgroup pays where contexts differ and costs where all are short of the bound, the more so the fewer
+    units are free (contexts at the bound, spread up to it, at half of it, one run and two: 17 sequences, bound
+    1,900: 37.1 / 37.6 / 22.5 and 33.6 / 29.5 / 22.6 us, 768: 19.4 / 18.8 / 12.8 and 20.5 / 17.3 / 15.7; 24, 1,900:
+    37.1 / 36.7 / 22.2 and 38.5 / 31.2 / 24.5, 1,024: 23.3 / 23.7 / 15.9 and 26.4 / 22.2 / 19.7; 32, 2,048: 48.4 /
+    40.3 / 27.2 and 50.6 / 37.8 / 31.2, 3,072: 67.9 / 56.6 / 38.1 and 70.3 / 49.5 / 40.4).  About two pages per run
+    at least, and at most 64."""
     pages = max(1, -(-max_ctx // page))
     heads = max(1, batch * nkv)
     want = max(1, max(1, cus) // heads)
     n = 1 << (want.bit_length() - 1)
-    if n <= 4 and 2 * n * heads <= 2 * cus and pages >= (24 if n >= 2 else 32):
+    if n <= 4 and n * heads <= cus and pages >= (24 if n > 1 else 44 * (heads / cus) ** 2):
         n *= 2
     most = max(1, min(pages // 2, 64))
     n = min(n, 1 << (most - 1).bit_length())
