@@ -58,6 +58,24 @@ def test_tiles(rt, M, N, K_):
         assert torch.equal(again, f32)
 
 
+# rows that are added to: four columns at once where they lie at 16 bytes, each by itself where not; the last block of a tile of 24 begins at its
+# eighth row, and columns end in the middle of a tile
+@pytest.mark.parametrize("rt", [16, 24, 32])
+@pytest.mark.parametrize("M,N,K_", [(1, 16, 1024), (9, 100, 1024), (16, 72, 1024), (24, 44, 512), (33, 4104, 256), (64, 120, 1024), (97, 49, 1024), (128, 200, 640)])
+def test_rows_added_to(rt, M, N, K_):
+    from braidinfer_amd import kernels as K
+    code = 7 + 16 * (rt // 8 - 1)
+    a, _, w, _ = operands(M, N, K_, M + rt)
+    f32 = torch.empty(M, N, device="cuda")
+    K.gemm(a, w, f32, kernel=code)
+    for lead in (0, 4, 3):
+        room = torch.randn(M, N + 12 - N % 4, device="cuda")
+        want = room.clone()
+        want[:, lead:lead + N] += f32
+        K.gemm(a, w, room[:, lead:lead + N], accumulate=True, kernel=code)
+        assert torch.equal(room, want)
+
+
 @pytest.mark.parametrize("rt", [16, 32])
 @pytest.mark.parametrize("M,I,K_", [(1, 8, 1024), (16, 264, 1024), (24, 40, 512), (50, 72, 1024), (64, 328, 2048), (90, 200, 1152), (128, 24, 1024)])
 def test_gated_unit(rt, M, I, K_):
