@@ -76,6 +76,27 @@ def test_rows_added_to(rt, M, N, K_):
         assert torch.equal(room, want)
 
 
+# the sum of a product's runs by one and by four columns a thread
+@pytest.mark.parametrize("M,N,K_,parts", [(70, 2048, 1024, 4), (70, 2052, 1024, 4), (128, 1028, 2048, 8), (66, 3072, 640, 2)])
+def test_sums_of_runs(M, N, K_, parts):
+    from braidinfer_amd import kernels as K
+    a, w, _, want = operands(M, N, K_, N)
+    scratch = torch.full((parts * M * N,), float("nan"), device="cuda")
+    for lead in (0, 1):
+        room = torch.full((M, N + 4), 7.0, device="cuda")
+        K.gemm(a, w, room[:, lead:lead + N], kernel=6 + 16 * parts, scratch=scratch)
+        assert off(room[:, lead:lead + N], want) < bound(K_)
+        assert bool((room[:, :lead] == 7.0).all()) and bool((room[:, lead + N:] == 7.0).all())
+        base = torch.randn(M, N + 4, device="cuda")
+        got = base.clone()
+        K.gemm(a, w, got[:, lead:lead + N], accumulate=True, kernel=6 + 16 * parts, scratch=scratch)
+        base[:, lead:lead + N] += room[:, lead:lead + N]
+        assert torch.equal(got, base)
+    half = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    K.gemm(a, w, half, kernel=6 + 16 * parts, scratch=scratch)
+    assert torch.equal(half, room[:, 1:1 + N].to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("rt", [16, 32])
 @pytest.mark.parametrize("M,I,K_", [(1, 8, 1024), (16, 264, 1024), (24, 40, 512), (50, 72, 1024), (64, 328, 2048), (90, 200, 1152), (128, 24, 1024)])
 def test_gated_unit(rt, M, I, K_):
