@@ -5,8 +5,8 @@
 // Kernels:
 //  * gemm_stream_tile: up to 16 rows (decode), and up to 128 against few weight rows: a workgroup a tile of 16 to 32 weight rows
 //    over all of K, weights and activations brought into per-wave LDS rings by direct global-to-LDS loads.
-//  * gemm_stream: up to 16 rows with an RMS norm before or behind, where tiles are many or K long: the same streaming by one
-//    resident workgroup per compute unit.
+//  * gemm_stream: up to 16 rows where tiles are many and K short or long, and with an RMS norm before or behind: the same streaming
+//    by one resident workgroup per compute unit.
 //  * gemm_tile: LDS-staged tiles for many rows (prompts): 4 waves, each a TM x TN grid of
 //    v_mfma_f32_32x32x16_bf16 blocks; global loads of the next k-tile are issued before the
 //    current one is multiplied and written to the other LDS buffer after it.
@@ -1594,7 +1594,7 @@ static int split_parts(int M, int N, int K, int mode, size_t scratch_bytes) {
 }
 
 // ------------------------------------------------------------------ gemm_stream ------
-// M <= 16, K in steps of 128, a norm before or behind: weight streaming by workgroups that stay.  One workgroup per
+// M <= 16, K in steps of 128: weight streaming by workgroups that stay.  One workgroup per
 // compute unit walks over tiles of 16 weight rows (tile t of workgroup b is b + t * grid);
 // its 8 waves take the tile's 128-wide k-chunks in turn.  A wave brings a chunk of the
 // tile (16 rows x 256 bytes) and the same chunk of the activations (8 or 16 rows) into a
@@ -1645,7 +1645,7 @@ template <int RT, int XR, int KC, int S, int NW, int MODE, int NORM>
 __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C, int M, int N, int K, size_t lda,
                                                               size_t ldc, int ntiles, StreamNorm nrm, int wl) {
-    static_assert((NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC), "norm forms");
+    static_assert(NORM == 0 || (NORM == 1 && MODE == OUT_F32_ACC) || (NORM == 2 && MODE != OUT_F32_ACC), "norm forms");
     constexpr int STEPS = KC / 32;
     constexpr int ROWB = KC * 2;
     constexpr int STAGE = (RT + XR) * ROWB;
@@ -1814,7 +1814,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_stream_kernel(const bf16* __rest
                                 if (NORM == 2) v *= rstd[m];
                                 const size_t idx = (size_t)m * ldc + n;
                                 if (MODE == OUT_BF16) ((bf16*)C)[idx] = (bf16)v;
-                                else ((float*)C)[idx] = v;
+                                else if (MODE == OUT_F32) ((float*)C)[idx] = v;
+                                // one add per element and product, without a read that this wave would
+                                // have to wait for behind its loads in flight
+                                else unsafeAtomicAdd((float*)C + idx, v);
                             }
                         }
                     }
@@ -1858,6 +1861,7 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
         if (mode == OUT_BF16) BR_STREAM(OUT_BF16);
         else if (mode == OUT_F32) BR_STREAM(OUT_F32);
         else if (mode == OUT_SWIGLU) BR_STREAM(OUT_SWIGLU);
+        else if constexpr (NORM == 0) BR_STREAM(OUT_F32_ACC);
         else return BR_BAD_ARG;
     }
 #undef BR_STREAM
@@ -2186,7 +2190,7 @@ static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, vo
     return BR_BAD_ARG;
 }
 // The weight rows of a workgroup (16, 24 or 32) where gemm_stream_tile is the faster kernel, else 0.
-// Up to 16 rows always (K in steps of 128 from 1,024): the fewest weight rows for the busiest compute unit, the same for every number
+// Up to 16 rows always (K in steps of 128 from 1,024; but see resident_pays): the fewest weight rows for the busiest compute unit, the same for every number
 // of rows, so that a row's bits do not depend on the others'; of two that are alike the taller where one round covers the matrix
 // (8,192 x 4,096: 12.6 us by 32, 13.7 by 16), else the lower, of which two workgroups share a unit (32,768 x 4,096 by 8 rows:
 // 43.9 by 16, 46.0 by 24, 46.5 by 32).  One resident workgroup a unit that walked tiles of 16 rows, as gemm_stream does, took, at 1, 8
@@ -2215,6 +2219,17 @@ static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) 
     const double other = M <= 64 ? 0.96 * (6.2 + 0.043 * M + 1.61 * mb + 1.6e-6 * M * N + 4.7e-6 * M * K - (mode == OUT_SWIGLU ? 2.4 : 0.0))
                                  : 9.1 + 1.9 * mb + 0.125e-3 * K + 0.41e-3 * N + 0.027 * M;
     return best < other ? best_rt : 0;
+}
+
+// Where products of up to 16 rows without a norm stay with gemm_stream's resident workgroups (the same for every number of rows): a chunk
+// a wave, or two and an add into rows, is over before the tile's two stages have anything to hide, so that many tiles pay a workgroup's start each
+// (K 1,024 by 8 rows, us, tiles and resident: 16,384 weight rows 8.7 / 8.2, 65,536 27.9 / 23.1, gated 28,672 14.4 / 12.3, added into float rows 2,048
+// 4.2 / 3.9; K 2,048 added 2,048 5.2 / 4.9), but not where 24 or 32 rows balance one round (6,144 5.0 / 5.4, 8,192 5.5 / 5.7) nor from K 1,152
+// on, of which resident waves take two uneven shares (65,536 by 8 rows 29.5 / 34.4); and long K over more than one round (K 12,288 to 14,336,
+// 10,240 to 16,384 weight rows by 8 rows 45.0 / 43.4 to 73.8 / 70.5; K 11,008 41.2 / 41.0).
+static bool resident_pays(int N, int K, int mode, int cus) {
+    if (N > 32 * cus) return K == 1024 || K >= 12288;
+    return N <= 16 * cus && (K == 1024 || (mode == OUT_F32_ACC && K <= 2048 && N <= 12 * cus));
 }
 
 // Whether the norm forms of up to 16 rows, too, leave gemm_stream: one round of tiles (every workgroup reads all sums of squares:
@@ -2661,7 +2676,13 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     if (kernel == 7 && !chosen && forced_parts) {      // 7 + 16 b: a workgroup a tile of 8 (b + 1) weight rows, b = 1, 2, 3
         return launch_stream_tile(8 * (forced_parts + 1), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
     }
-    if (kernel == 7) return launch_stream_tile(tile_rows(M, N, K, mode, br_device_cus()), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
+    if (kernel == 7) {
+        const int cus = br_device_cus();
+        if (resident_pays(N, K, mode, cus))
+            return M <= 8 ? launch_stream<8, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl)
+                          : launch_stream<16, 0>(A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
+        return launch_stream_tile(tile_rows(M, N, K, mode, cus), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
+    }
     int parts = 1;
     if (chosen && M > 128 && (kernel == 5 || kernel == 6) && quad_takes(C, M, N, K, lda, ldc)) {
         // More than 128 rows, K in steps of 64: the tiles of one wave per SIMD, where the product's addresses
@@ -2804,7 +2825,8 @@ extern "C" int br_gemm_bf16_tile_choice(int M, int N, int K, int mode, size_t sc
 
 // Whether a product of up to 128 aligned rows goes to gemm_stream_tile (17 to 64 rows: when asked for one without runs).
 extern "C" int br_gemm_bf16_whole_pays(int M, int N, int K, int by16) {
-    return tile_rows(M, N, K, OUT_BF16, br_device_cus(), by16 != 0) != 0;
+    const int cus = br_device_cus();
+    return tile_rows(M, N, K, OUT_BF16, cus, by16 != 0) != 0 && (M > 16 || !resident_pays(N, K, OUT_BF16, cus));
 }
 
 static bool stream_takes(const void* A, const void* W, int M, int K, size_t lda) {

@@ -216,6 +216,35 @@ def test_where_the_rule_takes_it(M, N, K_, pays):
             assert torch.equal(total.view(M, N), alone)
 
 
+# up to 16 rows, on both sides of the lines between tiles and resident workgroups: columns below and above one round, one chunk a wave and more
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,K_,tiles", [(4096, 1024, False), (4100, 1024, True), (8192, 1024, True), (8194, 1024, False), (20480, 1024, False), (20480, 1152, True),
+                                        (3072, 2048, True), (8208, 11008, True), (8208, 12288, False)])
+def test_where_resident_workgroups_stay(M, N, K_, tiles):
+    from braidinfer_amd import kernels as K
+    assert K.gemm_whole_pays(M, N, K_) == tiles
+    a, _, w, want = operands(M, N, K_, 7, blocked=N % 16 == 0 and N > 8192)
+    out, one = torch.empty(M, N, device="cuda"), torch.empty(1, N, device="cuda")
+    K.gemm(a, w, out)
+    assert off(out, want) < bound(K_)
+    half = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    K.gemm(a, w, half)
+    assert torch.equal(half, out.to(torch.bfloat16))
+    base = torch.randn(M, N, device="cuda")
+    got, last = base.clone(), base[M - 1:].clone()
+    K.gemm(a, w, got, accumulate=True)
+    assert off(got, base.double() + want) < bound(K_)
+    K.gemm(a[M - 1:], w, one)                            # a row's bits do not depend on the others
+    K.gemm(a[M - 1:], w, last, accumulate=True)
+    assert torch.equal(one, out[M - 1:]) and torch.equal(last, got[M - 1:])
+    if N % 16 == 0:
+        act = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
+        K.gemm_swiglu(a, w, act)
+        gu = want.view(M, N // 16, 2, 8)
+        g, u = gu[:, :, 0].reshape(M, -1), gu[:, :, 1].reshape(M, -1)
+        assert off(act, g / (1 + torch.exp(-g)) * u) < 2 ** -8
+
+
 @pytest.mark.parametrize("M,N,K_", [(65, 4096, 4096), (128, 1028, 1024), (100, 2048, 2048)])
 def test_one_run_left_for_the_norm(M, N, K_):
     from braidinfer_amd import kernels as K
