@@ -2364,14 +2364,23 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
     for (int j = 0; j < D; ++j)
         if (is_u < my_units) WIDE_ISSUE();
     if constexpr (!BRANCHES) if (scale) {
-        // wave w takes the tiles w, w + 8, .. of all rows, a lane a row; the eight sums are added at the first unit's end
+        // wave w takes the tiles w, w + 8, .. of all rows, a lane a row; the first wave adds the eight sums
         float t = 0.f;
         if (lane < M) {
 #pragma unroll 8
             for (int c = wave; c < nrm.ssq_tiles; c += NW) t += nrm.ssq[(size_t)c * SSQ_LD + lane];
         }
         sq[tid] = t;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the barrier in front of the first chunk publishes it: units may have one chunk
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (wave == 0) {
+            t = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) t += sq[w * 64 + lane];
+            rstd[lane] = rsqrtf(t * nrm.inv_k + nrm.eps);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the barrier in front of the first chunk publishes it
+        }
     }
     if (my_units > 0) WIDE_RUN_LENGTH(0, cp_left);
     while (cp_u < my_units) {
@@ -2429,12 +2438,6 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
         const int n0 = (unit / parts) * H;
         if (++cp_u < my_units) WIDE_RUN_LENGTH(cp_u, cp_left);
         float* red = (float*)st;                 // [H][RLD]
-        if constexpr (!BRANCHES) if (scale && cp_u == 1 && tid < 64) {
-            float t = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) t += sq[w * 64 + tid];
-            rstd[tid] = rsqrtf(t * nrm.inv_k + nrm.eps);
-        }
         __builtin_amdgcn_s_barrier();            // every wave has read its operands of the stage
         asm volatile("" ::: "memory");
         if (khalf == 1) {

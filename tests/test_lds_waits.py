@@ -16,8 +16,10 @@ def test_waits_for_loads_are_waits_for_reads(source, waits):
 
 
 def test_sums_of_squares_are_in_lds_before_a_barrier():
-    """All waves write sums that one wave adds: nothing else orders the two where a workgroup's first unit has a single chunk."""
+    """All waves write sums that one wave adds, and one wave what all read: nothing else orders them where a workgroup's first unit
+    has a single chunk."""
     with open(os.path.join(CSRC, "gemm_bf16.hip")) as f:
         source = f.read()
-    after = re.findall(r"sq\[tid\] = t;\s*([^;]*);", source)
-    assert len(after) == 1 and "s_waitcnt lgkmcnt(0)" in after[0], after
+    for write in (r"sq\[tid\] = t;", r"rstd\[lane\] = [^;]*;"):
+        after = re.findall(write + r"\s*([^;]*);", source)
+        assert len(after) == 1 and "s_waitcnt lgkmcnt(0)" in after[0], after
