@@ -1550,7 +1550,7 @@ static int launch_split_sum(const float* scratch, int parts, void* C, int M, int
     // still has them; four a thread spread a row over fewer (128 x 128 tiles with their sum, K 4,096, us by one and by four: 2,048 columns in 16
     // runs by 66, 96 and 128 rows 12.8 / 16.4, 13.4 / 18.7, 14.3 / 21.0, in 8 runs 15.5 / 17.0, 15.7 / 18.3, 16.0 / 19.2; 1,024 by 200 rows in 8 runs
     // 16.0 / 17.2.  8,192 columns in 4 runs by 96 rows 31.3 / 26.2, where four a thread make the eight; between them alike.)
-    const int vec = N > 2048 && N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0 && (uintptr_t)scratch % 16 == 0 ? 4 : 1;
+    const int vec = (mode == OUT_SWIGLU ? N / 2 : N) > 2048 && N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0 && (uintptr_t)scratch % 16 == 0 ? 4 : 1;
     const unsigned blocks = (unsigned)((results / vec + 255) / 256);
 #define BR_SUM(MODE_)                                                                                                          \
     do {                                                                                                                       \
