@@ -2197,27 +2197,32 @@ static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, vo
 // and 16 rows: 6,144 x 4,096 12.2 / 12.7 / 13.8 (now 10.6 / 10.9 / 11.0), 32,768 x 4,096 45.3 / 47.0 / 54.3 (43.3 / 43.9 / 49.2),
 // 5,120 x 13,824 32.0 / 32.9 / 36.8 (25.5 / 27.2 / 28.0), 4,096 x 14,336 21.2 / 21.4 / 24.3 (20.7 / 21.5 / 23.5), 2,048 x 8,192
 // 10.7 / 9.9 / 11.2 (9.9 / 9.8 / 11.6).
-// More rows: by counts in microseconds, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at nine numbers of rows from 17
-// to 96, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's; gemm_stream_wide
-// with the sum of its runs (up to 64 rows); the eight-wave tiles with theirs (beyond).  Single rounds only: matrices of more (32,768 x 4,096
-// by 32 rows: 47 us shared, 50 by tiles) have no sums to save.
-// The line it draws gains 1.3 in the mean over these, and loses 5 % at most.  by16: whole blocks of 16 columns only (NORM 1).
+// More rows, by counts in microseconds.  Up to 64, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at rows from 17
+// to 64, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's, against gemm_stream_wide
+// with the sum of its runs.  Single rounds only: matrices of more (32,768 x 4,096 by 32 rows: 47 us shared, 50 by tiles) have no sums to save.
+// Beyond 64, fitted to 143 shapes (256 to 8,192 weight rows, K 512 to 14,336) at six numbers of rows, mean error 5 %, against the
+// eight-wave tiles with the sum of theirs, 7 % and less 8 %, since these differ by up to a fifth from card to card: 8,192 x 14,336 by
+// 65 rows 49 to 54 us on three cards, 62 by tiles on each; 7,168 x 11,008 38 and 48; 8,192 x 4,096 28 and 20; 4,096 x 4,096 21 and 15.
+// The lines gain 1.25 in the mean over these shapes and lose 6 % at most.  by16: whole blocks of 16 columns only (NORM 1).
 static int tile_rows(int M, int N, int K, int mode, int cus, bool by16 = false) {
     if (M <= 0 || M > TILE_MAX_ROWS || K % 128 || K < (M <= 16 ? 1024 : 256) || cus <= 0 || (M > 16 && N > 32 * cus)) return 0;
     int best_rt = 0;
     double best = 1e30;
     const bool low = M <= 16 && N > 32 * cus;
+    const int m16 = (M + 15) / 16 * 16;
     for (int i = 0; i < 3; ++i) {
         const int rt = low ? 16 + 8 * i : 32 - 8 * i;
         if (rt == 24 && (mode == OUT_SWIGLU || by16)) continue;
         const int rounds = (N + rt * cus - 1) / (rt * cus);
-        const double t = M <= 16 ? (double)rounds * rt : 3.1 + rounds * (double)(rt + M) * K * 2.9e-5 + (double)N * K * 1.27e-7;
+        const double t = M <= 16   ? (double)rounds * rt
+                         : M <= 64 ? 3.1 + rounds * (double)(rt + M) * K * 2.9e-5 + (double)N * K * 1.27e-7
+                                   : 2.6 + rounds * ((double)(rt + m16) * K * 2.83e-5 + 0.016 * m16) + (double)N * K * 1.09e-7;
         if (t < best * (1.0 - 1e-9)) { best = t; best_rt = rt; }
     }
     if (M <= 16) return best_rt;
     const double mb = (double)N * K * 2e-7;                              // weights in 10 MB
     const double other = M <= 64 ? 0.96 * (6.2 + 0.043 * M + 1.61 * mb + 1.6e-6 * M * N + 4.7e-6 * M * K - (mode == OUT_SWIGLU ? 2.4 : 0.0))
-                                 : 9.1 + 1.9 * mb + 0.125e-3 * K + 0.41e-3 * N + 0.027 * M;
+                                 : 8.2 + 1.04 * mb + 0.63e-3 * K + 0.59e-3 * N + 0.025 * M;
     return best < other ? best_rt : 0;
 }
 

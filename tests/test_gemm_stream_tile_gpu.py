@@ -194,7 +194,9 @@ def test_a_prepared_norm_over_runs_of_one_chunk(M, N, K_, runs):
 
 @pytest.mark.parametrize("M,N,K_,pays", [(8, 6144, 4096, True), (8, 8192, 4096, True), (8, 8208, 4096, True), (16, 5120, 13824, True), (1, 28672, 4096, True), (24, 4096, 4096, True),
                                          (64, 4096, 4096, True), (64, 4096, 14336, False), (64, 28672, 4096, False), (67, 4096, 4096, True),
-                                         (67, 4096, 14336, False), (67, 12288, 4096, False), (128, 2048, 2048, True), (129, 2048, 2048, False), (24, 4096, 4160, False)])
+                                         (67, 4096, 14336, False), (67, 12288, 4096, False), (128, 2048, 2048, True), (129, 2048, 2048, False), (24, 4096, 4160, False),
+                                         (65, 8192, 4096, True), (65, 8192, 14336, False), (72, 7168, 9216, False), (80, 2048, 4096, False), (96, 6144, 4096, True),
+                                         (128, 8192, 5120, False), (65, 1024, 2048, True)])
 def test_where_the_rule_takes_it(M, N, K_, pays):
     from braidinfer_amd import kernels as K
     assert K.gemm_whole_pays(M, N, K_) == pays
