@@ -155,11 +155,12 @@ __device__ __forceinline__ float block_sum_once(float v, float* scratch) {
 // in registers between the sums and the scaling.  With `w2` the kernel goes on: the row it has just added
 // to (the residual row) is normed once more with the weight `w2` into `y2` (compute dtype): the norm
 // behind one half of a layer and the norm in front of the next in one pass over the row.
-// Few rows are bound by a chain of latencies (loads, four sums over the block), so that everything the row
-// needs is asked for before the first sum and a sum takes one barrier; many rows by memory.  (8 rows of
-// 4,096 with `w2`: 6.3 us a launch among others; 7.9 with the weights and the residual row asked for
-// where they are used and two barriers a sum; 5,018 rows 52 either way.)
-template <typename T, typename T2, bool ADD, int VPT>
+// Few rows are bound by a chain of latencies (loads, four sums over the block), so that everything the row needs is asked for before
+// the first sum (AHEAD) and a sum takes one barrier; many rows by memory, and what is asked for early then holds registers that
+// more workgroups could use: rows that are added to ask late from 2 M elements on.  (us a launch among others, with `w2`, ahead / late / late with
+// two barriers a sum: 8 rows of 4,096 4.4 / 4.7 / 5.1; 1,024 of 2,048 6.3 / 6.2 / 6.5; 2,048 of 2,048 11.0 / 9.5 / 9.9; 8,000 of 1,024
+// 20.3 / 19.0 / 18.8.  Rows that are only normed gain ahead at any number: 8,000 of 4,096 28.9 / 30.2 / 31.3.)
+template <typename T, typename T2, bool ADD, int VPT, bool AHEAD>
 __global__ __launch_bounds__(256) void layernorm_vec_kernel(const float* __restrict__ x, const float* __restrict__ w, T* __restrict__ y,
                                      const int* __restrict__ rows, int H, float eps, int center, int plain,
                                      const float* __restrict__ w2, T2* __restrict__ y2, float eps2, int center2) {
@@ -174,9 +175,11 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(const float* __restr
         const int i = threadIdx.x + j * blockDim.x;
         if (i < nv) {
             v[j] = xr[i];
-            wv[j] = ((const f32x4*)w)[i];
-            if (ADD) acc[j] = ((const f32x4*)yr)[i];
-            if (ADD && w2) w2v[j] = ((const f32x4*)w2)[i];
+            if (AHEAD) {
+                wv[j] = ((const f32x4*)w)[i];
+                if (ADD) acc[j] = ((const f32x4*)yr)[i];
+                if (ADD && w2) w2v[j] = ((const f32x4*)w2)[i];
+            }
         }
     }
     float sm = 0.f;
@@ -201,6 +204,10 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(const float* __restr
     for (int j = 0; j < VPT; ++j) {
         const int i = threadIdx.x + j * blockDim.x;
         if (i < nv) {
+            if (!AHEAD) {
+                wv[j] = ((const f32x4*)w)[i];
+                if (ADD) acc[j] = ((const f32x4*)yr)[i];
+            }
             if (ADD) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) { acc[j][e] += v[j][e] * inv * wv[j][e]; v[j][e] = acc[j][e]; sm2 += acc[j][e]; }
@@ -244,6 +251,7 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(const float* __restr
     for (int j = 0; j < VPT; ++j) {
         const int i = threadIdx.x + j * blockDim.x;
         if (i < nv) {
+            if (!AHEAD) w2v[j] = ((const f32x4*)w2)[i];
             float o[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = v[j][e] * inv2 * w2v[j][e];
@@ -268,11 +276,18 @@ extern "C" int br_layernorm(const float* x, const float* w, void* y, int y_is_bf
     const bool vec = (H % 4 == 0) && (H / 4 <= 4 * threads) &&
                      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)w2 | (uintptr_t)y2) % 16 == 0);
     if (vec) {
+        const bool ahead = !add || (size_t)R * H < 2000000;
+#define BR_LN(T_, T2_, ADD_, ...)                                                                                                \
+    do {                                                                                                                        \
+        if (ahead) layernorm_vec_kernel<T_, T2_, ADD_, 4, true><<<R, threads, 0, s>>>(x, w, (T_*)y, rows, H, eps, center, plain, __VA_ARGS__); \
+        else layernorm_vec_kernel<T_, T2_, ADD_, 4, false><<<R, threads, 0, s>>>(x, w, (T_*)y, rows, H, eps, center, plain, __VA_ARGS__);      \
+    } while (0)
         if (add) {
-            if (y2_is_bf16) layernorm_vec_kernel<float, bf16, true, 4><<<R, threads, 0, s>>>(x, w, (float*)y, rows, H, eps, center, plain, w2, (bf16*)y2, eps2, center2);
-            else layernorm_vec_kernel<float, float, true, 4><<<R, threads, 0, s>>>(x, w, (float*)y, rows, H, eps, center, plain, w2, (float*)y2, eps2, center2);
-        } else if (y_is_bf16) layernorm_vec_kernel<bf16, float, false, 4><<<R, threads, 0, s>>>(x, w, (bf16*)y, rows, H, eps, center, plain, nullptr, nullptr, 0.f, 0);
-        else layernorm_vec_kernel<float, float, false, 4><<<R, threads, 0, s>>>(x, w, (float*)y, rows, H, eps, center, plain, nullptr, nullptr, 0.f, 0);
+            if (y2_is_bf16) BR_LN(float, bf16, true, w2, (bf16*)y2, eps2, center2);
+            else BR_LN(float, float, true, w2, (float*)y2, eps2, center2);
+        } else if (y_is_bf16) BR_LN(bf16, float, false, nullptr, nullptr, 0.f, 0);
+        else BR_LN(float, float, false, nullptr, nullptr, 0.f, 0);
+#undef BR_LN
         return br_check_launch();
     }
     if (add) layernorm_kernel<float, true><<<R, threads, 0, s>>>(x, w, (float*)y, rows, H, eps, center, plain);

@@ -141,6 +141,33 @@ def test_layer_norm_kernels():
         assert np.abs(out.cpu().numpy() - P.layer_norm(x[[T - 1, 0]].astype(np.float64), w, 1e-5)).max() < 2e-5
 
 
+@pytest.mark.parametrize("R,H", [(2049, 1024), (8200, 256), (513, 4096), (700, 3068)])
+@pytest.mark.parametrize("center", [True, False])
+def test_layer_norms_of_many_rows(R, H, center):
+    """Rows that ask for their weights ahead and late, on both sides of the line: the same bits, and those of the norm in 64 bits up to rounding."""
+    from braidinfer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(R)
+    y, x0 = torch.randn(R, H, device="cuda", generator=g), torch.randn(R, H, device="cuda", generator=g)
+    w, w2 = (1 + 0.2 * torch.randn(H, device="cuda", generator=g) for _ in range(2))
+
+    def run(a, b):
+        x, out = x0[a:b].clone(), torch.empty(b - a, H, dtype=torch.bfloat16, device="cuda")
+        K.layernorm(y[a:b], w, x, 1e-5, center=center, add=True, then=(w2, out, 1e-6, center))
+        plain = torch.empty(b - a, H, device="cuda")
+        K.layernorm(y[a:b], w, plain, 1e-5, center=center)
+        rows, as_they_are = x0[a:b].clone(), torch.empty_like(out)
+        K.layernorm(y[a:b], w, rows, 1e-5, center=center, add=True, then=(None, as_they_are, 0.0, False))
+        assert torch.equal(rows, x) and torch.equal(as_they_are, x.to(torch.bfloat16))
+        return x, out, plain
+    whole = run(0, R)
+    for a, b in ((0, 3), (R // 2, R // 2 + 100), (R - 1, R)):
+        assert all(torch.equal(f[a:b], s) for f, s in zip(whole, run(a, b)))
+    v = y.double() - (y.double().mean(1, keepdim=True) if center else 0.0)
+    want = x0.double() + v * torch.rsqrt((v * v).mean(1, keepdim=True) + 1e-5) * w.double()
+    assert float((whole[0].double() - want).norm() / want.norm()) < 2 ** -22      # a few roundings of an element, sums of 4,096 by trees
+    assert float((whole[2].double() - (want - x0.double())).norm() / want.norm()) < 2 ** -22
+
+
 @pytest.mark.parametrize("H,d,e", [(2, 16, 32), (1, 18, 80), (3, 6, 8), (2, 128, 128), (1, 70, 200)])
 def test_gated_recurrence_kernels(H, d, e):
     """scan (with its gates) and head norm against the plain recurrence: two sequences in unequal portions, the state
