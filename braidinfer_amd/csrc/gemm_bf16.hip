@@ -1893,11 +1893,6 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
 constexpr int tile_waves(int RT, int MB) { return 640 / (RT + 16 * MB) < 8 ? 640 / (RT + 16 * MB) : 8; }     // 160 KB of LDS
 #define TILE_KC 64
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ const bf16* uniform(const bf16* p) {
-    const unsigned long long a = (unsigned long long)p;
-    return (const bf16*)((unsigned long long)(unsigned)uniform((int)(unsigned)a) |
-                         (unsigned long long)(unsigned)uniform((int)(a >> 32)) << 32);
-}
 template <int RT, int MB, int NORM>
 __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                                    void* __restrict__ C, int M, int N, int K, size_t lda,
@@ -2196,7 +2191,8 @@ static int launch_stream_tile(int rt, int norm, const bf16* A, const bf16* W, vo
 // 43.9 by 16, 46.0 by 24, 46.5 by 32).  One resident workgroup a unit that walked tiles of 16 rows, as gemm_stream does, took, at 1, 8
 // and 16 rows: 6,144 x 4,096 12.2 / 12.7 / 13.8 (now 10.6 / 10.9 / 11.0), 32,768 x 4,096 45.3 / 47.0 / 54.3 (43.3 / 43.9 / 49.2),
 // 5,120 x 13,824 32.0 / 32.9 / 36.8 (25.5 / 27.2 / 28.0), 4,096 x 14,336 21.2 / 21.4 / 24.3 (20.7 / 21.5 / 23.5), 2,048 x 8,192
-// 10.7 / 9.9 / 11.2 (9.9 / 9.8 / 11.6).
+// 10.7 / 9.9 / 11.2 (9.9 / 9.8 / 11.6).  Against up to 4,096 weight rows, where 16 balance one round either way, tiles gain 2 to 10 % at one row
+// and lose 2 to 5 % at 9 to 16 (2,048 x 8,192 added into rows 12.3 and 11.8).
 // More rows, by counts in microseconds.  Up to 64, fitted to 18 shapes (512 to 12,288 weight rows, K 1,024 to 14,336) at rows from 17
 // to 64, mean error 5 %: a tile's rows and activations over a unit's path at 69 GB/s, and its share of the memory's, against gemm_stream_wide
 // with the sum of its runs.  Single rounds only: matrices of more (32,768 x 4,096 by 32 rows: 47 us shared, 50 by tiles) have no sums to save.
@@ -2239,7 +2235,9 @@ static bool resident_pays(int N, int K, int mode, int cus) {
 
 // Whether the norm forms of up to 16 rows, too, leave gemm_stream: one round of tiles (every workgroup reads all sums of squares:
 // 28,672 x 4,096 by 8 rows 38.7 us by tiles, 37.2 by resident workgroups; 6,144 x 4,096 11.5 and 12.9), and K below 8,192 (4,096 x 14,336
-// by 8 and 16 rows 21.4 and 24.0 against 20.9 and 23.2; 4,096 x 4,096 8.1 and 9.0 against 8.6 and 9.0).
+// by 8 and 16 rows 21.4 and 24.0 against 20.9 and 23.2; 4,096 x 4,096 8.1 and 9.0 against 8.6 and 9.0).  Resident over tiles, K 1,024 to
+// 7,168: a norm prepared by 1, 8 and 16 rows 1.02 to 1.10, 1.00 to 1.05 and 0.97 to 1.05 against up to 4,096 weight rows, 1.03 to 1.26 against
+// 5,120 to 8,192; one used 1.00 to 1.13 and 1.01 to 1.37 (6,144 the most).
 static bool tile_norms(int M, int N, int K, int cus) { return M > 16 || (N <= 32 * cus && K < 8192); }
 
 // What launch_stream_tile needs of its operands beside aligned rows.
