@@ -1889,7 +1889,10 @@ static int launch_stream(const bf16* A, const bf16* W, void* C, int M, int N, in
 //
 // NORM 1, 2: as gemm_stream's forms (the tile's columns as sums of squares by 16); C, or the sums of squares, are asked for
 // before the first weights and used at the end.  NORM 3: products of several inputs by stacked weights in one launch
-// (br_gemm_bf16_branches); a tile lies in one branch.
+// (br_gemm_bf16_branches); a tile lies in one branch.  NORM 4: float rows that 16-byte stores can take are added to, and asked for ahead
+// as NORM 1 does (added in memory instead, a column at a time, it took, us: 64 rows, 6,144 x 4,096 22.8, now 17.4; 96 rows 30.4,
+// 22.3; 128 rows, 6,144 x 1,024 24.6, 12.7; 8,192 x 4,096 by 64 rows 22.8, 18.8).  A form of its own: asked for under a test of `mode`, the
+// products that add to nothing waited 0.2 us for it.
 constexpr int tile_waves(int RT, int MB) { return 640 / (RT + 16 * MB) < 8 ? 640 / (RT + 16 * MB) : 8; }     // 160 KB of LDS
 #define TILE_KC 64
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -1923,9 +1926,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
     const int q_row = lane % QR, q_tile = wave * QT + lane / QR;
     f32x4 c_pre[PER], g_pre[PER];
     float q_pre[QN];
-    // What is added to, asked for ahead as NORM 1 does (added in memory instead, a column at a time, it took, us: 64 rows, 6,144 x 4,096
-    // 22.8, now 17.4; 96 rows 30.4, 22.3; 128 rows, 6,144 x 1,024 24.6, 12.7; 8,192 x 4,096 by 64 rows 22.8, 18.8).
-    if constexpr (NORM == 0) if (mode == OUT_F32_ACC && vec) {
+    if constexpr (NORM == 4) {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int t = block_of(i), m = row_of(t), n = col_of(t);
@@ -2060,7 +2061,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
             for (int w = 1; w < NW; ++w) q += sq[w * 64 + m];
             v *= rsqrtf(q * nrm.inv_k + nrm.eps);
         }
-        if (mode == OUT_SWIGLU) {
+        if (NORM != 4 && mode == OUT_SWIGLU) {
             // 16 weight rows are 8 gates, then the 8 up values of the same outputs
             f32x4 up;
 #pragma unroll
@@ -2109,9 +2110,9 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
         }
         float* to = (float*)C + (size_t)m * ldc + n + branch_gap(nrm, n0);
         bf16* to16 = (bf16*)C + (size_t)m * ldc + n;
-        if (vec) {                                     // N in steps of 4: all four columns
-            if constexpr (NORM == 0) if (mode == OUT_F32_ACC) v = c_pre[i] + v;
-            if (mode == OUT_BF16) {
+        if (NORM == 4 || (vec && mode != OUT_F32_ACC)) {   // N in steps of 4: all four columns
+            if constexpr (NORM == 4) v = c_pre[i] + v;
+            if (NORM != 4 && mode == OUT_BF16) {
                 bf16x4 o;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
@@ -2146,6 +2147,7 @@ static int launch_tile_form(const bf16* A, const bf16* W, void* C, int M, int N,
     int vec = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0;
     if constexpr (NORM == 1) vec = vec && (nrm.ldx % 4 == 0 && (uintptr_t)nrm.xg % 8 == 0 && (uintptr_t)nrm.gain % 16 == 0);
     if constexpr (NORM == 3) vec = vec && nrm.gap % 4 == 0;
+    if constexpr (NORM == 0) if (vec && mode == OUT_F32_ACC) return launch_tile_form<RT, MB, 4>(A, W, C, M, N, K, lda, ldc, mode, s, nrm, wl);
     kern<<<(N + RT - 1) / RT, 64 * tile_waves(RT, MB), lds, s>>>(A, W, C, M, N, K, lda, ldc, mode, vec, nrm, wl);
     return br_check_launch();
 }
