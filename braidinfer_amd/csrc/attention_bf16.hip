@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* _
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
             const float wj = __shfl(w, s0 % 64 + j);
-            O += wj < 0.f ? 0.f : v[j] * wj;          // a weight that underflows is 0: a sum that is not finite shows, as in one run
+            O += (wj < 0.f ? 0.f : v[j]) * wj;        // one rounding a run; a weight that underflows is 0: a sum that is not finite shows, as in one run
         }
         if (s0 + AHEAD < nsplit) ask(s0 + AHEAD);
     }
