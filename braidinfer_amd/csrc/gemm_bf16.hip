@@ -2086,7 +2086,7 @@ __global__ __launch_bounds__(64 * tile_waves(RT, MB)) void gemm_stream_tile_kern
             for (int e = 0; e < 4; ++e) q += h[e] * h[e];
             q += __shfl_xor(q, 16, 64);
             q += __shfl_xor(q, 32, 64);
-            if (m >= M || n >= N) continue;            // a tile of 32 rows may end 16 columns behind the last one
+            if (m >= M || (RT > 16 && n >= N)) continue;   // a tile of 32 rows may end 16 columns behind the last one
             if (g == 0) nrm.ssq[(size_t)(n / 16) * SSQ_LD + m] = q;
             float* to = (float*)C + (size_t)m * ldc + n;
             bf16* xg = nrm.xg + (size_t)m * nrm.ldx + n;
