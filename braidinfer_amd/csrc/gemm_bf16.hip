@@ -498,13 +498,14 @@ __device__ __forceinline__ void quad_wait_loads() {
 }
 
 // Products of several experts in one launch (GROUPED): expert e's activation rows are the pairs first[e] .. first[e + 1] - 1
-// (rows of A themselves, or with `order` the rows order[p] / top), its weights lie N rows behind the expert before.  With
+// (rows of A themselves, or with `order` the rows order[p] / top; `per` is 2^32 / top rounded up, or 0 where that is not exact), its weights lie N rows behind the expert before.  With
 // the gated epilogue weight row v of a tile is gate row 8 (v / 16) + v % 16 or, from v % 16 = 8 on, the up row N / 2 behind
 // it, so that the matrices stay as they are stacked; `alpha` > 0: the clamped unit.
 struct QuadGroups {
     const int* first;
     const int* order;
     int experts, top;
+    unsigned per;
     float limit, alpha;
 };
 __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr) {
@@ -517,56 +518,114 @@ __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr
 }
 
 // acc[i][j][r]: weight row (output column) n1 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, activation
-// row m1 + 32 j + lane % 32.  Needs ldc % 4 == 0 and C aligned to 16 bytes.
-template <int TI, int TJ, int MODE, bool GROUPED>
-__device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __restrict__ C, int M, int N, size_t ldc,
-                                              int m1, int n1, int lane, const QuadGroups& gr) {
+// row m1 + 32 WVM j + lane % 32.  Needs ldc % 4 == 0 and C aligned to 16 bytes.
+// What is only written goes through the wave's piece of LDS, 32 rows at a time, so that an instruction writes whole runs of rows: as
+// the blocks lie, it would write 16 or 32 bytes of each of 32 rows, and 256 workgroups that end a round together wait for the L2's
+// requests.  8,192 x 8,192 by K = 1,024 in bfloat16 153 -> 130 us; 6,144 x 4,096 by 3,625 rows 155.5 -> 150, by 7,001 rows 282 -> 272; float
+// 12,288 x 4,096 by 7,001 rows 573 -> 565.  What is added to stays as the blocks lie: its reads and writes fill the memory's time
+// either way, and through LDS (with up to half of the values asked for some k-tiles ahead) 4,096 x 4,096 by 3,625 and 5,018 rows took
+// 112.5 and 167 us against 111.5 and 164, 4,096 x 14,336 by 7,001 rows 674 against 648.
+template <int TI, int MODE>
+struct QuadStrip {
+    static constexpr int ES = MODE == OUT_BF16 || MODE == OUT_SWIGLU ? 2 : 4;            // bytes of an element
+    static constexpr int RB = TI * 32 / (MODE == OUT_SWIGLU ? 2 : 1) * ES;                // of a row
+    static constexpr int LD = RB + 16;                                                   // from row to row, off the banks' stride
+    static constexpr int BYTES = MODE == OUT_F32_ACC ? 0 : 32 * LD;
+};
+template <int TI, int TJ, int WVM, int MODE, bool GROUPED>
+__device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __restrict__ C, int M, int N, size_t ldc, int m1, int n1, int lane,
+                                              const QuadGroups& gr, unsigned char* lds) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    if constexpr (MODE == OUT_F32_ACC) {
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-        const int m = m1 + j * 32 + (lane & 31);
-        if (m >= M) continue;
+        for (int j = 0; j < TJ; ++j) {
+            const int m = m1 + j * 32 * WVM + (lane & 31);
+            if (m >= M) continue;
 #pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            const int nb = n1 + i * 32 + 4 * (lane >> 5);
-            if (MODE == OUT_SWIGLU) {
+            for (int i = 0; i < TI; ++i) {
+                const int nb = n1 + i * 32 + 4 * (lane >> 5);
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int n = nb + 16 * h;                      // gate columns n .. n + 3, N a multiple of 16
-                    if (n >= N) continue;
-                    bf16x4 v;
+                for (int q = 0; q < 4; ++q) {
+                    const int n = nb + 8 * q;
+                    const size_t at = (size_t)m * ldc + n;
+                    if (n + 3 < N) {
+                        f32x4 v = *(const f32x4*)((float*)C + at);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        v[e] = (bf16)(GROUPED ? quad_glu(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e], gr)
-                                              : silu_mul(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]));
-                    *(bf16x4*)((bf16*)C + (size_t)m * ldc + (n >> 4) * 8 + (n & 7)) = v;
+                        for (int e = 0; e < 4; ++e) v[e] += acc[i][j][4 * q + e];
+                        *(f32x4*)((float*)C + at) = v;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (n + e < N) store_out<MODE>(C, at + e, acc[i][j][4 * q + e]);
+                    }
                 }
-                continue;
             }
+        }
+    } else {
+        struct __attribute__((packed, aligned(8))) Out { unsigned w[4]; };               // bfloat16 rows are aligned to 8 bytes
+        typedef QuadStrip<TI, MODE> S;
+        constexpr int CH = S::RB / 16, EL = 16 / S::ES;                                  // pieces of 16 bytes of a row, elements of one
+        if (MODE == OUT_SWIGLU) {
+            N >>= 1;
+            n1 >>= 1;
+        }
+        unsigned char* const put = lds + (lane & 31) * S::LD + 4 * (lane >> 5) * S::ES;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = nb + 8 * q;
-                const size_t at = (size_t)m * ldc + n;
-                if (n + 3 < N) {
+        for (int j = 0; j < TJ; ++j) {
+            const int mj = m1 + j * 32 * WVM;
+            if (mj >= M) break;
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+                if (MODE == OUT_SWIGLU) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {                   // gate rows 32 i + 16 h + 4 (lane / 32) + 0 .. 3, up rows 8 on
+                        bf16x4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            v[e] = (bf16)(GROUPED ? quad_glu(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e], gr)
+                                                  : silu_mul(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]));
+                        *(bf16x4*)(put + (16 * i + 8 * h) * 2) = v;
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
                     if (MODE == OUT_BF16) {
                         bf16x4 v;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) v[e] = (bf16)acc[i][j][4 * q + e];
-                        *(bf16x4*)((bf16*)C + at) = v;
+                        *(bf16x4*)(put + (32 * i + 8 * q) * 2) = v;
                     } else {
                         f32x4 v;
-                        if (MODE == OUT_F32_ACC) v = *(const f32x4*)((float*)C + at);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = (MODE == OUT_F32_ACC ? v[e] : 0.f) + acc[i][j][4 * q + e];
-                        *(f32x4*)((float*)C + at) = v;
+                        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * q + e];
+                        *(f32x4*)(put + (32 * i + 8 * q) * 4) = v;
                     }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < N) store_out<MODE>(C, at + e, acc[i][j][4 * q + e]);
                 }
             }
+            // (the wave's own writes and reads of LDS are executed in order)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int t = 0; t < CH / 2; ++t) {
+                const int c = t * 64 + lane, row = c / CH, piece = c % CH, m = mj + row, n = n1 + piece * EL;
+                if (m >= M || n >= N) continue;
+                const unsigned char* from = lds + row * S::LD + piece * 16;
+                const size_t at = (size_t)m * ldc + n;
+                if (n + EL <= N) {
+                    if (S::ES == 2) *(Out*)((bf16*)C + at) = *(const Out*)from;
+                    else *(f32x4*)((float*)C + at) = *(const f32x4*)from;
+                } else {
+                    for (int e = 0; e < EL && n + e < N; ++e) {
+                        if (S::ES == 2) ((bf16*)C)[at + e] = ((const bf16*)from)[e];
+                        else ((float*)C)[at + e] = ((const float*)from)[e];
+                    }
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
     }
 }
@@ -579,76 +638,30 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     constexpr int SA = BM * 128, SB = BN * 128;          // bytes of a stage of activation rows, of weight rows
     constexpr int WVN = 4 / WVM;                         // the four waves: WVM along the activation rows x WVN
     constexpr int TI = BN / WVN / 32, TJ = BM / WVM / 32; // blocks of a wave: weight rows, activation rows
-    constexpr int NM = TI * TJ;                          // matrix instructions per k-step of 16
     constexpr int LA = BM / 32, LB = BN / 32;            // wave-loads per wave and stage
     // An operand with three stages is asked for during the first three k-steps of 16 of a k-tile, into the
     // stage that the barrier before freed, and has a whole k-tile more to arrive; one with two stages after
     // the barrier, into the stage just read.  Either way k-tile t asks for k-tile t + 2.
     constexpr bool EARLY_A = NSA == 3, EARLY_B = NSB == 3;
-    constexpr int NEARLY = (EARLY_A ? LA : 0) + (EARLY_B ? LB : 0), NLATE = LA + LB - NEARLY;
     static_assert((WVM == 2 || WVM == 4) && BM % (32 * WVM) == 0 && BN % (32 * WVN) == 0 && BM % 32 == 0 && BN % 32 == 0 &&
                       NSA * SA + NSB * SB <= 160 * 1024 && TI * TJ * 16 <= 256, "tile");
     static_assert((NSA == 2 || NSA == 3) && (NSB == 2 || NSB == 3), "two or three stages an operand");
-    static_assert(TI + TJ <= NM && NLATE <= 2 * NM, "schedule");
+    static_assert(TI + TJ <= TI * TJ, "schedule");
+    static_assert(4 * QuadStrip<TI, MODE>::BYTES <= NSA * SA + NSB * SB, "the epilogue's strips");
     __shared__ __attribute__((aligned(1024))) unsigned char st[NSA * SA + NSB * SB];
     // blockIdx.y: which run of k-tiles this workgroup sums (one run, or the parts of a split product, each
     // into a float matrix of its own `part_stride` elements on; runs start at an even k-tile)
     void* C = MODE == OUT_F32 ? (void*)((float*)C_ + blockIdx.y * part_stride) : C_;
     const int kt0 = (int)blockIdx.y * kt_per_part;
-    int total = tiles_m * tiles_n;
-    int pid = blockIdx.x;
-    if constexpr (GROUPED) {                             // the tiles that the experts' pairs make; the grid is a bound
-        int sum = 0;
-        for (int e = threadIdx.x & 63; e < gr.experts; e += 64) sum += (gr.first[e + 1] - gr.first[e] + BM - 1) / BM;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-        total = __builtin_amdgcn_readfirstlane(sum) * tiles_n;
-        if (pid >= total) return;
-    }
-    {
-        const int per = total / 8, xcd = pid % 8, idx = pid / 8;
-        if (pid < per * 8) pid = xcd * per + idx;
-    }
-    int m0, n0;
-    if constexpr (GROUPED) {                             // expert by expert, an expert's row tiles of the same weights in turn
-        int e = 0, p0 = 0, nt = 0, before = 0;
-        for (int e0 = 0, run = 0; e0 < gr.experts; e0 += 64) {
-            const int l = e0 + (threadIdx.x & 63);
-            const int a = l < gr.experts ? gr.first[l] : 0, b = l < gr.experts ? gr.first[l + 1] : 0;
-            const int mine = (b - a + BM - 1) / BM * tiles_n;
-            int sum = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if ((int)(threadIdx.x & 63) >= o) sum += v;
-            }
-            const unsigned long long here = __ballot(run + sum > pid && run + sum - mine <= pid);
-            if (here) {
-                const int at = __ffsll(here) - 1;
-                e = e0 + at;
-                p0 = __builtin_amdgcn_readlane(a, at);
-                M = __builtin_amdgcn_readlane(b, at);
-                nt = __builtin_amdgcn_readlane(mine, at) / tiles_n;
-                before = run + __builtin_amdgcn_readlane(sum - mine, at);
-                break;
-            }
-            run += __builtin_amdgcn_readlane(sum, 63);
-        }
-        const int in = pid - before;
-        m0 = p0 + in % nt * BM;
-        n0 = in / nt * BN;
-        W += (size_t)e * N * K;
-    } else {
-        const int grp = pid / (8 * tiles_m), in = pid - grp * 8 * tiles_m;
-        int gn = tiles_n - grp * 8;
-        if (gn > 8) gn = 8;
-        const int tile_n = grp * 8 + in % gn, tile_m = in / gn;
-        m0 = tile_m * BM, n0 = tile_n * BN;
-    }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = (wave / WVN) * (BM / WVM), wn = (wave % WVN) * (BN / WVN);
+    const int wm = (wave / WVN) * 32, wn = (wave % WVN) * (BN / WVN);   // a wave's blocks of activation rows lie 32 WVM apart
     const int lrow = lane & 31, g = lane >> 5;
+    int nk = K / DMA_BK - kt0;                                         // k-tiles of this run
+    if (nk > kt_per_part) nk = kt_per_part;
+    const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)st);
 
+    // One tile: rows m0 .. of A up to row m_end against the weight rows n0 .. of W_, k-tiles kt0 .. kt0 + nk.
+    auto tile = [&](const bf16* A_, const bf16* W_, int m0, int n0, int m_end) {
     f32x16 acc[TI][TJ];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
@@ -663,7 +676,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     int row0 = 0;
     if constexpr (GROUPED) {
         if (!gr.order) {
-            A += (size_t)m0 * lda;
+            A_ += (size_t)m0 * lda;
             row0 = m0;
         }
     }
@@ -674,9 +687,9 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         const int c = (lane & 7) ^ ((R >> 1) & 7);
         if (q < LA) {
             int r = m0 + R;
-            if (r > M - 1) r = M - 1;
+            if (r > m_end - 1) r = m_end - 1;
             if constexpr (GROUPED) {
-                r = gr.order ? gr.order[r] / gr.top : r - row0;
+                r = gr.order ? (gr.per ? (int)__umulhi((unsigned)gr.order[r], gr.per) : gr.order[r] / gr.top) : r - row0;
             }
             offA[q] = (unsigned)((size_t)r * lda * 2 + c * 16);
         }
@@ -688,11 +701,10 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         }
     }
     // at the next k-tile to ask for
-    unsigned long long baseA = (unsigned long long)A + (size_t)kt0 * 128;
-    unsigned long long baseW = (unsigned long long)W + (wl ? (size_t)(kt0 >> 1) * (WL_BLOCK_ELEMS * 2) : (size_t)kt0 * 128);
+    unsigned long long baseA = (unsigned long long)A_ + (size_t)kt0 * 128;
+    unsigned long long baseW = (unsigned long long)W_ + (wl ? (size_t)(kt0 >> 1) * (WL_BLOCK_ELEMS * 2) : (size_t)kt0 * 128);
     int knext = kt0;
     const unsigned hopW = wl ? WL_BLOCK_ELEMS * 2 - 128 : 128;                        // bytes from an odd k-tile on
-    const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)st);
     // where this wave's loads of the next k-tile to ask for land, and which stage that is
     unsigned ldsA = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
     unsigned ldsB = __builtin_amdgcn_readfirstlane(lds0 + NSA * SA + wave * 1024);
@@ -716,17 +728,6 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         constexpr int q = decltype(q_)::value;
         quad_load<q * 4096>(ldsB, offB[q], baseW);
     };
-    // the x-th early load (A's first where both operands are early), the x-th late load
-    auto early = [&](auto x_) {
-        constexpr int x = decltype(x_)::value;
-        if constexpr (EARLY_A && x < LA) loadA(x_);
-        else loadB(std::integral_constant<int, x - (EARLY_A ? LA : 0)>{});
-    };
-    auto late = [&](auto x_) {
-        constexpr int x = decltype(x_)::value;
-        if constexpr (!EARLY_A && x < LA) loadA(x_);
-        else loadB(std::integral_constant<int, x - (!EARLY_A ? LA : 0)>{});
-    };
     auto next_tile = [&]() {                       // the pointers and the stages to load go on by a k-tile
         baseA += 128;
         baseW += (knext & 1) ? hopW : 128;
@@ -736,92 +737,218 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         ldsB += slotB == NSB - 1 ? (unsigned)(-(NSB - 1) * SB) : (unsigned)SB;
         slotB = slotB == NSB - 1 ? 0 : slotB + 1;
     };
-    // One k-step of 16 from operand set `use`: NM matrix instructions, and between them the LDS reads of set
-    // `use ^ 1` (k-step rk of the stage that ra/rb point into) and the direct loads [E0, E1) of the early
-    // ones or [L0, L1) of the late ones, evenly.
-    auto substep = [&](auto use_, auto rd_, auto rk_, auto e0_, auto e1_, auto l0_, auto l1_) {
-        constexpr int use = decltype(use_)::value, rk = decltype(rk_)::value;
-        constexpr bool RD = decltype(rd_)::value;
-        constexpr int E0 = decltype(e0_)::value, E1 = decltype(e1_)::value, L0 = decltype(l0_)::value, L1 = decltype(l1_)::value;
-        static_for<0, NM>([&](auto n_) {
-            constexpr int n = decltype(n_)::value;
-            // block (i, j): weight rows i (the instruction's first operand, so the result's rows), activation rows j
-            constexpr int i = n / TJ, j = (i & 1) ? TJ - 1 - n % TJ : n % TJ;
-            quad_mfma(acc[i][j], fb[use][i], fa[use][j]);
-            if constexpr (RD && n < TJ) quad_read<n * 4096>(fa[use ^ 1][n], ra[rk]);
-            if constexpr (RD && n >= TJ && n < TJ + TI) quad_read<(n - TJ) * 4096>(fb[use ^ 1][n - TJ], rb[rk]);
-            static_for<E0 + n * (E1 - E0) / NM, E0 + (n + 1) * (E1 - E0) / NM>(early);
-            static_for<L0 + n * (L1 - L0) / NM, L0 + (n + 1) * (L1 - L0) / NM>(late);
-        });
-        if constexpr (RD) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    };
-    using T = std::true_type;
-    using F = std::false_type;
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I3 = std::integral_constant<int, 3>;
-    // One k-tile from the stages in use.  Not LAST: before its last k-step every wave waits for its own
-    // loads of the next k-tile (the early ones of the one after may be on their way) and for the others at
-    // a barrier, which also says that all have read these stages; then it reads the next k-tile's first
-    // operands.  LOADS: it asks for the k-tile two on, the early loads before the barrier, the late ones after.
-    auto step = [&](auto loads_, auto last_) {
-        constexpr bool LOADS = decltype(loads_)::value, LAST = decltype(last_)::value;
-        constexpr int NE = LOADS ? NEARLY : 0, NL = LOADS ? NLATE : 0;
-        using Z = std::integral_constant<int, 0>;
-        substep(I0{}, T{}, I1{}, Z{}, std::integral_constant<int, NE / 3>{}, Z{}, Z{});
-        substep(I1{}, T{}, I2{}, std::integral_constant<int, NE / 3>{}, std::integral_constant<int, 2 * NE / 3>{}, Z{}, Z{});
-        substep(I0{}, T{}, I3{}, std::integral_constant<int, 2 * NE / 3>{}, std::integral_constant<int, NE>{}, Z{}, Z{});
-        if constexpr (LAST) {
-            substep(I1{}, F{}, I0{}, Z{}, Z{}, Z{}, Z{});
-        } else {
-            quad_wait_loads<NE>();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            const unsigned da = curA == NSA - 1 ? (unsigned)(-(NSA - 1) * SA) : (unsigned)SA;
-            const unsigned db = curB == NSB - 1 ? (unsigned)(-(NSB - 1) * SB) : (unsigned)SB;
+    // The k-loop over TV blocks of activation rows a wave: all of a tile's, or fewer where its rows end.
+    auto run = [&](auto tv_) {
+        constexpr int TV = decltype(tv_)::value;
+        constexpr int NM = TI * TV, NR = TI + TV;  // matrix instructions and operand reads per k-step of 16
+        constexpr int LV = LA / TJ * TV;           // wave-loads of activation rows per wave and stage
+        constexpr int NEARLY = (EARLY_A ? LV : 0) + (EARLY_B ? LB : 0), NLATE = LV + LB - NEARLY;
+        static_assert(NLATE <= (TV == TJ ? 2 : 4) * NM, "schedule");
+        // the x-th early load (A's first where both operands are early), the x-th late load
+        auto early = [&](auto x_) {
+            constexpr int x = decltype(x_)::value;
+            if constexpr (EARLY_A && x < LV) loadA(x_);
+            else loadB(std::integral_constant<int, x - (EARLY_A ? LV : 0)>{});
+        };
+        auto late = [&](auto x_) {
+            constexpr int x = decltype(x_)::value;
+            if constexpr (!EARLY_A && x < LV) loadA(x_);
+            else loadB(std::integral_constant<int, x - (!EARLY_A ? LV : 0)>{});
+        };
+        // One k-step of 16 from operand set `use`: NM matrix instructions, and between them the LDS reads of set
+        // `use ^ 1` (k-step rk of the stage that ra/rb point into) and the direct loads [E0, E1) of the early
+        // ones or [L0, L1) of the late ones, evenly.
+        auto substep = [&](auto use_, auto rd_, auto rk_, auto e0_, auto e1_, auto l0_, auto l1_) {
+            constexpr int use = decltype(use_)::value, rk = decltype(rk_)::value;
+            constexpr bool RD = decltype(rd_)::value;
+            constexpr int E0 = decltype(e0_)::value, E1 = decltype(e1_)::value, L0 = decltype(l0_)::value, L1 = decltype(l1_)::value;
+            static_for<0, NM>([&](auto n_) {
+                constexpr int n = decltype(n_)::value;
+                // block (i, j): weight rows i (the instruction's first operand, so the result's rows), activation rows j
+                constexpr int i = n / TV, j = (i & 1) ? TV - 1 - n % TV : n % TV;
+                quad_mfma(acc[i][j], fb[use][i], fa[use][j]);
+                constexpr int R0 = NM >= NR ? (n < NR ? n : NR) : n * NR / NM, R1 = NM >= NR ? (n < NR ? n + 1 : NR) : (n + 1) * NR / NM;
+                static_for<R0, R1>([&](auto r_) {
+                    constexpr int r = decltype(r_)::value;
+                    if constexpr (RD && r < TV) quad_read<r * WVM * 4096>(fa[use ^ 1][r], ra[rk]);
+                    if constexpr (RD && r >= TV) quad_read<(r - TV) * 4096>(fb[use ^ 1][r - TV], rb[rk]);
+                });
+                static_for<E0 + n * (E1 - E0) / NM, E0 + (n + 1) * (E1 - E0) / NM>(early);
+                static_for<L0 + n * (L1 - L0) / NM, L0 + (n + 1) * (L1 - L0) / NM>(late);
+            });
+            if constexpr (RD) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        };
+        using T = std::true_type;
+        using F = std::false_type;
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        // One k-tile from the stages in use.  Not LAST: before its last k-step every wave waits for its own
+        // loads of the next k-tile (the early ones of the one after may be on their way) and for the others at
+        // a barrier, which also says that all have read these stages; then it reads the next k-tile's first
+        // operands.  LOADS: it asks for the k-tile two on, the early loads before the barrier, the late ones after.
+        auto step = [&](auto loads_, auto last_) {
+            constexpr bool LOADS = decltype(loads_)::value, LAST = decltype(last_)::value;
+            constexpr int NE = LOADS ? NEARLY : 0, NL = LOADS ? NLATE : 0;
+            using Z = std::integral_constant<int, 0>;
+            substep(I0{}, T{}, I1{}, Z{}, std::integral_constant<int, NE / 3>{}, Z{}, Z{});
+            substep(I1{}, T{}, I2{}, std::integral_constant<int, NE / 3>{}, std::integral_constant<int, 2 * NE / 3>{}, Z{}, Z{});
+            substep(I0{}, T{}, I3{}, std::integral_constant<int, 2 * NE / 3>{}, std::integral_constant<int, NE>{}, Z{}, Z{});
+            if constexpr (LAST) {
+                substep(I1{}, F{}, I0{}, Z{}, Z{}, Z{}, Z{});
+            } else {
+                quad_wait_loads<NE>();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                const unsigned da = curA == NSA - 1 ? (unsigned)(-(NSA - 1) * SA) : (unsigned)SA;
+                const unsigned db = curB == NSB - 1 ? (unsigned)(-(NSB - 1) * SB) : (unsigned)SB;
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {                           // reads: the next stages
-                ra[kk] += da;
-                rb[kk] += db;
+                for (int kk = 0; kk < 4; ++kk) {                       // reads: the next stages
+                    ra[kk] += da;
+                    rb[kk] += db;
+                }
+                curA = curA == NSA - 1 ? 0 : curA + 1;
+                curB = curB == NSB - 1 ? 0 : curB + 1;
+                substep(I1{}, T{}, I0{}, Z{}, Z{}, Z{}, std::integral_constant<int, NL>{});
+                if constexpr (LOADS) next_tile();
             }
-            curA = curA == NSA - 1 ? 0 : curA + 1;
-            curB = curB == NSB - 1 ? 0 : curB + 1;
-            substep(I1{}, T{}, I0{}, Z{}, Z{}, Z{}, std::integral_constant<int, NL>{});
-            if constexpr (LOADS) next_tile();
-        }
-    };
+        };
 
-    int nk = K / DMA_BK - kt0;                                         // k-tiles of this run
-    if (nk > kt_per_part) nk = kt_per_part;
-    static_for<0, LA>(loadA);                                          // the first two k-tiles
-    static_for<0, LB>(loadB);
-    next_tile();
-    if (nk > 1) {
-        static_for<0, LA>(loadA);
+        static_for<0, LV>(loadA);                                      // the first two k-tiles
         static_for<0, LB>(loadB);
         next_tile();
-        quad_wait_loads<LA + LB>();
-    } else {
-        quad_wait_loads<0>();
-    }
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    static_for<0, TJ>([&](auto n_) { quad_read<decltype(n_)::value * 4096>(fa[0][decltype(n_)::value], ra[0]); });
-    static_for<0, TI>([&](auto n_) { quad_read<decltype(n_)::value * 4096>(fb[0][decltype(n_)::value], rb[0]); });
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    // Statements that name the accumulators: what the compiler wrote into one (the zeroes) is written before
-    // its statement, and a matrix instruction must not read a register in the states right after its write.
-    static_for<0, NM>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
-    int t = 0;
-    for (; t + 2 < nk; ++t) step(T{}, F{});
-    for (; t + 1 < nk; ++t) step(F{}, F{});
-    step(F{}, T{});
+        if (nk > 1) {
+            static_for<0, LV>(loadA);
+            static_for<0, LB>(loadB);
+            next_tile();
+            quad_wait_loads<LV + LB>();
+        } else {
+            quad_wait_loads<0>();
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        static_for<0, TV>([&](auto n_) {
+            constexpr int n = decltype(n_)::value;
+            quad_read<n * WVM * 4096>(fa[0][n], ra[0]);
+        });
+        static_for<0, TI>([&](auto n_) {
+            constexpr int n = decltype(n_)::value;
+            quad_read<n * 4096>(fb[0][n], rb[0]);
+        });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        // Statements that name the accumulators: what the compiler wrote into one (the zeroes) is written before
+        // its statement, and a matrix instruction must not read a register in the states right after its write.
+        static_for<0, TI * TJ>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
+        int t = 0;
+        for (; t + 2 < nk; ++t) step(T{}, F{});
+        for (; t + 1 < nk; ++t) step(F{}, F{});
+        step(F{}, T{});
+    };
+    const int blocks = (m_end - m0 + 32 * WVM - 1) / (32 * WVM);       // of 32 rows a wave
+    if (blocks >= TJ) run(std::integral_constant<int, TJ>{});
+    else if (TJ > 3 && blocks == 3) run(std::integral_constant<int, (TJ > 3 ? 3 : 1)>{});
+    else if (TJ > 2 && blocks == 2) run(std::integral_constant<int, (TJ > 2 ? 2 : 1)>{});
+    else run(std::integral_constant<int, 1>{});
     // the last matrix instructions' results are not in their registers yet; the epilogue's reads of an
     // accumulator stay behind the statement that names it
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-    static_for<0, NM>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
-    quad_epilogue<TI, TJ, MODE, GROUPED>(acc, C, M, N, ldc, m0 + wm, n0 + wn, lane, gr);
+    static_for<0, TI * TJ>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
+    __builtin_amdgcn_s_barrier();                                      // every wave has read its last operands
+    asm volatile("" ::: "memory");
+    quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(acc, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, st + wave * QuadStrip<TI, MODE>::BYTES);
+    };
+
+    if constexpr (!GROUPED) {
+        const int total = tiles_m * tiles_n;
+        int pid = blockIdx.x;
+        const int per = total / 8, xcd = pid % 8, idx = pid / 8;
+        if (pid < per * 8) pid = xcd * per + idx;
+        const int grp = pid / (8 * tiles_m), in = pid - grp * 8 * tiles_m;
+        int gn = tiles_n - grp * 8;
+        if (gn > 8) gn = 8;
+        const int tile_n = grp * 8 + in % gn, tile_m = in / gn;
+        tile(A, W, tile_m * BM, tile_n * BN, M);
+    } else {
+        // Expert by expert, column of tiles by column, an expert's row tiles of the same weights in turn.  The columns are cut into
+        // eight runs of about equal cost, one to an XCD, whose workgroups take its tiles in turn.  (What a tile of few rows costs is its
+        // weights: shares of a whole tile's time.)
+        auto tile_cost = [](int rows) {
+            const int b = (rows + 32 * WVM - 1) / (32 * WVM);
+            return TJ != 4 ? 1 : b == 4 ? 15 : b == 3 ? 12 : b == 2 ? 10 : 9;
+        };
+        // this lane's expert of a block of 64: its pairs, tiles of one column and their cost, and those before it in the block
+        struct Lane { int a, b, nt, cost, nt0, cost0; };
+        auto wave_scan = [](int v) {                                   // v of this lane and all before
+            v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);            // row_shr 1, 2, 4, 8
+            v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+            v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+            v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+            v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);            // row_bcast 15, 31
+            v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+            return v;
+        };
+        auto lane_of = [&](int e0) {
+            Lane v;
+            const int e = e0 + lane;
+            v.a = e < gr.experts ? gr.first[e] : 0;
+            v.b = e < gr.experts ? gr.first[e + 1] : 0;
+            const int rows = v.b - v.a, rem = rows % BM;
+            v.nt = (rows + BM - 1) / BM;
+            v.cost = rows / BM * tile_cost(BM) + (rem ? tile_cost(rem) : 0);
+            v.nt0 = wave_scan(v.nt) - v.nt;
+            v.cost0 = wave_scan(v.cost) - v.cost;
+            return v;
+        };
+        auto last_lane = [](int v) { return __builtin_amdgcn_readlane(v, 63); };
+        Lane v = lane_of(0);
+        int cost = last_lane(v.cost0 + v.cost);
+        for (int e0 = 64; e0 < gr.experts; e0 += 64) {
+            const Lane u = lane_of(e0);
+            cost += last_lane(u.cost0 + u.cost);
+        }
+        // the tiles in front of the first column that starts at `at` or more of the cost of all columns
+        const int xcd = blockIdx.x % 8;
+        const long long whole = (long long)cost * tiles_n;
+        long long at[2] = {whole * xcd / 8, whole * (xcd + 1) / 8};
+        int edge[2] = {0, 0};
+        for (int e0 = 0, nt0 = 0, cost0 = 0; e0 < gr.experts; e0 += 64) {
+            if (e0) v = lane_of(e0);
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const long long d = at[x] - (long long)(cost0 + v.cost0) * tiles_n;     // of the cost, behind this expert's start
+                const unsigned long long behind = __ballot(d > 0 && v.cost > 0);
+                if (behind) {
+                    const int l = 63 - __clzll(behind), c = __builtin_amdgcn_readlane(v.cost, l);
+                    const long long dl = at[x] - (long long)(cost0 + __builtin_amdgcn_readlane(v.cost0, l)) * tiles_n;
+                    const int cols = dl >= (long long)c * tiles_n ? tiles_n : (int)(((unsigned)dl + c - 1) / (unsigned)c);
+                    edge[x] = (nt0 + __builtin_amdgcn_readlane(v.nt0, l)) * tiles_n + cols * __builtin_amdgcn_readlane(v.nt, l);
+                }
+            }
+            nt0 += last_lane(v.nt0 + v.nt);
+            cost0 += last_lane(v.cost0 + v.cost);
+        }
+        for (int job = edge[0] + (int)(blockIdx.x / 8); job < edge[1]; job += (int)(gridDim.x / 8)) {
+            int e = 0, p0 = 0, end = 0, nt = 1, before = 0;
+            for (int e0 = 0, nt0 = 0; e0 < gr.experts; e0 += 64) {
+                if (gr.experts > 64) v = lane_of(e0);
+                const unsigned long long here = __ballot((nt0 + v.nt0) * tiles_n <= job && job < (nt0 + v.nt0 + v.nt) * tiles_n);
+                if (here) {
+                    const int l = __ffsll(here) - 1;
+                    e = e0 + l;
+                    p0 = __builtin_amdgcn_readlane(v.a, l);
+                    end = __builtin_amdgcn_readlane(v.b, l);
+                    nt = __builtin_amdgcn_readlane(v.nt, l);
+                    before = (nt0 + __builtin_amdgcn_readlane(v.nt0, l)) * tiles_n;
+                    break;
+                }
+                nt0 += last_lane(v.nt0 + v.nt);
+            }
+            const int in = job - before;
+            tile(A, W + (size_t)e * N * K, p0 + in % nt * BM, in / nt * BN, end);
+            __builtin_amdgcn_s_barrier();                              // the strips have been read, the stages may be filled again
+        }
+    }
 }
 
 static int launch_split_sum(const float* scratch, int parts, void* C, int M, int N, size_t ldc, int mode, hipStream_t s);
@@ -3054,8 +3181,8 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
     // no more tiles than the pairs make when every expert's last one is nearly empty
     const int tn = (N + BN - 1) / BN, nk = K / DMA_BK;
     const long long tm = (long long)pairs / BM + (gr.experts < pairs ? gr.experts : pairs);
-    if (tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
-    const unsigned grid = (unsigned)(tm * tn);
+    if (tm * tn > 0x7fffffc0LL) return BR_BAD_ARG;
+    const unsigned grid = (unsigned)((tm * tn + 7) / 8 * 8);
 #define BR_EXPERTS(MODE_) \
     gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, MODE_, true><<<grid, 256, 0, s>>>(A, W, C, 0, N, K, (size_t)K, ldc, 0, tn, nk, 0, WL_ROWS, gr)
     if (mode == OUT_SWIGLU) BR_EXPERTS(OUT_SWIGLU);
@@ -3096,7 +3223,8 @@ extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, 
     if (!br_experts_tiles_takes(N, K) || E <= 0 || top <= 0 || (gated && !out_is_bf16) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 != 0 ||
         !quad_takes(C, order ? a_rows : min(a_rows, 256), N, K, K, ldc))
         return BR_BAD_ARG;
-    const QuadGroups gr = {first, order, E, top, limit, alpha};
+    const bool exact = top > 1 && (unsigned long long)pairs * top < (1ull << 32);
+    const QuadGroups gr = {first, order, E, top, exact ? (unsigned)(((1ull << 32) + top - 1) / top) : 0u, limit, alpha};
     const int mode = gated ? OUT_SWIGLU : out_is_bf16 ? OUT_BF16 : OUT_F32;
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
