@@ -3201,28 +3201,19 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
     return br_check_launch();
 }
 
-// 128x256 or 256x256 tiles: the fewer rounds of workgroups by the times a k-tile of `choose_quad`, with every expert's pairs
-// taken as the mean and half a standard deviation of evenly drawn ones, rounded up to tiles (their real numbers stay on the
-// device).  32 experts of 1,792 by 4,096, 8 chosen, gated product / down in us with 128 rows a tile against 256: 200 tokens
-// 179 / 102 against 228 / 112, 800 tokens 295 / 162 against 255 / 135, 1,200 tokens 417 / 213 against 432 / 217, 1,800 tokens
-// 500 / 279 against 445 / 231 (1.19 and 0.91 PFLOP/s), 8,000 tokens 1,892 / 1,208 against 1,626 / 955.  Before, the rows
-// copied into the experts' order, tiles of 128x128 through registers and the unit in a launch of its own: 234 / 122, 522 /
-// 267, 782 / 387, 1,074 / 543; 8,000 tokens expert by expert 2,365 / 1,115.
-// The down product (`gated` false) has a short k and writes float rows: from four rounds of 128-row tiles on the taller tile gains more there than
-// the k-tiles say.  The same experts, down in us with 128 rows a tile against 256, scores drawn evenly and unevenly: 1,000 tokens 188 / 191
-// against 173 / 173, 1,400 tokens 220 / 246 against 211 / 204, 2,400 tokens 362 / 388 against 317 / 312; 16 experts of 1,408 by 2,048, 4 chosen,
-// 5,000 tokens 148 / 148 against 133 / 131; with fewer rounds: 600 tokens 33 / 31 against 43 / 42, 2,400 tokens 74 / 73 against 83 / 82.
+// 128x256 or 256x256 tiles, by the pairs an expert on average (their real numbers stay on the device) and the rounds of workgroups that
+// tiles of 128 rows make.  A tile multiplies only the blocks of 64 rows that it has, so what is counted against the taller tile is the
+// experts with few pairs, whose weights it streams by fewer workgroups.  32 experts of 1,792 by 4,096, us with 128 rows a tile against
+// 256, rows an expert uneven as random weights draw them (half to twice the mean):
+//   gated product: 112 pairs on average 226 / 208, 150 225 / 243 (another draw 230 / 286), 225 323 / 345, 300 343 / 341, 450 480 / 483, 603
+//     615 / 567, 675 680 / 652;  equal rows: 128 192 / 198, 160 257 / 226, 200 279 / 252, 256 294 / 261, 300 364 / 427, 400 440 / 443
+//   down (short k, float rows): 112 132 / 139, 150 155 / 153, 225 184 / 168, 300 215 / 203, 450 290 / 273, 603 363 / 327, 675 412 / 375;
+//     equal rows: 128 117 / 118, 160 151 / 125, 256 170 / 149, 300 207 / 213, 400 264 / 238
+// With fewer than four rounds too few workgroups are left: 16 experts of 1,408 by 2,048, 4 chosen, down: 600 tokens 33 / 43, 2,400 tokens
+// 74 / 82, but 5,000 tokens 148 / 133.
 static bool experts_tall_tiles(int pairs, int E, int N, bool gated, int cus) {
-    const double mean = (double)pairs / E, high = mean + 0.5 * sqrt(mean);
-    double t[2];
-    bool many = false;
-    for (int i = 0; i < 2; ++i) {
-        const int bm = i ? 256 : 128, k = i ? 0 : 1;
-        const double units = E * ceil(high / bm) * ((N + 255) / 256), whole = floor(units / cus), share = units / cus - whole;
-        if (i == 0) many = units >= 4.0 * cus;
-        t[i] = whole * QUAD_FULL[k] + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) * QUAD_FULL[k] : 0.0);
-    }
-    return t[1] <= (!gated && many ? 1.2 : 1.03) * t[0];
+    const double mean = (double)pairs / E, units = E * ceil(mean / 128) * ((N + 255) / 256);
+    return units >= 4.0 * cus && mean >= (gated ? 448.0 : 136.0);
 }
 
 extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, const int* order, void* C, int gated, int out_is_bf16,
