@@ -12,6 +12,8 @@
 //
 // reference: op_linear_proj, kernels/megakernel_ops.hip:166-276 (one block per output row, f32 accumulate).
 #include "common.h"
+#include <algorithm>
+#include <type_traits>
 
 #define F32_BM 64
 #define F32_BN 64
@@ -175,18 +177,29 @@ __global__ __launch_bounds__(512) void gemm_f32_stream_kernel(const float* __res
     }
 }
 
-// Any M: 16 TJ rows x 128 columns by four waves along the columns (16 TJ x 32 each), two LDS stages of 32 k by direct loads,
-// bound by the matrix cores: 28,672 x 4,096 at 64 / 279 / 2,048 rows 188 / 634 / 3,573 us (80 / 103 / 135 TFLOP/s; the 64x64
-// tiles of one thread a sum 678 / 2,442 / 12,669), 4,096 x 14,336 at 279 rows 281 (2,078; segments apart).  Error against 64
-// bits at 64 rows of 4,096: 4.1e-7 of the norm, 1.1e-6 with one ascending sum.
-// TJ is chosen so that the rows fill their tiles (279 rows: three of 96).  SPLIT: segment
-// blockIdx.y alone, into a matrix of its own.  The accumulators hold the product transposed: four columns of a row a lane.
+// Any M: 16 TJ rows x 64 columns by four waves along the columns (16 TJ x 16 each), two workgroups to a compute unit, a ring of two or three
+// LDS stages of 32 k by direct loads, bound by the matrix cores.  A wave has the operands of 16 k in registers twice: while one set is
+// multiplied, the other is read from LDS and the direct loads of the stage that is two or three on are asked for one at a time (the
+// path into LDS takes one of them per 16 cycles: bunched behind the barrier they held up the products).  28,672 x 4,096 at 20 / 128 / 279 / 450
+// rows 105 -> 92, 274 -> 257, 602 -> 553, 1,022 -> 912 us, 4,096 x 14,336 at 279 rows 279 -> 266 (123 TFLOP/s; a loop of the instruction alone
+// makes 155, at a clock of 2.4 GHz where this kernel is given 2.1 to 2.2).  Before: 128 columns by waves of 32, operands read before their products.
+// More stages, at one workgroup to a compute unit or two: nothing.  Error against 64 bits at 64 rows of 4,096: 4.1e-7 of the norm, 1.1e-6 with
+// one ascending sum.  TJ is chosen so that the rows fill their tiles (279 rows: three of 96).  SPLIT: segment blockIdx.y alone, into a
+// matrix of its own.  The accumulators hold the product transposed: four columns of a row a lane.
+#define F32_TN 64
+template <int N_, class F>
+__device__ __forceinline__ void f32_for(F&& f) {
+    if constexpr (N_ > 0) {
+        f32_for<N_ - 1>(f);
+        f(std::integral_constant<int, N_ - 1>{});
+    }
+}
 template <int TJ, int MODE, bool SPLIT>
-__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int M, int N, int K, size_t lda, size_t ldc,
                                                             int tiles_m, int a_aligned, int c_aligned) {
-    constexpr int BM = 16 * TJ, BN = 128, ROWB = 128, TI = 2, STAGE = (BM + BN) * ROWB;
-    __shared__ __attribute__((aligned(1024))) unsigned char st[2 * STAGE];
+    constexpr int BM = 16 * TJ, BN = F32_TN, ROWB = 128, STAGE = (BM + BN) * ROWB, S = TJ <= 3 || TJ == 5 ? 3 : 2;
+    __shared__ __attribute__((aligned(1024))) unsigned char st[S * STAGE];
     int pid = blockIdx.x;
     {
         const int total = gridDim.x, per = total / 8, xcd = pid % 8, idx = pid / 8;
@@ -200,101 +213,167 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     const int s0 = SPLIT ? (int)blockIdx.y : 0, s1 = SPLIT ? s0 + 1 : F32_SEGS;
     const int kt0 = s0 * nch / F32_SEGS * 2, kt1 = s1 * nch / F32_SEGS * 2;      // stages of 32 k
     auto sw = [](int row) { return (row >> 1) & 7; };
-    auto issue = [&](int kt) {
-        const unsigned base = __builtin_amdgcn_readfirstlane(lds0 + (kt & 1) * STAGE);
-        const int k0 = kt * 32;
-#pragma unroll
-        for (int q = 0; q < BM / 8; q += 4)
-            if (q + wave < BM / 8)
-                f32_bring<ROWB>(base + (q + wave) * 1024, (q + wave) * 8, lane, a_aligned, false,
-                                [&](int row, int col) { return A + (size_t)min(m0 + row, M - 1) * lda + k0 + col * 4; }, sw);
-#pragma unroll
-        for (int q = 0; q < BN / 8; q += 4)
-            f32_bring<ROWB>(base + BM * ROWB + (q + wave) * 1024, (q + wave) * 8, lane, true, false,
+    constexpr int NA = (BM / 8 + 3) / 4, NB = BN / 32;         // a wave's loads of a stage (four times NA where rows lie anywhere)
+    // load q of stage kt: of activation rows, then of weight rows
+    auto bring = [&](auto aligned_, int q, unsigned base, int k0) {
+        constexpr bool ALIGNED = decltype(aligned_)::value;
+        if (q < NA) {
+            const int r8 = min(4 * q + wave, BM / 8 - 1);     // (every wave has the same number of loads on its way; the last rows twice)
+            f32_bring<ROWB>(base + r8 * 1024, r8 * 8, lane, ALIGNED, false,
+                            [&](int row, int col) { return A + (size_t)min(m0 + row, M - 1) * lda + k0 + col * 4; }, sw);
+        } else {
+            const int r8 = 4 * (q - NA) + wave;
+            f32_bring<ROWB>(base + BM * ROWB + r8 * 1024, r8 * 8, lane, true, false,
                             [&](int row, int col) { return W + (size_t)min(n0 + row, N - 1) * K + k0 + col * 4; }, sw);
+        }
     };
-    f32x4 acc[TI][TJ], sum[TI][TJ];
+    auto stage_at = [&](int kt) { return __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(kt - kt0) % S * STAGE); };
+    auto issue = [&](int kt) {
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+        for (int q = 0; q < NA + NB; ++q) {
+            if (a_aligned) bring(std::true_type{}, q, stage_at(kt), kt * 32);
+            else bring(std::false_type{}, q, stage_at(kt), kt * 32);
+        }
+    };
+    f32x4 acc[TJ], sum[TJ];
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) { acc[i][j][r] = 0.f; sum[i][j][r] = 0.f; }
-    if (kt0 < kt1) issue(kt0);
+        for (int r = 0; r < 4; ++r) { acc[j][r] = 0.f; sum[j][r] = 0.f; }
+    // Two sets of operands, of 16 k each: one is multiplied while the other is read from LDS.
+    struct Set { f32x4 wf, af[TJ]; };
+    auto read = [&](Set& o, int kt, int b, auto r_) {         // operand r of k-step b of stage kt
+        constexpr int r = decltype(r_)::value;
+        const unsigned char* ap = st + (unsigned)(kt - kt0) % S * STAGE;
+        const unsigned char* wp = ap + (BM + wave * 16) * ROWB;
+        const int col = ((4 * b + g) ^ sw(r16)) * 16;
+        if constexpr (r == 0) o.wf = *(const f32x4*)(wp + r16 * ROWB + col);
+        else o.af[r - 1] = *(const f32x4*)(ap + (16 * (r - 1) + r16) * ROWB + col);
+    };
+    // the products of a set, `then(n)` behind the n-th; what `then` does stays there
+    constexpr int NM = 4 * TJ;
+    auto multiply = [&](const Set& o, auto then) {
+        f32_for<NM>([&](auto n_) {
+            constexpr int e = decltype(n_)::value / TJ, j = decltype(n_)::value % TJ;
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.wf[e], o.af[j][e], acc[j], 0, 0, 0);
+            then(n_);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // operand reads behind every second product (TJ = 1 has fewer products than that takes: behind each)
+    auto reading = [&](Set& o, int kt, int b, auto n_) {
+        constexpr int n = decltype(n_)::value, each = NM >= 2 * (TJ + 1) ? 2 : 1;
+        if constexpr (n % each == 0 && n / each <= TJ) {
+            read(o, kt, b, std::integral_constant<int, n / each>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // all but the loads of the last `LEFT` stages asked for have come
+    auto arrived = [&](auto left_) {
+        constexpr int LEFT = decltype(left_)::value;
+        constexpr int FOURS = LEFT * (4 * NA + NB) < 63 ? LEFT * (4 * NA + NB) : 63;
+        static_assert(LEFT * (NA + NB) < 64, "vmcnt");
+        if (a_aligned) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT * (NA + NB)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(FOURS) : "memory");
+    };
+    Set x0, x1;
+    if (kt0 < kt1) {
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            if (kt0 + i < kt1) issue(kt0 + i);
+        if (kt0 + S <= kt1) arrived(std::integral_constant<int, S - 1>{});
+        else arrived(std::integral_constant<int, 0>{});
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        f32_for<TJ + 1>([&](auto r_) { read(x0, kt0, 0, r_); });
+    }
     int seg = s0, seg_end = (s0 + 1) * nch / F32_SEGS * 2;
     for (int kt = kt0; kt < kt1; ++kt) {
         while (kt == seg_end) {                               // a segment is whole: onto the sum, in order
 #pragma unroll
-            for (int i = 0; i < TI; ++i)
+            for (int j = 0; j < TJ; ++j)
 #pragma unroll
-                for (int j = 0; j < TJ; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) { sum[i][j][r] += acc[i][j][r]; acc[i][j][r] = 0.f; }
+                for (int r = 0; r < 4; ++r) { sum[j][r] += acc[j][r]; acc[j][r] = 0.f; }
             ++seg;
             seg_end = (seg + 1) * nch / F32_SEGS * 2;
         }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        multiply(x0, [&](auto n_) { reading(x1, kt, 1, n_); });
+        // the next stage has come, and this one has been read by all waves: it is asked for again behind the barrier
+        if (kt + S <= kt1) arrived(std::integral_constant<int, S - 2>{});
+        else arrived(std::integral_constant<int, 0>{});
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (kt + 1 < kt1) issue(kt + 1);
-        const unsigned char* ap = st + (kt & 1) * STAGE;
-        const unsigned char* wp = ap + (BM + wave * 32) * ROWB;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            f32x4 af[TJ], wf[TI];
-#pragma unroll
-            for (int i = 0; i < TI; ++i) wf[i] = *(const f32x4*)(wp + (16 * i + r16) * ROWB + (((4 * b + g) ^ sw(r16)) * 16));
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) af[j] = *(const f32x4*)(ap + (16 * j + r16) * ROWB + (((4 * b + g) ^ sw(r16)) * 16));
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < TI; ++i)
-#pragma unroll
-                    for (int j = 0; j < TJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
+        const bool more = kt + S < kt1;
+        if (more && !a_aligned) issue(kt + S);
+        if (more && a_aligned) {
+            const unsigned base = stage_at(kt + S);
+            const int k0 = (kt + S) * 32;
+            multiply(x1, [&](auto n_) {
+                reading(x0, kt + 1, 0, n_);
+                f32_for<NA + NB>([&](auto q_) {
+                    constexpr int q = decltype(q_)::value;
+                    if constexpr (decltype(n_)::value == (2 * q + 1) * NM / (2 * (NA + NB))) {
+                        bring(std::true_type{}, q, base, k0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            });
+        } else if (kt + 1 < kt1) {
+            multiply(x1, [&](auto n_) { reading(x0, kt + 1, 0, n_); });
+        } else {
+            multiply(x1, [](auto) {});
         }
-        // every wave's reads of this stage are waited for ahead of the loop's next barrier, behind which the loads of the one after go into it
     }
     if (SPLIT) C += (size_t)blockIdx.y * M * N;
+    const int n = n0 + wave * 16 + 4 * g;
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
         const int m = m0 + 16 * j + r16;
         if (m >= M) continue;
+        float* c = C + (size_t)m * ldc + n;
+        f32x4 v = sum[j];
 #pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            const int n = n0 + wave * 32 + 16 * i + 4 * g;
-            float* c = C + (size_t)m * ldc + n;
-            f32x4 v = sum[i][j];
+        for (int r = 0; r < 4; ++r) v[r] += acc[j][r];
+        if (c_aligned && n + 3 < N) {
+            if (MODE == 1) {
+                const f32x4 o = *(const f32x4*)c;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] += acc[i][j][r];
-            if (c_aligned && n + 3 < N) {
-                if (MODE == 1) {
-                    const f32x4 o = *(const f32x4*)c;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = o[r] + v[r];
-                }
-                *(f32x4*)c = v;
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < N) c[r] = MODE == 1 ? c[r] + v[r] : v[r];
+                for (int r = 0; r < 4; ++r) v[r] = o[r] + v[r];
             }
+            *(f32x4*)c = v;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) c[r] = MODE == 1 ? c[r] + v[r] : v[r];
         }
     }
 }
 
-// C (+)= the segments' matrices [F32_SEGS][M][N], added in order; a thread an element.
-template <int MODE>
+// C (+)= the segments' matrices [F32_SEGS][M][N], added in order; a thread VEC neighbours of a row.
+template <int MODE, int VEC>
 __global__ __launch_bounds__(256) void gemm_f32_segments_kernel(const float* __restrict__ part, float* __restrict__ C, int M, int N,
                                                                 size_t ldc) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, all = (size_t)M * N;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * VEC, all = (size_t)M * N;
     if (i >= all) return;
-    float v = 0.f;
+    vec p[F32_SEGS];
 #pragma unroll
-    for (int s = 0; s < F32_SEGS; ++s) v += part[s * all + i];
-    float* c = C + i / N * ldc + i % N;
-    *c = MODE == 1 ? *c + v : v;
+    for (int s = 0; s < F32_SEGS; ++s) p[s] = *(const vec*)(part + s * all + i);
+    const int row = (int)(i / (unsigned)N), col = (int)(i - (size_t)row * N);
+    float* c = C + (size_t)row * ldc + col;
+    vec v;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        v[e] = 0.f;
+#pragma unroll
+        for (int s = 0; s < F32_SEGS; ++s) v[e] += p[s][e];
+    }
+    if (MODE == 1) {
+        const vec o = *(const vec*)c;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[e] = o[e] + v[e];
+    }
+    *(vec*)c = v;
 }
 
 template <int XR>
@@ -318,25 +397,64 @@ static int launch_f32_stream(const float* A, const float* W, float* C, int M, in
     return br_check_launch();
 }
 
+template <int TJ, bool SPLIT>
+static int launch_f32_tiles(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int acc, int aligned,
+                            float* scratch, hipStream_t s) {
+    const int tm = (M + 16 * TJ - 1) / (16 * TJ), tn = (N + F32_TN - 1) / F32_TN;
+    if (SPLIT) {
+        const dim3 grid((unsigned)(tm * tn), F32_SEGS);
+        gemm_f32_tile_kernel<TJ, 0, SPLIT><<<grid, 256, 0, s>>>(A, W, scratch, M, N, K, lda, (size_t)N, tm, aligned, N % 4 == 0 && (uintptr_t)scratch % 16 == 0);
+        const size_t all = (size_t)M * N;
+        const bool fours = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C | (uintptr_t)scratch) % 16 == 0;
+        const unsigned blocks = (unsigned)(((fours ? all / 4 : all) + 255) / 256);
+        if (fours && acc) gemm_f32_segments_kernel<1, 4><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+        else if (fours) gemm_f32_segments_kernel<0, 4><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+        else if (acc) gemm_f32_segments_kernel<1, 1><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+        else gemm_f32_segments_kernel<0, 1><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
+    } else {
+        const int c_aligned = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+        if (acc) gemm_f32_tile_kernel<TJ, 1, SPLIT><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
+        else gemm_f32_tile_kernel<TJ, 0, SPLIT><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
+    }
+    return br_check_launch();
+}
+
+// Whole rounds of tiles (two workgroups to a compute unit) go as they are; the weight rows behind them, or all where there is no whole
+// round, segment by segment, every segment in a workgroup of its own, where that is counted the faster: in runs of columns whose
+// segments' sums fit the scratch.  In us: a tile's work at 0.5 MFLOP a us and compute unit (a lone workgroup 0.7 of two beside
+// each other), the segments' sums written and read at 4 TB/s, 8 for the launches.  279 rows by 28,672 x 4,096: 512 tiles of 1,344 twice, 320 in
+// segments: 553 us, 602 at once; 640 rows by 4,096 x 14,336, whose segments do not fit at once: 593 us, 864 with no segments; 350 rows by
+// 6,144 x 4,096 193, 254.
 template <int TJ>
 static int launch_f32_tile(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int acc, int aligned,
                            int cus, float* scratch, size_t scratch_floats, hipStream_t s) {
-    const int tm = (M + 16 * TJ - 1) / (16 * TJ), tn = (N + 127) / 128;
-    const long long tiles = (long long)tm * tn;
-    if (tiles > 0x7fffffffLL) return BR_BAD_ARG;
-    const int c_aligned = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
-    // fewer tiles than two a compute unit: every segment in a workgroup of its own
-    if (tiles < 2 * cus && K >= 512 && (size_t)F32_SEGS * M * N <= scratch_floats) {
-        const dim3 grid((unsigned)tiles, F32_SEGS);
-        gemm_f32_tile_kernel<TJ, 0, true><<<grid, 256, 0, s>>>(A, W, scratch, M, N, K, lda, (size_t)N, tm, aligned, N % 4 == 0 && (uintptr_t)scratch % 16 == 0);
-        const unsigned blocks = (unsigned)(((size_t)M * N + 255) / 256);
-        if (acc) gemm_f32_segments_kernel<1><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
-        else gemm_f32_segments_kernel<0><<<blocks, 256, 0, s>>>(scratch, C, M, N, ldc);
-        return br_check_launch();
+    const int tm = (M + 16 * TJ - 1) / (16 * TJ), tn = (N + F32_TN - 1) / F32_TN, round = 2 * cus;
+    if ((long long)tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
+    const double w = 2.0 * 16 * TJ * F32_TN * K / 0.5e6;
+    int whole = tn, run = 0;                                           // columns of tiles: as they are, of a run in segments
+    const int fit = (int)std::min<size_t>(scratch_floats / ((size_t)F32_SEGS * M * F32_TN), (size_t)tn);
+    if (K >= F32_KC * F32_SEGS && fit > 0) {
+        const int first = (int)((long long)tm * tn / round * round / tm), left = tn - first;
+        const long long rest = (long long)tm * left;
+        const double as_is = rest <= cus ? 1.4 * w : 2.0 * w;
+        const int runs = left > 0 ? (left + fit - 1) / fit : 0, each = runs ? (left + runs - 1) / runs : 0;
+        double in_segments = 0.0;
+        for (int c = 0; c < left; c += each) {
+            const long long u = (long long)tm * std::min(each, left - c) * F32_SEGS, tail = u % round;
+            in_segments += 8.0 + w / F32_SEGS * (2.0 * (u / round) + (tail == 0 ? 0.0 : tail <= cus ? 1.4 : 2.0)) + (double)u * 16 * TJ * F32_TN * 8 / 4e6;
+        }
+        if (left > 0 && in_segments < as_is) whole = first, run = each;
     }
-    if (acc) gemm_f32_tile_kernel<TJ, 1, false><<<(unsigned)tiles, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
-    else gemm_f32_tile_kernel<TJ, 0, false><<<(unsigned)tiles, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, aligned, c_aligned);
-    return br_check_launch();
+    if (whole > 0) {
+        const int rc = launch_f32_tiles<TJ, false>(A, W, C, M, std::min(N, whole * F32_TN), K, lda, ldc, acc, aligned, nullptr, s);
+        if (rc != BR_OK) return rc;
+    }
+    for (int c = whole; c < tn; c += run) {
+        const int n = c * F32_TN;
+        const int rc = launch_f32_tiles<TJ, true>(A, W + (size_t)n * K, C + n, M, std::min(N - n, run * F32_TN), K, lda, ldc, acc, aligned, scratch, s);
+        if (rc != BR_OK) return rc;
+    }
+    return BR_OK;
 }
 
 // `scratch`: room for the segments' sums of products with few tiles (null: none).

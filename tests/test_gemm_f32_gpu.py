@@ -46,3 +46,21 @@ def test_rows_that_lie_anywhere(M):
         K.gemm(wide_a[:, shift:shift + Kd], w, wide_o[:, shift:shift + N])
         assert torch.equal(wide_o[:, shift:shift + N], want)
         assert torch.all(wide_o[:, :shift] == 7.0) and torch.all(wide_o[:, shift + N:] == 7.0)
+
+
+# more tiles than two a compute unit: whole rounds, then segments in one run of columns, in several (a scratch that holds few), and in none
+@pytest.mark.parametrize("M,N", [(40, 33000), (150, 20500), (320, 7001), (600, 4096)])
+def test_whole_rounds_and_segments_behind_them(M, N):
+    from braidinfer_amd import kernels as K
+    Kd = 576
+    a, w, base = rnd(M, Kd, seed=6), rnd(N, Kd, seed=7), rnd(M, N, seed=8)
+    want = torch.empty(M, N, device="cuda")
+    for r in range(0, M, 16):                             # 16 rows at a time: the streaming kernel
+        K.gemm(a[r:r + 16], w, want[r:r + 16])
+    for floats in (0, 8 * M * 64, 8 * M * 640, 8 * M * 4096 + 3, 8 * M * N):
+        room = torch.empty(floats, device="cuda") if floats else None
+        out = torch.full((M, N), 7.0, device="cuda")
+        K.gemm(a, w, out, scratch=room)
+        assert torch.equal(out, want)
+        K.gemm(a, w, base.copy_(out), accumulate=True, scratch=room)
+        assert torch.equal(base, want + want)
