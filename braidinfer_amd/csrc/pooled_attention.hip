@@ -632,38 +632,18 @@ __device__ __forceinline__ bf16x8 pwa_load_vt8(const bf16* __restrict__ vrow, in
 // acc[r] the key 16 (r / 8) + 8 g + r % 8.
 __device__ __forceinline__ int pwa_key_of_row(int c) { return 16 * (c >> 4) + 8 * ((c >> 2) & 1) + 4 * ((c >> 3) & 1) + (c & 3); }
 
-// One block of 32 keys (rows kb .. kb + 31 of a unit): `kblock` is the block's first key row (rows `ks` elements
-// apart), `vblock` the first value channel at the block's first row (channels `vs` elements apart), in the cache
-// or in LDS; rows of the block from `limit` on are not written and their values read as zero.  A key is seen by
-// this lane's query if first_ok <= key <= last_ok.  EARLY: all of the block's keys and values are asked for before the
-// first product, without a branch between them (channels from dv on read the last row, and nobody writes what becomes of it;
-// a key row's elements from dk on, at most 127, are the next row's or the values' that follow the keys in a page, not used).
-template <int NBK, int NBV, bool EARLY = false>
-__device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int ks, const bf16* __restrict__ vblock, int vs,
-                                          int kb, int limit, int first_ok, int last_ok, int dk, int dv, int c, int g,
-                                          const bf16x8* qf, f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
-    const bf16* krow = kblock + (size_t)pwa_key_of_row(c) * ks;
-    bf16x8 ke[EARLY ? 2 * NBK : 1], ve[EARLY ? 2 * NBV : 1];
-    if constexpr (EARLY) {
-#pragma unroll
-        for (int s = 0; s < 2 * NBK; ++s)
-            ke[s] = *(const bf16x8*)(kblock + (unsigned)(pwa_key_of_row(c) * ks + 8 * g) + s * 16);
-#pragma unroll
-        for (int i = 0; i < 2 * NBV; ++i)
-            ve[i] = *(const bf16x8*)(vblock + (unsigned)(min(i / 2 * 32 + c, dv - 1) * vs + 8 * g) + (i & 1) * 16);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+// One block of 32 keys (rows kb .. kb + 31 of a unit): `key(s)` gives this lane's 8 elements s * 16 + 8 g .. of its key row, `value(i, h)` 8
+// values of channel 32 i + c at the rows 16 h + 8 g .. of the block; `between` runs behind the scores' products.  A key is seen
+// by this lane's query if first_ok <= key <= last_ok.
+template <int NBK, int NBV, class Key, class Value, class Between>
+__device__ __forceinline__ void pwa_block_of(Key key, Value value, Between between, int kb, int first_ok, int last_ok, int g, const bf16x8* qf,
+                                             f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
     f32x16 s_acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
 #pragma unroll
-    for (int s = 0; s < 2 * NBK; ++s) {
-        const int d = s * 16 + 8 * g;
-        bf16x8 kf;
-        if constexpr (EARLY) kf = d < dk ? ke[s] : pwa_zero8();
-        else kf = (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
-        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], s_acc, 0, 0, 0);
-    }
+    for (int s = 0; s < 2 * NBK; ++s) s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(key(s), qf[s], s_acc, 0, 0, 0);
+    between();
     if (cap_out != 0.f) {
         // bounded scores: cap tanh(s scale / cap), tanh z = 1 - 2 / (exp(2 z) + 1); cap_in = 2 log2(e) scale / cap and
         // cap_out = cap / scale, so that the multiplication by scale2 below leaves the bounded score in base 2
@@ -708,26 +688,51 @@ __device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int k
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc_o[i][r] *= corr;
         }
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 0), p1, acc_o[i], 0, 0, 0);
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 1), p2, acc_o[i], 0, 0, 0);
+    }
+}
+
+// The same with `kblock` the block's first key row (rows `ks` elements apart) and `vblock` the first value channel at the block's first row
+// (channels `vs` elements apart), in the cache or in LDS; rows of the block from `limit` on are not written and their values
+// read as zero.  EARLY: all of the block's keys and values are asked for before the
+// first product, without a branch between them (channels from dv on read the last row, and nobody writes what becomes of it;
+// a key row's elements from dk on, at most 127, are the next row's or the values' that follow the keys in a page, not used).
+template <int NBK, int NBV, bool EARLY = false>
+__device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int ks, const bf16* __restrict__ vblock, int vs,
+                                          int kb, int limit, int first_ok, int last_ok, int dk, int dv, int c, int g,
+                                          const bf16x8* qf, f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
+    const bf16* krow = kblock + (size_t)pwa_key_of_row(c) * ks;
+    bf16x8 ke[EARLY ? 2 * NBK : 1], ve[EARLY ? 2 * NBV : 1];
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int s = 0; s < 2 * NBK; ++s)
+            ke[s] = *(const bf16x8*)(kblock + (unsigned)(pwa_key_of_row(c) * ks + 8 * g) + s * 16);
+#pragma unroll
+        for (int i = 0; i < 2 * NBV; ++i)
+            ve[i] = *(const bf16x8*)(vblock + (unsigned)(min(i / 2 * 32 + c, dv - 1) * vs + 8 * g) + (i & 1) * 16);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    auto key = [&](int s) {
+        const int d = s * 16 + 8 * g;
+        if constexpr (EARLY) return d < dk ? ke[s] : pwa_zero8();
+        else return (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
+    };
+    auto value = [&](int i, int h) {
         const int ch = i * 32 + c;
-        bf16x8 v1 = pwa_zero8(), v2 = pwa_zero8();
         if constexpr (EARLY) {
-            v1 = ve[2 * i];
-            v2 = ve[2 * i + 1];
+            bf16x8 v = ve[2 * i + h];
             if (limit < 32) {                             // uniform
 #pragma unroll
-                for (int x = 0; x < 8; ++x) {
-                    if (8 * g + x >= limit) v1[x] = (bf16)0.f;
-                    if (16 + 8 * g + x >= limit) v2[x] = (bf16)0.f;
-                }
+                for (int x = 0; x < 8; ++x)
+                    if (16 * h + 8 * g + x >= limit) v[x] = (bf16)0.f;
             }
-        } else if (ch < dv) {
-            const bf16* vrow = vblock + (size_t)ch * vs;
-            v1 = pwa_load_vt8(vrow, 8 * g, limit);
-            v2 = pwa_load_vt8(vrow, 16 + 8 * g, limit);
+            return v;
+        } else {
+            return ch < dv ? pwa_load_vt8(vblock + (size_t)ch * vs, 16 * h + 8 * g, limit) : pwa_zero8();
         }
-        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p1, acc_o[i], 0, 0, 0);
-        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p2, acc_o[i], 0, 0, 0);
-    }
+    };
+    pwa_block_of<NBK, NBV>(key, value, [] {}, kb, first_ok, last_ok, g, qf, acc_o, m, lsum, scale2, cap_in, cap_out);
 }
 
 // Which tile of 128 rows a workgroup takes: the last tiles (most keys) first, so that the long workgroups start
@@ -1214,6 +1219,181 @@ __global__ __launch_bounds__(256, ((NBK <= 4 && NBV <= 4) ? 2 : 1)) void pwa_pre
         }
 }
 
+// The same for keys of DK and values of DV elements (steps of 32) through a ring of two LDS stages filled by direct loads: a stage holds
+// a page's keys [64][DK] and values [DV][64] as they lie in the cache, 16-byte columns exchanged by the row (through the column that
+// a lane fetches) so that 16 lanes' operand reads spread over the banks; the page after the one that is multiplied is on its way, and
+// nothing passes through registers.  The workgroup's page numbers lie in LDS.  Where one workgroup fills a compute unit (DK + DV > 256: its
+// LDS, and the sums of 32 rows take 80 to 112 registers a lane) a block's keys are read together and its values ahead of the softmax.
+// 1,801 tokens, 32 heads of 256 / 224 over one row of keys: 343 us before, with a test and a wait at every operand and 38 values spilled.
+#define PWA_MAX_LIST 3840
+template <int DK, int DV>
+__global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_kernel(
+    const bf16* __restrict__ q, bf16* __restrict__ out, const int* __restrict__ cu_seqlens,
+    const int* __restrict__ slots, const int* __restrict__ ctx_lens, const int* __restrict__ block_table,
+    int table_stride, const bf16* __restrict__ storage, const int* __restrict__ pooled_table, int pooled_stride,
+    const bf16* __restrict__ pooled, int nq, int nkv, int size, int pool, float scale, int sink, const float* __restrict__ sinks, int pair,
+    int chunk, int keep, float softcap, int maps) {
+    constexpr int NBK = DK / 32, NBV = DV / 32, KCOLS = DK / 8, KB = PWA_PAGE * DK * 2, STAGE = KB + DV * PWA_PAGE * 2;
+    constexpr int KINSTR = KB / 1024, NDMA = STAGE / 1024 / 4;       // wave-loads of 1 KB: of the keys; per wave and page
+    constexpr bool ALONE = DK + DV > 256;
+    static_assert(DK % 32 == 0 && DV % 32 == 0 && STAGE % 4096 == 0 && (KCOLS % 16 == 0 || KCOLS % 16 == 8), "sizes");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char pwa_lds[];
+    int* list = (int*)(pwa_lds + 2 * STAGE);
+    const int b = blockIdx.z, kvh = blockIdx.y / maps, map = blockIdx.y % maps;
+    const int slot = slots[b];
+    const int t0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t0;
+    const int G = nq / (nkv * maps), kw = maps * DK;
+    const int rows_total = n_new * G;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg_row0 = pwa_tile(pair) * 128;
+    if (wg_row0 >= rows_total) return;                       // the whole workgroup
+    const int row0 = wg_row0 + wave * 32;
+    const bool wave_on = row0 < rows_total;
+    const int c = lane & 31, g = lane >> 5;
+    const int row = row0 + c;
+    const bool row_ok = wave_on && row < rows_total;
+    const int rr = row_ok ? row : rows_total - 1;
+    const int tok = rr / G, head = (kvh * G + rr % G) * maps + map;
+    bf16* orow = out + ((size_t)(t0 + tok) * nq + head) * DV;
+    if (slot < 0) {       // padding: no cache behind it
+        if (row_ok && g == 0) for (int d = 0; d < DV; ++d) orow[d] = (bf16)0.f;
+        return;
+    }
+    const int ctx = ctx_lens[b], start = ctx - n_new;
+    const int pq = start + tok;
+    // positions of this wave's rows and of the workgroup's
+    const int last_row = (row0 + 31 < rows_total ? row0 + 31 : rows_total - 1);
+    const int pq_min = start + (wave_on ? row0 : wg_row0) / G, pq_max = start + (wave_on ? last_row : wg_row0) / G;
+    const int wg_last = (wg_row0 + 127 < rows_total ? wg_row0 + 127 : rows_total - 1);
+    const int wg_min = start + wg_row0 / G, wg_max = start + wg_last / G;
+    // what the wave's rows see, and the pages the workgroup walks: pooled ones, the kept ones before the window, the window's
+    auto seen_of = [&](int p) { const int far = p - size - pool + 1; return (pool > 0 && far >= 0) ? far / pool + 1 : 0; };
+    const int seen = row_ok ? seen_of(pq) : 0, seen_wave = wave_on ? seen_of(pq_max) : 0;
+    const int far_pages = (seen_of(wg_max) + PWA_PAGE - 1) / PWA_PAGE;
+    const int first_page = pwa_lo(wg_min, size, chunk) / PWA_PAGE, lo_wave = pwa_lo(pq_min, size, chunk);
+    auto kept_of = [&](int p) { const int l = pwa_lo(p, size, chunk); return keep < l ? keep : l; };
+    const int kept = row_ok ? kept_of(pq) : 0, kept_wave = wave_on ? kept_of(pq_max) : 0;
+    const int kept_pages = (kept_of(wg_max) + PWA_PAGE - 1) / PWA_PAGE;
+    const int n_pages = far_pages + kept_pages + wg_max / PWA_PAGE - first_page + 1;      // at most PWA_MAX_LIST (the launcher checks)
+    const int written_far = pool > 0 ? ctx / pool : 0;
+    const int first_ok = row_ok ? pwa_lo(pq, size, chunk) : 1, last_ok = row_ok ? pq : 0;
+    const int* bt = block_table + (size_t)slot * table_stride;
+    const int* pt = pooled_table ? pooled_table + (size_t)slot * pooled_stride : nullptr;
+    for (int i = threadIdx.x; i < n_pages; i += 256)
+        list[i] = i < far_pages ? pt[i] : bt[i < far_pages + kept_pages ? i - far_pages : first_page + (i - far_pages - kept_pages)];
+
+    const bf16* qrow = q + ((size_t)(t0 + tok) * nq + head) * DK;
+    bf16x8 qf[2 * NBK];
+#pragma unroll
+    for (int s = 0; s < 2 * NBK; ++s) qf[s] = *(const bf16x8*)(qrow + s * 16 + 8 * g);
+    f32x16 acc_o[NBV];
+#pragma unroll
+    for (int i = 0; i < NBV; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc_o[i][r] = 0.f;
+    float m = sink ? (sinks ? sinks[head] * PWA_LOG2E : 0.f) : -INFINITY, lsum = (sink && g == 0) ? 1.f : 0.f;
+    const float scale2 = scale * PWA_LOG2E;
+    const bool capped = softcap > 0.f && scale != 0.f;
+    const float cap_in = capped ? 2.0f * PWA_LOG2E * scale / softcap : 0.f, cap_out = capped ? softcap / scale : 0.f;
+    const size_t page_elems = (size_t)nkv * PWA_PAGE * (kw + DV);
+    const size_t k_off = (size_t)kvh * PWA_PAGE * kw + (size_t)map * DK, v_off = (size_t)nkv * PWA_PAGE * kw + (size_t)kvh * DV * PWA_PAGE;
+    // the query and the sink have arrived before the loop: a wait for them inside would also wait for the page in flight
+#pragma unroll
+    for (int s = 0; s < 2 * NBK; ++s) asm volatile("" ::"v"(qf[s]));
+    asm volatile("" ::"v"(m));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                                         // the page numbers are in LDS
+
+    auto kswz = [](int r) { return KCOLS % 16 == 0 ? (r & 15) : ((r >> 1) & 7); };
+    const unsigned ring_lds = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)pwa_lds);
+    // this lane's part of each of its wave-loads: where it lies in a page (bytes)
+    unsigned goff[NDMA];
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+        const int in = wave * NDMA + i;
+        if (in < KINSTR) {
+            const int at = in * 64 + lane, r = at / KCOLS;
+            goff[i] = (unsigned)((k_off + (size_t)r * kw + ((at % KCOLS) ^ kswz(r)) * 8) * 2);
+        } else {
+            const int r = (in - KINSTR) * 8 + (lane >> 3);
+            goff[i] = (unsigned)((v_off + (size_t)r * PWA_PAGE + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2);
+        }
+    }
+    auto issue = [&](int n) {
+        const int number = __builtin_amdgcn_readfirstlane(list[n]);
+        const unsigned long long at = (unsigned long long)(n < far_pages ? pooled : storage) + (unsigned long long)number * page_elems * 2;
+        const unsigned long long pg = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
+                                      (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) {
+            const unsigned lds = __builtin_amdgcn_readfirstlane(ring_lds + (n & 1) * STAGE + (wave * NDMA + i) * 1024);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(goff[i]), "s"(pg) : "memory");
+        }
+    };
+    issue(0);
+    for (int n = 0; n < n_pages; ++n) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                        // every wave's part of page n is there; page n - 1 is done with
+        asm volatile("" ::: "memory");
+        if (n + 1 < n_pages) issue(n + 1);
+        const unsigned char* st = pwa_lds + (n & 1) * STAGE;
+        const bool far = n < far_pages, early = !far && n < far_pages + kept_pages;
+        const int page_row0 = (far ? n : (early ? n - far_pages : first_page + (n - far_pages - kept_pages))) * PWA_PAGE;
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            const int kb = page_row0 + 32 * hb;
+            const bool mine = wave_on && (far ? kb < seen_wave : (early ? kb < kept_wave : (kb + 31 >= lo_wave && kb <= pq_max)));     // wave-uniform
+            if (!mine) continue;
+            const int limit = (far ? written_far : ctx) - kb, kr = 32 * hb + pwa_key_of_row(c);
+            bf16x8 ke[ALONE ? 2 * NBK : 1], ve[ALONE ? 2 * NBV : 1];
+            auto key_at = [&](int s) { return *(const bf16x8*)(st + kr * (DK * 2) + (((2 * s + g) ^ kswz(kr)) * 16)); };
+            auto value_at = [&](int i, int h) {
+                const int ch = i * 32 + c;
+                return *(const bf16x8*)(st + KB + ch * 128 + (((4 * hb + 2 * h + g) ^ ((ch >> 1) & 7)) * 16));
+            };
+            if constexpr (ALONE) {
+#pragma unroll
+                for (int s = 0; s < 2 * NBK; ++s) ke[s] = key_at(s);
+            }
+            auto values = [&] {
+                if constexpr (ALONE) {
+#pragma unroll
+                    for (int i = 0; i < 2 * NBV; ++i) ve[i] = value_at(i / 2, i & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            auto key = [&](int s) { if constexpr (ALONE) return ke[s]; else return key_at(s); };
+            auto value = [&](int i, int h) {
+                bf16x8 v;
+                if constexpr (ALONE) v = ve[2 * i + h];
+                else v = value_at(i, h);
+                if (limit < 32) {                            // uniform: the last page's rows that are not written
+                    int live = limit - 16 * h - 8 * g;
+                    asm volatile("" : "+v"(live));           // (its compares stay inside the branch)
+#pragma unroll
+                    for (int x = 0; x < 8; ++x)
+                        if (x >= live) v[x] = (bf16)0.f;
+                }
+                return v;
+            };
+            pwa_block_of<NBK, NBV>(key, value, values, kb, (far || early) ? 0 : first_ok, far ? seen - 1 : (early ? kept - 1 : last_ok), g, qf, acc_o, m,
+                                   lsum, scale2, cap_in, cap_out);
+        }
+    }
+    lsum += __shfl_xor(lsum, 32, 64);
+    if (!row_ok) return;
+    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+#pragma unroll
+    for (int i = 0; i < NBV; ++i)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (bf16)(acc_o[i][4 * r4 + e] * inv);
+            *(bf16x4*)(orow + i * 32 + 8 * r4 + 4 * g) = o;
+        }
+}
+
 template <int NBK>
 static int pwa_prefill_launch_v(int nbv, dim3 grid, hipStream_t s, const bf16* q, bf16* out, const int* cu, const int* slots,
                                 const int* ctx, const int* bt, int ts, const bf16* st, const int* pt, int ps, const bf16* pl,
@@ -1260,6 +1440,33 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
     const int G = nq / (nkv * maps);
     dim3 grid((unsigned)(((size_t)max_new * G + 127) / 128), nkv * maps, B);
     const int nbk = (dk + 31) / 32, nbv = (dv + 31) / 32;
+    // whole page lists and 32-bit offsets into a page
+    const long long pages = (long long)table_stride + (pool > 0 ? pooled_stride : 0) + (keep > 0 ? (keep + PWA_PAGE - 1) / PWA_PAGE : 0);
+    if ((long long)grid.x * 128 >= 256 && pages <= PWA_MAX_LIST && ((uintptr_t)storage | (uintptr_t)pooled | (uintptr_t)q) % 16 == 0 &&
+        (unsigned long long)nkv * PWA_PAGE * ((unsigned long long)maps * dk + dv) * 2 < (1ull << 32)) {
+        const int cus = br_device_cus();
+        const int pair = cus > 0 && (long long)grid.x * grid.y * grid.z <= 2LL * cus;
+#define PWA_DMA(DK_, DV_)                                                                                                              \
+        if (dk == DK_ && dv == DV_) {                                                                                                  \
+            auto kern = pwa_prefill_dma_kernel<DK_, DV_>;                                                                              \
+            const size_t lds = (size_t)2 * PWA_PAGE * (DK_ + DV_) * 2 + (((size_t)pages + 3) & ~(size_t)3) * sizeof(int);               \
+            static bool set = false;                                                                                                   \
+            if (!set) {                                                                                                                \
+                if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,                                 \
+                                        2 * PWA_PAGE * (DK_ + DV_) * 2 + PWA_MAX_LIST * (int)sizeof(int)) != hipSuccess)               \
+                    return BR_LAUNCH_FAILED;                                                                                           \
+                set = true;                                                                                                            \
+            }                                                                                                                          \
+            kern<<<grid, 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,            \
+                                        (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, size, pool, scale, sink, sinks, pair, chunk, keep, \
+                                        softcap, maps);                                                                                \
+            return br_check_launch();                                                                                                  \
+        }
+        PWA_DMA(128, 128)
+        PWA_DMA(192, 160)
+        PWA_DMA(256, 224)
+#undef PWA_DMA
+    }
 #define PWA_K(KK) pwa_prefill_launch_v<KK>(nbv, grid, s, (const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride, \
                                            (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, dk, dv, size, pool, scale, sink, sinks, \
                                            chunk, keep, softcap, maps)
