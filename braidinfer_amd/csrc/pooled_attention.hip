@@ -682,12 +682,14 @@ __device__ __forceinline__ void pwa_block_of(Key key, Value value, Between betwe
     // the sums so far are scaled only when some lane's maximum moved
     const bool moved = __any(m_new != m);
     m = m_new;
+    if (moved) {
 #pragma unroll
-    for (int i = 0; i < NBV; ++i) {
-        if (moved) {
+        for (int i = 0; i < NBV; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc_o[i][r] *= corr;
-        }
+    }
+#pragma unroll
+    for (int i = 0; i < NBV; ++i) {
         acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 0), p1, acc_o[i], 0, 0, 0);
         acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 1), p2, acc_o[i], 0, 0, 0);
     }
@@ -1223,8 +1225,9 @@ __global__ __launch_bounds__(256, ((NBK <= 4 && NBV <= 4) ? 2 : 1)) void pwa_pre
 // a page's keys [64][DK] and values [DV][64] as they lie in the cache, 16-byte columns exchanged by the row (through the column that
 // a lane fetches) so that 16 lanes' operand reads spread over the banks; the page after the one that is multiplied is on its way, and
 // nothing passes through registers.  The workgroup's page numbers lie in LDS.  Where one workgroup fills a compute unit (DK + DV > 256: its
-// LDS, and the sums of 32 rows take 80 to 112 registers a lane) a block's keys are read together and its values ahead of the softmax.
-// 1,801 tokens, 32 heads of 256 / 224 over one row of keys: 343 us before, with a test and a wait at every operand and 38 values spilled.
+// LDS, and the sums of 32 rows take 80 to 112 registers a lane) a block's keys are read half a block ahead and its values in front of the softmax.
+// us with pages through registers, with this form: 1,801 tokens, 32 heads of 256 / 224 over one row of keys 292 / 131, 16 of 192 / 160 264 / 94; 3,517
+// and 1,501 tokens, 32 heads of 128 over 8, window 2,048 with pooled rows 300 / 202; three texts, 16 of 128 over 8 88 / 58.
 #define PWA_MAX_LIST 3840
 template <int DK, int DV>
 __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_kernel(
@@ -1345,7 +1348,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
             const bool mine = wave_on && (far ? kb < seen_wave : (early ? kb < kept_wave : (kb + 31 >= lo_wave && kb <= pq_max)));     // wave-uniform
             if (!mine) continue;
             const int limit = (far ? written_far : ctx) - kb, kr = 32 * hb + pwa_key_of_row(c);
-            bf16x8 ke[ALONE ? 2 * NBK : 1], ve[ALONE ? 2 * NBV : 1];
+            bf16x8 ke[ALONE ? NBK : 1], ve[ALONE ? 2 * NBV : 1];
             auto key_at = [&](int s) { return *(const bf16x8*)(st + kr * (DK * 2) + (((2 * s + g) ^ kswz(kr)) * 16)); };
             auto value_at = [&](int i, int h) {
                 const int ch = i * 32 + c;
@@ -1353,8 +1356,17 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
             };
             if constexpr (ALONE) {
 #pragma unroll
-                for (int s = 0; s < 2 * NBK; ++s) ke[s] = key_at(s);
+                for (int s = 0; s < NBK; ++s) ke[s] = key_at(s);
             }
+            auto key = [&](int s) {
+                if constexpr (ALONE) {
+                    const bf16x8 k = ke[s % NBK];
+                    if (s < NBK) ke[s] = key_at(s + NBK);
+                    return k;
+                } else {
+                    return key_at(s);
+                }
+            };
             auto values = [&] {
                 if constexpr (ALONE) {
 #pragma unroll
@@ -1362,22 +1374,17 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
-            auto key = [&](int s) { if constexpr (ALONE) return ke[s]; else return key_at(s); };
-            auto value = [&](int i, int h) {
-                bf16x8 v;
-                if constexpr (ALONE) v = ve[2 * i + h];
-                else v = value_at(i, h);
-                if (limit < 32) {                            // uniform: the last page's rows that are not written
-                    int live = limit - 16 * h - 8 * g;
-                    asm volatile("" : "+v"(live));           // (its compares stay inside the branch)
+            auto value = [&](int i, int h) { if constexpr (ALONE) return ve[2 * i + h]; else return value_at(i, h); };
+            auto written = [&](int i, int h) {               // the last page's rows that are not written read as zero
+                bf16x8 v = value(i, h);
 #pragma unroll
-                    for (int x = 0; x < 8; ++x)
-                        if (x >= live) v[x] = (bf16)0.f;
-                }
+                for (int x = 0; x < 8; ++x)
+                    if (16 * h + 8 * g + x >= limit) v[x] = (bf16)0.f;
                 return v;
             };
-            pwa_block_of<NBK, NBV>(key, value, values, kb, (far || early) ? 0 : first_ok, far ? seen - 1 : (early ? kept - 1 : last_ok), g, qf, acc_o, m,
-                                   lsum, scale2, cap_in, cap_out);
+            const int from = (far || early) ? 0 : first_ok, to = far ? seen - 1 : (early ? kept - 1 : last_ok);
+            if (limit >= 32) pwa_block_of<NBK, NBV>(key, value, values, kb, from, to, g, qf, acc_o, m, lsum, scale2, cap_in, cap_out);
+            else pwa_block_of<NBK, NBV>(key, written, values, kb, from, to, g, qf, acc_o, m, lsum, scale2, cap_in, cap_out);
         }
     }
     lsum += __shfl_xor(lsum, 32, 64);
