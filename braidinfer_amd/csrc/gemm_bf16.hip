@@ -517,6 +517,16 @@ struct QuadGroups {
     unsigned per;
     float limit, alpha;
 };
+// Several inputs by stacked weights in one launch (BRANCHES): the weight rows b * per .. of a column of tiles multiply the activations
+// `a_step` elements behind the branch before; results leave `gap` columns alone in front of branch gap_at / per.
+struct QuadBranches {
+    int per;
+    size_t a_step;
+    int gap_at, gap;
+};
+enum { QUAD_PLAIN = 0, QUAD_EXPERTS = 1, QUAD_BRANCHES = 2 };
+template <int KIND> struct QuadArg { typedef QuadGroups type; };
+template <> struct QuadArg<QUAD_BRANCHES> { typedef QuadBranches type; };
 __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr) {
     if (gr.alpha > 0.f) {
         g = fminf(g, gr.limit);
@@ -541,9 +551,9 @@ struct QuadStrip {
     static constexpr int LD = RB + 16;                                                   // from row to row, off the banks' stride
     static constexpr int BYTES = MODE == OUT_F32_ACC ? 0 : 32 * LD;
 };
-template <int TI, int TJ, int WVM, int MODE, bool GROUPED>
+template <int TI, int TJ, int WVM, int MODE, bool GROUPED, class Arg>
 __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __restrict__ C, int M, int N, size_t ldc, int m1, int n1, int lane,
-                                              const QuadGroups& gr, unsigned char* lds) {
+                                              const Arg& gr, unsigned char* lds) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     if constexpr (MODE == OUT_F32_ACC) {
@@ -575,6 +585,10 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
         struct __attribute__((packed, aligned(8))) Out { unsigned w[4]; };               // bfloat16 rows are aligned to 8 bytes
         typedef QuadStrip<TI, MODE> S;
         constexpr int CH = S::RB / 16, EL = 16 / S::ES;                                  // pieces of 16 bytes of a row, elements of one
+        auto unit = [&](float x, float u) {
+            if constexpr (GROUPED) return quad_glu(x, u, gr);
+            else return silu_mul(x, u);
+        };
         if (MODE == OUT_SWIGLU) {
             N >>= 1;
             n1 >>= 1;
@@ -592,8 +606,7 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
                         bf16x4 v;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            v[e] = (bf16)(GROUPED ? quad_glu(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e], gr)
-                                                  : silu_mul(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]));
+                            v[e] = (bf16)unit(acc[i][j][8 * h + e], acc[i][j][8 * h + 4 + e]);
                         *(bf16x4*)(put + (16 * i + 8 * h) * 2) = v;
                     }
                     continue;
@@ -639,11 +652,12 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
     }
 }
 
-template <int BM, int BN, int NSA, int NSB, int WVM, int MODE, bool GROUPED = false>
+template <int BM, int BN, int NSA, int NSB, int WVM, int MODE, int KIND = QUAD_PLAIN>
 __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                               void* __restrict__ C_, int M, int N, int K, size_t lda,
                                                               size_t ldc, int tiles_m, int tiles_n, int kt_per_part,
-                                                              size_t part_stride, int wl, QuadGroups gr) {
+                                                              size_t part_stride, int wl, typename QuadArg<KIND>::type gr) {
+    constexpr bool GROUPED = KIND == QUAD_EXPERTS;
     constexpr int SA = BM * 128, SB = BN * 128;          // bytes of a stage of activation rows, of weight rows
     constexpr int WVN = 4 / WVM;                         // the four waves: WVM along the activation rows x WVN
     constexpr int TI = BN / WVN / 32, TJ = BM / WVM / 32; // blocks of a wave: weight rows, activation rows
@@ -877,7 +891,13 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         int gn = tiles_n - grp * 8;
         if (gn > 8) gn = 8;
         const int tile_n = grp * 8 + in % gn, tile_m = in / gn;
-        tile(A, W, tile_m * BM, tile_n * BN, M);
+        if constexpr (KIND == QUAD_BRANCHES) {                         // (no tile lies across two branches)
+            const int n0 = tile_n * BN;
+            if (n0 >= gr.gap_at) C = (float*)C + gr.gap;
+            tile(A + (size_t)(n0 / gr.per) * gr.a_step, W, tile_m * BM, n0, M);
+        } else {
+            tile(A, W, tile_m * BM, tile_n * BN, M);
+        }
     } else {
         // Expert by expert, column of tiles by column, an expert's row tiles of the same weights in turn.  The columns are cut into
         // eight runs of about equal cost, one to an XCD, whose workgroups take its tiles in turn.  (What a tile of few rows costs is its
@@ -1025,25 +1045,26 @@ static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N,
 // three and a half rounds: 390 us, the half round 1.41 us a k-tile); plus what a launch costs besides and,
 // when split along k, the second launch and the traffic of the partial sums.  Returns the count.
 static const double QUAD_FULL[4] = {1.50, 0.85, 1.20, 1.39}, QUAD_FEW[4] = {1.08, 0.80, 0.92, 1.00};
-static double choose_quad(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* kernel, int* parts) {
-    const int nk = K / DMA_BK;
+static double quad_count(int M, int N, int K, int mode, int cus, int k, int p) {       // tile 12 + k in p runs
     static const int bm[4] = {256, 128, 256, 256}, bn[4] = {256, 256, 192, 224};
+    int kpp = (K / DMA_BK + p - 1) / p;
+    kpp += kpp & 1;
+    const long long units = (long long)((M + bm[k] - 1) / bm[k]) * ((N + bn[k] - 1) / bn[k]) * p, whole = units / cus;
+    const double share = (double)(units % cus) / cus;
+    const double rest = units % cus == 0 ? 0.0
+                        : whole        ? QUAD_FULL[k] * (0.9 + 0.1 * share)
+                                       : QUAD_FEW[k] + (QUAD_FULL[k] - QUAD_FEW[k]) * share * share * share;
+    const double t = kpp * ((double)whole * QUAD_FULL[k] + rest) + (mode == OUT_BF16 ? 8.0 : 12.0);
+    return p > 1 ? t + 5.0 + (double)p * M * N * 8.0 / 4e6 : t;
+}
+static double choose_quad(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* kernel, int* parts) {
     double best = 1e30;
     *kernel = 13;
     *parts = 1;
     for (int k = 0; k < 4; ++k) {
-        const long long tiles = (long long)((M + bm[k] - 1) / bm[k]) * ((N + bn[k] - 1) / bn[k]);
         for (int p = 1; p <= 16; p *= 2) {
-            if (p > 1 && (p * 4 > nk || N % 4 != 0 || (size_t)p * M * N * sizeof(float) > scratch_bytes)) break;
-            int kpp = (nk + p - 1) / p;
-            kpp += kpp & 1;
-            const long long units = tiles * p, whole = units / cus;
-            const double share = (double)(units % cus) / cus;
-            const double rest = units % cus == 0 ? 0.0
-                                : whole        ? QUAD_FULL[k] * (0.9 + 0.1 * share)
-                                               : QUAD_FEW[k] + (QUAD_FULL[k] - QUAD_FEW[k]) * share * share * share;
-            double t = kpp * ((double)whole * QUAD_FULL[k] + rest) + (mode == OUT_BF16 ? 8.0 : 12.0);
-            if (p > 1) t += 5.0 + (double)p * M * N * 8.0 / 4e6;
+            if (p > 1 && (p * 4 > K / DMA_BK || N % 4 != 0 || (size_t)p * M * N * sizeof(float) > scratch_bytes)) break;
+            const double t = quad_count(M, N, K, mode, cus, k, p);
             if (t < best - 1e-9) { best = t; *kernel = 12 + k; *parts = p; }
         }
     }
@@ -3067,11 +3088,42 @@ extern "C" int br_gemm_bf16_branches_takes(int M, int per, int K) {
     return M > 0 && M <= 64 && per > 0 && per % 128 == 0 && K % STREAM_KC == 0 && K / STREAM_KC >= STREAM_NW;
 }
 
+// Beyond 128 rows the branches make one product of whole 256-wide columns of tiles (256x256, 128x256).  Taken where that is counted faster than
+// a product for each (with as many runs along k as it likes), which it was at every size timed: few tiles need no runs, many fill their rounds.  Four
+// of 4,096 by 4,096, us by 129 / 512 / 1,024 / 1,801 / 3,000 / 7,000 rows one by one 94 / 138 / 184 / 236 / 372 / 809, at once 45 / 62 / 111 / 206 / 318 /
+// 739; of 2,048 by 2,048 66 / 76 / 98 / 107 / 123 / 232 and 25 / 27 / 37 / 58 / 101 / 230.
+static int branches_tile(int M, int branches, int per, int K, int cus) {       // 12, 13, or 0: a product for each
+    if (M <= 128 || branches < 2 || branches > 64 || per <= 0 || per % 256 || K <= 0 || K % DMA_BK || (long long)branches * per > 0x3fffffff || cus <= 0) return 0;
+    int k, p;
+    const double room = choose_quad(M, per, K, OUT_F32, cus, ~(size_t)0, &k, &p);
+    const double tall = quad_count(M, branches * per, K, OUT_F32, cus, 0, 1), flat = quad_count(M, branches * per, K, OUT_F32, cus, 1, 1);
+    if (min(tall, flat) >= branches * room) return 0;
+    return tall <= flat ? 12 : 13;
+}
+extern "C" int br_gemm_bf16_branches_pay(int M, int branches, int per, int K) { return branches_tile(M, branches, per, K, br_device_cus()) != 0; }
+
+template <int BM, int NSA, int NSB>
+static int launch_branches_tiles(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const QuadBranches& br, hipStream_t s) {
+    const int tm = (M + BM - 1) / BM, tn = N / 256;
+    if ((long long)tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
+    gemm_tile_quad_kernel<BM, 256, NSA, NSB, 2, OUT_F32, QUAD_BRANCHES><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, K / DMA_BK, 0,
+                                                                                                     WL_ROWS, br);
+    return br_check_launch();
+}
+
 // tail_rows > 0 (up to 16 rows, in steps of 16, at most per): further weight rows, multiplying one more branch's activations, the
 // tanh of whose sums goes to tail [M, tail_ld]: instead of two launches of their own, 8.4 us of a single-token step a layer.
 extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, int M, int branches, int per, int K, size_t a_step, size_t lda,
                                      size_t ldc, int gap_at, int gap, int tail_rows, void* tail, size_t tail_ld, hipStream_t s) {
     const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
+    if (const int kind = branches_tile(M, branches, per, K, br_device_cus())) {
+        if (tail_rows || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 || gap % 4 || gap_at < 0 || gap_at % per || ldc < (size_t)branches * per + gap ||
+            ((uintptr_t)A | (uintptr_t)W) % 16 || !quad_takes(C, M, branches * per, K, lda, ldc))
+            return BR_BAD_ARG;
+        const QuadBranches br = {per, a_step, gap_at, gap};
+        return kind == 12 ? launch_branches_tiles<256, QUAD12>(A, W, C, M, branches * per, K, lda, ldc, br, s)
+                          : launch_branches_tiles<128, QUAD13>(A, W, C, M, branches * per, K, lda, ldc, br, s);
+    }
     if (branches < 1 || branches > 64 || !br_gemm_bf16_branches_takes(M, per, K) || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 ||
         gap_at % per || ((uintptr_t)A | (uintptr_t)W) % 16 || ldc < (size_t)branches * per || (long long)branches * per > 0x3fffffff)
         return BR_BAD_ARG;
@@ -3193,7 +3245,7 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
     if (tm * tn > 0x7fffffc0LL) return BR_BAD_ARG;
     const unsigned grid = (unsigned)((tm * tn + 7) / 8 * 8);
 #define BR_EXPERTS(MODE_) \
-    gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, MODE_, true><<<grid, 256, 0, s>>>(A, W, C, 0, N, K, (size_t)K, ldc, 0, tn, nk, 0, WL_ROWS, gr)
+    gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, MODE_, QUAD_EXPERTS><<<grid, 256, 0, s>>>(A, W, C, 0, N, K, (size_t)K, ldc, 0, tn, nk, 0, WL_ROWS, gr)
     if (mode == OUT_SWIGLU) BR_EXPERTS(OUT_SWIGLU);
     else if (mode == OUT_F32) BR_EXPERTS(OUT_F32);
     else BR_EXPERTS(OUT_BF16);

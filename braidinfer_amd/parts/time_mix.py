@@ -117,7 +117,7 @@ class WKVTimeMix(Mixer):
         rows = step.ws.get("wkv_rows", (T, 5 * hd), torch.float32)
         low_t = step.ws.get("wkv_low_t", (T, self.rank), dt)
         tail = None
-        if self.w_four is not None and dt == torch.bfloat16 and K.gemm_branches_takes(T, hd, self.H):
+        if self.w_four is not None and dt == torch.bfloat16 and (K.gemm_branches_takes(T, hd, self.H) or K.gemm_branches_pay(T, 4, hd, self.H)):
             tail = low_t if self.w_five is not None and T <= 16 else None
             if tail is not None:
                 K.gemm_branches(mixes, self.w_five, rows, gap_at=3, gap=hd, tail=tail)

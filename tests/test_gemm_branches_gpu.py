@@ -26,6 +26,34 @@ def test_branches(M, B, per, K_, gap_at, gap):
     assert torch.all(wide[:, left] == 7.0)
 
 
+# more than 128 rows: the last tile of one row, whole tiles, tiles cut short; columns of tiles behind, in front of and without a gap; one
+# k-tile and more; more tiles than compute units; both tile heights
+@pytest.mark.parametrize("M", [129, 255, 257, 449, 1024])
+@pytest.mark.parametrize("B,per,K_,gap_at,gap", [(4, 256, 64, 3, 256), (2, 512, 192, 0, 4), (3, 256, 1024, 2, 12), (4, 2048, 512, 0, 0), (8, 4096, 128, 7, 8)])
+def test_branches_of_many_rows(M, B, per, K_, gap_at, gap):
+    from braidinfer_amd import kernels as K
+    assert K.gemm_branches_pay(M, B, per, K_)
+    test_branches(M, B, per, K_, gap_at, gap)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = torch.randn(B, M, K_, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(B * per, K_, generator=g, device="cuda").to(torch.bfloat16)
+    out, again = (torch.empty(M, B * per, device="cuda") for _ in range(2))
+    K.gemm_branches(a, w, out)
+    K.gemm_branches(a.flip(0).contiguous(), torch.cat(w.split(per)[::-1]), again)      # a branch's bits do not depend on its place
+    assert torch.equal(torch.cat(again.split(per, 1)[::-1], 1), out)
+
+
+def test_branches_of_many_rows_refuse():
+    from braidinfer_amd import kernels as K
+    from braidinfer_amd.errors import KernelError
+    for M, B, per, K_ in ((128, 4, 256, 1024), (129, 1, 256, 1024), (129, 4, 384, 1024), (129, 4, 256, 1056)):
+        assert not K.gemm_branches_pay(M, B, per, K_)
+    a, w = torch.zeros(2, 129, 64, dtype=torch.bfloat16, device="cuda"), torch.zeros(512, 64, dtype=torch.bfloat16, device="cuda")
+    for out in (torch.zeros(129, 515, device="cuda"), torch.zeros(129, 516, device="cuda")[:, 1:514]):
+        with pytest.raises(KernelError):
+            K.gemm_branches(a, w, out, gap_at=1, gap=out.shape[1] - 512)
+
+
 def test_branches_refuse():
     from braidinfer_amd import kernels as K
     from braidinfer_amd.errors import KernelError
