@@ -238,6 +238,18 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const C
     }
 }
 
+// The sequence that `rank` others of a step are longer than (of equal ones: that come before it).  Steps of more than 64 sequences: as they come.
+__device__ __forceinline__ int cw_by_length(const int* cu, int B, int rank) {
+    if (B > 64) return rank;
+    const int lane = threadIdx.x & 63, mine = lane < B ? cu[lane + 1] - cu[lane] : -1;
+    int before = 0;
+    for (int i = 0; i < B; ++i) {
+        const int other = __builtin_amdgcn_readlane(mine, i);
+        before += other > mine || (other == mine && i < lane);
+    }
+    return __ffsll((unsigned long long)__ballot(lane < B && before == rank)) - 1;
+}
+
 // A workgroup walks a sequence's chunks for 16 CB columns of one head; wave w holds the state's rows w D / 4 .. + D / 4 and adds a
 // quarter of every output element (its rows' share and, of the sum over A, the tokens 4 w .. + 4), the quarters are added
 // in a fixed order through LDS a chunk later.  Sums are kept short and their largest terms late, so that they round about as
@@ -250,7 +262,10 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const C
 // as many the compiler keeps the sums in accumulation registers and moves the state back and forth.  That, with the chunk before left
 // and A's product formed behind the update, took 142 us for 2,048 tokens of 32 heads where this takes 123 (a fixed decay 148 and 125,
 // delta rule 213 and 190; 64 heads of 64 x 64 113 and 106).  v: the values' columns of the rows, `ldv` apart.  grid (sequences * H,
-// e / (16 CB)): the workgroups of a head on one XCD where sequences * H is a multiple of 8.
+// e / (16 CB)), or where H is a multiple of 8 (H, e / (16 CB), sequences), the longest first: the workgroups of a head on one XCD where sequences * H
+// is a multiple of 8, and what a step's longest sequences need is not behind the others (with the sequences side by side two workgroups of the longest
+// shared a compute unit while others lay idle: 32 heads of 128 x 128, gated, 3,517 and 1,501 tokens 296 -> 247 us, 1,307, 804 and 301 142 -> 117, three times
+// 1,200, 300, 150 and 96 291 -> 224; equal ones as before).
 template <int D, int CB, int S, int FORM>
 __global__ __launch_bounds__(256, 2) void chunk_walk_kernel(const float* __restrict__ scratch, const float* __restrict__ v, int ldv,
                                                             float* __restrict__ o, float* __restrict__ state, size_t slot_stride,
@@ -263,7 +278,7 @@ __global__ __launch_bounds__(256, 2) void chunk_walk_kernel(const float* __restr
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     float* part = (float*)(smem + S * STAGE);                 // [PB][4][CB][16][17]
     float* pu = part + PB * 4 * CB * 272;                     // DELTA: [4][CB][64][4] the waves' shares of -W S
-    const int s = blockIdx.x / H, h = blockIdx.x - s * H, cb = blockIdx.y;
+    const int s = gridDim.z > 1 ? cw_by_length(cu_seqlens, gridDim.z, blockIdx.z) : blockIdx.x / H, h = blockIdx.x % H, cb = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int slot = slots[s], he = H * e;
@@ -538,27 +553,29 @@ static int chunk_walk(const CwIn& in, const CwPart& part, const float* scratch, 
         if (hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return BR_LAUNCH_FAILED;
         set = true;
     }
-    walk<<<dim3(B * in.H, in.e / (16 * CB)), 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding, part);
+    const dim3 grid = in.H % 8 == 0 && B <= 65535 ? dim3(in.H, in.e / (16 * CB), B) : dim3(B * in.H, in.e / (16 * CB));
+    walk<<<grid, 256, lds, s>>>(scratch, in.v, (int)in.v_stride, o, state, slot_stride, in.cu, in.slots, in.H, in.e, zero_padding, part);
     return br_check_launch();
 }
 
 template <int FORM, int D>
 static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state, size_t slot_stride, float* scratch, int B, int chunks,
-                     hipStream_t s) {
+                     int T, int max_new, hipStream_t s) {
     constexpr bool DELTA = FORM == CW_DELTA;
     chunk_prepare_kernel<FORM, D><<<dim3(chunks, in.H, B), D, 0, s>>>(in, part, scratch);
     const int rc = br_check_launch();
     if (rc != BR_OK) return rc;
-    // 16 columns a workgroup up to three workgroups to a compute unit (delta rule with heads of 128: one, it holds the most in
-    // LDS); beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of 128 x 128, gated, 2,048 tokens 122 / 166, 3,517 and
-    // 1,501 tokens 302 / 292, three times 1,000 156 / 154, four times 900 187 / 154, 16 times 300 303 / 227; fixed, 1,307, 804 and 301 tokens
-    // 162 / 164; delta rule, 2,048 tokens 190 / 282, twice 1,000 189 / 179, 16 times 300 518 / 392; 64 heads of 64 x 64, WKV, 1,801 tokens
-    // 94 / 119, three times 900 121 / 117, four times 171 / 136; delta rule, 900, 900 and 300 tokens 154 / 158.
+    // 16 columns a workgroup as long as the tokens are those of few sequences as long as the longest: 2.5 workgroups of 16 columns to a compute unit
+    // (delta rule with heads of 128, which holds the most in LDS: 1.9).  Beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of
+    // 128 x 128, gated, 2,048 tokens 125 / 167, 3,517 and 1,501 tokens 247 / 286, 1,307, 804 and 301 117 / 133, 1,500, 700, 400 and 200 141 / 153, 1,300, 900,
+    // 700, 500 and 300 183 / 158, three times 1,000 150 / 150, four times 900 170 / 149, 16 times 300 255 / 219; fixed, 1,307, 804 and 301 123 / 141; delta
+    // rule, 2,048 tokens 184 / 272, 3,517 and 1,501 442 / 569, 1,307, 804 and 301 226 / 232, 1,500, 700, 400 and 200 262 / 277, three times 1,000 273 / 250, twice
+    // 1,000 189 / 179; 64 heads of 64 x 64, WKV, 3,517 and 1,501 218 / 245, 1,300 .. 300 154 / 136; delta rule, 900, 900 and 300 154 / 158.
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    const long long units = (long long)part.longs * in.H * (in.e / 16);
+    const double units = min((double)T / max_new, (double)part.longs) * in.H * (in.e / 16);
 #define CW_WALK(CB, S) return chunk_walk<D, CB, S, FORM == CW_WKV ? CW_GLR : FORM>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
-    if (in.e % 32 || units <= (D == 128 && DELTA ? 1 : 3) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
+    if (in.e % 32 || units <= (D == 128 && DELTA ? 1.9 : 2.5) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
     if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
     else CW_WALK(2, (D == 64 ? 5 : 3));
 #undef CW_WALK
@@ -590,7 +607,7 @@ extern "C" int br_chunk_scan(int form, const float* q, const float* k, float* v,
     for (int from = 0; from < all; from += run) {
         const CwPart part = {least, longs, from, once ? 0 : run};
         const int chunks = all - from < run ? all - from : run;
-#define CW_RUN(F) d == 64 ? chunk_run<F, 64>(in, part, o, state, slot_stride, scratch, B, chunks, s) : chunk_run<F, 128>(in, part, o, state, slot_stride, scratch, B, chunks, s)
+#define CW_RUN(F) d == 64 ? chunk_run<F, 64>(in, part, o, state, slot_stride, scratch, B, chunks, T, max_new, s) : chunk_run<F, 128>(in, part, o, state, slot_stride, scratch, B, chunks, T, max_new, s)
         const int rc = form == CW_GLR ? CW_RUN(CW_GLR) : form == CW_WKV ? CW_RUN(CW_WKV) : form == CW_FIXED ? CW_RUN(CW_FIXED) : CW_RUN(CW_DELTA);
 #undef CW_RUN
         if (rc != BR_OK) return rc;

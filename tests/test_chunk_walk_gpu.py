@@ -342,3 +342,35 @@ def test_chunks_in_runs_where_the_scratch_is_small(form):
             assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     with pytest.raises(KernelError):
         run(longs * block - 4, longs=longs)
+
+
+# heads in steps of 8 and not; the longest sequence first, last and between, equal ones, more sequences than are ordered; a padding sequence among them
+@pytest.mark.parametrize("form,d,H", [("glr", 64, 8), ("fixed", 128, 8), ("delta", 128, 8), ("wkv", 64, 16), ("delta", 64, 12)])
+@pytest.mark.parametrize("lens", [[200, 40, 97, 16], [16, 40, 97, 200], [33, 180, 33, 180, 1], [17 + i % 3 for i in range(66)], [300, 20, 20, 20, 20, 20, 20]])
+def test_a_sequences_bits_do_not_depend_on_the_others(form, d, H, lens):
+    from braidinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(len(lens) + d)
+    T, B, e = sum(lens), len(lens), 32
+    i = {n: x.cuda() if torch.is_tensor(x) else x for n, x in inputs(form, T, H, H, d, e, False, g).items()}
+    n = 1
+    for x in K.glr_state_shape(H, d, e):
+        n *= x
+    first = torch.randn(B, n, generator=g).cuda()
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    vectors = {name: i[name] for name in ("b1", "b2") if name in i}
+    slots = [b if b != 1 else -1 for b in range(B)]
+
+    def run(t0, t1, some, state):
+        rows = {name: i[name][t0:t1] for name in ("z", "gb", "gc") if name in i}
+        at = [c - t0 for c in cu if t0 <= c <= t1]
+        o = torch.full((t1 - t0, H * e), 7.0, device="cuda")
+        scratch = torch.empty(K.chunk_scratch_floats(t1 - t0, len(some), H, d, e, form == "delta"), device="cuda")
+        K.chunk_scan(form, i["q"][t0:t1], i["k"][t0:t1], i["v"][t0:t1].clone(), o, state, torch.tensor(at, dtype=torch.int32, device="cuda"),
+                     torch.tensor(some, dtype=torch.int32, device="cuda"), scratch, len(some), H, H, d, e, max(b - a for a, b in zip(at, at[1:])), **rows, **vectors)
+        return o
+    together, alone = first.clone(), first.clone()
+    o = run(0, T, slots, together)
+    for b in range(B):
+        if slots[b] >= 0:
+            assert torch.equal(run(cu[b], cu[b + 1], [b], alone), o[cu[b]:cu[b + 1]]), b
+    assert torch.equal(together, alone) and torch.equal(together[1], first[1])
