@@ -768,13 +768,17 @@ __device__ __forceinline__ int kswz(int row, int cols) {      // the 16 key rows
 // the sums of `runs` float matrices [B, (nq + 2 nkv) HD], `run_stride` elements apart, as a
 // product cut along k leaves them.  Every value read from `q` is then the runs' sum in run
 // order, rounded to bf16: the bits the product's own sum kernel would have stored.
+// `fold`: the sequences of one round of workgroups over the compute units where there are up to two rounds; those behind it are
+// taken from the last on, so that in a batch in the order of its lengths a long and a short one share a compute unit (their numbers
+// lie a round apart).  The batch size otherwise.  Whole steps of eight layers, longest first: 64 sequences of 128 to 2,048
+// tokens 6,029 -> 5,960 us (four steps), 8 in 8 runs 3,327 -> 3,290.
 template <int HD, int S, bool FUSE>
 __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
     const bf16* __restrict__ q, size_t q_stride, bf16* __restrict__ out, const int* __restrict__ slots,
     const int* __restrict__ ctx_lens, const int* __restrict__ block_table, int table_stride,
     bf16* __restrict__ cache, int nq, int nkv, int window, float scale, int nsplit,
     float* __restrict__ part_o, float* __restrict__ part_ml, const float* __restrict__ cs,
-    const float* __restrict__ sn, int write_cache, const float* __restrict__ qruns, int runs, size_t run_stride) {
+    const float* __restrict__ sn, int write_cache, const float* __restrict__ qruns, int runs, size_t run_stride, int fold) {
     constexpr int NB = HD / 32;                      // 32-wide k-steps of the score product
     constexpr int KROWB = HD * 2, KCOLS = KROWB / 16; // a key row in bytes, in 16-byte columns
     constexpr int KB = PAGE * KROWB, STAGE = 2 * KB;  // keys, then values [HD][128 bytes]
@@ -786,7 +790,8 @@ __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
     extern __shared__ __attribute__((aligned(1024))) unsigned char dsm[];
     int* bts = (int*)(dsm + S * STAGE);
     const int G = nq / nkv, nhb = (G + 15) / 16;
-    const int split = blockIdx.x, kvh = blockIdx.y / nhb, hb = blockIdx.y % nhb, b = blockIdx.z;
+    const int split = blockIdx.x, kvh = blockIdx.y / nhb, hb = blockIdx.y % nhb;
+    const int b = (int)blockIdx.z < fold ? blockIdx.z : fold + gridDim.z - 1 - blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
@@ -1249,7 +1254,9 @@ static int attn_decode_launch(const void* q, size_t q_stride, void* out, const i
         // two stages leave room for two workgroups per CU; with at most one workgroup per CU
         // a third stage keeps two pages in flight instead (measured: 34 -> 32 us at 8 x 4096 tokens)
         const int cus = br_device_cus();
-        const bool deep = cus > 0 && (long long)nsplit * nkv * nhb * B <= cus;
+        const int each = nsplit * nkv * nhb;
+        const bool deep = cus > 0 && (long long)each * B <= cus;
+        const int fold = cus > 0 && !deep && cus % each == 0 && (long long)each * B <= 2LL * cus ? cus / each : B;
 #define BR_DECODE_LDS(HD_, S_, FUSE_)                                                                          \
     do {                                                                                                        \
         auto kern = attn_decode_lds_kernel<HD_, S_, FUSE_>;                                                     \
@@ -1263,7 +1270,7 @@ static int attn_decode_launch(const void* q, size_t q_stride, void* out, const i
         }                                                                                                       \
         kern<<<grid, 256, lds2, s>>>((const bf16*)q, q_stride, (bf16*)out, slots, ctx_lens, block_table,        \
                                      table_stride, (bf16*)cache, nq, nkv, window, scale, nsplit, part_o,        \
-                                     part_ml, cs, sn, write_cache, qruns, runs, run_stride);                    \
+                                     part_ml, cs, sn, write_cache, qruns, runs, run_stride, fold);              \
     } while (0)
         if (fuse) {
             if (hd == 128) { if (deep) BR_DECODE_LDS(128, 3, true); else BR_DECODE_LDS(128, 2, true); }
