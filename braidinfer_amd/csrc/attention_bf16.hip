@@ -15,6 +15,7 @@
 // so that the accumulator registers of a lane hold 8 consecutive keys: then the k-slots of
 // the second product are in key order and V^T is read 16 contiguous bytes at a time.
 #include "common.h"
+#include "prefill_order.h"
 #include "no_alloc.h"
 
 #define PAGE 64
@@ -386,7 +387,7 @@ template <int HD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_dma_kernel(
     const bf16* __restrict__ q, size_t q_stride, bf16* __restrict__ out, const int* __restrict__ cu_seqlens,
     const int* __restrict__ slots, const int* __restrict__ ctx_lens, const int* __restrict__ block_table,
-    int table_stride, const bf16* __restrict__ cache, int nq, int nkv, int window, float scale, int pair) {
+    int table_stride, const bf16* __restrict__ cache, int nq, int nkv, int window, float scale, const PrefillOrder order) {
     constexpr int NB = HD / 32, NW = 4;
     constexpr int KROWB = HD * 2, KCOLS = KROWB / 16;       // a key row in bytes, in 16-byte columns
     constexpr int KB = PAGE * KROWB, STAGE = 2 * KB;        // keys, then values [HD][128 bytes]
@@ -394,12 +395,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int KROWS = 1024 / KROWB;                     // key rows per wave-load
     extern __shared__ __attribute__((aligned(1024))) unsigned char dsm[];
     int* bts = (int*)(dsm + 2 * STAGE);
-    const int b = blockIdx.z, kvh = blockIdx.y;
+    int kvh, b, tile;
+    order.place(blockIdx.x, kvh, b, tile);
     const int slot = slots[b];
     const int t0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t0;
     const int G = nq / nkv;
     const int rows_total = n_new * G;
-    const int tile = (pair && ((blockIdx.y * 2 / gridDim.y) & 1)) ? blockIdx.x : gridDim.x - 1 - blockIdx.x;
     if (tile * (NW * 32) >= rows_total) return;           // the whole workgroup leaves together
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1149,9 +1150,9 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
     // LDS than with the fragments straight from the cache, which remains for head sizes beyond 192.
     if (variant == 0) variant = dma_ok ? 4 : hd <= 128 ? 3 : hd <= 192 ? 2 : 1;
     if (variant == 4) {
-        dim3 grid4(((size_t)max_new * G + 127) / 128, nkv, B);
-        const int cus = br_device_cus();
-        const int pair = cus > 0 && (long long)grid4.x * nkv * B <= 2LL * cus;
+        PrefillOrder order;
+        const unsigned grid4 = prefill_order(order, (long long)max_new * G, nkv, B, br_device_cus(), 2);
+        if (!grid4) return BR_BAD_ARG;
 #define BR_PREFILL_DMA(HD_)                                                                                \
     do {                                                                                                   \
         auto kern = attn_prefill_dma_kernel<HD_>;                                                          \
@@ -1164,7 +1165,7 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
         }                                                                                                  \
         kern<<<grid4, 256, lds4, s>>>((const bf16*)q, q_stride, (bf16*)out, cu_seqlens, slots, ctx_lens,  \
                                       block_table, table_stride, (const bf16*)cache, nq, nkv, window,      \
-                                      scale, pair);                                                        \
+                                      scale, order);                                                       \
     } while (0)
         if (hd == 128) BR_PREFILL_DMA(128); else BR_PREFILL_DMA(64);
 #undef BR_PREFILL_DMA

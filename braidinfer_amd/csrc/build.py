@@ -45,7 +45,7 @@ MODULES: Dict[str, List[str]] = {
     "experts_wide": ["experts_wide.hip"],
     "streams": ["streams.hip"],
 }
-HEADERS = ["common.h", "no_alloc.h", "expert_units.h"]
+HEADERS = ["common.h", "no_alloc.h", "expert_units.h", "prefill_order.h"]
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

@@ -25,6 +25,7 @@
 // sequence's first `keep` tokens, wherever its window begins.  The kept rows that lie before the window are
 // walked first, like the pooled rows.  `softcap` > 0 bounds the scaled scores: s <- softcap tanh(s / softcap).
 #include "common.h"
+#include "prefill_order.h"
 
 #define MAX_EPL 8   // head widths up to 64 * MAX_EPL
 
@@ -1234,7 +1235,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
     const bf16* __restrict__ q, bf16* __restrict__ out, const int* __restrict__ cu_seqlens,
     const int* __restrict__ slots, const int* __restrict__ ctx_lens, const int* __restrict__ block_table,
     int table_stride, const bf16* __restrict__ storage, const int* __restrict__ pooled_table, int pooled_stride,
-    const bf16* __restrict__ pooled, int nq, int nkv, int size, int pool, float scale, int sink, const float* __restrict__ sinks, int pair,
+    const bf16* __restrict__ pooled, int nq, int nkv, int size, int pool, float scale, int sink, const float* __restrict__ sinks, const PrefillOrder order,
     int chunk, int keep, float softcap, int maps) {
     constexpr int NBK = DK / 32, NBV = DV / 32, KCOLS = DK / 8, KB = PWA_PAGE * DK * 2, STAGE = KB + DV * PWA_PAGE * 2;
     constexpr int KINSTR = KB / 1024, NDMA = STAGE / 1024 / 4;       // wave-loads of 1 KB: of the keys; per wave and page
@@ -1242,13 +1243,15 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
     static_assert(DK % 32 == 0 && DV % 32 == 0 && STAGE % 4096 == 0 && (KCOLS % 16 == 0 || KCOLS % 16 == 8), "sizes");
     extern __shared__ __attribute__((aligned(1024))) unsigned char pwa_lds[];
     int* list = (int*)(pwa_lds + 2 * STAGE);
-    const int b = blockIdx.z, kvh = blockIdx.y / maps, map = blockIdx.y % maps;
+    int hm, b, tile;                                         // (kv head, map), sequence, 128 rows
+    order.place(blockIdx.x, hm, b, tile);
+    const int kvh = hm / maps, map = hm % maps;
     const int slot = slots[b];
     const int t0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t0;
     const int G = nq / (nkv * maps), kw = maps * DK;
     const int rows_total = n_new * G;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wg_row0 = pwa_tile(pair) * 128;
+    const int wg_row0 = tile * 128;
     if (wg_row0 >= rows_total) return;                       // the whole workgroup
     const int row0 = wg_row0 + wave * 32;
     const bool wave_on = row0 < rows_total;
@@ -1451,10 +1454,10 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
     const long long pages = (long long)table_stride + (pool > 0 ? pooled_stride : 0) + (keep > 0 ? (keep + PWA_PAGE - 1) / PWA_PAGE : 0);
     if ((long long)grid.x * 128 >= 256 && pages <= PWA_MAX_LIST && ((uintptr_t)storage | (uintptr_t)pooled | (uintptr_t)q) % 16 == 0 &&
         (unsigned long long)nkv * PWA_PAGE * ((unsigned long long)maps * dk + dv) * 2 < (1ull << 32)) {
-        const int cus = br_device_cus();
-        const int pair = cus > 0 && (long long)grid.x * grid.y * grid.z <= 2LL * cus;
+        PrefillOrder order;
+        const unsigned units = prefill_order(order, (long long)max_new * G, nkv * maps, B, br_device_cus(), dk + dv <= 256 ? 2 : 1);
 #define PWA_DMA(DK_, DV_)                                                                                                              \
-        if (dk == DK_ && dv == DV_) {                                                                                                  \
+        if (units && dk == DK_ && dv == DV_) {                                                                                         \
             auto kern = pwa_prefill_dma_kernel<DK_, DV_>;                                                                              \
             const size_t lds = (size_t)2 * PWA_PAGE * (DK_ + DV_) * 2 + (((size_t)pages + 3) & ~(size_t)3) * sizeof(int);               \
             static bool set = false;                                                                                                   \
@@ -1464,8 +1467,8 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
                     return BR_LAUNCH_FAILED;                                                                                           \
                 set = true;                                                                                                            \
             }                                                                                                                          \
-            kern<<<grid, 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,            \
-                                        (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, size, pool, scale, sink, sinks, pair, chunk, keep, \
+            kern<<<units, 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,           \
+                                        (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, size, pool, scale, sink, sinks, order, chunk, keep, \
                                         softcap, maps);                                                                                \
             return br_check_launch();                                                                                                  \
         }
