@@ -194,6 +194,10 @@ __device__ __forceinline__ void f32_for(F&& f) {
         f(std::integral_constant<int, N_ - 1>{});
     }
 }
+template <int LEFT>
+__device__ __forceinline__ void f32_wait() {                  // all but the last LEFT loads, and all reads of LDS
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
+}
 template <int TJ, int MODE, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int M, int N, int K, size_t lda, size_t ldc,
@@ -273,8 +277,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
         constexpr int LEFT = decltype(left_)::value;
         constexpr int FOURS = LEFT * (4 * NA + NB) < 63 ? LEFT * (4 * NA + NB) : 63;
         static_assert(LEFT * (NA + NB) < 64, "vmcnt");
-        if (a_aligned) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT * (NA + NB)) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(FOURS) : "memory");
+        if (a_aligned) f32_wait<LEFT * (NA + NB)>();
+        else f32_wait<FOURS>();
     };
     Set x0, x1;
     if (kt0 < kt1) {
