@@ -1228,7 +1228,8 @@ __global__ __launch_bounds__(256, ((NBK <= 4 && NBV <= 4) ? 2 : 1)) void pwa_pre
 // nothing passes through registers.  The workgroup's page numbers lie in LDS.  Where one workgroup fills a compute unit (DK + DV > 256: its
 // LDS, and the sums of 32 rows take 80 to 112 registers a lane) a block's keys are read half a block ahead and its values in front of the softmax.
 // us with pages through registers, with this form: 1,801 tokens, 32 heads of 256 / 224 over one row of keys 292 / 131, 16 of 192 / 160 264 / 94; 3,517
-// and 1,501 tokens, 32 heads of 128 over 8, window 2,048 with pooled rows 300 / 202; three texts, 16 of 128 over 8 88 / 58.
+// and 1,501 tokens, 32 heads of 128 over 8, window 2,048 with pooled rows 300 / 202, in the order of prefill_order.h 180; three texts, 16 of 128 over 8
+// 88 / 58.
 #define PWA_MAX_LIST 3840
 template <int DK, int DV>
 __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_kernel(
