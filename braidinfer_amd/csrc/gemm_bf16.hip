@@ -34,16 +34,7 @@
 #define OUT_SWIGLU 3
 #define SSQ_LD 64           // row stride of the sums of squares that a product leaves for the next RMS norm
 
-// x / (1 + e^-y) by the vector units' base-2 exponential and reciprocal, the product with log2 e in two parts.  (Beyond +-10,000 the
-// quotient is x or 0, as it is at the infinities, of which the two parts would make a NaN.)  With expf and a division a gated 256x256 tile
-// spends 6 of its 100 us at K = 4,096 on them: 28,672 x 4,096 by 3,625 rows 692 -> 674 us, by 7,001 1,282 -> 1,253.
-__device__ __forceinline__ float sigmoid_times(float x, float y) {
-    y = __builtin_amdgcn_fmed3f(y, -1e4f, 1e4f);
-    const float t = y * -1.44269502f, lo = fmaf(y, -1.44269502f, -t) + y * -1.92596299e-8f;
-    const float e = __builtin_amdgcn_exp2f(t) * fmaf(lo, 0.693147181f, 1.f);
-    return x * __builtin_amdgcn_rcpf(1.f + e);
-}
-__device__ __forceinline__ float silu_mul(float g, float u) { return sigmoid_times(g, g) * u; }
+__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + expf(-g)) * u; }
 
 template <int MODE>
 __device__ __forceinline__ void store_out(void* C, size_t idx, float v) {
@@ -531,7 +522,7 @@ __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr
     if (gr.alpha > 0.f) {
         g = fminf(g, gr.limit);
         u = fminf(fmaxf(u, -gr.limit), gr.limit);
-        return sigmoid_times(g, gr.alpha * g) * (u + 1.0f);
+        return g / (1.0f + expf(-gr.alpha * g)) * (u + 1.0f);
     }
     return silu_mul(g, u);
 }
