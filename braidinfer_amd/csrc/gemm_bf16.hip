@@ -1123,12 +1123,12 @@ static int launch_tile_dma(const bf16* A, const bf16* W, void* C, int M, int N, 
 
 // Which direct-to-LDS tile (5: 128x256, one workgroup per CU; 6: 128x128, two; 10: 256x192, one, two
 // stages, not split) and how many runs of k-tiles for a product of more than 64 rows: the least time by
-// a rough count in microseconds, which it returns (rounds of workgroups over the chip times k-tiles times 1.0-1.7 us a
+// a rough count in microseconds (rounds of workgroups over the chip times k-tiles times 1.0-1.7 us a
 // k-tile, plus, when split, a launch and the traffic of the partial sums), runs of at least 4 k-tiles
 // that fit the scratch memory.  The 256x192 tile is there for shapes that it covers in fewer rounds:
 // 2,048 x 6,144 is 256 of them, one round, against 384 tiles of 128x256 (measured 103-118 against
 // 129-134 us); with equal rounds it loses (two stages, 1.5 times the work a k-tile for 1.5 times the time).
-static double choose_tile(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* kernel, int* parts) {
+static void choose_tile(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* kernel, int* parts) {
     const int nk = K / DMA_BK;
     double best = 1e30;
     *kernel = 5;
@@ -1158,7 +1158,6 @@ static double choose_tile(int M, int N, int K, int mode, int cus, size_t scratch
             if (t < best - 1e-9) { best = t; *kernel = k; *parts = p; }
         }
     }
-    return best;
 }
 
 // ----------------------------------------------------------------- gemm_skinny ------
@@ -2395,7 +2394,7 @@ static bool tile_norms(int M, int N, int K, int cus) { return M > 16 || (N <= 32
 static bool tile_takes(int M, int K, size_t lda) { return M > 0 && M <= TILE_MAX_ROWS && K % 128 == 0 && K >= 256 && lda >= (size_t)K; }
 
 // ------------------------------------------------------------- gemm_stream_wide ------
-// 16 < M <= 96, K in steps of 128: the same streaming by workgroups that stay, with the
+// 16 < M <= 64, K in steps of 128: the same streaming by workgroups that stay, with the
 // activations shared.  A unit of work is a tile of 16 HB weight rows (64 to 128) over one run of
 // k-chunks (the whole K, or one of `parts` runs); height and runs are chosen so that the units
 // fill the compute units in whole rounds (wide_shape below: 28,672 rows are 256 tiles of 112).
@@ -2445,10 +2444,8 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
 #pragma unroll
         for (int j = 0; j < MB; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Products that are cut into runs otherwise, several inputs' and those of more than 64 rows: sums of four chunks, added up
-    constexpr bool FAR = BRANCHES || MB > 4;
-    f32x4 far[TWO ? 2 : 1][MB];
-    if (FAR) {
+    f32x4 far[TWO ? 2 : 1][MB];                             // BRANCHES: the sums of the runs of four chunks before
+    if (BRANCHES) {
 #pragma unroll
         for (int t = 0; t < (TWO ? 2 : 1); ++t)
 #pragma unroll
@@ -2565,9 +2562,9 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
         }
         ++done;
         --cp_left;
-        if (FAR && (cp_left == 0 || (done & 3) == 0)) {
-            // they round no more than the runs (4,096 by 4,096, 24 and 64 rows: error against 64 bits 1.06e-7 of the result, cut into runs
-            // 1.06e-7 and 1.34e-7, one chain 2.7e-7)
+        if (BRANCHES && (cp_left == 0 || (done & 3) == 0)) {
+            // a product that is cut into runs otherwise: sums of four chunks, added up, round no more than those (4,096 by 4,096,
+            // 24 and 64 rows: error against 64 bits 1.06e-7 of the result, cut into runs 1.06e-7 and 1.34e-7, one chain 2.7e-7)
 #pragma unroll
             for (int t = 0; t < (TWO ? 2 : 1); ++t)
 #pragma unroll
@@ -2577,7 +2574,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
                 }
         }
         if (cp_left > 0) continue;
-        if (FAR) {
+        if (BRANCHES) {
 #pragma unroll
             for (int t = 0; t < (TWO ? 2 : 1); ++t)
 #pragma unroll
@@ -2665,7 +2662,7 @@ __global__ __launch_bounds__(512) void gemm_stream_wide_kernel(const bf16* __res
 // units, times the run's chunks, times what a chunk costs (its weight rows and a constant for
 // the activations, which come from the L2, and the barrier), plus the traffic of the partial
 // sums.  Ties go to fewer runs, then to lower tiles.
-static void wide_shape(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* hb_out, int* parts_out, int tallest = 8) {
+static void wide_shape(int M, int N, int K, int mode, int cus, size_t scratch_bytes, int* hb_out, int* parts_out) {
     const int nch = K / 128;
     double best_cost = 1e30;
     *hb_out = 4;
@@ -2675,7 +2672,7 @@ static void wide_shape(int M, int N, int K, int mode, int cus, size_t scratch_by
             break;
         const int cpp = (nch + parts - 1) / parts;
         if ((nch + cpp - 1) / cpp != parts) continue;                // it would leave a run empty
-        for (int hb = 4; hb <= tallest; ++hb) {
+        for (int hb = 4; hb <= 8; ++hb) {
             const int h = 16 * hb;
             const long long tiles = (N + h - 1) / h;
             const long long rounds = (tiles * parts + cus - 1) / cus;
@@ -2684,20 +2681,6 @@ static void wide_shape(int M, int N, int K, int mode, int cus, size_t scratch_by
             if (cost < best_cost * (1.0 - 1e-9)) { best_cost = cost; *hb_out = hb; *parts_out = parts; }
         }
     }
-}
-
-// Whether 65 to 96 rows, too, go by gemm_stream_wide: a product that it takes without runs along k and whose count is the smaller by a tenth.  A
-// chunk costs 0.0094 us a weight row (and 16 for the activations) with up to 80 rows, 0.0118 with up to 96; the other side is
-// choose_tile's.  us by the tiles of eight waves and their runs / here, cold weights: gated 28,672 x 4,096 by 67 rows 49.3 / 44.2, by 80 50.1 / 46.2, by 81
-// 49.9 / 53.0 (stays), 17,920 x 4,096 by 67 39.0 / 34.1, by 96 41.8 / 40.0, 11,264 x 2,048 by 67 21.5 / 15.5, by 96 23.7 / 17.1; 16,384 x 4,096 by 67
-// 35.7 / 29.6, by 96 35.6 / 32.5, 12,288 x 4,096 by 67 30.4 / 28.6, by 96 30.5 / 32.0 (stays); 32,768 x 4,096 in float by 67 55.6 / 50.4, by 81 56.1 / 65.3
-// (stays).  Added into float rows the runs' sum can be shared with a norm: those stay.
-static bool wide_rows_pay(int M, int N, int K, int mode, int cus, size_t scratch_bytes) {
-    if (M <= 64 || M > 96 || mode == OUT_F32_ACC || cus <= 0) return false;
-    int hb, parts, k, p;
-    wide_shape(M, N, K, mode, cus, 0, &hb, &parts, M <= 80 ? 8 : 7);
-    const long long rounds = ((long long)((N + 16 * hb - 1) / (16 * hb)) + cus - 1) / cus;
-    return (double)rounds * (K / 128) * (16 * hb + 16) * (M <= 80 ? 0.0094 : 0.0118) < 0.9 * choose_tile(M, N, K, mode, cus, scratch_bytes, &k, &p);
 }
 
 // norm: 0 none; 1 the product is added into the residual rows C and prepares the next RMS norm
@@ -2716,8 +2699,7 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
     if (!cus) return BR_LAUNCH_FAILED;
     const int nch = K / 128;
     int hb, parts;
-    wide_shape(M, N, K, mode, cus, scratch ? scratch_bytes : 0, &hb, &parts, MB <= 5 ? 8 : 7);
-    if (norm && MB > 4) return BR_BAD_ARG;
+    wide_shape(M, N, K, mode, cus, scratch ? scratch_bytes : 0, &hb, &parts);
     if (leave && (parts < 2 || norm == 1 || force_hb || force_parts)) return BR_BAD_ARG;
     if (force_hb) {
         if (force_hb < 4 || force_hb > 8) return BR_BAD_ARG;
@@ -2760,9 +2742,7 @@ static int launch_stream_wide(const bf16* A, const bf16* W, void* C, int M, int 
         case 5: BR_WIDE(5); break;
         case 6: BR_WIDE(6); break;
         case 7: BR_WIDE(7); break;
-        default:
-            if constexpr (MB <= 5) BR_WIDE(8);
-            else return BR_BAD_ARG;
+        default: BR_WIDE(8); break;
     }
 #undef BR_WIDE
     int rc = br_check_launch();
@@ -2812,7 +2792,7 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     const bool dma_ok = aligned && K % DMA_BK == 0;
     const bool stream_ok = aligned && M <= 16 && K % STREAM_KC == 0 && K / STREAM_KC >= STREAM_NW;
     if (kernel >= 4 && kernel <= 6 && !dma_ok) return BR_BAD_ARG;
-    const bool wide_ok = aligned && M > 16 && M <= 96 && K % 128 == 0 && K >= 256 &&
+    const bool wide_ok = aligned && M > 16 && M <= 64 && K % 128 == 0 && K >= 256 &&
                          (!scratch || (uintptr_t)scratch % 16 == 0);
     if ((kernel == 7 && (forced_parts ? !(aligned && tile_takes(M, K, lda)) : !stream_ok)) || (kernel == 8 && !wide_ok) || kernel > 15 || kernel < 0 || (kernel >= 10 && !dma_ok) ||
         (kernel == 11 && mode != OUT_SWIGLU) ||
@@ -2839,14 +2819,15 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
     }
     if (kernel == 0)
         kernel = stream_ok ? 7
-                 : wide_ok && M <= 64 ? 8
+                 : wide_ok ? 8
                  : (aligned && M <= 64) ? (wl ? 9 : 3) : (!dma_ok ? 1 : (N > 128 ? 5 : 6));
     if (kernel == 9) return launch_tile_dma<64, 128, 1, 4, 3>(A, W, C, M, N, K, lda, ldc, mode, s, 1, nullptr, wl);
     if (kernel == 8) {
         const int fh = chosen ? 0 : forced_parts % 16, fp = chosen ? 0 : forced_parts / 16;
-#define BR_WIDE_ROWS(MB_) launch_stream_wide<MB_>(A, W, C, M, N, K, lda, ldc, mode, (float*)scratch, scratch_bytes, s, 0, StreamNorm{}, fh, fp, wl)
-        return M <= 32 ? BR_WIDE_ROWS(2) : M <= 64 ? BR_WIDE_ROWS(4) : M <= 80 ? BR_WIDE_ROWS(5) : BR_WIDE_ROWS(6);
-#undef BR_WIDE_ROWS
+        return M <= 32 ? launch_stream_wide<2>(A, W, C, M, N, K, lda, ldc, mode, (float*)scratch, scratch_bytes, s, 0,
+                                               StreamNorm{}, fh, fp, wl)
+                       : launch_stream_wide<4>(A, W, C, M, N, K, lda, ldc, mode, (float*)scratch, scratch_bytes, s, 0,
+                                               StreamNorm{}, fh, fp, wl);
     }
     if (kernel == 7 && !chosen && forced_parts) {      // 7 + 16 b: a workgroup a tile of 8 (b + 1) weight rows, b = 1, 2, 3
         return launch_stream_tile(8 * (forced_parts + 1), 0, A, W, C, M, N, K, lda, ldc, mode, s, StreamNorm{}, wl);
@@ -2885,9 +2866,6 @@ extern "C" int br_gemm_bf16_ex(const void* A_, const void* W_, void* C, int M, i
             }
         }
     }
-    if (chosen && wide_ok && wide_rows_pay(M, N, K, mode, br_device_cus(), scratch ? scratch_bytes : 0))
-        return M <= 80 ? launch_stream_wide<5>(A, W, C, M, N, K, lda, ldc, mode, nullptr, 0, s, 0, StreamNorm{}, 0, 0, wl)
-                       : launch_stream_wide<6>(A, W, C, M, N, K, lda, ldc, mode, nullptr, 0, s, 0, StreamNorm{}, 0, 0, wl);
     if (chosen && (kernel == 5 || kernel == 6)) {
         const int cus = br_device_cus();
         if (cus > 0) choose_tile(M, N, K, mode, cus, (scratch && (uintptr_t)scratch % 16 == 0) ? scratch_bytes : 0, &kernel, &parts);
