@@ -649,6 +649,9 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
                                                               size_t ldc, int tiles_m, int tiles_n, int kt_per_part,
                                                               size_t part_stride, int wl, typename QuadArg<KIND>::type gr) {
     constexpr bool GROUPED = KIND == QUAD_EXPERTS;
+    // Branches by tiles of 128 rows: runs of kt_per_part k-tiles, one after another, whose sums are added up in registers in the order and with the
+    // bits of gemm_split_sum_kernel (a tile of 256 rows has no registers left for them).
+    constexpr bool RUNS = KIND == QUAD_BRANCHES && BM == 128;
     constexpr int SA = BM * 128, SB = BN * 128;          // bytes of a stage of activation rows, of weight rows
     constexpr int WVN = 4 / WVM;                         // the four waves: WVM along the activation rows x WVN
     constexpr int TI = BN / WVN / 32, TJ = BM / WVM / 32; // blocks of a wave: weight rows, activation rows
@@ -683,6 +686,13 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    f32x16 sum[RUNS ? TI : 1][RUNS ? TJ : 1];
+    if constexpr (RUNS) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) sum[i][j] = acc[i][j];
+    }
 
     // wave-load q of this wave: rows (4 q + wave) 8 .. + 8 of the operand's tile, reached by a 32-bit byte
     // offset from the matrix's first element (the launcher checks that this suffices); the pairs of an expert
@@ -719,6 +729,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     unsigned long long baseW = (unsigned long long)W_ + (wl ? (size_t)(kt0 >> 1) * (WL_BLOCK_ELEMS * 2) : (size_t)kt0 * 128);
     int knext = kt0;
     const unsigned hopW = wl ? WL_BLOCK_ELEMS * 2 - 128 : 128;                        // bytes from an odd k-tile on
+    for (int rest = K / DMA_BK - nk;;) {                 // run by run (RUNS), or once
     // where this wave's loads of the next k-tile to ask for land, and which stage that is
     unsigned ldsA = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
     unsigned ldsB = __builtin_amdgcn_readfirstlane(lds0 + NSA * SA + wave * 1024);
@@ -870,7 +881,23 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     static_for<0, TI * TJ>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
     __builtin_amdgcn_s_barrier();                                      // every wave has read its last operands
     asm volatile("" ::: "memory");
-    quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(acc, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, st + wave * QuadStrip<TI, MODE>::BYTES);
+    if constexpr (!RUNS) {
+        break;
+    } else {
+        static_for<0, TI * TJ>([&](auto n_) {
+            constexpr int i = decltype(n_)::value / TJ, j = decltype(n_)::value % TJ;
+            sum[i][j] += acc[i][j];
+            acc[i][j] = f32x16(0.f);
+            quad_touch(acc[i][j]);                                     // block by block: no second copy of them all
+        });
+        if (!rest) break;
+        nk = rest < kt_per_part ? rest : kt_per_part;
+        rest -= nk;
+    }
+    }
+    unsigned char* const strip = st + wave * QuadStrip<TI, MODE>::BYTES;
+    if constexpr (RUNS) quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(sum, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
+    else quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(acc, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
     };
 
     if constexpr (!GROUPED) {
@@ -3079,41 +3106,56 @@ extern "C" int br_gemm_bf16_branches_takes(int M, int per, int K) {
     return M > 0 && M <= 64 && per > 0 && per % 128 == 0 && K % STREAM_KC == 0 && K / STREAM_KC >= STREAM_NW;
 }
 
-// Beyond 128 rows the branches make one product of whole 256-wide columns of tiles (256x256, 128x256).  Taken where that is counted faster than
-// a product for each (with as many runs along k as it likes), which it was at every size timed: few tiles need no runs, many fill their rounds.  Four
-// of 4,096 by 4,096, us by 129 / 512 / 1,024 / 1,801 / 3,000 / 7,000 rows one by one 94 / 138 / 184 / 236 / 372 / 809, at once 45 / 62 / 111 / 206 / 318 /
-// 739; of 2,048 by 2,048 66 / 76 / 98 / 107 / 123 / 232 and 25 / 27 / 37 / 58 / 101 / 230.
-static int branches_tile(int M, int branches, int per, int K, int cus) {       // 12, 13, or 0: a product for each
+// Beyond 128 rows the branches make one product of whole 256-wide columns of tiles (256x256, 128x256).  `room`: the bytes of scratch that a product
+// for each would be given.  Where that would be cut into runs along k, the tiles of 128 rows add up the same runs (`run` k-tiles each;
+// one chain over all of K rounds more: 4,096 by 4,096, 300 rows: error against 64 bits 4.0e-7 of the result, four runs 1.9e-7), so that the
+// bits are those of the products one by one.  Taken where it is counted faster, which it was at every size timed: few tiles need no sum kernels, many
+// fill their rounds.  Four of 4,096 by 4,096, us by 129 / 300 / 512 / 640 / 1,024 / 1,801 / 3,000 / 7,000 rows one by one 94 / 114 / 140 / 166 / 184 / 234 / 369 /
+// 786, at once 68 / 65 / 72 / 118 / 131 / 206 / 319 / 740 (as one chain 55 / 60 / 67 / 84 / 109 up to 1,024); of 2,048 by 2,048 66 / 72 / 82 / 88 / 122 / 115 / 126 / 224 and
+// 43 / 37 / 40 / 40 / 38 / 56 / 104 / 228.  A run costs about 2 us besides its k-tiles: the ring starts anew.
+static int branches_tile(int M, int branches, int per, int K, size_t room, int cus, int* run) {       // 12, 13, or 0: a product for each
     if (M <= 128 || branches < 2 || branches > 64 || per <= 0 || per % 256 || K <= 0 || K % DMA_BK || (long long)branches * per > 0x3fffffff || cus <= 0) return 0;
-    int k, p;
-    const double room = choose_quad(M, per, K, OUT_F32, cus, ~(size_t)0, &k, &p);
-    const double tall = quad_count(M, branches * per, K, OUT_F32, cus, 0, 1), flat = quad_count(M, branches * per, K, OUT_F32, cus, 1, 1);
-    if (min(tall, flat) >= branches * room) return 0;
+    const int nk = K / DMA_BK, N = branches * per;
+    int k, p, rest_k, rest_p;
+    const double one = choose_quad(M, per, K, OUT_F32, cus, room, &k, &p);
+    if (quad_whole_rounds(M, per, K, OUT_F32, cus, room, one, &rest_k, &rest_p)) {
+        if (rest_p > 1) return 0;                                    // columns with runs and columns without
+        p = 1;
+    }
+    int kpp = (nk + p - 1) / p;
+    kpp += kpp & 1;
+    *run = p > 1 ? kpp : nk;
+    const double tall = p > 1 ? 1e30 : quad_count(M, N, K, OUT_F32, cus, 0, 1);
+    const double flat = quad_count(M, N, K, OUT_F32, cus, 1, 1) + (p > 1 ? 2.0 * p : 0.0);
+    if (min(tall, flat) >= branches * one) return 0;
     return tall <= flat ? 12 : 13;
 }
-extern "C" int br_gemm_bf16_branches_pay(int M, int branches, int per, int K) { return branches_tile(M, branches, per, K, br_device_cus()) != 0; }
+extern "C" int br_gemm_bf16_branches_pay(int M, int branches, int per, int K, size_t room) {
+    int run;
+    return branches_tile(M, branches, per, K, room, br_device_cus(), &run) != 0;
+}
 
 template <int BM, int NSA, int NSB>
-static int launch_branches_tiles(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const QuadBranches& br, hipStream_t s) {
+static int launch_branches_tiles(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const QuadBranches& br, int run, hipStream_t s) {
     const int tm = (M + BM - 1) / BM, tn = N / 256;
     if ((long long)tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
-    gemm_tile_quad_kernel<BM, 256, NSA, NSB, 2, OUT_F32, QUAD_BRANCHES><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, K / DMA_BK, 0,
-                                                                                                     WL_ROWS, br);
+    gemm_tile_quad_kernel<BM, 256, NSA, NSB, 2, OUT_F32, QUAD_BRANCHES><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, run, 0, WL_ROWS, br);
     return br_check_launch();
 }
 
 // tail_rows > 0 (up to 16 rows, in steps of 16, at most per): further weight rows, multiplying one more branch's activations, the
 // tanh of whose sums goes to tail [M, tail_ld]: instead of two launches of their own, 8.4 us of a single-token step a layer.
 extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, int M, int branches, int per, int K, size_t a_step, size_t lda,
-                                     size_t ldc, int gap_at, int gap, int tail_rows, void* tail, size_t tail_ld, hipStream_t s) {
+                                     size_t ldc, int gap_at, int gap, int tail_rows, void* tail, size_t tail_ld, size_t room, hipStream_t s) {
     const bf16 *A = (const bf16*)A_, *W = (const bf16*)W_;
-    if (const int kind = branches_tile(M, branches, per, K, br_device_cus())) {
+    int run;
+    if (const int kind = branches_tile(M, branches, per, K, room, br_device_cus(), &run)) {
         if (tail_rows || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 || gap % 4 || gap_at < 0 || gap_at % per || ldc < (size_t)branches * per + gap ||
             ((uintptr_t)A | (uintptr_t)W) % 16 || !quad_takes(C, M, branches * per, K, lda, ldc))
             return BR_BAD_ARG;
         const QuadBranches br = {per, a_step, gap_at, gap};
-        return kind == 12 ? launch_branches_tiles<256, QUAD12>(A, W, C, M, branches * per, K, lda, ldc, br, s)
-                          : launch_branches_tiles<128, QUAD13>(A, W, C, M, branches * per, K, lda, ldc, br, s);
+        return kind == 12 ? launch_branches_tiles<256, QUAD12>(A, W, C, M, branches * per, K, lda, ldc, br, run, s)
+                          : launch_branches_tiles<128, QUAD13>(A, W, C, M, branches * per, K, lda, ldc, br, run, s);
     }
     if (branches < 1 || branches > 64 || !br_gemm_bf16_branches_takes(M, per, K) || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 ||
         gap_at % per || ((uintptr_t)A | (uintptr_t)W) % 16 || ldc < (size_t)branches * per || (long long)branches * per > 0x3fffffff)

@@ -485,17 +485,18 @@ def gemm_branches_takes(M: int, per: int, Kd: int) -> bool:
     return bool(_fn("gemm_bf16", "br_gemm_bf16_branches_takes", [c_int] * 3)(M, per, Kd))
 
 
-def gemm_branches_pay(M: int, branches: int, per: int, Kd: int) -> bool:
-    """Whether more than 128 rows against `per` weight rows a branch (in steps of 256) go faster by `gemm_branches` than branch by branch."""
-    return bool(_fn("gemm_bf16", "br_gemm_bf16_branches_pay", [c_int] * 4)(M, branches, per, Kd))
+def gemm_branches_pay(M: int, branches: int, per: int, Kd: int, room: int = 0) -> bool:
+    """Whether more than 128 rows against `per` weight rows a branch (in steps of 256) go faster by `gemm_branches` than branch by branch,
+    with `room` floats of scratch for each, whose bits they have."""
+    return bool(_fn("gemm_bf16", "br_gemm_bf16_branches_pay", [c_int] * 4 + [c_size_t])(M, branches, per, Kd, room * 4))
 
 
 def gemm_branches(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gap_at: int = 0, gap: int = 0,
-                  tail: Optional[torch.Tensor] = None) -> None:
+                  tail: Optional[torch.Tensor] = None, room: int = 0) -> None:
     """out[:, b * per + j (+ gap where b >= gap_at)] = a[b] @ w[b * per + j]^T for the branches b of a [B, M, K] (bfloat16, up to 64
     rows each or as many as `gemm_branches_pay` says, dense), w [B * per, K] their stacked weights, out float32 [M, B * per + gap]: one launch for all branches.  `gap`
     columns of `out` in front of branch `gap_at` are left alone.  `tail` (bfloat16 [M, R], up to 16 rows, R in steps of 16 up to
-    per): a has one more branch, w R more rows, and tail = tanh(a[B] @ w[B * per:]^T)."""
+    per): a has one more branch, w R more rows, and tail = tanh(a[B] @ w[B * per:]^T).  `room`: as for `gemm_branches_pay`."""
     _dev("gemm_branches", a, w, tail)
     B, M, Kd = a.shape
     R = 0
@@ -505,13 +506,13 @@ def gemm_branches(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gap_at: i
              "gemm_branches: tail bfloat16 [M <= 16, R], R in steps of 16")
     N = w.shape[0] - R
     _req(a.dtype == w.dtype == torch.bfloat16 and w.shape == (N + R, Kd) and N > 0 and N % B == 0 and R <= N // B
-         and (gemm_branches_takes(M, N // B, Kd) or (R == 0 and gap % 4 == 0 and gemm_branches_pay(M, B, N // B, Kd))),
+         and (gemm_branches_takes(M, N // B, Kd) or (R == 0 and gap % 4 == 0 and gemm_branches_pay(M, B, N // B, Kd, room))),
          "gemm_branches: bfloat16 [B, M <= 64, K] and [B * per, K], K in steps of 128 from 1,024, per in steps of 128, or rows and sizes that gemm_branches_pay names")
     _req(out.is_cuda and out.dtype == torch.float32 and out.shape == (M, N + gap) and out.stride(1) == 1 and gap >= 0 and 0 <= gap_at <= B,
          "gemm_branches: out float32 [M, B * per + gap]")
-    f = _fn("gemm_bf16", "br_gemm_bf16_branches", [_P, _P, _P, c_int, c_int, c_int, c_int, c_size_t, c_size_t, c_size_t, c_int, c_int, c_int, _P, c_size_t, _P])
+    f = _fn("gemm_bf16", "br_gemm_bf16_branches", [_P, _P, _P, c_int, c_int, c_int, c_int, c_size_t, c_size_t, c_size_t, c_int, c_int, c_int, _P, c_size_t, c_size_t, _P])
     _check(f(_ptr(a), _ptr(w), _ptr(out), M, B, N // B, Kd, M * Kd, Kd, out.stride(0) if M > 1 else N + gap, gap_at * (N // B), gap, R, _ptr(tail), R,
-             _stream()), "gemm_branches")
+             room * 4, _stream()), "gemm_branches")
 
 
 def gemm_swiglu(a: torch.Tensor, w_gu: torch.Tensor, out: torch.Tensor, kernel: int = 0,

@@ -13,6 +13,11 @@ from .. import kernels as K
 from .base import NormedInput, ProductRuns, ResidualSink
 
 
+def split_room(rows: int) -> int:
+    """Floats of scratch that `linear` gives a product of so many rows: those that may be split along k."""
+    return K.GEMM_SCRATCH_FLOATS if 16 < rows <= 1024 else 0
+
+
 def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False, whole: bool = True) -> None:
     """out (+)= a @ w^T.  `accumulate` needs a float32 `out`.  `w` is [N, K] or what
     `stream_layout` made of it.
@@ -42,9 +47,8 @@ def linear(a, w: torch.Tensor, out, ws, accumulate: bool = False, whole: bool = 
                 K.gemm(a, w, tmp)
                 K.convert(tmp, out)
                 return
-            scratch = None
-            if 16 < a.shape[0] <= 1024:     # products that may be split along k
-                scratch = ws.get("gemm_scratch", (K.GEMM_SCRATCH_FLOATS,), torch.float32)
+            room = split_room(a.shape[0])
+            scratch = ws.get("gemm_scratch", (room,), torch.float32) if room else None
             K.gemm(a, w, out, accumulate, scratch=scratch, whole=whole)
             return
     if w.dtype == torch.float32 and a.dtype == torch.bfloat16:

@@ -28,7 +28,7 @@ from ..errors import ConfigError, StepError
 from ..weights import TensorSpec
 from .base import Mixer, MixerContext, Runtime, register_part
 from .gated_recurrence import HGRN2, chunk_scratch, in_chunks, pieces_for
-from .linear import blocks_at_load, linear, stream_layout
+from .linear import blocks_at_load, linear, split_room, stream_layout
 
 BRANCHES = ("r", "k", "v", "g", "w")
 
@@ -117,12 +117,13 @@ class WKVTimeMix(Mixer):
         rows = step.ws.get("wkv_rows", (T, 5 * hd), torch.float32)
         low_t = step.ws.get("wkv_low_t", (T, self.rank), dt)
         tail = None
-        if self.w_four is not None and dt == torch.bfloat16 and (K.gemm_branches_takes(T, hd, self.H) or K.gemm_branches_pay(T, 4, hd, self.H)):
+        room = split_room(T)
+        if self.w_four is not None and dt == torch.bfloat16 and (K.gemm_branches_takes(T, hd, self.H) or K.gemm_branches_pay(T, 4, hd, self.H, room)):
             tail = low_t if self.w_five is not None and T <= 16 else None
             if tail is not None:
                 K.gemm_branches(mixes, self.w_five, rows, gap_at=3, gap=hd, tail=tail)
             else:
-                K.gemm_branches(mixes[:4], self.w_four, rows, gap_at=3, gap=hd)
+                K.gemm_branches(mixes[:4], self.w_four, rows, gap_at=3, gap=hd, room=room)
         else:
             for i, s in enumerate(("r", "k", "v")):
                 linear(mixes[i], self.w[s], rows[:, i * hd:(i + 1) * hd], step.ws)

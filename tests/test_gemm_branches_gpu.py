@@ -43,6 +43,25 @@ def test_branches_of_many_rows(M, B, per, K_, gap_at, gap):
     assert torch.equal(torch.cat(again.split(per, 1)[::-1], 1), out)
 
 
+# eight, four, two runs along k and none; rows that end inside a tile; a last run that is shorter (K = 1,344: 22 k-tiles in runs of 6)
+@pytest.mark.parametrize("M", [129, 130, 300, 512, 700, 1024])
+@pytest.mark.parametrize("B,per,K_", [(4, 4096, 4096), (4, 2048, 2048), (2, 512, 1344), (3, 256, 1024)])
+def test_branches_have_the_bits_of_the_products_one_by_one(M, B, per, K_):
+    from braidinfer_amd import kernels as K
+    room = K.GEMM_SCRATCH_FLOATS
+    assert K.gemm_branches_pay(M, B, per, K_, room)
+    g = torch.Generator(device="cuda").manual_seed(M + K_)
+    a = torch.randn(B, M, K_, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(B * per, K_, generator=g, device="cuda").to(torch.bfloat16)
+    scratch = torch.full((room,), float("nan"), device="cuda")
+    want, out = torch.empty(M, B * per, device="cuda"), torch.full((M, B * per + 8), 7.0, device="cuda")
+    for b in range(B):
+        K.gemm(a[b], w[b * per:(b + 1) * per], want[:, b * per:(b + 1) * per], scratch=scratch)
+    K.gemm_branches(a, w, out, gap_at=1, gap=8, room=room)
+    assert torch.equal(out[:, :per], want[:, :per]) and torch.equal(out[:, per + 8:], want[:, per:])
+    assert torch.all(out[:, per:per + 8] == 7.0)
+
+
 def test_branches_of_many_rows_refuse():
     from braidinfer_amd import kernels as K
     from braidinfer_amd.errors import KernelError
