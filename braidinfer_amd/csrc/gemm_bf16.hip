@@ -3116,6 +3116,7 @@ extern "C" int br_gemm_bf16_branches_takes(int M, int per, int K) {
 static int branches_tile(int M, int branches, int per, int K, size_t room, int cus, int* run) {       // 12, 13, or 0: a product for each
     if (M <= 128 || branches < 2 || branches > 64 || per <= 0 || per % 256 || K <= 0 || K % DMA_BK || (long long)branches * per > 0x3fffffff || cus <= 0) return 0;
     const int nk = K / DMA_BK, N = branches * per;
+    if (!quad_takes(nullptr, M, N, K, (size_t)K, 4)) return 0;
     int k, p, rest_k, rest_p;
     const double one = choose_quad(M, per, K, OUT_F32, cus, room, &k, &p);
     if (quad_whole_rounds(M, per, K, OUT_F32, cus, room, one, &rest_k, &rest_p)) {

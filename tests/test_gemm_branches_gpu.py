@@ -62,6 +62,13 @@ def test_branches_have_the_bits_of_the_products_one_by_one(M, B, per, K_):
     assert torch.all(out[:, per:per + 8] == 7.0)
 
 
+def test_branches_beyond_32_bit_offsets_go_one_by_one():
+    """What is said to pay is taken: rows and weights below 4 GB, as the tiles of four waves reach them."""
+    from braidinfer_amd import kernels as K
+    assert K.gemm_branches_pay(524287, 4, 4096, 4096) and not K.gemm_branches_pay(524288, 4, 4096, 4096)
+    assert K.gemm_branches_pay(1801, 63, 8192, 4096) and not K.gemm_branches_pay(1801, 64, 8192, 4096)
+
+
 def test_branches_of_many_rows_refuse():
     from braidinfer_amd import kernels as K
     from braidinfer_amd.errors import KernelError
