@@ -1334,7 +1334,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
             const unsigned lds = __builtin_amdgcn_readfirstlane(ring_lds + (n & 1) * STAGE + (wave * NDMA + i) * 1024);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(goff[i]), "s"(pg) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(goff[i]), "s"(pg) : "m0", "memory");
         }
     };
     issue(0);

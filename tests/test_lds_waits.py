@@ -23,3 +23,15 @@ def test_sums_of_squares_are_in_lds_before_a_barrier():
     for write in (r"sq\[tid\] = t;", r"rstd\[lane\] = [^;]*;"):
         after = re.findall(write + r"\s*([^;]*);", source)
         assert len(after) == 1 and "s_waitcnt lgkmcnt(0)" in after[0], after
+
+
+def test_statements_that_write_m0_say_so():
+    """A statement that writes m0 without naming it lets the compiler keep a value of its own there."""
+    for name in sorted(os.listdir(CSRC)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        with open(os.path.join(CSRC, name)) as f:
+            statements = re.findall(r'asm volatile\((.*?)\);', f.read().replace("\\\n", "\n"), re.S)
+        for text in statements:
+            if re.search(r"\bm0\b", text.split("::")[0]):
+                assert re.search(r':\s*[^:]*"m0"[^:]*$', text), (name, text)
