@@ -396,7 +396,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     extern __shared__ __attribute__((aligned(1024))) unsigned char dsm[];
     int* bts = (int*)(dsm + 2 * STAGE);
     int kvh, b, tile;
-    order.place(blockIdx.x, kvh, b, tile);
+    order.place(kvh, b, tile);
     const int slot = slots[b];
     const int t0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t0;
     const int G = nq / nkv;
@@ -1148,11 +1148,11 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
     // page barriers: 18 to 21 % faster at 8,192 tokens; beyond 128 four waves spill registers, beyond 192 eight do)
     // Short steps too: 16 to 64 new tokens over 1,024 to 8,192 earlier ones run 2.5 to 3 times faster through
     // LDS than with the fragments straight from the cache, which remains for head sizes beyond 192.
-    if (variant == 0) variant = dma_ok ? 4 : hd <= 128 ? 3 : hd <= 192 ? 2 : 1;
+    PrefillOrder order;
+    const unsigned grid4 = dma_ok ? prefill_order(order, (long long)max_new * G, nkv, B, br_device_cus(), 2) : 0;
+    if (variant == 4 && !grid4) return BR_BAD_ARG;
+    if (variant == 0) variant = grid4 ? 4 : hd <= 128 ? 3 : hd <= 192 ? 2 : 1;
     if (variant == 4) {
-        PrefillOrder order;
-        const unsigned grid4 = prefill_order(order, (long long)max_new * G, nkv, B, br_device_cus(), 2);
-        if (!grid4) return BR_BAD_ARG;
 #define BR_PREFILL_DMA(HD_)                                                                                \
     do {                                                                                                   \
         auto kern = attn_prefill_dma_kernel<HD_>;                                                          \
@@ -1163,7 +1163,7 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
                 return BR_LAUNCH_FAILED;                                                                   \
             set = true;                                                                                    \
         }                                                                                                  \
-        kern<<<grid4, 256, lds4, s>>>((const bf16*)q, q_stride, (bf16*)out, cu_seqlens, slots, ctx_lens,  \
+        kern<<<dim3(grid4, B), 256, lds4, s>>>((const bf16*)q, q_stride, (bf16*)out, cu_seqlens, slots, ctx_lens,  \
                                       block_table, table_stride, (const bf16*)cache, nq, nkv, window,      \
                                       scale, order);                                                       \
     } while (0)

@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void pwa_prefill_dma_k
     extern __shared__ __attribute__((aligned(1024))) unsigned char pwa_lds[];
     int* list = (int*)(pwa_lds + 2 * STAGE);
     int hm, b, tile;                                         // (kv head, map), sequence, 128 rows
-    order.place(blockIdx.x, hm, b, tile);
+    order.place(hm, b, tile);
     const int kvh = hm / maps, map = hm % maps;
     const int slot = slots[b];
     const int t0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t0;
@@ -1468,7 +1468,7 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
                     return BR_LAUNCH_FAILED;                                                                                           \
                 set = true;                                                                                                            \
             }                                                                                                                          \
-            kern<<<units, 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,           \
+            kern<<<dim3(units, B), 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,           \
                                         (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, size, pool, scale, sink, sinks, order, chunk, keep, \
                                         softcap, maps);                                                                                \
             return br_check_launch();                                                                                                  \

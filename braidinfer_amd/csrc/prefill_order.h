@@ -15,7 +15,8 @@
 // 700 89 / 79.
 struct PrefillOrder {
     int heads, B, tiles, side, fold, by_tile;
-    __device__ __forceinline__ void place(int id, int& head, int& b, int& tile) const {
+    __device__ __forceinline__ void place(int& head, int& b, int& tile) const {
+        int id = blockIdx.y * gridDim.x + blockIdx.x;
         if (!side) {
             tile = tiles - 1 - id % tiles;
             id /= tiles;
@@ -35,13 +36,14 @@ struct PrefillOrder {
     }
 };
 
-// For sequences of up to `rows` rows and workgroups of which `each` fit a compute unit; the number of workgroups, 0 where that is too large.
+// For sequences of up to `rows` rows and workgroups of 256 threads, of which `each` fit a compute unit; the grid's x, 0 where the grid is too large.
+// Its y is B: workgroups are numbered along x first, and a launch's 2^32 threads hold for x alone.
 static inline unsigned prefill_order(PrefillOrder& o, long long rows, int heads, int B, int cus, int each) {
     const int side = heads % 8 == 0 ? 1 : 8 % heads == 0 ? 8 / heads : 0;
     long long tiles = (rows + 127) / 128;
     if (side) tiles = (tiles + side - 1) / side * side;
-    if (tiles > 0x7fffffffLL || tiles * B > 0x7fffffffLL || tiles * B * heads > 0x7fffffffLL) return 0;
+    if (tiles > 0xffffff || tiles * heads > 0xffffff || tiles * heads * B > 0x7fffffffLL) return 0;
     const bool resident = each == 2 && cus > 0 && tiles * B * heads <= 2LL * cus;
     o = {heads, B, (int)tiles, side, side ? (resident && cus % heads == 0 ? cus / heads : (int)(tiles * B)) : resident, B <= 16};
-    return (unsigned)(tiles * B * heads);
+    return (unsigned)(tiles * heads);
 }

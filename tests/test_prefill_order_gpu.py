@@ -60,3 +60,21 @@ def test_rows_of_the_windowed_kernel(nq, nkv, dk, dv, lens):
     together = run(0, cu[-1], list(range(len(lens))))
     for b in range(len(lens)):
         assert torch.equal(run(cu[b], cu[b + 1], [b]), together[cu[b]:cu[b + 1]]), b
+
+
+# 2^24 workgroups and more in all: a launch may have 2^32 threads along each side of its grid
+@pytest.mark.parametrize("nq,nkv,B,max_new", [(32, 8, 600, 131072), (8, 8, 2048, 131072)])
+def test_many_sequences_and_a_long_one_allowed(nq, nkv, B, max_new):
+    from braidinfer_amd import kernels as K
+    hd = 64
+    g = torch.Generator().manual_seed(B)
+    lens = [1 + b % 3 for b in range(B)]
+    cu = [0] + torch.tensor(lens).cumsum(0).tolist()
+    cache = torch.randn(B, 2, nkv, 64, hd, generator=g).bfloat16().cuda()
+    q = torch.randn(cu[-1], nq * hd, generator=g).bfloat16().cuda()
+    args = (torch.tensor(cu, **I32), torch.arange(B, **I32), torch.tensor(lens, **I32), torch.arange(B, **I32)[:, None].contiguous(), cache, B)
+    outs = []
+    for longest in (3, max_new):
+        outs.append(torch.full((cu[-1], nq * hd), 7.0, dtype=torch.bfloat16, device="cuda"))
+        K.attention_prefill_bf16(q, nq * hd, outs[-1], *args, longest, nq, nkv, hd, 64, None, hd ** -0.5)
+    assert torch.equal(outs[0], outs[1]) and torch.isfinite(outs[0].float()).all()
