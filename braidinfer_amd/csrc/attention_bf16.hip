@@ -1149,9 +1149,10 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
     // Short steps too: 16 to 64 new tokens over 1,024 to 8,192 earlier ones run 2.5 to 3 times faster through
     // LDS than with the fragments straight from the cache, which remains for head sizes beyond 192.
     PrefillOrder order;
-    const unsigned grid4 = dma_ok ? prefill_order(order, (long long)max_new * G, nkv, B, br_device_cus(), 2) : 0;
-    if (variant == 4 && !grid4) return BR_BAD_ARG;
-    if (variant == 0) variant = grid4 ? 4 : hd <= 128 ? 3 : hd <= 192 ? 2 : 1;
+    dim3 grid4;
+    const bool ordered = dma_ok && prefill_order(order, grid4, (long long)max_new * G, nkv, B, br_device_cus(), 2);
+    if (variant == 4 && !ordered) return BR_BAD_ARG;
+    if (variant == 0) variant = ordered ? 4 : hd <= 128 ? 3 : hd <= 192 ? 2 : 1;
     if (variant == 4) {
 #define BR_PREFILL_DMA(HD_)                                                                                \
     do {                                                                                                   \
@@ -1163,7 +1164,7 @@ extern "C" int br_attn_prefill_bf16(const void* q, size_t q_stride, void* out, c
                 return BR_LAUNCH_FAILED;                                                                   \
             set = true;                                                                                    \
         }                                                                                                  \
-        kern<<<dim3(grid4, B), 256, lds4, s>>>((const bf16*)q, q_stride, (bf16*)out, cu_seqlens, slots, ctx_lens,  \
+        kern<<<grid4, 256, lds4, s>>>((const bf16*)q, q_stride, (bf16*)out, cu_seqlens, slots, ctx_lens,  \
                                       block_table, table_stride, (const bf16*)cache, nq, nkv, window,      \
                                       scale, order);                                                       \
     } while (0)

@@ -1456,9 +1456,10 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
     if ((long long)grid.x * 128 >= 256 && pages <= PWA_MAX_LIST && ((uintptr_t)storage | (uintptr_t)pooled | (uintptr_t)q) % 16 == 0 &&
         (unsigned long long)nkv * PWA_PAGE * ((unsigned long long)maps * dk + dv) * 2 < (1ull << 32)) {
         PrefillOrder order;
-        const unsigned units = prefill_order(order, (long long)max_new * G, nkv * maps, B, br_device_cus(), dk + dv <= 256 ? 2 : 1);
+        dim3 units;
+        const bool ordered = prefill_order(order, units, (long long)max_new * G, nkv * maps, B, br_device_cus(), dk + dv <= 256 ? 2 : 1);
 #define PWA_DMA(DK_, DV_)                                                                                                              \
-        if (units && dk == DK_ && dv == DV_) {                                                                                         \
+        if (ordered && dk == DK_ && dv == DV_) {                                                                                       \
             auto kern = pwa_prefill_dma_kernel<DK_, DV_>;                                                                              \
             const size_t lds = (size_t)2 * PWA_PAGE * (DK_ + DV_) * 2 + (((size_t)pages + 3) & ~(size_t)3) * sizeof(int);               \
             static bool set = false;                                                                                                   \
@@ -1468,7 +1469,7 @@ extern "C" int br_pwa_prefill_bf16(const void* q, void* out, const int* cu_seqle
                     return BR_LAUNCH_FAILED;                                                                                           \
                 set = true;                                                                                                            \
             }                                                                                                                          \
-            kern<<<dim3(units, B), 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,           \
+            kern<<<units, 256, lds, s>>>((const bf16*)q, (bf16*)out, cu_seqlens, slots, ctx_lens, block_table, table_stride,           \
                                         (const bf16*)storage, pooled_table, pooled_stride, (const bf16*)pooled, nq, nkv, size, pool, scale, sink, sinks, order, chunk, keep, \
                                         softcap, maps);                                                                                \
             return br_check_launch();                                                                                                  \

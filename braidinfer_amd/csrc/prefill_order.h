@@ -10,40 +10,46 @@
 // the last on: a long and a short one share a unit.  Other numbers of heads: a kv head's tiles in a row, every second half of the heads from
 // the first tile on where all are resident (`fold` 1).  us before (a kv head's tiles in a row) and now, 32 heads of 128 over 8: 2,048
 // tokens 65.5 / 61.6, 4,096 234 / 167, 7,001 (window 4,096) 450 / 384, 16,384 2,400 / 2,330, four times 2,000 215 / 170, eight times 1,000
-// 155 / 106, 16 times 500 114 / 74, 1,357 to 93 75 / 69, 3,000 and 1,000 137 / 106 (unturned 162), 1,000 and five times 50 34.1 / 35.0, 64 times 150
+// 155 / 106, 16 times 500 114 / 74, 1,357 to 93 75 / 69, 3,000 and 1,000 137 / 106 (unturned 162), 1,000 and five times 50 34.1 / 34.9, 64 times 150
 // 60.5 / 59.3 (over all at once 66), 32 times 200 46.9 / 44.9 (50.6); 32 over 4 heads of 64, 3,000 and 1,000 90 / 71; 32 over 2, 2,000, 1,500 and
 // 700 89 / 79.
+//
+// Nothing is divided that the grid can hold: five divisions a workgroup cost short prompts 0.4 us (67 tokens 8.9 and 8.6 without, 512 20.1 and 19.6, as before the order).
 struct PrefillOrder {
-    int heads, B, tiles, side, fold, by_tile;
+    int B, tiles, total, side, shift, fold, by_tile;         // total: tiles of all sequences; side = 1 << shift, or 0
     __device__ __forceinline__ void place(int& head, int& b, int& tile) const {
-        int id = blockIdx.y * gridDim.x + blockIdx.x;
-        if (!side) {
-            tile = tiles - 1 - id % tiles;
-            id /= tiles;
-            head = id % heads;
-            b = id / heads;
-            if (fold && ((head * 2 / heads) & 1)) tile = tiles - 1 - tile;
+        if (!side) {                                         // grid (tiles, heads, B)
+            head = blockIdx.y;
+            b = blockIdx.z;
+            tile = fold && ((head * 2 / (int)gridDim.y) & 1) ? (int)blockIdx.x : tiles - 1 - (int)blockIdx.x;
             return;
         }
-        head = id % heads;
-        int u = id / heads;
-        if (u >= fold) u = fold + tiles * B - 1 - u;
-        const int lo = u % side, rows = tiles / side;
-        u /= side;
-        const int hi = by_tile ? u / B : u % rows;
-        b = by_tile ? (u + hi + __popc(hi)) % B : u / rows;
-        tile = tiles - 1 - (hi * side + lo);
+        head = blockIdx.x;                                   // grid (heads, a run of all tiles, runs)
+        int u = blockIdx.z * gridDim.y + blockIdx.y;
+        b = 0;
+        tile = tiles;                                        // none
+        if (u >= total) return;
+        if (u >= fold) u = fold + total - 1 - u;
+        if (B > 1) {
+            const int lo = u & (side - 1);
+            u >>= shift;
+            const int hi = by_tile ? u / B : u % (tiles >> shift);
+            b = by_tile ? (u + hi + __popc(hi)) % B : u / (tiles >> shift);
+            u = (hi << shift) + lo;
+        }
+        tile = tiles - 1 - u;
     }
 };
 
-// For sequences of up to `rows` rows and workgroups of 256 threads, of which `each` fit a compute unit; the grid's x, 0 where the grid is too large.
-// Its y is B: workgroups are numbered along x first, and a launch's 2^32 threads hold for x alone.
-static inline unsigned prefill_order(PrefillOrder& o, long long rows, int heads, int B, int cus, int each) {
-    const int side = heads % 8 == 0 ? 1 : 8 % heads == 0 ? 8 / heads : 0;
+// For sequences of up to `rows` rows and workgroups of which `each` fit a compute unit; false where there are too many.
+static inline bool prefill_order(PrefillOrder& o, dim3& grid, long long rows, int heads, int B, int cus, int each) {
+    const int shift = heads % 8 == 0 ? 0 : heads == 4 ? 1 : heads == 2 ? 2 : heads == 1 ? 3 : -1;
     long long tiles = (rows + 127) / 128;
-    if (side) tiles = (tiles + side - 1) / side * side;
-    if (tiles > 0xffffff || tiles * heads > 0xffffff || tiles * heads * B > 0x7fffffffLL) return 0;
+    if (shift > 0) tiles = (tiles + (1 << shift) - 1) >> shift << shift;
+    if (tiles > 0xffffff || tiles * B > 0x7fffffffLL) return false;
     const bool resident = each == 2 && cus > 0 && tiles * B * heads <= 2LL * cus;
-    o = {heads, B, (int)tiles, side, side ? (resident && cus % heads == 0 ? cus / heads : (int)(tiles * B)) : resident, B <= 16};
-    return (unsigned)(tiles * heads);
+    const int total = (int)(tiles * B), run = total < 32768 ? total : 32768;
+    o = {B, (int)tiles, total, shift < 0 ? 0 : 1 << shift, shift, shift < 0 ? resident : resident && cus % heads == 0 ? cus / heads : total, B <= 16};
+    grid = shift < 0 ? dim3((unsigned)tiles, heads, B) : dim3(heads, run, (total - 1) / run + 1);
+    return true;
 }
