@@ -3302,9 +3302,16 @@ static bool experts_tall_tiles(int pairs, int E, int N, bool gated, int cus) {
     return units >= 4.0 * cus && mean >= (gated ? 448.0 : 136.0);
 }
 
+// rows of the tiles that br_experts_tiles takes
+extern "C" int br_experts_tiles_rows(int pairs, int E, int N, int gated) {
+    return pairs > 0 && E > 0 && N > 0 && experts_tall_tiles(pairs, E, N, gated != 0, br_device_cus()) ? 256 : 128;
+}
+
+// rows: 128 or 256 a tile (tests and measurements), 0 by the rule
 extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, const int* order, void* C, int gated, int out_is_bf16,
-                                int a_rows, int pairs, int E, int N, int K, int top, float limit, float alpha, hipStream_t s) {
+                                int a_rows, int pairs, int E, int N, int K, int top, float limit, float alpha, int rows, hipStream_t s) {
     if (pairs <= 0) return BR_OK;
+    if (rows != 0 && rows != 128 && rows != 256) return BR_BAD_ARG;
     const size_t ldc = gated ? (size_t)N / 2 : (size_t)N;
     if (!br_experts_tiles_takes(N, K) || E <= 0 || top <= 0 || (gated && !out_is_bf16) || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 != 0 ||
         !quad_takes(C, order ? a_rows : min(a_rows, 256), N, K, K, ldc))
@@ -3314,7 +3321,7 @@ extern "C" int br_experts_tiles(const void* A, const void* W, const int* first, 
     const int mode = gated ? OUT_SWIGLU : out_is_bf16 ? OUT_BF16 : OUT_F32;
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    if (experts_tall_tiles(pairs, E, N, gated != 0, cus))
+    if (rows ? rows == 256 : experts_tall_tiles(pairs, E, N, gated != 0, cus))
         return launch_experts_tiles<256, 256, 2, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
     return launch_experts_tiles<128, 256, 3, 3, 2>((const bf16*)A, (const bf16*)W, C, mode, pairs, N, K, ldc, gr, s);
 }

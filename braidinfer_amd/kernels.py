@@ -1714,9 +1714,15 @@ def experts_tiles_take(dtype: torch.dtype, W: int, F: int, tokens: int) -> bool:
             and _experts_gemm_tiles_take(2 * F, W) and _experts_gemm_tiles_take(W, F))
 
 
+def experts_tiles_rows(pairs: int, E: int, N: int, gated: bool) -> int:
+    """Activation rows of the tiles by which `experts_up_tiles` (`gated`, N = 2 F) and `experts_gemm` go: 128 or 256."""
+    return _fn("gemm_bf16", "br_experts_tiles_rows", [c_int] * 4)(pairs, E, N, int(gated))
+
+
 def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, order: torch.Tensor, y: torch.Tensor, top: int,
-                     limit: float = 0.0, alpha: float = 0.0) -> None:
-    """`experts_up_grouped` by the tiles of the prompt products, for steps of more tokens."""
+                     limit: float = 0.0, alpha: float = 0.0, rows: int = 0) -> None:
+    """`experts_up_grouped` by the tiles of the prompt products, for steps of more tokens.  `rows`: 128 or 256 a tile (tests and
+    measurements), 0 by `experts_tiles_rows`."""
     _dev("experts_up_tiles", h, w_gu, first, order, y)
     T, W = h.shape
     E, F2, _ = w_gu.shape
@@ -1725,22 +1731,22 @@ def experts_up_tiles(h: torch.Tensor, w_gu: torch.Tensor, first: torch.Tensor, o
          "experts_up_tiles: bfloat16, widths in steps of 64, rows below 4 GB")
     _req(w_gu.shape == (E, F2, W) and y.shape == (n, F2 // 2) and first.numel() in (E + 1, E + 2) and n == T * top
          and first.dtype == order.dtype == torch.int32, "experts_up_tiles: shapes")
-    f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
-    _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), 1, 1, T, n, E, F2, W, top, float(limit), float(alpha), _stream()),
+    f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, c_int, _P])
+    _check(f(_ptr(h), _ptr(w_gu), _ptr(first), _ptr(order), _ptr(y), 1, 1, T, n, E, F2, W, top, float(limit), float(alpha), rows, _stream()),
            "experts_up_tiles")
 
 
-def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: torch.Tensor) -> None:
+def experts_gemm(a: torch.Tensor, w: torch.Tensor, first: torch.Tensor, out: torch.Tensor, rows: int = 0) -> None:
     """out[p] = w[e] a[p] for the pairs p of every expert e in the experts' order (`experts_sort`): a [pairs, K] bfloat16
-    rows in that order, w [E, N, K] bfloat16, out [pairs, N] bfloat16 or float32; one launch for all experts."""
+    rows in that order, w [E, N, K] bfloat16, out [pairs, N] bfloat16 or float32; one launch for all experts.  `rows`: as for `experts_up_tiles`."""
     _dev("experts_gemm", a, w, first, out)
     n, Kd = a.shape
     E, N, _ = w.shape
     _req(a.dtype == w.dtype == torch.bfloat16 and Kd % 8 == 0 and w.shape == (E, N, Kd) and out.shape == (n, N)
          and first.dtype == torch.int32 and first.numel() in (E + 1, E + 2), "experts_gemm: bfloat16 [pairs, K] x [E, N, K], K in steps of 8")
     if _experts_gemm_tiles_take(N, Kd) and out.data_ptr() % 16 == 0:
-        f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, _P])
-        _check(f(_ptr(a), _ptr(w), _ptr(first), None, _ptr(out), 0, _is_bf16(out, "experts_gemm"), n, n, E, N, Kd, 1, 0.0, 0.0, _stream()),
+        f = _fn("gemm_bf16", "br_experts_tiles", [_P] * 5 + [c_int] * 8 + [c_float, c_float, c_int, _P])
+        _check(f(_ptr(a), _ptr(w), _ptr(first), None, _ptr(out), 0, _is_bf16(out, "experts_gemm"), n, n, E, N, Kd, 1, 0.0, 0.0, rows, _stream()),
                "experts_gemm")
         return
     f = _fn("routed_experts", "br_experts_gemm", [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P])
