@@ -3287,19 +3287,35 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
     return br_check_launch();
 }
 
-// 128x256 or 256x256 tiles, by the pairs an expert on average (their real numbers stay on the device) and the rounds of workgroups that
-// tiles of 128 rows make.  A tile multiplies only the blocks of 64 rows that it has, so what is counted against the taller tile is the
-// experts with few pairs, whose weights it streams by fewer workgroups.  32 experts of 1,792 by 4,096, us with 128 rows a tile against
-// 256, rows an expert uneven as random weights draw them (half to twice the mean):
-//   gated product: 112 pairs on average 226 / 208, 150 225 / 243 (another draw 230 / 286), 225 323 / 345, 300 343 / 341, 450 480 / 483, 603
-//     615 / 567, 675 680 / 652;  equal rows: 128 192 / 198, 160 257 / 226, 200 279 / 252, 256 294 / 261, 300 364 / 427, 400 440 / 443
-//   down (short k, float rows): 112 132 / 139, 150 155 / 153, 225 184 / 168, 300 215 / 203, 450 290 / 273, 603 363 / 327, 675 412 / 375;
-//     equal rows: 128 117 / 118, 160 151 / 125, 256 170 / 149, 300 207 / 213, 400 264 / 238
-// With fewer than four rounds too few workgroups are left: 16 experts of 1,408 by 2,048, 4 chosen, down: 600 tokens 33 / 43, 2,400 tokens
-// 74 / 82, but 5,000 tokens 148 / 133.
+// 128x256 or 256x256 tiles, for rows an expert of which the host knows the mean only.
+// Gated product: the fewer rounds of workgroups by the times a k-tile of `choose_quad`, with every expert's pairs taken as the mean and half a
+// standard deviation of evenly drawn ones, rounded up to tiles; from eight rounds of 128-row tiles on the taller one may be counted a fifth
+// longer, since a tile multiplies only the blocks of 64 rows that it has and there is no round of few tiles to wait for.  us with 128 rows a tile
+// against 256, equal rows an expert / rows that random weights draw (half to twice the mean; two draws):
+//   32 experts of 1,792 by 4,096: 64 pairs an expert 173, 176 / 183, 179; 179, 183.  112: 186, 192 / 211, 194; 209, 216.  160: 248, 213 / 247, 262; 249, 262.
+//     200: 283, 242 / 265, 284; 268, 278.  256 (128 rows taken): 287, 242 / 320, 308; 324, 303.  300: 355, 405 / 352, 368; 345, 344.  350: 390, 405 / 388,
+//     393; 383, 392.  400: 412, 419 / 437, 406; 445, 404.  450: 456, 439 / 483, 435; 471, 479.  512: 476, 449 / 524, 507; 516, 499.  603: 585, 556 / 598, 582; 604,
+//     568.  900: 827, 758 / 854, 820; 863, 770.  1,800: 1,637, 1,474 / 1,654, 1,483; 1,640, 1,476
+//   16 experts of 1,408 by 2,048: 96: 39, 40 / 39, 55; 50, 53.  136: 66, 45 / 61, 59; 65, 57.  225: 64, 59 / 65, 89; 64, 61.  300: 80, 111 / 78, 110; 96, 109.  450: 103,
+//     117 / 102, 118; 103, 120.  550 (128 rows taken): 124, 121 / 133, 121; 134, 123.  675: 164, 157 / 162, 173; 162, 173.  900: 204, 190 / 195, 184; 201, 186
+// Over 24 means from 64 to 1,800, these two shapes and equal, mildly and clearly uneven rows the choice takes 1.6 % longer than the faster height each
+// time; a line at 448 pairs took 3.5, always 128 rows 5.0.
+// Down product (short k, float rows): the taller tile from four rounds of 128-row tiles on, where an expert has more rows than such a tile.  Same
+// shapes: 32 experts 128 pairs 116, 116 / 134, 131; 128, 135, 150: 148, 122 / 153, 138; 153, 143, 300: 205, 208 / 212, 203; 208, 193, 603: 345, 313 / 364, 319; 369,
+// 330, 1,800: 951, 837 / 1,036, 852; 1,009, 861.  16 experts, fewer rounds up to 896 pairs: 160: 26, 30 / 26, 36; 25, 35, 300: 43, 42 / 44, 40; 44, 41, 450: 52, 48 /
+// 66, 75; 66, 77, 603: 71, 78 / 70, 77; 70, 78; 900: 98, 91 / 110, 101; 96, 101, 1,200: 138, 126 / 145, 129; 153, 125.
 static bool experts_tall_tiles(int pairs, int E, int N, bool gated, int cus) {
-    const double mean = (double)pairs / E, units = E * ceil(mean / 128) * ((N + 255) / 256);
-    return units >= 4.0 * cus && mean >= (gated ? 448.0 : 136.0);
+    const double mean = (double)pairs / E, high = mean + (gated ? 0.5 * sqrt(mean) : 0.0);
+    const int cols = (N + 255) / 256;
+    double t[2], rounds[2];
+    for (int i = 0; i < 2; ++i) {
+        const int bm = i ? 256 : 128, k = i ? 0 : 1;
+        rounds[i] = E * ceil(high / bm) * cols / cus;
+        const double whole = floor(rounds[i]), share = rounds[i] - whole;
+        t[i] = (whole + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) : 0.0)) * QUAD_FULL[k];
+    }
+    if (!gated) return mean > 128 && rounds[0] >= 4.0;
+    return t[1] <= (rounds[0] >= 8.0 ? 1.2 : 1.03) * t[0];
 }
 
 // rows of the tiles that br_experts_tiles takes
