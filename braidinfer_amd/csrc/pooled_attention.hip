@@ -620,31 +620,14 @@ __device__ __forceinline__ bf16x8 pwa_zero8() {
     for (int i = 0; i < 8; ++i) z[i] = (bf16)0.f;
     return z;
 }
-// 8 values V^T[channel][k .. k+7] of a page; rows at or beyond `limit` (not written yet) read as zero
-__device__ __forceinline__ bf16x8 pwa_load_vt8(const bf16* __restrict__ vrow, int k, int limit) {
-    bf16x8 v = *(const bf16x8*)(vrow + k);
-    if (k + 8 > limit) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) if (k + i >= limit) v[i] = (bf16)0.f;
-    }
-    return v;
-}
 // Row c (0..31) of a score block stands for this key of the block; lane (column, g) then holds in
 // acc[r] the key 16 (r / 8) + 8 g + r % 8.
 __device__ __forceinline__ int pwa_key_of_row(int c) { return 16 * (c >> 4) + 8 * ((c >> 2) & 1) + 4 * ((c >> 3) & 1) + (c & 3); }
 
-// One block of 32 keys (rows kb .. kb + 31 of a unit): `key(s)` gives this lane's 8 elements s * 16 + 8 g .. of its key row, `value(i, h)` 8
-// values of channel 32 i + c at the rows 16 h + 8 g .. of the block; `between` runs behind the scores' products.  A key is seen
-// by this lane's query if first_ok <= key <= last_ok.
-template <int NBK, int NBV, class Key, class Value, class Between>
-__device__ __forceinline__ void pwa_block_of(Key key, Value value, Between between, int kb, int first_ok, int last_ok, int g, const bf16x8* qf,
-                                             f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
-    f32x16 s_acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 2 * NBK; ++s) s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(key(s), qf[s], s_acc, 0, 0, 0);
-    between();
+// A block's scores s_acc (32 keys from kb on, of which this lane's query sees first_ok <= key <= last_ok) become the weights p1, p2 of its
+// values; `m` and `lsum` go on.  True where some lane's maximum moved: the sums so far are to be scaled by `corr`.
+__device__ __forceinline__ bool pwa_weights(f32x16& s_acc, int kb, int first_ok, int last_ok, int g, float& m, float& lsum, float scale2, float cap_in,
+                                            float cap_out, bf16x8& p1, bf16x8& p2, float& corr) {
     if (cap_out != 0.f) {
         // bounded scores: cap tanh(s scale / cap), tanh z = 1 - 2 / (exp(2 z) + 1); cap_in = 2 log2(e) scale / cap and
         // cap_out = cap / scale, so that the multiplication by scale2 below leaves the bounded score in base 2
@@ -670,9 +653,8 @@ __device__ __forceinline__ void pwa_block_of(Key key, Value value, Between betwe
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float m_new = fmaxf(m, mx);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float corr = __builtin_amdgcn_exp2f(m - m_use);
+    corr = __builtin_amdgcn_exp2f(m - m_use);
     float psum = 0.f;
-    bf16x8 p1, p2;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const float p = __builtin_amdgcn_exp2f(sv[r] - m_use);
@@ -680,27 +662,18 @@ __device__ __forceinline__ void pwa_block_of(Key key, Value value, Between betwe
         if (r < 8) p1[r] = (bf16)p; else p2[r - 8] = (bf16)p;
     }
     lsum = lsum * corr + psum;
-    // the sums so far are scaled only when some lane's maximum moved
     const bool moved = __any(m_new != m);
     m = m_new;
-    if (moved) {
-#pragma unroll
-        for (int i = 0; i < NBV; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc_o[i][r] *= corr;
-    }
-#pragma unroll
-    for (int i = 0; i < NBV; ++i) {
-        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 0), p1, acc_o[i], 0, 0, 0);
-        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 1), p2, acc_o[i], 0, 0, 0);
-    }
+    return moved;
 }
 
-// The same with `kblock` the block's first key row (rows `ks` elements apart) and `vblock` the first value channel at the block's first row
-// (channels `vs` elements apart), in the cache or in LDS; rows of the block from `limit` on are not written and their values
-// read as zero.  EARLY: all of the block's keys and values are asked for before the
-// first product, without a branch between them (channels from dv on read the last row, and nobody writes what becomes of it;
-// a key row's elements from dk on, at most 127, are the next row's or the values' that follow the keys in a page, not used).
+// One block of 32 keys (rows kb .. kb + 31 of a unit): `kblock` is the block's first key row (rows `ks` elements
+// apart), `vblock` the first value channel at the block's first row (channels `vs` elements apart), in the cache
+// or in LDS; rows of the block from `limit` on are not written and their values read as zero.  A key is seen by
+// this lane's query if first_ok <= key <= last_ok.  Channels from dv on read the last row, and nobody writes what becomes of it.  (No
+// branch here parts a wave's lanes between its products: with values read behind one of a lane's own, the form for keys of 192 and
+// values of 160 elements, which has no registers left, lost the zeroes.)  EARLY: all of the block's keys and values are asked for
+// before the first product (a key row's elements from dk on, at most 127, are the next row's or the values' that follow the keys in a page, not used).
 template <int NBK, int NBV, bool EARLY = false>
 __device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int ks, const bf16* __restrict__ vblock, int vs,
                                           int kb, int limit, int first_ok, int last_ok, int dk, int dv, int c, int g,
@@ -716,26 +689,73 @@ __device__ __forceinline__ void pwa_block(const bf16* __restrict__ kblock, int k
             ve[i] = *(const bf16x8*)(vblock + (unsigned)(min(i / 2 * 32 + c, dv - 1) * vs + 8 * g) + (i & 1) * 16);
         __builtin_amdgcn_sched_barrier(0);
     }
-    auto key = [&](int s) {
-        const int d = s * 16 + 8 * g;
-        if constexpr (EARLY) return d < dk ? ke[s] : pwa_zero8();
-        else return (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
-    };
-    auto value = [&](int i, int h) {
-        const int ch = i * 32 + c;
-        if constexpr (EARLY) {
-            bf16x8 v = ve[2 * i + h];
-            if (limit < 32) {                             // uniform
+    f32x16 s_acc;
 #pragma unroll
-                for (int x = 0; x < 8; ++x)
-                    if (16 * h + 8 * g + x >= limit) v[x] = (bf16)0.f;
-            }
-            return v;
-        } else {
-            return ch < dv ? pwa_load_vt8(vblock + (size_t)ch * vs, 16 * h + 8 * g, limit) : pwa_zero8();
+    for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2 * NBK; ++s) {
+        const int d = s * 16 + 8 * g;
+        bf16x8 kf;
+        if constexpr (EARLY) kf = d < dk ? ke[s] : pwa_zero8();
+        else kf = (d < dk) ? *(const bf16x8*)(krow + d) : pwa_zero8();
+        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], s_acc, 0, 0, 0);
+    }
+    bf16x8 p1, p2;
+    float corr;
+    const bool moved = pwa_weights(s_acc, kb, first_ok, last_ok, g, m, lsum, scale2, cap_in, cap_out, p1, p2, corr);
+    // Each group of values is asked for behind the scaling of its sums: pages that go through registers or come from the cache leave no
+    // registers for more (with all sums scaled first, 16 tokens behind 500: 32 heads of 128 39 -> 43 us, 16 of 128 / 256 63 -> 71).
+#pragma unroll
+    for (int i = 0; i < NBV; ++i) {
+        if (moved) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc_o[i][r] *= corr;
         }
-    };
-    pwa_block_of<NBK, NBV>(key, value, [] {}, kb, first_ok, last_ok, g, qf, acc_o, m, lsum, scale2, cap_in, cap_out);
+        bf16x8 v1, v2;
+        if constexpr (EARLY) {
+            v1 = ve[2 * i];
+            v2 = ve[2 * i + 1];
+        } else {
+            const bf16* vrow = vblock + (unsigned)(min(i * 32 + c, dv - 1) * vs + 8 * g);
+            v1 = *(const bf16x8*)vrow;
+            v2 = *(const bf16x8*)(vrow + 16);
+        }
+        if (limit < 32) {                                 // uniform
+#pragma unroll
+            for (int x = 0; x < 8; ++x) {
+                if (8 * g + x >= limit) v1[x] = (bf16)0.f;
+                if (16 + 8 * g + x >= limit) v2[x] = (bf16)0.f;
+            }
+        }
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p1, acc_o[i], 0, 0, 0);
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p2, acc_o[i], 0, 0, 0);
+    }
+}
+
+// The same with `key(s)` this lane's 8 elements s * 16 + 8 g .. of its key row and `value(i, h)` 8 values of channel 32 i + c at the rows 16 h + 8 g .. of
+// the block; `between` runs behind the scores' products.  One test for sums to scale, in front of all products with the values.
+template <int NBK, int NBV, class Key, class Value, class Between>
+__device__ __forceinline__ void pwa_block_of(Key key, Value value, Between between, int kb, int first_ok, int last_ok, int g, const bf16x8* qf,
+                                             f32x16* acc_o, float& m, float& lsum, float scale2, float cap_in, float cap_out) {
+    f32x16 s_acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2 * NBK; ++s) s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(key(s), qf[s], s_acc, 0, 0, 0);
+    between();
+    bf16x8 p1, p2;
+    float corr;
+    if (pwa_weights(s_acc, kb, first_ok, last_ok, g, m, lsum, scale2, cap_in, cap_out, p1, p2, corr)) {
+#pragma unroll
+        for (int i = 0; i < NBV; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc_o[i][r] *= corr;
+    }
+#pragma unroll
+    for (int i = 0; i < NBV; ++i) {
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 0), p1, acc_o[i], 0, 0, 0);
+        acc_o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(i, 1), p2, acc_o[i], 0, 0, 0);
+    }
 }
 
 // Which tile of 128 rows a workgroup takes: the last tiles (most keys) first, so that the long workgroups start
