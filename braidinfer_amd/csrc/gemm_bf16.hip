@@ -514,9 +514,17 @@ struct QuadBranches {
     int per;
     size_t a_step;
     int gap_at, gap;
+    int whole;
+};
+// `whole`: the last tile of rows multiplies all of its blocks, also those without rows.  For products of one round of workgroups: what it saves
+// ends no round earlier, and tiles that run ahead of the others read the weights from farther off than the L2 (gated 28,672 x 4,096 by
+// 129 / 150 / 192 rows 65 / 60 / 55 us with its rows alone, 57 / 52 / 53 whole; 4,096 x 14,336 by 900 106 and 101).
+struct QuadPlain {
+    int whole;
 };
 enum { QUAD_PLAIN = 0, QUAD_EXPERTS = 1, QUAD_BRANCHES = 2 };
-template <int KIND> struct QuadArg { typedef QuadGroups type; };
+template <int KIND> struct QuadArg { typedef QuadPlain type; };
+template <> struct QuadArg<QUAD_EXPERTS> { typedef QuadGroups type; };
 template <> struct QuadArg<QUAD_BRANCHES> { typedef QuadBranches type; };
 __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr) {
     if (gr.alpha > 0.f) {
@@ -870,7 +878,10 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         for (; t + 1 < nk; ++t) step(F{}, F{});
         step(F{}, T{});
     };
-    const int blocks = (m_end - m0 + 32 * WVM - 1) / (32 * WVM);       // of 32 rows a wave
+    int blocks = (m_end - m0 + 32 * WVM - 1) / (32 * WVM);             // of 32 rows a wave
+    if constexpr (!GROUPED) {
+        if (gr.whole) blocks = TJ;
+    }
     if (blocks >= TJ) run(std::integral_constant<int, TJ>{});
     else if (TJ > 3 && blocks == 3) run(std::integral_constant<int, (TJ > 3 ? 3 : 1)>{});
     else if (TJ > 2 && blocks == 2) run(std::integral_constant<int, (TJ > 2 ? 2 : 1)>{});
@@ -1032,8 +1043,9 @@ static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N,
         kpp += kpp & 1;
         parts = (nk + kpp - 1) / kpp;                                 // no empty run
         dim3 grid((unsigned)total, (unsigned)parts);
+        const QuadPlain whole = {total * parts <= br_device_cus()};
         gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<grid, 256, 0, s>>>(A, W, scratch, M, N, K, lda, (size_t)N, tm, tn, kpp,
-                                                                        (size_t)M * N, wl, QuadGroups{});
+                                                                        (size_t)M * N, wl, whole);
         int rc = br_check_launch();
         if (rc != BR_OK) return rc;
         if (leave) {                                                  // the runs' sums are the caller's
@@ -1043,14 +1055,15 @@ static int launch_tile_quad(const bf16* A, const bf16* W, void* C, int M, int N,
         return launch_split_sum(scratch, parts, C, M, N, ldc, mode, s);
     }
     if (leave) return BR_BAD_ARG;
+    const QuadPlain whole = {total <= br_device_cus()};
     if (mode == OUT_BF16)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_BF16><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_BF16><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, whole);
     else if (mode == OUT_F32)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, whole);
     else if (mode == OUT_F32_ACC)
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32_ACC><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_F32_ACC><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, whole);
     else
-        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_SWIGLU><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, QuadGroups{});
+        gemm_tile_quad_kernel<BM, BN, NSA, NSB, WVM, OUT_SWIGLU><<<(unsigned)total, 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, nk, 0, wl, whole);
     return br_check_launch();
 }
 
@@ -3137,9 +3150,10 @@ extern "C" int br_gemm_bf16_branches_pay(int M, int branches, int per, int K, si
 }
 
 template <int BM, int NSA, int NSB>
-static int launch_branches_tiles(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, const QuadBranches& br, int run, hipStream_t s) {
+static int launch_branches_tiles(const bf16* A, const bf16* W, float* C, int M, int N, int K, size_t lda, size_t ldc, QuadBranches br, int run, hipStream_t s) {
     const int tm = (M + BM - 1) / BM, tn = N / 256;
     if ((long long)tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
+    br.whole = (long long)tm * tn <= br_device_cus();
     gemm_tile_quad_kernel<BM, 256, NSA, NSB, 2, OUT_F32, QUAD_BRANCHES><<<(unsigned)(tm * tn), 256, 0, s>>>(A, W, C, M, N, K, lda, ldc, tm, tn, run, 0, WL_ROWS, br);
     return br_check_launch();
 }
@@ -3154,7 +3168,7 @@ extern "C" int br_gemm_bf16_branches(const void* A_, const void* W_, float* C, i
         if (tail_rows || lda < (size_t)K || lda % 8 || a_step % 8 || gap < 0 || gap % 4 || gap_at < 0 || gap_at % per || ldc < (size_t)branches * per + gap ||
             ((uintptr_t)A | (uintptr_t)W) % 16 || !quad_takes(C, M, branches * per, K, lda, ldc))
             return BR_BAD_ARG;
-        const QuadBranches br = {per, a_step, gap_at, gap};
+        const QuadBranches br = {per, a_step, gap_at, gap, 0};
         return kind == 12 ? launch_branches_tiles<256, QUAD12>(A, W, C, M, branches * per, K, lda, ldc, br, run, s)
                           : launch_branches_tiles<128, QUAD13>(A, W, C, M, branches * per, K, lda, ldc, br, run, s);
     }
