@@ -536,7 +536,7 @@ __device__ __forceinline__ float quad_glu(float g, float u, const QuadGroups& gr
 }
 
 // acc[i][j][r]: weight row (output column) n1 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, activation
-// row m1 + 32 WVM j + lane % 32.  Needs ldc % 4 == 0 and C aligned to 16 bytes.
+// row m1 + 32 ST j + lane % 32.  Needs ldc % 4 == 0 and C aligned to 16 bytes.
 // What is only written goes through the wave's piece of LDS, 32 rows at a time, so that an instruction writes whole runs of rows: as
 // the blocks lie, it would write 16 or 32 bytes of each of 32 rows, and 256 workgroups that end a round together wait for the L2's
 // requests.  8,192 x 8,192 by K = 1,024 in bfloat16 153 -> 130 us; 6,144 x 4,096 by 3,625 rows 155.5 -> 150, by 7,001 rows 282 -> 272; float
@@ -550,7 +550,7 @@ struct QuadStrip {
     static constexpr int LD = RB + 16;                                                   // from row to row, off the banks' stride
     static constexpr int BYTES = MODE == OUT_F32_ACC ? 0 : 32 * LD;
 };
-template <int TI, int TJ, int WVM, int MODE, bool GROUPED, class Arg>
+template <int TI, int TJ, int ST, int MODE, bool GROUPED, class Arg>
 __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __restrict__ C, int M, int N, size_t ldc, int m1, int n1, int lane,
                                               const Arg& gr, unsigned char* lds) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -558,7 +558,7 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
     if constexpr (MODE == OUT_F32_ACC) {
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
-            const int m = m1 + j * 32 * WVM + (lane & 31);
+            const int m = m1 + j * 32 * ST + (lane & 31);
             if (m >= M) continue;
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
@@ -595,7 +595,7 @@ __device__ __forceinline__ void quad_epilogue(f32x16 (&acc)[TI][TJ], void* __res
         unsigned char* const put = lds + (lane & 31) * S::LD + 4 * (lane >> 5) * S::ES;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
-            const int mj = m1 + j * 32 * WVM;
+            const int mj = m1 + j * 32 * ST;
             if (mj >= M) break;
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
@@ -679,7 +679,11 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     void* C = MODE == OUT_F32 ? (void*)((float*)C_ + blockIdx.y * part_stride) : C_;
     const int kt0 = (int)blockIdx.y * kt_per_part;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = (wave / WVN) * 32, wn = (wave % WVN) * (BN / WVN);   // a wave's blocks of activation rows lie 32 WVM apart
+    // A wave's blocks of activation rows lie 32 ST apart: side by side where the product is added to what is there (a wave then reads and writes neighbouring
+    // rows: 4,096 x 1,792 by 5,018 rows 89 us, 96 with the waves' blocks in turn), else the waves' blocks in turn, so that a last tile of few rows leaves
+    // every wave as many.
+    constexpr int ST = MODE == OUT_F32_ACC ? 1 : WVM;
+    const int wm = (wave / WVN) * (ST == 1 ? BM / WVM : 32), wn = (wave % WVN) * (BN / WVN);
     const int lrow = lane & 31, g = lane >> 5;
     int nk = K / DMA_BK - kt0;                                         // k-tiles of this run
     if (nk > kt_per_part) nk = kt_per_part;
@@ -803,7 +807,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
                 constexpr int R0 = NM >= NR ? (n < NR ? n : NR) : n * NR / NM, R1 = NM >= NR ? (n < NR ? n + 1 : NR) : (n + 1) * NR / NM;
                 static_for<R0, R1>([&](auto r_) {
                     constexpr int r = decltype(r_)::value;
-                    if constexpr (RD && r < TV) quad_read<r * WVM * 4096>(fa[use ^ 1][r], ra[rk]);
+                    if constexpr (RD && r < TV) quad_read<r * ST * 4096>(fa[use ^ 1][r], ra[rk]);
                     if constexpr (RD && r >= TV) quad_read<(r - TV) * 4096>(fb[use ^ 1][r - TV], rb[rk]);
                 });
                 static_for<E0 + n * (E1 - E0) / NM, E0 + (n + 1) * (E1 - E0) / NM>(early);
@@ -863,7 +867,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
         asm volatile("" ::: "memory");
         static_for<0, TV>([&](auto n_) {
             constexpr int n = decltype(n_)::value;
-            quad_read<n * WVM * 4096>(fa[0][n], ra[0]);
+            quad_read<n * ST * 4096>(fa[0][n], ra[0]);
         });
         static_for<0, TI>([&](auto n_) {
             constexpr int n = decltype(n_)::value;
@@ -882,7 +886,7 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     if constexpr (!GROUPED) {
         if (gr.whole) blocks = TJ;
     }
-    if (blocks >= TJ) run(std::integral_constant<int, TJ>{});
+    if (ST == 1 || blocks >= TJ) run(std::integral_constant<int, TJ>{});
     else if (TJ > 3 && blocks == 3) run(std::integral_constant<int, (TJ > 3 ? 3 : 1)>{});
     else if (TJ > 2 && blocks == 2) run(std::integral_constant<int, (TJ > 2 ? 2 : 1)>{});
     else run(std::integral_constant<int, 1>{});
@@ -890,8 +894,10 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     // accumulator stay behind the statement that names it
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     static_for<0, TI * TJ>([&](auto n_) { quad_touch(acc[decltype(n_)::value / TJ][decltype(n_)::value % TJ]); });
-    __builtin_amdgcn_s_barrier();                                      // every wave has read its last operands
-    asm volatile("" ::: "memory");
+    if (MODE != OUT_F32_ACC) {                                         // (which leaves LDS alone)
+        __builtin_amdgcn_s_barrier();                                  // every wave has read its last operands
+        asm volatile("" ::: "memory");
+    }
     if constexpr (!RUNS) {
         break;
     } else {
@@ -907,8 +913,8 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
     }
     }
     unsigned char* const strip = st + wave * QuadStrip<TI, MODE>::BYTES;
-    if constexpr (RUNS) quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(sum, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
-    else quad_epilogue<TI, TJ, WVM, MODE, GROUPED>(acc, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
+    if constexpr (RUNS) quad_epilogue<TI, TJ, ST, MODE, GROUPED>(sum, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
+    else quad_epilogue<TI, TJ, ST, MODE, GROUPED>(acc, C, m_end, N, ldc, m0 + wm, n0 + wn, lane, gr, strip);
     };
 
     if constexpr (!GROUPED) {
