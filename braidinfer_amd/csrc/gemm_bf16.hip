@@ -934,84 +934,51 @@ __global__ __launch_bounds__(256) void gemm_tile_quad_kernel(const bf16* __restr
             tile(A, W, tile_m * BM, tile_n * BN, M);
         }
     } else {
-        // Expert by expert, column of tiles by column, an expert's row tiles of the same weights in turn.  The columns are cut into
-        // eight runs of about equal cost, one to an XCD, whose workgroups take its tiles in turn.  (What a tile of few rows costs is its
-        // weights: shares of a whole tile's time.)
-        auto tile_cost = [](int rows) {
-            const int b = (rows + 32 * WVM - 1) / (32 * WVM);
-            return TJ != 4 ? 1 : b == 4 ? 15 : b == 3 ? 12 : b == 2 ? 10 : 9;
-        };
-        // this lane's expert of a block of 64: its pairs, tiles of one column and their cost, and those before it in the block
-        struct Lane { int a, b, nt, cost, nt0, cost0; };
-        auto wave_scan = [](int v) {                                   // v of this lane and all before
-            v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);            // row_shr 1, 2, 4, 8
-            v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-            v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-            v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-            v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);            // row_bcast 15, 31
-            v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-            return v;
-        };
+        // Expert by expert, column of tiles by column, an expert's row tiles of the same weights in turn; eight runs of as many tiles, one to an
+        // XCD.  (Runs of columns of about equal cost, by what a tile of few rows costs beside a whole one, left some XCDs a round more than the
+        // others: 32 experts of 1,792 by 4,096, 450 rows on average, gated 485 us against 446; 8 experts of 2,048 by 1,024, 400 rows, 73 against 43.)
+        // this lane's expert of a block of 64: its pairs, its tiles of one column and those before them in the block
+        struct Lane { int a, b, nt, nt0; };
         auto lane_of = [&](int e0) {
             Lane v;
             const int e = e0 + lane;
             v.a = e < gr.experts ? gr.first[e] : 0;
             v.b = e < gr.experts ? gr.first[e + 1] : 0;
-            const int rows = v.b - v.a, rem = rows % BM;
-            v.nt = (rows + BM - 1) / BM;
-            v.cost = rows / BM * tile_cost(BM) + (rem ? tile_cost(rem) : 0);
-            v.nt0 = wave_scan(v.nt) - v.nt;
-            v.cost0 = wave_scan(v.cost) - v.cost;
+            v.nt = (v.b - v.a + BM - 1) / BM;
+            int sum = v.nt;                                            // of this lane and all before
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x111, 0xf, 0xf, false);        // row_shr 1, 2, 4, 8
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x112, 0xf, 0xf, false);
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x114, 0xf, 0xf, false);
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x118, 0xf, 0xf, false);
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x142, 0xa, 0xf, false);        // row_bcast 15, 31
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x143, 0xc, 0xf, false);
+            v.nt0 = sum - v.nt;
             return v;
         };
-        auto last_lane = [](int v) { return __builtin_amdgcn_readlane(v, 63); };
+        auto tiles_of = [](const Lane& v) { return __builtin_amdgcn_readlane(v.nt0 + v.nt, 63); };
         Lane v = lane_of(0);
-        int cost = last_lane(v.cost0 + v.cost);
-        for (int e0 = 64; e0 < gr.experts; e0 += 64) {
-            const Lane u = lane_of(e0);
-            cost += last_lane(u.cost0 + u.cost);
-        }
-        // the tiles in front of the first column that starts at `at` or more of the cost of all columns
-        const int xcd = blockIdx.x % 8;
-        const long long whole = (long long)cost * tiles_n;
-        long long at[2] = {whole * xcd / 8, whole * (xcd + 1) / 8};
-        int edge[2] = {0, 0};
-        for (int e0 = 0, nt0 = 0, cost0 = 0; e0 < gr.experts; e0 += 64) {
+        long long total = tiles_of(v);
+        for (int e0 = 64; e0 < gr.experts; e0 += 64) total += tiles_of(lane_of(e0));
+        total *= tiles_n;
+        const int xcd = blockIdx.x % 8, job = (int)(total * xcd / 8) + (int)(blockIdx.x / 8);
+        if (job >= (int)(total * (xcd + 1) / 8)) return;               // the grid is a bound
+        int e = 0, p0 = 0, end = 0, nt = 1, before = 0;
+        for (int e0 = 0, nt0 = 0; e0 < gr.experts; e0 += 64) {
             if (e0) v = lane_of(e0);
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                const long long d = at[x] - (long long)(cost0 + v.cost0) * tiles_n;     // of the cost, behind this expert's start
-                const unsigned long long behind = __ballot(d > 0 && v.cost > 0);
-                if (behind) {
-                    const int l = 63 - __clzll(behind), c = __builtin_amdgcn_readlane(v.cost, l);
-                    const long long dl = at[x] - (long long)(cost0 + __builtin_amdgcn_readlane(v.cost0, l)) * tiles_n;
-                    const int cols = dl >= (long long)c * tiles_n ? tiles_n : (int)(((unsigned)dl + c - 1) / (unsigned)c);
-                    edge[x] = (nt0 + __builtin_amdgcn_readlane(v.nt0, l)) * tiles_n + cols * __builtin_amdgcn_readlane(v.nt, l);
-                }
+            const unsigned long long here = __ballot((nt0 + v.nt0) * tiles_n <= job && job < (nt0 + v.nt0 + v.nt) * tiles_n);
+            if (here) {
+                const int l = __ffsll(here) - 1;
+                e = e0 + l;
+                p0 = __builtin_amdgcn_readlane(v.a, l);
+                end = __builtin_amdgcn_readlane(v.b, l);
+                nt = __builtin_amdgcn_readlane(v.nt, l);
+                before = (nt0 + __builtin_amdgcn_readlane(v.nt0, l)) * tiles_n;
+                break;
             }
-            nt0 += last_lane(v.nt0 + v.nt);
-            cost0 += last_lane(v.cost0 + v.cost);
+            nt0 += tiles_of(v);
         }
-        for (int job = edge[0] + (int)(blockIdx.x / 8); job < edge[1]; job += (int)(gridDim.x / 8)) {
-            int e = 0, p0 = 0, end = 0, nt = 1, before = 0;
-            for (int e0 = 0, nt0 = 0; e0 < gr.experts; e0 += 64) {
-                if (gr.experts > 64) v = lane_of(e0);
-                const unsigned long long here = __ballot((nt0 + v.nt0) * tiles_n <= job && job < (nt0 + v.nt0 + v.nt) * tiles_n);
-                if (here) {
-                    const int l = __ffsll(here) - 1;
-                    e = e0 + l;
-                    p0 = __builtin_amdgcn_readlane(v.a, l);
-                    end = __builtin_amdgcn_readlane(v.b, l);
-                    nt = __builtin_amdgcn_readlane(v.nt, l);
-                    before = (nt0 + __builtin_amdgcn_readlane(v.nt0, l)) * tiles_n;
-                    break;
-                }
-                nt0 += last_lane(v.nt0 + v.nt);
-            }
-            const int in = job - before;
-            tile(A, W + (size_t)e * N * K, p0 + in % nt * BM, in / nt * BN, end);
-            __builtin_amdgcn_s_barrier();                              // the strips have been read, the stages may be filled again
-        }
+        const int in = job - before;
+        tile(A, W + (size_t)e * N * K, p0 + in % nt * BM, in / nt * BN, end);
     }
 }
 
