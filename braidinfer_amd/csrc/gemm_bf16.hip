@@ -3278,31 +3278,37 @@ static int launch_experts_tiles(const bf16* A, const bf16* W, void* C, int mode,
 // Gated product: the fewer rounds of workgroups by the times a k-tile of `choose_quad`, with every expert's pairs taken as the mean and half a
 // standard deviation of evenly drawn ones, rounded up to tiles; from eight rounds of 128-row tiles on the taller one may be counted a fifth
 // longer, since a tile multiplies only the blocks of 64 rows that it has and there is no round of few tiles to wait for.  us with 128 rows a tile
-// against 256, equal rows an expert / rows that random weights draw (half to twice the mean; two draws):
-//   32 experts of 1,792 by 4,096: 64 pairs an expert 173, 176 / 183, 179; 179, 183.  112: 186, 192 / 211, 194; 209, 216.  160: 248, 213 / 247, 262; 249, 262.
-//     200: 283, 242 / 265, 284; 268, 278.  256 (128 rows taken): 287, 242 / 320, 308; 324, 303.  300: 355, 405 / 352, 368; 345, 344.  350: 390, 405 / 388,
-//     393; 383, 392.  400: 412, 419 / 437, 406; 445, 404.  450: 456, 439 / 483, 435; 471, 479.  512: 476, 449 / 524, 507; 516, 499.  603: 585, 556 / 598, 582; 604,
-//     568.  900: 827, 758 / 854, 820; 863, 770.  1,800: 1,637, 1,474 / 1,654, 1,483; 1,640, 1,476
-//   16 experts of 1,408 by 2,048: 96: 39, 40 / 39, 55; 50, 53.  136: 66, 45 / 61, 59; 65, 57.  225: 64, 59 / 65, 89; 64, 61.  300: 80, 111 / 78, 110; 96, 109.  450: 103,
-//     117 / 102, 118; 103, 120.  550 (128 rows taken): 124, 121 / 133, 121; 134, 123.  675: 164, 157 / 162, 173; 162, 173.  900: 204, 190 / 195, 184; 201, 186
-// Over 24 means from 64 to 1,800, these two shapes and equal, mildly and clearly uneven rows the choice takes 1.6 % longer than the faster height each
-// time; a line at 448 pairs took 3.5, always 128 rows 5.0.
-// Down product (short k, float rows): the taller tile from four rounds of 128-row tiles on, where an expert has more rows than such a tile.  Same
-// shapes: 32 experts 128 pairs 116, 116 / 134, 131; 128, 135, 150: 148, 122 / 153, 138; 153, 143, 300: 205, 208 / 212, 203; 208, 193, 603: 345, 313 / 364, 319; 369,
-// 330, 1,800: 951, 837 / 1,036, 852; 1,009, 861.  16 experts, fewer rounds up to 896 pairs: 160: 26, 30 / 26, 36; 25, 35, 300: 43, 42 / 44, 40; 44, 41, 450: 52, 48 /
-// 66, 75; 66, 77, 603: 71, 78 / 70, 77; 70, 78; 900: 98, 91 / 110, 101; 96, 101, 1,200: 138, 126 / 145, 129; 153, 125.
+// and 256, equal rows an expert / rows that random weights draw (half to twice the mean; two draws):
+//   32 experts of 1,792 by 4,096: 64 pairs an expert 171, 174 / 185, 177; 179, 182.  112: 188, 191 / 219, 204; 215, 215.  160: 249, 222 / 261, 285; 254,
+//     264.  225: 274, 256 / 274, 325; 311, 324.  256 (128 rows taken): 281, 263 / 318, 335; 326, 331.  300: 356, 417 / 360, 395; 337, 333.  350: 392, 437 / 393,
+//     394; 384, 412.  400: 419, 441 / 441, 429; 447, 426.  450: 460, 448 / 489, 439; 479, 504.  512: 469, 453 / 525, 513; 517, 510.  603: 584, 558 / 602,
+//     572; 598, 582.  900: 823, 772 / 852, 835; 856, 768.  1,800: 1,629, 1,474 / 1,638, 1,504; 1,633, 1,476
+//   16 experts of 1,408 by 2,048: 64: 33, 34 / 38, 47; 39, 45.  136: 67, 47 / 61, 60; 65, 60.  225: 67, 64 / 66, 63; 66, 64.  300: 83, 121 / 72, 115; 72, 118.  450:
+//     105, 124 / 103, 121; 102, 124.  512 (128 rows taken): 106, 129 / 130, 125; 132, 124.  768: 171, 189 / 170, 188; 172, 186.  900: 203, 193 / 199, 194; 203,
+//     198.  1,800: 371, 380 / 374, 383; 373, 384
+// Over 24 means from 64 to 1,800, these two shapes and equal, mildly and clearly uneven rows the choice takes 1.3 % longer than the faster height each
+// time; a line at 448 pairs takes 2.9, always 128 rows 3.5.
+// Down product (short k, float rows), where an expert has more rows than the lower tile: the taller one from four rounds of 128-row tiles on, and with
+// fewer where its rounds are the fewer both so counted and for rows spread evenly over 0.7 to 1.3 times the mean.  Same shapes: 32 experts 128 pairs
+// 115, 115 / 132, 137; 127, 140, 160: 146, 124 / 149, 144; 147, 141, 300: 202, 205 / 208, 200; 206, 202, 603: 339, 311 / 362, 315; 362, 314, 1,800: 943, 841 / 1,024, 857;
+// 1,004, 860.  16 experts 160: 28, 32 / 30, 38; 30, 37, 225 (128 rows taken): 33, 40 / 46, 40; 46, 41, 300: 45, 43 / 45, 42; 46, 42, 400 (128): 52, 46 / 50, 73; 52, 73, 450
+// (128): 54, 47 / 68, 76; 55, 76, 603: 73, 78 / 74, 78; 73, 81, 768: 80, 83 / 94, 84; 95, 84, 1,200: 137, 126 / 142, 130; 143, 127.  1.2 % longer than the faster; four
+// rounds alone 1.8.
 static bool experts_tall_tiles(int pairs, int E, int N, bool gated, int cus) {
-    const double mean = (double)pairs / E, high = mean + (gated ? 0.5 * sqrt(mean) : 0.0);
-    const int cols = (N + 255) / 256;
-    double t[2], rounds[2];
-    for (int i = 0; i < 2; ++i) {
-        const int bm = i ? 256 : 128, k = i ? 0 : 1;
-        rounds[i] = E * ceil(high / bm) * cols / cus;
-        const double whole = floor(rounds[i]), share = rounds[i] - whole;
-        t[i] = (whole + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) : 0.0)) * QUAD_FULL[k];
-    }
-    if (!gated) return mean > 128 && rounds[0] >= 4.0;
-    return t[1] <= (rounds[0] >= 8.0 ? 1.2 : 1.03) * t[0];
+    const double mean = (double)pairs / E, high = mean + 0.5 * sqrt(mean);
+    // rounds of tiles of 128 (i = 0) or 256 rows for experts' rows spread evenly over `from` to `to`, and the time they take
+    auto rounds = [&](double from, double to, int i) {
+        double tiles = 0.0;
+        for (int q = 0; q < 16; ++q) tiles += ceil((from + (to - from) * (q + 0.5) / 16) / (128 << i));
+        return E * tiles / 16 * ((N + 255) / 256) / cus;
+    };
+    auto time = [&](double from, double to, int i) {
+        const double r = rounds(from, to, i), whole = floor(r), share = r - whole;
+        return (whole + (share > 0 ? (whole ? 0.9 + 0.1 * share : 0.6 + 0.4 * share * share * share) : 0.0)) * QUAD_FULL[i ? 0 : 1];
+    };
+    const double low = time(high, high, 0), tall = time(high, high, 1);
+    if (gated) return tall <= (rounds(high, high, 0) >= 8.0 ? 1.2 : 1.03) * low;
+    return mean > 128 && (rounds(mean, mean, 0) >= 4.0 || (tall <= 1.03 * low && time(0.7 * mean, 1.3 * mean, 1) <= time(0.7 * mean, 1.3 * mean, 0)));
 }
 
 // rows of the tiles that br_experts_tiles takes

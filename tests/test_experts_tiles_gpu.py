@@ -55,10 +55,11 @@ def test_heights_that_are_not_there():
         K.experts_gemm(rnd(4, 64, seed=1), rnd(1, 16, 64, seed=2), first, torch.empty(4, 16, device=DEV), rows=64)
 
 
-# 32 experts of 1,792 by 4,096 and 16 of 1,408 by 2,048: pairs an expert where equal rows and uneven ones are faster by the height named, or as fast
+# 32 experts of 1,792 by 4,096, 16 of 1,408 by 2,048 and 8 of 2,048 by 1,024: pairs an expert where equal rows and uneven ones are faster by the height named, or as fast
 @pytest.mark.parametrize("E,N,gated,tall,flat", [(32, 3584, True, (136, 150, 160, 400, 475, 512, 603, 675, 1800), (64, 96, 300, 350)),
                                                  (16, 2816, True, (136, 150, 160, 900, 1200), (64, 96, 300, 350, 400, 450, 475, 768)),
-                                                 (32, 4096, False, (150, 200, 400, 603, 1800), (64, 128)), (16, 2048, False, (1200, 1800), (64, 160, 603))])
+                                                 (32, 4096, False, (150, 200, 400, 603, 1800), (64, 128)), (16, 2048, False, (300, 350, 768, 1200, 1800), (64, 160, 603)),
+                                                 (8, 1024, False, (1100,), (400, 768))])
 def test_the_height_that_is_chosen(E, N, gated, tall, flat):
     assert torch.cuda.get_device_properties(0).multi_processor_count == 256
     assert [K.experts_tiles_rows(m * E, E, N, gated) for m in tall] == [256] * len(tall)
