@@ -239,15 +239,22 @@ __global__ __launch_bounds__(D) void chunk_prepare_kernel(const CwIn in, const C
 }
 
 // The sequence that `rank` others of a step are longer than (of equal ones: that come before it).  Steps of more than 64 sequences: as they come.
+// Where they come longest first, nothing is looked for; else bit by bit the largest key that more than `rank` are not below (counted one after
+// another, 64 sequences of 50 tokens took 336 us where the walk alone takes 286).
 __device__ __forceinline__ int cw_by_length(const int* cu, int B, int rank) {
     if (B > 64) return rank;
-    const int lane = threadIdx.x & 63, mine = lane < B ? cu[lane + 1] - cu[lane] : -1;
-    int before = 0;
-    for (int i = 0; i < B; ++i) {
-        const int other = __builtin_amdgcn_readlane(mine, i);
-        before += other > mine || (other == mine && i < lane);
+    const int lane = threadIdx.x & 63, at = lane < B ? lane : B - 1;
+    const int len = cu[at + 1] - cu[at], next = lane + 1 < B ? cu[at + 2] - cu[at + 1] : 0;
+    if (!__any(next > len)) return rank;
+    // above any other length the index alone counts, as for lengths that are equal
+    const int key = lane < B ? (len < (1 << 24) ? len : (1 << 24)) * 64 + 63 - lane : -1;
+    const int most = __builtin_amdgcn_readfirstlane(cu[B] - cu[0]);
+    int found = 0;
+    for (int bit = 31 - __clz((most < (1 << 24) ? most : (1 << 24)) | 1) + 6; bit >= 0; --bit) {
+        const int higher = found | 1 << bit;
+        if (__popcll(__ballot(key >= higher)) > rank) found = higher;
     }
-    return __ffsll((unsigned long long)__ballot(lane < B && before == rank)) - 1;
+    return __ffsll((unsigned long long)__ballot(key == found)) - 1;
 }
 
 // A workgroup walks a sequence's chunks for 16 CB columns of one head; wave w holds the state's rows w D / 4 .. + D / 4 and adds a
@@ -566,16 +573,19 @@ static int chunk_run(const CwIn& in, const CwPart& part, float* o, float* state,
     const int rc = br_check_launch();
     if (rc != BR_OK) return rc;
     // 16 columns a workgroup as long as the tokens are those of few sequences as long as the longest: 2.5 workgroups of 16 columns to a compute unit
-    // (delta rule with heads of 128, which holds the most in LDS: 1.9).  Beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of
-    // 128 x 128, gated, 2,048 tokens 125 / 167, 3,517 and 1,501 tokens 247 / 286, 1,307, 804 and 301 117 / 133, 1,500, 700, 400 and 200 141 / 153, 1,300, 900,
-    // 700, 500 and 300 183 / 158, three times 1,000 150 / 150, four times 900 170 / 149, 16 times 300 255 / 219; fixed, 1,307, 804 and 301 123 / 141; delta
-    // rule, 2,048 tokens 184 / 272, 3,517 and 1,501 442 / 569, 1,307, 804 and 301 226 / 232, 1,500, 700, 400 and 200 262 / 277, three times 1,000 273 / 250, twice
-    // 1,000 189 / 179; 64 heads of 64 x 64, WKV, 3,517 and 1,501 218 / 245, 1,300 .. 300 154 / 136; delta rule, 900, 900 and 300 154 / 158.
+    // (delta rule with heads of 128, which holds the most in LDS: 1.9), or 3 (1) of about equal ones, whose last round is as long as the others.
+    // Beyond, 32 columns, which share a chunk's loads.  us with 16 / 32: 32 heads of 128 x 128, gated, 2,048 tokens 127 / 168, 3,517 and 1,501 tokens
+    // 264 / 308, 1,307, 804 and 301 121 / 136, 1,500, 700, 400 and 200 145 / 156, 1,300, 900, 700, 500 and 300 186 / 161, three times 1,000 155 / 152, four
+    // times 900 175 / 152, 16 times 300 256 / 220, 64 times 50 339 / 290; fixed, 1,307, 804 and 301 127 / 142; delta rule, 2,048 tokens 189 / 275, 3,517 and 1,501
+    // 455 / 579, 1,307, 804 and 301 231 / 236, 1,500, 700, 400 and 200 270 / 284, twice 1,000 186 / 173, 700, 650 and 600 185 / 169; 16 heads, twice 1,000
+    // 104 / 146, three times 171 / 158, 1,300 .. 300 184 / 212; 64 heads of 64 x 64, WKV, 3,517 and 1,501 219 / 249, 1,300 .. 300 159 / 141; 12 heads, delta rule, 16
+    // times 300 75 / 86.
     const int cus = br_device_cus();
     if (!cus) return BR_LAUNCH_FAILED;
-    const double units = min((double)T / max_new, (double)part.longs) * in.H * (in.e / 16);
+    const bool equal = (double)T >= 0.9 * max_new * part.longs, held = D == 128 && DELTA;
+    const double units = (equal ? (double)part.longs : (double)T / max_new) * in.H * (in.e / 16);
 #define CW_WALK(CB, S) return chunk_walk<D, CB, S, FORM == CW_WKV ? CW_GLR : FORM>(in, part, scratch, o, state, slot_stride, B, FORM != CW_GLR, s)
-    if (in.e % 32 || units <= (D == 128 && DELTA ? 1.9 : 2.5) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
+    if (in.e % 32 || units <= (equal ? (held ? 1.0 : 3.0) : (held ? 1.9 : 2.5)) * cus) CW_WALK(1, (D == 64 ? 4 : 3));
     if constexpr (DELTA) CW_WALK(2, (D == 64 ? 4 : 2));
     else CW_WALK(2, (D == 64 ? 5 : 3));
 #undef CW_WALK
