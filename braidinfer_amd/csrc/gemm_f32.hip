@@ -425,27 +425,34 @@ static int launch_f32_tiles(const float* A, const float* W, float* C, int M, int
 
 // Whole rounds of tiles (two workgroups to a compute unit) go as they are; the weight rows behind them, or all where there is no whole
 // round, segment by segment, every segment in a workgroup of its own, where that is counted the faster: in runs of columns whose
-// segments' sums fit the scratch.  In us: a tile's work at 0.5 MFLOP a us and compute unit (a lone workgroup 0.7 of two beside
-// each other), the segments' sums written and read at 4 TB/s, 8 for the launches.  279 rows by 28,672 x 4,096: 512 tiles of 1,344 twice, 320 in
-// segments: 553 us, 602 at once; 640 rows by 4,096 x 14,336, whose segments do not fit at once: 593 us, 864 with no segments; 350 rows by
-// 6,144 x 4,096 193, 254.
+// segments' sums fit the scratch.  In us, fitted to 550 products of 17 to 450 rows (as they are within 5 % on average, in segments 8): a workgroup alone on
+// its compute unit takes 0.0062 + 0.0036 TJ a k, two beside each other 0.0108 + 0.0062 TJ; a launch 4; in segments 8 for the launches, 0.9 of
+// those times, and the segments' sums written and read at 4.8 TB/s.  Over those products the choice is 0.9 % slower than the faster form each time.  279 rows
+// by 28,672 x 4,096: 512 tiles of 1,344 twice, 320 in segments: 553 us, 602 at once; 640 rows by 4,096 x 14,336, whose segments do not fit at once: 593 us,
+// 864 with no segments; 350 rows by 6,144 x 4,096 193, 254.  As they are / in segments: 17 rows by 4,096 x 1,024 17.1 / 10.7, by 11,264 x 2,048 30.6 / 22.5, by
+// 28,672 x 2,048 42 / 45; 65 rows by 4,096 x 512 17 / 13.
 template <int TJ>
 static int launch_f32_tile(const float* A, const float* W, float* C, int M, int N, int K, size_t lda, size_t ldc, int acc, int aligned,
                            int cus, float* scratch, size_t scratch_floats, hipStream_t s) {
     const int tm = (M + 16 * TJ - 1) / (16 * TJ), tn = (N + F32_TN - 1) / F32_TN, round = 2 * cus;
     if ((long long)tm * tn > 0x7fffffffLL) return BR_BAD_ARG;
-    const double w = 2.0 * 16 * TJ * F32_TN * K / 0.5e6;
+    // the time of `tiles` workgroups of `k` each
+    auto rounds = [&](long long tiles, double k) {
+        const long long tail = tiles % round;
+        const double alone = k * (0.0062 + 0.0036 * TJ), beside = k * (0.0108 + 0.0062 * TJ);
+        return (double)(tiles / round) * beside + (tail == 0 ? 0.0 : tail <= cus ? alone : beside);
+    };
     int whole = tn, run = 0;                                           // columns of tiles: as they are, of a run in segments
     const int fit = (int)std::min<size_t>(scratch_floats / ((size_t)F32_SEGS * M * F32_TN), (size_t)tn);
     if (K >= F32_KC * F32_SEGS && fit > 0) {
         const int first = (int)((long long)tm * tn / round * round / tm), left = tn - first;
         const long long rest = (long long)tm * left;
-        const double as_is = rest <= cus ? 1.4 * w : 2.0 * w;
+        const double as_is = rounds(rest, K) + (first ? 0.0 : 4.0);
         const int runs = left > 0 ? (left + fit - 1) / fit : 0, each = runs ? (left + runs - 1) / runs : 0;
         double in_segments = 0.0;
         for (int c = 0; c < left; c += each) {
-            const long long u = (long long)tm * std::min(each, left - c) * F32_SEGS, tail = u % round;
-            in_segments += 8.0 + w / F32_SEGS * (2.0 * (u / round) + (tail == 0 ? 0.0 : tail <= cus ? 1.4 : 2.0)) + (double)u * 16 * TJ * F32_TN * 8 / 4e6;
+            const long long u = (long long)tm * std::min(each, left - c) * F32_SEGS;
+            in_segments += 8.0 + 0.9 * rounds(u, (double)K / F32_SEGS) + (double)u * 16 * TJ * F32_TN * 8 / 4.8e6;
         }
         if (left > 0 && in_segments < as_is) whole = first, run = each;
     }
