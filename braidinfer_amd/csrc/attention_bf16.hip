@@ -772,7 +772,7 @@ __device__ __forceinline__ int kswz(int row, int cols) {      // the 16 key rows
 // `fold`: the sequences of one round of workgroups over the compute units where there are up to two rounds; those behind it are
 // taken from the last on, so that in a batch in the order of its lengths a long and a short one share a compute unit (their numbers
 // lie a round apart).  The batch size otherwise.  Whole steps of eight layers, longest first: 64 sequences of 128 to 2,048
-// tokens 6,029 -> 5,960 us (four steps), 8 in 8 runs 3,327 -> 3,290.
+// tokens 6,039 -> 5,988 us (four steps), 8 in 8 runs 3,322 -> 3,293; the kernel alone, launched again and again, gains nothing.
 template <int HD, int S, bool FUSE>
 __global__ __launch_bounds__(256) void attn_decode_lds_kernel(
     const bf16* __restrict__ q, size_t q_stride, bf16* __restrict__ out, const int* __restrict__ slots,

@@ -1,5 +1,5 @@
 """The prompt products' tiles of four waves where their rows or columns end: fewer blocks of rows in the last tile, rows written in runs
-through LDS, and the experts' tiles cut into eight runs of about equal cost."""
+through LDS, and the experts' tiles in eight runs."""
 import pytest
 import torch
 
